@@ -16,6 +16,7 @@
 #ifndef LRQK_HIP_H
 #define LRQK_HIP_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #ifdef __cplusplus
@@ -44,6 +45,13 @@ const char* lrqk_last_error(void);
  * synchronises the device once.  One ctx per engine; calls on one ctx must not overlap. */
 int lrqk_ctx_create(lrqk_ctx** out);
 int lrqk_ctx_destroy(lrqk_ctx* ctx);
+/* Where the ctx takes its device memory from (default: hipMalloc / hipFree, which wait for the device).  alloc returns
+ * `bytes` of device memory of the current device for use on `stream`, or NULL; release takes a block back while work
+ * on that stream may still use it, so it must be stream-ordered as torch's caching allocator is (if calls on the ctx
+ * came on several streams, the library waits for the device before it releases).  Only while the ctx holds no memory.
+ * No counterpart in the reference. */
+int lrqk_ctx_set_allocator(lrqk_ctx* ctx, void* (*alloc)(size_t bytes, void* stream, void* user),
+                           void (*release)(void* block, void* user), void* user);
 /* Optional: pre-size the workspace so that later calls never allocate. */
 int lrqk_ctx_reserve(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d);
 

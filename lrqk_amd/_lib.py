@@ -17,6 +17,11 @@ F32, BF16 = 0, 1
 _lib = None
 
 
+# device memory for a ctx from the caller's allocator: (bytes, stream, user) -> address; (address, user)
+ALLOC_FN = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p)
+RELEASE_FN = ctypes.CFUNCTYPE(None, ctypes.c_void_p, ctypes.c_void_p)
+
+
 class LrqkError(RuntimeError):
     pass
 
@@ -42,6 +47,7 @@ def _sig(lib):
         "lrqk_last_error": ([], c.c_char_p),
         "lrqk_ctx_create": ([c.POINTER(vp)], i32),
         "lrqk_ctx_destroy": ([vp], i32),
+        "lrqk_ctx_set_allocator": ([vp, ALLOC_FN, RELEASE_FN, vp], i32),
         "lrqk_ctx_reserve": ([vp, i32, i64, i32, i32, i32, i32], i32),
         "lrqk_proxy_scores": ([vp, i64, vp, i32, i64, i32, i32, i32, vp, vp], i32),
         "lrqk_score_select": ([vp, vp, i64, vp, i32, i64, i32, i32, i32, i32, vp, i64, vp], i32),

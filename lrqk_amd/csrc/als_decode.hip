@@ -1226,6 +1226,7 @@ extern "C" int lrqk_als_decode(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, i
                                int n, const void* q, const void* k_new, int b, int hq, int hkv, int r, int d,
                                int max_iter, float tol, void* q_hat, void* k_hat, int64_t append_row, int dtype,
                                void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   GramAppend ap{nullptr, nullptr, nullptr, nullptr, -1, 0, hq, hkv};
   if (ctx) ctx->fs_valid = false;  // B_Q, B_K change behind the kept state of the decode step
   return als_decode_checked(ctx, b_q, b_k, a_k, head_stride, active_idx, idx_stride, k_prev, kprev_slots, n, q, k_new, b,

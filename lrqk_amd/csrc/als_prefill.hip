@@ -1205,6 +1205,7 @@ using namespace lrqk;
 extern "C" int lrqk_als_prefill(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, float* b_q,
                                 float* b_k, int b, int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol,
                                 int dtype, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   LRQK_REQUIRE(ctx && q && k && a_q && a_k && b_q && b_k, LRQK_EINVAL, "null pointer");
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(b > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && (int64_t)b * hq <= 65535, LRQK_EINVAL,

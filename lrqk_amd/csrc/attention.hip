@@ -765,6 +765,7 @@ using namespace lrqk;
 
 extern "C" int lrqk_attention(lrqk_ctx* ctx, const void* q, const void* k_act, const void* v_act, int n_slots,
                               int n_valid, void* out, int bh, int d, int dtype, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   LRQK_REQUIRE(ctx && q && k_act && v_act && out, LRQK_EINVAL, "null pointer");
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(bh > 0 && bh <= 65535 && d > 0, LRQK_EINVAL, "bad sizes bh=%d d=%d", bh, d);

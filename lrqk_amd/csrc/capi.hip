@@ -34,36 +34,28 @@ extern "C" const char* lrqk_last_error(void) { return g_err; }
 
 extern "C" int lrqk_ctx_create(lrqk_ctx** out) {
   LRQK_REQUIRE(out != nullptr, LRQK_EINVAL, "out is null");
-  *out = new lrqk_ctx();
+  lrqk_ctx* ctx = new lrqk_ctx();
+  ctx->each_buf([&](DevBuf& b) { b.pool = &ctx->pool; });
+  *out = ctx;
+  return LRQK_OK;
+}
+
+extern "C" int lrqk_ctx_set_allocator(lrqk_ctx* ctx, void* (*alloc)(size_t, void*, void*), void (*release)(void*, void*),
+                                      void* user) {
+  LRQK_REQUIRE(ctx != nullptr && (alloc != nullptr) == (release != nullptr), LRQK_EINVAL, "null pointer");
+  bool held = false;
+  ctx->each_buf([&](DevBuf& b) { held = held || b.p != nullptr; });
+  LRQK_REQUIRE(!held, LRQK_EINVAL, "the ctx already holds memory of its first allocator");
+  ctx->pool.alloc = alloc;
+  ctx->pool.release = release;
+  ctx->pool.user = user;
   return LRQK_OK;
 }
 
 extern "C" int lrqk_ctx_destroy(lrqk_ctx* ctx) {
   if (!ctx) return LRQK_OK;
-  (void)hipDeviceSynchronize();
-  ctx->keys.release();
-  ctx->hist.release();
-  ctx->cand.release();
-  ctx->cand_cnt.release();
-  ctx->attn_part.release();
-  ctx->als_part.release();
-  ctx->als_pre.release();
-  ctx->als_kq.release();
-  ctx->als_iter.release();
-  ctx->als_iter64.release();
-  ctx->fstate.release();
-  ctx->evk.release();
-  ctx->prefill_ws.release();
-  ctx->prefill_gd.release();
-  ctx->new_idx.release();
-  ctx->misc.release();
-  ctx->stage_dev.release();
-  ctx->vic_rows.release();
-  ctx->sidx_qa.release();
-  ctx->sidx_qs.release();
-  ctx->sidx_wm.release();
-  ctx->sidx_part.release();
-  ctx->vic_meta.release();
+  if (ctx->pool.must_wait() || ctx->stage_host || ctx->side || ctx->tev) (void)hipDeviceSynchronize();
+  ctx->each_buf([](DevBuf& b) { b.release(); });
   if (ctx->stage_host) (void)hipHostFree(ctx->stage_host);
   if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);
@@ -78,6 +70,7 @@ extern "C" int lrqk_ctx_destroy(lrqk_ctx* ctx) {
 extern "C" int lrqk_ctx_reserve(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d) {
   LRQK_REQUIRE(ctx != nullptr, LRQK_EINVAL, "ctx is null");
   LRQK_REQUIRE(bh > 0 && max_tokens >= 0 && topk > 0 && n_active > 0 && r > 0 && d > 0, LRQK_EINVAL, "bad sizes");
+  ctx->pool.enter(ctx->pool.stream);
   int rc;
   const int64_t key_stride = (max_tokens + 63) & ~(int64_t)63;
   if ((rc = ctx->keys.ensure((size_t)bh * key_stride * 4))) return rc;

@@ -9,34 +9,56 @@
 
 namespace lrqk {
 
+// Where the blocks of one ctx come from.  By default the HIP runtime; a caller whose process already has a caching
+// allocator hands its functions in (lrqk_ctx_set_allocator): a new ctx then costs a few lookups instead of about
+// twenty hipMalloc (75 .. 310 us each) and as many hipFree behind a device synchronisation, per prompt and layer.
+struct BufPool {
+  void* (*alloc)(size_t bytes, void* stream, void* user) = nullptr;
+  void (*release)(void* p, void* user) = nullptr;
+  void* user = nullptr;
+  hipStream_t stream = nullptr;  // the stream of the call at hand: blocks are allocated for it
+  bool used = false;
+  bool mixed = false;            // calls came on more than one stream: blocks may only go back after a device sync
+  void enter(hipStream_t st) {
+    mixed = mixed || (used && st != stream);
+    used = true;
+    stream = st;
+  }
+  // Work queued on `stream` may still read a block that goes back.  A stream-ordered allocator hands it out again on
+  // that stream only, so nothing has to wait unless another stream was used in between; the runtime's blocks wait.
+  bool must_wait() const { return !alloc || mixed; }
+};
+
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
-  // Grows (never shrinks).  Growing frees the old block after a device sync, because
-  // kernels of an earlier call may still be reading it.
+  BufPool* pool = nullptr;
+  // Grows (never shrinks); the contents are not kept.
   int ensure(size_t need) {
     if (need <= bytes) return LRQK_OK;
     size_t want = need + need / 4;
     void* np = nullptr;
-    LRQK_HIP_CHECK(hipMalloc(&np, want));
+    if (pool->alloc) {
+      np = pool->alloc(want, (void*)pool->stream, pool->user);
+      if (!np) return set_error(LRQK_EHIP, "the caller's allocator has no %zu bytes", want);
+    } else {
+      LRQK_HIP_CHECK(hipMalloc(&np, want));
+    }
     if (p) {
-      LRQK_HIP_CHECK(hipDeviceSynchronize());
-      LRQK_HIP_CHECK(hipFree(p));
+      if (pool->must_wait()) LRQK_HIP_CHECK(hipDeviceSynchronize());
+      release();
     }
     p = np;
     bytes = want;
     return LRQK_OK;
   }
-  // Same, and the block is zero-filled whenever it is (re)allocated.
-  int ensure_zeroed(size_t need) {
-    if (need <= bytes) return LRQK_OK;
-    int rc = ensure(need);
-    if (rc) return rc;
-    LRQK_HIP_CHECK(hipMemset(p, 0, bytes));
-    return LRQK_OK;
-  }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p) {
+      if (pool->alloc)
+        pool->release(p, pool->user);
+      else
+        (void)hipFree(p);
+    }
     p = nullptr;
     bytes = 0;
   }
@@ -45,6 +67,7 @@ struct DevBuf {
 }  // namespace lrqk
 
 struct lrqk_ctx {
+  lrqk::BufPool pool;
   lrqk::DevBuf keys;        // u32 [bh][key_stride]   orderable score keys
   lrqk::DevBuf hist;        // u32 [bh][4096]         first-level radix histogram
   lrqk::DevBuf cand;        // candidate (key,idx) pairs for the fast select path
@@ -110,6 +133,13 @@ struct lrqk_ctx {
   int tev_seen = 0;    // launches seen since timing was enabled
   int sel_bh = 0;      // head count the selector state (t_low, counters) was initialised for
   int last_short = 0, last_overflow = 0;  // split of the rescans seen by the last lrqk_select_stats
+  template <typename F>
+  void each_buf(F&& f) {
+    for (lrqk::DevBuf* b : {&keys, &hist, &cand, &cand_cnt, &attn_part, &als_part, &als_kq, &als_pre, &als_iter, &als_iter64,
+                            &fstate, &evk, &prefill_ws, &prefill_gd, &new_idx, &misc, &sidx_qa, &sidx_qs, &sidx_wm,
+                            &sidx_part, &vic_rows, &vic_meta, &stage_dev})
+      f(*b);
+  }
   int scan_wgs = 0;        // workgroups of the last scan through the score index (0: the last scan read A_K itself)
   int64_t scan_rows = 0;   // rows that scan covered (all heads)
 };

@@ -80,6 +80,7 @@ extern "C" int lrqk_fetch_rows_staged(lrqk_ctx* ctx, const void* kv_store, int64
                                       int n_slots, const int32_t* hit, int64_t hit_stride, const int32_t* miss_slots,
                                       const int32_t* miss_count, int b, int hq, int hkv, int d, int k, int dtype,
                                       void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   LRQK_REQUIRE(ctx && kv_store && k_act && v_act && hit && miss_slots && miss_count, LRQK_EINVAL, "null pointer");
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(b > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && d > 0, LRQK_EINVAL, "bad heads b=%d hq=%d hkv=%d", b, hq, hkv);

@@ -1770,6 +1770,7 @@ extern "C" int lrqk_proxy_scores(const void* a_k, int64_t head_stride, const voi
 extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
                                  int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
                                  int64_t out_stride, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   int rc = check_select_args(ctx, bh, m, topk, out_idx, out_stride);
   if (rc) return rc;
   LRQK_REQUIRE(a_k && q_hat, LRQK_EINVAL, "null pointer");
@@ -1793,6 +1794,7 @@ extern "C" int lrqk_score_select_diff(lrqk_ctx* ctx, const void* a_k, int64_t he
                                       int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* new_idx,
                                       int32_t* hit, int64_t hit_stride, uint8_t* evict, int32_t* miss_slots,
                                       int32_t* miss_count, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   LRQK_REQUIRE(ctx && a_k && q_hat && hit && miss_slots && miss_count, LRQK_EINVAL, "null pointer");
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(r > 0 && r <= LRQK_MAX_R, LRQK_EINVAL, "r=%d", r);
@@ -1817,6 +1819,7 @@ extern "C" int lrqk_score_select_diff(lrqk_ctx* ctx, const void* a_k, int64_t he
 
 extern "C" int lrqk_select_from_scores(lrqk_ctx* ctx, const float* scores, int bh, int64_t m, int topk,
                                        int32_t* out_idx, int64_t out_stride, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   int rc = check_select_args(ctx, bh, m, topk, out_idx, out_stride);
   if (rc) return rc;
   LRQK_REQUIRE(scores != nullptr, LRQK_EINVAL, "scores is null");

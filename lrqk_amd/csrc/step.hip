@@ -14,6 +14,7 @@ extern "C" int lrqk_decode_step(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, 
                                 int topk, int lite, int ring_slot, int32_t token, int64_t m, int64_t flush_row0,
                                 int max_iter, float tol, int round_scores, int no_hit_miss, void* q_hat, void* k_hat,
                                 void* attn_out, uint8_t* evict, int32_t* miss_count, int dtype, void* stream) {
+  if (ctx) ctx->pool.enter((hipStream_t)stream);
   LRQK_REQUIRE(ctx != nullptr, LRQK_EINVAL, "ctx is null");
   LRQK_REQUIRE(topk > 0 && lite > 0 && ring_slot >= 0 && ring_slot < lite, LRQK_EINVAL, "bad ring slot %d of %d", ring_slot,
                lite);

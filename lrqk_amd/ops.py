@@ -33,12 +33,34 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# A ctx takes its device memory from torch's caching allocator, for the stream of the call that needs it: a cache
+# object per prompt then reuses the blocks of the one before (nothing waits for the device), torch sees the memory in
+# its statistics and gives it back when it runs short.
+@_lib.ALLOC_FN
+def _torch_alloc(nbytes, stream, user):
+    try:
+        return torch.cuda.caching_allocator_alloc(nbytes, stream=stream or 0)
+    except Exception:  # nothing may pass through the C frames; the library reports the size it did not get
+        return None
+
+
+@_lib.RELEASE_FN
+def _torch_release(block, user):
+    try:
+        torch.cuda.caching_allocator_delete(block)
+    except Exception:  # the interpreter is shutting down
+        pass
+
+
 class Workspace:
     """Owns one lrqk_ctx (device scratch).  Not thread safe; one per engine."""
 
     def __init__(self):
         self._h = ctypes.c_void_p()
-        check(_lib.load().lrqk_ctx_create(ctypes.byref(self._h)))
+        lib = _lib.load()
+        check(lib.lrqk_ctx_create(ctypes.byref(self._h)))
+        self._allocator = (_torch_alloc, _torch_release)  # alive as long as the ctx may call them
+        check(lib.lrqk_ctx_set_allocator(self._h, *self._allocator, None))
 
     @property
     def handle(self):
