@@ -198,6 +198,15 @@ int lrqk_append_token(const void* k_new, const void* v_new, void* k_act, void* v
 int lrqk_flush_ring(const void* k_act, const void* v_act, int n_slots, int slot0, int count, void* kv_store,
                     int64_t cap, int64_t row0, int b, int hq, int hkv, int d, int dtype, void* stream);
 
+/* py:959-963 for a whole prompt, in two steps so that the copy over the host link runs beside the factorisation:
+ * lrqk_interleave_kv writes out[heads][l][2d] = [K row | V row] in device memory (k, v: [heads][l][d]);
+ * lrqk_store_rows copies those rows to store rows [row0, row0 + l) of every head of the pinned host store
+ * [heads][cap][2d] with a DMA engine, on a stream of the caller's choice (which waits for the first step; `rows` must
+ * stay until the copy is done). */
+int lrqk_interleave_kv(const void* k, const void* v, void* out, int heads, int64_t l, int d, int dtype, void* stream);
+int lrqk_store_rows(const void* rows, void* kv_store, int64_t cap, int64_t row0, int heads, int64_t l, int d,
+                    int dtype, void* stream);
+
 /* py:2326-2327 (flash_attn_with_kvcache, one query, scale 1/sqrt(d)) -- exact attention
  * over the first n_valid slots.  q,out: [bh][d]; k_act,v_act: [bh][n_slots][d]. */
 int lrqk_attention(lrqk_ctx* ctx, const void* q, const void* k_act, const void* v_act, int n_slots,

@@ -230,7 +230,21 @@ class LightAttentionIndicesFactory:
         self.current_len = seq_len
         # a new sequence: whatever the victim cache holds belongs to the previous one
         self.ws.victim_cache(self.victim_rows_effective)
+        stored = self._store_prompt(key_states, value_states) if seq_len > self.gpu_capacity else None
+        try:
+            self._factorise_prompt(query_states, key_states, value_states)
+        finally:
+            if stored is not None:
+                # What is queued from here on finds the prompt in the store (and the staging block may be reused).
+                # The event is recorded only now: its packet holds up the hardware queue of the side stream until
+                # the copy is done, and with four hardware queues one side stream in four shares this stream's
+                # (recorded right after the copy it made 128K prompts take 15 instead of 10 ms one time in four).
+                torch.cuda.current_stream(dev).wait_stream(stored[0])
 
+    def _factorise_prompt(self, query_states, key_states, value_states):
+        seq_len = query_states.shape[2]
+        k, L, g = self.attn_topk, self.num_lite_tokens, self.num_key_value_groups
+        dev = query_states.device
         from .factor import cast_lrqk_prefill
         A_Q, B_Q, A_K, B_K = cast_lrqk_prefill(query_states, key_states, r=self.r, lambda_Q=self.weights[0],
                                                lambda_K=self.weights[1], max_iter=self.max_iter[0], tol=self.tol[0],
@@ -257,7 +271,6 @@ class LightAttentionIndicesFactory:
             self._active_idx[:, :, :seq_len] = torch.arange(seq_len, dtype=torch.int32, device=dev)
             self._hit_len = k
         else:
-            self._store_prompt(key_states, value_states)
             # the rows are scanned where they will live (same values as A_K, which sync_cache copied there): the
             # score index that this first scan builds then stays valid for the decode steps
             hit = self.compute_hit_indices(query_states=A_Q[:, :, -1:, :],
@@ -274,10 +287,17 @@ class LightAttentionIndicesFactory:
             self._active_idx[:, :, k:] = torch.arange(lb, seq_len, dtype=torch.int32, device=dev)
         self.last_A_Q_row = A_Q[:, :, -1:, :]
 
+    # From this size on the prompt's rows go to the host store through a DMA engine, beside the factorisation.  The
+    # flush kernel holds the stream for bytes / 55 GB/s (38 us at this size); the copy needs a pass over the rows in
+    # device memory and about 25 us of host time for its stream and events.
+    _DMA_STORE_BYTES = 2 << 20
+
     def _store_prompt(self, key_states: torch.Tensor, value_states: torch.Tensor):
-        """The prompt's rows into the host store (what ``KVcpu.append`` does, lrqk_attention.py:959-963), written
-        by a kernel straight into the pinned block as [K|V] rows: a host-side ``copy_`` into the interleaved
-        layout goes through a staging copy and took 155 ms for a 128K prompt of 8 kv heads against 11 ms."""
+        """The prompt's rows into the host store (what ``KVcpu.append`` does, lrqk_attention.py:959-963).  Returns
+        ``(stream, staging)`` of a copy that is under way on that stream, or None if the stream's own order is enough.
+        (A host-side ``copy_`` into the interleaved layout goes through a staging copy and took 155 ms for a 128K
+        prompt of 8 kv heads; a kernel that writes the pinned block itself 9.8 ms during which nothing else runs: other
+        kernels beside it take twelve times their time.  A DMA engine takes 9.4 ms at 57 GB/s and slows nothing.)"""
         b, hkv, length, d = key_states.shape
         if self.KVcpu.dtype is None:
             self.KVcpu.dtype = key_states.dtype
@@ -285,9 +305,16 @@ class LightAttentionIndicesFactory:
             self.KVcpu.device = torch.device("cpu")
         if not (self.KVcpu.pin_memory and key_states.is_cuda):
             self.KVcpu.append(key_states, value_states)
-            return
+            return None
         row0 = self.KVcpu.extend((b, hkv, 0, 2 * d), length)
-        ops.flush_ring(key_states, value_states, 0, length, self.KVcpu.data, row0, hkv)
+        if 2 * key_states.numel() * key_states.element_size() < self._DMA_STORE_BYTES:
+            ops.flush_ring(key_states, value_states, 0, length, self.KVcpu.data, row0, hkv)
+            return None
+        rows = ops.interleave_kv(key_states, value_states)
+        side = torch.cuda.Stream(key_states.device)
+        side.wait_stream(torch.cuda.current_stream(key_states.device))
+        ops.store_rows(rows, self.KVcpu.data, row0, side)
+        return side, rows
 
     # ------------------------------------------------------------------ decode
     def _bookkeep_append(self) -> Tuple[int, int, int]:

@@ -320,6 +320,27 @@ def flush_ring(k_act, v_act, slot0: int, count: int, kv_store: torch.Tensor, row
                                       row0, b, hq, hkv, d, _dt(k_act), _stream(k_act)))
 
 
+def interleave_kv(k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """k, v [b,Hkv,l,d] contiguous -> [b,Hkv,l,2d] on the device, each token's K row followed by its V row."""
+    _need_cuda(k, v)
+    b, hkv, l, d = k.shape
+    assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape and v.dtype == k.dtype
+    out = torch.empty((b, hkv, l, 2 * d), dtype=k.dtype, device=k.device)
+    check(_lib.load().lrqk_interleave_kv(k.data_ptr(), v.data_ptr(), out.data_ptr(), b * hkv, l, d, _dt(k), _stream(k)))
+    return out
+
+
+def store_rows(rows: torch.Tensor, kv_store: torch.Tensor, row0: int, stream: torch.cuda.Stream):
+    """rows [b,Hkv,l,2d] on the device -> rows row0 .. row0 + l of the pinned host store [b,Hkv,cap,2d], by a DMA
+    engine on ``stream``.  The caller orders the stream and keeps ``rows`` until the copy is done."""
+    _need_cuda(rows)
+    b, hkv, l, d2 = rows.shape
+    assert rows.is_contiguous() and kv_store.is_contiguous() and kv_store.is_pinned() and kv_store.dtype == rows.dtype
+    assert tuple(kv_store.shape[:2]) == (b, hkv) and kv_store.shape[3] == d2
+    check(_lib.load().lrqk_store_rows(rows.data_ptr(), kv_store.data_ptr(), kv_store.shape[2], row0, b * hkv, l, d2 // 2,
+                                      _dt(rows), stream.cuda_stream))
+
+
 def attention(ws: Workspace, q: torch.Tensor, k_act: torch.Tensor, v_act: torch.Tensor,
               n_valid: Optional[int] = None) -> torch.Tensor:
     """q [b,H,1,d]; k_act,v_act [b,H,n,d] contiguous -> [b,H,1,d]."""
