@@ -242,13 +242,22 @@ int lrqk_als_decode(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64_t head
  * a_q,a_k: [bh][l][r] fp32 work buffers holding the initial factors on entry and the
  * result on return; b_q,b_k out: [bh][r][d] fp32.  The stopping test (batch-wide mean squared
  * change of A_Q and A_K below tol) is evaluated on the device: once it fires the remaining
- * launches return at once, and the host never waits.  r <= 32: bf16 input with d <= 128 runs on
- * the bf16 matrix cores (fp32 operands as three bf16 pieces each, fp32 accumulation), fp32 input
- * or d = 256 on fp32 MFMA tiles, other shapes -- and ranks up to 64 (README.md:124-131 of the reference
- * names r = 64) -- on a general kernel, as long as r (r + d) <= 12288.  Returns 0. */
+ * launches return at once, and the host never waits.  Rows of 64 or 128 elements (16-byte aligned): the
+ * iterations run on d x d Gram matrices in fp64 and the long axis is read twice whatever max_iter is (sums and result
+ * on the bf16 matrix cores, fp32 operands as three bf16 pieces, fp32 accumulation).  Other shapes row by row: r <= 32 on
+ * bf16 or fp32 matrix-core tiles, ranks up to 64 (README.md:124-131 of the reference names r = 64) on a general kernel,
+ * as long as r (r + d) <= 12288.  Returns 0. */
 int lrqk_als_prefill(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, float* b_q,
                      float* b_k, int b, int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol,
                      int dtype, void* stream);
+
+/* The same fit with its results where and as a cache keeps them: a_q0, a_k0 (fp32 [bh][l][r]) hold the initial factors
+ * and are work buffers; in the storage dtype come a_q (the last a_q_rows rows of every head, 1 or l: a cache asks for
+ * the last one only), a_k (heads a_k_stride >= l r elements apart, so that a growing buffer takes them as they are)
+ * and b_q, b_k [bh][r][d]. */
+int lrqk_als_prefill_store(lrqk_ctx* ctx, const void* q, const void* k, float* a_q0, float* a_k0, void* a_q,
+                           int64_t a_q_rows, void* a_k, int64_t a_k_stride, void* b_q, void* b_k, int b, int hq,
+                           int hkv, int64_t l, int r, int d, int max_iter, float tol, int dtype, void* stream);
 
 /* py:1506-1613 LightAttentionIndicesFactory.decode (main branch) + the attention call
  * site py:2326 -- one decode step of one layer as one host call that only enqueues

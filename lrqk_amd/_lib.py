@@ -73,6 +73,8 @@ def _sig(lib):
         "lrqk_als_decode": ([vp, vp, vp, vp, i64, vp, i64, vp, i32, i32, vp, vp, i32, i32, i32, i32, i32, i32, f32,
                              vp, vp, i64, i32, vp], i32),
         "lrqk_als_prefill": ([vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i64, i32, i32, i32, f32, i32, vp], i32),
+        "lrqk_als_prefill_store": ([vp, vp, vp, vp, vp, vp, i64, vp, i64, vp, vp, i32, i32, i32, i64, i32, i32, i32, f32,
+                                    i32, vp], i32),
         "lrqk_decode_step": ([vp, vp, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32,
                               i32, i32, i64, i64, i32, f32, i32, i32, vp, vp, vp, vp, vp, i32, vp], i32),
         "lrqk_select_stats": ([vp, c.POINTER(i32), c.POINTER(i32), i32], i32),

@@ -33,13 +33,17 @@ class AutoIncreaseTensor:
         pin = bool(self.pin_memory) and torch.cuda.is_available()
         return torch.zeros(shape, device=self.device, dtype=self.dtype, pin_memory=pin)
 
-    def _ensure(self, like_shape, length: int):
+    def _ensure(self, like_shape, length: int, overwritten: bool = False):
         target = self.current_len + length
         if self.data is None:
             cap = max(self.capacity, int(length * self.scaling_ratio))
             shape = list(like_shape)
             shape[self.dim] = cap
-            self.data = self._alloc(shape)
+            if overwritten and not self.pin_memory:
+                self.data = torch.empty(shape, device=self.device, dtype=self.dtype)
+                self.data.narrow(self.dim, length, cap - length).zero_()
+            else:
+                self.data = self._alloc(shape)
             self.capacity = cap
         elif target >= self.capacity:
             cap = self.capacity
@@ -69,10 +73,11 @@ class AutoIncreaseTensor:
         self.current_len += length
 
     @torch.inference_mode()
-    def extend(self, like_shape, length: int) -> int:
+    def extend(self, like_shape, length: int, overwritten: bool = False) -> int:
         """Make room for ``length`` more entries exactly as ``append`` would, without writing
-        them (a kernel fills the rows).  Returns the index of the first new entry."""
-        self._ensure(like_shape, length)
+        them (a kernel fills the rows).  Returns the index of the first new entry.  ``overwritten``: every
+        one of these rows is written before it is read, so a first allocation clears the rest only."""
+        self._ensure(like_shape, length, overwritten)
         first = self.current_len
         self.current_len += length
         return first

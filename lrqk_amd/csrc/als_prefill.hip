@@ -14,6 +14,7 @@
 // every other shape.  Both write the same partial-sum layout.
 #include <algorithm>
 #include <stdlib.h>
+#include <type_traits>
 
 #include "common.hpp"
 #include "ctx.hpp"
@@ -594,11 +595,9 @@ __device__ __forceinline__ bf16x8 pf_bf16x8(uint32_t a, uint32_t b, uint32_t c, 
   return __builtin_bit_cast(bf16x8, make_uint4(a, b, c, d));
 }
 
-// GRAMS = false: only A <- X Mt^T (the last pass of the iteration on Gram matrices, which needs neither the sums
-// over the new rows nor their change): the old rows are not read and nothing is reduced.
 // GIVEN = true: only the sums over the given rows of A (Mt must be null); the rows of A are requested one tile
 // ahead, like the rows of X.
-template <int NB, int NW, bool GRAMS = true, bool GIVEN = false>
+template <int NB, int NW, bool GIVEN = false>
 __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* __restrict__ X, int xh, int hq,
                                                                   int64_t l, int r, int d,
                                                                   const float* __restrict__ Mt, float* __restrict__ A,
@@ -719,7 +718,7 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
       issue(t0 + 32 * NW);
       issue_old(t0 + 32 * NW);
     }
-    if constexpr (GRAMS && !GIVEN) {
+    if constexpr (!GIVEN) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int64_t rr = min(t0 + pf_mfma_row(lane, v), l - 1);
@@ -745,20 +744,14 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
       for (int v = 0; v < 16; ++v) {
         const int row = pf_mfma_row(lane, v);
         if (row < rows && col < r) {
-          if constexpr (GRAMS) {
-            const float df = old[v] - c[v];
-            dsum = fmaf(df, df, dsum);
-          }
+          const float df = old[v] - c[v];
+          dsum = fmaf(df, df, dsum);
           Ah[(t0 + row) * r + col] = c[v];
         }
       }
     } else {
 #pragma unroll
       for (int v = 0; v < 16; ++v) c[v] = (pf_mfma_row(lane, v) < rows && col < r) ? old[v] : 0.0f;
-    }
-    if constexpr (!GRAMS) {
-      pf_wave_sync();  // this wave's reads of the tile precede its next staging writes
-      continue;
     }
     // the three pieces of C, eight rows (one k block) at a time
     bf16x8 cp[3][2];
@@ -842,7 +835,6 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
     }
     pf_wave_sync();  // this wave's reads of the tile precede its next staging writes
   }
-  if constexpr (!GRAMS) return;
   __syncthreads();  // every wave is done with its tile (and with Mt): the LDS is reused below
 
   // reduce the waves' tiles through LDS, one 32 x 32 block at a time (tile nb of G_AX: columns 32 nb + n)
@@ -1067,16 +1059,41 @@ __global__ __launch_bounds__(kPfSmallThreads) void pf_small32_kernel(int stage, 
                     [&](int i, int j, float x) { Mt[(int64_t)h * r * d + i * d + j] = x; });
 }
 
+__global__ void clear_flags_kernel(int* flags, int n) {  // (a kernel: the launches may be captured into a graph)
+  for (int i = threadIdx.x; i < n; i += blockDim.x) flags[i] = 0;
+}
+
 template <typename T>
 using PfPassFn = void (*)(const T*, int, int, int64_t, int, int, const float*, float*, float*, float*, const int*, int);
 
+// The sums over given factors against bf16 rows of 128 elements (a head per query head, rows per head of X).
+int prefill_given_sums_bf16(const bf16_t* x, int xh, int hq, int b, int64_t l, int r, float* a, float* part, int S,
+                            hipStream_t st) {
+  auto kern = pf_pass_bf16_kernel<4, 8, true>;
+  const size_t smem = std::max((size_t)8 * 32 * (128 + 16) * sizeof(uint16_t), (size_t)8 * 1024 * sizeof(float));
+  LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+  hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)(b * hq)), dim3(8 * kWave), smem, st, x, xh, hq, l, r, 128,
+                     (const float*)nullptr, a, part, (float*)nullptr, (const int*)nullptr, S);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
+}
+
 template <typename T>
-static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, float* b_q, float* b_k,
-                        int b, int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol, hipStream_t st) {
+static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, const PrefillOut& out, int b,
+                        int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol, hipStream_t st) {
   constexpr int VEC = Vec16<T>::N;
   const int bh = b * hq;
   const int ne = r * (r + d);
-  const bool mfma = r <= 32 && d % VEC == 0 && d <= 256 && ((uintptr_t)q % 16 == 0) && ((uintptr_t)k % 16 == 0);
+  const int iters = max_iter > 0 ? max_iter : 0;
+  const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)k % 16 == 0);
+  // Every iteration on d x d Gram matrices in fp64, the rows read twice (sums, result) whatever the iteration count:
+  // rows of 64 or 128 elements.  A prompt of fewer rows than two Gram matrices has is left to the row-by-row
+  // formulation (X^T X is then no smaller than X, and with about as many rows as the rank both are ill-posed), except
+  // bf16 rows of 128 elements at ranks up to 32.
+  const bool gram_domain = aligned && (d == 64 || d == 128) && !getenv("LRQK_PREFILL_ROWWISE") &&
+                           ((sizeof(T) == 2 && d == 128 && r <= 32) || l >= 2 * d);
+  if (gram_domain) return prefill_gram_domain<T>(ctx, (const T*)q, (const T*)k, a_q, a_k, out, b, hq, hkv, l, r, d, iters, tol, st);
+  const bool mfma = r <= 32 && d % VEC == 0 && d <= 256 && aligned;
   const bool small32 = r <= 32 && d <= kPfSmallThreads - 32 && d % 4 == 0;
   LRQK_REQUIRE(mfma || ne <= kPfThreads * kPfMaxPer, LRQK_ELIMIT, "r*(r+d)=%d exceeds %d", ne, kPfThreads * kPfMaxPer);
   // (the general pass: a 16 x 16 thread grid with ceil(r / 16) rows and 48 / that many columns of the sums per thread)
@@ -1085,26 +1102,24 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   // splits of the long axis: about one workgroup per CU (a pass keeps one wave per SIMD busy), but
   // at least 128 rows per split
   int S = std::max(1, std::min(64, 256 / bh));
-  // The row-by-row formulation solves its r x r systems from these sums in fp32, and a split adds its rows up in
+  // This formulation solves its r x r systems from these sums in fp32, and a split adds its rows up in
   // fp32: at most 2048 rows per split there (the partial sums are added in fp64), however few splits fill the GPU.
-  // (The iteration on Gram matrices takes only its first sums from here, where the systems are well conditioned.)
-  // (At most 64 splits per head: beyond 128K rows a split of the row-by-row formulation adds up l / 64 rows.)
-  // bf16 rows of 128 elements, 16-byte aligned: every iteration runs on the d x d Gram matrices (fp64)
-  const bool gram_domain = sizeof(T) == 2 && mfma && d == 128 && r <= 32 && !getenv("LRQK_PREFILL_ROWWISE");
-  if (!gram_domain) S = (int)std::min<int64_t>(64, std::max<int64_t>(S, (l + 2047) / 2048));
+  // (At most 64 splits per head: beyond 128K rows a split adds up l / 64 rows.)
+  S = (int)std::min<int64_t>(64, std::max<int64_t>(S, (l + 2047) / 2048));
   S = (int)std::max<int64_t>(1, std::min<int64_t>(S, (l + 127) / 128));
-  const int iters = max_iter > 0 ? max_iter : 0;
-  // workspace: partQ, partK, Mt, deltas[iters][2][bh][S], flags[iters+1]
+  // workspace: partQ, partK, Mt, b_q, b_k, deltas[iters][2][bh][S], flags[iters+1]
   const size_t n_part = (size_t)bh * S * ne;
   const size_t n_mt = (size_t)bh * r * d;
   const size_t n_delta = (size_t)(iters > 0 ? iters : 1) * 2 * bh * S;
-  const size_t total = (2 * n_part + n_mt + n_delta) * sizeof(float) + (size_t)(iters + 1) * sizeof(int);
+  const size_t total = (2 * n_part + 3 * n_mt + n_delta) * sizeof(float) + (size_t)(iters + 1) * sizeof(int);
   int rc = ctx->prefill_ws.ensure(total);
   if (rc) return rc;
   float* partQ = (float*)ctx->prefill_ws.p;
   float* partK = partQ + n_part;
   float* Mt = partK + n_part;
-  float* deltas = Mt + n_mt;
+  float* b_q = Mt + n_mt;
+  float* b_k = b_q + n_mt;
+  float* deltas = b_k + n_mt;
   int* flags = (int*)(deltas + n_delta);
 
   PfPassFn<T> pass = pf_pass_generic_kernel<T>;
@@ -1135,50 +1150,13 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   const dim3 grid((unsigned)S, (unsigned)bh), blk((unsigned)pass_threads), sblk(small32 ? kPfSmallThreads : kPfThreads);
   const T* Q = (const T*)q;
   const T* K = (const T*)k;
-  // bf16 rows of 128 elements: every iteration on the d x d Gram matrices (fp64), then one pass per side that
-  // applies the last Mq, Mk; the Q side's sums over the given factors are formed together with Q^T Q (one
-  // reading of Q), the K side's by the pass below (A_K has a head per query head, K per kv head)
-  const bool fused_sums = gram_domain && !getenv("LRQK_PREFILL_SEPARATE_SUMS");  // (the Q side's, with Q^T Q)
-  // (the iteration on Gram matrices writes every stopping flag before it reads it)
-  if (!gram_domain) LRQK_HIP_CHECK(hipMemsetAsync(flags, 0, (size_t)(iters + 1) * sizeof(int), st));
-  {
-    PfPassFn<T> first = pass;  // the sums over the given initial factors
-    if constexpr (sizeof(T) == 2) {
-      if (mfma && d == 128) {
-        first = (PfPassFn<T>)pf_pass_bf16_kernel<4, 8, true, true>;
-        if (smem_pass > 48 * 1024)
-          LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_pass));
-      }
-    }
-    if (!fused_sums)
-      hipLaunchKernelGGL(first, grid, blk, smem_pass, st, Q, hq, hq, l, r, d, (const float*)nullptr, a_q, partQ,
-                         (float*)nullptr, (const int*)nullptr, S);
-    hipLaunchKernelGGL(first, grid, blk, smem_pass, st, K, hkv, hq, l, r, d, (const float*)nullptr, a_k, partK,
-                       (float*)nullptr, (const int*)nullptr, S);
-    LRQK_HIP_CHECK(hipGetLastError());
-  }
-  if constexpr (sizeof(T) == 2) {
-    if (gram_domain) {
-      float *mt_q = nullptr, *mt_k = nullptr;
-      if ((rc = prefill_gram_domain(ctx, q, k, fused_sums ? nullptr : partQ, partK, S, fused_sums ? a_q : nullptr, b_q,
-                                    b_k, b, hq, hkv, l, r, iters, tol, flags, &mt_q, &mt_k, st)))
-        return rc;
-      if (iters > 0) {
-        PfPassFn<T> lean = (PfPassFn<T>)pf_pass_bf16_kernel<4, 8, false>;
-        if (smem_pass > 48 * 1024)
-          LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)lean, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_pass));
-        hipLaunchKernelGGL(lean, grid, blk, smem_pass, st, Q, hq, hq, l, r, d, (const float*)mt_q, a_q, partQ, deltas,
-                           (const int*)nullptr, S);
-        int rck = LRQK_OK;
-        if (getenv("LRQK_PREFILL_SEPARATE_SUMS") || !prefill_apply_shared(k, mt_k, a_k, b, hq, hkv, l, r, st, &rck))
-          hipLaunchKernelGGL(lean, grid, blk, smem_pass, st, K, hkv, hq, l, r, d, (const float*)mt_k, a_k, partK,
-                             deltas + (size_t)bh * S, (const int*)nullptr, S);
-        if (rck) return rck;
-        LRQK_HIP_CHECK(hipGetLastError());
-      }
-      return LRQK_OK;
-    }
-  }
+  hipLaunchKernelGGL(clear_flags_kernel, dim3(1), dim3(64), 0, st, flags, iters + 1);
+  // the sums over the given initial factors
+  hipLaunchKernelGGL(pass, grid, blk, smem_pass, st, Q, hq, hq, l, r, d, (const float*)nullptr, a_q, partQ, (float*)nullptr,
+                     (const int*)nullptr, S);
+  hipLaunchKernelGGL(pass, grid, blk, smem_pass, st, K, hkv, hq, l, r, d, (const float*)nullptr, a_k, partK, (float*)nullptr,
+                     (const int*)nullptr, S);
+  LRQK_HIP_CHECK(hipGetLastError());
   for (int it = 0; it < iters; ++it) {
     float* dq = deltas + ((size_t)it * 2 + 0) * bh * S;
     float* dk = deltas + ((size_t)it * 2 + 1) * bh * S;
@@ -1195,25 +1173,50 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   hipLaunchKernelGGL(small, dim3((unsigned)bh), sblk, smem_small, st, 2, iters, partQ, partK, S, bh, r, d, l, tol,
                      deltas, flags, Mt, b_q, b_k);
   LRQK_HIP_CHECK(hipGetLastError());
-  return LRQK_OK;
+  auto finish = [&](auto* o_q, auto* o_k, auto* ob_q, auto* ob_k) -> int {
+    using OUT = std::remove_reference_t<decltype(*o_q)>;
+    const int64_t n = out.a_q_rows * r, rd = (int64_t)bh * r * d;
+    int rcs;
+    if ((rcs = prefill_store<OUT>(a_q + (l - out.a_q_rows) * r, l * r, o_q, n, n, bh, st))) return rcs;
+    if ((rcs = prefill_store<OUT>(a_k, l * r, o_k, out.a_k_stride, l * r, bh, st))) return rcs;
+    if ((rcs = prefill_store<OUT>(b_q, rd, ob_q, rd, rd, 1, st))) return rcs;
+    return prefill_store<OUT>(b_k, rd, ob_k, rd, rd, 1, st);
+  };
+  if (out.storage && sizeof(T) == 2) return finish((T*)out.a_q, (T*)out.a_k, (T*)out.b_q, (T*)out.b_k);
+  return finish((float*)out.a_q, (float*)out.a_k, (float*)out.b_q, (float*)out.b_k);
 }
 
 }  // namespace lrqk
 
 using namespace lrqk;
 
-extern "C" int lrqk_als_prefill(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, float* b_q,
-                                float* b_k, int b, int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol,
-                                int dtype, void* stream) {
-  if (ctx) ctx->pool.enter((hipStream_t)stream);
-  LRQK_REQUIRE(ctx && q && k && a_q && a_k && b_q && b_k, LRQK_EINVAL, "null pointer");
+static int prefill_checked(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, const PrefillOut& out, int b,
+                           int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol, int dtype, void* stream) {
+  LRQK_REQUIRE(ctx && q && k && a_q && a_k && out.a_q && out.a_k && out.b_q && out.b_k, LRQK_EINVAL, "null pointer");
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(b > 0 && hq > 0 && hkv > 0 && hq % hkv == 0 && (int64_t)b * hq <= 65535, LRQK_EINVAL,
                "bad heads b=%d hq=%d hkv=%d", b, hq, hkv);
   LRQK_REQUIRE(r > 0 && r <= LRQK_MAX_R && d > 0 && l > 0 && l < ((int64_t)1 << 31), LRQK_EINVAL, "bad sizes r=%d d=%d l=%lld",
                r, d, (long long)l);
   LRQK_REQUIRE(max_iter <= 64, LRQK_ELIMIT, "max_iter=%d > 64", max_iter);
+  LRQK_REQUIRE((out.a_q_rows == 1 || out.a_q_rows == l) && out.a_k_stride >= l * r, LRQK_EINVAL,
+               "a_q_rows=%lld (1 or all %lld), a_k_stride=%lld", (long long)out.a_q_rows, (long long)l, (long long)out.a_k_stride);
+  ctx->pool.enter((hipStream_t)stream);
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == LRQK_F32) return prefill_impl<float>(ctx, q, k, a_q, a_k, b_q, b_k, b, hq, hkv, l, r, d, max_iter, tol, st);
-  return prefill_impl<bf16_t>(ctx, q, k, a_q, a_k, b_q, b_k, b, hq, hkv, l, r, d, max_iter, tol, st);
+  if (dtype == LRQK_F32) return prefill_impl<float>(ctx, q, k, a_q, a_k, out, b, hq, hkv, l, r, d, max_iter, tol, st);
+  return prefill_impl<bf16_t>(ctx, q, k, a_q, a_k, out, b, hq, hkv, l, r, d, max_iter, tol, st);
+}
+
+extern "C" int lrqk_als_prefill(lrqk_ctx* ctx, const void* q, const void* k, float* a_q, float* a_k, float* b_q,
+                                float* b_k, int b, int hq, int hkv, int64_t l, int r, int d, int max_iter, float tol,
+                                int dtype, void* stream) {
+  const PrefillOut out{a_q, a_k, b_q, b_k, l, l * r, false};
+  return prefill_checked(ctx, q, k, a_q, a_k, out, b, hq, hkv, l, r, d, max_iter, tol, dtype, stream);
+}
+
+extern "C" int lrqk_als_prefill_store(lrqk_ctx* ctx, const void* q, const void* k, float* a_q0, float* a_k0, void* a_q,
+                                      int64_t a_q_rows, void* a_k, int64_t a_k_stride, void* b_q, void* b_k, int b, int hq,
+                                      int hkv, int64_t l, int r, int d, int max_iter, float tol, int dtype, void* stream) {
+  const PrefillOut out{a_q, a_k, b_q, b_k, a_q_rows, a_k_stride, true};
+  return prefill_checked(ctx, q, k, a_q0, a_k0, out, b, hq, hkv, l, r, d, max_iter, tol, dtype, stream);
 }

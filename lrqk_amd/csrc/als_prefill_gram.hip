@@ -1,4 +1,4 @@
-// Prefill factorisation, iterations carried out on Gram matrices (bf16 input, d = 128, r <= 32).
+// Prefill factorisation, iterations carried out on Gram matrices (rows of 64 or 128 elements, r <= 64).
 //
 // After the first half-step of lrqk_attention.py:359-421 every factor is a linear image of its input,
 // A_Q = Q Mq and A_K = K Mk with Mq, Mk of size d x r.  Everything an iteration needs from the long axis
@@ -21,16 +21,13 @@
 // bf16 x bf16 products added in fp32 tile by tile and across tiles, then across splits in fp64.  Measured
 // against the fp64 restatement the results are closer than the same iteration in fp32 LAPACK.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "ctx.hpp"
+#include "prefill_pieces.hpp"
 
 namespace lrqk {
-
-typedef float gd_floatx16 __attribute__((ext_vector_type(16)));
-typedef __bf16 gd_bf16x8 __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ int gd_mfma_row(int lane, int v) { return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3); }
 
 // ----------------------------------------------------------------------------- X^T X
 // grid (S, x heads); 8 waves share the rows (128 per step, staged in LDS as they lie in memory); wave w owns
@@ -70,8 +67,6 @@ __global__ __launch_bounds__(kXtxThreads) void pf_xtx_kernel(const bf16_t* __res
   auto operand = [&](int row0, int nb) {
     const int s16 = lane & 15;
     const uint16_t* p = &x_s[(row0 + 8 * half + (s16 >> 2)) * kXtxLd + 32 * nb + (col & 16) + 4 * (s16 & 3)];
-    typedef short gd_v4s __attribute__((ext_vector_type(4)));
-    typedef gd_v4s __attribute__((address_space(3))) * gd_lds_v4s;
     const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
     const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 4 * kXtxLd));
     return __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -136,15 +131,6 @@ __global__ __launch_bounds__(kXtxThreads) void pf_xtx_kernel(const bf16_t* __res
 // through its heads' row groups one after the other, and their rows of A in flight together do not fit the
 // registers.  Requesting the rows of A a step ahead also made this kernel slower: 142 against 126 us at 32 heads
 // x 32K rows.)
-__device__ __forceinline__ void gd_split3(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = __float_as_uint(x) & 0xffff0000u;
-  const float r1 = x - __uint_as_float(hi);  // exact
-  mid = __float_as_uint(r1) & 0xffff0000u;
-  const float r2 = r1 - __uint_as_float(mid);  // exact, at most 8 significant bits
-  lo = __float_as_uint(r2) & 0xffff0000u;
-}
-__device__ __forceinline__ uint32_t gd_pack2(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xffff0000u); }
-
 __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __restrict__ X, int64_t l,
                                                               const float* __restrict__ A, int r,
                                                               float* __restrict__ part, float* __restrict__ xtx_part,
@@ -172,8 +158,6 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
   gd_floatx16 acc0, acc1, gAA, gAX[2];
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = gAA[v] = gAX[0][v] = gAX[1][v] = 0.0f;
-  typedef short gd_v4s __attribute__((ext_vector_type(4)));
-  typedef gd_v4s __attribute__((address_space(3))) * gd_lds_v4s;
   auto operand = [&](int row0, int nb) {  // rows row0 + 8 half .. + 7 of column 32 nb + col
     const int s16 = lane & 15;
     const uint16_t* p = &x_s[(row0 + 8 * half + (s16 >> 2)) * kXtxLd + 32 * nb + (col & 16) + 4 * (s16 & 3)];
@@ -326,10 +310,10 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
 // group (X times the three pieces), fp32 accuracy as in the row-by-row pass.  grid (S, kv heads); split s takes
 // the steps s, s + S, ...
 constexpr int kApLd = kXtxD + 8;  // bf16 elements per staged row: 16-byte operand reads want rows 4 banks apart
-template <int NH>
+template <int NH, typename OUT>
 __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16_t* __restrict__ X, int64_t l,
                                                                       const float* __restrict__ Mt, int r,
-                                                                      float* __restrict__ A, int S) {
+                                                                      OUT* __restrict__ A, int64_t a_stride, int S) {
   static_assert(NH == 2 || NH == 4, "query heads per kv head");
   extern __shared__ __align__(16) uint16_t ap_s[];
   uint16_t* x_s = ap_s;                          // [128][kApLd]
@@ -340,7 +324,7 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
   const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
   constexpr int WPH = kXtxWaves / NH, GPW = 4 / WPH;  // waves per head, row groups per wave and step
   const int hl = wave / WPH, g0 = (wave % WPH) * GPW;
-  float* Ah = A + ((int64_t)xh * NH + hl) * l * r;
+  OUT* Ah = A + ((int64_t)xh * NH + hl) * a_stride;
   for (int e = tid; e < NH * 32 * kXtxD; e += kXtxThreads) {
     const int hh = e / (32 * kXtxD), n = (e / kXtxD) % 32, k = e % kXtxD;
     const float v = n < r ? Mt[(((int64_t)xh * NH + hh) * r + n) * kXtxD + k] : 0.0f;
@@ -398,52 +382,58 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int64_t row = t0 + 32 * g + gd_mfma_row(lane, v);
-        if (row < l && col < r) Ah[row * r + col] = c[v];
+        if (row < l && col < r) gd_store(Ah, row * r + col, c[v]);
       }
     }
     __syncthreads();
   }
 }
 
-// A_K = K Mk for all query heads, reading K once per kv head.  Returns false if this grouping of heads has no
-// kernel here (the caller then runs its row-by-row pass).
-bool prefill_apply_shared(const void* k, const float* mt_k, float* a_k, int b, int hq, int hkv, int64_t l, int r,
-                          hipStream_t st, int* rc_out) {
-  *rc_out = LRQK_OK;
-  const int nh = hq / hkv, bkv = b * hkv;
-  if (nh != 2 && nh != 4) return false;
+template <typename OUT>
+static int apply_shared(const void* k, const float* mt_k, OUT* a_k, int64_t a_stride, int bkv, int nh, int64_t l, int r,
+                        hipStream_t st) {
   const int S = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + kXtxRows - 1) / kXtxRows));
   const size_t smem = (size_t)(kXtxRows + nh * 3 * 32) * kApLd * sizeof(uint16_t);
-  auto kern = nh == 2 ? pf_apply_shared_kernel<2> : pf_apply_shared_kernel<4>;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-  if (e != hipSuccess) {
-    *rc_out = set_error(LRQK_EHIP, "hipFuncSetAttribute failed: %s", hipGetErrorString(e));
-    return true;
-  }
+  auto kern = nh == 2 ? pf_apply_shared_kernel<2, OUT> : pf_apply_shared_kernel<4, OUT>;
+  LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)bkv), dim3(kXtxThreads), smem, st, (const bf16_t*)k, l, mt_k, r,
-                     a_k, S);
-  e = hipGetLastError();
-  if (e != hipSuccess) *rc_out = set_error(LRQK_EHIP, "launch failed: %s", hipGetErrorString(e));
-  return true;
+                     a_k, a_stride, S);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
 }
 
 // ----------------------------------------------------------------------------- d x d algebra, fp64
-constexpr int kGdThreads = 256;   // four waves: 32 of the 128 right-hand columns each (one wave per SIMD: 512 registers)
-constexpr int kGdD = 128;
-constexpr int kGdLd = 34;         // doubles per row of a transposed r x d matrix in LDS ([d][34], 16-byte rows)
-constexpr int kGdLg = 33;         // doubles per row of an r x r matrix in LDS
+// Everything below is templated on RT, the number of 16-row tiles that the rank is padded to (ranks up to 16, 32, 64:
+// RT = 1, 2, 4), and on the row width D (64 or 128); RP = 16 RT is the padded rank.  Padding costs the matrix cores'
+// time (a solve has RP / 4 dependent steps), so a rank of 16 does not run as 32 (28 against 51 us per
+// iteration at D = 128, 32 heads; RT = 4: 132 us).
+constexpr int kGdThreads = 256;   // four waves: D / 4 right-hand columns each (one wave per SIMD: 512 registers)
+template <int RT, int D>
+struct GdShape {
+  static constexpr int RP = 16 * RT;
+  static constexpr int CT = D / 64;       // 16-column tiles of a right-hand side per wave
+  static constexpr int LD = RP + 2;       // doubles per row of a transposed r x d matrix in LDS ([D][LD], 16-byte rows)
+  static constexpr int LG = RP + 1;       // doubles per row of an r x r matrix
+  // RT = 4: three D x LD matrices do not fit the LDS, so B shares its block with T / U (each is dead when the other is
+  // formed) and the r x r matrices lie in global memory (they stay in the L2)
+  static constexpr bool WIDE = RT == 4;
+  static constexpr int PIV = WIDE ? 2 * 2 * RP * 4 + (kGdThreads / 64) * 32 : (kGdThreads / 64) * (2 * RP * 4 + 32);
+  static constexpr size_t SMEM = ((size_t)(WIDE ? 2 : 3) * D * LD + (WIDE ? 0 : 3 * RP * LG) + PIV + 8) * sizeof(double);
+};
 
-// ---- two systems [W | RHS] (W 32 x 32 symmetric positive definite up to rounding, rows/columns beyond r the
-// identity; RHS 32 x 128) solved side by side by block Gauss-Jordan elimination on the fp64 matrix cores, four
+// ---- two systems [W | RHS] (W RP x RP symmetric positive definite up to rounding, rows/columns beyond r the
+// identity; RHS RP x D) solved side by side by block Gauss-Jordan elimination on the fp64 matrix cores, four
 // pivots per step.  The matrices live in the accumulator layout of 16 x 16 tiles (element v of lane l = row
-// 16 rt + l / 16 + 4 v, column 16 u + l % 16 of tile (rt, u)): each of the four waves holds W itself (every wave
-// eliminates its own copy: no wave waits for another, the solve has no barrier) and 32 columns of RHS.
-// Step m, with P the pivot columns 4 m .. 4 m + 3 (32 x 4) and D its rows 4 m .. 4 m + 3:
+// 16 rt + l / 16 + 4 v, column 16 u + l % 16 of tile (rt, u)).  Up to RT = 2 each of the four waves holds W itself
+// (every wave eliminates its own copy: no wave waits for another, the solve has no barrier) and D / 4 columns of RHS;
+// RT = 4 would need 256 registers for the copies and most of the products for work done four times over, so there
+// wave w holds column tile w of W and the pivot columns go round through LDS, one barrier per step.
+// Step m, with P the pivot columns 4 m .. 4 m + 3 (RP x 4) and D its rows 4 m .. 4 m + 3:
 //     X <- X - (P D^-1) X[4 m .. 4 m + 3, :] outside the pivot rows,   X[pivot rows] <- D^-1 X[pivot rows]
 // (one product: the pivot rows' accumulators are cleared and their left operand is D^-1 itself), which clears the
 // pivot columns elsewhere.  The right-hand
 // operand, four rows of X, is element m % 4 of the lane's own tile in row tile m / 4: no data moves for it.  The
-// left operand needs P by rows: the lanes that hold the pivot columns put them into the wave's own LDS slot, the
+// left operand needs P by rows: the lanes that hold the pivot columns put them into the LDS slot, the
 // two pivot blocks are inverted side by side in the two halves of the wave (by 2 x 2 blocks, no pivoting) and
 // handed round through the same slot.  The products on W come first (the next step waits for them only); those on
 // RHS run on the matrix cores while the next step's inverse is computed.
@@ -494,35 +484,44 @@ __device__ __forceinline__ void gd_inv4(const double (&D)[4][4], double (&R)[4][
   R[2][2] = t00; R[2][3] = t01; R[3][2] = t10; R[3][3] = t11;
 }
 
+template <int RT, int CT>
 struct GdSys {
-  gd_v4d w[2][2];  // W: [row tile][column tile]
-  gd_v4d x[2][2];  // this wave's columns of RHS: [row tile][column tile 2 wave + u]
+  static constexpr int WC = RT == 4 ? 1 : RT;  // column tiles of W that a wave holds (all of them, or tile `wave`)
+  gd_v4d w[RT][WC];  // W: [row tile][column tile]
+  gd_v4d x[RT][CT];  // this wave's columns of RHS: [row tile][column tile CT wave + u]
 };
-constexpr int kGdSlot = 2 * 128 + 32;                    // per wave: P of both systems, the two inverses
-constexpr int kGdPivDoubles = (kGdThreads / 64) * kGdSlot;
-__device__ __forceinline__ void gd_solve_pair(GdSys (&s)[2], double* __restrict__ piv) {
+template <int RT, int CT>
+__device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT> (&s)[2], double* __restrict__ piv) {
+  constexpr int RP = 16 * RT;
+  constexpr bool WIDE = RT == 4;
   const int lane = lane_id(), wave = wave_id();
   const int li = lane & 15, lk = lane >> 4;
-  double* pb = piv + wave * kGdSlot;
-  double* xch = pb + 256;
+  // P of both systems: the wave's own slot, or (WIDE) one of two slots that all waves read
+  double* own = piv + wave * (2 * RP * 4 + 32);
+  double* xch = WIDE ? piv + 2 * 2 * RP * 4 + wave * 32 : own + 2 * RP * 4;
 #pragma unroll
-  for (int m = 0; m < 8; ++m) {
+  for (int m = 0; m < 4 * RT; ++m) {
     const int tp = m >> 2, vp = m & 3;  // the pivots' tile (row tile of the pivot rows, column tile of W) and element
+    double* pb = WIDE ? piv + (m & 1) * 2 * RP * 4 : own;
     {
       const int kk = li - 4 * vp;
-      if (kk >= 0 && kk < 4) {
+      if ((!WIDE || wave == tp) && kk >= 0 && kk < 4) {
 #pragma unroll
         for (int sy = 0; sy < 2; ++sy)
 #pragma unroll
-          for (int rt = 0; rt < 2; ++rt)
+          for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) pb[sy * 128 + (16 * rt + lk + 4 * v) * 4 + kk] = s[sy].w[rt][tp][v];
+            for (int v = 0; v < 4; ++v) pb[sy * RP * 4 + (16 * rt + lk + 4 * v) * 4 + kk] = s[sy].w[rt][WIDE ? 0 : tp][v];
       }
     }
-    gd_wave_sync();
+    // (two slots: a wave that passes this barrier has read the slot of step m - 2, which step m wrote over)
+    if constexpr (WIDE)
+      __syncthreads();
+    else
+      gd_wave_sync();
     {
       const int mine = lane >> 5;
-      const double* P = pb + mine * 128;
+      const double* P = pb + mine * RP * 4;
       double D[4][4], R[4][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -540,24 +539,24 @@ __device__ __forceinline__ void gd_solve_pair(GdSys (&s)[2], double* __restrict_
       }
       gd_wave_sync();
     }
-    double aop[2][2];
+    double aop[2][RT];
 #pragma unroll
     for (int sy = 0; sy < 2; ++sy) {
-      const double* P = pb + sy * 128;
+      const double* P = pb + sy * RP * 4;
       double ic[4];  // column l / 16 of the inverse
 #pragma unroll
       for (int k = 0; k < 4; ++k) ic[k] = xch[sy * 16 + k * 4 + lk];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
+      for (int rt = 0; rt < RT; ++rt) {
         const int row = 16 * rt + li;
         const double2 lo = *reinterpret_cast<const double2*>(&P[row * 4]);
         const double2 hi = *reinterpret_cast<const double2*>(&P[row * 4 + 2]);
         // pivot rows: the rows of D^-1 themselves (their accumulators are cleared below, so they come out as
         // D^-1 X and not as X - (I - D^-1) X, which cancels in its leading digits when D is far from unit size:
         // with a diagonal of 1e12 solutions were off by 5e-3 where the conditioning allowed 1e-11)
-        const double own = xch[sy * 16 + (row & 3) * 4 + lk];
+        const double mine = xch[sy * 16 + (row & 3) * 4 + lk];
         const double oth = -fma(lo.x, ic[0], fma(lo.y, ic[1], fma(hi.x, ic[2], hi.y * ic[3])));
-        aop[sy][rt] = (row >> 2) == m ? own : oth;
+        aop[sy][rt] = (row >> 2) == m ? mine : oth;
       }
     }
     gd_wave_sync();  // (the reads of the slot precede the next step's writes)
@@ -565,115 +564,123 @@ __device__ __forceinline__ void gd_solve_pair(GdSys (&s)[2], double* __restrict_
 #pragma unroll
     for (int sy = 0; sy < 2; ++sy)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        if (u < tp) continue;
+      for (int u = 0; u < GdSys<RT, CT>::WC; ++u) {
+        if (WIDE ? wave < tp : u < tp) continue;  // (wave-uniform)
         const double bop = s[sy].w[tp][u][vp];
         s[sy].w[tp][u][vp] = 0.0;
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           s[sy].w[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[sy][rt], bop, s[sy].w[rt][u], 0, 0, 0);
       }
 #pragma unroll
     for (int sy = 0; sy < 2; ++sy)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < CT; ++u) {
         const double bop = s[sy].x[tp][u][vp];
         s[sy].x[tp][u][vp] = 0.0;
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
           s[sy].x[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[sy][rt], bop, s[sy].x[rt][u], 0, 0, 0);
       }
   }
+  if constexpr (WIDE) __syncthreads();  // (the next solve starts with slot 0 again)
 }
 
 // One system filled from fw(row, column of W) and fx(row, column of RHS) / its solution handed to g(row, column
 // of RHS, value).
-template <typename FW, typename FX>
-__device__ __forceinline__ void gd_fill(GdSys& t, FW&& fw, FX&& fx) {
+template <int RT, int CT, typename FW, typename FX>
+__device__ __forceinline__ void gd_fill(GdSys<RT, CT>& t, FW&& fw, FX&& fx) {
   const int lane = lane_id(), wave = wave_id();
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * rt + (lane >> 4) + 4 * v;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 16 * rt + (lane >> 4) + 4 * v;
-        t.w[rt][u][v] = fw(i, 16 * u + (lane & 15));
-        t.x[rt][u][v] = fx(i, 16 * (2 * wave + u) + (lane & 15));
-      }
+      for (int u = 0; u < GdSys<RT, CT>::WC; ++u) t.w[rt][u][v] = fw(i, 16 * (RT == 4 ? wave : u) + (lane & 15));
+#pragma unroll
+      for (int u = 0; u < CT; ++u) t.x[rt][u][v] = fx(i, 16 * (CT * wave + u) + (lane & 15));
+    }
 }
-template <typename G>
-__device__ __forceinline__ void gd_drain(const gd_v4d (&x)[2][2], G&& g) {
+template <int RT, int CT, typename G>
+__device__ __forceinline__ void gd_drain(const gd_v4d (&x)[RT][CT], G&& g) {
   const int lane = lane_id(), wave = wave_id();
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < CT; ++u)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) g(16 * rt + (lane >> 4) + 4 * v, 16 * (2 * wave + u) + (lane & 15), x[rt][u][v]);
+      for (int v = 0; v < 4; ++v) g(16 * rt + (lane >> 4) + 4 * v, 16 * (CT * wave + u) + (lane & 15), x[rt][u][v]);
 }
 
-// out[i][j] = sum over c < 128 of PT[c][i] * RT[c][j]   (two r x d matrices, stored transposed) on the fp64 matrix
-// cores, by waves 0..3: wave w owns the 16 x 16 tile (w / 2, w % 2) and runs its 32 products of depth 4 in a row.
-// Element v of a thread is out[gd_outer_row(v)][gd_outer_col()].  Rows/columns beyond r come out as what the zero
-// padding of PT, RT gives.
-__device__ __forceinline__ int gd_outer_row(int v) { return 16 * (wave_id() >> 1) + (lane_id() >> 4) + 4 * v; }
-__device__ __forceinline__ int gd_outer_col() { return 16 * (wave_id() & 1) + (lane_id() & 15); }
-__device__ __forceinline__ void gd_outer(const double* __restrict__ PT, const double* __restrict__ RT, double (&o)[4]) {
-  o[0] = o[1] = o[2] = o[3] = 0.0;
-  if (threadIdx.x < 256) {
-    const int lane = lane_id(), wave = wave_id();
-    const int li = lane & 15, lk = lane >> 4;
-    const double* pa = PT + lk * kGdLd + 16 * (wave >> 1) + li;
-    const double* pb = RT + lk * kGdLd + 16 * (wave & 1) + li;
-    gd_v4d acc = gd_v4d{0.0, 0.0, 0.0, 0.0};
+// f(i, j, sum over c < D of PT[c][i] * RT_[c][j])   (two r x d matrices, stored transposed) on the fp64 matrix
+// cores: RT x RT tiles of 16 x 16, D / 4 products of depth 4 in a row each; wave w owns tile row w (RT = 4), one tile
+// (RT = 2), and wave 0 the only tile of RT = 1.  Rows/columns beyond r come out as what the zero padding gives.
+template <int RT, int D, typename F>
+__device__ __forceinline__ void gd_outer(const double* __restrict__ PT, const double* __restrict__ QT, F&& f) {
+  constexpr int LD = GdShape<RT, D>::LD;
+  constexpr int NC = RT == 4 ? 4 : 1;  // column tiles per wave
+  const int lane = lane_id(), wave = wave_id();
+  if (RT == 1 && wave > 0) return;
+  const int li = lane & 15, lk = lane >> 4;
+  const int tr = RT == 4 ? wave : RT == 2 ? wave >> 1 : 0, tc = RT == 2 ? wave & 1 : 0;
+  const double* pa = PT + lk * LD + 16 * tr + li;
+  const double* pb = QT + lk * LD + 16 * tc + li;
+  gd_v4d acc[NC];
+#pragma unroll
+  for (int n = 0; n < NC; ++n) acc[n] = gd_v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll 8
-    for (int c = 0; c < kGdD; c += 4)
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(pa[c * kGdLd], pb[c * kGdLd], acc, 0, 0, 0);
+  for (int c = 0; c < D; c += 4) {
+    const double a = pa[c * LD];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) o[v] = acc[v];
+    for (int n = 0; n < NC; ++n) acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, pb[c * LD + 16 * n], acc[n], 0, 0, 0);
   }
+#pragma unroll
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) f(16 * tr + lk + 4 * v, 16 * (tc + n) + li, acc[n][v]);
 }
 
-// TT[c][i] = sum over k of MT[k][i] * S[k][c]   (the transposed form of Mt S, S symmetric d x d in global
+// TT[c][i] = sum over k of MT[k][i] * S[k][c]   (the transposed form of Mt S, S symmetric D x D in global
 // memory) on the fp64 matrix cores: 16 x 16 x 4 tiles, A operand lane l = Mt[i0 + l % 16][k0 + l / 16] (from the
-// LDS copy), B operand lane l = S[k0 + l / 16][c0 + l % 16] (16 independent loads per lane in flight), result
-// element v of lane l = row l / 16 + 4 v, column l % 16 of the tile.  Waves 0..3 take 32 columns each.
+// LDS copy), B operand lane l = S[k0 + l / 16][c0 + l % 16] (8 CT independent loads per lane in flight), result
+// element v of lane l = row l / 16 + 4 v, column l % 16 of the tile.  Each wave takes D / 4 columns.
 // One barrier.
+template <int RT, int D>
 __device__ __forceinline__ void gd_times_s(const double* __restrict__ MT, const double* __restrict__ S,
                                            double* __restrict__ TT) {
+  constexpr int LD = GdShape<RT, D>::LD, CT = GdShape<RT, D>::CT;
   const int lane = lane_id(), wave = wave_id();
-  if (wave < 4) {
-    const int li = lane & 15, lk = lane >> 4;
-    const int c0 = 32 * wave;
-    gd_v4d acc[2][2];
+  const int li = lane & 15, lk = lane >> 4;
+  const int c0 = 16 * CT * wave;
+  gd_v4d acc[RT][CT];
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = gd_v4d{0.0, 0.0, 0.0, 0.0};
-    for (int kb = 0; kb < kGdD; kb += 32) {
-      double bv[8][2];
+    for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = gd_v4d{0.0, 0.0, 0.0, 0.0};
+  for (int kb = 0; kb < D; kb += 32) {
+    double bv[8][CT];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+    for (int u = 0; u < 8; ++u)
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct) bv[u][ct] = S[(int64_t)(kb + 4 * u + lk) * kGdD + c0 + 16 * ct + li];
+      for (int ct = 0; ct < CT; ++ct) bv[u][ct] = S[(int64_t)(kb + 4 * u + lk) * D + c0 + 16 * ct + li];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int k = kb + 4 * u + lk;
-        const double a0 = MT[k * kGdLd + li], a1 = MT[k * kGdLd + 16 + li];
-        acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bv[u][0], acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bv[u][1], acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bv[u][0], acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bv[u][1], acc[1][1], 0, 0, 0);
+    for (int u = 0; u < 8; ++u) {
+      const int k = kb + 4 * u + lk;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        const double a = MT[k * LD + 16 * rt + li];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv[u][ct], acc[rt][ct], 0, 0, 0);
       }
     }
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) TT[(c0 + 16 * ct + li) * kGdLd + 16 * rt + lk + 4 * v] = acc[rt][ct][v];
   }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) TT[(c0 + 16 * ct + li) * LD + 16 * rt + lk + 4 * v] = acc[rt][ct][v];
   __syncthreads();
 }
 
@@ -696,15 +703,17 @@ struct GdArgs {
   int S_k;              // splits of partK
   const double* Sq;     // [bh][d][d]
   const double* Sk;     // [b * hkv][d][d]
-  double* G;            // [2][bh][32][32]  (side 0: Q, 1: K), padded with the identity
-  double* C;            // [2][bh][32][d]   zero rows beyond r
-  double* BqT;          // [bh][d][32]      B_Q of the state, transposed (written by an iteration for the next)
+  double* G;            // [2][bh][RP][RP]  (side 0: Q, 1: K), padded with the identity
+  double* C;            // [2][bh][RP][d]   zero rows beyond r
+  double* BqT;          // [bh][RP][d]      B_Q of the state (written by an iteration for the next)
+  double* Gs;           // [bh][2][RP][RP + 1]  RT = 4 only: the r x r matrices of an iteration
   double* delta;        // [iters][2][bh]   squared changes |A - A'|^2 per head
   int* flags;           // [iters + 1]
-  float* Mt_q;          // [bh][r][d]  Mq^T, Mk^T for the final row-by-row pass
+  float* Mt_q;          // [bh][r][d]  Mq^T, Mk^T for the final pass over the rows
   float* Mt_k;
-  float* b_q;           // [bh][r][d] outputs
-  float* b_k;
+  void* b_q;            // [bh][r][d] outputs, bf16 or fp32
+  void* b_k;
+  int out_bf16;
   int bh, hq, hkv, r;
   int64_t l;
   float tol;
@@ -715,12 +724,14 @@ struct GdArgs {
 //   blocks [nq, nq + nk)  Sk likewise over the bkv distinct K heads
 //   the rest              the state (G, C) of both sides from the first Gram passes: S partial sums of [G | C]
 //                         packed as [r][r + d] floats per head; G padded with the identity, C with zero rows
-//                         (20 blocks per head and side).
-constexpr int kGdInitBlocks = (32 * (32 + kGdD) + 255) / 256;
+//                         (RP (RP + d) / 256 blocks per head and side).
+template <int RP, int D>
 __global__ __launch_bounds__(256) void pf_gramdom_init_kernel(GdArgs a, const float* __restrict__ xq_part, int Sx,
                                                               const float* __restrict__ xk_part, int Sxk, int bkv,
                                                               double* __restrict__ Sq, double* __restrict__ Sk) {
-  constexpr int dd = kGdD * kGdD, per = dd / 256;
+  constexpr int dd = D * D, per = dd / 256;
+  constexpr int kBlocks = RP * (RP + D) / 256;
+  static_assert(RP * (RP + D) % 256 == 0 && dd % 256 == 0, "whole blocks");
   int blk = blockIdx.x;
   const int nq = a.bh * per, nk = bkv * per;
   if (blk < nq + nk) {
@@ -736,72 +747,86 @@ __global__ __launch_bounds__(256) void pf_gramdom_init_kernel(GdArgs a, const fl
     return;
   }
   blk -= nq + nk;
-  const int h = blk / (2 * kGdInitBlocks), side = (blk / kGdInitBlocks) & 1;
-  const int r = a.r, d = kGdD;
-  const int e = (blk % kGdInitBlocks) * 256 + threadIdx.x;
-  if (e >= 32 * (32 + d)) return;
-  const int ne = r * (r + d);
+  const int h = blk / (2 * kBlocks), side = (blk / kBlocks) & 1;
+  const int r = a.r;
+  const int e = (blk % kBlocks) * 256 + threadIdx.x;
+  const int ne = r * (r + D);
   const int Sn = side ? a.S_k : a.S;
   const float* part = (side ? a.partK : a.partQ) + (int64_t)h * Sn * ne;
-  const int i = e / (32 + d), j = e % (32 + d);
+  const int i = e / (RP + D), j = e % (RP + D);
   double v = 0.0;
-  if (i < r && (j >= 32 || j < r)) {
-    const int src = i * (r + d) + (j < 32 ? j : r + (j - 32));
+  if (i < r && (j >= RP || j < r)) {
+    const int src = i * (r + D) + (j < RP ? j : r + (j - RP));
+#pragma unroll 4
     for (int s = 0; s < Sn; ++s) v += (double)part[(int64_t)s * ne + src];
-  } else if (j < 32) {
+  } else if (j < RP) {
     v = i == j ? 1.0 : 0.0;
   }
-  if (j < 32)
-    a.G[((int64_t)side * a.bh + h) * 1024 + i * 32 + j] = v;
+  if (j < RP)
+    a.G[((int64_t)side * a.bh + h) * RP * RP + i * RP + j] = v;
   else
-    a.C[((int64_t)side * a.bh + h) * 32 * d + i * d + (j - 32)] = v;
+    a.C[((int64_t)side * a.bh + h) * RP * D + i * D + (j - RP)] = v;
 }
 
-// stage 0: one iteration `it`; stage 2: the final B_Q, B_K from the state.
-__global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int stage, int it, GdArgs a) {
+// What a launch of pf_gramdom_kernel does: a whole iteration `it`; the final B_Q, B_K from the state after `it`
+// iterations; or a part of an iteration: the first B_Q, the Q side's step, the K side's step.
+// RT = 4 runs in parts: with the systems of a whole iteration in one launch the compiler spills 280 registers, and a
+// launch more is 2 us where a step takes 50.
+enum GdPart { kGdWhole, kGdFinal, kGdStart, kGdQSide, kGdKSide };
+template <int RT, int D, int PART>
+__global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a) {
+  using Sh = GdShape<RT, D>;
+  constexpr int RP = Sh::RP, CT = Sh::CT, LD = Sh::LD, LG = Sh::LG, d = D;
   extern __shared__ __align__(16) double gsm[];
-  double* MT = gsm;                         // [128][34]  Mq'^T, later Mk'^T (transposed storage)
-  double* TT = MT + kGdD * kGdLd;           // [128][34]  T, later U
-  double* BT = TT + kGdD * kGdLd;           // [128][34]  B_Q, later B_K
-  double* Gs = BT + kGdD * kGdLd;           // [3][32][33]
-  double* piv = Gs + 3 * 32 * kGdLg;        // [2 buffers][2 systems][32][4]
-  double* red = piv + kGdPivDoubles;        // [8]
+  double* MT = gsm;                         // [D][LD]  Mq'^T, later Mk'^T (transposed storage)
+  double* TT = MT + D * LD;                 // [D][LD]  T, later U
+  double* BT = Sh::WIDE ? TT : TT + D * LD; // [D][LD]  B_Q, later B_K
+  double* piv = BT + D * LD;                // the solves' slots
+  double* red = piv + Sh::PIV;              // [8]
   const int tid = threadIdx.x;
   const int h = blockIdx.x;
-  const int r = a.r, d = kGdD, bh = a.bh;
+  const int r = a.r, bh = a.bh;
+  double* Gs = Sh::WIDE ? a.Gs + (int64_t)h * 2 * RP * LG : red + 8;  // [2 or 3][RP][LG]
   const int b = h / a.hq, kvh = (h % a.hq) / (a.hq / a.hkv);
   const double* Sq = a.Sq + (int64_t)h * d * d;
   const double* Sk = a.Sk + ((int64_t)b * a.hkv + kvh) * d * d;
-  double* Gq = a.G + (int64_t)h * 1024;
-  double* Gk = a.G + ((int64_t)bh + h) * 1024;
-  double* Cq = a.C + (int64_t)h * 32 * d;
-  double* Ck = a.C + ((int64_t)bh + h) * 32 * d;
+  double* Gq = a.G + (int64_t)h * RP * RP;
+  double* Gk = a.G + ((int64_t)bh + h) * RP * RP;
+  double* Cq = a.C + (int64_t)h * RP * d;
+  double* Ck = a.C + ((int64_t)bh + h) * RP * d;
 
   // ---- what an iteration reads of its state is requested before anything else: the handed-over B_Q and this
-  // wave's tiles of Ck and Cq (Cq is rewritten only at the end of the Q side's step, Ck at the end of the iteration)
-  const bool fresh = stage == 2 || it == 0;
-  constexpr int kBqPer = 32 * kGdD / kGdThreads;
-  double bq_pre[kBqPer];
-  gd_v4d ckt[2][2], cqt[2][2];
-  if (!fresh) {
-    const double* src = a.BqT + (int64_t)h * 32 * d;  // [32][d]
+  // wave's tiles of Ck and Cq (Cq is rewritten only at the end of the Q side's step, Ck at the end of the iteration).
+  // (In parts, C is read where it is used, and B_K goes from the Q side's step to the K side's in the block of the
+  // handed-over B_Q: each lane reads back what it wrote.)
+  constexpr bool FINAL = PART == kGdFinal, kHold = PART == kGdWhole;
+  static_assert(FINAL || kHold != Sh::WIDE, "RT = 4 in parts, the others whole");
+  const bool fresh = FINAL || PART == kGdStart || (kHold && it == 0);
+  constexpr int kBqPer = RP * D / kGdThreads;
+  double bq_pre[kHold ? kBqPer : 1];
+  gd_v4d ckt[kHold ? RT : 1][CT], cqt[kHold ? RT : 1][CT];
+  if (kHold && !fresh) {
+    const double* src = a.BqT + (int64_t)h * RP * d;  // [RP][d]
 #pragma unroll
-    for (int u = 0; u < kBqPer; ++u) bq_pre[u] = src[tid + u * kGdThreads];
+    for (int u = 0; u < (kHold ? kBqPer : 1); ++u) bq_pre[u] = src[tid + u * kGdThreads];
   }
-  if (stage == 0) {
+  if constexpr (kHold) {
     const int lane = lane_id(), wave = wave_id();
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < CT; ++u)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int e = (16 * rt + (lane >> 4) + 4 * v) * d + 16 * (2 * wave + u) + (lane & 15);
+          const int e = (16 * rt + (lane >> 4) + 4 * v) * d + 16 * (CT * wave + u) + (lane & 15);
           ckt[rt][u][v] = Ck[e];
           cqt[rt][u][v] = Cq[e];
         }
   }
-  if (stage == 0) {
+  if constexpr (PART == kGdKSide) {
+    if (a.flags[it]) return;
+  }
+  if constexpr (PART == kGdWhole || PART == kGdQSide) {
     // ---- the stopping test of the previous iteration (batch-wide, as the reference takes it)
     int done = 0;
     if (it > 0) {
@@ -827,121 +852,133 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int stage, int i
   // Of an iteration's r x r systems only two follow each other: B_K = Gk^-1 Ck does not depend on the Q side's
   // step and is solved beside it, and the next iteration's B_Q = Gq'^-1 Cq' is solved beside the K side's step
   // and handed over in `BqT`.  Iteration 0 (and the final stage) start from the state alone: B_Q and B_K side by side.
-  GdSys sy[2];
-  gd_v4d bk[2][2];  // B_K in the layout of the right-hand sides
-  double* BqT = a.BqT + (int64_t)h * 32 * d;  // [32][d]
+  GdSys<RT, CT> sy[2];
+  gd_v4d bk[kHold ? RT : 1][CT];  // B_K in the layout of the right-hand sides
+  double* BqT = a.BqT + (int64_t)h * RP * d;  // [RP][d]
+  if constexpr (PART != kGdQSide && PART != kGdKSide) {
   if (fresh) {
-    gd_fill(sy[0], [&](int i, int j) { return Gq[i * 32 + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
-    if (stage == 2)
-      gd_fill(sy[1], [&](int i, int j) { return Gk[i * 32 + j]; }, [&](int i, int cc) { return Ck[i * d + cc]; });
+    gd_fill(sy[0], [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
+    if constexpr (FINAL)
+      gd_fill(sy[1], [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return Ck[i * d + cc]; });
     else
       gd_fill(sy[1], [&](int i, int j) { return i == j ? 1.0 : 0.0; }, [&](int, int) { return 0.0; });
     gd_solve_pair(sy, piv);
-    if (stage == 2) {
-      float* oq = a.b_q + (int64_t)h * r * d;
-      float* ok = a.b_k + (int64_t)h * r * d;
-      gd_drain(sy[0].x, [&](int i, int cc, double v) { if (i < r) oq[i * d + cc] = (float)v; });
-      gd_drain(sy[1].x, [&](int i, int cc, double v) { if (i < r) ok[i * d + cc] = (float)v; });
+    if constexpr (FINAL) {
+      const int64_t o = (int64_t)h * r * d;
+      auto put = [&](void* dst, int i, int cc, double v) {
+        if (i >= r) return;
+        if (a.out_bf16)
+          st_f32<bf16_t>((bf16_t*)dst, o + i * d + cc, (float)v);
+        else
+          ((float*)dst)[o + i * d + cc] = (float)v;
+      };
+      gd_drain(sy[0].x, [&](int i, int cc, double v) { put(a.b_q, i, cc, v); });
+      gd_drain(sy[1].x, [&](int i, int cc, double v) { put(a.b_k, i, cc, v); });
       return;
     }
-    gd_drain(sy[0].x, [&](int i, int cc, double v) { BT[cc * kGdLd + i] = v; });
-  } else {
+    if constexpr (PART == kGdStart) {
+      gd_drain(sy[0].x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+      return;
+    }
+    gd_drain(sy[0].x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
+  } else if constexpr (kHold) {
 #pragma unroll
     for (int u = 0; u < kBqPer; ++u) {
       const int e = tid + u * kGdThreads;
-      BT[(e % d) * kGdLd + e / d] = bq_pre[u];
+      BT[(e % d) * LD + e / d] = bq_pre[u];
     }
   }
+  }
+  if constexpr (PART == kGdQSide) {
+#pragma unroll 8
+    for (int e = tid; e < RP * d; e += kGdThreads) BT[(e % d) * LD + e / d] = BqT[e];
+  }
+  if constexpr (PART == kGdWhole || PART == kGdQSide) {
   __syncthreads();
   // ---- W1 = Gk + B_Q B_Q^T
-  {
-    double o[4];
-    gd_outer(BT, BT, o);
-    const int j = gd_outer_col();
-#pragma unroll
-    for (int u = 0; u < 4; ++u) Gs[gd_outer_row(u) * kGdLg + j] = Gk[gd_outer_row(u) * 32 + j] + o[u];
-  }
+  gd_outer<RT, D>(BT, BT, [&](int i, int j, double o) { Gs[i * LG + j] = Gk[i * RP + j] + o; });
   __syncthreads();
   // ---- Mq'^T = W1^-1 (Ck + B_Q) beside B_K = Gk^-1 Ck
-  gd_fill(sy[0], [&](int i, int j) { return Gs[i * kGdLg + j]; }, [&](int i, int cc) { return BT[cc * kGdLd + i]; });
-  gd_fill(sy[1], [&](int i, int j) { return Gk[i * 32 + j]; }, [&](int, int) { return 0.0; });
+  gd_fill(sy[0], [&](int i, int j) { return Gs[i * LG + j]; }, [&](int i, int cc) { return BT[cc * LD + i]; });
+  gd_fill(sy[1], [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return kHold ? 0.0 : Ck[i * d + cc]; });
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      sy[0].x[rt][u] += ckt[rt][u];
-      sy[1].x[rt][u] = ckt[rt][u];
+    for (int u = 0; u < CT; ++u) {
+      if constexpr (kHold) sy[1].x[rt][u] = ckt[rt][u];
+      sy[0].x[rt][u] += sy[1].x[rt][u];
     }
   __syncthreads();  // (every read of B_Q precedes the rewriting of the B tile below)
   gd_solve_pair(sy, piv);
+  if constexpr (kHold) {
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) bk[rt][u] = sy[1].x[rt][u];
+      for (int u = 0; u < CT; ++u) bk[rt][u] = sy[1].x[rt][u];
+  } else {
+    gd_drain(sy[1].x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+  }
   // ---- the B tile now holds B_K; Mq'^T goes to its tile and to the caller, with the sum of Cq (the old one) . Mq'^T
-  gd_drain(bk, [&](int i, int cc, double v) { BT[cc * kGdLd + i] = v; });
+  gd_drain(sy[1].x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
   double part_q = 0.0;
   {
     float* mt = a.Mt_q + (int64_t)h * r * d;
     gd_drain(sy[0].x, [&](int i, int cc, double v) {
-      MT[cc * kGdLd + i] = v;
+      MT[cc * LD + i] = v;
       if (i < r) mt[i * d + cc] = (float)v;
+      if constexpr (!kHold) part_q = fma(Cq[i * d + cc], v, part_q);
     });
+    if constexpr (kHold) {
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < CT; ++u)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) part_q = fma(cqt[rt][u][v], sy[0].x[rt][u][v], part_q);
+          for (int v = 0; v < 4; ++v) part_q = fma(cqt[rt][u][v], sy[0].x[rt][u][v], part_q);
+    }
   }
   double tr_old = 0.0;
-  if (tid < 32) tr_old = tid < r ? Gq[tid * 32 + tid] : 0.0;
+  if (tid < RP) tr_old = tid < r ? Gq[tid * RP + tid] : 0.0;
   __syncthreads();
-  {
-    double o[4];
-    gd_outer(BT, BT, o);
-    if (tid < 256) {
-      const int j = gd_outer_col();
-#pragma unroll
-      for (int u = 0; u < 4; ++u) Gs[32 * kGdLg + gd_outer_row(u) * kGdLg + j] = o[u];
-    }
-  }
+  gd_outer<RT, D>(BT, BT, [&](int i, int j, double o) { Gs[RP * LG + i * LG + j] = o; });
+  if constexpr (Sh::WIDE) __syncthreads();  // (T is formed in the block that holds B_K)
   // ---- T = Mq'^T Sq, Gq' = Mq'^T T^T
-  gd_times_s(MT, Sq, TT);
+  gd_times_s<RT, D>(MT, Sq, TT);
   {
-    double o[4];
-    gd_outer(MT, TT, o);
     double tr_new = 0.0;
-    if (tid < 256) {
-      const int j = gd_outer_col();
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = gd_outer_row(u);
-        const double v = (i < r && j < r) ? o[u] : (i == j ? 1.0 : 0.0);
-        Gs[2 * 32 * kGdLg + i * kGdLg + j] = v;
-        Gq[i * 32 + j] = v;
-        if (i == j && i < r) tr_new += v;
-      }
-    }
+    gd_outer<RT, D>(MT, TT, [&](int i, int j, double o) {
+      const double v = (i < r && j < r) ? o : (i == j ? 1.0 : 0.0);
+      if constexpr (kHold) Gs[2 * RP * LG + i * LG + j] = v;
+      Gq[i * RP + j] = v;
+      if (i == j && i < r) tr_new += v;
+    });
     const double dq = gd_block_sum(tr_old - 2.0 * part_q + tr_new, red);
     if (tid == 0) a.delta[((int64_t)it * 2 + 0) * bh + h] = dq;
   }
   // Cq' = T (rows beyond r stay zero: Mq'^T has zero rows there)
-  if (tid < d) {
-#pragma unroll
-    for (int i = 0; i < 32; ++i) Cq[i * d + tid] = TT[tid * kGdLd + i];
+#pragma unroll 8
+  for (int e = tid; e < RP * d; e += kGdThreads) Cq[e] = TT[(e % d) * LD + e / d];
   }
+  if constexpr (PART == kGdWhole || PART == kGdKSide) {
   // ---- Mk'^T = (Gq' + B_K B_K^T)^-1 (T + B_K) beside the next B_Q = Gq'^-1 T
   {
-    const double* Gn = Gs + 2 * 32 * kGdLg;
-    const double* Gb = Gs + 32 * kGdLg;
-    gd_fill(sy[0], [&](int i, int j) { return Gn[i * kGdLg + j]; }, [&](int i, int cc) { return TT[cc * kGdLd + i]; });
-    gd_fill(sy[1], [&](int i, int j) { return Gn[i * kGdLg + j] + Gb[i * kGdLg + j]; },
-            [&](int i, int cc) { return TT[cc * kGdLd + i]; });
+    const double* Gb = Gs + RP * LG;
+    if constexpr (kHold) {
+      const double* Gn = Gs + 2 * RP * LG;
+      gd_fill(sy[0], [&](int i, int j) { return Gn[i * LG + j]; }, [&](int i, int cc) { return TT[cc * LD + i]; });
+      gd_fill(sy[1], [&](int i, int j) { return Gn[i * LG + j] + Gb[i * LG + j]; },
+              [&](int i, int cc) { return TT[cc * LD + i]; });
+    } else {
+      gd_fill(sy[0], [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
+      gd_fill(sy[1], [&](int i, int j) { return Gq[i * RP + j] + Gb[i * LG + j]; },
+              [&](int i, int cc) { return Cq[i * d + cc] + BqT[i * d + cc]; });
+    }
+    if constexpr (kHold) {
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) sy[1].x[rt][u] += bk[rt][u];
+        for (int u = 0; u < CT; ++u) sy[1].x[rt][u] += bk[rt][u];
+    }
   }
   __syncthreads();
   gd_solve_pair(sy, piv);
@@ -950,126 +987,172 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int stage, int i
   {
     float* mt = a.Mt_k + (int64_t)h * r * d;
     gd_drain(sy[1].x, [&](int i, int cc, double v) {
-      MT[cc * kGdLd + i] = v;
+      MT[cc * LD + i] = v;
       if (i < r) mt[i * d + cc] = (float)v;
+      if constexpr (!kHold) part_k = fma(Ck[i * d + cc], v, part_k);
     });
+    if constexpr (kHold) {
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt)
+      for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < CT; ++u)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) part_k = fma(ckt[rt][u][v], sy[1].x[rt][u][v], part_k);
+          for (int v = 0; v < 4; ++v) part_k = fma(ckt[rt][u][v], sy[1].x[rt][u][v], part_k);
+    }
   }
   double trk_old = 0.0;
-  if (tid < 32) trk_old = tid < r ? Gk[tid * 32 + tid] : 0.0;
+  if (tid < RP) trk_old = tid < r ? Gk[tid * RP + tid] : 0.0;
   __syncthreads();
   // ---- U = Mk'^T Sk, Gk' = Mk'^T U^T, Ck' = U
-  gd_times_s(MT, Sk, TT);
+  gd_times_s<RT, D>(MT, Sk, TT);
   {
-    double o[4];
-    gd_outer(MT, TT, o);
     double tr_new = 0.0;
-    if (tid < 256) {
-      const int j = gd_outer_col();
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int i = gd_outer_row(u);
-        const double v = (i < r && j < r) ? o[u] : (i == j ? 1.0 : 0.0);
-        Gk[i * 32 + j] = v;
-        if (i == j && i < r) tr_new += v;
-      }
-    }
+    gd_outer<RT, D>(MT, TT, [&](int i, int j, double o) {
+      const double v = (i < r && j < r) ? o : (i == j ? 1.0 : 0.0);
+      Gk[i * RP + j] = v;
+      if (i == j && i < r) tr_new += v;
+    });
     const double dk = gd_block_sum(trk_old - 2.0 * part_k + tr_new, red);
     if (tid == 0) a.delta[((int64_t)it * 2 + 1) * bh + h] = dk;
   }
-  if (tid < d) {
-#pragma unroll
-    for (int i = 0; i < 32; ++i) Ck[i * d + tid] = TT[tid * kGdLd + i];
+#pragma unroll 8
+  for (int e = tid; e < RP * d; e += kGdThreads) Ck[e] = TT[(e % d) * LD + e / d];
   }
 }
 
-// Workspace (bytes) of the Gram-domain iteration for bh heads over bkv distinct K heads.
-static size_t gramdom_bytes(int bh, int bkv, int Sx, int Sxk, int iters, size_t own_part_floats) {
-  const size_t dd = (size_t)kGdD * kGdD;
-  return ((size_t)bh * Sx + (size_t)bkv * Sxk) * dd * sizeof(float)      // X^T X partial sums
-         + own_part_floats * sizeof(float)                                // (G, C) partial sums of the fused kernel
-         + ((size_t)bh + bkv) * dd * sizeof(double)                       // Sq, Sk
-         + (size_t)2 * bh * (1024 + 32 * kGdD) * sizeof(double)           // G, C
-         + (size_t)bh * 32 * kGdD * sizeof(double)                        // B_Q handed from iteration to iteration
-         + (size_t)std::max(iters, 1) * 2 * bh * sizeof(double)           // squared changes
-         + (size_t)2 * bh * 32 * kGdD * sizeof(float) + 256;              // Mq^T, Mk^T
-}
-
-// Runs all iterations on the Gram matrices.  On return Mt_q / Mt_k (device pointers written to *mt_q, *mt_k)
-// hold Mq^T, Mk^T of the last iteration that ran, and b_q, b_k the final B factors; the caller applies
-// A_Q = Q Mq, A_K = K Mk.  The initial [G | C] sums: partK (and partQ) with S splits from the row-by-row pass; with
-// a_q0 (the given A_Q, [bh][l][r]) the Q side's are formed here together with Q^T Q and partQ is not read.
-int prefill_gram_domain(lrqk_ctx* ctx, const void* q, const void* k, const float* partQ, const float* partK, int S,
-                        const float* a_q0, float* b_q, float* b_k, int b, int hq, int hkv, int64_t l, int r, int iters,
-                        float tol, int* flags, float** mt_q, float** mt_k, hipStream_t st) {
-  const int bh = b * hq, bkv = b * hkv;
-  const int d = kGdD;
-  const bool fused = a_q0 != nullptr;
-  LRQK_REQUIRE(partK && (fused || partQ), LRQK_EINVAL, "neither partial sums nor initial factors");
-  // splits of the long axis for the X^T X sums: about two workgroups per CU for Q, one for K (with 64 splits of 8
-  // heads the partial sums are 33 MB to write and to add up: 25.6 + 18.5 us against 19.7 + 11.1 with 32).  The
-  // fused kernel: one workgroup per CU (registers), at most 4096 rows per split (its fp32 sums), at least one step each.
-  int Sx = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 512 / bh), (l + 511) / 512));
-  const int Sxk = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512));
-  int Spq = S;
-  if (fused) {
-    int64_t v = std::max<int64_t>(std::max(1, 256 / bh), (l + 4095) / 4096);
-    v = std::min<int64_t>(v, 64);
-    Sx = Spq = (int)std::max<int64_t>(1, std::min<int64_t>(v, (l + kXtxRows - 1) / kXtxRows));
-  }
-  const size_t ne = (size_t)r * (r + d);
-  const size_t own_part = fused ? (size_t)bh * Spq * ne : 0;
-  int rc = ctx->prefill_gd.ensure(gramdom_bytes(bh, bkv, Sx, Sxk, iters, own_part));
-  if (rc) return rc;
-  const size_t dd = (size_t)d * d;
-  char* p = (char*)ctx->prefill_gd.p;
-  double* Sq = (double*)p;                  p += (size_t)bh * dd * sizeof(double);
-  double* Sk = (double*)p;                  p += (size_t)bkv * dd * sizeof(double);
-  double* G = (double*)p;                   p += (size_t)2 * bh * 1024 * sizeof(double);
-  double* C = (double*)p;                   p += (size_t)2 * bh * 32 * d * sizeof(double);
-  double* BqT = (double*)p;                 p += (size_t)bh * 32 * d * sizeof(double);
-  double* delta = (double*)p;               p += (size_t)std::max(iters, 1) * 2 * bh * sizeof(double);
-  float* Mtq = (float*)p;                   p += (size_t)bh * 32 * d * sizeof(float);
-  float* Mtk = (float*)p;                   p += (size_t)bh * 32 * d * sizeof(float);
-  float* xq_part = (float*)p;               p += (size_t)bh * Sx * dd * sizeof(float);
-  float* xk_part = (float*)p;               p += (size_t)bkv * Sxk * dd * sizeof(float);
-  if (fused) {
-    float* pq = (float*)p;
-    LRQK_REQUIRE((uintptr_t)q % 16 == 0, LRQK_EINVAL, "rows must be 16-byte aligned");
-    hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)Spq, (unsigned)bh), dim3(kXtxThreads), 0, st, (const bf16_t*)q, l,
-                       a_q0, r, pq, xq_part, Spq);
-    partQ = pq;
-  } else {
-    hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sx, (unsigned)bh), dim3(kXtxThreads), 0, st, (const bf16_t*)q, l,
-                       xq_part, Sx);
-  }
-  hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sxk, (unsigned)bkv), dim3(kXtxThreads), 0, st, (const bf16_t*)k, l,
-                     xk_part, Sxk);
-  LRQK_HIP_CHECK(hipGetLastError());
-  const size_t smem = ((size_t)3 * kGdD * kGdLd + 3 * 32 * kGdLg + kGdPivDoubles + 8) * sizeof(double);
+template <int RT, int D>
+static int gramdom_run(const GdArgs& a, const float* xq_part, int Sx, const float* xk_part, int Sxk, int bkv, double* Sq,
+                       double* Sk, int iters, hipStream_t st) {
+  using Sh = GdShape<RT, D>;
+  constexpr int RP = Sh::RP;
+  constexpr bool WIDE = Sh::WIDE;
+  using Fn = void (*)(int, GdArgs);
+  const Fn last = pf_gramdom_kernel<RT, D, kGdFinal>;
+  const Fn start = WIDE ? pf_gramdom_kernel<RT, D, WIDE ? kGdStart : kGdFinal> : nullptr;
+  const Fn steps[2] = {pf_gramdom_kernel<RT, D, WIDE ? kGdQSide : kGdWhole>,
+                       WIDE ? pf_gramdom_kernel<RT, D, WIDE ? kGdKSide : kGdWhole> : nullptr};
+  static_assert(Sh::SMEM <= 160 * 1024, "LDS");
   static std::atomic<bool> attr_dev[kMaxDeviceSlots];
   std::atomic<bool>& attr = attr_dev[per_device_slot()];
   if (!attr) {
-    LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)pf_gramdom_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)smem));
+    for (Fn f : {last, start, steps[0], steps[1]})
+      if (f)
+        LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Sh::SMEM));
     attr = true;
   }
-  GdArgs a{partQ, partK, Spq, S, Sq, Sk, G, C, BqT, delta, flags, Mtq, Mtk, b_q, b_k, bh, hq, hkv, r, l, tol};
-  const unsigned init_blocks = (unsigned)(((size_t)bh + bkv) * (dd / 256) + (size_t)2 * bh * kGdInitBlocks);
-  hipLaunchKernelGGL(pf_gramdom_init_kernel, dim3(init_blocks), dim3(256), 0, st, a, (const float*)xq_part, Sx,
-                     (const float*)xk_part, Sxk, bkv, Sq, Sk);
+  const unsigned init_blocks = (unsigned)(((size_t)a.bh + bkv) * (D * D / 256) + (size_t)2 * a.bh * (RP * (RP + D) / 256));
+  hipLaunchKernelGGL((pf_gramdom_init_kernel<RP, D>), dim3(init_blocks), dim3(256), 0, st, a, xq_part, Sx, xk_part, Sxk, bkv,
+                     Sq, Sk);
+  if (start && iters > 0) hipLaunchKernelGGL(start, dim3((unsigned)a.bh), dim3(kGdThreads), Sh::SMEM, st, 0, a);
   for (int it = 0; it < iters; ++it)
-    hipLaunchKernelGGL(pf_gramdom_kernel, dim3((unsigned)bh), dim3(kGdThreads), smem, st, 0, it, a);
-  hipLaunchKernelGGL(pf_gramdom_kernel, dim3((unsigned)bh), dim3(kGdThreads), smem, st, 2, iters, a);
+    for (Fn f : steps)
+      if (f) hipLaunchKernelGGL(f, dim3((unsigned)a.bh), dim3(kGdThreads), Sh::SMEM, st, it, a);
+  hipLaunchKernelGGL(last, dim3((unsigned)a.bh), dim3(kGdThreads), Sh::SMEM, st, iters, a);
   LRQK_HIP_CHECK(hipGetLastError());
-  *mt_q = Mtq;
-  *mt_k = Mtk;
   return LRQK_OK;
 }
+
+// The whole factorisation on Gram matrices: q [b][hq][l][d], k [b][hkv][l][d], 16-byte aligned, d = 64 or 128, r <= 64;
+// a_q0, a_k0: the given factors, fp32 [b hq][l][r].
+template <typename T>
+int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, float* a_k0, const PrefillOut& out, int b, int hq,
+                        int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st) {
+  const int bh = b * hq, bkv = b * hkv;
+  // bf16 rows of 128 elements and ranks up to 32 have kernels of their own for the passes: the Q side's sums with Q^T Q
+  // from one reading of Q, K^T K alone, A_K for several query heads from one reading of K
+  const bool tuned = sizeof(T) == 2 && d == 128 && r <= 32;
+  const int RP = r <= 16 ? 16 : r <= 32 ? 32 : 64;
+  const size_t ne = (size_t)r * (r + d), dd = (size_t)d * d;
+  // Splits of the long axis: one workgroup per CU and launch (the kernels' registers), at most 4096 rows per split
+  // (its fp32 sums; the splits are added in fp64), at least one step of rows each.
+  auto splits = [&](int heads) {
+    int64_t v = std::max<int64_t>(std::max(1, 256 / heads), (l + 4095) / 4096);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(v, 64), (l + 127) / 128));
+  };
+  const int S = splits(bh), Sx = S;
+  // (K^T K: with 64 splits of 8 heads the partial sums are 33 MB to write and to add up: 25.6 + 18.5 us against
+  // 19.7 + 11.1 with 32)
+  const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
+                        : hkv == hq ? S : splits(bkv);
+  const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
+  const size_t bytes = ((size_t)bh + bkv) * dd * 8 + (size_t)2 * bh * RP * (RP + d) * 8 + (size_t)bh * RP * d * 8 +
+                       (RP == 64 ? (size_t)bh * 2 * RP * (RP + 1) * 8 : 0) + (size_t)std::max(iters, 1) * 2 * bh * 8 +
+                       (size_t)2 * bh * RP * d * 4 + ((size_t)bh * Sx + (size_t)bkv * Sxk) * dd * 4 +
+                       (size_t)2 * bh * S * ne * 4 + n_flags * 4;
+  int rc = ctx->prefill_gd.ensure(bytes);
+  if (rc) return rc;
+  char* p = (char*)ctx->prefill_gd.p;
+  auto take = [&](size_t n) {
+    char* at = p;
+    p += n;
+    return at;
+  };
+  GdArgs a{};
+  double* Sq = (double*)take((size_t)bh * dd * 8);
+  double* Sk = (double*)take((size_t)bkv * dd * 8);
+  a.Sq = Sq;
+  a.Sk = Sk;
+  a.G = (double*)take((size_t)2 * bh * RP * RP * 8);
+  a.C = (double*)take((size_t)2 * bh * RP * d * 8);
+  a.BqT = (double*)take((size_t)bh * RP * d * 8);
+  if (RP == 64) a.Gs = (double*)take((size_t)bh * 2 * RP * (RP + 1) * 8);
+  a.delta = (double*)take((size_t)std::max(iters, 1) * 2 * bh * 8);
+  a.Mt_q = (float*)take((size_t)bh * RP * d * 4);
+  a.Mt_k = (float*)take((size_t)bh * RP * d * 4);
+  float* xq_part = (float*)take((size_t)bh * Sx * dd * 4);
+  float* xk_part = (float*)take((size_t)bkv * Sxk * dd * 4);
+  float* partQ = (float*)take((size_t)bh * S * ne * 4);
+  float* partK = (float*)take((size_t)bh * S * ne * 4);
+  a.flags = (int*)take(n_flags * 4);
+  a.partQ = partQ;
+  a.partK = partK;
+  a.S = a.S_k = S;
+  a.b_q = out.b_q;
+  a.b_k = out.b_k;
+  a.out_bf16 = out.storage && sizeof(T) == 2;
+  a.bh = bh;
+  a.hq = hq;
+  a.hkv = hkv;
+  a.r = r;
+  a.l = l;
+  a.tol = tol;
+
+  if (tuned) {
+    hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)S, (unsigned)bh), dim3(kXtxThreads), 0, st, (const bf16_t*)q, l, a_q0, r,
+                       partQ, xq_part, S);
+    if ((rc = prefill_given_sums_bf16((const bf16_t*)k, hkv, hq, b, l, r, a_k0, partK, S, st))) return rc;
+    hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sxk, (unsigned)bkv), dim3(kXtxThreads), 0, st, (const bf16_t*)k, l,
+                       xk_part, Sxk);
+    LRQK_HIP_CHECK(hipGetLastError());
+  } else {
+    if ((rc = prefill_stream_sums<T>(q, hq, hq, b, l, r, d, a_q0, partQ, S, xq_part, Sx, st))) return rc;
+    if ((rc = prefill_stream_sums<T>(k, hkv, hq, b, l, r, d, a_k0, partK, S, xk_part, Sxk, st))) return rc;
+  }
+#define LRQK_GD_RUN(RTV, DV) gramdom_run<RTV, DV>(a, xq_part, Sx, xk_part, Sxk, bkv, Sq, Sk, iters, st)
+  rc = d == 64 ? (RP == 16 ? LRQK_GD_RUN(1, 64) : RP == 32 ? LRQK_GD_RUN(2, 64) : LRQK_GD_RUN(4, 64))
+               : (RP == 16 ? LRQK_GD_RUN(1, 128) : RP == 32 ? LRQK_GD_RUN(2, 128) : LRQK_GD_RUN(4, 128));
+#undef LRQK_GD_RUN
+  if (rc) return rc;
+  auto finish = [&](auto* a_q, auto* a_k) -> int {
+    using OUT = std::remove_reference_t<decltype(*a_q)>;
+    if (iters == 0) {  // the given factors are the result
+      int rcs = prefill_store<OUT>(a_q0 + (l - out.a_q_rows) * r, l * r, a_q, out.a_q_rows * r, out.a_q_rows * r, bh, st);
+      return rcs ? rcs : prefill_store<OUT>(a_k0, l * r, a_k, out.a_k_stride, l * r, bh, st);
+    }
+    const int64_t rows = out.a_q_rows;  // (the last ones)
+    int rcs = prefill_stream_apply<T, OUT>(q + (l - rows) * d, hq, hq, b, rows, l * d, r, d, a.Mt_q, a_q, rows * r, st);
+    if (rcs) return rcs;
+    const int nh = hq / hkv;
+    if (tuned && (nh == 2 || nh == 4))
+      return apply_shared<OUT>(k, a.Mt_k, a_k, out.a_k_stride, bkv, nh, l, r, st);
+    return prefill_stream_apply<T, OUT>(k, hkv, hq, b, l, l * d, r, d, a.Mt_k, a_k, out.a_k_stride, st);
+  };
+  if (out.storage && sizeof(T) == 2) return finish((T*)out.a_q, (T*)out.a_k);
+  return finish((float*)out.a_q, (float*)out.a_k);
+}
+template int prefill_gram_domain<float>(lrqk_ctx*, const float*, const float*, float*, float*, const PrefillOut&, int, int,
+                                        int, int64_t, int, int, int, float, hipStream_t);
+template int prefill_gram_domain<bf16_t>(lrqk_ctx*, const bf16_t*, const bf16_t*, float*, float*, const PrefillOut&, int, int,
+                                         int, int64_t, int, int, int, float, hipStream_t);
 
 }  // namespace lrqk

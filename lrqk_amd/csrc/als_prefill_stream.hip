@@ -1,0 +1,420 @@
+// The passes over the long axis for the prefill iterations on Gram matrices, for every input that als_prefill_gram.hip
+// has no kernel tuned for: fp32 rows, rows of 64 elements, ranks 33 .. 64.
+//
+//   sums   S = X^T X, and over given factors A the sums G = A^T A, C = A^T X
+//   apply  A = X M
+//
+// All on the bf16 matrix cores (32x32x16) with fp32 accuracy: an fp32 operand is the exact sum of three bf16 pieces, a
+// product of two pieces is exact in fp32, and all piece pairs but lo x lo (2^-32) are formed.  Both are bound by HBM
+// (every input read once), so the shape of the kernels follows the memory: a wave streams 32-row groups of its own
+// through a private LDS tile, the next group already requested, and never meets another wave before the end.
+// 32 heads of 16384 bf16 rows of 128, rank 64: sums over the given factors 98 us (268 MB; 20 us of matrix-core time),
+// Q^T Q 32 us, A_K 77 us; the row-by-row kernels for this rank took 1.3 ms per pass, ten passes for four iterations.
+#include <algorithm>
+
+#include "common.hpp"
+#include "ctx.hpp"
+#include "prefill_pieces.hpp"
+
+namespace lrqk {
+
+constexpr int kStWaves = 4, kStThreads = kStWaves * kWave;
+
+__device__ __forceinline__ void st_wave_sync() {  // orders one wave's LDS writes and reads
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// a x b over piece pairs, smallest first (PA, PB = 1: a bf16 operand as it is), KB k blocks, into a fresh accumulator:
+// the matrix cores do not round to nearest when they add to a large one, so a 32-row group's sum joins the running
+// total by ordinary fp32 additions.
+template <int PA, int PB>
+__device__ __forceinline__ gd_floatx16 st_product(const gd_bf16x8 (&a)[2][PA], const gd_bf16x8 (&b)[2][PB]) {
+  gd_floatx16 t;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+#pragma unroll
+  for (int w = PA + PB - 2; w >= 0; --w)  // (a piece of index p is 2^-8p of its number)
+#pragma unroll
+    for (int i = PA - 1; i >= 0; --i) {
+      const int j = w - i;
+      if (j < 0 || j >= PB || (PA == 3 && PB == 3 && w == 4)) continue;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kb][i], b[kb][j], t, 0, 0, 0);
+    }
+  return t;
+}
+
+// AT: 32-column tiles of A (ranks up to 32, 64); DB: 32-column blocks of X (64, 128 elements); GIVEN: sums over the
+// given factors, a head per query head (X of its kv head); XTX: X^T X, a head per head of X.  Both in one launch where
+// the accumulators allow it (DB = 2: up to 10 tiles; DB = 4 would need 15 to 21 of 16 registers each beside the
+// operands), else one launch each.
+// grid (S, heads); 4 waves; split s of a head takes every S-th set of 4 x 32 rows, so the workgroups of a head walk its
+// rows side by side.  part: [head][S][r][r + d]; xtx_part: [head][S][d][d] (both triangles).
+template <typename T, int AT, int DB, bool GIVEN, bool XTX>
+__global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __restrict__ X, int xh, int hq, int64_t l,
+                                                                    int r, const float* __restrict__ A,
+                                                                    float* __restrict__ part,
+                                                                    float* __restrict__ xtx_part, int S) {
+  constexpr int D = 32 * DB;
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int P = F32 ? 3 : 1;
+  constexpr int VEC = Vec16<T>::N;
+  // row stride of the LDS tile in elements.  bf16: the transposing reads want successive rows 8 banks apart; fp32: a
+  // read takes one column of rows 4 apart in the wave's halves, which 8 floats of padding put 32 banks apart
+  constexpr int LDX = F32 ? D + 8 : D + 16;
+  constexpr int NL = 32 * D / (kWave * VEC);
+  constexpr int TILE = 32 * LDX * (int)sizeof(T);
+  constexpr int SMEM = kStWaves * (TILE > 4096 ? TILE : 4096);
+  __shared__ __align__(16) char smem[SMEM];
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int col = lane & 31, half = lane >> 5;
+  T* x_s = reinterpret_cast<T*>(smem + wave * (SMEM / kStWaves));
+  const int h = blockIdx.y, s = blockIdx.x;
+  const int64_t xhead = GIVEN ? (int64_t)(h / hq) * xh + (h % hq) / (hq / xh) : h;
+  const T* Xh = X + xhead * l * D;
+  const float* Ah = A + (int64_t)h * l * r;
+
+  constexpr int NAA = AT * (AT + 1) / 2, NXX = DB * (DB + 1) / 2;
+  gd_floatx16 gAA[GIVEN ? NAA : 1], gAX[GIVEN ? AT : 1][GIVEN ? DB : 1], gXX[XTX ? NXX : 1];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    if constexpr (GIVEN) {
+#pragma unroll
+      for (int i = 0; i < NAA; ++i) gAA[i][v] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < AT; ++i)
+#pragma unroll
+        for (int n = 0; n < DB; ++n) gAX[i][n][v] = 0.0f;
+    }
+    if constexpr (XTX) {
+#pragma unroll
+      for (int i = 0; i < NXX; ++i) gXX[i][v] = 0.0f;
+    }
+  }
+
+  gd_u32x4 pre[NL];
+  float arow[GIVEN ? AT : 1][16];
+  auto issue = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * VEC;
+      pre[i] = *reinterpret_cast<const gd_u32x4*>(Xh + min(t0 + e / D, l - 1) * D + e % D);
+    }
+    if constexpr (GIVEN) {
+#pragma unroll
+      for (int at = 0; at < AT; ++at)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          arow[at][v] = Ah[min(t0 + gd_mfma_row(lane, v), l - 1) * r + min(32 * at + col, r - 1)];
+    }
+  };
+  const int64_t stride = (int64_t)S * kStWaves * 32;
+  const int64_t first = ((int64_t)s * kStWaves + wave) * 32;
+  if (first < l) issue(first);
+  for (int64_t t0 = first; t0 < l; t0 += stride) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * VEC;
+      *reinterpret_cast<gd_u32x4*>(&x_s[(e / D) * LDX + e % D]) = t0 + e / D < l ? pre[i] : gd_u32x4{0, 0, 0, 0};
+    }
+    // the pieces of this group's rows of A: element v of a lane is row gd_mfma_row(lane, v) of its column, so eight at
+    // a time are an operand's k elements (X comes out of LDS in the same order)
+    gd_bf16x8 cp[GIVEN ? AT : 1][2][3];
+    if constexpr (GIVEN) {
+#pragma unroll
+      for (int at = 0; at < AT; ++at)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          float f[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            f[q] = t0 + gd_mfma_row(lane, 8 * kb + q) < l && 32 * at + col < r ? arow[at][8 * kb + q] : 0.0f;
+          gd_split3x8(f, cp[at][kb]);
+        }
+    }
+    st_wave_sync();
+    if (t0 + stride < l) issue(t0 + stride);
+    // rows 16 kb + 4 half .. + 3 and the same + 8 of column 32 nb + col
+    auto operand = [&](int nb, gd_bf16x8 (&x)[2][P]) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        if constexpr (F32) {
+          float f[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) f[q] = ((const float*)x_s)[gd_mfma_row(lane, 8 * kb + q) * LDX + 32 * nb + col];
+          gd_split3x8(f, x[kb]);
+        } else {
+          const int s16 = lane & 15;
+          const uint16_t* p = (const uint16_t*)x_s + (16 * kb + 4 * half + (s16 >> 2)) * LDX + 32 * nb + (col & 16) + 4 * (s16 & 3);
+          const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
+          const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 8 * LDX));
+          x[kb][0] = __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+      }
+    };
+    if constexpr (GIVEN) {
+#pragma unroll
+      for (int ta = 0; ta < AT; ++ta)
+#pragma unroll
+        for (int tb = ta; tb < AT; ++tb) {
+          const gd_floatx16 t = st_product<3, 3>(cp[ta], cp[tb]);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) gAA[ta + tb][v] += t[v];
+        }
+    }
+    gd_bf16x8 xb[XTX ? DB : 1][2][P];
+#pragma unroll
+    for (int nb = 0; nb < DB; ++nb) {
+      gd_bf16x8(&x)[2][P] = xb[XTX ? nb : 0];
+      operand(nb, x);
+      if constexpr (GIVEN) {
+#pragma unroll
+        for (int at = 0; at < AT; ++at) {
+          const gd_floatx16 t = st_product<3, P>(cp[at], x);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) gAX[at][nb][v] += t[v];
+        }
+      }
+      if constexpr (XTX) {
+#pragma unroll
+        for (int n2 = 0; n2 <= nb; ++n2) {
+          const gd_floatx16 t = st_product<P, P>(xb[n2], x);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) gXX[nb * (nb + 1) / 2 + n2][v] += t[v];
+        }
+      }
+    }
+    st_wave_sync();  // this wave's reads of the tile precede its next staging writes
+  }
+  // the four waves' tiles, one at a time: f(row, column, sum)
+  float* sm = reinterpret_cast<float*>(smem);
+  auto reduce = [&](const gd_floatx16& acc, auto&& f) {
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sm[wave * 1024 + gd_mfma_row(lane, v) * 32 + col] = acc[v];
+    __syncthreads();
+#pragma unroll
+    for (int o = tid; o < 1024; o += kStThreads)
+      f(o >> 5, o & 31, (sm[o] + sm[1024 + o]) + (sm[2048 + o] + sm[3072 + o]));
+  };
+  if constexpr (GIVEN) {
+    const int ld = r + D;
+    float* out = part + ((int64_t)h * S + s) * r * ld;
+#pragma unroll
+    for (int ta = 0; ta < AT; ++ta) {
+#pragma unroll
+      for (int tb = ta; tb < AT; ++tb)
+        reduce(gAA[ta + tb], [&](int m, int n, float v) {
+          m += 32 * ta;
+          n += 32 * tb;
+          if (m < r && n < r) {
+            out[m * ld + n] = v;
+            if (ta != tb) out[n * ld + m] = v;
+          }
+        });
+#pragma unroll
+      for (int nb = 0; nb < DB; ++nb)
+        reduce(gAX[ta][nb], [&](int m, int n, float v) {
+          if (32 * ta + m < r) out[(32 * ta + m) * ld + r + 32 * nb + n] = v;
+        });
+    }
+  }
+  if constexpr (XTX) {
+    float* out = xtx_part + ((int64_t)h * S + s) * D * D;
+#pragma unroll
+    for (int nb = 0; nb < DB; ++nb)
+#pragma unroll
+      for (int n2 = 0; n2 <= nb; ++n2)
+        reduce(gXX[nb * (nb + 1) / 2 + n2], [&](int m, int n, float v) {
+          out[(32 * n2 + m) * D + 32 * nb + n] = v;
+          if (n2 != nb) out[(32 * nb + n) * D + 32 * n2 + m] = v;
+        });
+  }
+}
+
+// A = X M for every query head (l rows of its kv head's X, heads x_stride elements apart): M^T (fp32, [head][r][d]) in LDS as three bf16 pieces, X through the
+// wave's private tile.  A: OUT, heads `a_stride` elements apart, rows of r.  grid (S, query heads); the workgroups of
+// the query heads that share a kv head lie next to each other, so K comes from the caches after the first of them.
+template <typename T, int AT, int DB, typename OUT>
+__global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_apply_kernel(
+    const T* __restrict__ X, int xh, int hq, int64_t l, int64_t x_stride, int r, const float* __restrict__ Mt,
+    OUT* __restrict__ A, int64_t a_stride, int S) {
+  constexpr int D = 32 * DB;
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int NW = F32 ? 4 : 8, NT = NW * kWave;
+  constexpr int P = F32 ? 3 : 1;
+  constexpr int VEC = Vec16<T>::N;
+  constexpr int LDM = D + 8, LDX = F32 ? D + 4 : D + 8;  // (16-byte operand reads want rows 4 banks apart)
+  constexpr int NL = 32 * D / (kWave * VEC);
+  extern __shared__ __align__(16) char ap_smem[];
+  uint16_t* mt_s = reinterpret_cast<uint16_t*>(ap_smem);                                 // [3][32 AT][LDM]
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  T* x_s = reinterpret_cast<T*>(ap_smem + 3 * 32 * AT * LDM * 2) + wave * 32 * LDX;      // this wave's rows of X
+  const int col = lane & 31, half = lane >> 5;
+  const int h = blockIdx.y, s = blockIdx.x;
+  const T* Xh = X + ((int64_t)(h / hq) * xh + (h % hq) / (hq / xh)) * x_stride;
+  OUT* Ah = A + (int64_t)h * a_stride;
+  for (int e = tid; e < 32 * AT * D; e += NT) {
+    const int n = e / D, k = e % D;
+    const float v = n < r ? Mt[((int64_t)h * r + n) * D + k] : 0.0f;
+    uint32_t p0, p1, p2;
+    gd_split3(v, p0, p1, p2);
+    mt_s[(0 * 32 * AT + n) * LDM + k] = (uint16_t)(p0 >> 16);
+    mt_s[(1 * 32 * AT + n) * LDM + k] = (uint16_t)(p1 >> 16);
+    mt_s[(2 * 32 * AT + n) * LDM + k] = (uint16_t)(p2 >> 16);
+  }
+  gd_u32x4 pre[NL];
+  auto issue = [&](int64_t t0) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * VEC;
+      pre[i] = *reinterpret_cast<const gd_u32x4*>(Xh + min(t0 + e / D, l - 1) * D + e % D);
+    }
+  };
+  const int64_t stride = (int64_t)S * NW * 32;
+  const int64_t first = ((int64_t)s * NW + wave) * 32;
+  if (first < l) issue(first);
+  __syncthreads();  // M staged
+  for (int64_t t0 = first; t0 < l; t0 += stride) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * VEC;
+      *reinterpret_cast<gd_u32x4*>(&x_s[(e / D) * LDX + e % D]) = pre[i];  // (rows beyond l are never stored from)
+    }
+    st_wave_sync();
+    if (t0 + stride < l) issue(t0 + stride);
+    gd_floatx16 c[AT];
+#pragma unroll
+    for (int at = 0; at < AT; ++at)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) c[at][v] = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < D / 16; ++kb) {
+      gd_bf16x8 xa[P];
+      if constexpr (F32) {
+        const float4 lo = *reinterpret_cast<const float4*>(&x_s[col * LDX + 16 * kb + 8 * half]);
+        const float4 hi = *reinterpret_cast<const float4*>(&x_s[col * LDX + 16 * kb + 8 * half + 4]);
+        const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        gd_split3x8(f, xa);
+      } else {
+        xa[0] = *reinterpret_cast<const gd_bf16x8*>(&x_s[col * LDX + 16 * kb + 8 * half]);
+      }
+#pragma unroll
+      for (int at = 0; at < AT; ++at) {
+        gd_bf16x8 m[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          m[p] = *reinterpret_cast<const gd_bf16x8*>(&mt_s[(p * 32 * AT + 32 * at + col) * LDM + 16 * kb + 8 * half]);
+#pragma unroll
+        for (int w = P + 1; w >= 0; --w)
+#pragma unroll
+          for (int i = P - 1; i >= 0; --i) {
+            if (w - i < 0 || w - i >= 3 || (P == 3 && w == 4)) continue;
+            c[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[i], m[w - i], c[at], 0, 0, 0);
+          }
+      }
+    }
+#pragma unroll
+    for (int at = 0; at < AT; ++at)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int64_t row = t0 + gd_mfma_row(lane, v);
+        if (row < l && 32 * at + col < r) gd_store(Ah, row * r + 32 * at + col, c[at][v]);
+      }
+    st_wave_sync();  // this wave's reads of the tile precede its next staging writes
+  }
+}
+
+// fp32 factors (heads l rows apart) to the output's type and place
+template <typename OUT>
+__global__ __launch_bounds__(256) void pf_store_factors_kernel(const float* __restrict__ src, int64_t src_stride,
+                                                               OUT* __restrict__ dst, int64_t dst_stride, int64_t n) {
+  const float* s = src + (int64_t)blockIdx.y * src_stride;
+  OUT* d = dst + (int64_t)blockIdx.y * dst_stride;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) gd_store(d, i, s[i]);
+}
+
+template <typename OUT>
+int prefill_store(const float* src, int64_t src_stride, OUT* dst, int64_t dst_stride, int64_t n, int heads, hipStream_t st) {
+  if (n <= 0 || (const void*)src == (const void*)dst) return LRQK_OK;
+  const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 1023) / 1024, 4096 / heads + 1));
+  hipLaunchKernelGGL((pf_store_factors_kernel<OUT>), dim3(blocks, (unsigned)heads), dim3(256), 0, st, src, src_stride, dst,
+                     dst_stride, n);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
+}
+template int prefill_store<float>(const float*, int64_t, float*, int64_t, int64_t, int, hipStream_t);
+template int prefill_store<bf16_t>(const float*, int64_t, bf16_t*, int64_t, int64_t, int, hipStream_t);
+
+template <typename T, int AT, int DB>
+static int sums_impl(const T* x, int xh, int hq, int b, int64_t l, int r, const float* a, float* part, int S, float* xtx,
+                     int Sx, hipStream_t st) {
+  const dim3 given((unsigned)S, (unsigned)(b * hq)), heads((unsigned)Sx, (unsigned)(b * xh)), blk(kStThreads);
+  if (DB == 2 && xh == hq && S == Sx) {
+    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, 2, true, true>), given, blk, 0, st, x, xh, hq, l, r, a, part, xtx, S);
+  } else {
+    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, true, false>), given, blk, 0, st, x, xh, hq, l, r, a, part, xtx, S);
+    hipLaunchKernelGGL((pf_stream_sums_kernel<T, 1, DB, false, true>), heads, blk, 0, st, x, xh, hq, l, r, a, part, xtx, Sx);
+  }
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
+}
+
+// Sums of one side: over the given factors ([b * hq] heads, S splits) and X^T X ([b * xh] heads, Sx splits).
+template <typename T>
+int prefill_stream_sums(const T* x, int xh, int hq, int b, int64_t l, int r, int d, const float* a, float* part, int S,
+                        float* xtx, int Sx, hipStream_t st) {
+  if (d == 64)
+    return r <= 32 ? sums_impl<T, 1, 2>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st)
+                   : sums_impl<T, 2, 2>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st);
+  return r <= 32 ? sums_impl<T, 1, 4>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st)
+                 : sums_impl<T, 2, 4>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st);
+}
+template int prefill_stream_sums<float>(const float*, int, int, int, int64_t, int, int, const float*, float*, int, float*,
+                                        int, hipStream_t);
+template int prefill_stream_sums<bf16_t>(const bf16_t*, int, int, int, int64_t, int, int, const float*, float*, int, float*,
+                                         int, hipStream_t);
+
+template <typename T, int AT, int DB, typename OUT>
+static int apply_impl(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, const float* mt, OUT* a, int64_t a_stride,
+                      hipStream_t st) {
+  constexpr int D = 32 * DB, NW = sizeof(T) == 4 ? 4 : 8;
+  constexpr size_t smem = (size_t)3 * 32 * AT * (D + 8) * 2 + (size_t)NW * 32 * (sizeof(T) == 4 ? D + 4 : D + 8) * sizeof(T);
+  static_assert(smem <= 160 * 1024, "LDS");
+  auto kern = pf_stream_apply_kernel<T, AT, DB, OUT>;
+  static std::atomic<bool> attr_dev[kMaxDeviceSlots];
+  std::atomic<bool>& attr = attr_dev[per_device_slot()];
+  if (!attr) {
+    LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    attr = true;
+  }
+  // every workgroup stages M (52 KB in, up to 104 KB of fp32 read): enough of them to fill the GPU once, no more
+  const int bh = b * hq;
+  const int per_cu = std::max(1, (int)(160 * 1024 / smem));
+  const int64_t S = std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (l + 32 * NW - 1) / (32 * NW)));
+  hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)bh), dim3(NW * kWave), smem, st, x, xh, hq, l, x_stride, r, mt, a, a_stride,
+                     (int)S);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
+}
+
+// A = X M for all b * hq query heads: l rows per head, X's heads x_stride and A's a_stride elements apart.
+template <typename T, typename OUT>
+int prefill_stream_apply(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, int d, const float* mt,
+                         OUT* a, int64_t a_stride, hipStream_t st) {
+  if (d == 64)
+    return r <= 32 ? apply_impl<T, 1, 2>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st)
+                   : apply_impl<T, 2, 2>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st);
+  return r <= 32 ? apply_impl<T, 1, 4>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st)
+                 : apply_impl<T, 2, 4>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st);
+}
+template int prefill_stream_apply<float, float>(const float*, int, int, int, int64_t, int64_t, int, int, const float*,
+                                                float*, int64_t, hipStream_t);
+template int prefill_stream_apply<bf16_t, float>(const bf16_t*, int, int, int, int64_t, int64_t, int, int, const float*,
+                                                 float*, int64_t, hipStream_t);
+template int prefill_stream_apply<bf16_t, bf16_t>(const bf16_t*, int, int, int, int64_t, int64_t, int, int, const float*,
+                                                  bf16_t*, int64_t, hipStream_t);
+
+}  // namespace lrqk

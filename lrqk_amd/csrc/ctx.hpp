@@ -161,13 +161,30 @@ int score_select_diff(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const
                       uint8_t* evict, int32_t* miss_slots, int32_t* miss_count, int replace_all, hipStream_t st,
                       int32_t* miss_old = nullptr, const VictimView* vic = nullptr, int32_t* miss_new = nullptr,
                       bool want_new_idx = true);
-// Prefill iterations on Gram matrices (bf16 input, d = 128, r <= 32); see als_prefill_gram.hip.
-int prefill_gram_domain(lrqk_ctx* ctx, const void* q, const void* k, const float* partQ, const float* partK, int S,
-                        const float* a_q0, float* b_q, float* b_k, int b, int hq, int hkv, int64_t l, int r, int iters,
-                        float tol, int* flags, float** mt_q, float** mt_k, hipStream_t st);
-// A_K = K Mk with K read once per kv head (bf16 rows of 128); false: no kernel for this head grouping.
-bool prefill_apply_shared(const void* k, const float* mt_k, float* a_k, int b, int hq, int hkv, int64_t l, int r,
-                          hipStream_t st, int* rc_out);
+// Where a prefill factorisation leaves its results.  `storage`: in the inputs' type, else fp32.
+struct PrefillOut {
+  void* a_q;           // [bh][a_q_rows][r], the last a_q_rows rows (1 or all)
+  void* a_k;           // heads a_k_stride elements apart, rows of r
+  void* b_q;           // [bh][r][d]
+  void* b_k;
+  int64_t a_q_rows, a_k_stride;
+  bool storage;
+};
+// Prefill iterations on Gram matrices; see als_prefill_gram.hip.
+template <typename T>
+int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, float* a_k0, const PrefillOut& out, int b, int hq,
+                        int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st);
+// Its passes over the long axis; see als_prefill_stream.hip (every shape) and als_prefill.hip (bf16 rows of 128, r <= 32).
+template <typename T>
+int prefill_stream_sums(const T* x, int xh, int hq, int b, int64_t l, int r, int d, const float* a, float* part, int S,
+                        float* xtx, int Sx, hipStream_t st);
+template <typename T, typename OUT>
+int prefill_stream_apply(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, int d, const float* mt,
+                         OUT* a, int64_t a_stride, hipStream_t st);
+int prefill_given_sums_bf16(const bf16_t* x, int xh, int hq, int b, int64_t l, int r, float* a, float* part, int S,
+                            hipStream_t st);
+template <typename OUT>
+int prefill_store(const float* src, int64_t src_stride, OUT* dst, int64_t dst_stride, int64_t n, int heads, hipStream_t st);
 // The factor update with the ring append of (k_new, v_new) at slot `slot` as token `token` folded
 // into its first kernel.
 int als_decode_append(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64_t head_stride, int32_t* active_idx,

@@ -245,14 +245,7 @@ class LightAttentionIndicesFactory:
         seq_len = query_states.shape[2]
         k, L, g = self.attn_topk, self.num_lite_tokens, self.num_key_value_groups
         dev = query_states.device
-        from .factor import cast_lrqk_prefill
-        A_Q, B_Q, A_K, B_K = cast_lrqk_prefill(query_states, key_states, r=self.r, lambda_Q=self.weights[0],
-                                               lambda_K=self.weights[1], max_iter=self.max_iter[0], tol=self.tol[0],
-                                               init_method=self.init_aq_ak_method, init_factors=self.init_factors,
-                                               workspace=self.ws)
-        self.init_factors = None
-        self.sync_cache(B_Q, A_K, B_K)
-
+        A_Q = self._fit_prompt(query_states, key_states)
         if seq_len <= self.gpu_capacity:
             # k <= l <= k+L: everything stays resident, the first k tokens are the selected set
             self.KVcpu.append(key_states.narrow(2, 0, k), value_states.narrow(2, 0, k))
@@ -271,9 +264,9 @@ class LightAttentionIndicesFactory:
             self._active_idx[:, :, :seq_len] = torch.arange(seq_len, dtype=torch.int32, device=dev)
             self._hit_len = k
         else:
-            # the rows are scanned where they will live (same values as A_K, which sync_cache copied there): the
+            # the rows are scanned where they will live (A_K's rows in the growing buffer): the
             # score index that this first scan builds then stays valid for the decode steps
-            hit = self.compute_hit_indices(query_states=A_Q[:, :, -1:, :],
+            hit = self.compute_hit_indices(query_states=A_Q,
                                            key_states=self._A_K.data.narrow(2, 0, seq_len - L))
             self._hit_len = hit.shape[2]
             self._active_idx[:, :, :self._hit_len] = hit[..., 0].to(torch.int32)
@@ -285,7 +278,33 @@ class LightAttentionIndicesFactory:
             self.Kgpu[:, :, k:k + L, :] = repeat_kv(key_states.narrow(2, lb, L), g)
             self.Vgpu[:, :, k:k + L, :] = repeat_kv(value_states.narrow(2, lb, L), g)
             self._active_idx[:, :, k:] = torch.arange(lb, seq_len, dtype=torch.int32, device=dev)
-        self.last_A_Q_row = A_Q[:, :, -1:, :]
+        self.last_A_Q_row = A_Q
+
+    def _fit_prompt(self, query_states: torch.Tensor, key_states: torch.Tensor) -> torch.Tensor:
+        """The factorisation (lrqk_attention.py:1413-1424); leaves B_Q, B_K and the rows of A_K in the engine and returns
+        the last row of A_Q.  A_K is written where it will live and of A_Q only the last row is formed, unless the
+        factor buffer has a type of its own or a subclass takes the factors over."""
+        from .factor import _initial_factors, cast_lrqk_prefill
+        fit = dict(init_method=self.init_aq_ak_method, init_factors=self.init_factors)
+        self.init_factors = None
+        if self._A_K.device is None:
+            self._A_K.device = query_states.device
+        if self._A_K.dtype is None:
+            self._A_K.dtype = key_states.dtype
+        if self._A_K.dtype != query_states.dtype or self._is_overridden("sync_cache"):
+            A_Q, B_Q, A_K, B_K = cast_lrqk_prefill(query_states, key_states, r=self.r, max_iter=self.max_iter[0],
+                                                   tol=self.tol[0], workspace=self.ws, **fit)
+            self.sync_cache(B_Q, A_K, B_K)
+            return A_Q[:, :, -1:, :]
+        q = query_states.contiguous()
+        A_Q0, A_K0 = _initial_factors(q, key_states, self.r, **fit)
+        row0 = self._A_K.extend(A_K0.shape, q.shape[2], overwritten=True)
+        A_Q, self.B_Q, _, self.B_K = ops.als_prefill_store(self.ws, q, key_states, A_Q0, A_K0, self.max_iter[0], self.tol[0],
+                                                           a_k=self._A_K.data, row0=row0, last_query_row=True)
+        # rows of A_K were written: whatever the scan had indexed and the step had kept is dropped
+        self.ws.score_index(self.use_score_index)
+        self.ws.factor_state(self.use_factor_state)
+        return A_Q
 
     # From this size on the prompt's rows go to the host store through a DMA engine, beside the factorisation.  The
     # flush kernel holds the stream for bytes / 55 GB/s (38 us at this size); the copy needs a pass over the rows in

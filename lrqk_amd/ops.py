@@ -410,6 +410,33 @@ def als_prefill(ws: Workspace, q: torch.Tensor, k: torch.Tensor, a_q0: torch.Ten
     return a_q0, b_q, a_k0, b_k
 
 
+def als_prefill_store(ws: Workspace, q: torch.Tensor, k: torch.Tensor, a_q0: torch.Tensor, a_k0: torch.Tensor,
+                      max_iter: int, tol: float, a_k: Optional[torch.Tensor] = None, row0: int = 0,
+                      last_query_row: bool = False):
+    """The fit of als_prefill with its results in the inputs' type: (A_Q, B_Q, A_K, B_K).  A_K [b,Hq,l,r] goes to rows
+    row0 .. row0 + l of ``a_k`` [b,Hq,cap,r] if that is given (and A_K is then a view of it); with ``last_query_row``
+    A_Q is [b,Hq,1,r], its last row.  a_q0, a_k0 (fp32 [b,Hq,l,r]) are consumed."""
+    _need_cuda(q, k, a_q0, a_k0, a_k)
+    b, hq, l, d = q.shape
+    hkv = k.shape[1]
+    r = a_q0.shape[-1]
+    assert q.is_contiguous() and k.is_contiguous() and q.dtype == k.dtype
+    assert a_q0.dtype == torch.float32 and a_k0.dtype == torch.float32 and a_q0.is_contiguous() and a_k0.is_contiguous()
+    assert a_q0.shape == (b, hq, l, r) and a_k0.shape == (b, hq, l, r)
+    if a_k is None:
+        a_k, row0 = torch.empty((b, hq, l, r), dtype=q.dtype, device=q.device), 0
+    assert a_k.is_contiguous() and a_k.dtype == q.dtype and a_k.shape[:2] == (b, hq) and a_k.shape[3] == r
+    out = a_k.narrow(2, row0, l)
+    a_q = torch.empty((b, hq, 1 if last_query_row else l, r), dtype=q.dtype, device=q.device)
+    b_q = torch.empty((b, hq, r, d), dtype=q.dtype, device=q.device)
+    b_k = torch.empty((b, hq, r, d), dtype=q.dtype, device=q.device)
+    check(_lib.load().lrqk_als_prefill_store(ws.handle, q.data_ptr(), k.data_ptr(), a_q0.data_ptr(), a_k0.data_ptr(),
+                                             a_q.data_ptr(), a_q.shape[2], out.data_ptr(), a_k.shape[2] * r, b_q.data_ptr(),
+                                             b_k.data_ptr(), b, hq, hkv, l, r, d, int(max_iter), float(tol), _dt(q),
+                                             _stream(q)))
+    return a_q, b_q, out, b_k
+
+
 def decode_step(ws: Workspace, b_q, b_k, a_k, active_idx, k_act, v_act, kv_store, q, k_new, v_new, *, topk: int,
                 lite: int, ring_slot: int, token: int, m: int, flush_row0: int, max_iter: int, tol: float,
                 round_scores: bool, no_hit_miss: bool, q_hat, k_hat, attn_out=None, evict=None, miss_count=None):

@@ -61,3 +61,41 @@ def test_prompt_rows_to_the_host_store(ops, heads, l, d, dtype):
     assert (store[:, :, :5] == -7).all() and (store[:, :, 5 + l:] == -7).all()
     with pytest.raises(ValueError):
         ops.store_rows(rows, store, 10, side)
+
+
+@pytest.mark.parametrize("dtype,d,r,l,hq,hkv,iters", [
+    (torch.float32, 64, 1, 128, 2, 2, 1),        # the fewest rows the Gram matrices take, one column of factors
+    (torch.float32, 64, 16, 129, 6, 2, 2),       # a row beyond whole groups; three query heads per kv head
+    (torch.float32, 128, 17, 1000, 4, 4, 2),     # the first rank that is padded to two tiles
+    (torch.bfloat16, 64, 32, 4097, 4, 1, 3),     # more than one split
+    (torch.bfloat16, 64, 33, 515, 2, 1, 2),      # the first rank that is padded to four tiles
+    (torch.bfloat16, 128, 48, 257, 8, 2, 3),
+    (torch.float32, 128, 64, 2531, 2, 1, 4),
+    (torch.bfloat16, 128, 64, 9001, 2, 1, 4),
+    (torch.float32, 128, 40, 700, 2, 1, 0),      # no iteration: the given factors are the result
+])
+def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
+    """Every instance of the streaming kernels and of the fp64 iteration (row widths 64 and 128, ranks padded to 16, 32
+    and 64, fp32 and bf16 rows) against the oracle in fp64.  Limit: a sum of up to 1024 rows per wave adds 32 group sums
+    in fp32, each group exact to 2^-24 times its terms, so the sums are off by at most 34 x 2^-24 = 2e-6 of their
+    terms; random rows of rank above r keep the systems within a factor of ten of that."""
+    from lrqk_amd import synth
+    gen = torch.Generator().manual_seed(l + r)
+    Q, _ = synth.low_rank_noise(gen, 1, hq, l, d, min(d, 2 * r), 0.05, dtype)
+    K, _ = synth.low_rank_noise(gen, 1, hkv, l, d, min(d, 2 * r), 0.05, dtype)
+    A0 = torch.randn((1, hq, l, r), generator=gen)
+    A1 = torch.randn((1, hq, l, r), generator=gen)
+    ws = ops.Workspace()
+    got = ops.als_prefill(ws, Q.to(DEV), K.to(DEV), A0.to(DEV), A1.to(DEV), iters, 0.0)
+    ref = oracle.als_prefill_w1(Q.double(), oracle.repeat_kv(K, hq // hkv).double(), A0.double(), A1.double(), iters, 0.0)
+    for name, g, w in zip(("A_Q", "B_Q", "A_K", "B_K"), got, ref):
+        off = float((g.cpu().double() - w).norm() / w.norm())
+        print(f"{name}: {off:.2e}", flush=True)
+        assert off < 2e-5, name
+    # the same fit into a cache's buffers: the same numbers in the rows' type, nothing beside them touched
+    buf = torch.full((1, hq, l + 7, r), 9.0, dtype=dtype, device=DEV)
+    a_q, b_q, a_k, b_k = ops.als_prefill_store(ws, Q.to(DEV), K.to(DEV), A0.to(DEV), A1.to(DEV), iters, 0.0, a_k=buf, row0=3,
+                                               last_query_row=True)
+    assert torch.equal(a_q, got[0][:, :, -1:].to(dtype)) and torch.equal(buf[:, :, 3:3 + l], got[2].to(dtype))
+    assert torch.equal(b_q, got[1].to(dtype)) and torch.equal(b_k, got[3].to(dtype))
+    assert (buf[:, :, :3] == 9).all() and (buf[:, :, 3 + l:] == 9).all()
