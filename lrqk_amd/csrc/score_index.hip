@@ -4,6 +4,7 @@
 
 #include "common.hpp"
 #include "ctx.hpp"
+#include "prefill_pieces.hpp"
 
 namespace lrqk {
 
@@ -13,117 +14,165 @@ namespace lrqk {
 // one workgroup per head adds the parts and factors.  Anything degenerate (no rows, zero or
 // non-finite S, a non-positive pivot) gives W = I.
 constexpr int kSidxSample = 4096;
-constexpr int kSidxTile = 64;   // sample rows per LDS tile
 constexpr int kSidxParts = 16;  // workgroups per head in the first launch
+typedef float sidx_v16f __attribute__((ext_vector_type(16)));
+
+// Sums over a part's rows on the fp32 matrix pipe (32x32x2, two rows per product): lane (m, kh) holds element m of row
+// 2 kk + kh as both operands, so the rows go from memory straight into the product, eight products' worth requested at
+// a time.  Bound by the latency of those reads (a part is 256 rows): 158 us as 64-term chains on the vector ALUs with
+// two LDS reads each, 18 us here, at 32 heads and R = 64.
 template <typename T, int R>
 __global__ __launch_bounds__(256) void score_index_moments_kernel(const T* __restrict__ a_k, int64_t head_stride,
                                                                   int64_t rows, float* __restrict__ part) {
-  constexpr int LD = R + 1;
-  constexpr int EPT = (R * R + 255) / 256;  // entries of S per thread
-  __shared__ float tile[kSidxTile][LD];
+  constexpr int NT = (R + 31) / 32, NP = NT * (NT + 1) / 2;  // 32-column tiles; tile pairs on and above the diagonal
+  __shared__ float red[4][1024];
   const int h = blockIdx.y, p = blockIdx.x, tid = threadIdx.x;
+  const int lane = lane_id(), wave = wave_id(), m = lane & 31, kh = lane >> 5;
   const T* A = a_k + (int64_t)h * head_stride;
   const int64_t step = rows > 0 ? (rows + kSidxSample - 1) / kSidxSample : 1;
   const int64_t n = rows > 0 ? (rows + step - 1) / step : 0;  // sample size
   const int64_t per = (n + kSidxParts - 1) / kSidxParts;
   const int64_t n0 = min(n, p * per), n1 = min(n, n0 + per);
-  float acc[EPT];
+  sidx_v16f acc[NP];
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) acc[e] = 0.0f;
-  for (int64_t t0 = n0; t0 < n1; t0 += kSidxTile) {
-    const int cnt = (int)min((int64_t)kSidxTile, n1 - t0);
-    __syncthreads();
-    for (int x = tid; x < kSidxTile * R; x += 256) {
-      const int rr = x / R, c = x % R;
-      tile[rr][c] = rr < cnt ? ld_f32<T>(A, (t0 + rr) * step * R + c) : 0.0f;
-    }
-    __syncthreads();
+  for (int q = 0; q < NP; ++q)
 #pragma unroll
-    for (int e = 0; e < EPT; ++e) {
-      const int x = tid + e * 256;
-      if (x < R * R) {
-        const int i = x / R, j = x % R;
-        float sum = acc[e];
-        for (int rr = 0; rr < kSidxTile; ++rr) sum = fmaf(tile[rr][i], tile[rr][j], sum);
-        acc[e] = sum;
+    for (int v = 0; v < 16; ++v) acc[q][v] = 0.0f;
+  constexpr int U = 8;  // products in flight: 16 rows of this wave
+  for (int64_t t0 = n0 + wave * 2 * U; t0 < n1; t0 += 4 * 2 * U) {
+    float x[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t t = t0 + 2 * u + kh;
+#pragma unroll
+      for (int c = 0; c < NT; ++c) {
+        const float f = ld_f32<T>(A, min(t, n1 - 1) * step * R + min(32 * c + m, R - 1));
+        x[u][c] = t < n1 && 32 * c + m < R ? f : 0.0f;
       }
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < NT; ++c)
+#pragma unroll
+        for (int c2 = 0; c2 <= c; ++c2)
+          acc[c * (c + 1) / 2 + c2] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u][c2], x[u][c], acc[c * (c + 1) / 2 + c2], 0, 0, 0);
   }
   float* out = part + ((int64_t)h * kSidxParts + p) * R * R;
 #pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    const int x = tid + e * 256;
-    if (x < R * R) out[x] = acc[e];
-  }
+  for (int c = 0; c < NT; ++c)
+#pragma unroll
+    for (int c2 = 0; c2 <= c; ++c2) {
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < 16; ++v) red[wave][((v >> 2) * 8 + kh * 4 + (v & 3)) * 32 + m] = acc[c * (c + 1) / 2 + c2][v];
+      __syncthreads();
+      for (int x = tid; x < 1024; x += 256) {
+        const int i = 32 * c2 + (x >> 5), j = 32 * c + (x & 31);
+        if (i >= R || j >= R) continue;
+        const float sum = (red[0][x] + red[1][x]) + (red[2][x] + red[3][x]);
+        out[i * R + j] = sum;
+        if (c != c2) out[j * R + i] = sum;
+      }
+    }
 }
 
+// L^-1 by elimination of [S | I]: step c scales row c of the right half by 1 / sqrt(pivot) and takes l_i times it (and
+// l_i l_j on the left) off the rows below.  A thread of the 16 x 16 grid keeps rows ti + 16 a, columns tj + 16 b of both
+// halves in registers; the pivot column and row go round through LDS, one barrier per step (Cholesky in LDS with three
+// barriers per column and a substitution with one column per thread: 140 us at R = 64, 15 us at R = 16; 37 and 7 us here).
 template <int R>
 __global__ __launch_bounds__(256) void score_index_factor_kernel(const float* __restrict__ part, int64_t rows,
                                                                  float* __restrict__ wm) {
-  constexpr int LD = R + 1;
-  __shared__ float S[R][LD];
-  __shared__ float X[R][LD];
-  __shared__ int bad;
+  constexpr int N = R / 16;
+  __shared__ float colp[2][R];  // the pivot column of S
+  __shared__ float rowx[2][R];  // the pivot row of the right half
+  __shared__ float diag[R];
   const int h = blockIdx.x, tid = threadIdx.x;
+  const int ti = tid >> 4, tj = tid & 15;
   float* W = wm + (int64_t)h * (R * R + R);
   const int64_t step = rows > 0 ? (rows + kSidxSample - 1) / kSidxSample : 1;
   const int64_t n = rows > 0 ? (rows + step - 1) / step : 0;
-  if (tid == 0) bad = 0;
-  for (int x = tid; x < R * R; x += 256) {
-    float sum = 0.0f;
-    for (int p = 0; p < kSidxParts; ++p) sum += part[((int64_t)h * kSidxParts + p) * R * R + x];
-    S[x / R][x % R] = n > 0 ? sum / (float)n : 0.0f;
-  }
+  const float inv_n = n > 0 ? 1.0f / (float)n : 0.0f;
+  float S[N][N], X[N][N];
+  const float* ph = part + (int64_t)h * kSidxParts * R * R;
+#pragma unroll
+  for (int a = 0; a < N; ++a)
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      const int x = (ti + 16 * a) * R + tj + 16 * b;
+      float sum = 0.0f;
+#pragma unroll
+      for (int p = 0; p < kSidxParts; ++p) sum += ph[(int64_t)p * R * R + x];
+      S[a][b] = sum * inv_n;
+      X[a][b] = ti == tj && a == b ? 1.0f : 0.0f;
+      if (ti == tj && a == b) diag[ti + 16 * a] = S[a][b];
+    }
   __syncthreads();
   float tr = 0.0f;
-  for (int i = 0; i < R; ++i) tr += S[i][i];
+  for (int i = 0; i < R; ++i) tr += diag[i];
   // (1 % of the mean diagonal: directions that hold next to nothing are not blown up to unit size, where their
   // quantisation step would only add slack to the bound; 12 % fewer rows to rescore than with 0.01 % on the 128K stream)
   const float ridge = 1e-2f * tr / (float)R;
-  if (!(tr > 0.0f && tr < INFINITY) && tid == 0) bad = 1;
-  __syncthreads();
-  if (tid < R) S[tid][tid] += ridge;
-  // Cholesky, column by column (lower triangle of S becomes L)
-  for (int c = 0; c < R; ++c) {
-    __syncthreads();
-    const float piv = S[c][c];
-    if (!(piv > 0.0f && piv < INFINITY)) {
-      if (tid == 0) bad = 1;
-      break;  // uniform: every thread reads the same pivot
-    }
-    const float d = sqrtf(piv);
-    __syncthreads();
-    if (tid == 0) S[c][c] = d;
-    if (tid > c && tid < R) S[tid][c] /= d;
-    __syncthreads();
-    for (int x = tid; x < R * R; x += 256) {
-      const int i = x / R, j = x % R;
-      if (j > c && i >= j) S[i][j] -= S[i][c] * S[j][c];
+  bool bad = !(tr > 0.0f && tr < INFINITY);
+  if (ti == tj) {
+#pragma unroll
+    for (int a = 0; a < N; ++a) S[a][a] += ridge;
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+#pragma unroll 1
+    for (int t = 0; t < 16; ++t) {
+      const int c = 16 * k + t, buf = t & 1;  // (two slots: whoever passes a step's barrier has read the slot before)
+      if (tj == t) {
+#pragma unroll
+        for (int a = 0; a < N; ++a) colp[buf][ti + 16 * a] = S[a][k];
+      }
+      if (ti == t) {
+#pragma unroll
+        for (int b = 0; b < N; ++b) rowx[buf][tj + 16 * b] = X[k][b];
+      }
+      __syncthreads();
+      const float piv = colp[buf][c];
+      bad = bad || !(piv > 0.0f && piv < INFINITY);
+      const float inv = 1.0f / sqrtf(piv);
+      float li[N], lj[N], xr[N];
+#pragma unroll
+      for (int a = 0; a < N; ++a) {
+        li[a] = ti + 16 * a > c ? colp[buf][ti + 16 * a] * inv : 0.0f;
+        lj[a] = colp[buf][tj + 16 * a] * inv;
+        xr[a] = rowx[buf][tj + 16 * a] * inv;
+      }
+      if (ti == t) {
+#pragma unroll
+        for (int b = 0; b < N; ++b) X[k][b] = xr[b];
+      }
+#pragma unroll
+      for (int a = 0; a < N; ++a)
+#pragma unroll
+        for (int b = 0; b < N; ++b) {
+          S[a][b] = fmaf(-li[a], lj[b], S[a][b]);
+          X[a][b] = fmaf(-li[a], xr[b], X[a][b]);
+        }
     }
   }
-  __syncthreads();
-  // X = L^-1 by forward substitution, one column per thread
-  if (!bad && tid < R) {
-    const int c = tid;
-    for (int i = 0; i < R; ++i) X[i][c] = 0.0f;
-    X[c][c] = 1.0f / S[c][c];
-    for (int i = c + 1; i < R; ++i) {
-      float sum = 0.0f;
-      for (int k = c; k < i; ++k) sum = fmaf(S[i][k], X[k][c], sum);
-      X[i][c] = -sum / S[i][i];
+#pragma unroll
+  for (int a = 0; a < N; ++a)
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      const int i = ti + 16 * a, j = tj + 16 * b;
+      if (j <= i) bad = bad || !(fabsf(X[a][b]) < INFINITY) || (i == j && !(X[a][b] > 0.0f));
     }
-    for (int i = c; i < R; ++i)
-      if (!(fabsf(X[i][c]) < INFINITY)) bad = 1;
-    if (!(X[c][c] > 0.0f)) bad = 1;
-  }
-  __syncthreads();
-  const bool ident = bad != 0;
-  // W[i][j] = X[j][i] for i <= j, zero below the diagonal; then 1 / W_jj
-  for (int x = tid; x < R * R; x += 256) {
-    const int i = x / R, j = x % R;
-    W[x] = ident ? (i == j ? 1.0f : 0.0f) : (i <= j ? X[j][i] : 0.0f);
-  }
-  if (tid < R) W[R * R + tid] = ident ? 1.0f : 1.0f / X[tid][tid];
+  const bool ident = __syncthreads_or(bad) != 0;
+  // W[i][j] = L^-1[j][i] for i <= j, zero below the diagonal; then 1 / W_jj
+#pragma unroll
+  for (int a = 0; a < N; ++a)
+#pragma unroll
+    for (int b = 0; b < N; ++b) {
+      const int j = ti + 16 * a, i = tj + 16 * b;
+      W[i * R + j] = ident ? (i == j ? 1.0f : 0.0f) : (i <= j ? X[a][b] : 0.0f);
+      if (i == j) W[R * R + j] = ident ? 1.0f : 1.0f / X[a][b];
+    }
 }
 
 // One wave per row: lane i holds element i of the row, and column `lane` of W stays in registers.
@@ -147,18 +196,25 @@ __global__ __launch_bounds__(256) void score_index_build_kernel(const T* __restr
   }
 }
 
-// r = 32: the transform of 32 rows is one 32x32x32 product on the fp32 matrix pipe (16 steps of
-// mfma 32x32x2), and a second one on absolute values gives g.  Lane (m, kh) = (lane & 31, lane >> 5)
-// feeds A[m][2 kk + kh] (row m of the group) and B[2 kk + kh][m] (W); it receives, for v = 0..15,
-// C[row(v)][m] with row(v) = (v / 4) * 8 + kh * 4 + v % 4.  Any summation order inside the pipe
-// stays within the rounding bound the scale charges for.
-typedef float sidx_v16f __attribute__((ext_vector_type(16)));
-template <typename T>
-__global__ __launch_bounds__(256) void score_index_build32_kernel(const T* __restrict__ a_k, int64_t head_stride,
-                                                                  int64_t row0, int64_t row1, uint8_t* __restrict__ qa,
-                                                                  uint16_t* __restrict__ qs, const float* __restrict__ wm,
-                                                                  int64_t head_rows) {
-  constexpr int R = 32, VEC = Vec16<T>::N;
+// Many rows at a time: C^T = W^T A^T on the matrix cores, and a second product on absolute values for g.  A lane's
+// operand on the right is eight consecutive elements of one row as they lie in memory, and what it receives are 16 of
+// the 32 columns of that row's a' (column 8 (v / 4) + 4 (lane / 32) + v % 4 in element v): the maxima over a row are
+// taken in the lane, with one exchange between the wave's halves, and the codes leave as words of four.
+// bf16 rows: W as three bf16 pieces (products exact in fp32), |W| for g rounded up to one piece; fp32 rows: the fp32
+// pipe (32x32x2), a half of the wave taking a half of the row.  Any summation order inside the pipes
+// stays within the rounding bound the scale charges for, and a g that is too large by 2^-7 only loosens it.
+// Bound by HBM (a row read and R + 2 bytes written): 16384 rows of 64 elements, 32 heads: 101 MB in 46 us (253 us
+// with a wave per row); 131072 rows of 32: 411 MB in 111 us (454 us with the rows on the other side of the product
+// and two wave reductions per row).
+template <typename T, int R>
+__global__ __launch_bounds__(256) void score_index_build_rows_kernel(const T* __restrict__ a_k, int64_t head_stride,
+                                                                     int64_t row0, int64_t row1, uint8_t* __restrict__ qa,
+                                                                     uint16_t* __restrict__ qs, const float* __restrict__ wm,
+                                                                     int64_t head_rows) {
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int NT = (R + 31) / 32;               // 32-column tiles of a'
+  constexpr int KB = F32 ? R / 2 : R / 16;        // products per tile (and piece)
+  constexpr int NV = R < 32 ? R / 2 : 16;         // elements of a tile that a lane uses
   const int h = blockIdx.y;
   const int lane = lane_id(), m = lane & 31, kh = lane >> 5;
   const int64_t ngroups = (row1 - row0 + 31) / 32;
@@ -166,48 +222,96 @@ __global__ __launch_bounds__(256) void score_index_build32_kernel(const T* __res
   const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / kWave);
   const T* A = a_k + (int64_t)h * head_stride;
   const float* W = wm + (int64_t)h * (R * R + R);
-  float wb[16], wba[16];
+  // left operands: row j = 32 t + m of W^T
+  float wf[F32 ? NT : 1][F32 ? KB : 1];
+  gd_bf16x8 wp[F32 ? 1 : NT][F32 ? 1 : KB][3], wg[F32 ? 1 : NT][F32 ? 1 : KB];
 #pragma unroll
-  for (int kk = 0; kk < 16; ++kk) {
-    wb[kk] = W[(2 * kk + kh) * R + m];
-    wba[kk] = fabsf(wb[kk]);
-  }
-  for (int64_t grp = wave0; grp < ngroups; grp += nwaves) {
-    const int64_t r0 = row0 + grp * 32;
-    const int64_t row = min(r0 + m, row1 - 1);
-    float f[R];
-    {
-      Vec16<T> v[R / VEC];
+  for (int t = 0; t < NT; ++t) {
+    const int j = min(32 * t + m, R - 1);
+    const bool live = 32 * t + m < R;
+    if constexpr (F32) {
 #pragma unroll
-      for (int c = 0; c < R / VEC; ++c) v[c].load(A + row * R + c * VEC);
+      for (int k = 0; k < KB; ++k) wf[t][k] = live ? W[(kh * KB + k) * R + j] : 0.0f;
+    } else {
 #pragma unroll
-      for (int c = 0; c < R / VEC; ++c) v[c].unpack(f + c * VEC);
-    }
-    sidx_v16f acc, accg;
+      for (int k = 0; k < KB; ++k) {
+        float f[8];
+        uint32_t g[8];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = accg[v] = 0.0f;
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const float a = kh ? f[2 * kk + 1] : f[2 * kk];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, wb[kk], acc, 0, 0, 0);
-      accg = __builtin_amdgcn_mfma_f32_32x32x2f32(fabsf(a), wba[kk], accg, 0, 0, 0);
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      // maxima over the 32 columns of this half-wave's row
-      float mx = row_reduce(fabsf(acc[v]), [](float x, float y) { return fmaxf(x, y); });
-      float gx = row_reduce(accg[v], [](float x, float y) { return fmaxf(x, y); });
-      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-      gx = fmaxf(gx, __shfl_xor(gx, 16, kWave));
-      const unsigned long long okm = __ballot(accg[v] < INFINITY);  // false for NaN and infinity
-      const bool ok = (uint32_t)(kh ? okm >> 32 : okm) == 0xffffffffu;
-      const float scale = score_index_scale(mx, ok ? gx : INFINITY, R);
-      const uint8_t u = score_index_code(acc[v], 1.0f / scale);
-      const int64_t orow = r0 + (v >> 2) * 8 + kh * 4 + (v & 3);
-      if (orow < row1) {
-        qa[((int64_t)h * head_rows + orow) * R + m] = u;
-        if (m == 0) qs[(int64_t)h * head_rows + orow] = sidx_scale_bits(scale);
+        for (int q = 0; q < 8; ++q) {
+          f[q] = live ? W[(16 * k + 8 * kh + q) * R + j] : 0.0f;
+          g[q] = __float_as_uint(fabsf(f[q]));
+          g[q] += g[q] < 0x7f000000u ? 0xffffu : 0u;  // (truncated below: the next bf16 number up)
+        }
+        gd_split3x8(f, wp[t][k]);
+        typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+        wg[t][k] = __builtin_bit_cast(gd_bf16x8, v4u{gd_pack2(g[0], g[1]), gd_pack2(g[2], g[3]), gd_pack2(g[4], g[5]),
+                                                     gd_pack2(g[6], g[7])});
       }
+    }
+  }
+  constexpr int NLD = F32 ? R / 8 : KB;  // 16-byte loads per lane and group
+  gd_u32x4 pre[NLD];
+  auto issue = [&](int64_t grp) {
+    const T* src = A + min(row0 + grp * 32 + m, row1 - 1) * R;
+#pragma unroll
+    for (int c = 0; c < NLD; ++c)
+      pre[c] = *reinterpret_cast<const gd_u32x4*>(src + (F32 ? kh * (R / 2) + 4 * c : 16 * c + 8 * kh));
+  };
+  if (wave0 < ngroups) issue(wave0);
+  for (int64_t grp = wave0; grp < ngroups; grp += nwaves) {
+    gd_u32x4 cur[NLD];
+#pragma unroll
+    for (int c = 0; c < NLD; ++c) cur[c] = pre[c];
+    if (grp + nwaves < ngroups) issue(grp + nwaves);
+    sidx_v16f acc[NT], accg[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[t][v] = accg[t][v] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KB; ++k) {
+        if constexpr (F32) {
+          const float x = __uint_as_float(cur[k / 4][k % 4]);
+          acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[t][k], x, acc[t], 0, 0, 0);
+          accg[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(fabsf(wf[t][k]), fabsf(x), accg[t], 0, 0, 0);
+        } else {
+          const gd_bf16x8 x = __builtin_bit_cast(gd_bf16x8, cur[k]);
+          const gd_bf16x8 xa = __builtin_bit_cast(gd_bf16x8, cur[k] & 0x7fff7fffu);
+#pragma unroll
+          for (int p = 2; p >= 0; --p) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wp[t][k][p], x, acc[t], 0, 0, 0);
+          accg[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wg[t][k], xa, accg[t], 0, 0, 0);
+        }
+      }
+    }
+    float mx = 0.0f, gx = 0.0f;
+    bool ok = true;  // false for NaN and infinity anywhere in the row
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        mx = fmaxf(mx, fabsf(acc[t][v]));
+        gx = fmaxf(gx, accg[t][v]);
+        ok = ok && accg[t][v] < INFINITY;
+      }
+    if (!ok) gx = INFINITY;
+    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    gx = fmaxf(gx, __shfl_xor(gx, 32, kWave));
+    const float scale = score_index_scale(mx, gx, R);
+    const float inv = 1.0f / scale;
+    const int64_t row = row0 + grp * 32 + m;
+    if (row < row1) {
+      uint32_t* dst = reinterpret_cast<uint32_t*>(qa + ((int64_t)h * head_rows + row) * R);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int q = 0; q < NV / 4; ++q) {
+          uint32_t w = 0;
+#pragma unroll
+          for (int b = 0; b < 4; ++b) w |= (uint32_t)score_index_code(acc[t][4 * q + b], inv) << (8 * b);
+          dst[8 * t + 2 * q + kh] = w;
+        }
+      if (kh == 0) qs[(int64_t)h * head_rows + row] = sidx_scale_bits(scale);
     }
   }
 }
@@ -222,9 +326,10 @@ static void launch_build(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, in
                        (const T*)a_k, head_stride, upto, part);
     hipLaunchKernelGGL((score_index_factor_kernel<R>), dim3((unsigned)bh), dim3(256), 0, st, (const float*)part, upto, wm);
   }
-  if (R == 32 && upto - from >= 32) {
-    const unsigned blocks = (unsigned)std::min<int64_t>(1024, (upto - from + 127) / 128);
-    hipLaunchKernelGGL((score_index_build32_kernel<T>), dim3(blocks, (unsigned)bh), dim3(256), 0, st, (const T*)a_k,
+  if (upto - from >= 32) {
+    // (every wave loads and splits W: about four of its 32-row groups per wave, at most what the GPU holds at a time)
+    const unsigned blocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 2048 / bh), (upto - from + 511) / 512));
+    hipLaunchKernelGGL((score_index_build_rows_kernel<T, R>), dim3(blocks, (unsigned)bh), dim3(256), 0, st, (const T*)a_k,
                        head_stride, from, upto, (uint8_t*)ctx->sidx_qa.p, (uint16_t*)ctx->sidx_qs.p, wm, head_rows);
     return;
   }

@@ -99,3 +99,29 @@ def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
     assert torch.equal(a_q, got[0][:, :, -1:].to(dtype)) and torch.equal(buf[:, :, 3:3 + l], got[2].to(dtype))
     assert torch.equal(b_q, got[1].to(dtype)) and torch.equal(b_k, got[3].to(dtype))
     assert (buf[:, :, :3] == 9).all() and (buf[:, :, 3 + l:] == 9).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("r,m", [(16, 1025), (16, 4127), (32, 1056), (32, 9001), (64, 1060), (64, 5000)])
+def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
+    """The index of many rows at once (whole and partial groups of 32, every rank that has one): the selections are
+    those of the plain scan, also with rows that are zero, huge, infinite or not numbers, and the bounds are tight
+    enough that most rows are never looked at again."""
+    gen = torch.Generator(device=DEV).manual_seed(m + r)
+    mix = torch.randn((r, r), generator=gen, device=DEV)
+    a_k = (torch.randn((1, 3, m + 5, r), generator=gen, device=DEV) @ mix).to(dtype)
+    a_k[:, 0, 7] = 0
+    a_k[:, 1, 40] *= 3e4
+    a_k[:, 2, 33, 1] = float("inf")
+    a_k[:, 2, 64, 0] = float("nan")
+    q0 = torch.randn((1, 3, 1, r), generator=gen, device=DEV)
+    plain, indexed = ops.Workspace(), ops.Workspace()
+    indexed.score_index(True)
+    for step in range(3):   # (the first scan has no bound yet: every row is a candidate)
+        q = (q0 + 0.05 * step).to(dtype)
+        want = ops.score_select(plain, a_k, q, m, 100)
+        got = ops.score_select(indexed, a_k, q, m, 100)
+        assert torch.equal(got, want), step
+    rows, rescored = indexed.scan_stats()
+    print(f"rescored {rescored} of {rows}", flush=True)
+    assert rows == 3 * m and rescored < rows // 3
