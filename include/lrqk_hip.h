@@ -187,6 +187,12 @@ int lrqk_last_iterates(lrqk_ctx* ctx, double* out, int64_t n_doubles, int* bh, i
 int lrqk_gather_rows(const void* src, int64_t src_len, const int32_t* idx, int64_t idx_stride, int count,
                      void* dst, int n_slots, int b, int hq, int hkv, int d, int dtype, void* stream);
 
+/* py:1467-1504 -- the active set of a prompt of l >= topk + lite tokens: slots [0, topk) of k_act / v_act
+ * ([bh][topk + lite][d]) take the rows of k, v ([b][hkv][l][d] on the device) at active_idx[bh][0..topk), slots
+ * [topk, topk + lite) those of the last lite tokens, whose ids are written to active_idx. */
+int lrqk_fill_active(const void* k, const void* v, int64_t l, int32_t* active_idx, void* k_act, void* v_act, int topk,
+                     int lite, int b, int hq, int hkv, int d, int dtype, void* stream);
+
 /* py:1133-1135, 1185-1188 -- write the new token's k,v ([b][hkv][d]) into ring slot `slot`
  * of every query head and record its token id in active_idx[bh][slot]. */
 int lrqk_append_token(const void* k_new, const void* v_new, void* k_act, void* v_act, int n_slots, int slot,

@@ -64,6 +64,7 @@ def _sig(lib):
         "lrqk_ctx_factor_state": ([vp, i32], i32),
         "lrqk_last_iterates": ([vp, vp, i64, c.POINTER(i32), c.POINTER(i32), c.POINTER(i32), c.POINTER(i64)], i32),
         "lrqk_gather_rows": ([vp, i64, vp, i64, i32, vp, i32, i32, i32, i32, i32, i32, vp], i32),
+        "lrqk_fill_active": ([vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, vp], i32),
         "lrqk_append_token": ([vp, vp, vp, vp, i32, i32, vp, i64, i32, i32, i32, i32, i32, i32, vp], i32),
         "lrqk_flush_ring": ([vp, vp, i32, i32, i32, vp, i64, i64, i32, i32, i32, i32, i32, vp], i32),
         "lrqk_interleave_kv": ([vp, vp, vp, i32, i64, i32, i32, vp], i32),

@@ -56,6 +56,7 @@ extern "C" int lrqk_ctx_destroy(lrqk_ctx* ctx) {
   if (!ctx) return LRQK_OK;
   if (ctx->pool.must_wait() || ctx->stage_host || ctx->side || ctx->tev) (void)hipDeviceSynchronize();
   ctx->each_buf([](DevBuf& b) { b.release(); });
+  ctx->pool.close();
   if (ctx->stage_host) (void)hipHostFree(ctx->stage_host);
   if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
   if (ctx->side) (void)hipStreamDestroy(ctx->side);

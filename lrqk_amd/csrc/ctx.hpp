@@ -1,6 +1,7 @@
 // Library-owned device workspace.
 #pragma once
 #include <atomic>
+#include <vector>
 #include <hip/hip_runtime.h>
 
 #include "common.hpp"
@@ -27,38 +28,63 @@ struct BufPool {
   // Work queued on `stream` may still read a block that goes back.  A stream-ordered allocator hands it out again on
   // that stream only, so nothing has to wait unless another stream was used in between; the runtime's blocks wait.
   bool must_wait() const { return !alloc || mixed; }
+
+  void* take(size_t bytes) {
+    if (alloc) return alloc(bytes, (void*)stream, user);
+    void* p = nullptr;
+    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+  }
+  void give(void* p) {
+    if (alloc)
+      release(p, user);
+    else
+      (void)hipFree(p);
+  }
+  // Small blocks are cut from chunks that stay until the ctx goes: a dozen of a new ctx's buffers have a few hundred KB
+  // each, and a call of the caller's allocator is about 5 us of a prompt's host time.  (A buffer that grows leaves its
+  // old piece behind; it grows by a quarter at least.)
+  static constexpr size_t kChunk = 4u << 20, kSmall = 1u << 20;
+  std::vector<void*> chunks;
+  size_t chunk_left = 0;
+  void* small(size_t bytes) {
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (bytes > chunk_left) {
+      void* c = take(kChunk);
+      if (!c) return nullptr;
+      chunks.push_back(c);
+      chunk_left = kChunk;
+    }
+    chunk_left -= bytes;
+    return (char*)chunks.back() + chunk_left;
+  }
+  void close() {
+    for (void* c : chunks) give(c);
+    chunks.clear();
+    chunk_left = 0;
+  }
 };
 
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  bool small = false;  // a piece of one of the pool's chunks
   BufPool* pool = nullptr;
   // Grows (never shrinks); the contents are not kept.
   int ensure(size_t need) {
     if (need <= bytes) return LRQK_OK;
-    size_t want = need + need / 4;
-    void* np = nullptr;
-    if (pool->alloc) {
-      np = pool->alloc(want, (void*)pool->stream, pool->user);
-      if (!np) return set_error(LRQK_EHIP, "the caller's allocator has no %zu bytes", want);
-    } else {
-      LRQK_HIP_CHECK(hipMalloc(&np, want));
-    }
-    if (p) {
-      if (pool->must_wait()) LRQK_HIP_CHECK(hipDeviceSynchronize());
-      release();
-    }
+    const size_t want = need + need / 4;
+    const bool s = want <= BufPool::kSmall;
+    void* np = s ? pool->small(want) : pool->take(want);
+    if (!np) return set_error(LRQK_EHIP, "no %zu bytes of device memory", want);
+    if (p && !small && pool->must_wait()) LRQK_HIP_CHECK(hipDeviceSynchronize());
+    release();
     p = np;
     bytes = want;
+    small = s;
     return LRQK_OK;
   }
   void release() {
-    if (p) {
-      if (pool->alloc)
-        pool->release(p, pool->user);
-      else
-        (void)hipFree(p);
-    }
+    if (p && !small) pool->give(p);
     p = nullptr;
     bytes = 0;
   }

@@ -188,6 +188,33 @@ __global__ __launch_bounds__(256) void interleave_kv_kernel(const uint4* __restr
   }
 }
 
+// The active set of a prompt in one launch: slots [0, k) take the K and V rows of the selected tokens, slots
+// [k, k + lite) the last `lite` tokens' rows and their ids.  The rows come from the prompt's own K, V on the device.
+__global__ __launch_bounds__(256) void fill_active_kernel(const uint4* __restrict__ k_src, const uint4* __restrict__ v_src,
+                                                          int64_t l, int32_t* __restrict__ idx, uint4* __restrict__ k_act,
+                                                          uint4* __restrict__ v_act, int k, int lite, int hq, int hkv,
+                                                          int cpr) {
+  const int h = blockIdx.y, n = k + lite;
+  const int64_t src0 = ((int64_t)(h / hq) * hkv + (h % hq) / (hq / hkv)) * l;
+  int32_t* ids = idx + (int64_t)h * n;
+  const int chunks = 2 * cpr;
+  const int tpb = max(1, 256 / chunks);  // slots per workgroup and round
+  for (int c0 = 0; c0 < chunks; c0 += 256) {
+    const int t = threadIdx.x / chunks, c = c0 + threadIdx.x - t * chunks;
+    if (t >= tpb || c >= chunks) continue;
+    for (int slot = blockIdx.x * tpb + t; slot < n; slot += gridDim.x * tpb) {
+      const int64_t id = slot < k ? ids[slot] : l - lite + (slot - k);
+      if (id < 0 || id >= l) continue;
+      if (slot >= k && c == 0) ids[slot] = (int32_t)id;
+      const int64_t dst = ((int64_t)h * n + slot) * cpr, src = (src0 + id) * cpr;
+      if (c < cpr)
+        k_act[dst + c] = k_src[src + c];
+      else
+        v_act[dst + c - cpr] = v_src[src + c - cpr];
+    }
+  }
+}
+
 static int check_rows(int b, int hq, int hkv, int d, int dtype, int* cpr) {
   LRQK_REQUIRE(dtype == LRQK_F32 || dtype == LRQK_BF16, LRQK_EINVAL, "dtype=%d", dtype);
   LRQK_REQUIRE(b > 0 && hq > 0 && hkv > 0 && hq % hkv == 0, LRQK_EINVAL, "bad heads b=%d hq=%d hkv=%d", b, hq, hkv);
@@ -364,5 +391,23 @@ extern "C" int lrqk_store_rows(const void* rows, void* kv_store, int64_t cap, in
   const size_t row = (size_t)2 * d * elem_size(dtype);
   LRQK_HIP_CHECK(hipMemcpy2DAsync((char*)kv_store + (size_t)row0 * row, (size_t)cap * row, rows, (size_t)l * row,
                                   (size_t)l * row, (size_t)heads, hipMemcpyDeviceToHost, (hipStream_t)stream));
+  return LRQK_OK;
+}
+
+extern "C" int lrqk_fill_active(const void* k, const void* v, int64_t l, int32_t* active_idx, void* k_act, void* v_act,
+                                int topk, int lite, int b, int hq, int hkv, int d, int dtype, void* stream) {
+  int cpr;
+  int rc = check_rows(b, hq, hkv, d, dtype, &cpr);
+  if (rc) return rc;
+  LRQK_REQUIRE(k && v && active_idx && k_act && v_act, LRQK_EINVAL, "null pointer");
+  LRQK_REQUIRE(topk > 0 && lite > 0 && l >= (int64_t)topk + lite && l < ((int64_t)1 << 31), LRQK_EINVAL,
+               "a prompt of %lld tokens for %d + %d slots", (long long)l, topk, lite);
+  LRQK_REQUIRE(aligned16(k) && aligned16(v) && aligned16(k_act) && aligned16(v_act), LRQK_EINVAL,
+               "pointers must be 16-byte aligned");
+  const int tpb = std::max(1, 256 / (2 * cpr));
+  const int blocks = std::max(1, std::min((topk + lite + 2 * tpb - 1) / (2 * tpb), 8192 / (b * hq)));
+  hipLaunchKernelGGL(fill_active_kernel, dim3((unsigned)blocks, (unsigned)(b * hq)), dim3(256), 0, (hipStream_t)stream,
+                     (const uint4*)k, (const uint4*)v, l, active_idx, (uint4*)k_act, (uint4*)v_act, topk, lite, hq, hkv, cpr);
+  LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }

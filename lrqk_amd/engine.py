@@ -223,16 +223,19 @@ class LightAttentionIndicesFactory:
         dev, dt = query_states.device, query_states.dtype
         key_states = key_states.contiguous()
         value_states = value_states.contiguous()
-        self.Kgpu = torch.zeros((bsz, nheads, self.gpu_capacity, hdim), dtype=dt, device=dev)
-        self.Vgpu = torch.zeros((bsz, nheads, self.gpu_capacity, hdim), dtype=dt, device=dev)
-        self._active_idx = torch.full((bsz, nheads, self.gpu_capacity), -1, dtype=torch.int32, device=dev)
+        # the library's own stages write every slot for a prompt longer than the active set
+        custom = self._is_overridden("compute_hit_indices") or self._is_overridden("fetch_by_hit")
+        new = torch.empty if seq_len > self.gpu_capacity and not custom else torch.zeros
+        self.Kgpu = new((bsz, nheads, self.gpu_capacity, hdim), dtype=dt, device=dev)
+        self.Vgpu = new((bsz, nheads, self.gpu_capacity, hdim), dtype=dt, device=dev)
+        self._active_idx = torch.empty((bsz, nheads, self.gpu_capacity), dtype=torch.int32, device=dev)
         self.prefill_length = seq_len
         self.current_len = seq_len
         # a new sequence: whatever the victim cache holds belongs to the previous one
         self.ws.victim_cache(self.victim_rows_effective)
         stored = self._store_prompt(key_states, value_states) if seq_len > self.gpu_capacity else None
         try:
-            self._factorise_prompt(query_states, key_states, value_states)
+            self._factorise_prompt(query_states, key_states, value_states, custom)
         finally:
             if stored is not None:
                 # What is queued from here on finds the prompt in the store (and the staging block may be reused).
@@ -241,7 +244,7 @@ class LightAttentionIndicesFactory:
                 # (recorded right after the copy it made 128K prompts take 15 instead of 10 ms one time in four).
                 torch.cuda.current_stream(dev).wait_stream(stored[0])
 
-    def _factorise_prompt(self, query_states, key_states, value_states):
+    def _factorise_prompt(self, query_states, key_states, value_states, custom):
         seq_len = query_states.shape[2]
         k, L, g = self.attn_topk, self.num_lite_tokens, self.num_key_value_groups
         dev = query_states.device
@@ -261,23 +264,29 @@ class LightAttentionIndicesFactory:
                 self.lite_len = 0
             self.Kgpu.narrow(2, 0, seq_len).copy_(repeat_kv(key_states, g))
             self.Vgpu.narrow(2, 0, seq_len).copy_(repeat_kv(value_states, g))
+            self._active_idx.fill_(-1)
             self._active_idx[:, :, :seq_len] = torch.arange(seq_len, dtype=torch.int32, device=dev)
             self._hit_len = k
         else:
             # the rows are scanned where they will live (A_K's rows in the growing buffer): the
             # score index that this first scan builds then stays valid for the decode steps
-            hit = self.compute_hit_indices(query_states=A_Q,
-                                           key_states=self._A_K.data.narrow(2, 0, seq_len - L))
-            self._hit_len = hit.shape[2]
-            self._active_idx[:, :, :self._hit_len] = hit[..., 0].to(torch.int32)
-            self.fetch_by_hit(dst=self.Kgpu_topk_area, src=key_states, hit_indices=hit)
-            self.fetch_by_hit(dst=self.Vgpu_topk_area, src=value_states, hit_indices=hit)
             lb = seq_len - L
+            if not custom:
+                ops.score_select(self.ws, self._A_K.data, A_Q, lb, k, self.round_scores_to_storage, out=self._active_idx)
+                self._hit_len = k
+                ops.fill_active(key_states, value_states, self._active_idx, self.Kgpu, self.Vgpu, k)
+            else:
+                hit = self.compute_hit_indices(query_states=A_Q, key_states=self._A_K.data.narrow(2, 0, lb))
+                self._hit_len = hit.shape[2]
+                self._active_idx.fill_(-1)
+                self._active_idx[:, :, :self._hit_len] = hit[..., 0].to(torch.int32)
+                self.fetch_by_hit(dst=self.Kgpu_topk_area, src=key_states, hit_indices=hit)
+                self.fetch_by_hit(dst=self.Vgpu_topk_area, src=value_states, hit_indices=hit)
+                self.Kgpu[:, :, k:k + L, :] = repeat_kv(key_states.narrow(2, lb, L), g)
+                self.Vgpu[:, :, k:k + L, :] = repeat_kv(value_states.narrow(2, lb, L), g)
+                self._active_idx[:, :, k:] = torch.arange(lb, seq_len, dtype=torch.int32, device=dev)
             self.lite_indices = list(range(lb, seq_len))
             self.lite_len = 0
-            self.Kgpu[:, :, k:k + L, :] = repeat_kv(key_states.narrow(2, lb, L), g)
-            self.Vgpu[:, :, k:k + L, :] = repeat_kv(value_states.narrow(2, lb, L), g)
-            self._active_idx[:, :, k:] = torch.arange(lb, seq_len, dtype=torch.int32, device=dev)
         self.last_A_Q_row = A_Q
 
     def _fit_prompt(self, query_states: torch.Tensor, key_states: torch.Tensor) -> torch.Tensor:

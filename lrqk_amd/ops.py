@@ -302,6 +302,20 @@ def gather_rows(src: torch.Tensor, idx: torch.Tensor, dst: torch.Tensor, count: 
                                        hkv, d, _dt(src), _stream(dst)))
 
 
+def fill_active(k: torch.Tensor, v: torch.Tensor, active_idx: torch.Tensor, k_act: torch.Tensor, v_act: torch.Tensor,
+                topk: int):
+    """The active set of a prompt: slots 0 .. topk-1 of k_act, v_act [b,Hq,topk+lite,d] take the rows of k, v
+    [b,Hkv,l,d] that active_idx int32 [b,Hq,topk+lite] names there, the other slots the last tokens' (ids included)."""
+    _need_cuda(k, v, active_idx, k_act, v_act)
+    b, hkv, l, d = k.shape
+    _, hq, n, _ = k_act.shape
+    assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape and k_act.is_contiguous() and v_act.is_contiguous()
+    assert k.dtype == v.dtype == k_act.dtype == v_act.dtype and k_act.shape == v_act.shape == (b, hq, n, d)
+    assert active_idx.is_contiguous() and active_idx.dtype == torch.int32 and active_idx.shape == (b, hq, n)
+    check(_lib.load().lrqk_fill_active(k.data_ptr(), v.data_ptr(), l, active_idx.data_ptr(), k_act.data_ptr(),
+                                       v_act.data_ptr(), topk, n - topk, b, hq, hkv, d, _dt(k), _stream(k)))
+
+
 def append_token(k_new, v_new, k_act, v_act, slot: int, active_idx: Optional[torch.Tensor], token: int):
     _need_cuda(k_new, v_new, k_act, v_act)
     b, hkv = k_new.shape[:2]

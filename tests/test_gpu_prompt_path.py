@@ -125,3 +125,24 @@ def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
     rows, rescored = indexed.scan_stats()
     print(f"rescored {rescored} of {rows}", flush=True)
     assert rows == 3 * m and rescored < rows // 3
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,l,k,lite", [(torch.float32, 2, 1, 8, 12, 8, 4), (torch.bfloat16, 6, 2, 64, 515, 33, 7),
+                                                     (torch.float32, 4, 4, 256, 300, 100, 1)])
+def test_active_set_of_a_prompt(ops, dtype, hq, hkv, d, l, k, lite):
+    """Selected rows, then the last tokens' rows and ids (a prompt that just fills the set, slots beyond whole rounds of
+    a workgroup, rows of two and of 128 chunks)."""
+    gen = torch.Generator(device=DEV).manual_seed(l)
+    K = torch.randn((2, hkv, l, d), generator=gen, device=DEV).to(dtype)
+    V = torch.randn((2, hkv, l, d), generator=gen, device=DEV).to(dtype)
+    hit = torch.rand((2, hq, l - lite), generator=gen, device=DEV).argsort(-1)[:, :, :k].sort(-1).values.to(torch.int32)
+    ids = torch.cat([hit, torch.arange(l - lite, l, dtype=torch.int32, device=DEV).expand(2, hq, lite)], -1)
+    idx = torch.cat([hit, torch.full((2, hq, lite), -1, dtype=torch.int32, device=DEV)], -1).contiguous()
+    Ka = torch.empty((2, hq, k + lite, d), dtype=dtype, device=DEV)
+    Va = torch.empty_like(Ka)
+    ops.fill_active(K, V, idx, Ka, Va, k)
+    rows = ids.long().unsqueeze(-1).expand(-1, -1, -1, d)
+    g = hq // hkv
+    assert torch.equal(idx, ids)
+    assert torch.equal(Ka, torch.gather(K.repeat_interleave(g, 1), 2, rows))
+    assert torch.equal(Va, torch.gather(V.repeat_interleave(g, 1), 2, rows))
