@@ -335,8 +335,8 @@ __global__ __launch_bounds__(kFiltThreads) void score_filter_kernel(const T* __r
 
 // --------------------------------------------------------------------------- score + filter through the score index
 // Same output as score_filter_kernel (the candidate list of all rows with key >= bound, as a set), read from
-// the 8-bit copy of A_K in whitened coordinates: 34 bytes per row instead of 64.  Every wave solves
-// W q' = q (back substitution, lane i holds row i of W; q' ends up in scalar registers); for every
+// the 8-bit copy of A_K in whitened coordinates: 34 bytes per row instead of 64.  One wave of a workgroup solves
+// W q' = q (back substitution, lane i holds row i of W) for all of them; for every
 // row an upper bound of its (rounded) score follows from the copy:
 //   |score - s~| <= D = scale * |q'|_1 * kSidxDFactor,   s~ = scale * sum_j (u_j - 128) q'_j
 //   round_bf16(score) <= s~ + D + (|s~| + D) / 256       (half a bf16 ulp)
@@ -353,8 +353,11 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kScanU = 4;
 constexpr int kScanWaves = kFiltThreads / kWave;
 
+// (Workgroups per CU, that is waves per SIMD, that the registers are held to.  One more at R = 64 spills in the loop:
+// 127.6 against 119.4 us per step at 64K rows.)
+constexpr int scan_waves(int r) { return r == 64 ? 3 : r == 32 ? 4 : 5; }
 template <typename T, int R>
-__global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
+__global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_kernel(
     const T* __restrict__ a_k, int64_t head_stride, const T* __restrict__ q_hat, int64_t m, int r, int round_bf16,
     SelState st, uint2* __restrict__ cand, int cand_cap, FilterQ fq, ScoreIndexView six) {
   static_assert(R == 16 || R == 32 || R == 64, "the score index covers ranks 16, 32, 64");
@@ -365,7 +368,11 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
   constexpr int kHitCap = 2 * kWave;
   __shared__ uint32_t maybe_s[kScanWaves][kMaybeCap];
   __shared__ uint2 hits_s[kScanWaves][kHitCap];
-  __shared__ __align__(16) float qx_s[kScanWaves][R];  // the proxy query as the exact score uses it (a copy per wave)
+  // R = 16: every wave resolves the proxy query for itself (W is 1 KB then, and a barrier costs the first evaluation
+  // more than the reads: 63.0 against 62.1 us per step at 64K rows); else wave 0 does for the workgroup
+  constexpr bool kShare = R > 16;
+  __shared__ __align__(16) float qx_s[kShare ? 1 : kScanWaves][R];  // the proxy query as the exact score uses it
+  __shared__ __align__(16) float qp_s[R];                          // q'
   __shared__ int resc_s;
   const int h = blockIdx.y;
   const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
@@ -374,7 +381,6 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
   const uint16_t* QS = six.qs + (int64_t)h * six.head_rows;
   uint32_t* maybe = maybe_s[w];
   uint2* hits = hits_s[w];
-  if (tid == 0) resc_s = 0;
   const int sub = lane % QV;        // which 16 bytes of its row this lane reads
   const int lrow = lane / QV;       // row of this lane within a load
   const int64_t n_steps = (m + kStepRows - 1) / kStepRows;
@@ -399,19 +405,20 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
 
   const uint32_t t_prev = st.t_low[h];
   const float qn_prev = st.q_norm[h];
-  const bool pending = fq.iter_out != nullptr;
-  float sacc[kFiltMaxIt], oit[kFiltMaxIt];
-  if (pending) {
-    als_delta_sums<kFiltMaxIt>(fq.deltas, fq.bh, fq.max_iter, sacc);
-#pragma unroll
-    for (int it = 0; it < kFiltMaxIt; ++it)
-      oit[it] = fq.iter_out[((int64_t)h * fq.max_iter + min(it, fq.max_iter - 1)) * 2 * r + min(lane, r - 1)];
-  }
-  // row `lane` of W and 1 / W_ll (lanes >= R repeat the last row; their results are never read)
-  const float* Wm = six.wm + (int64_t)h * (R * R + R);
+  // The first rows are on their way while the proxy query and q' are resolved.  (With every wave on its own W is read
+  // once per wave: 50 MB at R = 64, a third of what the scan itself reads at 64K rows.)
   float qh[16];  // the 16 elements of q' that meet this lane's bytes
-  float qsum = 0.0f, ql1 = 0.0f, ql2 = 0.0f;
-  {
+  if (!kShare || w == 0) {
+    const bool pending = fq.iter_out != nullptr;
+    float sacc[kFiltMaxIt], oit[kFiltMaxIt];
+    if (pending) {
+      als_delta_sums<kFiltMaxIt>(fq.deltas, fq.bh, fq.max_iter, sacc);
+#pragma unroll
+      for (int it = 0; it < kFiltMaxIt; ++it)
+        oit[it] = fq.iter_out[((int64_t)h * fq.max_iter + min(it, fq.max_iter - 1)) * 2 * r + min(lane, r - 1)];
+    }
+    // row `lane` of W and 1 / W_ll (lanes >= R repeat the last row; their results are never read)
+    const float* Wm = six.wm + (int64_t)h * (R * R + R);
     float wrow[R];
     const float4* wp = reinterpret_cast<const float4*>(Wm + min(lane, R - 1) * R);
 #pragma unroll
@@ -433,30 +440,42 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
       if (blockIdx.x == 0 && tid < r) st_f32<T>((T*)fq.q_hat_out, (int64_t)h * r + tid, qv);
       q_lane = sizeof(T) == 2 ? round_to_bf16_f32(qv) : qv;
     }
-    if (lane < R) qx_s[w][lane] = lane < r ? q_lane : 0.0f;
+    if (lane < R) qx_s[kShare ? 0 : w][lane] = lane < r ? q_lane : 0.0f;
     // q' from W q' = q, last unknown first; lane i keeps the residual of equation i
-    float qc[R];
-    float resid = q_lane;
+    float resid = q_lane, qp = 0.0f;
 #pragma unroll
     for (int j = R - 1; j >= 0; --j) {
       const float x = sidx_readlane(resid * dinv, j);
-      qc[j] = x;
+      if constexpr (kShare)
+        qp = lane == j ? x : qp;
+      else
+        qh[j] = x;
       resid = __builtin_fmaf(-x, wrow[j], resid);
     }
+    if (kShare && lane < R) qp_s[lane] = qp;
+    if (tid == 0) resc_s = 0;
+  }
+  __syncthreads();
+  float qsum = 0.0f, ql1 = 0.0f, ql2 = 0.0f;
+  if constexpr (kShare) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      qsum += qc[j];
-      ql1 += fabsf(qc[j]);
-      ql2 = fmaf(qc[j], qc[j], ql2);
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      float x = qc[e];
-#pragma unroll
-      for (int c = 1; c < QV; ++c) x = sub == c ? qc[c * 16 + e] : x;
-      qh[e] = x;
+    for (int c = 0; c < 4; ++c) {
+      const float4 q4 = reinterpret_cast<const float4*>(qp_s)[4 * sub + c];
+      qh[4 * c + 0] = q4.x;
+      qh[4 * c + 1] = q4.y;
+      qh[4 * c + 2] = q4.z;
+      qh[4 * c + 3] = q4.w;
     }
   }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    qsum += qh[e];
+    ql1 += fabsf(qh[e]);
+    ql2 = fmaf(qh[e], qh[e], ql2);
+  }
+  qsum = group_sum(qsum, QV);
+  ql1 = group_sum(ql1, QV);
+  ql2 = group_sum(ql2, QV);
   const float qn = sqrtf(ql2);
   const uint32_t tl = rescaled_bound(t_prev, qn_prev, qn, round_bf16);
   if (tid == 0 && blockIdx.x == 0) {
@@ -467,7 +486,6 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
   const bool any = tl != 0xffffffffu;
   const float thr = key_score(tl);
   const float thr_lo = thr - fabsf(thr) * 1e-6f;
-  __syncthreads();  // (resc_s is zero)
 
   int n_maybe = 0, n_hits = 0, n_resc = 0;  // (wave-uniform)
   auto lds_wave_sync = [&]() {
@@ -508,7 +526,7 @@ __global__ __launch_bounds__(kFiltThreads) void score_prefilter_kernel(
       xv[c].unpack(f);
 #pragma unroll
       for (int e4 = 0; e4 < VEC / 4; ++e4) {
-        const float4 q4 = reinterpret_cast<const float4*>(qx_s[w])[(c * VEC) / 4 + e4];
+        const float4 q4 = reinterpret_cast<const float4*>(qx_s[kShare ? 0 : w])[(c * VEC) / 4 + e4];
         acc = __builtin_fmaf(f[4 * e4 + 0], q4.x, acc);
         acc = __builtin_fmaf(f[4 * e4 + 1], q4.y, acc);
         acc = __builtin_fmaf(f[4 * e4 + 2], q4.z, acc);
