@@ -112,12 +112,20 @@ class AutoIncreaseTensor:
 class AutoIncreaseTensorSharedKV(AutoIncreaseTensor):
     """K and V rows side by side on the last dim (lrqk_attention.py:959-963)."""
 
+    gpu: Optional[torch.device] = None  # the device whose current stream works on the rows behind torch's back
+
     def _alloc(self, shape):
         # Rows at and beyond current_len are never read (every access goes through a token id below it or
         # through tensor()), so the store is not cleared: clearing 0.8 GB of pinned memory is 4 ms of a
         # 128K layer prefill.  (The factor buffer keeps the zero fill: it is gathered at full capacity.)
         pin = bool(self.pin_memory) and torch.cuda.is_available()
-        return torch.empty(shape, device=self.device, dtype=self.dtype, pin_memory=pin)
+        store = torch.empty(shape, device=self.device, dtype=self.dtype, pin_memory=pin)
+        if pin and self.gpu is not None and store.numel():
+            # torch hands a freed pinned block out again once the work that it knows to use it is done.  The kernels
+            # and copies of the library are not in its books: one element copied by torch puts the current stream
+            # there, and whoever gets the block next finds everything queued on that stream until the release done.
+            torch.empty(1, dtype=store.dtype, device=self.gpu).copy_(store.view(-1)[:1], non_blocking=True)
+        return store
 
     @torch.inference_mode()
     def append(self, k: torch.Tensor, v: torch.Tensor):

@@ -334,6 +334,7 @@ class LightAttentionIndicesFactory:
         if not (self.KVcpu.pin_memory and key_states.is_cuda):
             self.KVcpu.append(key_states, value_states)
             return None
+        self.KVcpu.gpu = key_states.device
         row0 = self.KVcpu.extend((b, hkv, 0, 2 * d), length)
         if 2 * key_states.numel() * key_states.element_size() < self._DMA_STORE_BYTES:
             ops.flush_ring(key_states, value_states, 0, length, self.KVcpu.data, row0, hkv)

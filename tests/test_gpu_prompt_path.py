@@ -63,6 +63,34 @@ def test_prompt_rows_to_the_host_store(ops, heads, l, d, dtype):
         ops.store_rows(rows, store, 10, side)
 
 
+@pytest.mark.parametrize("context,name", [(1000, "kernel"), (9000, "copy engine")])
+def test_a_dropped_caches_store_waits_for_its_copies(ops, context, name):
+    """A cache that goes while its prompt is still on the way to the host store (written by a kernel or by a copy
+    engine): its pinned block is nobody else's before that work is done."""
+    from lrqk_amd import DynamicLRQKCache
+    gen = torch.Generator(device=DEV).manual_seed(context)
+    q = torch.randn((1, 4, context, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    k, v = (torch.randn((1, 2, context, 64), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2))
+    for attempt in range(2):   # (the first loads kernels, which waits for the device)
+        cache = DynamicLRQKCache(r=16, num_active_tokens=128, max_iter=1, lite_tokens=16, tol=0.0,
+                                 max_sequence_length=context + 64, num_key_value_groups=2)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(400_000_000)   # some tenths of a second
+        cache.update(q, k, v, 0)
+        store = cache.lwattn[0].KVcpu.data
+        place, shape = store.data_ptr(), store.shape
+        busy = torch.cuda.Event()
+        busy.record()
+        del cache, store
+        other = torch.empty(shape, dtype=torch.bfloat16, pin_memory=True)
+        early = not busy.query()
+        same = other.data_ptr() == place
+        torch.cuda.synchronize()
+        del other
+    print(name, "still under way:", early, flush=True)
+    assert early and not same
+
+
 @pytest.mark.parametrize("dtype,d,r,l,hq,hkv,iters", [
     (torch.float32, 64, 1, 128, 2, 2, 1),        # the fewest rows the Gram matrices take, one column of factors
     (torch.float32, 64, 16, 129, 6, 2, 2),       # a row beyond whole groups; three query heads per kv head
