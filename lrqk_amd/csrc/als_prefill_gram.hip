@@ -405,9 +405,14 @@ static int apply_shared(const void* k, const float* mt_k, OUT* a_k, int64_t a_st
 // ----------------------------------------------------------------------------- d x d algebra, fp64
 // Everything below is templated on RT, the number of 16-row tiles that the rank is padded to (ranks up to 16, 32, 64:
 // RT = 1, 2, 4), and on the row width D (64 or 128); RP = 16 RT is the padded rank.  Padding costs the matrix cores'
-// time (a solve has RP / 4 dependent steps), so a rank of 16 does not run as 32 (28 against 51 us per
-// iteration at D = 128, 32 heads; RT = 4: 132 us).
-constexpr int kGdThreads = 256;   // four waves: D / 4 right-hand columns each (one wave per SIMD: 512 registers)
+// time (a solve has RP / 4 dependent steps), so a rank of 16 does not run as 32 (24 against 42 us per
+// iteration at D = 128, 32 heads; RT = 4: 109 us).
+// Eight waves, two per SIMD: waves 0 .. 3 hold one system of a pair, waves 4 .. 7 the other (D / 4 right-hand columns
+// each).  A product occupies the matrix pipe for 64 cycles and a wave issues in order, so with both systems in one of
+// four waves the next pivot block waited behind the products of the step before; now the other wave of the SIMD works
+// meanwhile.  D = 128, 32 heads, four waves -> eight: the final pair alone 18.0 -> 12.4 us at RT = 2, 47.6 -> 33.0 at
+// RT = 4; an iteration 28 -> 24 us at RT = 1, 49 -> 42 at RT = 2, 133 -> 109 at RT = 4.
+constexpr int kGdThreads = 512;
 template <int RT, int D>
 struct GdShape {
   static constexpr int RP = 16 * RT;
@@ -417,26 +422,25 @@ struct GdShape {
   // RT = 4: three D x LD matrices do not fit the LDS, so B shares its block with T / U (each is dead when the other is
   // formed) and the r x r matrices lie in global memory (they stay in the L2)
   static constexpr bool WIDE = RT == 4;
-  static constexpr int PIV = WIDE ? 2 * 2 * RP * 4 + (kGdThreads / 64) * 32 : (kGdThreads / 64) * (2 * RP * 4 + 32);
+  static constexpr int PIV = (WIDE ? 2 * 2 : kGdThreads / 64) * RP * 4;
   static constexpr size_t SMEM = ((size_t)(WIDE ? 2 : 3) * D * LD + (WIDE ? 0 : 3 * RP * LG) + PIV + 8) * sizeof(double);
 };
 
 // ---- two systems [W | RHS] (W RP x RP symmetric positive definite up to rounding, rows/columns beyond r the
-// identity; RHS RP x D) solved side by side by block Gauss-Jordan elimination on the fp64 matrix cores, four
-// pivots per step.  The matrices live in the accumulator layout of 16 x 16 tiles (element v of lane l = row
-// 16 rt + l / 16 + 4 v, column 16 u + l % 16 of tile (rt, u)).  Up to RT = 2 each of the four waves holds W itself
-// (every wave eliminates its own copy: no wave waits for another, the solve has no barrier) and D / 4 columns of RHS;
-// RT = 4 would need 256 registers for the copies and most of the products for work done four times over, so there
-// wave w holds column tile w of W and the pivot columns go round through LDS, one barrier per step.
+// identity; RHS RP x D) solved side by side, one per half of the workgroup, by block Gauss-Jordan elimination on the
+// fp64 matrix cores, four pivots per step.  The matrices live in the accumulator layout of 16 x 16 tiles (element v of
+// lane l = row 16 rt + l / 16 + 4 v, column 16 u + l % 16 of tile (rt, u)).  Up to RT = 2 each of a system's four waves
+// holds W itself (every wave eliminates its own copy: no wave waits for another, the solve has no barrier) and D / 4
+// columns of RHS; RT = 4 would need 256 registers for the copies and most of the products for work done four times
+// over, so there wave w holds column tile w % 4 of W and the pivot columns go round through LDS, one barrier per step.
 // Step m, with P the pivot columns 4 m .. 4 m + 3 (RP x 4) and D its rows 4 m .. 4 m + 3:
 //     X <- X - (P D^-1) X[4 m .. 4 m + 3, :] outside the pivot rows,   X[pivot rows] <- D^-1 X[pivot rows]
 // (one product: the pivot rows' accumulators are cleared and their left operand is D^-1 itself), which clears the
 // pivot columns elsewhere.  The right-hand
 // operand, four rows of X, is element m % 4 of the lane's own tile in row tile m / 4: no data moves for it.  The
-// left operand needs P by rows: the lanes that hold the pivot columns put them into the LDS slot, the
-// two pivot blocks are inverted side by side in the two halves of the wave (by 2 x 2 blocks, no pivoting) and
-// handed round through the same slot.  The products on W come first (the next step waits for them only); those on
-// RHS run on the matrix cores while the next step's inverse is computed.
+// left operand needs P by rows: the lanes that hold the pivot columns put them into the LDS slot, and every lane inverts
+// the pivot block for itself (by 2 x 2 blocks, no pivoting).  The products on W come first (the next step waits for
+// them only).
 typedef double gd_v4d __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void gd_wave_sync() {  // orders one wave's LDS writes and reads
@@ -486,32 +490,29 @@ __device__ __forceinline__ void gd_inv4(const double (&D)[4][4], double (&R)[4][
 
 template <int RT, int CT>
 struct GdSys {
-  static constexpr int WC = RT == 4 ? 1 : RT;  // column tiles of W that a wave holds (all of them, or tile `wave`)
+  static constexpr int WC = RT == 4 ? 1 : RT;  // column tiles of W that a wave holds (all of them, or tile `wave % 4`)
   gd_v4d w[RT][WC];  // W: [row tile][column tile]
-  gd_v4d x[RT][CT];  // this wave's columns of RHS: [row tile][column tile CT wave + u]
+  gd_v4d x[RT][CT];  // this wave's columns of RHS: [row tile][column tile CT (wave % 4) + u]
 };
+// Solves the two systems of a pair, one per half of the workgroup (s: the system of this wave's half).
 template <int RT, int CT>
-__device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT> (&s)[2], double* __restrict__ piv) {
+__device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT>& s, double* __restrict__ piv) {
   constexpr int RP = 16 * RT;
   constexpr bool WIDE = RT == 4;
-  const int lane = lane_id(), wave = wave_id();
+  const int lane = lane_id(), wave = wave_id(), wq = wave & 3;
   const int li = lane & 15, lk = lane >> 4;
-  // P of both systems: the wave's own slot, or (WIDE) one of two slots that all waves read
-  double* own = piv + wave * (2 * RP * 4 + 32);
-  double* xch = WIDE ? piv + 2 * 2 * RP * 4 + wave * 32 : own + 2 * RP * 4;
 #pragma unroll
   for (int m = 0; m < 4 * RT; ++m) {
     const int tp = m >> 2, vp = m & 3;  // the pivots' tile (row tile of the pivot rows, column tile of W) and element
-    double* pb = WIDE ? piv + (m & 1) * 2 * RP * 4 : own;
+    // P: the wave's own slot, or (WIDE) one of two slots per system that its four waves read
+    double* P = piv + (WIDE ? (m & 1) * 2 + (wave >> 2) : wave) * RP * 4;
     {
       const int kk = li - 4 * vp;
-      if ((!WIDE || wave == tp) && kk >= 0 && kk < 4) {
+      if ((!WIDE || wq == tp) && kk >= 0 && kk < 4) {
 #pragma unroll
-        for (int sy = 0; sy < 2; ++sy)
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) pb[sy * RP * 4 + (16 * rt + lk + 4 * v) * 4 + kk] = s[sy].w[rt][WIDE ? 0 : tp][v];
+          for (int v = 0; v < 4; ++v) P[(16 * rt + lk + 4 * v) * 4 + kk] = s.w[rt][WIDE ? 0 : tp][v];
       }
     }
     // (two slots: a wave that passes this barrier has read the slot of step m - 2, which step m wrote over)
@@ -519,9 +520,10 @@ __device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT> (&s)[2], double* __r
       __syncthreads();
     else
       gd_wave_sync();
+    // every lane inverts the pivot block and keeps what its operands take of it: column l / 16, and the element of row
+    // l % 4 in that column
+    double ic[4], mine;
     {
-      const int mine = lane >> 5;
-      const double* P = pb + mine * RP * 4;
       double D[4][4], R[4][4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -530,58 +532,46 @@ __device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT> (&s)[2], double* __r
         D[i][0] = lo.x; D[i][1] = lo.y; D[i][2] = hi.x; D[i][3] = hi.y;
       }
       gd_inv4(D, R);
-      if ((lane & 31) == 0) {
+      // (by value: a choice between array elements is one between addresses, and puts the array into scratch memory)
+      auto pick = [](int i, double e0, double e1, double e2, double e3) {
+        const double c01 = i & 1 ? e1 : e0, c23 = i & 1 ? e3 : e2;
+        return i & 2 ? c23 : c01;
+      };
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          *reinterpret_cast<double2*>(&xch[mine * 16 + i * 4]) = make_double2(R[i][0], R[i][1]);
-          *reinterpret_cast<double2*>(&xch[mine * 16 + i * 4 + 2]) = make_double2(R[i][2], R[i][3]);
-        }
-      }
-      gd_wave_sync();
+      for (int k = 0; k < 4; ++k) ic[k] = pick(lk, R[k][0], R[k][1], R[k][2], R[k][3]);
+      mine = pick(li, ic[0], ic[1], ic[2], ic[3]);
     }
-    double aop[2][RT];
+    double aop[RT];
 #pragma unroll
-    for (int sy = 0; sy < 2; ++sy) {
-      const double* P = pb + sy * RP * 4;
-      double ic[4];  // column l / 16 of the inverse
-#pragma unroll
-      for (int k = 0; k < 4; ++k) ic[k] = xch[sy * 16 + k * 4 + lk];
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const int row = 16 * rt + li;
-        const double2 lo = *reinterpret_cast<const double2*>(&P[row * 4]);
-        const double2 hi = *reinterpret_cast<const double2*>(&P[row * 4 + 2]);
-        // pivot rows: the rows of D^-1 themselves (their accumulators are cleared below, so they come out as
-        // D^-1 X and not as X - (I - D^-1) X, which cancels in its leading digits when D is far from unit size:
-        // with a diagonal of 1e12 solutions were off by 5e-3 where the conditioning allowed 1e-11)
-        const double mine = xch[sy * 16 + (row & 3) * 4 + lk];
-        const double oth = -fma(lo.x, ic[0], fma(lo.y, ic[1], fma(hi.x, ic[2], hi.y * ic[3])));
-        aop[sy][rt] = (row >> 2) == m ? mine : oth;
-      }
+    for (int rt = 0; rt < RT; ++rt) {
+      const int row = 16 * rt + li;
+      const double2 lo = *reinterpret_cast<const double2*>(&P[row * 4]);
+      const double2 hi = *reinterpret_cast<const double2*>(&P[row * 4 + 2]);
+      // pivot rows: the rows of D^-1 themselves (their accumulators are cleared below, so they come out as
+      // D^-1 X and not as X - (I - D^-1) X, which cancels in its leading digits when D is far from unit size:
+      // with a diagonal of 1e12 solutions were off by 5e-3 where the conditioning allowed 1e-11)
+      const double oth = -fma(lo.x, ic[0], fma(lo.y, ic[1], fma(hi.x, ic[2], hi.y * ic[3])));
+      aop[rt] = (row >> 2) == m ? mine : oth;
     }
-    gd_wave_sync();  // (the reads of the slot precede the next step's writes)
+    if constexpr (!WIDE) gd_wave_sync();  // (the reads of the slot precede the next step's writes)
     // W: the column tiles from the pivots' on (those before hold finished unit columns: zero in the pivot rows)
 #pragma unroll
-    for (int sy = 0; sy < 2; ++sy)
+    for (int u = 0; u < GdSys<RT, CT>::WC; ++u) {
+      if (WIDE ? wq < tp : u < tp) continue;  // (wave-uniform)
+      const double bop = s.w[tp][u][vp];
+      s.w[tp][u][vp] = 0.0;
 #pragma unroll
-      for (int u = 0; u < GdSys<RT, CT>::WC; ++u) {
-        if (WIDE ? wave < tp : u < tp) continue;  // (wave-uniform)
-        const double bop = s[sy].w[tp][u][vp];
-        s[sy].w[tp][u][vp] = 0.0;
+      for (int rt = 0; rt < RT; ++rt)
+        s.w[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[rt], bop, s.w[rt][u], 0, 0, 0);
+    }
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          s[sy].w[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[sy][rt], bop, s[sy].w[rt][u], 0, 0, 0);
-      }
+    for (int u = 0; u < CT; ++u) {
+      const double bop = s.x[tp][u][vp];
+      s.x[tp][u][vp] = 0.0;
 #pragma unroll
-    for (int sy = 0; sy < 2; ++sy)
-#pragma unroll
-      for (int u = 0; u < CT; ++u) {
-        const double bop = s[sy].x[tp][u][vp];
-        s[sy].x[tp][u][vp] = 0.0;
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          s[sy].x[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[sy][rt], bop, s[sy].x[rt][u], 0, 0, 0);
-      }
+      for (int rt = 0; rt < RT; ++rt)
+        s.x[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[rt], bop, s.x[rt][u], 0, 0, 0);
+    }
   }
   if constexpr (WIDE) __syncthreads();  // (the next solve starts with slot 0 again)
 }
@@ -590,7 +580,7 @@ __device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT> (&s)[2], double* __r
 // of RHS, value).
 template <int RT, int CT, typename FW, typename FX>
 __device__ __forceinline__ void gd_fill(GdSys<RT, CT>& t, FW&& fw, FX&& fx) {
-  const int lane = lane_id(), wave = wave_id();
+  const int lane = lane_id(), wave = wave_id() & 3;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -604,7 +594,7 @@ __device__ __forceinline__ void gd_fill(GdSys<RT, CT>& t, FW&& fw, FX&& fx) {
 }
 template <int RT, int CT, typename G>
 __device__ __forceinline__ void gd_drain(const gd_v4d (&x)[RT][CT], G&& g) {
-  const int lane = lane_id(), wave = wave_id();
+  const int lane = lane_id(), wave = wave_id() & 3;
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -614,16 +604,17 @@ __device__ __forceinline__ void gd_drain(const gd_v4d (&x)[RT][CT], G&& g) {
 }
 
 // f(i, j, sum over c < D of PT[c][i] * RT_[c][j])   (two r x d matrices, stored transposed) on the fp64 matrix
-// cores: RT x RT tiles of 16 x 16, D / 4 products of depth 4 in a row each; wave w owns tile row w (RT = 4), one tile
-// (RT = 2), and wave 0 the only tile of RT = 1.  Rows/columns beyond r come out as what the zero padding gives.
+// cores: RT x RT tiles of 16 x 16, D / 4 products of depth 4 in a row each; a wave owns two tiles of a row (RT = 4), one
+// of the first four waves a tile (RT = 2), and wave 0 the only tile of RT = 1.  Rows/columns beyond r come out as what
+// the zero padding gives.
 template <int RT, int D, typename F>
 __device__ __forceinline__ void gd_outer(const double* __restrict__ PT, const double* __restrict__ QT, F&& f) {
   constexpr int LD = GdShape<RT, D>::LD;
-  constexpr int NC = RT == 4 ? 4 : 1;  // column tiles per wave
+  constexpr int NC = RT == 4 ? 2 : 1;  // column tiles per wave
   const int lane = lane_id(), wave = wave_id();
-  if (RT == 1 && wave > 0) return;
+  if (wave >= RT * RT / NC) return;
   const int li = lane & 15, lk = lane >> 4;
-  const int tr = RT == 4 ? wave : RT == 2 ? wave >> 1 : 0, tc = RT == 2 ? wave & 1 : 0;
+  const int tr = RT == 1 ? 0 : wave >> 1, tc = RT == 1 ? 0 : NC * (wave & 1);
   const double* pa = PT + lk * LD + 16 * tr + li;
   const double* pb = QT + lk * LD + 16 * tc + li;
   gd_v4d acc[NC];
@@ -643,44 +634,43 @@ __device__ __forceinline__ void gd_outer(const double* __restrict__ PT, const do
 
 // TT[c][i] = sum over k of MT[k][i] * S[k][c]   (the transposed form of Mt S, S symmetric D x D in global
 // memory) on the fp64 matrix cores: 16 x 16 x 4 tiles, A operand lane l = Mt[i0 + l % 16][k0 + l / 16] (from the
-// LDS copy), B operand lane l = S[k0 + l / 16][c0 + l % 16] (8 CT independent loads per lane in flight), result
-// element v of lane l = row l / 16 + 4 v, column l % 16 of the tile.  Each wave takes D / 4 columns.
+// LDS copy), B operand lane l = S[k0 + l / 16][c0 + l % 16] (16 independent loads per lane in flight), result
+// element v of lane l = row l / 16 + 4 v, column l % 16 of the tile.  Each wave takes a column tile (D = 64: two waves
+// share one, half of the row tiles each).
 // One barrier.
 template <int RT, int D>
 __device__ __forceinline__ void gd_times_s(const double* __restrict__ MT, const double* __restrict__ S,
                                            double* __restrict__ TT) {
-  constexpr int LD = GdShape<RT, D>::LD, CT = GdShape<RT, D>::CT;
+  constexpr int LD = GdShape<RT, D>::LD;
+  constexpr bool HALF = D == 64;
+  constexpr int NR = HALF ? (RT + 1) / 2 : RT;  // row tiles per wave
+  constexpr int U = 16;
   const int lane = lane_id(), wave = wave_id();
   const int li = lane & 15, lk = lane >> 4;
-  const int c0 = 16 * CT * wave;
-  gd_v4d acc[RT][CT];
+  const int c0 = 16 * (HALF ? wave & 3 : wave), r0 = HALF ? NR * (wave >> 2) : 0;
+  if (r0 < RT) {
+    gd_v4d acc[NR];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+    for (int rt = 0; rt < NR; ++rt) acc[rt] = gd_v4d{0.0, 0.0, 0.0, 0.0};
+    for (int kb = 0; kb < D; kb += 4 * U) {
+      double bv[U];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = gd_v4d{0.0, 0.0, 0.0, 0.0};
-  for (int kb = 0; kb < D; kb += 32) {
-    double bv[8][CT];
+      for (int u = 0; u < U; ++u) bv[u] = S[(int64_t)(kb + 4 * u + lk) * D + c0 + li];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
+      for (int u = 0; u < U; ++u) {
+        const int k = kb + 4 * u + lk;
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) bv[u][ct] = S[(int64_t)(kb + 4 * u + lk) * D + c0 + 16 * ct + li];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int k = kb + 4 * u + lk;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        const double a = MT[k * LD + 16 * rt + li];
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv[u][ct], acc[rt][ct], 0, 0, 0);
+        for (int rt = 0; rt < NR; ++rt) {
+          const double a = MT[k * LD + 16 * (r0 + rt) + li];
+          acc[rt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv[u], acc[rt], 0, 0, 0);
+        }
       }
     }
+#pragma unroll
+    for (int rt = 0; rt < NR; ++rt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) TT[(c0 + li) * LD + 16 * (r0 + rt) + lk + 4 * v] = acc[rt][v];
   }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) TT[(c0 + 16 * ct + li) * LD + 16 * rt + lk + 4 * v] = acc[rt][ct][v];
   __syncthreads();
 }
 
@@ -784,6 +774,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
   double* piv = BT + D * LD;                // the solves' slots
   double* red = piv + Sh::PIV;              // [8]
   const int tid = threadIdx.x;
+  const bool first = wave_id() < 4;         // this wave's half of the workgroup: the first system of a pair or the second
   const int h = blockIdx.x;
   const int r = a.r, bh = a.bh;
   double* Gs = Sh::WIDE ? a.Gs + (int64_t)h * 2 * RP * LG : red + 8;  // [2 or 3][RP][LG]
@@ -811,7 +802,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
     for (int u = 0; u < (kHold ? kBqPer : 1); ++u) bq_pre[u] = src[tid + u * kGdThreads];
   }
   if constexpr (kHold) {
-    const int lane = lane_id(), wave = wave_id();
+    const int lane = lane_id(), wave = wave_id() & 3;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
@@ -852,16 +843,17 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
   // Of an iteration's r x r systems only two follow each other: B_K = Gk^-1 Ck does not depend on the Q side's
   // step and is solved beside it, and the next iteration's B_Q = Gq'^-1 Cq' is solved beside the K side's step
   // and handed over in `BqT`.  Iteration 0 (and the final stage) start from the state alone: B_Q and B_K side by side.
-  GdSys<RT, CT> sy[2];
-  gd_v4d bk[kHold ? RT : 1][CT];  // B_K in the layout of the right-hand sides
+  GdSys<RT, CT> sy;
+  gd_v4d bk[kHold ? RT : 1][CT];  // B_K in the layout of the right-hand sides (second half)
   double* BqT = a.BqT + (int64_t)h * RP * d;  // [RP][d]
   if constexpr (PART != kGdQSide && PART != kGdKSide) {
   if (fresh) {
-    gd_fill(sy[0], [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
-    if constexpr (FINAL)
-      gd_fill(sy[1], [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return Ck[i * d + cc]; });
+    if (first)
+      gd_fill(sy, [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
+    else if (FINAL)
+      gd_fill(sy, [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return Ck[i * d + cc]; });
     else
-      gd_fill(sy[1], [&](int i, int j) { return i == j ? 1.0 : 0.0; }, [&](int, int) { return 0.0; });
+      gd_fill(sy, [&](int i, int j) { return i == j ? 1.0 : 0.0; }, [&](int, int) { return 0.0; });
     gd_solve_pair(sy, piv);
     if constexpr (FINAL) {
       const int64_t o = (int64_t)h * r * d;
@@ -872,15 +864,15 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
         else
           ((float*)dst)[o + i * d + cc] = (float)v;
       };
-      gd_drain(sy[0].x, [&](int i, int cc, double v) { put(a.b_q, i, cc, v); });
-      gd_drain(sy[1].x, [&](int i, int cc, double v) { put(a.b_k, i, cc, v); });
+      void* dst = first ? a.b_q : a.b_k;
+      gd_drain(sy.x, [&](int i, int cc, double v) { put(dst, i, cc, v); });
       return;
     }
     if constexpr (PART == kGdStart) {
-      gd_drain(sy[0].x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+      if (first) gd_drain(sy.x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
       return;
     }
-    gd_drain(sy[0].x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
+    if (first) gd_drain(sy.x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
   } else if constexpr (kHold) {
 #pragma unroll
     for (int u = 0; u < kBqPer; ++u) {
@@ -899,31 +891,24 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
   gd_outer<RT, D>(BT, BT, [&](int i, int j, double o) { Gs[i * LG + j] = Gk[i * RP + j] + o; });
   __syncthreads();
   // ---- Mq'^T = W1^-1 (Ck + B_Q) beside B_K = Gk^-1 Ck
-  gd_fill(sy[0], [&](int i, int j) { return Gs[i * LG + j]; }, [&](int i, int cc) { return BT[cc * LD + i]; });
-  gd_fill(sy[1], [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return kHold ? 0.0 : Ck[i * d + cc]; });
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int u = 0; u < CT; ++u) {
-      if constexpr (kHold) sy[1].x[rt][u] = ckt[rt][u];
-      sy[0].x[rt][u] += sy[1].x[rt][u];
-    }
-  __syncthreads();  // (every read of B_Q precedes the rewriting of the B tile below)
-  gd_solve_pair(sy, piv);
+  if (first)
+    gd_fill(sy, [&](int i, int j) { return Gs[i * LG + j]; },
+            [&](int i, int cc) { return kHold ? BT[cc * LD + i] : BT[cc * LD + i] + Ck[i * d + cc]; });
+  else
+    gd_fill(sy, [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return kHold ? 0.0 : Ck[i * d + cc]; });
   if constexpr (kHold) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < CT; ++u) bk[rt][u] = sy[1].x[rt][u];
-  } else {
-    gd_drain(sy[1].x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+      for (int u = 0; u < CT; ++u) sy.x[rt][u] += ckt[rt][u];
   }
+  __syncthreads();  // (every read of B_Q precedes the rewriting of the B tile below)
+  gd_solve_pair(sy, piv);
   // ---- the B tile now holds B_K; Mq'^T goes to its tile and to the caller, with the sum of Cq (the old one) . Mq'^T
-  gd_drain(sy[1].x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
   double part_q = 0.0;
-  {
+  if (first) {
     float* mt = a.Mt_q + (int64_t)h * r * d;
-    gd_drain(sy[0].x, [&](int i, int cc, double v) {
+    gd_drain(sy.x, [&](int i, int cc, double v) {
       MT[cc * LD + i] = v;
       if (i < r) mt[i * d + cc] = (float)v;
       if constexpr (!kHold) part_q = fma(Cq[i * d + cc], v, part_q);
@@ -934,8 +919,18 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
 #pragma unroll
         for (int u = 0; u < CT; ++u)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) part_q = fma(cqt[rt][u][v], sy[0].x[rt][u][v], part_q);
+          for (int v = 0; v < 4; ++v) part_q = fma(cqt[rt][u][v], sy.x[rt][u][v], part_q);
     }
+  } else {
+    if constexpr (kHold) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int u = 0; u < CT; ++u) bk[rt][u] = sy.x[rt][u];
+    } else {
+      gd_drain(sy.x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+    }
+    gd_drain(sy.x, [&](int i, int cc, double v) { BT[cc * LD + i] = v; });
   }
   double tr_old = 0.0;
   if (tid < RP) tr_old = tid < r ? Gq[tid * RP + tid] : 0.0;
@@ -960,33 +955,34 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
   for (int e = tid; e < RP * d; e += kGdThreads) Cq[e] = TT[(e % d) * LD + e / d];
   }
   if constexpr (PART == kGdWhole || PART == kGdKSide) {
-  // ---- Mk'^T = (Gq' + B_K B_K^T)^-1 (T + B_K) beside the next B_Q = Gq'^-1 T
+  // ---- the next B_Q = Gq'^-1 T beside Mk'^T = (Gq' + B_K B_K^T)^-1 (T + B_K)
   {
     const double* Gb = Gs + RP * LG;
     if constexpr (kHold) {
       const double* Gn = Gs + 2 * RP * LG;
-      gd_fill(sy[0], [&](int i, int j) { return Gn[i * LG + j]; }, [&](int i, int cc) { return TT[cc * LD + i]; });
-      gd_fill(sy[1], [&](int i, int j) { return Gn[i * LG + j] + Gb[i * LG + j]; },
+      gd_fill(sy, [&](int i, int j) { return first ? Gn[i * LG + j] : Gn[i * LG + j] + Gb[i * LG + j]; },
               [&](int i, int cc) { return TT[cc * LD + i]; });
+      if (!first) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int u = 0; u < CT; ++u) sy.x[rt][u] += bk[rt][u];
+      }
+    } else if (first) {
+      gd_fill(sy, [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
     } else {
-      gd_fill(sy[0], [&](int i, int j) { return Gq[i * RP + j]; }, [&](int i, int cc) { return Cq[i * d + cc]; });
-      gd_fill(sy[1], [&](int i, int j) { return Gq[i * RP + j] + Gb[i * LG + j]; },
+      gd_fill(sy, [&](int i, int j) { return Gq[i * RP + j] + Gb[i * LG + j]; },
               [&](int i, int cc) { return Cq[i * d + cc] + BqT[i * d + cc]; });
     }
-    if constexpr (kHold) {
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int u = 0; u < CT; ++u) sy[1].x[rt][u] += bk[rt][u];
-    }
   }
-  __syncthreads();
+  __syncthreads();  // (also: B_K has been read when the next B_Q takes its block)
   gd_solve_pair(sy, piv);
-  gd_drain(sy[0].x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
   double part_k = 0.0;
-  {
+  if (first) {
+    gd_drain(sy.x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
+  } else {
     float* mt = a.Mt_k + (int64_t)h * r * d;
-    gd_drain(sy[1].x, [&](int i, int cc, double v) {
+    gd_drain(sy.x, [&](int i, int cc, double v) {
       MT[cc * LD + i] = v;
       if (i < r) mt[i * d + cc] = (float)v;
       if constexpr (!kHold) part_k = fma(Ck[i * d + cc], v, part_k);
@@ -997,7 +993,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
 #pragma unroll
         for (int u = 0; u < CT; ++u)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) part_k = fma(ckt[rt][u][v], sy[1].x[rt][u][v], part_k);
+          for (int v = 0; v < 4; ++v) part_k = fma(ckt[rt][u][v], sy.x[rt][u][v], part_k);
     }
   }
   double trk_old = 0.0;
