@@ -174,3 +174,22 @@ def test_active_set_of_a_prompt(ops, dtype, hq, hkv, d, l, k, lite):
     assert torch.equal(idx, ids)
     assert torch.equal(Ka, torch.gather(K.repeat_interleave(g, 1), 2, rows))
     assert torch.equal(Va, torch.gather(V.repeat_interleave(g, 1), 2, rows))
+
+
+@pytest.mark.parametrize("batch,hkv,l", [(1, 1, 300), (2, 3, 517), (1, 16, 1031)])
+def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
+    """A prompt whose first heads go ahead of the others (one head: a single copy; 6 and 16: pieces of 1 + 5, 2 + 14) is
+    in the host store as given, also when the next prompt uses the same copy stream at once."""
+    from lrqk_amd.engine import LightAttentionIndicesFactory as Engine
+    monkeypatch.setattr(Engine, "_DMA_STORE_BYTES", 1)
+    monkeypatch.setattr(Engine, "_DMA_PIECES_BYTES", 1)
+    gen = torch.Generator(device=DEV).manual_seed(l)
+    engines = []
+    for _ in range(2):
+        q, k, v = (torch.randn((batch, h, l, 64), generator=gen, device=DEV).to(torch.bfloat16) for h in (2 * hkv, hkv, hkv))
+        eng = Engine(num_lite_tokens=8, attn_topk=64, num_key_value_groups=2, r=16, max_iter=1, tol=0.0, capacity=l + 9)
+        eng.prefill(q, k, v)
+        engines.append((eng, torch.cat([k, v], -1)))
+    torch.cuda.current_stream().synchronize()
+    for eng, want in engines:
+        assert torch.equal(eng.KVcpu.tensor(), want.cpu())
