@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "ctx.hpp"
+#include "prefill_pieces.hpp"
 #include "small_inverse.hpp"
 
 namespace lrqk {
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
   constexpr int NT = NW * kWave;
   extern __shared__ __align__(16) float sm[];
   __shared__ float red[NW];
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   uint16_t* x_s = reinterpret_cast<uint16_t*>(sm) + wave * 32 * LDB;           // this wave's rows of X
   uint16_t* mt_s = reinterpret_cast<uint16_t*>(sm) + NW * 32 * LDB;            // [3][32][LDB] pieces of Mt
@@ -674,17 +675,15 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (((i + wave) % NL) * kWave + lane) * VEC;  // (the waves start at different KB of their tiles)
-      pre[i] = *reinterpret_cast<const uint4*>(Xh + base + (e < nvalid ? e : 0));
+      pre[i] = gd_at<uint4>(Xh + base, 2u * (uint32_t)(e < nvalid ? e : 0));
     }
   };
   float old_next[GIVEN ? 16 : 1];
   auto issue_old = [&](int64_t t0) {
     if constexpr (GIVEN) {
+      const int last = (int)min((int64_t)32, l - t0) - 1;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t rr = min(t0 + pf_mfma_row(lane, v), l - 1);
-        old_next[v] = Ah[rr * r + min(col, r - 1)];
-      }
+      for (int v = 0; v < 16; ++v) old_next[v] = gd_factor(Ah + t0 * r, pf_mfma_row(lane, v), last, r, min(col, r - 1));
     }
   };
   if (r0 + (int64_t)wave * 32 < r1) {
@@ -750,8 +749,9 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_bf16_kernel(const bf16_t* 
         }
       }
     } else {
+      const int valid = (col < r ? rows : 0) - 4 * half;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) c[v] = (pf_mfma_row(lane, v) < rows && col < r) ? old[v] : 0.0f;
+      for (int v = 0; v < 16; ++v) c[v] = gd_mfma_row0(v) < valid ? old[v] : 0.0f;
     }
     // the three pieces of C, eight rows (one k block) at a time
     bf16x8 cp[3][2];

@@ -51,11 +51,11 @@ __global__ __launch_bounds__(kXtxThreads) void pf_xtx_kernel(const bf16_t* __res
   // (65 against 54 us at 32 heads x 32K rows).
   uint4 pre_a[NL];
   auto issue = [&](int64_t t0, uint4 (&dst)[NL]) {
+    const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kXtxThreads + tid) * 8;  // element of the 128 x 128 step
-      const int64_t row = t0 + e / kXtxD;
-      dst[i] = *reinterpret_cast<const uint4*>(Xh + min(row, l - 1) * kXtxD + e % kXtxD);
+      dst[i] = gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
     }
   };
   gd_floatx16 acc0, acc1;
@@ -75,11 +75,12 @@ __global__ __launch_bounds__(kXtxThreads) void pf_xtx_kernel(const bf16_t* __res
   const int64_t stride = (int64_t)S * kXtxRows;
   // one step: stage `cur` (the rows from t0 on), ask for the next step into `cur`, multiply
   auto step = [&](int64_t t0, uint4 (&cur)[NL]) {
+    const int rows = (int)min((int64_t)kXtxRows, l - t0);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kXtxThreads + tid) * 8;
       const int row = e / kXtxD;
-      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = t0 + row < l ? cur[i] : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = row < rows ? cur[i] : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
     if (t0 + stride < l) issue(t0 + stride, cur);
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
   // the tile of X; at the end the waves' sums pass through it
   __shared__ __align__(16) uint16_t x_s[kXtxRows * kXtxLd];
   static_assert(sizeof(x_s) >= kXtxWaves * 1024 * sizeof(float), "the reduction uses the tile's LDS");
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   const int xh = blockIdx.y, s = blockIdx.x;
   const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
@@ -148,11 +149,11 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
   constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);
   uint4 pre_a[NL];
   auto issue = [&](int64_t t0, uint4 (&dst)[NL]) {
+    const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kXtxThreads + tid) * 8;
-      const int64_t row = t0 + e / kXtxD;
-      dst[i] = *reinterpret_cast<const uint4*>(Xh + min(row, l - 1) * kXtxD + e % kXtxD);
+      dst[i] = gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
     }
   };
   gd_floatx16 acc0, acc1, gAA, gAX[2];
@@ -175,16 +176,20 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
   const int64_t stride = (int64_t)S * kXtxRows;
   float arow[16];  // this wave's rows of A of the step being multiplied, requested at the start of the step
   auto step = [&](int64_t t0, uint4 (&cur)[NL]) {
+    const int rows = (int)min((int64_t)kXtxRows, l - t0);
+    const int group_rows = rows - 32 * wa;  // of this wave's group: below 1 beyond the end
+    {
+      const float* group = Ah + min(t0 + 32 * wa, l - 1) * r;
+      const int last = max(group_rows, 1) - 1;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {  // (requested first, consumed after the blocks of X^T X below)
-      const int64_t row = min(t0 + 32 * wa + gd_mfma_row(lane, v), l - 1);
-      arow[v] = Ah[row * r + min(col, r - 1)];
+      for (int v = 0; v < 16; ++v)  // (requested first, consumed after the blocks of X^T X below)
+        arow[v] = gd_factor(group, gd_mfma_row(lane, v), last, r, min(col, r - 1));
     }
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kXtxThreads + tid) * 8;
       const int row = e / kXtxD;
-      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = t0 + row < l ? cur[i] : make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = row < rows ? cur[i] : make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
     if (t0 + stride < l) issue(t0 + stride, cur);
@@ -207,7 +212,8 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
         acc1[v] += t1a[v];
       }
     }
-    if (t0 + 32 * wa < l) {  // (wave-uniform)
+    if (group_rows > 0) {  // (wave-uniform)
+      const int valid = (col < r ? group_rows : 0) - 4 * half;
       // the three pieces of the group's rows of A, eight rows (one k block) at a time
       gd_bf16x8 cp[3][2];
 #pragma unroll
@@ -216,8 +222,7 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const int v = 8 * kb + q;
-          const bool valid = t0 + 32 * wa + gd_mfma_row(lane, v) < l && col < r;
-          gd_split3(valid ? arow[v] : 0.0f, pc[0][q], pc[1][q], pc[2][q]);
+          gd_split3(gd_mfma_row0(v) < valid ? arow[v] : 0.0f, pc[0][q], pc[1][q], pc[2][q]);
         }
 #pragma unroll
         for (int pp = 0; pp < 3; ++pp)
@@ -318,7 +323,7 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
   extern __shared__ __align__(16) uint16_t ap_s[];
   uint16_t* x_s = ap_s;                          // [128][kApLd]
   uint16_t* mt_s = ap_s + kXtxRows * kApLd;      // [NH][3][32][kApLd]
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   const int xh = blockIdx.y, s = blockIdx.x;
   const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
@@ -338,10 +343,10 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
   static_assert(NL == 4, "four 16-byte loads per thread and step");
   uint4 pre0 = make_uint4(0, 0, 0, 0), pre1 = pre0, pre2 = pre0, pre3 = pre0;
   auto issue = [&](int64_t t0) {
+    const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
     auto ld = [&](int i) {
       const int e = (i * kXtxThreads + tid) * 8;
-      const int64_t row = t0 + e / kXtxD;
-      return *reinterpret_cast<const uint4*>(Xh + min(row, l - 1) * kXtxD + e % kXtxD);
+      return gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
     };
     pre0 = ld(0);
     pre1 = ld(1);
@@ -379,11 +384,7 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
           c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, m, c, 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t row = t0 + 32 * g + gd_mfma_row(lane, v);
-        if (row < l && col < r) gd_store(Ah, row * r + col, c[v]);
-      }
+      gd_store_tile(Ah + (t0 + 32 * g) * r, c, (int)min((int64_t)32, l - t0 - 32 * g), col, half, r);
     }
     __syncthreads();
   }

@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __r
   constexpr int TILE = 32 * LDX * (int)sizeof(T);
   constexpr int SMEM = kStWaves * (TILE > 4096 ? TILE : 4096);
   __shared__ __align__(16) char smem[SMEM];
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   T* x_s = reinterpret_cast<T*>(smem + wave * (SMEM / kStWaves));
   const int h = blockIdx.y, s = blockIdx.x;
@@ -97,42 +97,45 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __r
   gd_u32x4 pre[NL];
   float arow[GIVEN ? AT : 1][16];
   auto issue = [&](int64_t t0) {
+    const int last = (int)min((int64_t)32, l - t0) - 1;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kWave + lane) * VEC;
-      pre[i] = *reinterpret_cast<const gd_u32x4*>(Xh + min(t0 + e / D, l - 1) * D + e % D);
+      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * (uint32_t)sizeof(T));
     }
     if constexpr (GIVEN) {
 #pragma unroll
       for (int at = 0; at < AT; ++at)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          arow[at][v] = Ah[min(t0 + gd_mfma_row(lane, v), l - 1) * r + min(32 * at + col, r - 1)];
+          arow[at][v] = gd_factor(Ah + t0 * r, gd_mfma_row(lane, v), last, r, min(32 * at + col, r - 1));
     }
   };
   const int64_t stride = (int64_t)S * kStWaves * 32;
   const int64_t first = ((int64_t)s * kStWaves + wave) * 32;
   if (first < l) issue(first);
   for (int64_t t0 = first; t0 < l; t0 += stride) {
+    const int rows = (int)min((int64_t)32, l - t0);
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kWave + lane) * VEC;
-      *reinterpret_cast<gd_u32x4*>(&x_s[(e / D) * LDX + e % D]) = t0 + e / D < l ? pre[i] : gd_u32x4{0, 0, 0, 0};
+      *reinterpret_cast<gd_u32x4*>(&x_s[(e / D) * LDX + e % D]) = e / D < rows ? pre[i] : gd_u32x4{0, 0, 0, 0};
     }
     // the pieces of this group's rows of A: element v of a lane is row gd_mfma_row(lane, v) of its column, so eight at
     // a time are an operand's k elements (X comes out of LDS in the same order)
     gd_bf16x8 cp[GIVEN ? AT : 1][2][3];
     if constexpr (GIVEN) {
 #pragma unroll
-      for (int at = 0; at < AT; ++at)
+      for (int at = 0; at < AT; ++at) {
+        const int valid = (32 * at + col < r ? rows : 0) - 4 * half;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
           float f[8];
 #pragma unroll
-          for (int q = 0; q < 8; ++q)
-            f[q] = t0 + gd_mfma_row(lane, 8 * kb + q) < l && 32 * at + col < r ? arow[at][8 * kb + q] : 0.0f;
+          for (int q = 0; q < 8; ++q) f[q] = gd_mfma_row0(8 * kb + q) < valid ? arow[at][8 * kb + q] : 0.0f;
           gd_split3x8(f, cp[at][kb]);
         }
+      }
     }
     st_wave_sync();
     if (t0 + stride < l) issue(t0 + stride);
@@ -250,7 +253,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
   constexpr int NL = 32 * D / (kWave * VEC);
   extern __shared__ __align__(16) char ap_smem[];
   uint16_t* mt_s = reinterpret_cast<uint16_t*>(ap_smem);                                 // [3][32 AT][LDM]
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   T* x_s = reinterpret_cast<T*>(ap_smem + 3 * 32 * AT * LDM * 2) + wave * 32 * LDX;      // this wave's rows of X
   const int col = lane & 31, half = lane >> 5;
   const int h = blockIdx.y, s = blockIdx.x;
@@ -267,10 +270,11 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
   }
   gd_u32x4 pre[NL];
   auto issue = [&](int64_t t0) {
+    const int last = (int)min((int64_t)32, l - t0) - 1;
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kWave + lane) * VEC;
-      pre[i] = *reinterpret_cast<const gd_u32x4*>(Xh + min(t0 + e / D, l - 1) * D + e % D);
+      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * (uint32_t)sizeof(T));
     }
   };
   const int64_t stride = (int64_t)S * NW * 32;
@@ -318,11 +322,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
     }
 #pragma unroll
     for (int at = 0; at < AT; ++at)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t row = t0 + gd_mfma_row(lane, v);
-        if (row < l && 32 * at + col < r) gd_store(Ah, row * r + 32 * at + col, c[at][v]);
-      }
+      gd_store_tile(Ah + t0 * r, c[at], (int)min((int64_t)32, l - t0), 32 * at + col, half, r);
     st_wave_sync();  // this wave's reads of the tile precede its next staging writes
   }
 }

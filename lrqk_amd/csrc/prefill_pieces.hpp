@@ -15,6 +15,24 @@ typedef gd_v4s __attribute__((address_space(3))) * gd_lds_v4s;
 // C tile of a 32x32 matrix product: lane l, element v -> row (the column is l % 32)
 __device__ __forceinline__ int gd_mfma_row(int lane, int v) { return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3); }
 
+// the row of lane 0 in element v; the upper half of a wave is 4 rows further
+__device__ __forceinline__ constexpr int gd_mfma_row0(int v) { return ((v >> 2) << 3) + (v & 3); }
+
+// Rows of a group are addressed by 32-bit byte offsets from the group's first row, an address that the whole wave
+// shares (its wave's number made uniform by gd_wave): the load takes a scalar base and one register.  A 64-bit product
+// per row and lane costs 16 cycles: 48 of them were a third of a step's vector instructions in the kernels that sum over
+// the rows (32 heads of 32K bf16 rows, rank 32: K side's sums 64 -> 57 us, A_K 50 -> 46 us; three prompts of 2531 rows of
+// 64: 19.2 -> 16.7 us; 16K rows at rank 64, A_K 38.6 -> 33.6 us).
+__device__ __forceinline__ int gd_wave() { return __builtin_amdgcn_readfirstlane(wave_id()); }
+template <typename V>
+__device__ __forceinline__ V gd_at(const void* base, uint32_t bytes) {
+  return *reinterpret_cast<const V*>((const char*)base + bytes);
+}
+// element `col` of row min(row, last) of a group of rows of r floats (r < 2^22)
+__device__ __forceinline__ float gd_factor(const float* base, int row, int last, int r, int col) {
+  return gd_at<float>(base, __umul24((uint32_t)min(row, last), 4u * (uint32_t)r) + 4u * (uint32_t)col);
+}
+
 // An fp32 number as the exact sum of three bf16 numbers (8 + 8 + 8 mantissa bits, by truncation), as the upper halves
 // of fp32 bit patterns
 __device__ __forceinline__ void gd_split3(float x, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
@@ -41,5 +59,20 @@ __device__ __forceinline__ void gd_split3x8(const float (&x)[8], gd_bf16x8 (&p)[
 // is a branch per value in the kernels that write whole factors.
 __device__ __forceinline__ void gd_store(float* p, int64_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void gd_store(bf16_t* p, int64_t i, float v) { p[i].v = __builtin_bit_cast(uint16_t, (__bf16)v); }
+
+// The first `rows` rows (32, or fewer at the end of a head) of a C tile to rows of r factors from `base` on.
+template <typename OUT>
+__device__ __forceinline__ void gd_store_tile(OUT* base, const gd_floatx16& c, int rows, int col, int half, int r) {
+  if (col >= r) return;
+  const uint32_t at = (uint32_t)(4 * half * r + col) * (uint32_t)sizeof(OUT);
+  if (rows >= 32) {  // (wave-uniform)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) gd_store((OUT*)((char*)(base + gd_mfma_row0(v) * r) + at), 0, c[v]);
+  } else {
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (gd_mfma_row0(v) + 4 * half < rows) gd_store((OUT*)((char*)(base + gd_mfma_row0(v) * r) + at), 0, c[v]);
+  }
+}
 
 }  // namespace lrqk
