@@ -1122,8 +1122,8 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
                        xk_part, Sxk);
     LRQK_HIP_CHECK(hipGetLastError());
   } else {
-    if ((rc = prefill_stream_sums<T>(q, hq, hq, b, l, r, d, a_q0, partQ, S, xq_part, Sx, st))) return rc;
-    if ((rc = prefill_stream_sums<T>(k, hkv, hq, b, l, r, d, a_k0, partK, S, xk_part, Sxk, st))) return rc;
+    if ((rc = prefill_stream_sums<T>(q, k, hq, hkv, b, l, r, d, a_q0, a_k0, partQ, partK, S, xq_part, xk_part, Sxk, st)))
+      return rc;
   }
 #define LRQK_GD_RUN(RTV, DV) gramdom_run<RTV, DV>(a, xq_part, Sx, xk_part, Sxk, bkv, Sq, Sk, iters, st)
   rc = d == 64 ? (RP == 16 ? LRQK_GD_RUN(1, 64) : RP == 32 ? LRQK_GD_RUN(2, 64) : LRQK_GD_RUN(4, 64))
@@ -1137,12 +1137,12 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
       return rcs ? rcs : prefill_store<OUT>(a_k0, l * r, a_k, out.a_k_stride, l * r, bh, st);
     }
     const int64_t rows = out.a_q_rows;  // (the last ones)
-    int rcs = prefill_stream_apply<T, OUT>(q + (l - rows) * d, hq, hq, b, rows, l * d, r, d, a.Mt_q, a_q, rows * r, st);
-    if (rcs) return rcs;
     const int nh = hq / hkv;
-    if (tuned && (nh == 2 || nh == 4))
-      return apply_shared<OUT>(k, a.Mt_k, a_k, out.a_k_stride, bkv, nh, l, r, st);
-    return prefill_stream_apply<T, OUT>(k, hkv, hq, b, l, l * d, r, d, a.Mt_k, a_k, out.a_k_stride, st);
+    const bool shared = tuned && (nh == 2 || nh == 4);
+    int rcs = prefill_stream_apply<T, OUT>(shared ? nullptr : k, hkv, l, a.Mt_k, a_k, out.a_k_stride, q + (l - rows) * d, rows,
+                                           l * d, a.Mt_q, a_q, hq, b, r, d, st);
+    if (!rcs && shared) rcs = apply_shared<OUT>(k, a.Mt_k, a_k, out.a_k_stride, bkv, nh, l, r, st);
+    return rcs;
   };
   if (out.storage && sizeof(T) == 2) return finish((T*)out.a_q, (T*)out.a_k);
   return finish((float*)out.a_q, (float*)out.a_k);

@@ -8,8 +8,9 @@
 // product of two pieces is exact in fp32, and all piece pairs but lo x lo (2^-32) are formed.  Both are bound by HBM
 // (every input read once), so the shape of the kernels follows the memory: a wave streams 32-row groups of its own
 // through a private LDS tile, the next group already requested, and never meets another wave before the end.
-// 32 heads of 16384 bf16 rows of 128, rank 64: sums over the given factors 98 us (268 MB; 20 us of matrix-core time),
-// Q^T Q 32 us, A_K 77 us; the row-by-row kernels for this rank took 1.3 ms per pass, ten passes for four iterations.
+// 32 heads of 16384 bf16 rows of 128, rank 64: all sums 193 us (435 MB; two waves' worth of matrix-core and vector work
+// on one wave per SIMD, which the accumulators leave room for), A_K 34 us; the row-by-row kernels for this rank took
+// 1.3 ms per pass, ten passes for four iterations.
 #include <algorithm>
 
 #include "common.hpp"
@@ -46,17 +47,22 @@ __device__ __forceinline__ gd_floatx16 st_product(const gd_bf16x8 (&a)[2][PA], c
   return t;
 }
 
+template <typename T>
+constexpr int st_sums_smem(int db) {  // bytes of LDS: the waves' tiles, or their sums on the way out
+  const int tile = 32 * (32 * db + (sizeof(T) == 4 ? 8 : 16)) * (int)sizeof(T);
+  return kStWaves * (tile > 4096 ? tile : 4096);
+}
+
 // AT: 32-column tiles of A (ranks up to 32, 64); DB: 32-column blocks of X (64, 128 elements); GIVEN: sums over the
-// given factors, a head per query head (X of its kv head); XTX: X^T X, a head per head of X.  Both in one launch where
-// the accumulators allow it (DB = 2: up to 10 tiles; DB = 4 would need 15 to 21 of 16 registers each beside the
-// operands), else one launch each.
-// grid (S, heads); 4 waves; split s of a head takes every S-th set of 4 x 32 rows, so the workgroups of a head walk its
+// given factors, a head per query head (X of its kv head); XTX: X^T X, a head per head of X.  Both from one reading of X
+// where the accumulators allow it (DB = 2: up to 10 tiles; DB = 4 would need 15 to 21 of 16 registers each beside the
+// operands), else by workgroups of their own.
+// Split s of S of head h; 4 waves; a split takes every S-th set of 4 x 32 rows, so the workgroups of a head walk its
 // rows side by side.  part: [head][S][r][r + d]; xtx_part: [head][S][d][d] (both triangles).
 template <typename T, int AT, int DB, bool GIVEN, bool XTX>
-__global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __restrict__ X, int xh, int hq, int64_t l,
-                                                                    int r, const float* __restrict__ A,
-                                                                    float* __restrict__ part,
-                                                                    float* __restrict__ xtx_part, int S) {
+__device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* __restrict__ X, int xh, int hq, int64_t l,
+                                             int r, const float* __restrict__ A, float* __restrict__ part,
+                                             float* __restrict__ xtx_part, int S) {
   constexpr int D = 32 * DB;
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int P = F32 ? 3 : 1;
@@ -65,13 +71,10 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __r
   // read takes one column of rows 4 apart in the wave's halves, which 8 floats of padding put 32 banks apart
   constexpr int LDX = F32 ? D + 8 : D + 16;
   constexpr int NL = 32 * D / (kWave * VEC);
-  constexpr int TILE = 32 * LDX * (int)sizeof(T);
-  constexpr int SMEM = kStWaves * (TILE > 4096 ? TILE : 4096);
-  __shared__ __align__(16) char smem[SMEM];
+  constexpr int SMEM = st_sums_smem<T>(DB);
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   T* x_s = reinterpret_cast<T*>(smem + wave * (SMEM / kStWaves));
-  const int h = blockIdx.y, s = blockIdx.x;
   const int64_t xhead = GIVEN ? (int64_t)(h / hq) * xh + (h % hq) / (hq / xh) : h;
   const T* Xh = X + xhead * l * D;
   const float* Ah = A + (int64_t)h * l * r;
@@ -237,13 +240,62 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(const T* __r
   }
 }
 
-// A = X M for every query head (l rows of its kv head's X, heads x_stride elements apart): M^T (fp32, [head][r][d]) in LDS as three bf16 pieces, X through the
-// wave's private tile.  A: OUT, heads `a_stride` elements apart, rows of r.  grid (S, query heads); the workgroups of
+// The sums of both sides in one launch: one after the other they were up to four, 15 us each of a short prompt's host
+// time, and each with a last round of workgroups that left most of the GPU idle (4096 fp32 rows of 28 heads, rank 16:
+// 106 -> 73 us; three prompts of 2531 rows of 64: 44 -> 27; rank 64, 16K rows: 237 -> 193).  Workgroups in order: Q's sums
+// over the given factors [bh * S], K's [bh * S], Q^T Q [bh * S], K^T K [bkv * Sxk]; FUSED_Q / FUSED_K: the side's X^T X
+// comes with its sums.
+struct StSums {
+  const void *q, *k;
+  const float *a_q, *a_k;
+  float *part_q, *part_k, *xq_part, *xk_part;
+  int64_t l;
+  int hq, hkv, r, S, Sxk, given;  // given: workgroups of one side's sums over the given factors
+};
+template <typename T, int AT, int DB, bool FUSED_Q, bool FUSED_K>
+__global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(StSums g) {
+  __shared__ __align__(16) char smem[st_sums_smem<T>(DB)];
+  const T *q = (const T*)g.q, *k = (const T*)g.k;
+  int w = blockIdx.x;
+  if (w < g.given) {
+    st_sums_body<T, AT, DB, true, FUSED_Q>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, g.a_q, g.part_q, g.xq_part, g.S);
+    return;
+  }
+  w -= g.given;
+  if (w < g.given) {
+    st_sums_body<T, AT, DB, true, FUSED_K>(smem, w / g.S, w % g.S, k, g.hkv, g.hq, g.l, g.r, g.a_k, g.part_k, g.xk_part, g.S);
+    return;
+  }
+  w -= g.given;
+  if constexpr (!FUSED_Q) {
+    if (w < g.given) {
+      st_sums_body<T, 1, DB, false, true>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, nullptr, nullptr, g.xq_part, g.S);
+      return;
+    }
+    w -= g.given;
+  }
+  if constexpr (!FUSED_K)
+    st_sums_body<T, 1, DB, false, true>(smem, w / g.Sxk, w % g.Sxk, k, g.hkv, g.hq, g.l, g.r, nullptr, nullptr, g.xk_part,
+                                        g.Sxk);
+}
+
+// A = X M for every query head (its kv head's X): M^T (fp32, [head][r][d]) in LDS as three bf16 pieces, X through the
+// wave's private tile.  One launch for the sides given: workgroups (s, head) with s below side[0].S are the first side's
+// splits, the others the second's (a cache asks for one row of A_Q: alone that is a launch and 8 us).  The workgroups of
 // the query heads that share a kv head lie next to each other, so K comes from the caches after the first of them.
+template <typename T, typename OUT>
+struct StApply {
+  const T* x;
+  int xh, S;          // heads of x per sequence; splits of the rows (0: no such side)
+  int64_t l, x_stride;  // rows; elements between the heads of x
+  const float* mt;
+  OUT* a;             // heads a_stride elements apart, rows of r
+  int64_t a_stride;
+};
 template <typename T, int AT, int DB, typename OUT>
-__global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_apply_kernel(
-    const T* __restrict__ X, int xh, int hq, int64_t l, int64_t x_stride, int r, const float* __restrict__ Mt,
-    OUT* __restrict__ A, int64_t a_stride, int S) {
+__global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_apply_kernel(StApply<T, OUT> first_side,
+                                                                                          StApply<T, OUT> second_side,
+                                                                                          int hq, int r) {
   constexpr int D = 32 * DB;
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int NW = F32 ? 4 : 8, NT = NW * kWave;
@@ -256,9 +308,14 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   T* x_s = reinterpret_cast<T*>(ap_smem + 3 * 32 * AT * LDM * 2) + wave * 32 * LDX;      // this wave's rows of X
   const int col = lane & 31, half = lane >> 5;
-  const int h = blockIdx.y, s = blockIdx.x;
-  const T* Xh = X + ((int64_t)(h / hq) * xh + (h % hq) / (hq / xh)) * x_stride;
-  OUT* Ah = A + (int64_t)h * a_stride;
+  const int h = blockIdx.y;
+  const bool second = (int)blockIdx.x >= first_side.S;
+  const StApply<T, OUT>& g = second ? second_side : first_side;
+  const int s = second ? (int)blockIdx.x - first_side.S : (int)blockIdx.x, S = g.S;
+  const int64_t l = g.l;
+  const float* __restrict__ Mt = g.mt;
+  const T* __restrict__ Xh = g.x + ((int64_t)(h / hq) * g.xh + (h % hq) / (hq / g.xh)) * g.x_stride;
+  OUT* __restrict__ Ah = g.a + (int64_t)h * g.a_stride;
   for (int e = tid; e < 32 * AT * D; e += NT) {
     const int n = e / D, k = e % D;
     const float v = n < r ? Mt[((int64_t)h * r + n) * D + k] : 0.0f;
@@ -349,37 +406,35 @@ template int prefill_store<float>(const float*, int64_t, float*, int64_t, int64_
 template int prefill_store<bf16_t>(const float*, int64_t, bf16_t*, int64_t, int64_t, int, hipStream_t);
 
 template <typename T, int AT, int DB>
-static int sums_impl(const T* x, int xh, int hq, int b, int64_t l, int r, const float* a, float* part, int S, float* xtx,
-                     int Sx, hipStream_t st) {
-  const dim3 given((unsigned)S, (unsigned)(b * hq)), heads((unsigned)Sx, (unsigned)(b * xh)), blk(kStThreads);
-  if (DB == 2 && xh == hq && S == Sx) {
-    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, 2, true, true>), given, blk, 0, st, x, xh, hq, l, r, a, part, xtx, S);
-  } else {
-    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, true, false>), given, blk, 0, st, x, xh, hq, l, r, a, part, xtx, S);
-    hipLaunchKernelGGL((pf_stream_sums_kernel<T, 1, DB, false, true>), heads, blk, 0, st, x, xh, hq, l, r, a, part, xtx, Sx);
-  }
+static int sums_impl(const StSums& g, int b, hipStream_t st) {
+  const int bkv = b * g.hkv;
+  if (DB == 2 && g.hkv == g.hq && g.S == g.Sxk)
+    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, DB == 2, DB == 2>), dim3((unsigned)(2 * g.given)), dim3(kStThreads),
+                       0, st, g);
+  else
+    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, DB == 2, false>),
+                       dim3((unsigned)((DB == 2 ? 2 : 3) * g.given + bkv * g.Sxk)), dim3(kStThreads), 0, st, g);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
 
-// Sums of one side: over the given factors ([b * hq] heads, S splits) and X^T X ([b * xh] heads, Sx splits).
+// Sums of both sides: over the given factors ([b * hq] heads, S splits), Q^T Q ([b * hq] heads, S splits) and K^T K
+// ([b * hkv] heads, Sxk splits).
 template <typename T>
-int prefill_stream_sums(const T* x, int xh, int hq, int b, int64_t l, int r, int d, const float* a, float* part, int S,
-                        float* xtx, int Sx, hipStream_t st) {
-  if (d == 64)
-    return r <= 32 ? sums_impl<T, 1, 2>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st)
-                   : sums_impl<T, 2, 2>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st);
-  return r <= 32 ? sums_impl<T, 1, 4>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st)
-                 : sums_impl<T, 2, 4>(x, xh, hq, b, l, r, a, part, S, xtx, Sx, st);
+int prefill_stream_sums(const T* q, const T* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
+                        const float* a_k, float* part_q, float* part_k, int S, float* xq_part, float* xk_part, int Sxk,
+                        hipStream_t st) {
+  const StSums g{q, k, a_q, a_k, part_q, part_k, xq_part, xk_part, l, hq, hkv, r, S, Sxk, b * hq * S};
+  if (d == 64) return r <= 32 ? sums_impl<T, 1, 2>(g, b, st) : sums_impl<T, 2, 2>(g, b, st);
+  return r <= 32 ? sums_impl<T, 1, 4>(g, b, st) : sums_impl<T, 2, 4>(g, b, st);
 }
-template int prefill_stream_sums<float>(const float*, int, int, int, int64_t, int, int, const float*, float*, int, float*,
-                                        int, hipStream_t);
-template int prefill_stream_sums<bf16_t>(const bf16_t*, int, int, int, int64_t, int, int, const float*, float*, int, float*,
-                                         int, hipStream_t);
+template int prefill_stream_sums<float>(const float*, const float*, int, int, int, int64_t, int, int, const float*,
+                                        const float*, float*, float*, int, float*, float*, int, hipStream_t);
+template int prefill_stream_sums<bf16_t>(const bf16_t*, const bf16_t*, int, int, int, int64_t, int, int, const float*,
+                                         const float*, float*, float*, int, float*, float*, int, hipStream_t);
 
 template <typename T, int AT, int DB, typename OUT>
-static int apply_impl(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, const float* mt, OUT* a, int64_t a_stride,
-                      hipStream_t st) {
+static int apply_impl(StApply<T, OUT> g0, StApply<T, OUT> g1, int hq, int b, int r, hipStream_t st) {
   constexpr int D = 32 * DB, NW = sizeof(T) == 4 ? 4 : 8;
   constexpr size_t smem = (size_t)3 * 32 * AT * (D + 8) * 2 + (size_t)NW * 32 * (sizeof(T) == 4 ? D + 4 : D + 8) * sizeof(T);
   static_assert(smem <= 160 * 1024, "LDS");
@@ -393,28 +448,29 @@ static int apply_impl(const T* x, int xh, int hq, int b, int64_t l, int64_t x_st
   // every workgroup stages M (52 KB in, up to 104 KB of fp32 read): enough of them to fill the GPU once, no more
   const int bh = b * hq;
   const int per_cu = std::max(1, (int)(160 * 1024 / smem));
-  const int64_t S = std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (l + 32 * NW - 1) / (32 * NW)));
-  hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)bh), dim3(NW * kWave), smem, st, x, xh, hq, l, x_stride, r, mt, a, a_stride,
-                     (int)S);
+  for (StApply<T, OUT>* g : {&g0, &g1})
+    g->S = !g->x ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (g->l + 32 * NW - 1) / (32 * NW)));
+  hipLaunchKernelGGL(kern, dim3((unsigned)(g0.S + g1.S), (unsigned)bh), dim3(NW * kWave), smem, st, g0, g1, hq, r);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
 
-// A = X M for all b * hq query heads: l rows per head, X's heads x_stride and A's a_stride elements apart.
+// A_K = K Mk (l rows) and A_Q = Q Mq (q_rows rows) for all b * hq query heads; without k only the latter.  q: the first of
+// those rows, heads q_stride elements apart.
 template <typename T, typename OUT>
-int prefill_stream_apply(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, int d, const float* mt,
-                         OUT* a, int64_t a_stride, hipStream_t st) {
-  if (d == 64)
-    return r <= 32 ? apply_impl<T, 1, 2>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st)
-                   : apply_impl<T, 2, 2>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st);
-  return r <= 32 ? apply_impl<T, 1, 4>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st)
-                 : apply_impl<T, 2, 4>(x, xh, hq, b, l, x_stride, r, mt, a, a_stride, st);
+int prefill_stream_apply(const T* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride, const T* q,
+                         int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r, int d,
+                         hipStream_t st) {
+  const StApply<T, OUT> gk{k, hkv, 0, l, l * d, mt_k, a_k, a_k_stride};
+  const StApply<T, OUT> gq{q, hq, 0, q_rows, q_stride, mt_q, a_q, q_rows * r};
+  if (d == 64) return r <= 32 ? apply_impl<T, 1, 2>(gk, gq, hq, b, r, st) : apply_impl<T, 2, 2>(gk, gq, hq, b, r, st);
+  return r <= 32 ? apply_impl<T, 1, 4>(gk, gq, hq, b, r, st) : apply_impl<T, 2, 4>(gk, gq, hq, b, r, st);
 }
-template int prefill_stream_apply<float, float>(const float*, int, int, int, int64_t, int64_t, int, int, const float*,
-                                                float*, int64_t, hipStream_t);
-template int prefill_stream_apply<bf16_t, float>(const bf16_t*, int, int, int, int64_t, int64_t, int, int, const float*,
-                                                 float*, int64_t, hipStream_t);
-template int prefill_stream_apply<bf16_t, bf16_t>(const bf16_t*, int, int, int, int64_t, int64_t, int, int, const float*,
-                                                  bf16_t*, int64_t, hipStream_t);
+template int prefill_stream_apply<float, float>(const float*, int, int64_t, const float*, float*, int64_t, const float*,
+                                                int64_t, int64_t, const float*, float*, int, int, int, int, hipStream_t);
+template int prefill_stream_apply<bf16_t, float>(const bf16_t*, int, int64_t, const float*, float*, int64_t, const bf16_t*,
+                                                 int64_t, int64_t, const float*, float*, int, int, int, int, hipStream_t);
+template int prefill_stream_apply<bf16_t, bf16_t>(const bf16_t*, int, int64_t, const float*, bf16_t*, int64_t, const bf16_t*,
+                                                  int64_t, int64_t, const float*, bf16_t*, int, int, int, int, hipStream_t);
 
 }  // namespace lrqk

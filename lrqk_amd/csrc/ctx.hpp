@@ -202,11 +202,13 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
                         int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st);
 // Its passes over the long axis; see als_prefill_stream.hip (every shape) and als_prefill.hip (bf16 rows of 128, r <= 32).
 template <typename T>
-int prefill_stream_sums(const T* x, int xh, int hq, int b, int64_t l, int r, int d, const float* a, float* part, int S,
-                        float* xtx, int Sx, hipStream_t st);
+int prefill_stream_sums(const T* q, const T* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
+                        const float* a_k, float* part_q, float* part_k, int S, float* xq_part, float* xk_part, int Sxk,
+                        hipStream_t st);
 template <typename T, typename OUT>
-int prefill_stream_apply(const T* x, int xh, int hq, int b, int64_t l, int64_t x_stride, int r, int d, const float* mt,
-                         OUT* a, int64_t a_stride, hipStream_t st);
+int prefill_stream_apply(const T* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride, const T* q,
+                         int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r, int d,
+                         hipStream_t st);
 int prefill_given_sums_bf16(const bf16_t* x, int xh, int hq, int b, int64_t l, int r, float* a, float* part, int S,
                             hipStream_t st);
 template <typename OUT>
