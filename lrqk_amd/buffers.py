@@ -8,6 +8,9 @@ the newest token and relies on reading zeros there.
 """
 from __future__ import annotations
 
+import collections
+import math
+import threading
 from typing import Optional
 
 import torch
@@ -109,6 +112,25 @@ class AutoIncreaseTensor:
         return torch.take_along_dim(self.data, indices, self.dim if dim is None else dim, out=out)
 
 
+_ahead = threading.local()
+_AHEAD_BYTES = 1 << 30
+
+
+def _host_stores_ahead(device: torch.device, nbytes: int):
+    """Called before a store of ``nbytes`` is allocated.  A dropped cache's store is free once the GPU has done its work,
+    and the host queues a long prompt in a twentieth of the time that this takes (0.5 of 9.7 ms at 128K): a program that
+    makes a cache per prompt would hold a store for every prompt that it is ahead.  So the calling thread waits here as
+    long as the stores it has allocated since work that the GPU has not finished exceed 1 GiB, but never for the last."""
+    pending = _ahead.__dict__.setdefault(device.index, collections.deque())
+    while pending and pending[0][0].query():
+        pending.popleft()
+    while len(pending) > 1 and sum(n for _, n in pending) + nbytes > _AHEAD_BYTES:
+        pending.popleft()[0].synchronize()
+    mark = torch.cuda.Event()
+    mark.record(torch.cuda.current_stream(device))
+    pending.append((mark, nbytes))
+
+
 class AutoIncreaseTensorSharedKV(AutoIncreaseTensor):
     """K and V rows side by side on the last dim (lrqk_attention.py:959-963)."""
 
@@ -119,6 +141,8 @@ class AutoIncreaseTensorSharedKV(AutoIncreaseTensor):
         # through tensor()), so the store is not cleared: clearing 0.8 GB of pinned memory is 4 ms of a
         # 128K layer prefill.  (The factor buffer keeps the zero fill: it is gathered at full capacity.)
         pin = bool(self.pin_memory) and torch.cuda.is_available()
+        if pin and self.gpu is not None:
+            _host_stores_ahead(self.gpu, math.prod(shape) * self.dtype.itemsize)
         store = torch.empty(shape, device=self.device, dtype=self.dtype, pin_memory=pin)
         if pin and self.gpu is not None and store.numel():
             # torch hands a freed pinned block out again once the work that it knows to use it is done.  The kernels

@@ -91,6 +91,27 @@ def test_a_dropped_caches_store_waits_for_its_copies(ops, context, name):
     assert early and not same
 
 
+def test_a_host_ahead_of_the_gpu_holds_few_stores(ops, monkeypatch):
+    """A cache per prompt, each dropped before the GPU has come to it: the host waits instead of taking a pinned block for
+    every prompt that it is ahead (the newest and one before it here, and one on its way back)."""
+    from lrqk_amd import DynamicLRQKCache, buffers
+    monkeypatch.setattr(buffers, "_AHEAD_BYTES", 1)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn((1, 4, 3000, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    k, v = (torch.randn((1, 2, 3000, 64), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2))
+    places = set()
+    for _ in range(8):
+        cache = DynamicLRQKCache(r=16, num_active_tokens=128, max_iter=1, lite_tokens=16, tol=0.0,
+                                 max_sequence_length=3264, num_key_value_groups=2)
+        cache.update(q, k, v, 0)
+        places.add(cache.lwattn[0].KVcpu.data.data_ptr())
+        torch.cuda._sleep(30_000_000)
+        del cache
+    torch.cuda.synchronize()
+    print("blocks", len(places), flush=True)
+    assert len(places) <= 4
+
+
 @pytest.mark.parametrize("dtype,d,r,l,hq,hkv,iters", [
     (torch.float32, 64, 1, 128, 2, 2, 1),        # the fewest rows the Gram matrices take, one column of factors
     (torch.float32, 64, 16, 129, 6, 2, 2),       # a row beyond whole groups; three query heads per kv head
