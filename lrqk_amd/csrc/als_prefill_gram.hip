@@ -13,8 +13,8 @@
 //     Mk'^T = (Gq' + B_K B_K^T)^-1 (T + B_K)          U = Mk'^T Sk      Gk' = Mk'^T U^T     Ck' = U
 // and this holds from the first iteration on (there G, C come from the given initial factors).  The long
 // axis is read for Sq, Sk and the initial (G, C) before the loop and once more at the end, to form
-// A_Q = Q Mq and A_K = K Mk: six passes whatever the iteration count, where the row-by-row formulation
-// makes two per iteration plus two.
+// A_Q = Q Mq and A_K = K Mk, whatever the iteration count; the row-by-row formulation reads it twice per
+// iteration and twice more.
 //
 // Sq and Sk square the condition number of the inputs, so the d x d algebra is done in fp64 (vector
 // ALU: these are 32 independent problems of a few MFLOP each); the sums Sq, Sk themselves are exact

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void flush_ring_kernel(const uint4* __restrict
 }
 
 // A prompt's K and V rows side by side, [K row | V row] per token, in device memory: the form of the host store, so
-// that one wide copy by a DMA engine moves them (lrqk_store_prompt).  Bound by HBM (every byte read and written once):
+// that one wide copy by a DMA engine moves them (lrqk_store_rows).  Bound by HBM (every byte read and written once):
 // a workgroup takes 256 / chunks tokens at a time, one 16-byte chunk per thread, four such groups in flight.
 // 131072 tokens of 8 heads, 512-byte rows: 1.07 GB in 0.18 ms (6 TB/s).
 __global__ __launch_bounds__(256) void interleave_kv_kernel(const uint4* __restrict__ k, const uint4* __restrict__ v,
@@ -400,7 +400,7 @@ extern "C" int lrqk_fill_active(const void* k, const void* v, int64_t l, int32_t
   int rc = check_rows(b, hq, hkv, d, dtype, &cpr);
   if (rc) return rc;
   LRQK_REQUIRE(k && v && active_idx && k_act && v_act, LRQK_EINVAL, "null pointer");
-  LRQK_REQUIRE(topk > 0 && lite > 0 && l >= (int64_t)topk + lite && l < ((int64_t)1 << 31), LRQK_EINVAL,
+  LRQK_REQUIRE(topk > 0 && lite >= 0 && l >= (int64_t)topk + lite && l < ((int64_t)1 << 31), LRQK_EINVAL,
                "a prompt of %lld tokens for %d + %d slots", (long long)l, topk, lite);
   LRQK_REQUIRE(aligned16(k) && aligned16(v) && aligned16(k_act) && aligned16(v_act), LRQK_EINVAL,
                "pointers must be 16-byte aligned");

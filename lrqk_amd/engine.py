@@ -364,10 +364,14 @@ class LightAttentionIndicesFactory:
             ahead = max(1, b * hkv // 8)
             pieces = tuple((k[:, h], v[:, h], rows_of[:, h]) for h in (slice(0, ahead), slice(ahead, None)))
         rows = []
-        for k, v, out in pieces:
-            rows.append(ops.interleave_kv(k, v))
-            side.wait_stream(torch.cuda.current_stream(dev))
-            ops.store_rows(rows[-1], out, row0, side)
+        try:
+            for k, v, out in pieces:
+                rows.append(ops.interleave_kv(k, v))
+                side.wait_stream(torch.cuda.current_stream(dev))
+                ops.store_rows(rows[-1], out, row0, side)
+        except BaseException:  # the first copy may be under way from a block that this frame is about to release
+            torch.cuda.current_stream(dev).wait_stream(side)
+            raise
         return side, rows
 
     # ------------------------------------------------------------------ decode

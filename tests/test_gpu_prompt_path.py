@@ -177,10 +177,10 @@ def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
 
 
 @pytest.mark.parametrize("dtype,hq,hkv,d,l,k,lite", [(torch.float32, 2, 1, 8, 12, 8, 4), (torch.bfloat16, 6, 2, 64, 515, 33, 7),
-                                                     (torch.float32, 4, 4, 256, 300, 100, 1)])
+                                                     (torch.float32, 4, 4, 256, 300, 100, 1), (torch.bfloat16, 4, 2, 64, 90, 16, 0)])
 def test_active_set_of_a_prompt(ops, dtype, hq, hkv, d, l, k, lite):
     """Selected rows, then the last tokens' rows and ids (a prompt that just fills the set, slots beyond whole rounds of
-    a workgroup, rows of two and of 128 chunks)."""
+    a workgroup, rows of two and of 128 chunks, no ring)."""
     gen = torch.Generator(device=DEV).manual_seed(l)
     K = torch.randn((2, hkv, l, d), generator=gen, device=DEV).to(dtype)
     V = torch.randn((2, hkv, l, d), generator=gen, device=DEV).to(dtype)
