@@ -121,6 +121,8 @@ def test_a_host_ahead_of_the_gpu_holds_few_stores(ops, monkeypatch):
     (torch.bfloat16, 128, 48, 257, 8, 2, 3),
     (torch.float32, 128, 64, 2531, 2, 1, 4),
     (torch.bfloat16, 128, 64, 9001, 2, 1, 4),
+    (torch.bfloat16, 128, 24, 1055, 8, 2, 2),    # four and two query heads from one reading of K: rows of whole groups
+    (torch.bfloat16, 128, 18, 300, 4, 2, 2),     # of four factors, rows that are none
     (torch.float32, 128, 40, 700, 2, 1, 0),      # no iteration: the given factors are the result
 ])
 def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
