@@ -310,12 +310,10 @@ __global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __re
 // ----------------------------------------------------------------------------- A = X Mt^T for heads that share X
 // The K side's last pass: the NH query heads of a kv head take their rows of A_K from the same rows of K, so one
 // workgroup stages 128 rows of K per step (as pf_xtx_kernel does) and applies the NH heads' Mt to them: K is read
-// once per kv head instead of once per query head.  Wave w takes head w / (8 / NH) and NH / 2 of the step's four 32-row
-// groups; 24 products of 32x32x16 per group (X times the three bf16 pieces of Mt), fp32 accuracy as in the row-by-row
-// pass.  A wave keeps its head's Mt in registers (24 operands of four): read from LDS for every group it was three of
-// four LDS reads, 512 KB per step and CU where the products take 3072 cycles.  The rows of K alternate between two
-// buffers, so a step has one barrier.  grid (S, kv heads); split s takes the steps s, s + S, ...
-// 8 heads of 32K rows, four query heads each, rank 32: 48.5 -> 45.9 us (134 MB).
+// once per kv head instead of once per query head.  Mt (fp32) lies in LDS as three bf16 pieces per head, X as it
+// is; wave w takes head w / (8 / NH) and NH / 2 of the step's four 32-row groups; 24 products of 32x32x16 per
+// group (X times the three pieces), fp32 accuracy as in the row-by-row pass.  grid (S, kv heads); split s takes
+// the steps s, s + S, ...
 constexpr int kApLd = kXtxD + 8;  // bf16 elements per staged row: 16-byte operand reads want rows 4 banks apart
 template <int NH, typename OUT>
 __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16_t* __restrict__ X, int64_t l,
@@ -323,6 +321,8 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
                                                                       OUT* __restrict__ A, int64_t a_stride, int S) {
   static_assert(NH == 2 || NH == 4, "query heads per kv head");
   extern __shared__ __align__(16) uint16_t ap_s[];
+  uint16_t* x_s = ap_s;                          // [128][kApLd]
+  uint16_t* mt_s = ap_s + kXtxRows * kApLd;      // [NH][3][32][kApLd]
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
   const int xh = blockIdx.y, s = blockIdx.x;
@@ -330,27 +330,14 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
   constexpr int WPH = kXtxWaves / NH, GPW = 4 / WPH;  // waves per head, row groups per wave and step
   const int hl = wave / WPH, g0 = (wave % WPH) * GPW;
   OUT* Ah = A + ((int64_t)xh * NH + hl) * a_stride;
-  constexpr int KB = kXtxD / 16;
-  gd_bf16x8 m[KB][3];  // lane (col, half): row col of this head's Mt, elements 16 kb + 8 half ..
-  {
-    const float* row = Mt + (((int64_t)xh * NH + hl) * r + min(col, r - 1)) * kXtxD + 8 * half;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      union {
-        uint16_t u[8];
-        gd_bf16x8 v;
-      } o[3];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        uint32_t p0, p1, p2;
-        gd_split3(col < r ? row[16 * kb + j] : 0.0f, p0, p1, p2);
-        o[0].u[j] = (uint16_t)(p0 >> 16);
-        o[1].u[j] = (uint16_t)(p1 >> 16);
-        o[2].u[j] = (uint16_t)(p2 >> 16);
-      }
-#pragma unroll
-      for (int pp = 0; pp < 3; ++pp) m[kb][pp] = o[pp].v;
-    }
+  for (int e = tid; e < NH * 32 * kXtxD; e += kXtxThreads) {
+    const int hh = e / (32 * kXtxD), n = (e / kXtxD) % 32, k = e % kXtxD;
+    const float v = n < r ? Mt[(((int64_t)xh * NH + hh) * r + n) * kXtxD + k] : 0.0f;
+    uint32_t p0, p1, p2;
+    gd_split3(v, p0, p1, p2);
+    mt_s[((hh * 3 + 0) * 32 + n) * kApLd + k] = (uint16_t)(p0 >> 16);
+    mt_s[((hh * 3 + 1) * 32 + n) * kApLd + k] = (uint16_t)(p1 >> 16);
+    mt_s[((hh * 3 + 2) * 32 + n) * kApLd + k] = (uint16_t)(p2 >> 16);
   }
   constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);
   static_assert(NL == 4, "four 16-byte loads per thread and step");
@@ -366,43 +353,40 @@ __global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16
     pre2 = ld(2);
     pre3 = ld(3);
   };
+  auto stage = [&](int i, const uint4& v) {
+    const int e = (i * kXtxThreads + tid) * 8;
+    *reinterpret_cast<uint4*>(&x_s[(e / kXtxD) * kApLd + e % kXtxD]) = v;  // (rows beyond l are never stored from)
+  };
   const int64_t stride = (int64_t)S * kXtxRows;
   const int64_t first = (int64_t)s * kXtxRows;
   if (first < l) issue(first);
-  uint16_t* x_s = ap_s;  // [2][128][kApLd], the half of this step
   for (int64_t t0 = first; t0 < l; t0 += stride) {
-    auto stage = [&](int i, const uint4& v) {
-      const int e = (i * kXtxThreads + tid) * 8;
-      *reinterpret_cast<uint4*>(&x_s[(e / kXtxD) * kApLd + e % kXtxD]) = v;  // (rows beyond l are never stored from)
-    };
     stage(0, pre0);
     stage(1, pre1);
     stage(2, pre2);
     stage(3, pre3);
-    // (whoever is past this barrier has done with the step before, whose half the next step overwrites)
-    __syncthreads();
+    __syncthreads();  // (the first one also covers the staging of Mt)
     if (t0 + stride < l) issue(t0 + stride);
-    gd_floatx16 c[GPW];
-#pragma unroll
-    for (int j = 0; j < GPW; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) c[j][v] = 0.0f;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int pp = 0; pp < 3; ++pp)
-#pragma unroll
-        for (int j = 0; j < GPW; ++j) {
-          const gd_bf16x8 xa =
-              *reinterpret_cast<const gd_bf16x8*>(&x_s[(32 * (g0 + j) + col) * kApLd + kb * 16 + 8 * half]);
-          c[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, m[kb][pp], c[j], 0, 0, 0);
-        }
 #pragma unroll
     for (int j = 0; j < GPW; ++j) {
-      const int64_t row0 = t0 + 32 * (g0 + j);
-      if (row0 < l) gd_store_tile(Ah + row0 * r, c[j], (int)min((int64_t)32, l - row0), col, half, r);
+      const int g = g0 + j;
+      if (t0 + 32 * g >= l) continue;  // (wave-uniform)
+      gd_floatx16 c;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) c[v] = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < kXtxD / 16; ++kb) {
+        const gd_bf16x8 xa = *reinterpret_cast<const gd_bf16x8*>(&x_s[(32 * g + col) * kApLd + kb * 16 + 8 * half]);
+#pragma unroll
+        for (int pp = 0; pp < 3; ++pp) {
+          const gd_bf16x8 m =
+              *reinterpret_cast<const gd_bf16x8*>(&mt_s[((hl * 3 + pp) * 32 + col) * kApLd + kb * 16 + 8 * half]);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, m, c, 0, 0, 0);
+        }
+      }
+      gd_store_tile(Ah + (t0 + 32 * g) * r, c, (int)min((int64_t)32, l - t0 - 32 * g), col, half, r);
     }
-    x_s = x_s == ap_s ? ap_s + kXtxRows * kApLd : ap_s;
+    __syncthreads();
   }
 }
 
@@ -410,7 +394,7 @@ template <typename OUT>
 static int apply_shared(const void* k, const float* mt_k, OUT* a_k, int64_t a_stride, int bkv, int nh, int64_t l, int r,
                         hipStream_t st) {
   const int S = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + kXtxRows - 1) / kXtxRows));
-  const size_t smem = (size_t)2 * kXtxRows * kApLd * sizeof(uint16_t);
+  const size_t smem = (size_t)(kXtxRows + nh * 3 * 32) * kApLd * sizeof(uint16_t);
   auto kern = nh == 2 ? pf_apply_shared_kernel<2, OUT> : pf_apply_shared_kernel<4, OUT>;
   LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
   hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)bkv), dim3(kXtxThreads), smem, st, (const bf16_t*)k, l, mt_k, r,
