@@ -248,7 +248,7 @@ int lrqk_als_decode(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64_t head
  * a_q,a_k: [bh][l][r] fp32 work buffers holding the initial factors on entry and the
  * result on return; b_q,b_k out: [bh][r][d] fp32.  The stopping test (batch-wide mean squared
  * change of A_Q and A_K below tol) is evaluated on the device: once it fires the remaining
- * launches return at once, and the host never waits.  Rows of 64 or 128 elements (16-byte aligned): the
+ * launches return at once, and the host never waits.  bf16 rows of 64 or 128 elements (16-byte aligned): the
  * iterations run on d x d Gram matrices in fp64 and the long axis is read twice whatever max_iter is (sums and result
  * on the bf16 matrix cores, fp32 operands as three bf16 pieces, fp32 accumulation).  Other shapes row by row: r <= 32 on
  * bf16 or fp32 matrix-core tiles, ranks up to 64 (README.md:124-131 of the reference names r = 64) on a general kernel,

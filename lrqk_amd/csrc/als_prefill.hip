@@ -1087,12 +1087,18 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   const int iters = max_iter > 0 ? max_iter : 0;
   const bool aligned = ((uintptr_t)q % 16 == 0) && ((uintptr_t)k % 16 == 0);
   // Every iteration on d x d Gram matrices in fp64, the rows read twice (sums, result) whatever the iteration count:
-  // rows of 64 or 128 elements.  A prompt of fewer rows than two Gram matrices has is left to the row-by-row
+  // bf16 rows of 64 or 128 elements.  A prompt of fewer rows than two Gram matrices has is left to the row-by-row
   // formulation (X^T X is then no smaller than X, and with about as many rows as the rank both are ill-posed), except
-  // bf16 rows of 128 elements at ranks up to 32.
-  const bool gram_domain = aligned && (d == 64 || d == 128) && !getenv("LRQK_PREFILL_ROWWISE") &&
-                           ((sizeof(T) == 2 && d == 128 && r <= 32) || l >= 2 * d);
-  if (gram_domain) return prefill_gram_domain<T>(ctx, (const T*)q, (const T*)k, a_q, a_k, out, b, hq, hkv, l, r, d, iters, tol, st);
+  // rows of 128 elements at ranks up to 32.
+  // fp32 rows stay with the row-by-row formulation.  Its factors are 5e-6 .. 8e-5 off the ones from Gram matrices, and a
+  // decode step of an ill-conditioned head makes up to 4e-4 of that (a token at the edge of the active set changes
+  // places): more than fp32 results may move, whichever side is the closer one.
+  if constexpr (sizeof(T) == 2) {
+    const bool gram_domain = aligned && (d == 64 || d == 128) && !getenv("LRQK_PREFILL_ROWWISE") &&
+                             ((d == 128 && r <= 32) || l >= 2 * d);
+    if (gram_domain)
+      return prefill_gram_domain(ctx, (const T*)q, (const T*)k, a_q, a_k, out, b, hq, hkv, l, r, d, iters, tol, st);
+  }
   const bool mfma = r <= 32 && d % VEC == 0 && d <= 256 && aligned;
   const bool small32 = r <= 32 && d <= kPfSmallThreads - 32 && d % 4 == 0;
   LRQK_REQUIRE(mfma || ne <= kPfThreads * kPfMaxPer, LRQK_ELIMIT, "r*(r+d)=%d exceeds %d", ne, kPfThreads * kPfMaxPer);

@@ -1,4 +1,4 @@
-// Prefill factorisation, iterations carried out on Gram matrices (rows of 64 or 128 elements, r <= 64).
+// Prefill factorisation, iterations carried out on Gram matrices (bf16 rows of 64 or 128 elements, r <= 64).
 //
 // After the first half-step of lrqk_attention.py:359-421 every factor is a linear image of its input,
 // A_Q = Q Mq and A_K = K Mk with Mq, Mk of size d x r.  Everything an iteration needs from the long axis
@@ -1051,13 +1051,12 @@ static int gramdom_run(const GdArgs& a, const float* xq_part, int Sx, const floa
 
 // The whole factorisation on Gram matrices: q [b][hq][l][d], k [b][hkv][l][d], 16-byte aligned, d = 64 or 128, r <= 64;
 // a_q0, a_k0: the given factors, fp32 [b hq][l][r].
-template <typename T>
-int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, float* a_k0, const PrefillOut& out, int b, int hq,
-                        int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st) {
+int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* a_q0, float* a_k0, const PrefillOut& out,
+                        int b, int hq, int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st) {
   const int bh = b * hq, bkv = b * hkv;
-  // bf16 rows of 128 elements and ranks up to 32 have kernels of their own for the passes: the Q side's sums with Q^T Q
+  // rows of 128 elements and ranks up to 32 have kernels of their own for the passes: the Q side's sums with Q^T Q
   // from one reading of Q, K^T K alone, A_K for several query heads from one reading of K
-  const bool tuned = sizeof(T) == 2 && d == 128 && r <= 32;
+  const bool tuned = d == 128 && r <= 32;
   const int RP = r <= 16 ? 16 : r <= 32 ? 32 : 64;
   const size_t ne = (size_t)r * (r + d), dd = (size_t)d * d;
   // Splits of the long axis: one workgroup per CU and launch (the kernels' registers), at most 4096 rows per split
@@ -1106,7 +1105,7 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
   a.S = a.S_k = S;
   a.b_q = out.b_q;
   a.b_k = out.b_k;
-  a.out_bf16 = out.storage && sizeof(T) == 2;
+  a.out_bf16 = out.storage;
   a.bh = bh;
   a.hq = hq;
   a.hkv = hkv;
@@ -1115,14 +1114,14 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
   a.tol = tol;
 
   if (tuned) {
-    hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)S, (unsigned)bh), dim3(kXtxThreads), 0, st, (const bf16_t*)q, l, a_q0, r,
+    hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)S, (unsigned)bh), dim3(kXtxThreads), 0, st, q, l, a_q0, r,
                        partQ, xq_part, S);
-    if ((rc = prefill_given_sums_bf16((const bf16_t*)k, hkv, hq, b, l, r, a_k0, partK, S, st))) return rc;
-    hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sxk, (unsigned)bkv), dim3(kXtxThreads), 0, st, (const bf16_t*)k, l,
-                       xk_part, Sxk);
+    if ((rc = prefill_given_sums_bf16(k, hkv, hq, b, l, r, a_k0, partK, S, st))) return rc;
+    hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sxk, (unsigned)bkv), dim3(kXtxThreads), 0, st, k, l, xk_part,
+                       Sxk);
     LRQK_HIP_CHECK(hipGetLastError());
   } else {
-    if ((rc = prefill_stream_sums<T>(q, k, hq, hkv, b, l, r, d, a_q0, a_k0, partQ, partK, S, xq_part, xk_part, Sxk, st)))
+    if ((rc = prefill_stream_sums(q, k, hq, hkv, b, l, r, d, a_q0, a_k0, partQ, partK, S, xq_part, xk_part, Sxk, st)))
       return rc;
   }
 #define LRQK_GD_RUN(RTV, DV) gramdom_run<RTV, DV>(a, xq_part, Sx, xk_part, Sxk, bkv, Sq, Sk, iters, st)
@@ -1139,17 +1138,13 @@ int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, floa
     const int64_t rows = out.a_q_rows;  // (the last ones)
     const int nh = hq / hkv;
     const bool shared = tuned && (nh == 2 || nh == 4);
-    int rcs = prefill_stream_apply<T, OUT>(shared ? nullptr : k, hkv, l, a.Mt_k, a_k, out.a_k_stride, q + (l - rows) * d, rows,
-                                           l * d, a.Mt_q, a_q, hq, b, r, d, st);
+    int rcs = prefill_stream_apply<OUT>(shared ? nullptr : k, hkv, l, a.Mt_k, a_k, out.a_k_stride, q + (l - rows) * d, rows,
+                                        l * d, a.Mt_q, a_q, hq, b, r, d, st);
     if (!rcs && shared) rcs = apply_shared<OUT>(k, a.Mt_k, a_k, out.a_k_stride, bkv, nh, l, r, st);
     return rcs;
   };
-  if (out.storage && sizeof(T) == 2) return finish((T*)out.a_q, (T*)out.a_k);
+  if (out.storage) return finish((bf16_t*)out.a_q, (bf16_t*)out.a_k);
   return finish((float*)out.a_q, (float*)out.a_k);
 }
-template int prefill_gram_domain<float>(lrqk_ctx*, const float*, const float*, float*, float*, const PrefillOut&, int, int,
-                                        int, int64_t, int, int, int, float, hipStream_t);
-template int prefill_gram_domain<bf16_t>(lrqk_ctx*, const bf16_t*, const bf16_t*, float*, float*, const PrefillOut&, int, int,
-                                         int, int64_t, int, int, int, float, hipStream_t);
 
 }  // namespace lrqk

@@ -1,5 +1,5 @@
 // The passes over the long axis for the prefill iterations on Gram matrices, for every input that als_prefill_gram.hip
-// has no kernel tuned for: fp32 rows, rows of 64 elements, ranks 33 .. 64.
+// has no kernel tuned for: rows of 64 elements, ranks 33 .. 64.
 //
 //   sums   S = X^T X, and over given factors A the sums G = A^T A, C = A^T X
 //   apply  A = X M
@@ -27,7 +27,7 @@ __device__ __forceinline__ void st_wave_sync() {  // orders one wave's LDS write
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// a x b over piece pairs, smallest first (PA, PB = 1: a bf16 operand as it is), KB k blocks, into a fresh accumulator:
+// a x b over piece pairs, smallest first (PB = 1: a bf16 operand as it is), two k blocks, into a fresh accumulator:
 // the matrix cores do not round to nearest when they add to a large one, so a 32-row group's sum joins the running
 // total by ordinary fp32 additions.
 template <int PA, int PB>
@@ -47,9 +47,8 @@ __device__ __forceinline__ gd_floatx16 st_product(const gd_bf16x8 (&a)[2][PA], c
   return t;
 }
 
-template <typename T>
 constexpr int st_sums_smem(int db) {  // bytes of LDS: the waves' tiles, or their sums on the way out
-  const int tile = 32 * (32 * db + (sizeof(T) == 4 ? 8 : 16)) * (int)sizeof(T);
+  const int tile = 32 * (32 * db + 16) * (int)sizeof(bf16_t);
   return kStWaves * (tile > 4096 ? tile : 4096);
 }
 
@@ -59,24 +58,20 @@ constexpr int st_sums_smem(int db) {  // bytes of LDS: the waves' tiles, or thei
 // operands), else by workgroups of their own.
 // Split s of S of head h; 4 waves; a split takes every S-th set of 4 x 32 rows, so the workgroups of a head walk its
 // rows side by side.  part: [head][S][r][r + d]; xtx_part: [head][S][d][d] (both triangles).
-template <typename T, int AT, int DB, bool GIVEN, bool XTX>
-__device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* __restrict__ X, int xh, int hq, int64_t l,
-                                             int r, const float* __restrict__ A, float* __restrict__ part,
+template <int AT, int DB, bool GIVEN, bool XTX>
+__device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const bf16_t* __restrict__ X, int xh, int hq,
+                                             int64_t l, int r, const float* __restrict__ A, float* __restrict__ part,
                                              float* __restrict__ xtx_part, int S) {
   constexpr int D = 32 * DB;
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int P = F32 ? 3 : 1;
-  constexpr int VEC = Vec16<T>::N;
-  // row stride of the LDS tile in elements.  bf16: the transposing reads want successive rows 8 banks apart; fp32: a
-  // read takes one column of rows 4 apart in the wave's halves, which 8 floats of padding put 32 banks apart
-  constexpr int LDX = F32 ? D + 8 : D + 16;
+  constexpr int VEC = Vec16<bf16_t>::N;
+  constexpr int LDX = D + 16;  // elements per row of the LDS tile: the transposing reads want successive rows 8 banks apart
   constexpr int NL = 32 * D / (kWave * VEC);
-  constexpr int SMEM = st_sums_smem<T>(DB);
+  constexpr int SMEM = st_sums_smem(DB);
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int col = lane & 31, half = lane >> 5;
-  T* x_s = reinterpret_cast<T*>(smem + wave * (SMEM / kStWaves));
+  uint16_t* x_s = reinterpret_cast<uint16_t*>(smem + wave * (SMEM / kStWaves));
   const int64_t xhead = GIVEN ? (int64_t)(h / hq) * xh + (h % hq) / (hq / xh) : h;
-  const T* Xh = X + xhead * l * D;
+  const bf16_t* Xh = X + xhead * l * D;
   const float* Ah = A + (int64_t)h * l * r;
 
   constexpr int NAA = AT * (AT + 1) / 2, NXX = DB * (DB + 1) / 2;
@@ -104,7 +99,7 @@ __device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* 
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kWave + lane) * VEC;
-      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * (uint32_t)sizeof(T));
+      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * 2u);
     }
     if constexpr (GIVEN) {
 #pragma unroll
@@ -143,21 +138,14 @@ __device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* 
     st_wave_sync();
     if (t0 + stride < l) issue(t0 + stride);
     // rows 16 kb + 4 half .. + 3 and the same + 8 of column 32 nb + col
-    auto operand = [&](int nb, gd_bf16x8 (&x)[2][P]) {
+    auto operand = [&](int nb, gd_bf16x8 (&x)[2][1]) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
-        if constexpr (F32) {
-          float f[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) f[q] = ((const float*)x_s)[gd_mfma_row(lane, 8 * kb + q) * LDX + 32 * nb + col];
-          gd_split3x8(f, x[kb]);
-        } else {
-          const int s16 = lane & 15;
-          const uint16_t* p = (const uint16_t*)x_s + (16 * kb + 4 * half + (s16 >> 2)) * LDX + 32 * nb + (col & 16) + 4 * (s16 & 3);
-          const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
-          const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 8 * LDX));
-          x[kb][0] = __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        }
+        const int s16 = lane & 15;
+        const uint16_t* p = x_s + (16 * kb + 4 * half + (s16 >> 2)) * LDX + 32 * nb + (col & 16) + 4 * (s16 & 3);
+        const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
+        const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 8 * LDX));
+        x[kb][0] = __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
     };
     if constexpr (GIVEN) {
@@ -170,15 +158,15 @@ __device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* 
           for (int v = 0; v < 16; ++v) gAA[ta + tb][v] += t[v];
         }
     }
-    gd_bf16x8 xb[XTX ? DB : 1][2][P];
+    gd_bf16x8 xb[XTX ? DB : 1][2][1];
 #pragma unroll
     for (int nb = 0; nb < DB; ++nb) {
-      gd_bf16x8(&x)[2][P] = xb[XTX ? nb : 0];
+      gd_bf16x8(&x)[2][1] = xb[XTX ? nb : 0];
       operand(nb, x);
       if constexpr (GIVEN) {
 #pragma unroll
         for (int at = 0; at < AT; ++at) {
-          const gd_floatx16 t = st_product<3, P>(cp[at], x);
+          const gd_floatx16 t = st_product<3, 1>(cp[at], x);
 #pragma unroll
           for (int v = 0; v < 16; ++v) gAX[at][nb][v] += t[v];
         }
@@ -186,7 +174,7 @@ __device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* 
       if constexpr (XTX) {
 #pragma unroll
         for (int n2 = 0; n2 <= nb; ++n2) {
-          const gd_floatx16 t = st_product<P, P>(xb[n2], x);
+          const gd_floatx16 t = st_product<1, 1>(xb[n2], x);
 #pragma unroll
           for (int v = 0; v < 16; ++v) gXX[nb * (nb + 1) / 2 + n2][v] += t[v];
         }
@@ -241,41 +229,40 @@ __device__ __forceinline__ void st_sums_body(char* smem, int h, int s, const T* 
 }
 
 // The sums of both sides in one launch: one after the other they were up to four, 15 us each of a short prompt's host
-// time, and each with a last round of workgroups that left most of the GPU idle (4096 fp32 rows of 28 heads, rank 16:
-// 106 -> 73 us; three prompts of 2531 rows of 64: 44 -> 27; rank 64, 16K rows: 237 -> 193).  Workgroups in order: Q's sums
-// over the given factors [bh * S], K's [bh * S], Q^T Q [bh * S], K^T K [bkv * Sxk]; FUSED_Q / FUSED_K: the side's X^T X
-// comes with its sums.
+// time, and each with a last round of workgroups that left most of the GPU idle (three prompts of 2531 rows of 64:
+// 44 -> 27 us; rank 64, 16K rows: 237 -> 193).  Workgroups in order: Q's sums over the given factors [bh * S], K's
+// [bh * S], Q^T Q [bh * S], K^T K [bkv * Sxk]; FUSED_Q / FUSED_K: the side's X^T X comes with its sums.
 struct StSums {
-  const void *q, *k;
+  const bf16_t *q, *k;
   const float *a_q, *a_k;
   float *part_q, *part_k, *xq_part, *xk_part;
   int64_t l;
   int hq, hkv, r, S, Sxk, given;  // given: workgroups of one side's sums over the given factors
 };
-template <typename T, int AT, int DB, bool FUSED_Q, bool FUSED_K>
+template <int AT, int DB, bool FUSED_Q, bool FUSED_K>
 __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(StSums g) {
-  __shared__ __align__(16) char smem[st_sums_smem<T>(DB)];
-  const T *q = (const T*)g.q, *k = (const T*)g.k;
+  __shared__ __align__(16) char smem[st_sums_smem(DB)];
+  const bf16_t *q = g.q, *k = g.k;
   int w = blockIdx.x;
   if (w < g.given) {
-    st_sums_body<T, AT, DB, true, FUSED_Q>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, g.a_q, g.part_q, g.xq_part, g.S);
+    st_sums_body<AT, DB, true, FUSED_Q>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, g.a_q, g.part_q, g.xq_part, g.S);
     return;
   }
   w -= g.given;
   if (w < g.given) {
-    st_sums_body<T, AT, DB, true, FUSED_K>(smem, w / g.S, w % g.S, k, g.hkv, g.hq, g.l, g.r, g.a_k, g.part_k, g.xk_part, g.S);
+    st_sums_body<AT, DB, true, FUSED_K>(smem, w / g.S, w % g.S, k, g.hkv, g.hq, g.l, g.r, g.a_k, g.part_k, g.xk_part, g.S);
     return;
   }
   w -= g.given;
   if constexpr (!FUSED_Q) {
     if (w < g.given) {
-      st_sums_body<T, 1, DB, false, true>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, nullptr, nullptr, g.xq_part, g.S);
+      st_sums_body<1, DB, false, true>(smem, w / g.S, w % g.S, q, g.hq, g.hq, g.l, g.r, nullptr, nullptr, g.xq_part, g.S);
       return;
     }
     w -= g.given;
   }
   if constexpr (!FUSED_K)
-    st_sums_body<T, 1, DB, false, true>(smem, w / g.Sxk, w % g.Sxk, k, g.hkv, g.hq, g.l, g.r, nullptr, nullptr, g.xk_part,
+    st_sums_body<1, DB, false, true>(smem, w / g.Sxk, w % g.Sxk, k, g.hkv, g.hq, g.l, g.r, nullptr, nullptr, g.xk_part,
                                         g.Sxk);
 }
 
@@ -283,38 +270,36 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(StSums g) {
 // wave's private tile.  One launch for the sides given: workgroups (s, head) with s below side[0].S are the first side's
 // splits, the others the second's (a cache asks for one row of A_Q: alone that is a launch and 8 us).  The workgroups of
 // the query heads that share a kv head lie next to each other, so K comes from the caches after the first of them.
-template <typename T, typename OUT>
+template <typename OUT>
 struct StApply {
-  const T* x;
+  const bf16_t* x;
   int xh, S;          // heads of x per sequence; splits of the rows (0: no such side)
   int64_t l, x_stride;  // rows; elements between the heads of x
   const float* mt;
   OUT* a;             // heads a_stride elements apart, rows of r
   int64_t a_stride;
 };
-template <typename T, int AT, int DB, typename OUT>
-__global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_apply_kernel(StApply<T, OUT> first_side,
-                                                                                          StApply<T, OUT> second_side,
-                                                                                          int hq, int r) {
+constexpr int kStApplyWaves = 8;
+template <int AT, int DB, typename OUT>
+__global__ __launch_bounds__(kStApplyWaves * kWave) void pf_stream_apply_kernel(StApply<OUT> first_side,
+                                                                               StApply<OUT> second_side, int hq, int r) {
   constexpr int D = 32 * DB;
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int NW = F32 ? 4 : 8, NT = NW * kWave;
-  constexpr int P = F32 ? 3 : 1;
-  constexpr int VEC = Vec16<T>::N;
-  constexpr int LDM = D + 8, LDX = F32 ? D + 4 : D + 8;  // (16-byte operand reads want rows 4 banks apart)
+  constexpr int NW = kStApplyWaves, NT = NW * kWave;
+  constexpr int VEC = Vec16<bf16_t>::N;
+  constexpr int LDM = D + 8, LDX = D + 8;  // (16-byte operand reads want rows 4 banks apart)
   constexpr int NL = 32 * D / (kWave * VEC);
   extern __shared__ __align__(16) char ap_smem[];
   uint16_t* mt_s = reinterpret_cast<uint16_t*>(ap_smem);                                 // [3][32 AT][LDM]
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
-  T* x_s = reinterpret_cast<T*>(ap_smem + 3 * 32 * AT * LDM * 2) + wave * 32 * LDX;      // this wave's rows of X
+  uint16_t* x_s = mt_s + 3 * 32 * AT * LDM + wave * 32 * LDX;                            // this wave's rows of X
   const int col = lane & 31, half = lane >> 5;
   const int h = blockIdx.y;
   const bool second = (int)blockIdx.x >= first_side.S;
-  const StApply<T, OUT>& g = second ? second_side : first_side;
+  const StApply<OUT>& g = second ? second_side : first_side;
   const int s = second ? (int)blockIdx.x - first_side.S : (int)blockIdx.x, S = g.S;
   const int64_t l = g.l;
   const float* __restrict__ Mt = g.mt;
-  const T* __restrict__ Xh = g.x + ((int64_t)(h / hq) * g.xh + (h % hq) / (hq / g.xh)) * g.x_stride;
+  const bf16_t* __restrict__ Xh = g.x + ((int64_t)(h / hq) * g.xh + (h % hq) / (hq / g.xh)) * g.x_stride;
   OUT* __restrict__ Ah = g.a + (int64_t)h * g.a_stride;
   for (int e = tid; e < 32 * AT * D; e += NT) {
     const int n = e / D, k = e % D;
@@ -331,7 +316,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
       const int e = (i * kWave + lane) * VEC;
-      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * (uint32_t)sizeof(T));
+      pre[i] = gd_at<gd_u32x4>(Xh + t0 * D, (uint32_t)(min(e / D, last) * D + e % D) * 2u);
     }
   };
   const int64_t stride = (int64_t)S * NW * 32;
@@ -353,15 +338,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
       for (int v = 0; v < 16; ++v) c[at][v] = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < D / 16; ++kb) {
-      gd_bf16x8 xa[P];
-      if constexpr (F32) {
-        const float4 lo = *reinterpret_cast<const float4*>(&x_s[col * LDX + 16 * kb + 8 * half]);
-        const float4 hi = *reinterpret_cast<const float4*>(&x_s[col * LDX + 16 * kb + 8 * half + 4]);
-        const float f[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        gd_split3x8(f, xa);
-      } else {
-        xa[0] = *reinterpret_cast<const gd_bf16x8*>(&x_s[col * LDX + 16 * kb + 8 * half]);
-      }
+      const gd_bf16x8 xa = *reinterpret_cast<const gd_bf16x8*>(&x_s[col * LDX + 16 * kb + 8 * half]);
 #pragma unroll
       for (int at = 0; at < AT; ++at) {
         gd_bf16x8 m[3];
@@ -369,12 +346,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 4 : 8) * kWave) void pf_stream_ap
         for (int p = 0; p < 3; ++p)
           m[p] = *reinterpret_cast<const gd_bf16x8*>(&mt_s[(p * 32 * AT + 32 * at + col) * LDM + 16 * kb + 8 * half]);
 #pragma unroll
-        for (int w = P + 1; w >= 0; --w)
-#pragma unroll
-          for (int i = P - 1; i >= 0; --i) {
-            if (w - i < 0 || w - i >= 3 || (P == 3 && w == 4)) continue;
-            c[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[i], m[w - i], c[at], 0, 0, 0);
-          }
+        for (int p = 2; p >= 0; --p) c[at] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, m[p], c[at], 0, 0, 0);
       }
     }
 #pragma unroll
@@ -405,14 +377,14 @@ int prefill_store(const float* src, int64_t src_stride, OUT* dst, int64_t dst_st
 template int prefill_store<float>(const float*, int64_t, float*, int64_t, int64_t, int, hipStream_t);
 template int prefill_store<bf16_t>(const float*, int64_t, bf16_t*, int64_t, int64_t, int, hipStream_t);
 
-template <typename T, int AT, int DB>
+template <int AT, int DB>
 static int sums_impl(const StSums& g, int b, hipStream_t st) {
   const int bkv = b * g.hkv;
   if (DB == 2 && g.hkv == g.hq && g.S == g.Sxk)
-    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, DB == 2, DB == 2>), dim3((unsigned)(2 * g.given)), dim3(kStThreads),
-                       0, st, g);
+    hipLaunchKernelGGL((pf_stream_sums_kernel<AT, DB, DB == 2, DB == 2>), dim3((unsigned)(2 * g.given)), dim3(kStThreads), 0,
+                       st, g);
   else
-    hipLaunchKernelGGL((pf_stream_sums_kernel<T, AT, DB, DB == 2, false>),
+    hipLaunchKernelGGL((pf_stream_sums_kernel<AT, DB, DB == 2, false>),
                        dim3((unsigned)((DB == 2 ? 2 : 3) * g.given + bkv * g.Sxk)), dim3(kStThreads), 0, st, g);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
@@ -420,25 +392,20 @@ static int sums_impl(const StSums& g, int b, hipStream_t st) {
 
 // Sums of both sides: over the given factors ([b * hq] heads, S splits), Q^T Q ([b * hq] heads, S splits) and K^T K
 // ([b * hkv] heads, Sxk splits).
-template <typename T>
-int prefill_stream_sums(const T* q, const T* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
+int prefill_stream_sums(const bf16_t* q, const bf16_t* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
                         const float* a_k, float* part_q, float* part_k, int S, float* xq_part, float* xk_part, int Sxk,
                         hipStream_t st) {
   const StSums g{q, k, a_q, a_k, part_q, part_k, xq_part, xk_part, l, hq, hkv, r, S, Sxk, b * hq * S};
-  if (d == 64) return r <= 32 ? sums_impl<T, 1, 2>(g, b, st) : sums_impl<T, 2, 2>(g, b, st);
-  return r <= 32 ? sums_impl<T, 1, 4>(g, b, st) : sums_impl<T, 2, 4>(g, b, st);
+  if (d == 64) return r <= 32 ? sums_impl<1, 2>(g, b, st) : sums_impl<2, 2>(g, b, st);
+  return r <= 32 ? sums_impl<1, 4>(g, b, st) : sums_impl<2, 4>(g, b, st);
 }
-template int prefill_stream_sums<float>(const float*, const float*, int, int, int, int64_t, int, int, const float*,
-                                        const float*, float*, float*, int, float*, float*, int, hipStream_t);
-template int prefill_stream_sums<bf16_t>(const bf16_t*, const bf16_t*, int, int, int, int64_t, int, int, const float*,
-                                         const float*, float*, float*, int, float*, float*, int, hipStream_t);
 
-template <typename T, int AT, int DB, typename OUT>
-static int apply_impl(StApply<T, OUT> g0, StApply<T, OUT> g1, int hq, int b, int r, hipStream_t st) {
-  constexpr int D = 32 * DB, NW = sizeof(T) == 4 ? 4 : 8;
-  constexpr size_t smem = (size_t)3 * 32 * AT * (D + 8) * 2 + (size_t)NW * 32 * (sizeof(T) == 4 ? D + 4 : D + 8) * sizeof(T);
+template <int AT, int DB, typename OUT>
+static int apply_impl(StApply<OUT> g0, StApply<OUT> g1, int hq, int b, int r, hipStream_t st) {
+  constexpr int D = 32 * DB, NW = kStApplyWaves;
+  constexpr size_t smem = (size_t)(3 * 32 * AT + NW * 32) * (D + 8) * sizeof(bf16_t);
   static_assert(smem <= 160 * 1024, "LDS");
-  auto kern = pf_stream_apply_kernel<T, AT, DB, OUT>;
+  auto kern = pf_stream_apply_kernel<AT, DB, OUT>;
   static std::atomic<bool> attr_dev[kMaxDeviceSlots];
   std::atomic<bool>& attr = attr_dev[per_device_slot()];
   if (!attr) {
@@ -448,7 +415,7 @@ static int apply_impl(StApply<T, OUT> g0, StApply<T, OUT> g1, int hq, int b, int
   // every workgroup stages M (52 KB in, up to 104 KB of fp32 read): enough of them to fill the GPU once, no more
   const int bh = b * hq;
   const int per_cu = std::max(1, (int)(160 * 1024 / smem));
-  for (StApply<T, OUT>* g : {&g0, &g1})
+  for (StApply<OUT>* g : {&g0, &g1})
     g->S = !g->x ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (g->l + 32 * NW - 1) / (32 * NW)));
   hipLaunchKernelGGL(kern, dim3((unsigned)(g0.S + g1.S), (unsigned)bh), dim3(NW * kWave), smem, st, g0, g1, hq, r);
   LRQK_HIP_CHECK(hipGetLastError());
@@ -457,20 +424,18 @@ static int apply_impl(StApply<T, OUT> g0, StApply<T, OUT> g1, int hq, int b, int
 
 // A_K = K Mk (l rows) and A_Q = Q Mq (q_rows rows) for all b * hq query heads; without k only the latter.  q: the first of
 // those rows, heads q_stride elements apart.
-template <typename T, typename OUT>
-int prefill_stream_apply(const T* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride, const T* q,
-                         int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r, int d,
-                         hipStream_t st) {
-  const StApply<T, OUT> gk{k, hkv, 0, l, l * d, mt_k, a_k, a_k_stride};
-  const StApply<T, OUT> gq{q, hq, 0, q_rows, q_stride, mt_q, a_q, q_rows * r};
-  if (d == 64) return r <= 32 ? apply_impl<T, 1, 2>(gk, gq, hq, b, r, st) : apply_impl<T, 2, 2>(gk, gq, hq, b, r, st);
-  return r <= 32 ? apply_impl<T, 1, 4>(gk, gq, hq, b, r, st) : apply_impl<T, 2, 4>(gk, gq, hq, b, r, st);
+template <typename OUT>
+int prefill_stream_apply(const bf16_t* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride,
+                         const bf16_t* q, int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r,
+                         int d, hipStream_t st) {
+  const StApply<OUT> gk{k, hkv, 0, l, l * d, mt_k, a_k, a_k_stride};
+  const StApply<OUT> gq{q, hq, 0, q_rows, q_stride, mt_q, a_q, q_rows * r};
+  if (d == 64) return r <= 32 ? apply_impl<1, 2>(gk, gq, hq, b, r, st) : apply_impl<2, 2>(gk, gq, hq, b, r, st);
+  return r <= 32 ? apply_impl<1, 4>(gk, gq, hq, b, r, st) : apply_impl<2, 4>(gk, gq, hq, b, r, st);
 }
-template int prefill_stream_apply<float, float>(const float*, int, int64_t, const float*, float*, int64_t, const float*,
-                                                int64_t, int64_t, const float*, float*, int, int, int, int, hipStream_t);
-template int prefill_stream_apply<bf16_t, float>(const bf16_t*, int, int64_t, const float*, float*, int64_t, const bf16_t*,
-                                                 int64_t, int64_t, const float*, float*, int, int, int, int, hipStream_t);
-template int prefill_stream_apply<bf16_t, bf16_t>(const bf16_t*, int, int64_t, const float*, bf16_t*, int64_t, const bf16_t*,
-                                                  int64_t, int64_t, const float*, bf16_t*, int, int, int, int, hipStream_t);
+template int prefill_stream_apply<float>(const bf16_t*, int, int64_t, const float*, float*, int64_t, const bf16_t*, int64_t,
+                                         int64_t, const float*, float*, int, int, int, int, hipStream_t);
+template int prefill_stream_apply<bf16_t>(const bf16_t*, int, int64_t, const float*, bf16_t*, int64_t, const bf16_t*, int64_t,
+                                          int64_t, const float*, bf16_t*, int, int, int, int, hipStream_t);
 
 }  // namespace lrqk

@@ -196,19 +196,17 @@ struct PrefillOut {
   int64_t a_q_rows, a_k_stride;
   bool storage;
 };
-// Prefill iterations on Gram matrices; see als_prefill_gram.hip.
-template <typename T>
-int prefill_gram_domain(lrqk_ctx* ctx, const T* q, const T* k, float* a_q0, float* a_k0, const PrefillOut& out, int b, int hq,
-                        int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st);
-// Its passes over the long axis; see als_prefill_stream.hip (every shape) and als_prefill.hip (bf16 rows of 128, r <= 32).
-template <typename T>
-int prefill_stream_sums(const T* q, const T* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
+// Prefill iterations on Gram matrices (bf16 rows); see als_prefill_gram.hip.
+int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* a_q0, float* a_k0, const PrefillOut& out,
+                        int b, int hq, int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st);
+// Its passes over the long axis; see als_prefill_stream.hip (every shape) and als_prefill.hip (rows of 128, r <= 32).
+int prefill_stream_sums(const bf16_t* q, const bf16_t* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
                         const float* a_k, float* part_q, float* part_k, int S, float* xq_part, float* xk_part, int Sxk,
                         hipStream_t st);
-template <typename T, typename OUT>
-int prefill_stream_apply(const T* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride, const T* q,
-                         int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r, int d,
-                         hipStream_t st);
+template <typename OUT>
+int prefill_stream_apply(const bf16_t* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride,
+                         const bf16_t* q, int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r,
+                         int d, hipStream_t st);
 int prefill_given_sums_bf16(const bf16_t* x, int xh, int hq, int b, int64_t l, int r, float* a, float* part, int S,
                             hipStream_t st);
 template <typename OUT>

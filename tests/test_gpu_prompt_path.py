@@ -152,6 +152,22 @@ def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
     assert (buf[:, :, :3] == 9).all() and (buf[:, :, 3 + l:] == 9).all()
 
 
+@pytest.mark.parametrize("d,r,l", [(64, 16, 700), (64, 48, 129), (128, 32, 5000), (128, 64, 2531)])
+def test_fp32_rows_are_factorised_row_by_row(ops, monkeypatch, d, r, l):
+    """fp32 prompts take the row-by-row formulation, to the bit, at every width and rank that bf16 rows take to Gram
+    matrices: an fp32 generation goes on from these factors, and those of the other formulation are 1e-5 away."""
+    gen = torch.Generator(device=DEV).manual_seed(d + l)
+    Q = torch.randn((1, 4, l, d), generator=gen, device=DEV)
+    K = torch.randn((1, 2, l, d), generator=gen, device=DEV)
+    A0, A1 = (torch.randn((1, 4, l, r), generator=gen, device=DEV) for _ in range(2))
+    ws = ops.Workspace()
+    got = ops.als_prefill(ws, Q, K, A0.clone(), A1.clone(), 2, 0.0)
+    monkeypatch.setenv("LRQK_PREFILL_ROWWISE", "1")
+    want = ops.als_prefill(ws, Q, K, A0.clone(), A1.clone(), 2, 0.0)
+    for name, g, w in zip(("A_Q", "B_Q", "A_K", "B_K"), got, want):
+        assert torch.equal(g, w), name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("r,m", [(16, 1025), (16, 4127), (32, 1056), (32, 9001), (64, 1060), (64, 5000)])
 def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
