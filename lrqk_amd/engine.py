@@ -246,6 +246,8 @@ class LightAttentionIndicesFactory:
         self.current_len = seq_len
         # a new sequence: whatever the victim cache holds belongs to the previous one
         self.ws.victim_cache(self.victim_rows_effective)
+        if self.KVcpu.pin_memory and key_states.is_cuda:
+            self.KVcpu.gpu = key_states.device   # before anything allocates the store: a short prompt's steps use it too
         stored = self._store_prompt(key_states, value_states) if seq_len > self.gpu_capacity else None
         try:
             self._factorise_prompt(query_states, key_states, value_states, custom)
@@ -350,7 +352,6 @@ class LightAttentionIndicesFactory:
         if not (self.KVcpu.pin_memory and key_states.is_cuda):
             self.KVcpu.append(key_states, value_states)
             return None
-        self.KVcpu.gpu = key_states.device
         row0 = self.KVcpu.extend((b, hkv, 0, 2 * d), length)
         if 2 * key_states.numel() * key_states.element_size() < self._DMA_STORE_BYTES:
             ops.flush_ring(key_states, value_states, 0, length, self.KVcpu.data, row0, hkv)

@@ -91,6 +91,42 @@ def test_a_dropped_caches_store_waits_for_its_copies(ops, context, name):
     assert early and not same
 
 
+@pytest.mark.parametrize("capacity,tokens", [(9000, 0), (200, 80)])
+def test_a_short_prompts_store_waits_for_its_flushes(ops, capacity, tokens):
+    """The same for a prompt that fits the active set, whose store only the decode steps' kernels write (a flush of the
+    ring per 16 tokens): as it was allocated, and after it has grown (from 200 rows, within 80 tokens)."""
+    from lrqk_amd import DynamicLRQKCache
+    gen = torch.Generator(device=DEV).manual_seed(capacity)
+
+    def rows(heads, n):
+        return torch.randn((1, heads, n, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    prompt = rows(4, 140), rows(2, 140), rows(2, 140)
+    token = rows(4, 1), rows(2, 1), rows(2, 1)
+    for attempt in range(2):   # (the first loads kernels, which waits for the device)
+        cache = DynamicLRQKCache(r=16, num_active_tokens=128, max_iter=1, lite_tokens=16, tol=0.0,
+                                 max_sequence_length=capacity, num_key_value_groups=2)
+        cache.update(*prompt, 0)
+        first = cache.lwattn[0].KVcpu.data.data_ptr()
+        for _ in range(tokens):
+            cache.update(*token, 0)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(400_000_000)   # some tenths of a second
+        for _ in range(20):
+            cache.update(*token, 0)
+        store = cache.lwattn[0].KVcpu.data
+        place, shape = store.data_ptr(), store.shape
+        assert (place != first) == (tokens > 0)
+        busy = torch.cuda.Event()
+        busy.record()
+        del cache, store
+        other = torch.empty(shape, dtype=torch.bfloat16, pin_memory=True)
+        early = not busy.query()
+        same = other.data_ptr() == place
+        torch.cuda.synchronize()
+        del other
+    assert early and not same
+
+
 def test_a_host_ahead_of_the_gpu_holds_few_stores(ops, monkeypatch):
     """A cache per prompt, each dropped before the GPU has come to it: the host waits instead of taking a pinned block for
     every prompt that it is ahead (the newest and one before it here, and one on its way back)."""
