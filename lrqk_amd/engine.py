@@ -248,16 +248,30 @@ class LightAttentionIndicesFactory:
         self.ws.victim_cache(self.victim_rows_effective)
         if self.KVcpu.pin_memory and key_states.is_cuda:
             self.KVcpu.gpu = key_states.device   # before anything allocates the store: a short prompt's steps use it too
-        stored = self._store_prompt(key_states, value_states) if seq_len > self.gpu_capacity else None
+        # The store and the rows of A_K are extended ahead of work that may fail (memory, sizes that the library
+        # refuses): a prompt that raises leaves both, and the given initial factors, as they were, and another one
+        # can be tried.
+        before = [(buf, dict(vars(buf))) for buf in (self.KVcpu, self._A_K)]
+        init_factors = self.init_factors
         try:
-            self._factorise_prompt(query_states, key_states, value_states, custom)
-        finally:
-            if stored is not None:
-                # What is queued from here on finds the prompt in the store (and the staging block may be reused).
-                # The event is recorded only now: its packet holds up the hardware queue of the side stream until
-                # the copy is done, and with four hardware queues one side stream in four shares this stream's
-                # (recorded right after the copy it made 128K prompts take 15 instead of 10 ms one time in four).
-                torch.cuda.current_stream(dev).wait_stream(stored[0])
+            stored = self._store_prompt(key_states, value_states) if seq_len > self.gpu_capacity else None
+            try:
+                self._factorise_prompt(query_states, key_states, value_states, custom)
+            finally:
+                if stored is not None:
+                    # What is queued from here on finds the prompt in the store (and the staging block may be reused).
+                    # The event is recorded only now: its packet holds up the hardware queue of the side stream until
+                    # the copy is done, and with four hardware queues one side stream in four shares this stream's
+                    # (recorded right after the copy it made 128K prompts take 15 instead of 10 ms one time in four).
+                    torch.cuda.current_stream(dev).wait_stream(stored[0])
+        except BaseException:
+            for buf, state in before:
+                vars(buf).clear()
+                vars(buf).update(state)
+            if self._A_K.data is not None:   # rows beyond the last one are zero
+                self._A_K.data.narrow(2, len(self._A_K), self._A_K.capacity - len(self._A_K)).zero_()
+            self.init_factors = init_factors
+            raise
 
     def _factorise_prompt(self, query_states, key_states, value_states, custom):
         seq_len = query_states.shape[2]

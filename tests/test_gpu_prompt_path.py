@@ -268,3 +268,41 @@ def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
     torch.cuda.current_stream().synchronize()
     for eng, want in engines:
         assert torch.equal(eng.KVcpu.tensor(), want.cpu())
+
+
+@pytest.mark.parametrize("fails_at,first,second", [("als_prefill_store", 300, 260), ("als_prefill_store", 66, 300),
+                                                   ("score_select", 300, 90)])
+def test_a_prompt_that_failed_leaves_nothing_behind(ops, monkeypatch, fails_at, first, second):
+    """An engine whose prefill raised takes the next prompt as a new one does: the same store, factors and steps past a
+    flush of the ring."""
+    from lrqk_amd.engine import LightAttentionIndicesFactory as Engine
+    gen = torch.Generator(device=DEV).manual_seed(first)
+
+    def rows(heads, n):
+        return torch.randn((1, heads, n, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    lost = rows(4, first), rows(2, first), rows(2, first)
+    prompt = rows(4, second), rows(2, second), rows(2, second)
+    tokens = [(rows(4, 1), rows(2, 1), rows(2, 1)) for _ in range(20)]
+    start = tuple(torch.randn((1, 4, second, 16), generator=gen, device=DEV) for _ in range(2))
+    tried, fresh = (Engine(num_lite_tokens=8, attn_topk=64, num_key_value_groups=2, r=16, max_iter=2, tol=0.0, capacity=1200)
+                    for _ in range(2))
+    tried.init_factors = kept = tuple(torch.randn((1, 4, first, 16), generator=gen, device=DEV) for _ in range(2))
+
+    def out_of_memory(*a, **kw):
+        raise torch.cuda.OutOfMemoryError("planted")
+    with monkeypatch.context() as m:
+        m.setattr(ops, fails_at, out_of_memory)
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            tried.prefill(*lost)
+    left = tried.init_factors
+    for eng in (tried, fresh):
+        eng.init_factors = start
+        eng.prefill(*prompt)
+        for t in tokens:
+            eng.decode(*t)
+    torch.cuda.synchronize()
+    assert torch.equal(tried.KVcpu.tensor(), fresh.KVcpu.tensor())
+    assert torch.equal(tried._A_K.data, fresh._A_K.data)
+    assert torch.equal(tried.hit_indices, fresh.hit_indices) and torch.equal(tried.last_q_hat, fresh.last_q_hat)
+    assert torch.equal(tried.Kgpu, fresh.Kgpu) and torch.equal(tried.Vgpu, fresh.Vgpu)
+    assert left is kept
