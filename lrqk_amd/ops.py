@@ -40,15 +40,15 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 def _torch_alloc(nbytes, stream, user):
     try:
         return torch.cuda.caching_allocator_alloc(nbytes, stream=stream or 0)
-    except Exception:  # nothing may pass through the C frames; the library reports the size it did not get
-        return None
+    except BaseException:  # nothing may pass through the C frames, an interrupt included: a callback that is left by an
+        return None        # exception hands C an address that nobody wrote.  The library reports the size it did not get.
 
 
 @_lib.RELEASE_FN
 def _torch_release(block, user):
     try:
         torch.cuda.caching_allocator_delete(block)
-    except Exception:  # the interpreter is shutting down
+    except BaseException:  # the interpreter is shutting down
         pass
 
 

@@ -102,3 +102,21 @@ def test_bench_refuses_more_than_one_gpu():
                        timeout=120)
     assert p.returncode != 0
     assert "one GPU" in p.stderr
+
+
+@pytest.mark.parametrize("raised", [KeyboardInterrupt, SystemExit, MemoryError, RuntimeError])
+def test_an_allocator_that_raises_hands_out_nothing(monkeypatch, raised):
+    """The callbacks that a workspace takes its memory from, called as C calls them: whatever ends them, an interrupt
+    included, C sees a null pointer and never what happens to lie in the place of the result."""
+    import sys
+
+    def interrupted(*a, **kw):
+        raise raised()
+    left = []
+    monkeypatch.setattr(torch.cuda, "caching_allocator_alloc", interrupted)
+    monkeypatch.setattr(torch.cuda, "caching_allocator_delete", interrupted)
+    monkeypatch.setattr(sys, "unraisablehook", left.append)
+    assert ops._torch_alloc(64, 0, None) is None
+    ops._torch_release(4096, None)
+    monkeypatch.undo()
+    assert not left
