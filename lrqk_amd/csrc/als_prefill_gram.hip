@@ -1059,15 +1059,17 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   const bool tuned = d == 128 && r <= 32;
   const int RP = r <= 16 ? 16 : r <= 32 ? 32 : 64;
   const size_t ne = (size_t)r * (r + d), dd = (size_t)d * d;
-  // Splits of the long axis: one workgroup per CU and launch (the kernels' registers), at most 4096 rows per split
-  // (its fp32 sums; the splits are added in fp64), at least one step of rows each.
+  // Splits of the long axis: one workgroup per CU and launch (the kernels' registers; no more than 64 of a head for that),
+  // at most 4096 rows per split however long the prompt (its fp32 sums; the splits are added in fp64; B of 8M equal
+  // rows is 1.7e-5 off with 64 splits, 2.2e-7 with 2048), at least one step of rows each.
   auto splits = [&](int heads) {
-    int64_t v = std::max<int64_t>(std::max(1, 256 / heads), (l + 4095) / 4096);
-    return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(v, 64), (l + 127) / 128));
+    const int64_t v = std::max<int64_t>(std::max(1, std::min(64, 256 / heads)), (l + 4095) / 4096);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(v, (l + 127) / 128));
   };
   const int S = splits(bh), Sx = S;
   // (K^T K: with 64 splits of 8 heads the partial sums are 33 MB to write and to add up: 25.6 + 18.5 us against
-  // 19.7 + 11.1 with 32)
+  // 19.7 + 11.1 with 32.  No bound on the rows of a split here: its sums are of exact products, and 32 kv heads of 64K
+  // rows add 8192 of them up in fp32)
   const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
                         : hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;

@@ -188,6 +188,24 @@ def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
     assert (buf[:, :, :3] == 9).all() and (buf[:, :, 3 + l:] == 9).all()
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_sums_over_millions_of_rows(ops, d):
+    """However long the prompt, a split adds 4096 rows up in fp32: the given factors of 8M equal rows, whose sums never
+    cancel, and the B that follows from them.  Limit: a wave adds 32 groups of 32 rows (d 64: as many; the K side at
+    d 128: 16) to its total, each addition off by at most 2^-25 of the total so far, 16 x 2^-24 of it in the end; 8 waves'
+    totals, the group's own 32 x 3 products and the last rounding are below 8 x 2^-24; both for A^T A and A^T X."""
+    l = 1 << 23
+    X = torch.ones((1, 1, l, d), device=DEV, dtype=torch.bfloat16)
+    ws = ops.Workspace()
+    for a in (1.3, 1.4142135, 1.61803398, 1.9):
+        A0 = torch.full((1, 1, l, 1), a, device=DEV)
+        got = ops.als_prefill(ws, X, X, A0.clone(), A0.clone(), 0, 0.0)
+        for name, g in (("B_Q", got[1]), ("B_K", got[3])):
+            off = float((g.double() * float(A0[0, 0, 0, 0]) - 1).abs().max()) * 2 ** 24
+            print(f"{name} {a}: {off:.1f} x 2^-24", flush=True)
+            assert off < 2 * (16 + 8), name
+
+
 @pytest.mark.parametrize("d,r,l", [(64, 16, 700), (64, 48, 129), (128, 32, 5000), (128, 64, 2531)])
 def test_fp32_rows_are_factorised_row_by_row(ops, monkeypatch, d, r, l):
     """fp32 prompts take the row-by-row formulation, to the bit, at every width and rank that bf16 rows take to Gram
