@@ -11,6 +11,7 @@ from __future__ import annotations
 import collections
 import math
 import threading
+import weakref
 from typing import Optional
 
 import torch
@@ -120,15 +121,29 @@ def _host_stores_ahead(device: torch.device, nbytes: int):
     """Called before a store of ``nbytes`` is allocated.  A dropped cache's store is free once the GPU has done its work,
     and the host queues a long prompt in a twentieth of the time that this takes (0.5 of 9.7 ms at 128K): a program that
     makes a cache per prompt would hold a store for every prompt that it is ahead.  So the calling thread waits here as
-    long as the stores it has allocated since work that the GPU has not finished exceed 1 GiB, but never for the last."""
-    pending = _ahead.__dict__.setdefault(device.index, collections.deque())
+    long as the stores that it allocated, that came back since and that the GPU still works on exceed 1 GiB with the new
+    one, but never for the last.  Stores in use count for nothing: waiting would not free them.  Returns the list that
+    the new store's release is to be noted in (``_store_came_back``)."""
+    pending = _ahead.__dict__.setdefault(device.index, collections.deque())   # (mark, bytes), oldest first
     while pending and pending[0][0].query():
         pending.popleft()
-    while len(pending) > 1 and sum(n for _, n in pending) + nbytes > _AHEAD_BYTES:
+    # (by index: a store that another thread or the collector drops meanwhile appends to the list)
+    while len(pending) > 1 and sum(pending[i][1] for i in range(len(pending))) + nbytes > _AHEAD_BYTES:
         pending.popleft()[0].synchronize()
-    mark = torch.cuda.Event()
-    mark.record(torch.cuda.current_stream(device))
-    pending.append((mark, nbytes))
+    return pending
+
+
+def _store_came_back(pending, stream: torch.cuda.Stream, nbytes: int):
+    """A store is released: what its stream has been given until now is what the GPU may still do with it."""
+    try:
+        with torch.cuda.stream(stream):
+            if torch.cuda.is_current_stream_capturing():   # (the mark would become part of the graph)
+                return
+            mark = torch.cuda.Event()
+            mark.record()
+        pending.append((mark, nbytes))
+    except Exception:  # the interpreter or the device is going
+        pass
 
 
 class AutoIncreaseTensorSharedKV(AutoIncreaseTensor):
@@ -141,10 +156,10 @@ class AutoIncreaseTensorSharedKV(AutoIncreaseTensor):
         # through tensor()), so the store is not cleared: clearing 0.8 GB of pinned memory is 4 ms of a
         # 128K layer prefill.  (The factor buffer keeps the zero fill: it is gathered at full capacity.)
         pin = bool(self.pin_memory) and torch.cuda.is_available()
-        if pin and self.gpu is not None:
-            _host_stores_ahead(self.gpu, math.prod(shape) * self.dtype.itemsize)
+        ahead = _host_stores_ahead(self.gpu, math.prod(shape) * self.dtype.itemsize) if pin and self.gpu is not None else None
         store = torch.empty(shape, device=self.device, dtype=self.dtype, pin_memory=pin)
-        if pin and self.gpu is not None and store.numel():
+        if ahead is not None and store.numel():
+            weakref.finalize(store, _store_came_back, ahead, torch.cuda.current_stream(self.gpu), store.nbytes).atexit = False
             # torch hands a freed pinned block out again once the work that it knows to use it is done.  The kernels
             # and copies of the library are not in its books: one element copied by torch puts the current stream
             # there, and whoever gets the block next finds everything queued on that stream until the release done.

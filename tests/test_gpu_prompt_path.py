@@ -148,6 +148,30 @@ def test_a_host_ahead_of_the_gpu_holds_few_stores(ops, monkeypatch):
     assert len(places) <= 4
 
 
+def test_stores_of_live_caches_are_not_waited_for(ops, monkeypatch):
+    """The host waits for stores that come back, not for those of caches in use: the layers of a model."""
+    from lrqk_amd import DynamicLRQKCache, buffers
+    monkeypatch.setattr(buffers, "_AHEAD_BYTES", 1)
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn((1, 4, 3000, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    k, v = (torch.randn((1, 2, 3000, 64), generator=gen, device=DEV).to(torch.bfloat16) for _ in range(2))
+
+    def model():
+        return DynamicLRQKCache(r=16, num_active_tokens=128, max_iter=1, lite_tokens=16, tol=0.0, max_sequence_length=3264,
+                                num_key_value_groups=2)
+    for attempt in range(2):   # (the first loads kernels and takes pinned memory, which waits for the device)
+        cache = model()
+        torch.cuda.synchronize()
+        torch.cuda._sleep(400_000_000)
+        slept = torch.cuda.Event()
+        slept.record()
+        for layer in range(5):
+            cache.update(q, k, v, layer)
+        waited = slept.query()
+        torch.cuda.synchronize()
+    assert not waited
+
+
 @pytest.mark.parametrize("dtype,d,r,l,hq,hkv,iters", [
     (torch.float32, 64, 1, 128, 2, 2, 1),        # the fewest rows the Gram matrices take, one column of factors
     (torch.float32, 64, 16, 129, 6, 2, 2),       # a row beyond whole groups; three query heads per kv head
