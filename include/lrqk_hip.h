@@ -42,7 +42,8 @@ int lrqk_version(void);
 const char* lrqk_last_error(void);
 
 /* Workspace (radix keys, histograms, split partials), sized on demand; growing it
- * synchronises the device once.  One ctx per engine; calls on one ctx must not overlap. */
+ * synchronises the device once (not with an allocator of the caller's).  One ctx per engine; calls on one ctx must not
+ * overlap. */
 int lrqk_ctx_create(lrqk_ctx** out);
 int lrqk_ctx_destroy(lrqk_ctx* ctx);
 /* Where the ctx takes its device memory from (default: hipMalloc / hipFree, which wait for the device).  alloc returns
@@ -52,8 +53,11 @@ int lrqk_ctx_destroy(lrqk_ctx* ctx);
  * No counterpart in the reference. */
 int lrqk_ctx_set_allocator(lrqk_ctx* ctx, void* (*alloc)(size_t bytes, void* stream, void* user),
                            void (*release)(void* block, void* user), void* user);
-/* Optional: pre-size the workspace so that later calls never allocate. */
+/* Optional: pre-size the workspace so that later calls never allocate.  The memory is taken for the stream of the last
+ * call (none yet: the null stream); lrqk_ctx_reserve_on names the stream that the calls to come are made on, so that a
+ * ctx with an allocator of the caller's can go without waiting for the device. */
 int lrqk_ctx_reserve(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d);
+int lrqk_ctx_reserve_on(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d, void* stream);
 
 /* py:1260-1263 -- proxy scores A_K[:m] . q_hat^T as fp32 [bh][m].
  * a_k: [bh] heads of head_stride elements each, rows of r elements; q_hat: [bh][r].

@@ -49,6 +49,7 @@ def _sig(lib):
         "lrqk_ctx_destroy": ([vp], i32),
         "lrqk_ctx_set_allocator": ([vp, ALLOC_FN, RELEASE_FN, vp], i32),
         "lrqk_ctx_reserve": ([vp, i32, i64, i32, i32, i32, i32], i32),
+        "lrqk_ctx_reserve_on": ([vp, i32, i64, i32, i32, i32, i32, vp], i32),
         "lrqk_proxy_scores": ([vp, i64, vp, i32, i64, i32, i32, i32, vp, vp], i32),
         "lrqk_score_select": ([vp, vp, i64, vp, i32, i64, i32, i32, i32, i32, vp, i64, vp], i32),
         "lrqk_score_select_diff": ([vp, vp, i64, vp, i32, i64, i32, i32, i32, i32, vp, vp, i64, vp, vp, vp, vp], i32),

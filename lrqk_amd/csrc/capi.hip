@@ -69,9 +69,14 @@ extern "C" int lrqk_ctx_destroy(lrqk_ctx* ctx) {
 }
 
 extern "C" int lrqk_ctx_reserve(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d) {
+  return lrqk_ctx_reserve_on(ctx, bh, max_tokens, topk, n_active, r, d, ctx ? (void*)ctx->pool.stream : nullptr);
+}
+
+extern "C" int lrqk_ctx_reserve_on(lrqk_ctx* ctx, int bh, int64_t max_tokens, int topk, int n_active, int r, int d,
+                                   void* stream) {
   LRQK_REQUIRE(ctx != nullptr, LRQK_EINVAL, "ctx is null");
   LRQK_REQUIRE(bh > 0 && max_tokens >= 0 && topk > 0 && n_active > 0 && r > 0 && d > 0, LRQK_EINVAL, "bad sizes");
-  ctx->pool.enter(ctx->pool.stream);
+  ctx->pool.enter((hipStream_t)stream);
   int rc;
   const int64_t key_stride = (max_tokens + 63) & ~(int64_t)63;
   if ((rc = ctx->keys.ensure((size_t)bh * key_stride * 4))) return rc;

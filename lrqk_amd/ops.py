@@ -67,7 +67,9 @@ class Workspace:
         return self._h
 
     def reserve(self, bh, max_tokens, topk, n_active, r, d):
-        check(_lib.load().lrqk_ctx_reserve(self._h, bh, max_tokens, topk, n_active, r, d))
+        """Memory for the calls to come, which are made on the stream that is current now."""
+        check(_lib.load().lrqk_ctx_reserve_on(self._h, bh, max_tokens, topk, n_active, r, d,
+                                              torch.cuda.current_stream().cuda_stream if torch.cuda.is_available() else None))
 
     def set_fetch_mode(self, mode: str, host_threads: int = 0):
         """'direct': the fetch kernel reads the pinned store itself (default); 'staged': host gather +

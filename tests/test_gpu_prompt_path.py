@@ -39,6 +39,25 @@ def test_workspace_memory_is_the_caching_allocators(ops, streams):
         assert torch.cuda.memory_allocated() == before
 
 
+def test_a_reserved_workspace_goes_without_waiting(ops):
+    """Memory that is reserved while a stream is current is that stream's: the workspace is used there and dropped
+    without waiting for the device."""
+    scores = torch.randn((2, 3, 5000), device=DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ws = ops.Workspace()
+        ws.reserve(6, 5000, 512, 528, 16, 64)
+        ops.select_from_scores(ws, scores, 512)
+        torch.cuda._sleep(400_000_000)
+        busy = torch.cuda.Event()
+        busy.record()
+        ws.close()
+        waited = busy.query()
+    torch.cuda.synchronize()
+    assert not waited
+
+
 @pytest.mark.parametrize("heads,l,d,dtype", [(3, 1, 16, torch.bfloat16), (2, 257, 80, torch.bfloat16),
                                              (5, 1023, 64, torch.float32), (1, 4099, 256, torch.float32),
                                              (70, 130, 128, torch.bfloat16)])
