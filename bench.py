@@ -151,6 +151,66 @@ FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix peak, published
 BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak, published
 
 
+def prefill_roofline(w, l, iters, ms):
+    """What one factorisation of ``l`` tokens moves and multiplies, against the peaks, at ``ms`` per call."""
+    bh, bkv, r, d = w.batch * w.num_heads, w.batch * w.num_kv_heads, w.r, w.head_dim
+    # one pass = apply (2 l d r) + Grams (2 l r (r + d)); 2 initial Gram passes + 2 passes per iteration
+    flops = bh * (2 * 2.0 * l * r * (r + d) + iters * 2 * (2.0 * l * d * r + 2.0 * l * r * (r + d)))
+    e = 2 if w.dtype == torch.bfloat16 else 4
+    # HBM bytes: every pass reads X once; apply passes read and write A (fp32), Gram passes read A
+    bytes_ = bh * ((2 + 2 * iters) * l * d * e + 2 * l * r * 4 + iters * 2 * 2 * l * r * 4)
+    tf = flops / (ms * 1e-3) / 1e12
+    tuned = d == 128 and r <= 32
+    # (the library's rule for the formulation, als_prefill.hip)
+    if e == 2 and (tuned or (d in (64, 128) and l >= 2 * d)) and not os.environ.get("LRQK_PREFILL_ROWWISE"):
+        # bf16 rows of 64 or 128 elements: the iterations run on d x d Gram matrices (fp64, 32 small independent
+        # problems), and the long axis is read a fixed number of times whatever the iteration count: Q twice (sums over
+        # the given factors together with Q^T Q; the final A_Q = Q Mq) or, at rows of 128 and ranks above 32, three times
+        # (Q^T Q on its own), K three times, once per kv head (sums over the given factors, K^T K, the final A_K = K Mk;
+        # rows of 64 with a kv head per query head: K^T K with the sums).  HBM bytes: those + the initial factors read +
+        # the final factors written (fp32).
+        reads_q = 2 if tuned or d == 64 else 3
+        reads_k = 2 if d == 64 and bh == bkv else 3
+        bytes_g = (float(reads_q) * bh + float(reads_k) * bkv) * l * d * e + 4.0 * bh * l * r * 4
+        gbs = bytes_g / (ms * 1e-3) / 1e9
+        # executed bf16 MFMAs of 32x32x16 per 32 rows, with ta x 32 columns of factors and td x 32 of X: the initial Grams
+        # (three-piece operands, 16 per tile of A^T A and 6 per tile of A^T X), X^T X (two per block; the tuned kernels
+        # form both triangles) and the apply (three pieces): 40, 32 and 24 at rows of 128 and ranks up to 32
+        ta, td = (r + 31) // 32, d // 32
+        mf_given, mf_apply = 8 * ta * (ta + 1) + 6 * ta * td, 6 * ta * td
+        mf_xtx = 2 * td * td if tuned else td * (td + 1)
+        exec_flops = (l / 32.0) * (bh * 2 * (mf_given + mf_apply) + (bh + bkv) * mf_xtx) * 2.0 * 32 * 32 * 16
+        passes = ("pf_sums_kernel + pf_pass_bf16_kernel + pf_xtx_kernel + pf_apply_shared_kernel" if tuned else
+                  "pf_stream_sums_kernel + pf_stream_apply_kernel")
+        roof = {"bound": "hbm", "kernel": f"{passes} ({reads_q} readings of Q, {reads_k} of K); pf_gramdom_kernel (fp64 "
+                                          "d x d algebra per head, latency-bound) between them",
+                "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
+                "traffic": None, "hbm_bytes_per_call": round(bytes_g),
+                "algorithmic_flops_per_call": round(flops), "algorithmic_equiv_tflops": round(tf, 2),
+                "executed_bf16_mfma_tflops": round(exec_flops / (ms * 1e-3) / 1e12, 1),
+                "executed_bf16_mfma_frac": round(exec_flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4),
+                "readings_of_the_long_axis": {"Q": reads_q, "K": reads_k}, "row_by_row_formulation_readings": 1 + iters}
+    elif e == 2 and d <= 128 and r <= 32:
+        # bf16 input: the passes run on the bf16 matrix cores (fp32 operands as three bf16 pieces), where the
+        # arithmetic is far from any limit; what bounds them is the stream over X and A
+        gbs = bytes_ / (ms * 1e-3) / 1e9
+        # executed bf16 flops: per 32 rows 24 (apply) + 8 (identity) + 24 + 16 (Grams) MFMAs of 32x32x16
+        mf_apply, mf_gram = 72, 48
+        exec_flops = bh * (l / 32.0) * (2 * mf_gram + iters * 2 * mf_apply) * 2.0 * 32 * 32 * 16
+        roof = {"bound": "hbm", "kernel": "pf_pass_bf16_kernel", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+                "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
+                "hbm_bytes_per_call": round(bytes_), "algorithmic_flops_per_call": round(flops),
+                "algorithmic_tflops": round(tf, 2),
+                "executed_bf16_mfma_tflops": round(exec_flops / (ms * 1e-3) / 1e12, 1),
+                "executed_bf16_mfma_frac": round(exec_flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)}
+    else:
+        roof = {"bound": "mfma", "kernel": "pf_pass_mfma_kernel" if r <= 32 else "pf_pass_generic_kernel", "achieved": round(tf, 2),
+                "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
+                "traffic": None, "flops_per_call": round(flops), "hbm_bytes_per_call": round(bytes_),
+                "hbm_frac": round(bytes_ / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
+    return roof
+
+
 def prefill_als(a):
     """Times lrqk_als_prefill on synthetic low-rank + noise Q, K and reports fit residuals."""
     from lrqk_amd import synth, ops
@@ -203,51 +263,8 @@ def prefill_als(a):
                "sample": f"fp32 torch-CPU factorisation of {len(hs)} of the {w.num_heads} heads at the full length "
                          f"on {threads} threads, scaled to all heads"}
         cpu.update(host)
-    # one pass = apply (2 l d r) + Grams (2 l r (r + d)); 2 initial Gram passes + 2 passes per iteration
-    flops = bh * (2 * 2.0 * l * r * (r + d) + iters * 2 * (2.0 * l * d * r + 2.0 * l * r * (r + d)))
+    roof = prefill_roofline(w, l, iters, ms)
     e = 2 if w.dtype == torch.bfloat16 else 4
-    # HBM bytes: every pass reads X once; apply passes read and write A (fp32), Gram passes read A
-    bytes_ = bh * ((2 + 2 * iters) * l * d * e + 2 * l * r * 4 + iters * 2 * 2 * l * r * 4)
-    tf = flops / (ms * 1e-3) / 1e12
-    bkv = w.batch * w.num_kv_heads
-    if e == 2 and d == 128 and r <= 32 and not os.environ.get("LRQK_PREFILL_ROWWISE"):
-        # bf16 rows of 128 elements: the iterations run on d x d Gram matrices (fp64, 32 small independent problems),
-        # and the long axis is read a fixed number of times whatever the iteration count: Q twice (sums over the
-        # given factors together with Q^T Q; the final A_Q = Q Mq), K three times, once per kv head (sums over the
-        # given factors, K^T K, the final A_K = K Mk).  HBM bytes: those + the initial factors read + the final
-        # factors written (fp32).
-        bytes_g = (2.0 * bh + 3.0 * bkv) * l * d * e + 4.0 * bh * l * r * 4
-        gbs = bytes_g / (ms * 1e-3) / 1e9
-        # executed bf16 MFMAs of 32x32x16 per 32 rows: 40 per side (initial Grams, three-piece operands),
-        # 32 per input head (X^T X), 24 per side (apply)
-        exec_flops = (l / 32.0) * (bh * 2 * (40 + 24) + (bh + bkv) * 32) * 2.0 * 32 * 32 * 16
-        roof = {"bound": "hbm", "kernel": "pf_sums_kernel + pf_pass_bf16_kernel + pf_xtx_kernel + pf_apply_shared_kernel "
-                                          "(two readings of Q, three of K); pf_gramdom_kernel (fp64 d x d algebra per "
-                                          "head, latency-bound) between them",
-                "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
-                "traffic": None, "hbm_bytes_per_call": round(bytes_g),
-                "algorithmic_flops_per_call": round(flops), "algorithmic_equiv_tflops": round(tf, 2),
-                "executed_bf16_mfma_tflops": round(exec_flops / (ms * 1e-3) / 1e12, 1),
-                "executed_bf16_mfma_frac": round(exec_flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4),
-                "readings_of_the_long_axis": {"Q": 2, "K": 3}, "row_by_row_formulation_readings": 1 + iters}
-    elif e == 2 and d <= 128:
-        # bf16 input: the passes run on the bf16 matrix cores (fp32 operands as three bf16 pieces), where the
-        # arithmetic is far from any limit; what bounds them is the stream over X and A
-        gbs = bytes_ / (ms * 1e-3) / 1e9
-        # executed bf16 flops: per 32 rows 24 (apply) + 8 (identity) + 24 + 16 (Grams) MFMAs of 32x32x16
-        mf_apply, mf_gram = 72, 48
-        exec_flops = bh * (l / 32.0) * (2 * mf_gram + iters * 2 * mf_apply) * 2.0 * 32 * 32 * 16
-        roof = {"bound": "hbm", "kernel": "pf_pass_bf16_kernel", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                "hbm_bytes_per_call": round(bytes_), "algorithmic_flops_per_call": round(flops),
-                "algorithmic_tflops": round(tf, 2),
-                "executed_bf16_mfma_tflops": round(exec_flops / (ms * 1e-3) / 1e12, 1),
-                "executed_bf16_mfma_frac": round(exec_flops / (ms * 1e-3) / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)}
-    else:
-        roof = {"bound": "mfma", "kernel": "pf_pass_mfma_kernel", "achieved": round(tf, 2),
-                "peak": FP32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(tf / FP32_MFMA_PEAK_TFLOPS, 4),
-                "traffic": None, "flops_per_call": round(flops), "hbm_bytes_per_call": round(bytes_),
-                "hbm_frac": round(bytes_ / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
     out = {"metric": "lrqk_prefill_als_ms", "value": round(ms, 3), "unit": "ms", "n_gpus": 1, "steps": steps,
            "warmup": warm, "ms_per_step": round(ms, 3), "higher_is_better": False, "scaling": "weak",
            "vs_baseline": None, "dtype": "f32", "data": "synthetic",

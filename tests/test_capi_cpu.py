@@ -120,3 +120,22 @@ def test_an_allocator_that_raises_hands_out_nothing(monkeypatch, raised):
     ops._torch_release(4096, None)
     monkeypatch.undo()
     assert not left
+
+
+@pytest.mark.parametrize("dtype,d,r,l,kernels,per_iteration", [
+    (torch.bfloat16, 128, 32, 100, "pf_sums_kernel", False), (torch.bfloat16, 128, 64, 256, "pf_stream_sums_kernel", False),
+    (torch.bfloat16, 64, 16, 4096, "pf_stream_sums_kernel", False), (torch.bfloat16, 64, 16, 127, "pf_pass_bf16_kernel", True),
+    (torch.bfloat16, 128, 64, 255, "pf_pass_generic_kernel", True), (torch.float32, 128, 16, 4096, "pf_pass_mfma_kernel", True),
+    (torch.float32, 64, 64, 4096, "pf_pass_generic_kernel", True)])
+def test_the_benchmark_prices_the_formulation_that_runs(monkeypatch, dtype, d, r, l, kernels, per_iteration):
+    """The bytes of a factorisation follow its iterations only where it runs row by row, and the kernels named are the
+    ones of the library's rule (type, row width, rank, rows)."""
+    import sys
+    monkeypatch.syspath_prepend(os.path.dirname(HERE))
+    monkeypatch.delenv("LRQK_PREFILL_ROWWISE", raising=False)
+    import bench
+    from lrqk_amd import synth
+    w = synth.Workload("t", 8, 2, d, 1, dtype, l, r, 64, 8, (1, 1), (0.0, 0.0), 0)
+    one, four = (bench.prefill_roofline(w, l, n, 1.0) for n in (1, 4))
+    assert one["kernel"].startswith(kernels)
+    assert (one["hbm_bytes_per_call"] != four["hbm_bytes_per_call"]) == per_iteration
