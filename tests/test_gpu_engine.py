@@ -740,6 +740,67 @@ def test_long_fp32_prompt_every_head(lrqk, oracle):
             del Q, K, A_Q0, A_K0, got
 
 
+@pytest.mark.parametrize("heads,r,k,l,iters,steps", [(8, 16, 512, 4096, (1, 1), 24), (8, 32, 512, 2531, (2, 2), 24),
+                                                     (16, 64, 8192, 40000, (4, 4), 8)])   # (many scores close to the k-th)
+def test_fp32_generation_against_fp64(lrqk, oracle, heads, r, k, l, iters, steps):
+    """A whole fp32 generation (prompt, then tokens past a flush of the ring), each side on its own factors
+    throughout: the engine, the oracle in fp64, and the oracle in fp32 as the measure of what fp32 arithmetic leaves.
+    q_hat, k_hat, B_Q, B_K, A_K and the proxy scores are held to max(1e-4, 4 x the fp32 oracle's own deviation).  The
+    sets may then differ by tokens at their edge, and by no others: a token that only one side selected has an fp64 score
+    within twice the largest deviation of the scores of the k-th one (whichever side ranked it, its score and the k-th
+    each moved by at most that).  The attention is exact over the engine's own set; against the oracle's set it may
+    differ by what the tokens that changed places weigh there, times the spread of the values."""
+    from lrqk_amd import synth
+    w = synth.Workload("t", heads, 2, 128, 1, torch.float32, l, r, k, 16, iters, (1e-8, 1e-8), steps, 3 * r // 2, 0.05)
+    Q, K, V, bases, gen = synth.prompt_qkv(w, r)
+    Q *= 4
+    start = synth.init_factors(w, l, 1)
+    stream = synth.DecodeStream(w, Q[:, :, -1:], bases, gen)
+    eng = lrqk.LightAttentionIndicesFactory(num_lite_tokens=16, attn_topk=k, num_key_value_groups=heads // 2, r=r,
+                                            max_iter=iters, tol=(1e-8, 1e-8), capacity=l + 64)
+    eng.init_factors, eng.attn_in_step = start, True
+    eng.prefill(Q.to(DEV), K.to(DEV), V.to(DEV))
+    o64, o32 = (oracle.OracleLayer(num_lite_tokens=16, attn_topk=k, num_key_value_groups=heads // 2, r=r, max_iter=iters,
+                                   tol=(1e-8, 1e-8), capacity=l + 64, compute_dtype=c) for c in (torch.float64, torch.float32))
+    for o in (o64, o32):
+        o.prefill(Q, K, V, A_Q0=start[0], A_K0=start[1])
+    tag, changed = f"fp32 generation r{r}", 0
+    for step in range(steps):
+        q, kk, vv = stream.next()
+        eng.decode(q.to(DEV), kk.to(DEV), vv.to(DEV))
+        for o in (o64, o32):
+            o.decode(q, kk, vv)
+        got = {"q_hat": eng.last_q_hat, "k_hat": eng.last_k_hat, "B_Q": eng.B_Q, "B_K": eng.B_K, "A_K": eng.A_K}
+        got = {n: t.cpu().double() for n, t in got.items()}
+        exp, own = ({"q_hat": o.last_q_hat.double(), "k_hat": o.last_k_hat.double(), "B_Q": o.B_Q.double(),
+                     "B_K": o.B_K.double(), "A_K": o.A_K.double()} for o in (o64, o32))
+        for side in (got, exp, own):
+            side["scores"] = side["q_hat"] @ side["A_K"][:, :, :o64.last_m].transpose(-1, -2)   # [b,H,1,m]
+        for name in exp:
+            _note(tag, name, _rel(got[name], exp[name]), max(TOL["decode_fp32"], 4 * _rel(own[name], exp[name])))
+        moved = (got["scores"] - exp["scores"]).abs().amax(-1)[..., 0]                          # [b,H]
+        edge = exp["scores"][:, :, 0].topk(k).values[..., -1]
+        mine, theirs = eng.hit_indices.cpu()[..., 0], o64.hit_indices[..., 0]
+        attn = oracle.attention(q, eng.Kgpu.cpu(), eng.Vgpu.cpu())
+        _note(tag, "attention over its own set", _rel(eng.last_attn, attn), TOL["attention_fp32"])
+        full = oracle.attention(q, o64.Kgpu, o64.Vgpu)
+        logits = (q.double() @ oracle.repeat_kv(torch.cat([K, torch.zeros_like(K[:, :, :64])], 2), heads // 2).double()
+                  .transpose(-1, -2))[:, :, 0] / 128 ** 0.5
+        for h in range(heads):
+            only = set(mine[0, h].tolist()) ^ set(theirs[0, h].tolist())
+            changed += len(only) // 2
+            for t in only:
+                assert abs(float(exp["scores"][0, h, 0, t] - edge[0, h])) <= 2 * float(moved[0, h]), (step, h, t)
+            # the weights of both sets, those of the tokens that changed places relative to the smaller total
+            common = torch.logsumexp((q[0, h, 0].double() @ o64.Kgpu[0, h].double().T) / 128 ** 0.5, -1)
+            weigh = sum(float(torch.exp(logits[0, h, t] - common)) for t in only if t < l)
+            late = sum(t >= l for t in only)   # (tokens of the generation are not in K: none of them changes places)
+            spread = 2 * float(torch.cat([o64.Vgpu[0, h], eng.Vgpu[0, h].cpu()]).double().norm(dim=-1).max())
+            off = float((attn[0, h] - full[0, h]).norm())
+            assert late == 0 and off <= 1e-5 * float(full[0, h].norm()) + 2 * weigh * spread, (step, h, off, weigh)
+    _say(f"{tag}: {changed} tokens changed places in {steps} steps of {heads} heads")
+
+
 def test_llama_shape_32k_lockstep(lrqk, oracle):
     """The 32K benchmark configuration at its stated shape (Llama-3-8B heads, bf16, r 32, k 2048, lite 64,
     max_iter (2,2)), 24 steps in lock step with the oracle, every head of the prefill checked on the device."""
