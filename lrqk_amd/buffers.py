@@ -136,12 +136,13 @@ def _host_stores_ahead(device: torch.device, nbytes: int):
 def _store_came_back(pending, stream: torch.cuda.Stream, nbytes: int):
     """A store is released: what its stream has been given until now is what the GPU may still do with it."""
     try:
-        with torch.cuda.stream(stream):
-            if torch.cuda.is_current_stream_capturing():   # (the mark would become part of the graph)
-                return
+        if stream != torch.cuda.current_stream(stream.device):
+            with torch.cuda.stream(stream):
+                return _store_came_back(pending, stream, nbytes)
+        if not torch.cuda.is_current_stream_capturing():   # (the mark would become part of the graph)
             mark = torch.cuda.Event()
-            mark.record()
-        pending.append((mark, nbytes))
+            mark.record(stream)
+            pending.append((mark, nbytes))
     except Exception:  # the interpreter or the device is going
         pass
 
