@@ -16,8 +16,8 @@
 // A_Q = Q Mq and A_K = K Mk, whatever the iteration count; the row-by-row formulation reads it twice per
 // iteration and twice more.
 //
-// Sq and Sk square the condition number of the inputs, so the d x d algebra is done in fp64 (vector
-// ALU: these are 32 independent problems of a few MFLOP each); the sums Sq, Sk themselves are exact
+// Sq and Sk square the condition number of the inputs, so the d x d algebra is done in fp64 (on the matrix cores, one
+// workgroup per head: these are 32 independent problems of a few MFLOP each); the sums Sq, Sk themselves are exact
 // bf16 x bf16 products added in fp32 tile by tile and across tiles, then across splits in fp64.  Measured
 // against the fp64 restatement the results are closer than the same iteration in fp32 LAPACK.
 #include <algorithm>

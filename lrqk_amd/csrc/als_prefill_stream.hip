@@ -269,7 +269,8 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(StSums g) {
 // A = X M for every query head (its kv head's X): M^T (fp32, [head][r][d]) in LDS as three bf16 pieces, X through the
 // wave's private tile.  One launch for the sides given: workgroups (s, head) with s below side[0].S are the first side's
 // splits, the others the second's (a cache asks for one row of A_Q: alone that is a launch and 8 us).  The workgroups of
-// the query heads that share a kv head lie next to each other, so K comes from the caches after the first of them.
+// the query heads that share a kv head lie next to each other, so K comes from the last-level cache after the first of
+// them (not from an L2: they are on different XCDs, and the counters show K once per query head beyond the L2s).
 template <typename OUT>
 struct StApply {
   const bf16_t* x;
