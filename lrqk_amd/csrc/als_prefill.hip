@@ -1123,9 +1123,10 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   float* partQ = (float*)ctx->prefill_ws.p;
   float* partK = partQ + n_part;
   float* Mt = partK + n_part;
-  float* b_q = Mt + n_mt;
-  float* b_k = b_q + n_mt;
-  float* deltas = b_k + n_mt;
+  const bool convert = out.storage && sizeof(T) == 2;
+  float* b_q = convert ? Mt + n_mt : (float*)out.b_q;  // (fp32 results where they go; the place in the workspace stays unused)
+  float* b_k = convert ? Mt + 2 * n_mt : (float*)out.b_k;
+  float* deltas = Mt + 3 * n_mt;
   int* flags = (int*)(deltas + n_delta);
 
   PfPassFn<T> pass = pf_pass_generic_kernel<T>;
@@ -1188,7 +1189,7 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
     if ((rcs = prefill_store<OUT>(b_q, rd, ob_q, rd, rd, 1, st))) return rcs;
     return prefill_store<OUT>(b_k, rd, ob_k, rd, rd, 1, st);
   };
-  if (out.storage && sizeof(T) == 2) return finish((T*)out.a_q, (T*)out.a_k, (T*)out.b_q, (T*)out.b_k);
+  if (convert) return finish((T*)out.a_q, (T*)out.a_k, (T*)out.b_q, (T*)out.b_k);
   return finish((float*)out.a_q, (float*)out.a_k, (float*)out.b_q, (float*)out.b_k);
 }
 

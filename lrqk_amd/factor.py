@@ -70,6 +70,8 @@ def cast_lrqk_prefill(Q: torch.Tensor, K: torch.Tensor, r: int, lambda_Q: float 
     ws = workspace or ops.default_workspace()
     Qc, Kc = Q.contiguous(), K.contiguous()
     A_Q0, A_K0 = _initial_factors(Qc, Kc, r, init_method, init_factors)
+    if Qc.dtype == torch.float32:   # the factors are formed in place of the initial ones: nothing to convert or to copy
+        return (o for o in ops.als_prefill(ws, Qc, Kc, A_Q0, A_K0, max_iter, tol))
     return (o for o in ops.als_prefill_store(ws, Qc, Kc, A_Q0, A_K0, max_iter, tol))
 
 

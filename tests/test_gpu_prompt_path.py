@@ -249,6 +249,23 @@ def test_sums_over_millions_of_rows(ops, d):
             assert off < 2 * (16 + 8), name
 
 
+@pytest.mark.parametrize("d,r", [(64, 16), (128, 48), (32, 8)])
+def test_fp32_factors_are_not_copied(ops, monkeypatch, d, r):
+    """fp32 results of cast_lrqk_prefill lie where the initial factors lay, and are those of the form that writes them
+    into a cache's buffers."""
+    from lrqk_amd import cast_lrqk_prefill, factor
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    Q = torch.randn((1, 4, 300, d), generator=gen, device=DEV)
+    K = torch.randn((1, 2, 300, d), generator=gen, device=DEV)
+    start = tuple(torch.randn((1, 4, 300, r), generator=gen, device=DEV) for _ in range(2))
+    seen, make = [], factor._initial_factors
+    monkeypatch.setattr(factor, "_initial_factors", lambda *a: seen.append(make(*a)) or seen[-1])
+    got = tuple(cast_lrqk_prefill(Q, K, r, max_iter=2, tol=0.0, init_factors=start))
+    want = ops.als_prefill_store(ops.Workspace(), Q, K, start[0].clone(), start[1].clone(), 2, 0.0)
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
+    assert (got[0].data_ptr(), got[2].data_ptr()) == tuple(t.data_ptr() for t in seen[0])
+
+
 @pytest.mark.parametrize("d,r,l", [(64, 16, 700), (64, 48, 129), (128, 32, 5000), (128, 64, 2531)])
 def test_fp32_rows_are_factorised_row_by_row(ops, monkeypatch, d, r, l):
     """fp32 prompts take the row-by-row formulation, to the bit, at every width and rank that bf16 rows take to Gram
