@@ -458,35 +458,24 @@ __device__ __forceinline__ double gd_rcp(double x) {
   return fma(fma(-x, inv, 1.0), inv, inv);
 }
 
-// R = D^-1 for a 4 x 4 matrix with positive definite symmetric part, by 2 x 2 blocks (no pivoting):
-// D = [[A, B], [C, E]], S = E - C A^-1 B, D^-1 = [[A^-1 + Y S^-1 Z, -Y S^-1], [-S^-1 Z, S^-1]], Y = A^-1 B, Z = C A^-1.
+// D x = e for a 4 x 4 matrix with positive definite symmetric part, by 2 x 2 blocks (no pivoting): with
+// D = [[A, B], [C, E]], Y = A^-1 B and S = E - C Y,  x2 = S^-1 (e2 - C A^-1 e1),  x1 = A^-1 e1 - Y x2.
 // D is taken as it is, not as symmetric: the Gram sums it comes from are symmetric only up to their rounding, and
-// the elimination around it uses both triangles.
-__device__ __forceinline__ void gd_inv4(const double (&D)[4][4], double (&R)[4][4]) {
+// the elimination around it uses both triangles.  (A lane needs one column of the inverse: the whole of it took twice
+// the operations, and selecting a column from it 24 more.)
+__device__ __forceinline__ void gd_solve4(const double (&D)[4][4], const double (&e)[4], double (&x)[4]) {
   const double ia = gd_rcp(fma(D[0][0], D[1][1], -D[0][1] * D[1][0]));
-  const double a00 = D[1][1] * ia, a01 = -D[0][1] * ia, a10 = -D[1][0] * ia, a11 = D[0][0] * ia;  // A^-1
-  // Y = A^-1 B  (B = D[0..1][2..3]),  Z = C A^-1  (C = D[2..3][0..1])
-  const double y00 = fma(a00, D[0][2], a01 * D[1][2]), y01 = fma(a00, D[0][3], a01 * D[1][3]);
-  const double y10 = fma(a10, D[0][2], a11 * D[1][2]), y11 = fma(a10, D[0][3], a11 * D[1][3]);
-  const double z00 = fma(D[2][0], a00, D[2][1] * a10), z01 = fma(D[2][0], a01, D[2][1] * a11);
-  const double z10 = fma(D[3][0], a00, D[3][1] * a10), z11 = fma(D[3][0], a01, D[3][1] * a11);
-  // S = E - C Y
-  const double s00 = D[2][2] - fma(D[2][0], y00, D[2][1] * y10), s01 = D[2][3] - fma(D[2][0], y01, D[2][1] * y11);
-  const double s10 = D[3][2] - fma(D[3][0], y00, D[3][1] * y10), s11 = D[3][3] - fma(D[3][0], y01, D[3][1] * y11);
+  const double y00 = fma(D[1][1], D[0][2], -D[0][1] * D[1][2]) * ia, y01 = fma(D[1][1], D[0][3], -D[0][1] * D[1][3]) * ia;
+  const double y10 = fma(D[0][0], D[1][2], -D[1][0] * D[0][2]) * ia, y11 = fma(D[0][0], D[1][3], -D[1][0] * D[0][3]) * ia;
+  const double w0 = fma(D[1][1], e[0], -D[0][1] * e[1]) * ia, w1 = fma(D[0][0], e[1], -D[1][0] * e[0]) * ia;
+  const double s00 = fma(-D[2][1], y10, fma(-D[2][0], y00, D[2][2])), s01 = fma(-D[2][1], y11, fma(-D[2][0], y01, D[2][3]));
+  const double s10 = fma(-D[3][1], y10, fma(-D[3][0], y00, D[3][2])), s11 = fma(-D[3][1], y11, fma(-D[3][0], y01, D[3][3]));
   const double is = gd_rcp(fma(s00, s11, -s01 * s10));
-  const double t00 = s11 * is, t01 = -s01 * is, t10 = -s10 * is, t11 = s00 * is;  // S^-1
-  // U = Y S^-1 (upper right, negated), V = S^-1 Z (lower left, negated)
-  const double u00 = fma(y00, t00, y01 * t10), u01 = fma(y00, t01, y01 * t11);
-  const double u10 = fma(y10, t00, y11 * t10), u11 = fma(y10, t01, y11 * t11);
-  const double v00 = fma(t00, z00, t01 * z10), v01 = fma(t00, z01, t01 * z11);
-  const double v10 = fma(t10, z00, t11 * z10), v11 = fma(t10, z01, t11 * z11);
-  R[0][0] = a00 + fma(u00, z00, u01 * z10);
-  R[0][1] = a01 + fma(u00, z01, u01 * z11);
-  R[1][0] = a10 + fma(u10, z00, u11 * z10);
-  R[1][1] = a11 + fma(u10, z01, u11 * z11);
-  R[0][2] = -u00; R[0][3] = -u01; R[1][2] = -u10; R[1][3] = -u11;
-  R[2][0] = -v00; R[2][1] = -v01; R[3][0] = -v10; R[3][1] = -v11;
-  R[2][2] = t00; R[2][3] = t01; R[3][2] = t10; R[3][3] = t11;
+  const double g0 = fma(-D[2][1], w1, fma(-D[2][0], w0, e[2])), g1 = fma(-D[3][1], w1, fma(-D[3][0], w0, e[3]));
+  x[2] = fma(s11, g0, -s01 * g1) * is;
+  x[3] = fma(s00, g1, -s10 * g0) * is;
+  x[0] = fma(-y01, x[3], fma(-y00, x[2], w0));
+  x[1] = fma(-y11, x[3], fma(-y10, x[2], w1));
 }
 
 template <int RT, int CT>
@@ -496,14 +485,40 @@ struct GdSys {
   gd_v4d x[RT][CT];  // this wave's columns of RHS: [row tile][column tile CT (wave % 4) + u]
 };
 // Solves the two systems of a pair, one per half of the workgroup (s: the system of this wave's half).
+// A step waits for the step before it only through the column tile that holds its pivots; the products on the other
+// tiles (what is left of W, the right-hand columns) are a step behind, so that they run while the next pivot block is on
+// its way through LDS and inverted.  A step in cycles at
+// RT = 1, 2, 4, one wave per SIMD: 1080, 1450, 2070 with the products of a step behind its inversion and a lane's column
+// picked from the whole inverse; 800, 1000, 1450 now (64 of them a product of 16 x 16 x 4).
 template <int RT, int CT>
 __device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT>& s, double* __restrict__ piv) {
-  constexpr int RP = 16 * RT;
+  constexpr int RP = 16 * RT, STEPS = 4 * RT;
   constexpr bool WIDE = RT == 4;
-  const int lane = lane_id(), wave = wave_id(), wq = wave & 3;
+  const int lane = lane_id(), wave = gd_wave(), wq = wave & 3;
   const int li = lane & 15, lk = lane >> 4;
+  const double unit[4] = {lk == 0 ? 1.0 : 0.0, lk == 1 ? 1.0 : 0.0, lk == 2 ? 1.0 : 0.0, lk == 3 ? 1.0 : 0.0};
+  double aop[RT];
+  // the product of step m on a column of tiles
+  auto product = [&](int m, auto& t, int u) {
+    const int tp = m >> 2, vp = m & 3;
+    const double bop = t[tp][u][vp];
+    t[tp][u][vp] = 0.0;
 #pragma unroll
-  for (int m = 0; m < 4 * RT; ++m) {
+    for (int rt = 0; rt < RT; ++rt) t[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[rt], bop, t[rt][u], 0, 0, 0);
+  };
+  // what step m leaves for later: the tiles of W beyond the next pivots' (those before it hold finished columns, which
+  // nothing reads again), and the right-hand columns
+  auto behind = [&](int m) {
+    if constexpr (!WIDE) {
+#pragma unroll
+      for (int u = 0; u < RT; ++u)
+        if (u > (m + 1) >> 2) product(m, s.w, u);
+    }
+#pragma unroll
+    for (int u = 0; u < CT; ++u) product(m, s.x, u);
+  };
+#pragma unroll
+  for (int m = 0; m < STEPS; ++m) {
     const int tp = m >> 2, vp = m & 3;  // the pivots' tile (row tile of the pivot rows, column tile of W) and element
     // P: the wave's own slot, or (WIDE) one of two slots per system that its four waves read
     double* P = piv + (WIDE ? (m & 1) * 2 + (wave >> 2) : wave) * RP * 4;
@@ -521,59 +536,44 @@ __device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT>& s, double* __restri
       __syncthreads();
     else
       gd_wave_sync();
-    // every lane inverts the pivot block and keeps what its operands take of it: column l / 16, and the element of row
-    // l % 4 in that column
-    double ic[4], mine;
-    {
-      double D[4][4], R[4][4];
+    double D[4][4], prow[RT][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double2 lo = *reinterpret_cast<const double2*>(&P[(4 * m + i) * 4]);
-        const double2 hi = *reinterpret_cast<const double2*>(&P[(4 * m + i) * 4 + 2]);
-        D[i][0] = lo.x; D[i][1] = lo.y; D[i][2] = hi.x; D[i][3] = hi.y;
-      }
-      gd_inv4(D, R);
-      // (by value: a choice between array elements is one between addresses, and puts the array into scratch memory)
-      auto pick = [](int i, double e0, double e1, double e2, double e3) {
-        const double c01 = i & 1 ? e1 : e0, c23 = i & 1 ? e3 : e2;
-        return i & 2 ? c23 : c01;
-      };
-#pragma unroll
-      for (int k = 0; k < 4; ++k) ic[k] = pick(lk, R[k][0], R[k][1], R[k][2], R[k][3]);
-      mine = pick(li, ic[0], ic[1], ic[2], ic[3]);
+    for (int i = 0; i < 4; ++i) {
+      const double2 lo = *reinterpret_cast<const double2*>(&P[(4 * m + i) * 4]);
+      const double2 hi = *reinterpret_cast<const double2*>(&P[(4 * m + i) * 4 + 2]);
+      D[i][0] = lo.x; D[i][1] = lo.y; D[i][2] = hi.x; D[i][3] = hi.y;
     }
-    double aop[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      const int row = 16 * rt + li;
-      const double2 lo = *reinterpret_cast<const double2*>(&P[row * 4]);
-      const double2 hi = *reinterpret_cast<const double2*>(&P[row * 4 + 2]);
+      const double2 lo = *reinterpret_cast<const double2*>(&P[(16 * rt + li) * 4]);
+      const double2 hi = *reinterpret_cast<const double2*>(&P[(16 * rt + li) * 4 + 2]);
+      prow[rt][0] = lo.x; prow[rt][1] = lo.y; prow[rt][2] = hi.x; prow[rt][3] = hi.y;
+    }
+    if (m > 0) behind(m - 1);
+    // every lane solves for its column l / 16 of the pivot block's inverse, and keeps that column's element of row l % 4
+    double ic[4];
+    gd_solve4(D, unit, ic);
+    // (by value: a choice between array elements is one between addresses, and puts the array into scratch memory)
+    auto pick = [](int i, double e0, double e1, double e2, double e3) {
+      const double c01 = i & 1 ? e1 : e0, c23 = i & 1 ? e3 : e2;
+      return i & 2 ? c23 : c01;
+    };
+    const double mine = pick(li, ic[0], ic[1], ic[2], ic[3]);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
       // pivot rows: the rows of D^-1 themselves (their accumulators are cleared below, so they come out as
       // D^-1 X and not as X - (I - D^-1) X, which cancels in its leading digits when D is far from unit size:
       // with a diagonal of 1e12 solutions were off by 5e-3 where the conditioning allowed 1e-11)
-      const double oth = -fma(lo.x, ic[0], fma(lo.y, ic[1], fma(hi.x, ic[2], hi.y * ic[3])));
-      aop[rt] = (row >> 2) == m ? mine : oth;
+      const double oth = -fma(prow[rt][0], ic[0], fma(prow[rt][1], ic[1], fma(prow[rt][2], ic[2], prow[rt][3] * ic[3])));
+      aop[rt] = ((16 * rt + li) >> 2) == m ? mine : oth;
     }
     if constexpr (!WIDE) gd_wave_sync();  // (the reads of the slot precede the next step's writes)
-    // W: the column tiles from the pivots' on (those before hold finished unit columns: zero in the pivot rows)
-#pragma unroll
-    for (int u = 0; u < GdSys<RT, CT>::WC; ++u) {
-      if (WIDE ? wq < tp : u < tp) continue;  // (wave-uniform)
-      const double bop = s.w[tp][u][vp];
-      s.w[tp][u][vp] = 0.0;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        s.w[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[rt], bop, s.w[rt][u], 0, 0, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < CT; ++u) {
-      const double bop = s.x[tp][u][vp];
-      s.x[tp][u][vp] = 0.0;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        s.x[rt][u] = __builtin_amdgcn_mfma_f64_16x16x4f64(aop[rt], bop, s.x[rt][u], 0, 0, 0);
+    // W: the column tile of the next pivots (WIDE: every wave its own tile, unless it holds finished columns)
+    if (m + 1 < STEPS) {
+      if (!WIDE || wq >= (m + 1) >> 2) product(m, s.w, WIDE ? 0 : (m + 1) >> 2);
     }
   }
+  behind(STEPS - 1);
   if constexpr (WIDE) __syncthreads();  // (the next solve starts with slot 0 again)
 }
 
