@@ -491,7 +491,7 @@ struct GdSys {
 // RT = 1, 2, 4, one wave per SIMD: 1080, 1450, 2070 with the products of a step behind its inversion and a lane's column
 // picked from the whole inverse; 800, 1000, 1450 now (64 of them a product of 16 x 16 x 4).
 template <int RT, int CT>
-__device__ __forceinline__ void gd_solve_pair(GdSys<RT, CT>& s, double* __restrict__ piv) {
+__device__ __forceinline__ void gd_solve(GdSys<RT, CT>& s, double* __restrict__ piv) {
   constexpr int RP = 16 * RT, STEPS = 4 * RT;
   constexpr bool WIDE = RT == 4;
   const int lane = lane_id(), wave = gd_wave(), wq = wave & 3;
@@ -694,11 +694,14 @@ struct GdArgs {
   int S_k;              // splits of partK
   const double* Sq;     // [bh][d][d]
   const double* Sk;     // [b * hkv][d][d]
-  double* G;            // [2][bh][RP][RP]  (side 0: Q, 1: K), padded with the identity
+  double* G;            // [2][bh][g_parts][RP][RP]  (side 0: Q, 1: K), padded with the identity
+  int g_parts;          // 1, or the column slices whose addends of G stand side by side (the init kernel's state is the first)
   double* C;            // [2][bh][RP][d]   zero rows beyond r
   double* BqT;          // [bh][RP][d]      B_Q of the state (written by an iteration for the next)
+  double* B;            // in slices: [2][bh][RP][d]  B_Q, B_K of the state
+  double* BB;           // in slices: [2][bh][d / 64][RP][RP]  addends of B_Q B_Q^T, B_K B_K^T
   double* Gs;           // [bh][2][RP][RP + 1]  RT = 4 only: the r x r matrices of an iteration
-  double* delta;        // [iters][2][bh]   squared changes |A - A'|^2 per head
+  double* delta;        // [iters][2][bh]   squared changes |A - A'|^2 per head (in slices: [..][g_parts] addends)
   int* flags;           // [iters + 1]
   float* Mt_q;          // [bh][r][d]  Mq^T, Mk^T for the final pass over the rows
   float* Mt_k;
@@ -754,7 +757,7 @@ __global__ __launch_bounds__(256) void pf_gramdom_init_kernel(GdArgs a, const fl
     v = i == j ? 1.0 : 0.0;
   }
   if (j < RP)
-    a.G[((int64_t)side * a.bh + h) * RP * RP + i * RP + j] = v;
+    a.G[((int64_t)side * a.bh + h) * a.g_parts * RP * RP + i * RP + j] = v;
   else
     a.C[((int64_t)side * a.bh + h) * RP * D + i * D + (j - RP)] = v;
 }
@@ -855,7 +858,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
       gd_fill(sy, [&](int i, int j) { return Gk[i * RP + j]; }, [&](int i, int cc) { return Ck[i * d + cc]; });
     else
       gd_fill(sy, [&](int i, int j) { return i == j ? 1.0 : 0.0; }, [&](int, int) { return 0.0; });
-    gd_solve_pair(sy, piv);
+    gd_solve(sy, piv);
     if constexpr (FINAL) {
       const int64_t o = (int64_t)h * r * d;
       auto put = [&](void* dst, int i, int cc, double v) {
@@ -904,7 +907,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
       for (int u = 0; u < CT; ++u) sy.x[rt][u] += ckt[rt][u];
   }
   __syncthreads();  // (every read of B_Q precedes the rewriting of the B tile below)
-  gd_solve_pair(sy, piv);
+  gd_solve(sy, piv);
   // ---- the B tile now holds B_K; Mq'^T goes to its tile and to the caller, with the sum of Cq (the old one) . Mq'^T
   double part_q = 0.0;
   if (first) {
@@ -977,7 +980,7 @@ __global__ __launch_bounds__(kGdThreads) void pf_gramdom_kernel(int it, GdArgs a
     }
   }
   __syncthreads();  // (also: B_K has been read when the next B_Q takes its block)
-  gd_solve_pair(sy, piv);
+  gd_solve(sy, piv);
   double part_k = 0.0;
   if (first) {
     gd_drain(sy.x, [&](int i, int cc, double v) { BqT[i * d + cc] = v; });
@@ -1049,6 +1052,308 @@ static int gramdom_run(const GdArgs& a, const float* xq_part, int Sx, const floa
   return LRQK_OK;
 }
 
+// ---- an iteration in two launches over slices of 32 of the D columns
+// One workgroup per head leaves most of the CUs idle: 32 heads use 32 of 256, and a head's algebra (4.4 MFLOP an
+// iteration at RT = 2, 14.7 at RT = 4) is 14 and 48 us of one CU's fp64 matrix cores.  Here a side's step is one launch of
+// several workgroups per head, four waves each (two waves of a SIMD share its fp64 units: 8 waves take 1.7 times as long
+// for a solve as 4).  With Y = C + B, the slices' workgroups form
+//     Z = Y S for their columns, then [M | T] = W^-1 [Y | Z] for their columns of M and of T = M^T S at once
+// (the whole of M is nowhere needed), and their addend of G' = M^T T^T; the pair's other system, B = G^-1 C with B B^T,
+// has workgroups of its own, 64 columns each.  What a launch exchanges with the next one is T, B and the addends of
+// G' and B B^T, which the consumers add up.
+template <int RT, int D>
+struct GsShape {
+  static constexpr int RP = 16 * RT, LD = RP + 2, LG = RP + 1;
+  static constexpr int NS = D / 32, NP = D / 64;  // workgroups of a head: slices, and for the other system
+  static constexpr int LX = D + 4;                // doubles per row of Y: lanes of 16 rows read 16 different bank pairs
+  static constexpr int PIV = 4 * RP * 4;
+  static constexpr int WB = (RP * LG > 32 * LD ? RP * LG + 1 : 32 * LD) & ~1;
+  // W (later the slice of M, transposed), Y (plain: 64 columns of B, transposed), Z / T (transposed), slots, sums
+  static constexpr size_t SMEM = ((size_t)WB + RP * LX + 32 * LD + PIV + 16) * sizeof(double);
+  static_assert(64 * LD <= RP * LX, "the block of Y is used twice");
+};
+constexpr int kGsThreads = 256, kGsWaves = kGsThreads / kWave;
+
+// The systems of a launch (`plain`: the workgroups behind the slices):
+//   kGsStart  (all plain)   B_Q = Gq^-1 Cq
+//   kGsQ      Mq'^T = (Gk + B_Q B_Q^T)^-1 (Ck + B_Q)    plain: B_K = Gk^-1 Ck
+//   kGsK      Mk'^T = (Gq' + B_K B_K^T)^-1 (Cq' + B_K)  plain: B_Q = Gq'^-1 Cq'
+//   kGsFinal  (all plain)   the results  B_Q = Gq^-1 Cq  and  B_K = Gk^-1 Ck
+// What is read of the state is requested before the stopping test.
+enum GsStage { kGsStart, kGsQ, kGsK, kGsFinal };
+template <int RT, int D, int STAGE>
+__global__ __launch_bounds__(kGsThreads, 2) void pf_gs_kernel(int it, GdArgs a) {
+  using Sh = GsShape<RT, D>;
+  constexpr int RP = Sh::RP, LD = Sh::LD, LG = Sh::LG, LX = Sh::LX, NS = Sh::NS, NP = Sh::NP, NT = kGsThreads;
+  constexpr bool STEP = STAGE == kGsQ || STAGE == kGsK;
+  constexpr int PER = RP * RP / NT, PERX = RP * D / NT;
+  constexpr int NR = RT / 2;  // row tiles of Z per wave
+  extern __shared__ __align__(16) double gsm[];
+  double* WL = gsm;                     // [RP][LG]  W; then [32][LD]  the slice of M, transposed
+  double* YL = WL + Sh::WB;              // [RP][LX]  Y; plain: [64][LD]  B, transposed
+  double* TT = YL + RP * LX;            // [32][LD]  Z, then T, transposed
+  double* piv = TT + 32 * LD;           // the solves' slots
+  double* red = piv + Sh::PIV;          // [3][4]
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
+  const int li = lane & 15, lk = lane >> 4;
+  const int s = blockIdx.y, h = blockIdx.x, r = a.r, bh = a.bh;
+  if (h >= bh) return;
+  const bool plain = !STEP || s >= NS;
+  const int ws = STAGE == kGsQ ? 1 : STAGE == kGsK ? 0 : (STAGE == kGsFinal && s >= NP ? 1 : 0);  // the side of W and C
+  const int os = 1 - ws;                                                      // a step: the side that takes the new M
+  const int np = STAGE == kGsStart ? 1 : STAGE == kGsK ? NS : it > 0 ? NS : 1;  // addends of G: one before a side's first step
+  const int64_t rows = ((int64_t)ws * bh + h) * RP * D, orows = ((int64_t)os * bh + h) * RP * D;
+  const double* G = a.G + ((int64_t)ws * bh + h) * NS * RP * RP;
+  double* Go = a.G + (((int64_t)os * bh + h) * NS + s) * RP * RP;  // this slice's addend
+  // this lane's column of the solve: plain workgroups 64 of B; slices 32 of M (waves 0, 1) and of T (waves 2, 3)
+  const int pc = 64 * (STAGE == kGsStart ? s : STAGE == kGsFinal ? s % NP : s - NS) + 16 * wave + li;
+  const int c0 = plain ? pc : 32 * s + 16 * (wave & 1) + li;
+  GdSys<RT, 1> sy;
+
+  double w[PER];
+#pragma unroll
+  for (int u = 0; u < PER; ++u) w[u] = G[tid + u * NT];
+  if (np > 1) {
+#pragma unroll
+    for (int p = 1; p < NS; ++p)
+#pragma unroll
+      for (int u = 0; u < PER; ++u) w[u] += G[(int64_t)p * RP * RP + tid + u * NT];
+  }
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = (tid + u * NT) / RP, j = (tid + u * NT) % RP;
+    w[u] = i < r && j < r ? w[u] : (i == j ? 1.0 : 0.0);
+  }
+  double sv[STEP ? D / 4 : 1];  // S, the right-hand operand of Z: column tile wave % 2 of the slice
+  gd_v4d old[RT];               // the other side's C, for the change of its factor
+  double change = 0.0;
+  if (plain) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sy.x[rt][0][v] = a.C[rows + (16 * rt + lk + 4 * v) * D + c0];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) WL[(tid + u * NT) / RP * LG + (tid + u * NT) % RP] = w[u];
+  }
+  if constexpr (STEP) {
+    if (!plain) {
+      const double* BB = a.BB + ((int64_t)os * bh + h) * NP * RP * RP;
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int u = 0; u < PER; ++u) w[u] += BB[(int64_t)p * RP * RP + tid + u * NT];
+#pragma unroll
+      for (int u = 0; u < PER; ++u) WL[(tid + u * NT) / RP * LG + (tid + u * NT) % RP] = w[u];
+#pragma unroll
+      for (int u = 0; u < PERX; ++u) {
+        const int e = tid + u * NT;
+        YL[e / D * LX + e % D] = a.C[rows + e] + a.B[orows + e];
+      }
+      const double* S;
+      if constexpr (STAGE == kGsQ) {
+        S = a.Sq + (int64_t)h * D * D;
+      } else {
+        const int b = h / a.hq, kvh = (h % a.hq) / (a.hq / a.hkv);
+        S = a.Sk + ((int64_t)b * a.hkv + kvh) * D * D;
+      }
+      S += lk * D + c0;
+#pragma unroll
+      for (int u = 0; u < D / 4; ++u) sv[u] = S[4 * u * D];
+      if (wave < 2) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) old[rt][v] = a.C[orows + (16 * rt + lk + 4 * v) * D + c0];
+      }
+      if ((it > 0 || s == 0) && tid < r) change = Go[tid * (RP + 1)];
+    }
+  }
+
+  asm volatile("" ::: "memory");  // (the loads stay in front of the test)
+  if constexpr (STAGE == kGsK) {
+    if (a.flags[it]) return;
+  }
+  if constexpr (STAGE == kGsQ) {
+    // ---- the stopping test of the previous iteration (batch-wide, as the reference takes it)
+    int done = 0;
+    if (it > 0) {
+      const int64_t n_add = (int64_t)bh * NS;
+      const double* dq = a.delta + (int64_t)(it - 1) * 2 * n_add;
+      double sq = 0.0, sk = 0.0;
+      for (int64_t i = tid; i < n_add; i += NT) {
+        sq += dq[i];
+        sk += dq[n_add + i];
+      }
+      done = a.flags[it - 1];
+      for (int off = 32; off > 0; off >>= 1) {
+        sq += __shfl_xor(sq, off, kWave);
+        sk += __shfl_xor(sk, off, kWave);
+      }
+      if (lane == 0) {
+        red[wave] = sq;
+        red[4 + wave] = sk;
+      }
+      __syncthreads();
+      sq = red[0] + red[1] + red[2] + red[3];
+      sk = red[4] + red[5] + red[6] + red[7];
+      const double n = (double)bh * (double)a.l * (double)r;
+      done = done || fmax(sq / n, sk / n) < (double)a.tol;
+    }
+    if (h == 0 && s == 0 && tid == 0) a.flags[it] = done;
+    if (done) return;
+  }
+
+  __syncthreads();
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int u = 0; u < GdSys<RT, 1>::WC; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sy.w[rt][u][v] = WL[(16 * rt + lk + 4 * v) * LG + 16 * (RT == 4 ? wave : u) + li];
+  if constexpr (STEP) {
+    if (!plain) {
+      // ---- Z = Y S: wave w takes column tile w % 2 and half of the row tiles
+      const int r0 = 16 * NR * (wave >> 1);
+      gd_v4d z[NR];
+#pragma unroll
+      for (int n = 0; n < NR; ++n) z[n] = gd_v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int u = 0; u < D / 4; ++u)
+#pragma unroll
+        for (int n = 0; n < NR; ++n)
+          z[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(YL[(r0 + 16 * n + li) * LX + 4 * u + lk], sv[u], z[n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < NR; ++n)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) TT[(16 * (wave & 1) + li) * LD + r0 + 16 * n + lk + 4 * v] = z[n][v];
+      __syncthreads();
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = 16 * rt + lk + 4 * v;
+          sy.x[rt][0][v] = wave < 2 ? YL[i * LX + c0] : TT[(16 * (wave & 1) + li) * LD + i];
+        }
+    }
+  }
+  gd_solve(sy, piv);
+
+  if constexpr (STAGE == kGsFinal) {
+    void* dst = s >= NP ? a.b_k : a.b_q;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * rt + lk + 4 * v;
+        if (i >= r) continue;
+        const int64_t o = (int64_t)h * r * D + i * D + c0;
+        if (a.out_bf16)
+          st_f32<bf16_t>((bf16_t*)dst, o, (float)sy.x[rt][0][v]);
+        else
+          ((float*)dst)[o] = (float)sy.x[rt][0][v];
+      }
+    return;
+  }
+  // f(i, j, sum over c < N of PT[c][i] * QT[c][j]): a wave has a tile (RT = 2) or a row of tiles (RT = 4)
+  constexpr int NC = RT * RT / kGsWaves;
+  const int tr = wave * NC / RT, tc = wave * NC % RT;
+  auto outer = [&](const double* PT, const double* QT, auto n, auto&& f) {
+    gd_v4d acc[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[k] = gd_v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < decltype(n)::value; c += 4) {
+      const double av = PT[(c + lk) * LD + 16 * tr + li];
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, QT[(c + lk) * LD + 16 * (tc + k) + li], acc[k], 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) f(16 * tr + lk + 4 * v, 16 * (tc + k) + li, acc[k][v]);
+  };
+  if (plain) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = 16 * rt + lk + 4 * v;
+        a.B[rows + i * D + c0] = sy.x[rt][0][v];
+        YL[(16 * wave + li) * LD + i] = sy.x[rt][0][v];
+      }
+    __syncthreads();
+    double* out = a.BB + (((int64_t)ws * bh + h) * NP + (c0 >> 6)) * RP * RP;
+    outer(YL, YL, std::integral_constant<int, 64>{}, [&](int i, int j, double v) { out[i * RP + j] = v; });
+    return;
+  }
+  if constexpr (STEP) {
+    if (wave < 2) {
+      float* mt = (STAGE == kGsQ ? a.Mt_q : a.Mt_k) + (int64_t)h * r * D + c0;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = 16 * rt + lk + 4 * v;
+          if (i < r) mt[i * D] = (float)sy.x[rt][0][v];
+          change = fma(-2.0 * old[rt][v], sy.x[rt][0][v], change);
+          WL[(16 * wave + li) * LD + i] = sy.x[rt][0][v];
+        }
+    } else {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = 16 * rt + lk + 4 * v;
+          a.C[orows + i * D + c0] = sy.x[rt][0][v];
+          TT[(16 * (wave & 1) + li) * LD + i] = sy.x[rt][0][v];
+        }
+    }
+    __syncthreads();
+    outer(WL, TT, std::integral_constant<int, 32>{}, [&](int i, int j, double v) {
+      Go[i * RP + j] = v;
+      if (i == j && i < r) change += v;
+    });
+    for (int off = 32; off > 0; off >>= 1) change += __shfl_xor(change, off, kWave);
+    if (lane == 0) red[8 + wave] = change;
+    __syncthreads();
+    if (tid == 0) a.delta[(((int64_t)it * 2 + os) * bh + h) * NS + s] = red[8] + red[9] + red[10] + red[11];
+  }
+}
+
+template <int RT, int D>
+static int gramslice_run(const GdArgs& a, const float* xq_part, int Sx, const float* xk_part, int Sxk, int bkv, double* Sq,
+                         double* Sk, int iters, hipStream_t st) {
+  using Sh = GsShape<RT, D>;
+  constexpr int RP = Sh::RP, NS = Sh::NS, NP = Sh::NP;
+  using Fn = void (*)(int, GdArgs);
+  constexpr Fn start = pf_gs_kernel<RT, D, kGsStart>, q_side = pf_gs_kernel<RT, D, kGsQ>, k_side = pf_gs_kernel<RT, D, kGsK>,
+               last = pf_gs_kernel<RT, D, kGsFinal>;
+  static_assert(Sh::SMEM <= 160 * 1024, "LDS");
+  static std::atomic<bool> attr_dev[kMaxDeviceSlots];
+  std::atomic<bool>& attr = attr_dev[per_device_slot()];
+  if (!attr) {
+    for (Fn f : {start, q_side, k_side, last})
+      LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Sh::SMEM));
+    attr = true;
+  }
+  const unsigned init_blocks = (unsigned)(((size_t)a.bh + bkv) * (D * D / 256) + (size_t)2 * a.bh * (RP * (RP + D) / 256));
+  hipLaunchKernelGGL((pf_gramdom_init_kernel<RP, D>), dim3(init_blocks), dim3(256), 0, st, a, xq_part, Sx, xk_part, Sxk, bkv,
+                     Sq, Sk);
+  // Workgroups go round the XCDs in the order of their index: with a multiple of 8 heads in a row the workgroups of one
+  // head share an XCD, and what they all read comes into its L2 once.
+  const unsigned bh = ((unsigned)a.bh + 7) & ~7u;
+  const dim3 blk(kGsThreads);
+  if (iters > 0) hipLaunchKernelGGL(start, dim3(bh, NP), blk, Sh::SMEM, st, 0, a);
+  for (int it = 0; it < iters; ++it) {
+    hipLaunchKernelGGL(q_side, dim3(bh, NS + NP), blk, Sh::SMEM, st, it, a);
+    hipLaunchKernelGGL(k_side, dim3(bh, NS + NP), blk, Sh::SMEM, st, it, a);
+  }
+  hipLaunchKernelGGL(last, dim3(bh, 2 * NP), blk, Sh::SMEM, st, iters, a);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
+}
+
 // The whole factorisation on Gram matrices: q [b][hq][l][d], k [b][hkv][l][d], 16-byte aligned, d = 64 or 128, r <= 64;
 // a_q0, a_k0: the given factors, fp32 [b hq][l][r].
 int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* a_q0, float* a_k0, const PrefillOut& out,
@@ -1073,8 +1378,16 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
                         : hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
-  const size_t bytes = ((size_t)bh + bkv) * dd * 8 + (size_t)2 * bh * RP * (RP + d) * 8 + (size_t)bh * RP * d * 8 +
-                       (RP == 64 ? (size_t)bh * 2 * RP * (RP + 1) * 8 : 0) + (size_t)std::max(iters, 1) * 2 * bh * 8 +
+  // In slices while a launch of an iteration has at most 1.5 workgroups per CU (64 heads at d = 128): 32 heads, four
+  // iterations, the whole fit of 8192 rows 313 -> 253 us at rank 32 and 667 -> 460 at rank 64; 64 heads 294 -> 253 and
+  // 622 -> 547; 96 heads 249 -> 260 and 674 -> 747 (what the slices repeat then costs more than idle CUs do); d = 64: 32
+  // heads 170 -> 148, 96 heads 158 -> 154.  Ranks up to 16: an iteration whole takes 16 .. 24 us, two launches as long.
+  const bool slices = RP > 16 && (int64_t)bh * (d / 32 + d / 64) <= 384;
+  const size_t g_parts = slices ? d / 32 : 1;
+  const size_t n_state = slices ? (size_t)bh * 2 * (RP * d + d / 64 * RP * RP)
+                                : (size_t)bh * RP * d + (RP == 64 ? (size_t)bh * 2 * RP * (RP + 1) : 0);
+  const size_t n_delta = (size_t)std::max(iters, 1) * 2 * bh * g_parts;
+  const size_t bytes = ((size_t)bh + bkv) * dd * 8 + (size_t)2 * bh * RP * (g_parts * RP + d) * 8 + (n_state + n_delta) * 8 +
                        (size_t)2 * bh * RP * d * 4 + ((size_t)bh * Sx + (size_t)bkv * Sxk) * dd * 4 +
                        (size_t)2 * bh * S * ne * 4 + n_flags * 4;
   int rc = ctx->prefill_gd.ensure(bytes);
@@ -1090,11 +1403,17 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   double* Sk = (double*)take((size_t)bkv * dd * 8);
   a.Sq = Sq;
   a.Sk = Sk;
-  a.G = (double*)take((size_t)2 * bh * RP * RP * 8);
+  a.G = (double*)take((size_t)2 * bh * g_parts * RP * RP * 8);
+  a.g_parts = (int)g_parts;
   a.C = (double*)take((size_t)2 * bh * RP * d * 8);
-  a.BqT = (double*)take((size_t)bh * RP * d * 8);
-  if (RP == 64) a.Gs = (double*)take((size_t)bh * 2 * RP * (RP + 1) * 8);
-  a.delta = (double*)take((size_t)std::max(iters, 1) * 2 * bh * 8);
+  if (slices) {
+    a.B = (double*)take((size_t)2 * bh * RP * d * 8);
+    a.BB = (double*)take((size_t)2 * bh * (d / 64) * RP * RP * 8);
+  } else {
+    a.BqT = (double*)take((size_t)bh * RP * d * 8);
+    if (RP == 64) a.Gs = (double*)take((size_t)bh * 2 * RP * (RP + 1) * 8);
+  }
+  a.delta = (double*)take(n_delta * 8);
   a.Mt_q = (float*)take((size_t)bh * RP * d * 4);
   a.Mt_k = (float*)take((size_t)bh * RP * d * 4);
   float* xq_part = (float*)take((size_t)bh * Sx * dd * 4);
@@ -1127,9 +1446,14 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
       return rc;
   }
 #define LRQK_GD_RUN(RTV, DV) gramdom_run<RTV, DV>(a, xq_part, Sx, xk_part, Sxk, bkv, Sq, Sk, iters, st)
+#define LRQK_GS_RUN(RTV, DV) gramslice_run<RTV, DV>(a, xq_part, Sx, xk_part, Sxk, bkv, Sq, Sk, iters, st)
+  if (slices)
+    rc = d == 64 ? (RP == 32 ? LRQK_GS_RUN(2, 64) : LRQK_GS_RUN(4, 64)) : (RP == 32 ? LRQK_GS_RUN(2, 128) : LRQK_GS_RUN(4, 128));
+  else
   rc = d == 64 ? (RP == 16 ? LRQK_GD_RUN(1, 64) : RP == 32 ? LRQK_GD_RUN(2, 64) : LRQK_GD_RUN(4, 64))
                : (RP == 16 ? LRQK_GD_RUN(1, 128) : RP == 32 ? LRQK_GD_RUN(2, 128) : LRQK_GD_RUN(4, 128));
 #undef LRQK_GD_RUN
+#undef LRQK_GS_RUN
   if (rc) return rc;
   auto finish = [&](auto* a_q, auto* a_k) -> int {
     using OUT = std::remove_reference_t<decltype(*a_q)>;

@@ -231,6 +231,26 @@ def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
     assert (buf[:, :, :3] == 9).all() and (buf[:, :, 3 + l:] == 9).all()
 
 
+@pytest.mark.parametrize("d,r,heads,tol", [(64, 17, 128, 0.0), (64, 32, 129, 0.0), (128, 32, 64, 0.0), (128, 24, 65, 0.0),
+                                           (128, 33, 64, 0.0), (128, 64, 65, 0.0), (64, 64, 1, 0.0), (128, 32, 9, 1e30)])
+def test_fit_in_slices_and_whole(ops, oracle, d, r, heads, tol):
+    """The iteration in slices of a head's columns (up to 64 heads of 128 and 128 of 64; head counts that are no multiple
+    of the XCDs) and whole (one head more), and a fit that stops at its second iteration: against the oracle in fp64, with
+    the limit of the test above."""
+    gen = torch.Generator().manual_seed(heads + r)
+    from lrqk_amd import synth
+    l = 2 * d + 5
+    Q, _ = synth.low_rank_noise(gen, 1, heads, l, d, min(d, 2 * r), 0.05, torch.bfloat16)
+    K, _ = synth.low_rank_noise(gen, 1, heads, l, d, min(d, 2 * r), 0.05, torch.bfloat16)
+    A0, A1 = (torch.randn((1, heads, l, r), generator=gen) for _ in range(2))
+    got = ops.als_prefill(ops.Workspace(), Q.to(DEV), K.to(DEV), A0.to(DEV), A1.to(DEV), 3, tol)
+    ref = oracle.als_prefill_w1(*(t.to(DEV).double() for t in (Q, K, A0, A1)), 3, tol)
+    for name, g, w in zip(("A_Q", "B_Q", "A_K", "B_K"), got, ref):
+        off = float(((g.double() - w).flatten(2).norm(dim=2) / w.flatten(2).norm(dim=2)).max())
+        print(f"{name}: {off:.2e}", flush=True)
+        assert off < 2e-5, name
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_sums_over_millions_of_rows(ops, d):
     """However long the prompt, a split adds 4096 rows up in fp32: the given factors of 8M equal rows, whose sums never
