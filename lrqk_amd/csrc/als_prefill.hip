@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kPfThreads) void pf_small_generic_kernel(int stage,
 // ============================================================================ MFMA path
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-constexpr int kPfSmallThreads = 320;  // one thread per column of [32 x 32 | 32 x d], d <= 288
+constexpr int kPfSmallThreads = 512;
 
 // C tile of mfma_f32_32x32x2f32: lane l, element v -> row (the column is l & 31)
 __device__ __forceinline__ int pf_mfma_row(int lane, int v) { return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3); }
@@ -886,54 +886,65 @@ struct PfSmallShared {
 };
 
 // X = G^-1 RHS for the packed block G0 = [G (r x r) | RHS (r x d)] in LDS: the waves of the workgroup share
-// the 32-column blocks of the right-hand side, two per solve; emit(i, j, x) for i < r, j < d.
-template <typename Emit>
+// the 32-column blocks of the right-hand side, two (cb0, cb0 + 1) per solve; emit(i, j, x) for i < r, j < d.
+template <int PIVOTS, typename Emit>
 __device__ __forceinline__ void pf_solve_blocks(const float* G0, int r, int d, int cb0, float* scale, Emit&& emit) {
   const int ld = r + d;
-  solve_sweep_mfma<2>([&](int i, int j) { return G0[min(i, r - 1) * ld + min(j, r - 1)]; },
-                      [&](int b, int i, int col) {
-                        const int j = (cb0 + b) * 32 + col;
-                        const float x = G0[min(i, r - 1) * ld + r + min(j, d - 1)];
-                        return j < d ? x : 0.0f;
-                      },
-                      r, scale,
-                      [&](int b, int i, int col, float x) {
-                        const int j = (cb0 + b) * 32 + col;
-                        if (j < d) emit(i, j, x);
-                      });
+  solve_sweep_mfma<2, PIVOTS>([&](int i, int j) { return G0[min(i, r - 1) * ld + min(j, r - 1)]; },
+                              [&](int b, int i, int col) {
+                                const int j = (cb0 + b) * 32 + col;
+                                const float x = G0[min(i, r - 1) * ld + r + min(j, d - 1)];
+                                return j < d ? x : 0.0f;
+                              },
+                              r, scale,
+                              [&](int b, int i, int col, float x) {
+                                const int j = (cb0 + b) * 32 + col;
+                                if (j < d) emit(i, j, x);
+                              });
 }
 
-// sum of the S partial [r][r+d] blocks; 16 elements x 8 partials of loads in flight per thread
-__device__ __forceinline__ void pf_reduce_part(const float* __restrict__ part, int S, int ne, float* dst) {
-  constexpr int EB = 16;
-  for (int e0 = threadIdx.x; e0 < ne; e0 += EB * kPfSmallThreads) {
-    float v[EB];
-    double w[EB];  // (more than 16 partial sums -- long prompts -- are added in fp64)
+// dst[side][e] = sum of the S partial [r][r+d] blocks of a side, in their order; up to NB partials of an element (four
+// elements at a time where the blocks allow it) are requested before the first is added.
+template <typename V, int NV>
+__device__ __forceinline__ void pf_reduce_vec(const float* __restrict__ pq, const float* __restrict__ pk, int S, int ne,
+                                              int sides, float* dst) {
+  constexpr int NB = 16;
+  const int nv = ne / NV;
+  for (int t = threadIdx.x; t < sides * nv; t += kPfSmallThreads) {
+    const int side = t >= nv ? 1 : 0, e = (t - side * nv) * NV;
+    const float* src = (side ? pk : pq) + e;
+    float v[NV];
+    double w[NV];  // (more than 16 partial sums -- long prompts -- are added in fp64)
 #pragma unroll
-    for (int q = 0; q < EB; ++q) {
+    for (int q = 0; q < NV; ++q) {
       v[q] = 0.0f;
       w[q] = 0.0;
     }
-    for (int s0 = 0; s0 < S; s0 += 8) {
-      float x[EB][8];
+    for (int s0 = 0; s0 < S; s0 += NB) {
+      V x[NB];
 #pragma unroll
-      for (int q = 0; q < EB; ++q)
+      for (int u = 0; u < NB; ++u)
+        if (s0 + u < S) x[u] = *reinterpret_cast<const V*>(src + (int64_t)(s0 + u) * ne);  // (uniform)
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          x[q][u] = part[(int64_t)min(s0 + u, S - 1) * ne + min(e0 + q * kPfSmallThreads, ne - 1)];
+      for (int u = 0; u < NB; ++u)
+        if (s0 + u < S) {
+          const float* xf = reinterpret_cast<const float*>(&x[u]);
 #pragma unroll
-      for (int q = 0; q < EB; ++q)
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (s0 + u < S) {
-            v[q] += x[q][u];
-            w[q] += (double)x[q][u];
+          for (int q = 0; q < NV; ++q) {
+            v[q] += xf[q];
+            w[q] += (double)xf[q];
           }
+        }
     }
 #pragma unroll
-    for (int q = 0; q < EB; ++q)
-      if (e0 + q * kPfSmallThreads < ne) dst[e0 + q * kPfSmallThreads] = S > 16 ? (float)w[q] : v[q];
+    for (int q = 0; q < NV; ++q) dst[side * ne + e + q] = S > 16 ? (float)w[q] : v[q];
   }
+}
+__device__ __forceinline__ void pf_reduce_part(const float* pq, const float* pk, int S, int ne, int sides, float* dst) {
+  if (ne % 4 == 0)  // (blocks start at multiples of 16 bytes then)
+    pf_reduce_vec<float4, 4>(pq, pk, S, ne, sides, dst);
+  else
+    pf_reduce_vec<float, 1>(pq, pk, S, ne, sides, dst);
 }
 
 // G0[i][c] (packed [r][r+d]) <- G[i][c] + (c < r ? (B B^T)[i][c] : B[i][c-r]),  B in LDS [r][d+4], d % 4 == 0
@@ -964,6 +975,10 @@ __device__ __forceinline__ void pf_add_bbt(const float* G, const float* Bs, int 
 // stage 0: (stopping test) B_Q, B_K from the current Grams, then Mt for the A_Q update
 // stage 1: Mt for the A_K update from the new A_Q Grams
 // stage 2: final B_Q, B_K
+// One workgroup per head: latency of the partial sums (3 us) and of two solves in a row.  28 heads, rank 16, 9 splits,
+// stages 0, 1, 2: 43, 21, 32 -> 18, 11, 9 us (sums requested at once, pivots without tests and copies, one place for
+// all solves instead of three: 88 -> 18 KB of code); same results to the bit.
+template <int PIVOTS>
 __global__ __launch_bounds__(kPfSmallThreads) void pf_small32_kernel(int stage, int it, const float* __restrict__ partQ,
                                                                      const float* __restrict__ partK, int S, int bh,
                                                                      int r, int d, int64_t l, float tol,
@@ -1026,37 +1041,31 @@ __global__ __launch_bounds__(kPfSmallThreads) void pf_small32_kernel(int stage, 
 
   const float* pq = partQ + (int64_t)h * S * ne;
   const float* pk = partK + (int64_t)h * S * ne;
-  if (stage == 0 || stage == 2) {
-    pf_reduce_part(pq, S, ne, G1);
-    pf_reduce_part(pk, S, ne, G2);
-    __syncthreads();
-    // B_Q = (A_Q^T A_Q)^-1 A_Q^T Q and B_K likewise: both systems side by side, two column blocks per wave
-    for (int job = wave; job < 2 * njob; job += kWaves) {
-      if (job < njob) {
-        pf_solve_blocks(G1, r, d, 2 * job, sh.scale[wave], [&](int i, int j, float x) {
-          Bs[i * (d + 4) + j] = x;
-          b_q[(int64_t)h * r * d + i * d + j] = x;
-        });
-      } else {
-        pf_solve_blocks(G2, r, d, 2 * (job - njob), sh.scale[wave],
-                        [&](int i, int j, float x) { b_k[(int64_t)h * r * d + i * d + j] = x; });
-      }
-    }
-    if (stage == 2) return;
-    __syncthreads();
-    // Mt_Q = (A_K^T A_K + B_Q B_Q^T)^-1 (A_K^T K + B_Q)
-    pf_add_bbt(G2, Bs, r, d, G0);
-  } else {
-    // stage 1: Mt_K = (A_Q^T A_Q + B_K B_K^T)^-1 (A_Q^T Q + B_K)
-    pf_reduce_part(pq, S, ne, G1);
-    for (int e = tid; e < r * d; e += kPfSmallThreads) Bs[(e / d) * (d + 4) + e % d] = b_k[(int64_t)h * r * d + e];
-    __syncthreads();
-    pf_add_bbt(G1, Bs, r, d, G0);
-  }
+  const int64_t hrd = (int64_t)h * r * d;
+  pf_reduce_part(pq, pk, S, ne, stage == 1 ? 1 : 2, G1);
+  if (stage == 1)
+    for (int e = tid; e < r * d; e += kPfSmallThreads) Bs[(e / d) * (d + 4) + e % d] = b_k[hrd + e];
   __syncthreads();
-  for (int job = wave; job < njob; job += kWaves)
-    pf_solve_blocks(G0, r, d, 2 * job, sh.scale[wave],
-                    [&](int i, int j, float x) { Mt[(int64_t)h * r * d + i * d + j] = x; });
+  // Stages 0 and 2: B_Q = (A_Q^T A_Q)^-1 A_Q^T Q and B_K likewise, both systems side by side, two column blocks per wave.
+  // Then (stages 0 and 1) G0 and Mt.  (One place for both solves: the sweeps are a lot of code.)
+  for (int part = stage == 1 ? 1 : 0; part < (stage == 2 ? 1 : 2); ++part) {
+    if (part == 1) {
+      // Mt_Q = (A_K^T A_K + B_Q B_Q^T)^-1 (A_K^T K + B_Q),  Mt_K = (A_Q^T A_Q + B_K B_K^T)^-1 (A_Q^T Q + B_K)
+      pf_add_bbt(stage == 0 ? G2 : G1, Bs, r, d, G0);
+      __syncthreads();
+    }
+    for (int job = wave; job < (part == 1 ? njob : 2 * njob); job += kWaves) {
+      const bool k_side = job >= njob;
+      float* out = (part == 1 ? Mt : k_side ? b_k : b_q) + hrd;
+      const bool keep = part == 0 && !k_side;
+      pf_solve_blocks<PIVOTS>(part == 1 ? G0 : k_side ? G2 : G1, r, d, 2 * (k_side ? job - njob : job), sh.scale[wave],
+                              [&](int i, int j, float x) {
+                                if (keep) Bs[i * (d + 4) + j] = x;
+                                out[i * d + j] = x;
+                              });
+    }
+    __syncthreads();
+  }
 }
 
 __global__ void clear_flags_kernel(int* flags, int n) {  // (a kernel: the launches may be captured into a graph)
@@ -1100,7 +1109,7 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
       return prefill_gram_domain(ctx, (const T*)q, (const T*)k, a_q, a_k, out, b, hq, hkv, l, r, d, iters, tol, st);
   }
   const bool mfma = r <= 32 && d % VEC == 0 && d <= 256 && aligned;
-  const bool small32 = r <= 32 && d <= kPfSmallThreads - 32 && d % 4 == 0;
+  const bool small32 = r <= 32 && d <= 288 && d % 4 == 0;
   LRQK_REQUIRE(mfma || ne <= kPfThreads * kPfMaxPer, LRQK_ELIMIT, "r*(r+d)=%d exceeds %d", ne, kPfThreads * kPfMaxPer);
   // (the general pass: a 16 x 16 thread grid with ceil(r / 16) rows and 48 / that many columns of the sums per thread)
   LRQK_REQUIRE(mfma || (r <= 64 && 16 * (kPfMaxPer / ((r + 15) / 16)) >= r + d), LRQK_ELIMIT,
@@ -1146,7 +1155,7 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
       }
     }
   }
-  auto small = small32 ? pf_small32_kernel : pf_small_generic_kernel;
+  auto small = !small32 ? pf_small_generic_kernel : r <= 16 ? pf_small32_kernel<16> : pf_small32_kernel<32>;
   const size_t smem_small = small32 ? ((size_t)3 * ne + 4 + (size_t)r * (d + 4)) * sizeof(float)
                                     : ((size_t)ne + (size_t)r * (r + d + 1) + (size_t)r * (d + 1)) * sizeof(float);
   LRQK_REQUIRE(smem_small <= 160 * 1024 && smem_pass <= 160 * 1024, LRQK_ELIMIT, "r=%d d=%d need too much LDS", r, d);

@@ -1,6 +1,8 @@
 // Inverse of a small symmetric positive definite matrix on the matrix cores, shared by the decode
 // and the prefill half of the factorisation.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace lrqk {
@@ -117,16 +119,20 @@ __device__ __forceinline__ void invert_sweep_mfma(GetG&& g, int r, float* sbuf, 
 // g(i, j): element of G (any i, j < 32; values outside r x r are ignored); rhs(b, i, col): element (i, col)
 // of block b (0 outside the matrix); emit(b, i, col, x) receives X for i < r.  sbuf: 32 floats of LDS
 // owned by this wave.
-template <int NB, typename GetG, typename GetR, typename Emit>
+// PIVOTS (16 or 32, at least r): the pivots that are swept; those of the identity block change nothing that is used.  A
+// test per pivot instead made the compiler copy all 16 (NB + 1) accumulators every time, and selects between
+// expressions became divergent branches: 1000 cycles a pivot, about 220 now (three products of 64).
+template <int NB, int PIVOTS, typename GetG, typename GetR, typename Emit>
 __device__ __forceinline__ void solve_sweep_mfma(GetG&& g, GetR&& rhs, int r, float* sbuf, Emit&& emit) {
   const int lane = lane_id();
   const int col = lane & 31, half = lane >> 5;
+  constexpr int VN = PIVOTS / 2;  // elements of a lane that are rows below PIVOTS
   v16f acc, xr[NB];
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     const int i = mfma_row(lane, v);
-    const float x = g(i, col);
-    acc[v] = (i < r && col < r) ? x : (i == col ? 1.0f : 0.0f);
+    const float x = v < VN ? g(i, col) : 0.0f;
+    acc[v] = (v < VN && i < r && col < r) ? x : (i == col ? 1.0f : 0.0f);
   }
   const float s_col = col < r ? __builtin_amdgcn_rsqf(g(col, col)) : 1.0f;
   __builtin_amdgcn_wave_barrier();  // (an earlier use of sbuf by this wave is complete)
@@ -150,34 +156,41 @@ __device__ __forceinline__ void solve_sweep_mfma(GetG&& g, GetR&& rhs, int r, fl
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int i = mfma_row(lane, v);
-      xr[b][v] = i < r ? rhs(b, i, col) * sr[v] : 0.0f;
+      xr[b][v] = v < VN && i < r ? rhs(b, i, col) * sr[v] : 0.0f;
     }
 #pragma unroll
-  for (int p = 0; p < 32; ++p) {
-    if (p < r) {  // (wave-uniform)
-      const int v = ((p >> 3) << 2) + (p & 3), hp = (p >> 2) & 1;
-      const float rv = acc[v];
-      const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rv), p + 32 * hp));
-      float rc = __builtin_amdgcn_rcpf(d);
-      rc = fmaf(fmaf(-d, rc, 1.0f), rc, rc);
-      const bool inhalf = half == hp, isp = col == p;
-      const float A = inhalf ? (isp ? 1.0f - rc : rv * rc) : (isp ? 2.0f : 0.0f);
-      const float B = inhalf ? (isp ? d - 1.0f : rv) : (isp ? 1.0f : 0.0f);
+  for (int p = 0; p < PIVOTS; ++p) {
+    const int v = ((p >> 3) << 2) + (p & 3), hp = (p >> 2) & 1;
+    const float rv = acc[v];
+    const float d = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rv), p + 32 * hp));
+    float rc = __builtin_amdgcn_rcpf(d);
+    rc = fmaf(fmaf(-d, rc, 1.0f), rc, rc);
+    const bool inhalf = half == hp, isp = col == p;
+    float a_in = rv * rc, a_p = 1.0f - rc, b_p = d - 1.0f;
+    asm volatile("" : "+v"(a_in), "+v"(a_p), "+v"(b_p));  // (values, not branches)
+    const float A = inhalf ? (isp ? a_p : a_in) : (isp ? 2.0f : 0.0f);
+    const float B = inhalf ? (isp ? b_p : rv) : (isp ? 1.0f : 0.0f);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(-A, B, acc, 0, 0, 0);  // (first: the next pivot waits for it)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const float BR = inhalf ? xr[b][v] : 0.0f;
-        xr[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(-A, BR, xr[b], 0, 0, 0);
-      }
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(-A, B, acc, 0, 0, 0);
+    for (int b = 0; b < NB; ++b) {
+      const float BR = inhalf ? xr[b][v] : 0.0f;
+      xr[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(-A, BR, xr[b], 0, 0, 0);
     }
   }
+  auto out = [&](auto full) {
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int i = mfma_row(lane, v);
-      if (i < r) emit(b, i, col, xr[b][v] * sr[v]);
-    }
+      for (int v = 0; v < VN; ++v) {
+        const int i = mfma_row(lane, v);
+        if (decltype(full)::value || i < r) emit(b, i, col, xr[b][v] * sr[v]);
+      }
+  };
+  if (r == PIVOTS)  // (uniform; no test per row)
+    out(std::true_type{});
+  else
+    out(std::false_type{});
 }
 
 }  // namespace lrqk
