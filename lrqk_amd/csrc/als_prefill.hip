@@ -9,9 +9,9 @@
 // it fires the remaining launches of the loop return immediately, so the host never
 // waits inside the loop.
 //
-// Two implementations of each kernel: fp32 MFMA (32x32x2) tiles for r <= 32 and head
-// dimensions that are a multiple of the 16-byte vector, and a generic VALU version for
-// every other shape.  Both write the same partial-sum layout.
+// Implementations of each kernel: fp32 MFMA (32x32x2) tiles for r <= 32 and head dimensions that are a
+// multiple of the 16-byte vector, fp32 MFMA (16x16x4) tiles for r = 33 .. 64 and fp32 rows of 64 or 128, and a
+// generic VALU version for every other shape.  All write the same partial-sum layout.
 #include <algorithm>
 #include <stdlib.h>
 #include <type_traits>
@@ -1068,6 +1068,327 @@ __global__ __launch_bounds__(kPfSmallThreads) void pf_small32_kernel(int stage, 
   }
 }
 
+// ============================================================================ ranks 33 .. 64, fp32 rows of 64 or 128
+// The products of the fp32 matrix cores are chains of fused multiply-adds in the order of their k index
+// (32x32x2 and 16x16x4 alike), so tiles of 16 x 16 that take a sum's terms in the general kernels' order have the
+// general kernels' results to the bit: the columns of a row for C = X Mt^T, the rows of a split for A^T [A | X].
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kPfWideThreads = 512;
+// Row strides of 20 floats beyond a multiple of 64: an operand of 16 rows x 4 columns meets every bank once, one of
+// 4 rows x 16 columns a few twice.
+constexpr int kPfWideLda = 64 + 20;
+
+// One workgroup per split and head, 32 rows at a time.  Apply: wave w has the tile of rows 16 (w % 2), columns 16 (w / 2)
+// of C.  Sums: wave w has rank columns 16 (w / 2) and half of the tiles of [A | X].  Bound by the matrix cores (5 K of a
+// tile's 8 K cycles) and three barriers a tile.  24 heads of 2091 rows, rank 64: 142 -> 35 us a pass.
+template <int D>
+__global__ __launch_bounds__(kPfWideThreads, 4) void pf_pass_wide_kernel(const float* __restrict__ X, int xh, int hq,
+                                                                         int64_t l, int r, int, const float* __restrict__ Mt,
+                                                                         float* __restrict__ A, float* __restrict__ part,
+                                                                         float* __restrict__ delta_part,
+                                                                         const int* __restrict__ done_flag, int S) {
+  if (done_flag && *done_flag) return;
+  constexpr int LDX = D + 20, LDA = kPfWideLda, NT = kPfWideThreads;
+  constexpr int NX = 32 * D / (NT * 4);        // 16-byte loads of X per thread and tile
+  constexpr int NA = 32 * 64 / NT;             // elements of A per thread and tile
+  constexpr int NC = (4 + D / 16) / 2;         // tiles of [A | X] per wave
+  extern __shared__ __align__(16) float sm[];
+  float* x_s = sm;               // [32][LDX]
+  float* a_s = x_s + 32 * LDX;   // [32][LDA], zero beyond r and beyond the last row
+  float* m_s = a_s + 32 * LDA;   // [64][LDX]  Mt (apply only)
+  __shared__ float red[NT / kWave];
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
+  const int li = lane & 15, lk = lane >> 4;
+  const int h = blockIdx.y, s = blockIdx.x;
+  const int b = h / hq, head = h % hq;
+  const float* Xh = X + ((int64_t)b * xh + head / (hq / xh)) * l * D;
+  float* Ah = A + (int64_t)h * l * r;
+  const bool apply = Mt != nullptr;
+  if (apply)
+    for (int e = tid; e < 64 * D; e += NT) {
+      const int n = e / D, k = e % D;
+      m_s[n * LDX + k] = n < r ? Mt[((int64_t)h * r + n) * D + k] : 0.0f;
+    }
+  const int64_t rows_per_split = (l + S - 1) / S;
+  const int64_t r0 = (int64_t)s * rows_per_split;
+  const int64_t r1 = min(l, r0 + rows_per_split);
+  const int jt = wave >> 1, tr = wave & 1;     // apply: tile (tr, jt) of C; sums: rows jt, tiles tr * NC .. of [A | X]
+  float4 pre_x[NX];
+  float pre_a[NA];                             // given: rows of A as they go to LDS; apply: the old values of the tile of C
+  auto issue = [&](int64_t t0) {
+    const int last = (int)min((int64_t)32, r1 - t0) - 1;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = (i * NT + tid) * 4;
+      pre_x[i] = *reinterpret_cast<const float4*>(Xh + (t0 + min(e / D, last)) * D + e % D);
+    }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int row = apply ? 16 * tr + 4 * lk + i : (i * NT + tid) / 64, j = apply ? 16 * jt + li : tid % 64;
+      pre_a[i] = Ah[(t0 + min(row, last)) * r + min(j, r - 1)];
+    }
+  };
+  static_assert(NA == 4, "a lane's four elements of a tile of C");
+  floatx4 acc[NC];
+#pragma unroll
+  for (int n = 0; n < NC; ++n) acc[n] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  float dsum = 0.0f;
+  if (r0 < r1) issue(r0);
+  for (int64_t t0 = r0; t0 < r1; t0 += 32) {
+    const int rows = (int)min((int64_t)32, r1 - t0);
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = (i * NT + tid) * 4;
+      *reinterpret_cast<float4*>(&x_s[e / D * LDX + e % D]) = e / D < rows ? pre_x[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    float old[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      old[i] = pre_a[i];
+      if (!apply) {
+        const int row = (i * NT + tid) / 64, j = tid % 64;
+        a_s[row * LDA + j] = row < rows && j < r ? old[i] : 0.0f;
+      }
+    }
+    __syncthreads();  // (the first one also covers the staging of Mt)
+    if (t0 + 32 < r1) issue(t0 + 32);
+    if (apply) {
+      floatx4 c = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      const float* xa = x_s + (16 * tr + li) * LDX + lk;
+      const float* mb = m_s + (16 * jt + li) * LDX + lk;
+#pragma unroll 8
+      for (int k = 0; k < D; k += 4) c = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[k], mb[k], c, 0, 0, 0);
+      const int j = 16 * jt + li;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int row = 16 * tr + 4 * lk + v;
+        const bool ok = row < rows && j < r;
+        if (ok) {
+          const float df = old[v] - c[v];
+          dsum = fmaf(df, df, dsum);
+          Ah[(t0 + row) * r + j] = c[v];
+        }
+        a_s[row * LDA + j] = ok ? c[v] : 0.0f;
+      }
+      __syncthreads();
+    }
+    const float* aa = a_s + lk * LDA + 16 * jt + li;
+#pragma unroll
+    for (int k = 0; k < 32; k += 4) {
+      const float av = aa[k * LDA];
+#pragma unroll
+      for (int n = 0; n < NC; ++n) {
+        const int ct = tr * NC + n;  // (wave-uniform)
+        const float bv = ct < 4 ? a_s[(k + lk) * LDA + 16 * ct + li] : x_s[(k + lk) * LDX + 16 * (ct - 4) + li];
+        acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc[n], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  const int ld = r + D;
+  float* out = part + ((int64_t)h * S + s) * r * ld;
+#pragma unroll
+  for (int n = 0; n < NC; ++n) {
+    const int ct = tr * NC + n, c = 16 * (ct < 4 ? ct : ct - 4) + li;
+    if (ct < 4 && c >= r) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int j = 16 * jt + 4 * lk + v;
+      if (j < r) out[j * ld + (ct < 4 ? c : r + c)] = acc[n][v];
+    }
+  }
+  if (apply) {
+    dsum = wave_sum(dsum);
+    if (lane == 0) red[wave] = dsum;
+    __syncthreads();
+    if (tid == 0) {
+      float t = 0.0f;
+      for (int w = 0; w < NT / kWave; ++w) t += red[w];
+      delta_part[(int64_t)h * S + s] = t;
+    }
+  }
+}
+
+// The stages of pf_small_generic_kernel for 32 < r <= 64 and d <= 128, with its operations in its order (same results to
+// the bit): wave w keeps rows 8 w .. 8 w + 7 of [G | RHS] in registers, lane and column lane + 64 k; a pivot row goes
+// round through LDS, one barrier per pivot (two slots).  Workgroup (h, 0): B_Q (stages 0 and 2), then Mt; (h, 1): B_K.
+// A dependent chain of 0.2 us a pivot: 24 heads, rank 64: 947 -> 104 us a stage (median).
+constexpr int kPfWideLdb = 128 + 20;
+__global__ __launch_bounds__(kPfWideThreads, 2) void pf_small_wide_kernel(
+    int stage, int it, const float* __restrict__ partQ, const float* __restrict__ partK, int S, int bh, int r, int d, int64_t l,
+    float tol, const float* __restrict__ delta_all, int* __restrict__ flags, float* __restrict__ Mt, float* __restrict__ b_q,
+    float* __restrict__ b_k) {
+  constexpr int NT = kPfWideThreads, NW = NT / kWave;
+  static_assert(NW * 8 == 64, "64 rows");
+  __shared__ __align__(16) float Bs[64][kPfWideLdb];  // B, zero beyond r and d
+  __shared__ float GG[64][65];                        // B B^T
+  __shared__ float prow[2][192];
+  __shared__ float red[2][NW];
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
+  const int li = lane & 15, lk = lane >> 4;
+  const int h = blockIdx.x;
+  const bool k_side = blockIdx.y != 0;
+  if (stage == 1 && k_side) return;
+  const int ld = r + d, ne = r * ld;
+  const int64_t hrd = (int64_t)h * r * d;
+  if (stage == 0) {
+    int done = 0;
+    if (it > 0) {
+      const float* dq = delta_all + ((int64_t)(it - 1) * 2 + 0) * bh * S;
+      const float* dk = delta_all + ((int64_t)(it - 1) * 2 + 1) * bh * S;
+      done = flags[it - 1];
+      float sq = 0.0f, sk = 0.0f;
+      for (int i = tid; i < bh * S; i += NT) {
+        sq += dq[i];
+        sk += dk[i];
+      }
+      sq = wave_sum(sq);
+      sk = wave_sum(sk);
+      if (lane == 0) {
+        red[0][wave] = sq;
+        red[1][wave] = sk;
+      }
+      __syncthreads();
+      sq = sk = 0.0f;
+      for (int w = 0; w < NW; ++w) {
+        sq += red[0][w];
+        sk += red[1][w];
+      }
+      const float n = (float)bh * (float)l * (float)r;
+      done = done || fmaxf(sq / n, sk / n) < tol;
+    }
+    // (every workgroup computes the same decision; nothing it reads is overwritten by a launch of this iteration)
+    if (h == 0 && !k_side && tid == 0) flags[it] = done;
+    if (done) return;
+  } else if (stage == 1) {
+    if (flags[it]) return;
+  }
+
+  float M[8][3];  // rows 8 wave + e, columns lane + 64 k of [G | RHS]
+  // the sum of a side's partial blocks, in split order (more than 16 of them in fp64)
+  auto load_sums = [&](const float* part) {
+    const float* src = part + (int64_t)h * S * ne;
+    int at[8][3];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        at[e][k] = min(8 * wave + e, r - 1) * ld + min(lane + 64 * k, ld - 1);
+        M[e][k] = 0.0f;
+      }
+    if (S <= 16) {
+#pragma unroll 2
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) M[e][k] += src[(int64_t)s * ne + at[e][k]];
+    } else {
+      double w[8][3];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) w[e][k] = 0.0;
+#pragma unroll 2
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) w[e][k] += (double)src[(int64_t)s * ne + at[e][k]];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) M[e][k] = (float)w[e][k];
+    }
+  };
+  // Gauss-Jordan without pivoting: columns beyond the pivot's of every row but its own; then X = RHS / diagonal.
+  auto solve = [&](float* out, bool keep) {
+    for (int pw = 0; 8 * pw < r; ++pw) {
+#pragma unroll
+      for (int pe = 0; pe < 8; ++pe) {
+        const int p = 8 * pw + pe;
+        if (p >= r) break;  // (uniform)
+        float* row = prow[pe & 1];
+        if (wave == pw) {
+#pragma unroll
+          for (int k = 0; k < 3; ++k) row[lane + 64 * k] = M[pe][k];
+        }
+        __syncthreads();
+        const float x0 = row[lane], x1 = row[lane + 64], x2 = row[lane + 128];
+        const float inv = 1.0f / row[p];
+        const bool beyond = lane > p;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (e == pe && wave == pw) continue;  // (wave-uniform)
+          const float mp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(M[e][0]), p));
+          const float f = -(mp * inv);
+          const float m0 = fmaf(f, x0, M[e][0]);
+          M[e][0] = beyond ? m0 : M[e][0];
+          M[e][1] = fmaf(f, x1, M[e][1]);
+          M[e][2] = fmaf(f, x2, M[e][2]);
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int i = 8 * wave + e;
+      if (i >= r) break;  // (wave-uniform)
+      const float diag = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(M[e][0]), i));
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int c = lane + 64 * k - r;
+        if (c >= 0 && c < d) {
+          const float v = M[e][k] / diag;
+          out[hrd + i * d + c] = v;
+          if (keep) Bs[i][c] = v;
+        }
+      }
+    }
+  };
+  // M <- M + [B B^T | B]
+  auto add_b = [&] {
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int ti = wave >> 1, tj = 2 * (wave & 1) + n;
+      floatx4 g = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+      for (int k = 0; k < 128; k += 4)
+        if (k < d)  // (uniform; what lies beyond d is zero)
+          g = __builtin_amdgcn_mfma_f32_16x16x4f32(Bs[16 * ti + li][k + lk], Bs[16 * tj + li][k + lk], g, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) GG[16 * ti + 4 * lk + v][16 * tj + li] = g[v];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int i = 8 * wave + e, c = lane + 64 * k;
+        if (c < r)
+          M[e][k] += GG[i][c];
+        else if (c < ld)
+          M[e][k] += Bs[i][c - r];
+      }
+  };
+
+  if (stage != 2 && !k_side)
+    for (int e = tid; e < 64 * kPfWideLdb; e += NT) {
+      const int i = e / kPfWideLdb, c = e % kPfWideLdb;
+      Bs[i][c] = stage == 1 && i < r && c < d ? b_k[hrd + i * d + c] : 0.0f;
+    }
+  __syncthreads();
+  if (stage != 1) {
+    load_sums(k_side ? partK : partQ);
+    solve(k_side ? b_k : b_q, !k_side && stage == 0);
+    if (k_side || stage == 2) return;
+  }
+  // Mt_Q = (A_K^T A_K + B_Q B_Q^T)^-1 (A_K^T K + B_Q),  Mt_K = (A_Q^T A_Q + B_K B_K^T)^-1 (A_Q^T Q + B_K)
+  load_sums(stage == 0 ? partK : partQ);
+  add_b();
+  solve(Mt, false);
+}
+
 __global__ void clear_flags_kernel(int* flags, int n) {  // (a kernel: the launches may be captured into a graph)
   for (int i = threadIdx.x; i < n; i += blockDim.x) flags[i] = 0;
 }
@@ -1156,14 +1477,25 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
     }
   }
   auto small = !small32 ? pf_small_generic_kernel : r <= 16 ? pf_small32_kernel<16> : pf_small32_kernel<32>;
-  const size_t smem_small = small32 ? ((size_t)3 * ne + 4 + (size_t)r * (d + 4)) * sizeof(float)
+  const bool wide = sizeof(T) == 4 && r > 32 && r <= 64 && (d == 64 || d == 128) && aligned;
+  if constexpr (sizeof(T) == 4) {
+    if (wide) {
+      pass = d == 64 ? pf_pass_wide_kernel<64> : pf_pass_wide_kernel<128>;
+      pass_threads = kPfWideThreads;
+      smem_pass = (size_t)(32 * (d + 20) + 32 * kPfWideLda + 64 * (d + 20)) * sizeof(float);
+    }
+  }
+  const bool small_wide = r > 32 && r <= 64 && d <= 128;
+  if (small_wide) small = pf_small_wide_kernel;
+  const size_t smem_small = small_wide ? 0 : small32 ? ((size_t)3 * ne + 4 + (size_t)r * (d + 4)) * sizeof(float)
                                     : ((size_t)ne + (size_t)r * (r + d + 1) + (size_t)r * (d + 1)) * sizeof(float);
   LRQK_REQUIRE(smem_small <= 160 * 1024 && smem_pass <= 160 * 1024, LRQK_ELIMIT, "r=%d d=%d need too much LDS", r, d);
   if (smem_pass > 48 * 1024)
     LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)pass, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_pass));
   if (smem_small > 48 * 1024)
     LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)small, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_small));
-  const dim3 grid((unsigned)S, (unsigned)bh), blk((unsigned)pass_threads), sblk(small32 ? kPfSmallThreads : kPfThreads);
+  const dim3 grid((unsigned)S, (unsigned)bh), blk((unsigned)pass_threads);
+  const dim3 sgrid((unsigned)bh, small_wide ? 2 : 1), sblk(small_wide ? kPfWideThreads : small32 ? kPfSmallThreads : kPfThreads);
   const T* Q = (const T*)q;
   const T* K = (const T*)k;
   hipLaunchKernelGGL(clear_flags_kernel, dim3(1), dim3(64), 0, st, flags, iters + 1);
@@ -1176,17 +1508,17 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   for (int it = 0; it < iters; ++it) {
     float* dq = deltas + ((size_t)it * 2 + 0) * bh * S;
     float* dk = deltas + ((size_t)it * 2 + 1) * bh * S;
-    hipLaunchKernelGGL(small, dim3((unsigned)bh), sblk, smem_small, st, 0, it, partQ, partK, S, bh, r, d, l, tol,
+    hipLaunchKernelGGL(small, sgrid, sblk, smem_small, st, 0, it, partQ, partK, S, bh, r, d, l, tol,
                        deltas, flags, Mt, b_q, b_k);
     hipLaunchKernelGGL(pass, grid, blk, smem_pass, st, Q, hq, hq, l, r, d, (const float*)Mt, a_q, partQ, dq,
                        (const int*)(flags + it), S);
-    hipLaunchKernelGGL(small, dim3((unsigned)bh), sblk, smem_small, st, 1, it, partQ, partK, S, bh, r, d, l, tol,
+    hipLaunchKernelGGL(small, sgrid, sblk, smem_small, st, 1, it, partQ, partK, S, bh, r, d, l, tol,
                        deltas, flags, Mt, b_q, b_k);
     hipLaunchKernelGGL(pass, grid, blk, smem_pass, st, K, hkv, hq, l, r, d, (const float*)Mt, a_k, partK, dk,
                        (const int*)(flags + it), S);
     LRQK_HIP_CHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(small, dim3((unsigned)bh), sblk, smem_small, st, 2, iters, partQ, partK, S, bh, r, d, l, tol,
+  hipLaunchKernelGGL(small, sgrid, sblk, smem_small, st, 2, iters, partQ, partK, S, bh, r, d, l, tol,
                      deltas, flags, Mt, b_q, b_k);
   LRQK_HIP_CHECK(hipGetLastError());
   auto finish = [&](auto* o_q, auto* o_k, auto* ob_q, auto* ob_k) -> int {

@@ -302,6 +302,27 @@ def test_fp32_rows_are_factorised_row_by_row(ops, monkeypatch, d, r, l):
         assert torch.equal(g, w), name
 
 
+@pytest.mark.parametrize("d,r,hq,hkv,l,iters,tol", [
+    (128, 64, 4, 2, 33, 2, 0.0), (128, 33, 3, 1, 1000, 2, 0.0), (128, 48, 2, 2, 1, 1, 0.0),    # one row beyond a tile; one row
+    (64, 64, 2, 1, 5, 1, 0.0), (64, 40, 4, 1, 257, 0, 0.0), (128, 63, 1, 1, 40000, 1, 0.0),    # 20 partial sums: added in fp64
+    (128, 56, 4, 4, 300, 4, 1e30)])                                                            # stops at its second iteration
+def test_wide_fp32_rows_as_the_general_kernel(ops, d, r, hq, hkv, l, iters, tol):
+    """Ranks 33 to 64 of fp32 rows on the matrix cores: the factors of the general kernel (which takes rows that are not
+    16-byte aligned), to the bit."""
+    gen = torch.Generator(device=DEV).manual_seed(r + l)
+    Q, K = (torch.randn((1, h, l, d), generator=gen, device=DEV) for h in (hq, hkv))
+    A0, A1 = (torch.randn((1, hq, l, r), generator=gen, device=DEV) for _ in range(2))
+
+    def off(t):   # the same values 4 bytes beyond a multiple of 16
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    ws = ops.Workspace()
+    got = ops.als_prefill(ws, Q, K, A0.clone(), A1.clone(), iters, tol)
+    want = ops.als_prefill(ws, off(Q), off(K), A0.clone(), A1.clone(), iters, tol)
+    for name, g, w in zip(("A_Q", "B_Q", "A_K", "B_K"), got, want):
+        assert torch.isfinite(g).all() or l < r, name
+        assert torch.equal(g, w) or l < r and torch.equal(g.isfinite(), w.isfinite()), name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("r,m", [(16, 1025), (16, 4127), (32, 1056), (32, 9001), (64, 1060), (64, 5000)])
 def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
