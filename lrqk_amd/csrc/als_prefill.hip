@@ -317,6 +317,7 @@ __global__ __launch_bounds__(kPfThreads) void pf_small_generic_kernel(int stage,
 
 // ============================================================================ MFMA path
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kPfSmallThreads = 512;
 
@@ -554,6 +555,177 @@ __global__ __launch_bounds__(NW * kWave) void pf_pass_mfma_kernel(const T* __res
       }
     }
     __syncthreads();
+  }
+  if (apply) {
+    dsum = wave_sum(dsum);
+    if (lane == 0) red[wave] = dsum;
+    __syncthreads();
+    if (tid == 0) {
+      float t = 0.0f;
+      for (int w = 0; w < NW; ++w) t += red[w];
+      delta_part[(int64_t)h * S + s] = t;
+    }
+  }
+}
+
+// ---- the same pass for r <= 16 and fp32 rows of exactly D = 64 or 128 elements, on 16x16x4 tiles: a 32-wide tile is half
+// zeros at these ranks.  The products of the fp32 matrix cores are chains of fused multiply-adds in the order of their k
+// index (32x32x2 and 16x16x4 alike), and every sum here takes its terms in the order of pf_pass_mfma_kernel: the results
+// are that kernel's to the bit.
+//   apply: k in the order 0, D/2, 1, D/2 + 1, ...   A row of X lies in LDS in four quarters (column c = D/2 hi + 2 s + par
+//          in quarter hi + 2 par, place s), so a lane's operands of four products are 16 consecutive bytes.
+//   sums:  rows in the order 0 4 1 5 | 2 6 3 7 | 8 12 9 13 | 10 14 11 15 (+ 16).  Row m of an apply tile is row
+//          pf16_row(m) of the 16, which leaves C in the layout of the sums' left operand.  Tile n of A^T X holds the
+//          columns at places 8 i + n (D = 128), so a lane reads its row's 8 operands as 32 bytes.
+// Bound by the matrix cores (4352 of ~6000 cycles per wave and tile, two waves per SIMD) and the ends of the launch; Mt
+// stays in registers, the rows of A are requested a tile ahead like those of X, and the waves' sums meet in LDS at once.
+// 28 heads of 4096 rows, rank 16: 41 -> 23 us a pass (mean of sums alone and apply).
+__device__ __forceinline__ int pf16_row(int m) {  // 0 2 8 10 by m % 4, 0 4 1 5 by m / 4
+  return ((m & 2) << 2) + ((m & 1) << 1) + ((m & 4) ? 4 : 0) + ((m & 8) ? 1 : 0);
+}
+constexpr int kPf16Waves = 8;
+template <int D>
+struct Pf16Shape {
+  static constexpr int LDX = D + 4;        // floats per staged row
+  static constexpr int NT = D / 16;        // tiles of A^T X
+  static constexpr size_t SMEM = (size_t)kPf16Waves * 32 * LDX * sizeof(float);
+  static_assert((NT + 1) * 256 <= 32 * LDX, "a wave's sums fit its tile's LDS");
+};
+template <int D>
+__global__ __launch_bounds__(kPf16Waves * kWave, 2) void pf_pass_mfma16_kernel(
+    const float* __restrict__ X, int xh, int hq, int64_t l, int r, int, const float* __restrict__ Mt, float* __restrict__ A,
+    float* __restrict__ part, float* __restrict__ delta_part, const int* __restrict__ done_flag, int S) {
+  if (done_flag && *done_flag) return;
+  using Sh = Pf16Shape<D>;
+  constexpr int LDX = Sh::LDX, NT = Sh::NT, HALF = D / 2, QUART = D / 4, NW = kPf16Waves;
+  constexpr int NL = 32 * D / (kWave * 4);  // 16-byte loads per lane and tile
+  extern __shared__ __align__(16) float sm[];
+  __shared__ float red[NW];
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
+  const int li = lane & 15, lk = lane >> 4;
+  float* x_s = sm + wave * 32 * LDX;
+  const int h = blockIdx.y, s = blockIdx.x;
+  const int b = h / hq, head = h % hq;
+  const float* Xh = X + ((int64_t)b * xh + head / (hq / xh)) * l * D;
+  float* Ah = A + (int64_t)h * l * r;
+  const bool apply = Mt != nullptr;
+  const int64_t rows_per_split = (((l + S - 1) / S) + 31) / 32 * 32;
+  const int64_t r0 = (int64_t)s * rows_per_split;
+  const int64_t r1 = min(l, r0 + rows_per_split);
+
+  float4 pre[NL];
+  float old_next[8];  // rows of A: element 4 t + v is row 16 t + pf16_row(4 lk + v)
+  auto issue = [&](int64_t t0) {
+    const int last = (int)min((int64_t)32, r1 - t0) - 1;
+    const float* xt = Xh + t0 * D;
+    const float* at = Ah + t0 * r;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * 4;
+      pre[i] = gd_at<float4>(xt, 4u * (uint32_t)(min(e / D, last) * D + e % D));
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      old_next[q] = gd_factor(at, 16 * (q >> 2) + pf16_row(4 * lk + (q & 3)), last, r, min(li, r - 1));
+  };
+  const int64_t first = r0 + (int64_t)wave * 32;
+  if (first < r1) issue(first);
+  float mt[QUART];  // this lane's operands of the apply: row li of Mt, its quarter of the columns
+  if (apply) {
+    const float* Mh = Mt + ((int64_t)h * r + min(li, r - 1)) * D + (lk & 1) * HALF + (lk >> 1);
+#pragma unroll
+    for (int k = 0; k < QUART; ++k) mt[k] = li < r ? Mh[2 * k] : 0.0f;
+  }
+  floatx4 gAA = floatx4{0.0f, 0.0f, 0.0f, 0.0f}, gAX[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) gAX[n] = gAA;
+  float dsum = 0.0f;
+
+  for (int64_t t0 = first; t0 < r1; t0 += 32 * NW) {
+    const int rows = (int)min((int64_t)32, r1 - t0);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int e = (i * kWave + lane) * 4, row = e / D, c = e % D;
+      const float4 x = row < rows ? pre[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      float* at = x_s + row * LDX + (c / HALF) * QUART + (c % HALF) / 2;
+      *reinterpret_cast<float2*>(at) = make_float2(x.x, x.z);
+      *reinterpret_cast<float2*>(at + 2 * QUART) = make_float2(x.y, x.w);
+    }
+    float old[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) old[q] = old_next[q];
+    pf_wave_sync();
+    if (t0 + 32 * NW < r1) issue(t0 + 32 * NW);
+    floatx4 c[2];
+    if (apply) {
+      c[0] = c[1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+      const float* xa = x_s + pf16_row(li) * LDX + lk * QUART;
+#pragma unroll
+      for (int k = 0; k < QUART; k += 4) {
+        const float4 a0 = *reinterpret_cast<const float4*>(xa + k);
+        const float4 a1 = *reinterpret_cast<const float4*>(xa + 16 * LDX + k);
+        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.x, mt[k], c[0], 0, 0, 0);
+        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.x, mt[k], c[1], 0, 0, 0);
+        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.y, mt[k + 1], c[0], 0, 0, 0);
+        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.y, mt[k + 1], c[1], 0, 0, 0);
+        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.z, mt[k + 2], c[0], 0, 0, 0);
+        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.z, mt[k + 2], c[1], 0, 0, 0);
+        c[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0.w, mt[k + 3], c[0], 0, 0, 0);
+        c[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1.w, mt[k + 3], c[1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int row = 16 * (q >> 2) + pf16_row(4 * lk + (q & 3));
+        if (row < rows && li < r) {
+          const float v = c[q >> 2][q & 3], df = old[q] - v;
+          dsum = fmaf(df, df, dsum);
+          Ah[(t0 + row) * r + li] = v;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        c[q >> 2][q & 3] = 16 * (q >> 2) + pf16_row(4 * lk + (q & 3)) < rows && li < r ? old[q] : 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      float xb[NT];
+      const float* xr = x_s + (16 * (q >> 2) + pf16_row(4 * lk + (q & 3))) * LDX + NT * li;
+#pragma unroll
+      for (int n = 0; n < NT; n += 4) {
+        const float4 x4 = *reinterpret_cast<const float4*>(xr + n);
+        xb[n] = x4.x; xb[n + 1] = x4.y; xb[n + 2] = x4.z; xb[n + 3] = x4.w;
+      }
+      const float cv = c[q >> 2][q & 3];
+      gAA = __builtin_amdgcn_mfma_f32_16x16x4f32(cv, cv, gAA, 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) gAX[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(cv, xb[n], gAX[n], 0, 0, 0);
+    }
+    pf_wave_sync();  // this wave's reads of the tile precede its next staging writes
+  }
+  // the waves' sums side by side in LDS (each in its own tile's place), added in the waves' order
+  const auto keep = [&](int t, const floatx4& g) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x_s[t * 256 + (4 * lk + v) * 16 + li] = g[v];
+  };
+  keep(0, gAA);
+#pragma unroll
+  for (int n = 0; n < NT; ++n) keep(n + 1, gAX[n]);
+  __syncthreads();
+  const int ld = r + D;
+  float* out = part + ((int64_t)h * S + s) * r * ld;
+  for (int e = tid; e < (NT + 1) * 256; e += NW * kWave) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) v += sm[w * 32 * LDX + e];
+    const int t = e >> 8, j = (e >> 4) & 15, n = e & 15;
+    if (j >= r) continue;
+    if (t == 0) {
+      if (n < r) out[j * ld + n] = v;
+    } else {
+      const int at = NT * n + t - 1, q = at / QUART;  // place in the row: quarter q
+      out[j * ld + r + (q & 1) * HALF + 2 * (at % QUART) + (q >> 1)] = v;
+    }
   }
   if (apply) {
     dsum = wave_sum(dsum);
@@ -1072,7 +1244,6 @@ __global__ __launch_bounds__(kPfSmallThreads) void pf_small32_kernel(int stage, 
 // The products of the fp32 matrix cores are chains of fused multiply-adds in the order of their k index
 // (32x32x2 and 16x16x4 alike), so tiles of 16 x 16 that take a sum's terms in the general kernels' order have the
 // general kernels' results to the bit: the columns of a row for C = X Mt^T, the rows of a split for A^T [A | X].
-typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kPfWideThreads = 512;
 // Row strides of 20 floats beyond a multiple of 64: an operand of 16 rows x 4 columns meets every bank once, one of
 // 4 rows x 16 columns a few twice.
@@ -1474,6 +1645,12 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
         pass = nb == 1 ? pf_pass_bf16_kernel<1, 8> : nb == 2 ? pf_pass_bf16_kernel<2, 8> : pf_pass_bf16_kernel<4, 8>;
         smem_pass = std::max((size_t)(8 + 3) * 32 * (32 * nb + 16) * sizeof(uint16_t), (size_t)8 * 1024 * sizeof(float));
       }
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (mfma && r <= 16 && (d == 64 || d == 128)) {
+      pass = d == 64 ? pf_pass_mfma16_kernel<64> : pf_pass_mfma16_kernel<128>;
+      smem_pass = d == 64 ? Pf16Shape<64>::SMEM : Pf16Shape<128>::SMEM;
     }
   }
   auto small = !small32 ? pf_small_generic_kernel : r <= 16 ? pf_small32_kernel<16> : pf_small32_kernel<32>;

@@ -323,6 +323,26 @@ def test_wide_fp32_rows_as_the_general_kernel(ops, d, r, hq, hkv, l, iters, tol)
         assert torch.equal(g, w) or l < r and torch.equal(g.isfinite(), w.isfinite()), name
 
 
+@pytest.mark.parametrize("d,r,hq,hkv,l,iters,tol", [
+    (128, 16, 6, 2, 1000, 2, 0.0), (128, 1, 2, 1, 33, 1, 0.0), (128, 15, 1, 1, 40000, 1, 0.0),  # 20 partial sums: in fp64
+    (64, 16, 4, 4, 257, 3, 0.0), (64, 9, 3, 1, 31, 2, 0.0), (64, 16, 2, 1, 2531, 0, 0.0), (128, 16, 4, 2, 300, 4, 1e30)])
+def test_narrow_fp32_rows_as_wide_tiles(ops, d, r, hq, hkv, l, iters, tol):
+    """Ranks up to 16 of fp32 rows of 64 and 128 on 16-wide tiles: rows whose last four elements are zero have the factors
+    of the 32-wide tiles that rows without them take, to the bit (a product with zero changes no sum)."""
+    gen = torch.Generator(device=DEV).manual_seed(r + l)
+    Q, K = (torch.randn((1, h, l, d), generator=gen, device=DEV) for h in (hq, hkv))
+    Q[..., -4:], K[..., -4:] = 0, 0
+    A0, A1 = (torch.randn((1, hq, l, r), generator=gen, device=DEV) for _ in range(2))
+    ws = ops.Workspace()
+    got = ops.als_prefill(ws, Q, K, A0.clone(), A1.clone(), iters, tol)
+    want = ops.als_prefill(ws, Q[..., :-4].contiguous(), K[..., :-4].contiguous(), A0.clone(), A1.clone(), iters, tol)
+    for name, g, w in zip(("A_Q", "B_Q", "A_K", "B_K"), got, want):
+        if name in ("B_Q", "B_K"):
+            assert (g[..., -4:] == 0).all(), name
+            g = g[..., :-4]
+        assert torch.isfinite(g).all() and torch.equal(g, w), name
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("r,m", [(16, 1025), (16, 4127), (32, 1056), (32, 9001), (64, 1060), (64, 5000)])
 def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
