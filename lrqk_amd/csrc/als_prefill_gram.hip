@@ -699,7 +699,7 @@ struct GdArgs {
   double* C;            // [2][bh][RP][d]   zero rows beyond r
   double* BqT;          // [bh][RP][d]      B_Q of the state (written by an iteration for the next)
   double* B;            // in slices: [2][bh][RP][d]  B_Q, B_K of the state
-  double* BB;           // in slices: [2][bh][d / 64][RP][RP]  addends of B_Q B_Q^T, B_K B_K^T
+  double* BB;           // in slices: [2][bh][RP][RP]  B_Q B_Q^T, B_K B_K^T
   double* Gs;           // [bh][2][RP][RP + 1]  RT = 4 only: the r x r matrices of an iteration
   double* delta;        // [iters][2][bh]   squared changes |A - A'|^2 per head (in slices: [..][g_parts] addends)
   int* flags;           // [iters + 1]
@@ -1055,26 +1055,27 @@ static int gramdom_run(const GdArgs& a, const float* xq_part, int Sx, const floa
 // ---- an iteration in two launches over slices of 32 of the D columns
 // One workgroup per head leaves most of the CUs idle: 32 heads use 32 of 256, and a head's algebra (4.4 MFLOP an
 // iteration at RT = 2, 14.7 at RT = 4) is 14 and 48 us of one CU's fp64 matrix cores.  Here a side's step is one launch of
-// several workgroups per head, four waves each (two waves of a SIMD share its fp64 units: 8 waves take 1.7 times as long
-// for a solve as 4).  With Y = C + B, the slices' workgroups form
-//     Z = Y S for their columns, then [M | T] = W^-1 [Y | Z] for their columns of M and of T = M^T S at once
-// (the whole of M is nowhere needed), and their addend of G' = M^T T^T; the pair's other system, B = G^-1 C with B B^T,
-// has workgroups of its own, 64 columns each.  What a launch exchanges with the next one is T, B and the addends of
-// G' and B B^T, which the consumers add up.
+// several workgroups per head, four waves each (two waves of a SIMD share its fp64 units: eight waves take 1.7 times as
+// long for the same columns):
+//   * a slice's workgroup solves for the whole M (a solve is a dependent chain: D / 64 tiles of right-hand columns per wave
+//     run beside it) and forms its columns of T = M^T S and its addend of G' = M^T T^T;
+//   * one more solves the pair's other system, B = G^-1 C, and forms B B^T.
+// What a launch exchanges with the next one is T, B, B B^T and the addends of G', which the consumers add up.
+// ([M | T] = W^-1 [Y | Y S] for the slice's columns is 10 % less work, but T is then M^T S only up to the solve's rounding.)
+// An iteration at D = 128, 32 heads: 44 -> 30 us at RT = 2, 108 -> 57 at RT = 4.
 template <int RT, int D>
 struct GsShape {
   static constexpr int RP = 16 * RT, LD = RP + 2, LG = RP + 1;
-  static constexpr int NS = D / 32, NP = D / 64;  // workgroups of a head: slices, and for the other system
-  static constexpr int LX = D + 4;                // doubles per row of Y: lanes of 16 rows read 16 different bank pairs
+  static constexpr int NS = D / 32;  // slices
+  static constexpr int CT = D / 64;  // column tiles of a solve per wave
   static constexpr int PIV = 4 * RP * 4;
-  static constexpr int WB = (RP * LG > 32 * LD ? RP * LG + 1 : 32 * LD) & ~1;
-  // W (later the slice of M, transposed), Y (plain: 64 columns of B, transposed), Z / T (transposed), slots, sums
-  static constexpr size_t SMEM = ((size_t)WB + RP * LX + 32 * LD + PIV + 16) * sizeof(double);
-  static_assert(64 * LD <= RP * LX, "the block of Y is used twice");
+  static constexpr int WB = (RP * LG + 1) & ~1;
+  // W, M or B (transposed), T (transposed), slots, sums
+  static constexpr size_t SMEM = ((size_t)WB + D * LD + 32 * LD + PIV + 16) * sizeof(double);
 };
 constexpr int kGsThreads = 256, kGsWaves = kGsThreads / kWave;
 
-// The systems of a launch (`plain`: the workgroups behind the slices):
+// The systems of a launch (`plain`: the last workgroup of a head):
 //   kGsStart  (all plain)   B_Q = Gq^-1 Cq
 //   kGsQ      Mq'^T = (Gk + B_Q B_Q^T)^-1 (Ck + B_Q)    plain: B_K = Gk^-1 Ck
 //   kGsK      Mk'^T = (Gq' + B_K B_K^T)^-1 (Cq' + B_K)  plain: B_Q = Gq'^-1 Cq'
@@ -1084,31 +1085,32 @@ enum GsStage { kGsStart, kGsQ, kGsK, kGsFinal };
 template <int RT, int D, int STAGE>
 __global__ __launch_bounds__(kGsThreads, 2) void pf_gs_kernel(int it, GdArgs a) {
   using Sh = GsShape<RT, D>;
-  constexpr int RP = Sh::RP, LD = Sh::LD, LG = Sh::LG, LX = Sh::LX, NS = Sh::NS, NP = Sh::NP, NT = kGsThreads;
+  constexpr int RP = Sh::RP, LD = Sh::LD, LG = Sh::LG, NS = Sh::NS, CT = Sh::CT, NT = kGsThreads;
   constexpr bool STEP = STAGE == kGsQ || STAGE == kGsK;
-  constexpr int PER = RP * RP / NT, PERX = RP * D / NT;
-  constexpr int NR = RT / 2;  // row tiles of Z per wave
+  constexpr int PER = RP * RP / NT;
+  constexpr int NR = RT / 2;  // row tiles of T per wave
+  constexpr bool EARLY = RT == 2 || D == 64;  // S is requested ahead of the solve (else the registers do not go round)
   extern __shared__ __align__(16) double gsm[];
-  double* WL = gsm;                     // [RP][LG]  W; then [32][LD]  the slice of M, transposed
-  double* YL = WL + Sh::WB;              // [RP][LX]  Y; plain: [64][LD]  B, transposed
-  double* TT = YL + RP * LX;            // [32][LD]  Z, then T, transposed
-  double* piv = TT + 32 * LD;           // the solves' slots
-  double* red = piv + Sh::PIV;          // [3][4]
+  double* WL = gsm;             // [RP][LG]  W
+  double* ML = WL + Sh::WB;     // [D][LD]   M or B, transposed (not in W's block: other waves may still read that)
+  double* TT = ML + D * LD;     // [32][LD]  the slice of T, transposed
+  double* piv = TT + 32 * LD;   // the solves' slots
+  double* red = piv + Sh::PIV;  // [3][4]
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   const int li = lane & 15, lk = lane >> 4;
   const int s = blockIdx.y, h = blockIdx.x, r = a.r, bh = a.bh;
   if (h >= bh) return;
   const bool plain = !STEP || s >= NS;
-  const int ws = STAGE == kGsQ ? 1 : STAGE == kGsK ? 0 : (STAGE == kGsFinal && s >= NP ? 1 : 0);  // the side of W and C
-  const int os = 1 - ws;                                                      // a step: the side that takes the new M
+  const int ws = STAGE == kGsQ ? 1 : STAGE == kGsK ? 0 : (STAGE == kGsFinal ? s : 0);  // the side of W and C
+  const int os = 1 - ws;                                                               // a step: the side that takes the new M
   const int np = STAGE == kGsStart ? 1 : STAGE == kGsK ? NS : it > 0 ? NS : 1;  // addends of G: one before a side's first step
   const int64_t rows = ((int64_t)ws * bh + h) * RP * D, orows = ((int64_t)os * bh + h) * RP * D;
   const double* G = a.G + ((int64_t)ws * bh + h) * NS * RP * RP;
   double* Go = a.G + (((int64_t)os * bh + h) * NS + s) * RP * RP;  // this slice's addend
-  // this lane's column of the solve: plain workgroups 64 of B; slices 32 of M (waves 0, 1) and of T (waves 2, 3)
-  const int pc = 64 * (STAGE == kGsStart ? s : STAGE == kGsFinal ? s % NP : s - NS) + 16 * wave + li;
-  const int c0 = plain ? pc : 32 * s + 16 * (wave & 1) + li;
-  GdSys<RT, 1> sy;
+  const int c0 = 16 * CT * wave + li;                              // this lane's column of the solve, and + 16 u
+  const int tc = 32 * s + 16 * (wave & 1) + li;                    // of the slice of T
+  const int tr = 16 * NR * (wave >> 1);                            // first row of the wave's tiles of T
+  GdSys<RT, CT> sy;
 
   double w[PER];
 #pragma unroll
@@ -1124,47 +1126,44 @@ __global__ __launch_bounds__(kGsThreads, 2) void pf_gs_kernel(int it, GdArgs a) 
     const int i = (tid + u * NT) / RP, j = (tid + u * NT) % RP;
     w[u] = i < r && j < r ? w[u] : (i == j ? 1.0 : 0.0);
   }
-  double sv[STEP ? D / 4 : 1];  // S, the right-hand operand of Z: column tile wave % 2 of the slice
-  gd_v4d old[RT];               // the other side's C, for the change of its factor
-  double change = 0.0;
-  if (plain) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) sy.x[rt][0][v] = a.C[rows + (16 * rt + lk + 4 * v) * D + c0];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) WL[(tid + u * NT) / RP * LG + (tid + u * NT) % RP] = w[u];
-  }
   if constexpr (STEP) {
     if (!plain) {
-      const double* BB = a.BB + ((int64_t)os * bh + h) * NP * RP * RP;
+      const double* BB = a.BB + ((int64_t)os * bh + h) * RP * RP;
 #pragma unroll
-      for (int p = 0; p < NP; ++p)
+      for (int u = 0; u < PER; ++u) w[u] += BB[tid + u * NT];
+    }
+  }
 #pragma unroll
-        for (int u = 0; u < PER; ++u) w[u] += BB[(int64_t)p * RP * RP + tid + u * NT];
+  for (int u = 0; u < PER; ++u) WL[(tid + u * NT) / RP * LG + (tid + u * NT) % RP] = w[u];
 #pragma unroll
-      for (int u = 0; u < PER; ++u) WL[(tid + u * NT) / RP * LG + (tid + u * NT) % RP] = w[u];
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int u = 0; u < PERX; ++u) {
-        const int e = tid + u * NT;
-        YL[e / D * LX + e % D] = a.C[rows + e] + a.B[orows + e];
-      }
-      const double* S;
-      if constexpr (STAGE == kGsQ) {
-        S = a.Sq + (int64_t)h * D * D;
-      } else {
-        const int b = h / a.hq, kvh = (h % a.hq) / (a.hq / a.hkv);
-        S = a.Sk + ((int64_t)b * a.hkv + kvh) * D * D;
-      }
-      S += lk * D + c0;
+    for (int u = 0; u < CT; ++u)
 #pragma unroll
-      for (int u = 0; u < D / 4; ++u) sv[u] = S[4 * u * D];
-      if (wave < 2) {
+      for (int v = 0; v < 4; ++v) sy.x[rt][u][v] = a.C[rows + (16 * rt + lk + 4 * v) * D + c0 + 16 * u];
+  double sv[STEP ? D / 4 : 1];  // S, the right-hand operand of T: column tile wave % 2 of the slice
+  auto s_loads = [&] {
+    const double* S;
+    if constexpr (STAGE == kGsQ) {
+      S = a.Sq + (int64_t)h * D * D;
+    } else {
+      const int b = h / a.hq, kvh = (h % a.hq) / (a.hq / a.hkv);
+      S = a.Sk + ((int64_t)b * a.hkv + kvh) * D * D;
+    }
+    S += lk * D + tc;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
+    for (int u = 0; u < D / 4; ++u) sv[u] = S[4 * u * D];
+  };
+  double change = 0.0;
+  if constexpr (STEP) {
+    if (!plain) {
 #pragma unroll
-          for (int v = 0; v < 4; ++v) old[rt][v] = a.C[orows + (16 * rt + lk + 4 * v) * D + c0];
-      }
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int u = 0; u < CT; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) sy.x[rt][u][v] += a.B[orows + (16 * rt + lk + 4 * v) * D + c0 + 16 * u];
+      if constexpr (EARLY) s_loads();
       if ((it > 0 || s == 0) && tid < r) change = Go[tid * (RP + 1)];
     }
   }
@@ -1207,110 +1206,112 @@ __global__ __launch_bounds__(kGsThreads, 2) void pf_gs_kernel(int it, GdArgs a) 
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int u = 0; u < GdSys<RT, 1>::WC; ++u)
+    for (int u = 0; u < GdSys<RT, CT>::WC; ++u)
 #pragma unroll
       for (int v = 0; v < 4; ++v) sy.w[rt][u][v] = WL[(16 * rt + lk + 4 * v) * LG + 16 * (RT == 4 ? wave : u) + li];
-  if constexpr (STEP) {
-    if (!plain) {
-      // ---- Z = Y S: wave w takes column tile w % 2 and half of the row tiles
-      const int r0 = 16 * NR * (wave >> 1);
-      gd_v4d z[NR];
-#pragma unroll
-      for (int n = 0; n < NR; ++n) z[n] = gd_v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int u = 0; u < D / 4; ++u)
-#pragma unroll
-        for (int n = 0; n < NR; ++n)
-          z[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(YL[(r0 + 16 * n + li) * LX + 4 * u + lk], sv[u], z[n], 0, 0, 0);
-#pragma unroll
-      for (int n = 0; n < NR; ++n)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) TT[(16 * (wave & 1) + li) * LD + r0 + 16 * n + lk + 4 * v] = z[n][v];
-      __syncthreads();
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * rt + lk + 4 * v;
-          sy.x[rt][0][v] = wave < 2 ? YL[i * LX + c0] : TT[(16 * (wave & 1) + li) * LD + i];
-        }
-    }
-  }
   gd_solve(sy, piv);
 
   if constexpr (STAGE == kGsFinal) {
-    void* dst = s >= NP ? a.b_k : a.b_q;
+    void* dst = s ? a.b_k : a.b_q;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 16 * rt + lk + 4 * v;
-        if (i >= r) continue;
-        const int64_t o = (int64_t)h * r * D + i * D + c0;
-        if (a.out_bf16)
-          st_f32<bf16_t>((bf16_t*)dst, o, (float)sy.x[rt][0][v]);
-        else
-          ((float*)dst)[o] = (float)sy.x[rt][0][v];
-      }
+      for (int u = 0; u < CT; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = 16 * rt + lk + 4 * v;
+          if (i >= r) continue;
+          const int64_t o = (int64_t)h * r * D + i * D + c0 + 16 * u;
+          if (a.out_bf16)
+            st_f32<bf16_t>((bf16_t*)dst, o, (float)sy.x[rt][u][v]);
+          else
+            ((float*)dst)[o] = (float)sy.x[rt][u][v];
+        }
     return;
   }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int u = 0; u < CT; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) ML[(c0 + 16 * u) * LD + 16 * rt + lk + 4 * v] = sy.x[rt][u][v];
   // f(i, j, sum over c < N of PT[c][i] * QT[c][j]): a wave has a tile (RT = 2) or a row of tiles (RT = 4)
   constexpr int NC = RT * RT / kGsWaves;
-  const int tr = wave * NC / RT, tc = wave * NC % RT;
+  const int otr = wave * NC / RT, otc = wave * NC % RT;
   auto outer = [&](const double* PT, const double* QT, auto n, auto&& f) {
     gd_v4d acc[NC];
 #pragma unroll
     for (int k = 0; k < NC; ++k) acc[k] = gd_v4d{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
+#pragma unroll 8
     for (int c = 0; c < decltype(n)::value; c += 4) {
-      const double av = PT[(c + lk) * LD + 16 * tr + li];
+      const double av = PT[(c + lk) * LD + 16 * otr + li];
 #pragma unroll
       for (int k = 0; k < NC; ++k)
-        acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, QT[(c + lk) * LD + 16 * (tc + k) + li], acc[k], 0, 0, 0);
+        acc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, QT[(c + lk) * LD + 16 * (otc + k) + li], acc[k], 0, 0, 0);
     }
 #pragma unroll
     for (int k = 0; k < NC; ++k)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) f(16 * tr + lk + 4 * v, 16 * (tc + k) + li, acc[k][v]);
+      for (int v = 0; v < 4; ++v) f(16 * otr + lk + 4 * v, 16 * (otc + k) + li, acc[k][v]);
   };
   if (plain) {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = 16 * rt + lk + 4 * v;
-        a.B[rows + i * D + c0] = sy.x[rt][0][v];
-        YL[(16 * wave + li) * LD + i] = sy.x[rt][0][v];
-      }
+      for (int u = 0; u < CT; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) a.B[rows + (16 * rt + lk + 4 * v) * D + c0 + 16 * u] = sy.x[rt][u][v];
     __syncthreads();
-    double* out = a.BB + (((int64_t)ws * bh + h) * NP + (c0 >> 6)) * RP * RP;
-    outer(YL, YL, std::integral_constant<int, 64>{}, [&](int i, int j, double v) { out[i * RP + j] = v; });
+    double* out = a.BB + ((int64_t)ws * bh + h) * RP * RP;
+    outer(ML, ML, std::integral_constant<int, D>{}, [&](int i, int j, double v) { out[i * RP + j] = v; });
     return;
   }
   if constexpr (STEP) {
-    if (wave < 2) {
+    if constexpr (!EARLY) s_loads();
+    const bool in_slice = CT * wave / 2 == s;  // this wave's columns of M are the slice's
+    gd_v4d old[RT][CT];                        // there, the other side's C, for the change of its factor
+    if (in_slice) {
       float* mt = (STAGE == kGsQ ? a.Mt_q : a.Mt_k) + (int64_t)h * r * D + c0;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * rt + lk + 4 * v;
-          if (i < r) mt[i * D] = (float)sy.x[rt][0][v];
-          change = fma(-2.0 * old[rt][v], sy.x[rt][0][v], change);
-          WL[(16 * wave + li) * LD + i] = sy.x[rt][0][v];
-        }
-    } else {
+        for (int u = 0; u < CT; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const int i = 16 * rt + lk + 4 * v;
+            old[rt][u][v] = a.C[orows + i * D + c0 + 16 * u];
+            if (i < r) mt[i * D + 16 * u] = (float)sy.x[rt][u][v];
+          }
+    }
+    __syncthreads();
+    // ---- T = M^T S: wave w takes column tile w % 2 of the slice and half of the row tiles
+    gd_v4d t[NR];
+#pragma unroll
+    for (int n = 0; n < NR; ++n) t[n] = gd_v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < D / 4; ++u)
+#pragma unroll
+      for (int n = 0; n < NR; ++n)
+        t[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(ML[(4 * u + lk) * LD + tr + 16 * n + li], sv[u], t[n], 0, 0, 0);
+    if (in_slice) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = 16 * rt + lk + 4 * v;
-          a.C[orows + i * D + c0] = sy.x[rt][0][v];
-          TT[(16 * (wave & 1) + li) * LD + i] = sy.x[rt][0][v];
-        }
+        for (int u = 0; u < CT; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) change = fma(-2.0 * old[rt][u][v], sy.x[rt][u][v], change);
     }
+    __syncthreads();  // (the slice's old C has been read)
+#pragma unroll
+    for (int n = 0; n < NR; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = tr + 16 * n + lk + 4 * v;
+        a.C[orows + i * D + tc] = t[n][v];
+        TT[(16 * (wave & 1) + li) * LD + i] = t[n][v];
+      }
     __syncthreads();
-    outer(WL, TT, std::integral_constant<int, 32>{}, [&](int i, int j, double v) {
+    outer(ML + 32 * s * LD, TT, std::integral_constant<int, 32>{}, [&](int i, int j, double v) {
       Go[i * RP + j] = v;
       if (i == j && i < r) change += v;
     });
@@ -1325,7 +1326,7 @@ template <int RT, int D>
 static int gramslice_run(const GdArgs& a, const float* xq_part, int Sx, const float* xk_part, int Sxk, int bkv, double* Sq,
                          double* Sk, int iters, hipStream_t st) {
   using Sh = GsShape<RT, D>;
-  constexpr int RP = Sh::RP, NS = Sh::NS, NP = Sh::NP;
+  constexpr int RP = Sh::RP, NS = Sh::NS;
   using Fn = void (*)(int, GdArgs);
   constexpr Fn start = pf_gs_kernel<RT, D, kGsStart>, q_side = pf_gs_kernel<RT, D, kGsQ>, k_side = pf_gs_kernel<RT, D, kGsK>,
                last = pf_gs_kernel<RT, D, kGsFinal>;
@@ -1344,12 +1345,12 @@ static int gramslice_run(const GdArgs& a, const float* xq_part, int Sx, const fl
   // head share an XCD, and what they all read comes into its L2 once.
   const unsigned bh = ((unsigned)a.bh + 7) & ~7u;
   const dim3 blk(kGsThreads);
-  if (iters > 0) hipLaunchKernelGGL(start, dim3(bh, NP), blk, Sh::SMEM, st, 0, a);
+  if (iters > 0) hipLaunchKernelGGL(start, dim3(bh, 1), blk, Sh::SMEM, st, 0, a);
   for (int it = 0; it < iters; ++it) {
-    hipLaunchKernelGGL(q_side, dim3(bh, NS + NP), blk, Sh::SMEM, st, it, a);
-    hipLaunchKernelGGL(k_side, dim3(bh, NS + NP), blk, Sh::SMEM, st, it, a);
+    hipLaunchKernelGGL(q_side, dim3(bh, NS + 1), blk, Sh::SMEM, st, it, a);
+    hipLaunchKernelGGL(k_side, dim3(bh, NS + 1), blk, Sh::SMEM, st, it, a);
   }
-  hipLaunchKernelGGL(last, dim3(bh, 2 * NP), blk, Sh::SMEM, st, iters, a);
+  hipLaunchKernelGGL(last, dim3(bh, 2), blk, Sh::SMEM, st, iters, a);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
@@ -1378,13 +1379,14 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
                         : hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
-  // In slices while a launch of an iteration has at most 1.5 workgroups per CU (64 heads at d = 128): 32 heads, four
-  // iterations, the whole fit of 8192 rows 313 -> 253 us at rank 32 and 667 -> 460 at rank 64; 64 heads 294 -> 253 and
-  // 622 -> 547; 96 heads 249 -> 260 and 674 -> 747 (what the slices repeat then costs more than idle CUs do); d = 64: 32
-  // heads 170 -> 148, 96 heads 158 -> 154.  Ranks up to 16: an iteration whole takes 16 .. 24 us, two launches as long.
-  const bool slices = RP > 16 && (int64_t)bh * (d / 32 + d / 64) <= 384;
+  // In slices while a launch of an iteration has few workgroups per CU (96 heads of 128 at ranks to 32, 64 above): four
+  // iterations, the whole fit of 8192 rows of 32 heads 313 -> 258 us at rank 32 and 681 -> 492 at rank 64; 64 heads 295 ->
+  // 271 and 632 -> 606; 96 heads 262 -> 250 and 689 -> 708; 128 heads 359 -> 396 and 760 -> 1000 (what the slices repeat
+  // then costs more than idle CUs do); d = 64: 32 heads 170 -> 145, 96 heads 156 -> 151.  Ranks up to 16: an iteration
+  // whole takes 16 .. 24 us, two launches as long.
+  const bool slices = RP > 16 && (int64_t)bh * (d / 32 + 1) <= (RP == 32 ? 480 : 320);
   const size_t g_parts = slices ? d / 32 : 1;
-  const size_t n_state = slices ? (size_t)bh * 2 * (RP * d + d / 64 * RP * RP)
+  const size_t n_state = slices ? (size_t)bh * 2 * (RP * d + RP * RP)
                                 : (size_t)bh * RP * d + (RP == 64 ? (size_t)bh * 2 * RP * (RP + 1) : 0);
   const size_t n_delta = (size_t)std::max(iters, 1) * 2 * bh * g_parts;
   const size_t bytes = ((size_t)bh + bkv) * dd * 8 + (size_t)2 * bh * RP * (g_parts * RP + d) * 8 + (n_state + n_delta) * 8 +
@@ -1408,7 +1410,7 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   a.C = (double*)take((size_t)2 * bh * RP * d * 8);
   if (slices) {
     a.B = (double*)take((size_t)2 * bh * RP * d * 8);
-    a.BB = (double*)take((size_t)2 * bh * (d / 64) * RP * RP * 8);
+    a.BB = (double*)take((size_t)2 * bh * RP * RP * 8);
   } else {
     a.BqT = (double*)take((size_t)bh * RP * d * 8);
     if (RP == 64) a.Gs = (double*)take((size_t)bh * 2 * RP * (RP + 1) * 8);
