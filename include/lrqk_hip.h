@@ -162,6 +162,13 @@ int lrqk_ctx_score_index(lrqk_ctx* ctx, int enable);
  * contents before the ctx is used for another prompt.  0 switches it off.  Memory: bh *
  * rows_per_head rows of 2*d elements plus 2 bytes per (head, store row). */
 int lrqk_ctx_victim_cache(lrqk_ctx* ctx, int rows_per_head);
+/* After lrqk_score_select over a prompt of l tokens, with the victim cache of ctx empty: puts the K and V rows of the
+ * tokens that come next in the selection's order (about topk / 2 per head) into the cache, from the prompt's k, v
+ * ([b][hkv][l][d] on the device); the first steps then find most of the tokens that enter the active set there.
+ * cap: rows of the store that lrqk_decode_step will be given (another one empties the cache).  Does nothing where that
+ * selection is not the ctx's last one or the step would not use the cache. */
+int lrqk_victim_fill(lrqk_ctx* ctx, const void* k, const void* v, int64_t l, int64_t cap, int b, int hq, int hkv, int d,
+                     int dtype, void* stream);
 /* Rows that lrqk_decode_step fetched over the host link since the last reset (the other missed
  * rows came from the victim cache).  Synchronises.  Counts only while the victim cache is on. */
 int lrqk_victim_stats(lrqk_ctx* ctx, int64_t* host_rows, int reset);

@@ -143,6 +143,10 @@ struct lrqk_ctx {
   int vic_req = 0;          // FIFO rows per head asked for
   int vic_bh = 0, vic_chunks = 0;
   bool vic_dirty = true;    // (re)initialise before the next use
+  // tokens of rank k .. 1.5 k of the last selection over a prompt, for the victim cache: i32 [bh][next_cap], i32 [bh] counts
+  lrqk::DevBuf next_ids;
+  int next_bh = 0, next_cap = 0;
+  bool next_valid = false;  // listed, and not used yet
   // staged miss fetch: pinned host staging, its device twin, side stream and event (created on first use)
   lrqk::DevBuf stage_dev;
   void* stage_host = nullptr;
@@ -163,7 +167,7 @@ struct lrqk_ctx {
   void each_buf(F&& f) {
     for (lrqk::DevBuf* b : {&keys, &hist, &cand, &cand_cnt, &attn_part, &als_part, &als_kq, &als_pre, &als_iter, &als_iter64,
                             &fstate, &evk, &prefill_ws, &prefill_gd, &new_idx, &misc, &sidx_qa, &sidx_qs, &sidx_wm,
-                            &sidx_part, &vic_rows, &vic_meta, &stage_dev})
+                            &sidx_part, &vic_rows, &vic_meta, &next_ids, &stage_dev})
       f(*b);
   }
   int scan_wgs = 0;        // workgroups of the last scan through the score index (0: the last scan read A_K itself)

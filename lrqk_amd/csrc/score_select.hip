@@ -168,6 +168,10 @@ struct SelState {
   int* stats;
   int* rescored;     // per workgroup of the last index scan: rows whose bound passed (rescored exactly)
   int rescored_cap;
+  // A prompt's selection also lists the tokens of rank k .. 1.5 k (any order), for the victim cache; null: not asked for.
+  int32_t* next_ids;  // [bh][next_cap]
+  int* next_cnt;      // [bh]
+  int next_cap;
 };
 
 __global__ void init_select_state_kernel(SelState st, int bh) {
@@ -938,9 +942,11 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
       need_eq = need3;
     }
   }
-  const uint32_t Tk = lo + (offT << tz);
+  const uint32_t Tk = lo + (offT << tz), Tlow = lo + (offE << tz);
+  __shared__ int s_next;
   if (tid == 0) {
-    st.t_low[h] = lo + (offE << tz);  // rank >= 1.5k (rounded down to the resolved bits)
+    s_next = 0;
+    st.t_low[h] = Tlow;  // rank >= 1.5k (rounded down to the resolved bits)
     st.q_norm[h] = mode == 0 ? st.q_cur[h] : 0.0f;
   }
 
@@ -966,8 +972,13 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
     for_each([&](uint32_t key, int64_t idx) {
       const int64_t rel = idx - c0;
       if (key >= Tk && rel >= 0 && rel < span) atomicOr(key > Tk ? &gt[rel >> 5] : &eq[rel >> 5], 1u << (rel & 31));
+      if (st.next_ids && c0 == 0 && key < Tk && key >= Tlow) {
+        const int p = atomicAdd(&s_next, 1);
+        if (p < st.next_cap) st.next_ids[(int64_t)h * st.next_cap + p] = (int32_t)idx;
+      }
     });
     __syncthreads();
+    if (st.next_ids && c0 == 0 && tid == 0) st.next_cnt[h] = min(s_next, st.next_cap);
     const int w0 = tid * W;
     uint32_t gwr[kWordsPT], ewr[kWordsPT];
 #pragma unroll
@@ -1594,6 +1605,9 @@ static int prepare_select(lrqk_ctx* ctx, int bh, int64_t m, int topk, hipStream_
   sb->st.stats = (int*)(base + 6 * bh);
   sb->st.rescored = (int*)(base + 6 * bh + 3);
   sb->st.rescored_cap = bh + kRescSlots;
+  sb->st.next_ids = nullptr;
+  sb->st.next_cnt = nullptr;
+  sb->st.next_cap = 0;
   if (before != ctx->cand_cnt.p || ctx->sel_bh != bh) {
     hipLaunchKernelGGL(init_select_state_kernel, dim3((unsigned)((bh + 255) / 256)), dim3(256), 0, st, sb->st, bh);
     LRQK_HIP_CHECK(hipGetLastError());
@@ -1802,6 +1816,17 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
   if (m <= topk) return arange_result(bh, m, out_idx, out_stride, st);
   SelectBufs sb;
   if ((rc = prepare_select(ctx, bh, m, topk, st, &sb))) return rc;
+  // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it
+  ctx->next_valid = false;
+  if (ctx->vic_req > 0 && ctx->vic_dirty) {
+    const int cap = std::min(topk, ctx->vic_req);
+    if ((rc = ctx->next_ids.ensure((size_t)bh * (cap + 1) * sizeof(int32_t)))) return rc;
+    sb.st.next_ids = (int32_t*)ctx->next_ids.p;
+    sb.st.next_cnt = sb.st.next_ids + (size_t)bh * cap;
+    sb.st.next_cap = ctx->next_cap = cap;
+    ctx->next_bh = bh;
+    ctx->next_valid = true;
+  }
   DiffArgs df{nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0};
   if (dtype == LRQK_F32)
     rc = dispatch_filter_select<float>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, 0, topk, out_idx, out_stride, df, st);

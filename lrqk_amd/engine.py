@@ -36,6 +36,8 @@ def _copy_stream(device: torch.device) -> torch.cuda.Stream:
 
 class LightAttentionIndicesFactory:
     no_hit_miss = False
+    # a prompt's next best tokens go into the victim cache, where the first steps look for what they miss
+    fill_victims = True
 
     def __init__(self, num_lite_tokens: int = 1, attn_topk: int = 128, num_key_value_groups: int = 1, r: int = 16,
                  max_iter: Union[int, Tuple[int, int]] = 2, tol: Union[float, Tuple[float, float]] = 1e-4,
@@ -304,6 +306,8 @@ class LightAttentionIndicesFactory:
                 ops.score_select(self.ws, self._A_K.data, A_Q, lb, k, self.round_scores_to_storage, out=self._active_idx)
                 self._hit_len = k
                 ops.fill_active(key_states, value_states, self._active_idx, self.Kgpu, self.Vgpu, k)
+                if self.fill_victims and not self.no_hit_miss and self._fetch_mode == "direct" and key_states.is_cuda:
+                    ops.victim_fill(self.ws, key_states, value_states, self.Kgpu.shape[1], self.KVcpu.data.shape[2])
             else:
                 hit = self.compute_hit_indices(query_states=A_Q, key_states=self._A_K.data.narrow(2, 0, lb))
                 self._hit_len = hit.shape[2]
@@ -521,6 +525,7 @@ class LightAttentionIndicesOffloadPrefill(LightAttentionIndicesFactory):
     """Between a layer's prefill and its first decode, park the active set and the key
     factors in pinned host memory (lrqk_attention.py:1616-1680).  The copies run on a side
     stream and are ordered by events in both directions."""
+    fill_victims = False   # (device memory that the first decode takes)
 
     def prefill(self, query_states, key_states, value_states):
         super().prefill(query_states, key_states, value_states)

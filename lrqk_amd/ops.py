@@ -318,6 +318,15 @@ def fill_active(k: torch.Tensor, v: torch.Tensor, active_idx: torch.Tensor, k_ac
                                        v_act.data_ptr(), topk, n - topk, b, hq, hkv, d, _dt(k), _stream(k)))
 
 
+def victim_fill(ws: Workspace, k: torch.Tensor, v: torch.Tensor, hq: int, capacity: int):
+    """The rows of k, v [b,Hkv,l,d] of the tokens that the last ``score_select`` of ``ws`` left out by the least go into its
+    empty victim cache; ``capacity``: rows of the host store of the steps to come."""
+    _need_cuda(k, v)
+    b, hkv, l, d = k.shape
+    assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape and k.dtype == v.dtype
+    check(_lib.load().lrqk_victim_fill(ws.handle, k.data_ptr(), v.data_ptr(), l, capacity, b, hq, hkv, d, _dt(k), _stream(k)))
+
+
 def append_token(k_new, v_new, k_act, v_act, slot: int, active_idx: Optional[torch.Tensor], token: int):
     _need_cuda(k_new, v_new, k_act, v_act)
     b, hkv = k_new.shape[:2]
