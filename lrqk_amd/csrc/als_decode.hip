@@ -522,26 +522,34 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
     const float* c0 = cred + (wave ? 0 : 2048);
     const float gsel = wave ? 1.0f : 0.0f;
     auto elem = [&](int i, int j) { return fmaf(gsel, G[i * 32 + j], c0[i * 32 + j] + c0[1024 + i * 32 + j]); };
-    invert_sweep_mfma(elem, r, Mx + 32 * wave, wave ? GQi : GKi);
+    float* const inv = wave ? GQi : GKi;
+    if (r & 1)  // (uniform)
+      invert_sweep_mfma<32, true>(elem, r, Mx + 32 * wave, inv);
+    else if (r <= 16)
+      invert_sweep_mfma<16, false>(elem, r, Mx + 32 * wave, inv);
+    else
+      invert_sweep_mfma<32, false>(elem, r, Mx + 32 * wave, inv);
   }
   __syncthreads();
   // ---- k_hat_0 and the alternating rank-1 solves, all inside the first wave: lane c (and c + 32)
   // holds column c of both inverses and element c of every vector; a vector element is
   // broadcast with readlane, so the chain of small solves needs no barrier and no LDS round trip.
-  if (wave == 0) {
+  // (N: the elements that can differ from zero, 16 or 32)
+  auto iterate = [&](auto n_c) {
+    constexpr int N = decltype(n_c)::value;
     const int c = lane & 31;
-    float cK[32], cQ[32];
+    float cK[N], cQ[N];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
+    for (int i = 0; i < N; ++i) {
       cK[i] = GKi[i * kLdi + c];
       cQ[i] = GQi[i * kLdi + c];
     }
     const float rq = rhs_q[c], kb = kB[c], sqk = s_qk;
     // y_c = sum_i b_i col[i]  (b lane-distributed)
-    auto vecmat = [&](float bvec, const float (&col)[32]) {
+    auto vecmat = [&](float bvec, const float (&col)[N]) {
       float y0 = 0.0f, y1 = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 32; i += 2) {
+      for (int i = 0; i < N; i += 2) {
         y0 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i)), col[i], y0);
         y1 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i + 1)), col[i + 1], y1);
       }
@@ -551,7 +559,7 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
     // x = b (G + v^T v)^-1 from G^-1 (Sherman-Morrison): x = y - (y.v / (1 + z.v)) z, y = b G^-1, z = v G^-1.
     // Both right-hand sides have the form b = b0 + s v, so y = b0 G^-1 + s z: b0 G^-1 is formed once
     // (for the k side it is k_hat_0 itself) and every solve costs one vector-matrix product.
-    auto rank1 = [&](float y0, float v, const float (&col)[32]) {
+    auto rank1 = [&](float y0, float v, const float (&col)[N]) {
       const float z = vecmat(v, col);
       const float y = fmaf(sqk, z, y0);
       const float alpha = dot32(y, v) / (1.0f + dot32(z, v));
@@ -573,7 +581,12 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
       }
       hk = nk;
     }
-  }
+  };
+  if (wave != 0) return;
+  if (r <= 16)  // (uniform)
+    iterate(std::integral_constant<int, 16>{});
+  else
+    iterate(std::integral_constant<int, 32>{});
 }
 
 // ----------------------------------------------------------------------------- ranks beyond one matrix-core tile

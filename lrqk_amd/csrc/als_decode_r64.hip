@@ -243,7 +243,9 @@ constexpr int kS64Ld = 65;  // row stride of a 64 x 64 matrix in LDS
 // the sweeps on p and p + 1 as the two k elements of one rank-2 MFMA update, the 2 that every sweep leaves on its
 // diagonal entry taken off at the end -- on the accumulators of 2 x 2 tiles: row p (and p + 1) of both column
 // blocks makes the operands, A_i = B_i / d for the rows of either block.  Rows and columns >= r form an identity
-// block.  sbuf: 64 floats.
+// block, whose pivots change nothing: PIVOTS (48 or 64, at least r) are swept without a test.  (Behind a test per pair the
+// compiler copies all 64 accumulators per pair: the solve 26.2 -> 24.9 us.)  sbuf: 64 floats.
+template <int PIVOTS>
 __device__ __forceinline__ void invert64_sweep_mfma(float* G, int r, float* sbuf) {
   const int lane = lane_id();
   const int col = lane & 31, half = lane >> 5;
@@ -278,8 +280,8 @@ __device__ __forceinline__ void invert64_sweep_mfma(float* G, int r, float* sbuf
   // branches; the matrix is finite, so a product with a weight of 0 is 0)
   const float in0 = half == 0 ? 1.0f : 0.0f, in1 = 1.0f - in0;
 #pragma unroll
-  for (int p = 0; p < 64; p += 2) {
-    if (p < r) {  // (wave-uniform)
+  for (int p = 0; p < PIVOTS; p += 2) {
+    {
       const int P = p >> 5, pl = p & 31;
       const int v = ((pl >> 3) << 2) + (pl & 3), hp = (pl >> 2) & 1;  // rows p, p + 1: elements v, v + 1 of half hp
       const float r0P = acc[P][P][v], r1P = acc[P][P][v + 1];
@@ -481,8 +483,12 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   if (tid < 64) rhs_s[tid] += tid < r ? aw_s[tid] : 0.0f;
   __syncthreads();
   // ---- both inverses, side by side
-  if (wave == 0) invert64_sweep_mfma(GQ, r, sbuf[0]);
-  if (wave == 1) invert64_sweep_mfma(GK, r, sbuf[1]);
+  if (wave < 2) {
+    if (r <= 48)  // (uniform)
+      invert64_sweep_mfma<48>(wave ? GK : GQ, r, sbuf[wave]);
+    else
+      invert64_sweep_mfma<64>(wave ? GK : GQ, r, sbuf[wave]);
+  }
   __syncthreads();
   if (wave != 0) return;
   // ---- the alternating iterations, lane c <-> element c of every vector (zeros beyond r)

@@ -558,7 +558,12 @@ def _als_inputs(g, b, hq, hkv, n, d, r, cap, dtype):
                                                 (torch.bfloat16, 4, 4, 333, 128, 40),
                                                 # ... an odd one (A_K rows one element at a time), 56, 64 in fp32
                                                 (torch.float32, 2, 1, 100, 64, 33), (torch.bfloat16, 2, 2, 150, 128, 56),
-                                                (torch.float32, 4, 2, 272, 128, 64)])
+                                                (torch.float32, 4, 2, 272, 128, 64),
+                                                # the last even and the odd rank of 16-pivot sweeps, and the ranks past it;
+                                                # 48 (the last of 48-pivot sweeps)
+                                                (torch.float32, 2, 1, 90, 64, 2), (torch.float32, 2, 1, 150, 64, 15),
+                                                (torch.float32, 2, 1, 150, 64, 18), (torch.float32, 2, 1, 150, 64, 31),
+                                                (torch.bfloat16, 2, 2, 200, 128, 48)])
 @pytest.mark.parametrize("max_iter,tol", [(1, 0.0), (2, 0.0), (3, 1e30), (4, 1e-6)])
 def test_als_decode(ops, ws, oracle, dtype, hq, hkv, n, d, r, max_iter, tol):
     _check_als_decode(ops, ws, oracle, dtype, hq, hkv, n, d, r, max_iter, tol)
