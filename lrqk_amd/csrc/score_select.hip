@@ -1813,19 +1813,24 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
   LRQK_REQUIRE(r > 0 && r <= LRQK_MAX_R, LRQK_EINVAL, "r=%d", r);
   LRQK_REQUIRE(head_stride >= m * r, LRQK_EINVAL, "head_stride=%lld < m*r", (long long)head_stride);
   hipStream_t st = (hipStream_t)stream;
+  ctx->next_valid = false;
   if (m <= topk) return arange_result(bh, m, out_idx, out_stride, st);
   SelectBufs sb;
   if ((rc = prepare_select(ctx, bh, m, topk, st, &sb))) return rc;
-  // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it
-  ctx->next_valid = false;
+  // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it (without memory for
+  // the list, or in a capture that would have to take it, there is none)
   if (ctx->vic_req > 0 && ctx->vic_dirty) {
     const int cap = std::min(topk, ctx->vic_req);
-    if ((rc = ctx->next_ids.ensure((size_t)bh * (cap + 1) * sizeof(int32_t)))) return rc;
-    sb.st.next_ids = (int32_t*)ctx->next_ids.p;
-    sb.st.next_cnt = sb.st.next_ids + (size_t)bh * cap;
-    sb.st.next_cap = ctx->next_cap = cap;
-    ctx->next_bh = bh;
-    ctx->next_valid = true;
+    const size_t need = (size_t)bh * (cap + 1) * sizeof(int32_t);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (need > ctx->next_ids.bytes) LRQK_HIP_CHECK(hipStreamIsCapturing(st, &capturing));
+    if (capturing == hipStreamCaptureStatusNone && ctx->next_ids.ensure(need) == LRQK_OK) {
+      sb.st.next_ids = (int32_t*)ctx->next_ids.p;
+      sb.st.next_cnt = sb.st.next_ids + (size_t)bh * cap;
+      sb.st.next_cap = ctx->next_cap = cap;
+      ctx->next_bh = bh;
+      ctx->next_valid = true;
+    }
   }
   DiffArgs df{nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0};
   if (dtype == LRQK_F32)

@@ -390,6 +390,41 @@ def test_active_set_of_a_prompt(ops, dtype, hq, hkv, d, l, k, lite):
     assert torch.equal(Va, torch.gather(V.repeat_interleave(g, 1), 2, rows))
 
 
+@pytest.mark.parametrize("dtype,batch,hq,hkv,d,l,k,rows", [
+    (torch.bfloat16, 1, 4, 2, 64, 1500, 100, 128), (torch.float32, 2, 6, 3, 128, 901, 64, 7), (torch.float32, 1, 2, 2, 8, 700, 33, 1),
+    (torch.float32, 1, 4, 1, 256, 600, 64, 96),     # (rows wider than the cache takes: it stays empty)
+    (torch.bfloat16, 1, 4, 4, 128, 80, 64, 96)])    # (fewer tokens left over than the cache has rows)
+def test_cache_filled_by_the_prompt_is_invisible(ops, dtype, batch, hq, hkv, d, l, k, rows):
+    """The next best tokens of a prompt in the victim cache change where a missed row comes from and nothing else; and rows
+    do come from it."""
+    from lrqk_amd.engine import LightAttentionIndicesFactory as Engine
+    gen = torch.Generator(device=DEV).manual_seed(l)
+
+    def draw(heads, n):
+        return torch.randn((batch, heads, n, d), generator=gen, device=DEV).to(dtype)
+    engines = []
+    for fill in (False, True):
+        eng = Engine(num_lite_tokens=8, attn_topk=k, num_key_value_groups=hq // hkv, r=8, max_iter=2, tol=0.0, capacity=l + 64)
+        eng.fill_victims, eng.victim_rows, eng.attn_in_step = fill, rows, True
+        engines.append(eng)
+    q, kk, vv = draw(hq, l), draw(hkv, l), draw(hkv, l)
+    start = tuple(torch.randn((batch, hq, l, 8), generator=gen, device=DEV) for _ in range(2))
+    for eng in engines:
+        eng.init_factors = tuple(x.clone() for x in start)
+        eng.prefill(q, kk, vv)
+        eng.ws.victim_stats(reset=True)
+    a, b = engines
+    for step in range(12):   # (a flush of the ring among them)
+        t = q[:, :, -1:] + 0.1 * draw(hq, 1), draw(hkv, 1), draw(hkv, 1)   # (near the prompt's last query)
+        for eng in engines:
+            eng.decode(*t)
+        assert torch.equal(a._active_idx, b._active_idx) and torch.equal(a.last_attn, b.last_attn), step
+        assert torch.equal(a.Kgpu, b.Kgpu) and torch.equal(a.Vgpu, b.Vgpu), step
+    without, filled = (eng.ws.victim_stats() for eng in engines)
+    print(f"rows over the host link: {without} without, {filled} with", flush=True)
+    assert filled < without or d == 256 or rows < 96   # (a few rows are replaced before they are asked for)
+
+
 @pytest.mark.parametrize("batch,hkv,l", [(1, 1, 300), (2, 3, 517), (1, 16, 1031)])
 def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
     """A prompt whose first heads go ahead of the others (one head: a single copy; 6 and 16: pieces of 1 + 5, 2 + 14) is
