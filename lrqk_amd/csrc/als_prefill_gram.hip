@@ -406,13 +406,12 @@ static int apply_shared(const void* k, const float* mt_k, OUT* a_k, int64_t a_st
 // ----------------------------------------------------------------------------- d x d algebra, fp64
 // Everything below is templated on RT, the number of 16-row tiles that the rank is padded to (ranks up to 16, 32, 64:
 // RT = 1, 2, 4), and on the row width D (64 or 128); RP = 16 RT is the padded rank.  Padding costs the matrix cores'
-// time (a solve has RP / 4 dependent steps), so a rank of 16 does not run as 32 (24 against 42 us per
-// iteration at D = 128, 32 heads; RT = 4: 109 us).
-// Eight waves, two per SIMD: waves 0 .. 3 hold one system of a pair, waves 4 .. 7 the other (D / 4 right-hand columns
-// each).  A product occupies the matrix pipe for 64 cycles and a wave issues in order, so with both systems in one of
-// four waves the next pivot block waited behind the products of the step before; now the other wave of the SIMD works
-// meanwhile.  D = 128, 32 heads, four waves -> eight: the final pair alone 18.0 -> 12.4 us at RT = 2, 47.6 -> 33.0 at
-// RT = 4; an iteration 28 -> 24 us at RT = 1, 49 -> 42 at RT = 2, 133 -> 109 at RT = 4.
+// time (a solve has RP / 4 dependent steps of 800 to 1450 cycles, see gd_solve), so a rank of 16 does not run as 32.
+// One workgroup per head takes ranks up to 16, and heads enough to fill the CUs by themselves; the others go in slices
+// (pf_gs_kernel below).  Eight waves, two per SIMD: waves 0 .. 3 hold one system of a pair, waves 4 .. 7 the other (D / 4
+// right-hand columns each), so that a wave waiting for its pivot block leaves the matrix cores to the other.  Against four
+// waves with both systems (D = 128, 32 heads, elimination without products a step behind): the final pair 18.0 -> 12.4 us at
+// RT = 2, 47.6 -> 33.0 at RT = 4; an iteration 28 -> 24 us at RT = 1, 49 -> 42 at RT = 2, 133 -> 109 at RT = 4.
 constexpr int kGdThreads = 512;
 template <int RT, int D>
 struct GdShape {
