@@ -363,7 +363,7 @@ constexpr int scan_waves(int r) { return r == 64 ? 3 : r == 32 ? 4 : 5; }
 template <typename T, int R>
 __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_kernel(
     const T* __restrict__ a_k, int64_t head_stride, const T* __restrict__ q_hat, int64_t m, int r, int round_bf16,
-    SelState st, uint2* __restrict__ cand, int cand_cap, FilterQ fq, ScoreIndexView six) {
+    SelState st, uint2* __restrict__ cand, int cand_cap, FilterQ fq, ScoreIndexView six, bool heads_first) {
   static_assert(R == 16 || R == 32 || R == 64, "the score index covers ranks 16, 32, 64");
   constexpr int QV = R / 16;                  // lanes per row
   constexpr int kRowsPerLoad = kWave / QV;    // rows that one load of a wave covers
@@ -378,7 +378,9 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
   __shared__ __align__(16) float qx_s[kShare ? 1 : kScanWaves][R];  // the proxy query as the exact score uses it
   __shared__ __align__(16) float qp_s[R];                          // q'
   __shared__ int resc_s;
-  const int h = blockIdx.x;
+  // (the grid's order is the host's choice)
+  const int h = heads_first ? blockIdx.x : blockIdx.y;
+  const int wg = heads_first ? blockIdx.y : blockIdx.x, n_wgs = heads_first ? gridDim.y : gridDim.x;
   const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
   const T* A = a_k + (int64_t)h * head_stride;
   const uint8_t* QA = six.qa + (int64_t)h * six.head_rows * R;
@@ -388,8 +390,8 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
   const int sub = lane % QV;        // which 16 bytes of its row this lane reads
   const int lrow = lane / QV;       // row of this lane within a load
   const int64_t n_steps = (m + kStepRows - 1) / kStepRows;
-  const int64_t s_stride = (int64_t)gridDim.y * kScanWaves;
-  int64_t s_cur = (int64_t)blockIdx.y * kScanWaves + w;
+  const int64_t s_stride = (int64_t)n_wgs * kScanWaves;
+  int64_t s_cur = (int64_t)wg * kScanWaves + w;
   const bool has_work = s_cur < n_steps;  // (wave-uniform)
 
   u32x4_t buf[2][kScanU];
@@ -441,7 +443,7 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
       float qv = oit[0];
 #pragma unroll
       for (int it = 1; it < kFiltMaxIt; ++it) qv = chosen == it ? oit[it] : qv;
-      if (blockIdx.y == 0 && tid < r) st_f32<T>((T*)fq.q_hat_out, (int64_t)h * r + tid, qv);
+      if (wg == 0 && tid < r) st_f32<T>((T*)fq.q_hat_out, (int64_t)h * r + tid, qv);
       q_lane = sizeof(T) == 2 ? round_to_bf16_f32(qv) : qv;
     }
     if (lane < R) qx_s[kShare ? 0 : w][lane] = lane < r ? q_lane : 0.0f;
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
   ql2 = group_sum(ql2, QV);
   const float qn = sqrtf(ql2);
   const uint32_t tl = rescaled_bound(t_prev, qn_prev, qn, round_bf16);
-  if (tid == 0 && blockIdx.y == 0) {
+  if (tid == 0 && wg == 0) {
     st.t_used[h] = tl;
     st.q_cur[h] = qn;
   }
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
   }
   __syncthreads();
   if (tid == 0) {
-    const int slot = h * (int)gridDim.y + (int)blockIdx.y;
+    const int slot = h * n_wgs + wg;
     if (slot < st.rescored_cap) st.rescored[slot] = resc_s;
   }
 }
@@ -1511,6 +1513,7 @@ __global__ __launch_bounds__(kSelThreads) void select_step_kernel(const uint2* _
                                                                   int32_t* __restrict__ out_all, int64_t out_stride,
                                                                   DiffArgs df) {
   LRQK_SEL_LDS(L);
+  st.next_ids = nullptr;  // (a prompt's selection only)
   const int h = blockIdx.x;
   const int n = __builtin_amdgcn_readfirstlane(st.cand_count[h * kCountStride]);
   const int lvl = __builtin_amdgcn_readfirstlane(st.level[h]);
@@ -1690,12 +1693,16 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
       constexpr int kStepRowsWg = (kWave / (R / 16)) * kScanU * kScanWaves;  // rows one step of a workgroup's waves covers
       const int64_t need = (m + kStepRowsWg - 1) / kStepRowsWg;
       const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(need, slots / bh));
-      // The heads in a row: workgroups go round the XCDs in the order of their index, so a head's workgroups (eight
-      // heads and more, a multiple of 8 of them) share an XCD, its list counter and what they read of its state.  32 heads:
-      // 14.7 -> 14.2 us at 32K rows, 28.7 -> 27.9 at 128K (the step's other launches: no faster, the fetch slower by 1 .. 12 us).
-      const dim3 grid_st((unsigned)bh, (unsigned)wgs);
+      // Up to 32 heads of 32K rows and more stand in a row: workgroups go round the XCDs in the order of their index, so a
+      // head's workgroups (eight heads and more, a multiple of 8 of them) share an XCD, its list counter and what they read
+      // of its state.  At 128K rows (a head after the other -> in a row) 8 heads 18.9 -> 17.1 us, 16 heads 20.1 -> 18.9, 28 and
+      // 32 heads 0.5 less; 24 the same.  Beyond 32 heads neighbouring workgroups should read neighbouring rows: 64 heads a step of
+      // 129 us in 136, 256 heads the scan 219 -> 229.  At 8K rows 0.3 us more.  (The step's other launches: no faster with the
+      // heads in a row, the fetch slower by 1 .. 12 us.)
+      const bool heads_first = bh <= 32 && m >= 32768;
+      const dim3 grid_st((unsigned)(heads_first ? bh : wgs), (unsigned)(heads_first ? wgs : bh));
       hipLaunchKernelGGL((score_prefilter_kernel<T, R>), grid_st, dim3(kFiltThreads), 0, st, (const T*)a_k,
-                         head_stride, (const T*)q_hat, m, r, round_bf16, sb.st, sb.cand, sb.cand_cap, fq, six);
+                         head_stride, (const T*)q_hat, m, r, round_bf16, sb.st, sb.cand, sb.cand_cap, fq, six, heads_first);
       via_index = true;
       ctx->scan_wgs = (int)std::min<int64_t>(wgs * bh, sb.st.rescored_cap);
       ctx->scan_rows = (int64_t)bh * m;
