@@ -27,6 +27,7 @@
 
 namespace lrqk {
 
+typedef __bf16 gram_bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kGramThreads = 256;
 constexpr int kGramWaves = kGramThreads / kWave;
 constexpr int kGramChunk = 32;  // tokens per wave per chunk = 16 MFMA steps
@@ -35,7 +36,7 @@ constexpr int kSolveThreads = 256;
 
 
 // Everything the solve needs from B_Q, B_K, q and the new k -- B_Q B_Q^T and B_K B_K^T (four 32 x 32
-// tiles: matrix x two addends), q B_Q^T, k B_K^T and q . k -- does not depend on the Gram
+// tiles: matrix x half of the d axis), q B_Q^T, k B_K^T and q . k -- does not depend on the Gram
 // pass over the active rows, so two more workgroups per head of that launch form it beside them.
 // out (kPreNe floats per head): tiles [4][1024] | q B_Q^T [32] | k B_K^T [32] | q . k.
 constexpr int kPreNe = 4 * 1024 + 32 + 32 + 1;
@@ -44,8 +45,8 @@ __device__ __forceinline__ void als_bgram_body(const T* __restrict__ b_q, const 
                                                const T* __restrict__ q, const T* __restrict__ k_new, int h, int hq,
                                                int hkv, int r, int d, int vshift, float* __restrict__ out,
                                                float* __restrict__ sm, int which) {
-  // Two workgroups per head, one per matrix (which = 0: B_Q with q, 1: B_K with k): B B^T (bf16: a tile per wave; fp32:
-  // waves 0 and 1 a half-sum each), waves 2 and 3 the 32 products with the vector, wave 0 of the first also q . k.
+  // Two workgroups per head, one per matrix (which = 0: B_Q with q, 1: B_K with k): waves 0 and 1 form the
+  // two half-sums of B B^T, waves 2 and 3 the 32 products with the vector, wave 0 of the first also q . k.
   constexpr int VEC = Vec16<T>::N;
   constexpr int kMaxVec = 8;  // 16-byte vectors per thread: r * d / VEC <= 2048
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
@@ -86,47 +87,44 @@ __device__ __forceinline__ void als_bgram_body(const T* __restrict__ b_q, const 
     }
   }
   __syncthreads();
-  if constexpr (sizeof(T) == 2) {
-    // bf16: B B^T on the fp64 matrix cores, a 16 x 16 tile per wave, left as two addends (the value rounded to fp32, and the
-    // rest).  k_hat solves with B_K B_K^T, whose condition multiplies the error of these sums; rows rounded to bf16 make it
-    // 1e5 and more on prompts of rank r, and as fp32 chains over d / 2 the sums were most of what k_hat was off by (a prompt
-    // of 32K rank-32 rows at r 32, 24 steps: 15 steps more than 5e-3 from fp64, 3 now).  In time it is a draw: as many
-    // cycles of the matrix cores per wave, beside the pass over the rows (a token at 32K: 60.3 us either way).
-    static_assert(kGramThreads == 4 * kWave, "a tile per wave");
-    const int li = lane & 15, lk = lane >> 4;
-    const int ti = 16 * (wave >> 1), tj = 16 * (wave & 1);
-    const float* Pi = B + (ti + li) * ld + lk;
-    const float* Pj = B + (tj + li) * ld + lk;
-    v4d acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 8
-    for (int kk = 0; kk < d; kk += 4)  // d >= 8 is a power of two
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)Pi[kk], (double)Pj[kk], acc, 0, 0, 0);
-    float* mine = out + which * 2 * 1024;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int e = (ti + lk + 4 * v) * 32 + tj + li;
-      const float hi = (float)acc[v];
-      mine[e] = hi;
-      mine[1024 + e] = (float)(acc[v] - (double)hi);
-    }
-  }
   if (wave < 2) {
-    if constexpr (sizeof(T) != 2) {
-      // B B^T on the matrix cores: wave -> half of the d axis
-      const int col = lane & 31, khalf = lane >> 5;
-      const int half = wave;
-      const float* Bp = B + col * ld + khalf;
-      v16f acc;
+    // B B^T on the matrix cores: wave -> half of the d axis
+    const int col = lane & 31, khalf = lane >> 5;
+    const int half = wave;
+    v16f acc;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    if (sizeof(T) == 2 && d >= 32) {
+      // bf16: 16 elements of d per product, each in a fresh accumulator and added in fp32.  k_hat solves with B_K B_K^T, whose
+      // condition multiplies the error of these sums (1e5 and more on prompts of rank r): as fp32 chains over d / 2 they
+      // were most of what k_hat was off by: on a prompt of 32K rank-32 rows at r 32 more than 5e-3 in 15 of 24 steps, now in 2
+      // (sums in fp64: 3).  A token takes as long as with either.
+      const float* Bp = B + col * ld + half * (d / 2) + 8 * khalf;
+#pragma unroll 4
+      for (int c = 0; c < d / 2; c += 16) {
+        uint32_t u[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) u[e] = __float_as_uint(Bp[c + e]);
+        const gram_bf16x8 op = __builtin_bit_cast(
+            gram_bf16x8, make_uint4((u[0] >> 16) | (u[1] & 0xffff0000u), (u[2] >> 16) | (u[3] & 0xffff0000u),
+                                    (u[4] >> 16) | (u[5] & 0xffff0000u), (u[6] >> 16) | (u[7] & 0xffff0000u)));
+        v16f t;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op, op, t, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] += t[v];
+      }
+    } else {
+      const float* Bp = B + col * ld + khalf;
       const int k1 = (half + 1) * (d / 2);
 #pragma unroll 8
       for (int kk = half * (d / 2); kk < k1; kk += 2)  // d >= 8 is a power of two
         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(Bp[kk], Bp[kk], acc, 0, 0, 0);
-      float* mine = out + (which * 2 + half) * 1024;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) mine[mfma_row(lane, v) * 32 + col] = acc[v];
     }
+    float* mine = out + (which * 2 + half) * 1024;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) mine[mfma_row(lane, v) * 32 + col] = acc[v];
     if (which == 0 && wave == 0) {
       float v = 0.0f;
       for (int c = lane; c < d; c += kWave) v = fmaf(vec[c], oth[c], v);
@@ -286,7 +284,6 @@ __global__ __launch_bounds__(kGramThreads) void als_gram_kernel(const T* __restr
 // cost); a wave walks its rows chunk by chunk with the next chunk's K and A rows and the ids of the chunk after
 // it already requested, and no workgroup barrier inside the loop; all LDS is one static block shared by the
 // roles, so the launch is bounded by registers (4 workgroups per CU), not by the extra workgroups' B tile.
-typedef __bf16 gram_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 gram_bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int kGramSmemFloats = 32 * (128 + 1) + 2 * 128;  // the extra workgroups' need at d = 128 (>= 4 * kGramNe)
 static_assert(kGramSmemFloats >= kGramWaves * kGramNe, "the cross-wave reduction fits the shared block");
@@ -500,7 +497,7 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
   float* hat_q = hat_k + 32;
   float* new_k = hat_q + 32;
   float* tmp = new_k + 32;
-  float* cred = tmp + 32;           // [2 matrices][2 addends][32*32] tiles of B B^T (from the Gram launch)
+  float* cred = tmp + 32;           // [2 matrices][2 halves of d][32*32] tiles of B B^T (from the Gram launch)
   (void)hat_k; (void)hat_q; (void)new_k; (void)tmp;
 
   // ---- every global load of the kernel is issued here, back to back

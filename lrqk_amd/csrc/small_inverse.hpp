@@ -8,7 +8,6 @@
 namespace lrqk {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef double v4d __attribute__((ext_vector_type(4)));
 
 // C tile of mfma_f32_32x32x2f32: lane l, element v -> row (the column is l & 31)
 __device__ __forceinline__ int mfma_row(int lane, int v) { return ((v >> 2) << 3) + ((lane >> 5) << 2) + (v & 3); }
