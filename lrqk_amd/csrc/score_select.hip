@@ -1830,7 +1830,10 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
     const int cap = std::min(topk, ctx->vic_req);
     const size_t need = (size_t)bh * (cap + 1) * sizeof(int32_t);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (need > ctx->next_ids.bytes) LRQK_HIP_CHECK(hipStreamIsCapturing(st, &capturing));
+    if (need > ctx->next_ids.bytes && hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+      (void)hipGetLastError();  // (another stream's capture)
+      capturing = hipStreamCaptureStatusActive;
+    }
     if (capturing == hipStreamCaptureStatusNone && ctx->next_ids.ensure(need) == LRQK_OK) {
       sb.st.next_ids = (int32_t*)ctx->next_ids.p;
       sb.st.next_cnt = sb.st.next_ids + (size_t)bh * cap;
