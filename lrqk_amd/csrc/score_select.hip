@@ -168,10 +168,13 @@ struct SelState {
   int* stats;
   int* rescored;     // per workgroup of the last index scan: rows whose bound passed (rescored exactly)
   int rescored_cap;
-  // A prompt's selection also lists the tokens of rank k .. 1.5 k (any order), for the victim cache; null: not asked for.
-  int32_t* next_ids;  // [bh][next_cap]
-  int* next_cnt;      // [bh]
-  int next_cap;
+};
+
+// The tokens of rank k .. 1.5 k (any order), listed beside a prompt's selection for the victim cache.
+struct NextList {
+  int32_t* ids;  // [bh][cap]
+  int* cnt;      // [bh]
+  int cap;
 };
 
 __global__ void init_select_state_kernel(SelState st, int bh) {
@@ -764,13 +767,15 @@ struct SelLds {
 
 // n_list: the length of the head's candidate list if the caller has read it already (and every thread of the
 // workgroup with it), else -1.
-template <typename T, int R>
+// LIST: a prompt's selection, without a diff, that also fills `next`.  An instantiation of its own: with the list behind a
+// test at run time the kernels without it kept its state as well (select_kernel 6 .. 12 -> 17 spilled vector registers).
+template <typename T, int R, bool LIST = false>
 __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const uint2* __restrict__ cand_all, int cand_cap,
                                                SelState st, uint32_t* __restrict__ keys_all, int64_t key_stride,
                                                const T* __restrict__ a_k, int64_t head_stride,
                                                const T* __restrict__ q_hat, int64_t m, int r, int round_bf16, int k,
                                                int32_t* __restrict__ out_all, int64_t out_stride, DiffArgs df,
-                                               int n_list, int bound_rank_k = 0) {
+                                               int n_list, int bound_rank_k = 0, NextList next = NextList{}) {
   uint32_t* const dyn = L.dyn;
   uint32_t* const hist = L.hist;
   uint32_t* const hist_b = L.hist_b;
@@ -791,7 +796,7 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
   constexpr int kDiffIpt = kFusedDiffMaxK / kSelThreads;
   const int ipt = (k + kSelThreads - 1) / kSelThreads;  // items per thread actually in use (<= kDiffIpt)
   int32_t hv[kDiffIpt];
-  if (df.hit != nullptr && !df.replace_all) {
+  if (!LIST && df.hit != nullptr && !df.replace_all) {
 #pragma unroll
     for (int u = 0; u < kDiffIpt; ++u)
       hv[u] = df.hit[(int64_t)h * df.hit_stride + min(tid * ipt + u, k - 1)];
@@ -944,17 +949,29 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
       need_eq = need3;
     }
   }
-  const uint32_t Tk = lo + (offT << tz), Tlow = lo + (offE << tz);
-  __shared__ int s_next;
+  const uint32_t Tk = lo + (offT << tz);
   if (tid == 0) {
-    s_next = 0;
-    st.t_low[h] = Tlow;  // rank >= 1.5k (rounded down to the resolved bits)
+    st.t_low[h] = lo + (offE << tz);  // rank >= 1.5k (rounded down to the resolved bits)
     st.q_norm[h] = mode == 0 ? st.q_cur[h] : 0.0f;
+  }
+
+  if constexpr (LIST) {
+    const uint32_t Tlow = lo + (offE << tz);
+    if (tid == 0) s_n = 0;  // (the list's length has been read)
+    __syncthreads();
+    for_each([&](uint32_t key, int64_t idx) {
+      if (key < Tk && key >= Tlow) {
+        const int p = atomicAdd(&s_n, 1);
+        if (p < next.cap) next.ids[(int64_t)h * next.cap + p] = (int32_t)idx;
+      }
+    });
+    __syncthreads();
+    if (tid == 0) next.cnt[h] = min(s_n, next.cap);
   }
 
   // ---- ordered output through two bitmaps over the token ids: gt (key > T), eq (key == T).
   // Every index with key > T is emitted, plus the first need_eq indices with key == T.
-  const bool do_diff = df.hit != nullptr;
+  const bool do_diff = !LIST && df.hit != nullptr;
   int32_t* new_s = reinterpret_cast<int32_t*>(dyn + 2 * kChunkWords);  // [k] when do_diff
   int out_pos = 0, eq_seen = 0;
   for (int64_t c0 = 0; c0 < m; c0 += kChunkBits) {
@@ -974,13 +991,8 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
     for_each([&](uint32_t key, int64_t idx) {
       const int64_t rel = idx - c0;
       if (key >= Tk && rel >= 0 && rel < span) atomicOr(key > Tk ? &gt[rel >> 5] : &eq[rel >> 5], 1u << (rel & 31));
-      if (st.next_ids && c0 == 0 && key < Tk && key >= Tlow) {
-        const int p = atomicAdd(&s_next, 1);
-        if (p < st.next_cap) st.next_ids[(int64_t)h * st.next_cap + p] = (int32_t)idx;
-      }
     });
     __syncthreads();
-    if (st.next_ids && c0 == 0 && tid == 0) st.next_cnt[h] = min(s_next, st.next_cap);
     const int w0 = tid * W;
     uint32_t gwr[kWordsPT], ewr[kWordsPT];
 #pragma unroll
@@ -1153,16 +1165,16 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
   if (tid == 0 && df.miss_count) df.miss_count[h] = n_pair;
 }
 
-template <typename T, int R>
+template <typename T, int R, bool LIST = false>
 __global__ __launch_bounds__(kSelThreads) void select_kernel(int mode, const uint2* __restrict__ cand_all, int cand_cap,
                                                              SelState st, uint32_t* __restrict__ keys_all,
                                                              int64_t key_stride, const T* __restrict__ a_k,
                                                              int64_t head_stride, const T* __restrict__ q_hat, int64_t m,
                                                              int r, int round_bf16, int k, int32_t* __restrict__ out_all,
-                                                             int64_t out_stride, DiffArgs df) {
+                                                             int64_t out_stride, DiffArgs df, NextList next) {
   LRQK_SEL_LDS(L);
-  select_generic<T, R>(L, mode, cand_all, cand_cap, st, keys_all, key_stride, a_k, head_stride, q_hat, m, r, round_bf16, k,
-                       out_all, out_stride, df, -1);
+  select_generic<T, R, LIST>(L, mode, cand_all, cand_cap, st, keys_all, key_stride, a_k, head_stride, q_hat, m, r, round_bf16,
+                             k, out_all, out_stride, df, -1, 0, next);
 }
 
 // --------------------------------------------------------------------------- select + diff of the decode step
@@ -1513,7 +1525,6 @@ __global__ __launch_bounds__(kSelThreads) void select_step_kernel(const uint2* _
                                                                   int32_t* __restrict__ out_all, int64_t out_stride,
                                                                   DiffArgs df) {
   LRQK_SEL_LDS(L);
-  st.next_ids = nullptr;  // (a prompt's selection only)
   const int h = blockIdx.x;
   const int n = __builtin_amdgcn_readfirstlane(st.cand_count[h * kCountStride]);
   const int lvl = __builtin_amdgcn_readfirstlane(st.level[h]);
@@ -1608,9 +1619,6 @@ static int prepare_select(lrqk_ctx* ctx, int bh, int64_t m, int topk, hipStream_
   sb->st.stats = (int*)(base + 6 * bh);
   sb->st.rescored = (int*)(base + 6 * bh + 3);
   sb->st.rescored_cap = bh + kRescSlots;
-  sb->st.next_ids = nullptr;
-  sb->st.next_cnt = nullptr;
-  sb->st.next_cap = 0;
   if (before != ctx->cand_cnt.p || ctx->sel_bh != bh) {
     hipLaunchKernelGGL(init_select_state_kernel, dim3((unsigned)((bh + 255) / 256)), dim3(256), 0, st, sb->st, bh);
     LRQK_HIP_CHECK(hipGetLastError());
@@ -1622,7 +1630,8 @@ static int prepare_select(lrqk_ctx* ctx, int bh, int64_t m, int topk, hipStream_
 template <typename T, int R>
 static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void* a_k, int64_t head_stride,
                                 const void* q_hat, int bh, int64_t m, int r, int round_bf16, int topk, int32_t* out_idx,
-                                int64_t out_stride, const DiffArgs& df, hipStream_t st, bool want_out = true) {
+                                int64_t out_stride, const DiffArgs& df, hipStream_t st, bool want_out = true,
+                                const NextList* next = nullptr) {
   size_t smem = select_smem(topk, df.hit != nullptr);
   // the decode step's select + diff (no ascending output): as long as its bitmaps fit the LDS beside the
   // generic path's blocks
@@ -1639,11 +1648,11 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
       step_allowed = smem;
     }
   }
-  static std::atomic<size_t> smem_allowed_dev[kMaxDeviceSlots];
-  std::atomic<size_t>& smem_allowed = smem_allowed_dev[per_device_slot()];
+  const auto select = next ? select_kernel<T, R, true> : select_kernel<T, R>;
+  static std::atomic<size_t> smem_allowed_dev[2][kMaxDeviceSlots];
+  std::atomic<size_t>& smem_allowed = smem_allowed_dev[next != nullptr][per_device_slot()];
   if (!step_path && smem > smem_allowed) {
-    LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)select_kernel<T, R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)smem));
+    LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)select, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     smem_allowed = smem;
   }
   const bool timed = ctx->tev && ctx->tev_used < ctx->tev_pairs && (ctx->tev_seen++ % ctx->tev_every) == 0;
@@ -1722,9 +1731,9 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
                        sb.st, sb.keys, sb.key_stride, (const T*)a_k, head_stride, (const T*)q_hat, m, r, round_bf16, topk,
                        out_idx, out_stride, df);
   else
-    hipLaunchKernelGGL((select_kernel<T, R>), dim3((unsigned)bh), dim3(kSelThreads), smem, st, 0, sb.cand, sb.cand_cap,
-                       sb.st, sb.keys, sb.key_stride, (const T*)a_k, head_stride, (const T*)q_hat, m, r, round_bf16, topk,
-                       out_idx, out_stride, df);
+    hipLaunchKernelGGL(select, dim3((unsigned)bh), dim3(kSelThreads), smem, st, 0, sb.cand, sb.cand_cap, sb.st, sb.keys,
+                       sb.key_stride, (const T*)a_k, head_stride, (const T*)q_hat, m, r, round_bf16, topk, out_idx,
+                       out_stride, df, next ? *next : NextList{});
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
@@ -1733,11 +1742,11 @@ template <typename T>
 static int dispatch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void* a_k, int64_t head_stride,
                                   const void* q_hat, int bh, int64_t m, int r, int round_bf16, int topk,
                                   int32_t* out_idx, int64_t out_stride, const DiffArgs& df, hipStream_t st,
-                                  bool want_out = true) {
+                                  bool want_out = true, const NextList* next = nullptr) {
   const bool vec_ok = ((uintptr_t)a_k % 16 == 0) && ((head_stride * sizeof(T)) % 16 == 0);
 #define LRQK_FS_CASE(RR)                                                                                            \
   return launch_filter_select<T, RR>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, round_bf16, topk, out_idx, out_stride, \
-                                     df, st, want_out)
+                                     df, st, want_out, next)
   if (vec_ok && r == 64) LRQK_FS_CASE(64);
   if (vec_ok && r == 32) LRQK_FS_CASE(32);
   if (vec_ok && r == 16) LRQK_FS_CASE(16);
@@ -1826,6 +1835,7 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
   if ((rc = prepare_select(ctx, bh, m, topk, st, &sb))) return rc;
   // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it (without memory for
   // the list, or in a capture that would have to take it, there is none)
+  NextList next{};
   if (ctx->vic_req > 0 && ctx->vic_dirty) {
     const int cap = std::min(topk, ctx->vic_req);
     const size_t need = (size_t)bh * (cap + 1) * sizeof(int32_t);
@@ -1835,19 +1845,20 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
       capturing = hipStreamCaptureStatusActive;
     }
     if (capturing == hipStreamCaptureStatusNone && ctx->next_ids.ensure(need) == LRQK_OK) {
-      sb.st.next_ids = (int32_t*)ctx->next_ids.p;
-      sb.st.next_cnt = sb.st.next_ids + (size_t)bh * cap;
-      sb.st.next_cap = ctx->next_cap = cap;
+      next = NextList{(int32_t*)ctx->next_ids.p, (int32_t*)ctx->next_ids.p + (size_t)bh * cap, cap};
+      ctx->next_cap = cap;
       ctx->next_bh = bh;
       ctx->next_valid = true;
     }
   }
   DiffArgs df{nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0};
+  const NextList* list = next.ids ? &next : nullptr;
   if (dtype == LRQK_F32)
-    rc = dispatch_filter_select<float>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, 0, topk, out_idx, out_stride, df, st);
+    rc = dispatch_filter_select<float>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, 0, topk, out_idx, out_stride, df, st, true,
+                                       list);
   else
     rc = dispatch_filter_select<bf16_t>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, round_bf16, topk, out_idx,
-                                        out_stride, df, st);
+                                        out_stride, df, st, true, list);
   return rc ? rc : topk;
 }
 
@@ -1904,7 +1915,7 @@ extern "C" int lrqk_select_from_scores(lrqk_ctx* ctx, const float* scores, int b
   DiffArgs df{nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0};
   hipLaunchKernelGGL((select_kernel<float, 0>), dim3((unsigned)bh), dim3(kSelThreads), smem, st, 1, sb.cand, sb.cand_cap,
                      sb.st, sb.keys, sb.key_stride, (const float*)nullptr, (int64_t)0, (const float*)nullptr, m, 1, 0,
-                     topk, out_idx, out_stride, df);
+                     topk, out_idx, out_stride, df, NextList{});
   LRQK_HIP_CHECK(hipGetLastError());
   return topk;
 }
