@@ -363,10 +363,10 @@ constexpr int kScanWaves = kFiltThreads / kWave;
 // (Workgroups per CU, that is waves per SIMD, that the registers are held to.  One more at R = 64 spills in the loop:
 // 127.6 against 119.4 us per step at 64K rows.)
 constexpr int scan_waves(int r) { return r == 64 ? 3 : r == 32 ? 4 : 5; }
-template <typename T, int R>
+template <typename T, int R, bool HEADS_FIRST>
 __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_kernel(
     const T* __restrict__ a_k, int64_t head_stride, const T* __restrict__ q_hat, int64_t m, int r, int round_bf16,
-    SelState st, uint2* __restrict__ cand, int cand_cap, FilterQ fq, ScoreIndexView six, bool heads_first) {
+    SelState st, uint2* __restrict__ cand, int cand_cap, FilterQ fq, ScoreIndexView six) {
   static_assert(R == 16 || R == 32 || R == 64, "the score index covers ranks 16, 32, 64");
   constexpr int QV = R / 16;                  // lanes per row
   constexpr int kRowsPerLoad = kWave / QV;    // rows that one load of a wave covers
@@ -381,9 +381,10 @@ __global__ __launch_bounds__(kFiltThreads, scan_waves(R)) void score_prefilter_k
   __shared__ __align__(16) float qx_s[kShare ? 1 : kScanWaves][R];  // the proxy query as the exact score uses it
   __shared__ __align__(16) float qp_s[R];                          // q'
   __shared__ int resc_s;
-  // (the grid's order is the host's choice)
-  const int h = heads_first ? blockIdx.x : blockIdx.y;
-  const int wg = heads_first ? blockIdx.y : blockIdx.x, n_wgs = heads_first ? gridDim.y : gridDim.x;
+  // (the grid's order is the host's choice.  Not an argument: the grid's size would then be read at an address that waits for
+  // the argument, in front of everything else: 0.3 .. 0.5 us of a scan of 32 heads x 10K rows, 0.6 of 256 x 128K)
+  const int h = HEADS_FIRST ? blockIdx.x : blockIdx.y;
+  const int wg = HEADS_FIRST ? blockIdx.y : blockIdx.x, n_wgs = HEADS_FIRST ? gridDim.y : gridDim.x;
   const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
   const T* A = a_k + (int64_t)h * head_stride;
   const uint8_t* QA = six.qa + (int64_t)h * six.head_rows * R;
@@ -1692,7 +1693,7 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
       int slots = slots_a;
       if (slots == 0) {
         int per_cu = 0, dev = 0, n_cu = 0;
-        LRQK_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, score_prefilter_kernel<T, R>,
+        LRQK_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, score_prefilter_kernel<T, R, false>,
                                                                     kFiltThreads, 0));
         LRQK_HIP_CHECK(hipGetDevice(&dev));
         LRQK_HIP_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1710,8 +1711,9 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
       // heads in a row, the fetch slower by 1 .. 12 us.)
       const bool heads_first = bh <= 32 && m >= 32768;
       const dim3 grid_st((unsigned)(heads_first ? bh : wgs), (unsigned)(heads_first ? wgs : bh));
-      hipLaunchKernelGGL((score_prefilter_kernel<T, R>), grid_st, dim3(kFiltThreads), 0, st, (const T*)a_k,
-                         head_stride, (const T*)q_hat, m, r, round_bf16, sb.st, sb.cand, sb.cand_cap, fq, six, heads_first);
+      const auto scan = heads_first ? score_prefilter_kernel<T, R, true> : score_prefilter_kernel<T, R, false>;
+      hipLaunchKernelGGL(scan, grid_st, dim3(kFiltThreads), 0, st, (const T*)a_k, head_stride, (const T*)q_hat, m, r,
+                         round_bf16, sb.st, sb.cand, sb.cand_cap, fq, six);
       via_index = true;
       ctx->scan_wgs = (int)std::min<int64_t>(wgs * bh, sb.st.rescored_cap);
       ctx->scan_rows = (int64_t)bh * m;
