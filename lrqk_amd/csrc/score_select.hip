@@ -1703,13 +1703,15 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
       constexpr int kStepRowsWg = (kWave / (R / 16)) * kScanU * kScanWaves;  // rows one step of a workgroup's waves covers
       const int64_t need = (m + kStepRowsWg - 1) / kStepRowsWg;
       const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(need, slots / bh));
-      // Up to 32 heads of 32K rows and more stand in a row: workgroups go round the XCDs in the order of their index, so a
-      // head's workgroups (eight heads and more, a multiple of 8 of them) share an XCD, its list counter and what they read
-      // of its state.  At 128K rows (a head after the other -> in a row) 8 heads 18.9 -> 17.1 us, 16 heads 20.1 -> 18.9, 28 and
-      // 32 heads 0.5 less; 24 the same.  Beyond 32 heads neighbouring workgroups should read neighbouring rows: 64 heads a step of
-      // 129 us in 136, 256 heads the scan 219 -> 229.  At 8K rows 0.3 us more.  (The step's other launches: no faster with the
-      // heads in a row, the fetch slower by 1 .. 12 us.)
-      const bool heads_first = bh <= 32 && m >= 32768;
+      // The heads stand in a row where the scan is long enough for it: workgroups go round the XCDs in the order of their
+      // index, so a head's workgroups share one XCD (8 heads and multiples of it) or a few, with its list counter and what
+      // they read of its state.  The edge lies between 384K rows of all heads (a head after the other -> in a row, us, r 32:
+      // 8 x 48K 12.9 -> 13.5, 16 x 24K 10.3 -> 11.1, 24 x 16K 10.2 -> 10.3, 32 x 12K 9.9 -> 9.6) and 448K .. 512K (28 x 16K 10.8
+      // -> 10.3, 8 x 64K 16.7 -> 14.3, 16 x 32K 13.0 -> 12.2, 32 x 16K 11.8 -> 10.6).  At 128K rows 1 and 2 heads the same, 4
+      // heads 26.0 -> 18.1, 8 18.9 -> 16.2, 16 20.3 -> 18.0, 28 26.3 -> 25.4, 32 28.8 -> 28.1; ranks 16 and 64 alike.  Beyond 32
+      // heads neighbouring workgroups should read neighbouring rows: 64 heads a step of 129 us in 136, 256 heads the scan
+      // 219 -> 229.  (The step's other launches: no faster with the heads in a row, the fetch slower by 1 .. 12 us.)
+      const bool heads_first = bh <= 32 && (int64_t)bh * m >= 416 * 1024;
       const dim3 grid_st((unsigned)(heads_first ? bh : wgs), (unsigned)(heads_first ? wgs : bh));
       const auto scan = heads_first ? score_prefilter_kernel<T, R, true> : score_prefilter_kernel<T, R, false>;
       hipLaunchKernelGGL(scan, grid_st, dim3(kFiltThreads), 0, st, (const T*)a_k, head_stride, (const T*)q_hat, m, r,

@@ -369,6 +369,23 @@ def test_selection_through_a_freshly_built_index(ops, dtype, r, m):
     assert rows == 3 * m and rescored < rows // 3
 
 
+@pytest.mark.parametrize("dtype,r,heads,m", [
+    (torch.bfloat16, 32, 13, 32767), (torch.bfloat16, 32, 13, 32768), (torch.float32, 16, 32, 13311), (torch.float32, 16, 32, 13313),
+    (torch.bfloat16, 64, 32, 14001), (torch.bfloat16, 32, 33, 13000), (torch.float32, 32, 1, 425984)])
+def test_selection_on_either_side_of_the_scans_orders(ops, dtype, r, heads, m):
+    """Scans of 416K rows of up to 32 heads take the heads in a row, others a head after the other: the selections are those
+    of the plain scan."""
+    gen = torch.Generator(device=DEV).manual_seed(heads + m)
+    a_k = torch.randn((1, heads, m + 3, r), generator=gen, device=DEV).to(dtype)
+    q0 = torch.randn((1, heads, 1, r), generator=gen, device=DEV)
+    plain, indexed = ops.Workspace(), ops.Workspace()
+    indexed.score_index(True)
+    for step in range(2):
+        q = (q0 + 0.05 * step).to(dtype)
+        assert torch.equal(ops.score_select(indexed, a_k, q, m, 300), ops.score_select(plain, a_k, q, m, 300)), step
+    assert indexed.scan_stats()[0] == heads * m
+
+
 @pytest.mark.parametrize("dtype,hq,hkv,d,l,k,lite", [(torch.float32, 2, 1, 8, 12, 8, 4), (torch.bfloat16, 6, 2, 64, 515, 33, 7),
                                                      (torch.float32, 4, 4, 256, 300, 100, 1), (torch.bfloat16, 4, 2, 64, 90, 16, 0)])
 def test_active_set_of_a_prompt(ops, dtype, hq, hkv, d, l, k, lite):
