@@ -1517,8 +1517,11 @@ __device__ __forceinline__ int bound_rank(int k, int level, int64_t n) {
 }
 constexpr int kCalmCalls = 32;  // usable lists in a row before a head's slack is halved again
 
+// Where the 80 KB of code begin is pinned: the caches of a CU's instructions hold 64 KB and every launch starts with cold
+// ones, and the same instructions took 11.2 .. 11.8 us (32 heads x 32K rows) and 15.1 .. 16.2 (256 x 128K) by their address,
+// which moves with every other kernel of this file.  On multiples of 8 KB 11.3 and 15.4, of 64 KB 11.7 and 15.7.
 template <typename T, int R>
-__global__ __launch_bounds__(kSelThreads) void select_step_kernel(const uint2* __restrict__ cand_all, int cand_cap,
+__global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void select_step_kernel(const uint2* __restrict__ cand_all, int cand_cap,
                                                                   SelState st, uint32_t* __restrict__ keys_all,
                                                                   int64_t key_stride, const T* __restrict__ a_k,
                                                                   int64_t head_stride, const T* __restrict__ q_hat,
