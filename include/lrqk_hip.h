@@ -75,6 +75,12 @@ int lrqk_proxy_scores(const void* a_k, int64_t head_stride, const void* q_hat, i
 int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
                       int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
                       int64_t out_stride, void* stream);
+/* The same for a prompt whose next best tokens lrqk_victim_fill shall put into the victim cache: where that cache is asked
+ * for and holds nothing, the ctx also lists, per head, the tokens that come next in the selection's order (about topk / 2 of
+ * them, at most the cache's rows; topk up to 4096). */
+int lrqk_score_select_next(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
+                           int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
+                           int64_t out_stride, void* stream);
 
 /* Same selection from caller-provided fp32 scores [bh][m] (test hook for tie cases). */
 int lrqk_select_from_scores(lrqk_ctx* ctx, const float* scores, int bh, int64_t m, int topk,
@@ -162,11 +168,10 @@ int lrqk_ctx_score_index(lrqk_ctx* ctx, int enable);
  * contents before the ctx is used for another prompt.  0 switches it off.  Memory: bh *
  * rows_per_head rows of 2*d elements plus 2 bytes per (head, store row). */
 int lrqk_ctx_victim_cache(lrqk_ctx* ctx, int rows_per_head);
-/* After lrqk_score_select over a prompt of l tokens, with the victim cache of ctx empty: puts the K and V rows of the
- * tokens that come next in the selection's order (about topk / 2 per head) into the cache, from the prompt's k, v
- * ([b][hkv][l][d] on the device); the first steps then find most of the tokens that enter the active set there.
- * cap: rows of the store that lrqk_decode_step will be given (another one empties the cache).  Does nothing where that
- * selection is not the ctx's last one or the step would not use the cache. */
+/* After lrqk_score_select_next over a prompt of l tokens: puts the K and V rows of the tokens that it listed into the
+ * empty victim cache, from the prompt's k, v ([b][hkv][l][d] on the device); the first steps then find most of the tokens
+ * that enter the active set there.  cap: rows of the store that lrqk_decode_step will be given (another one empties the
+ * cache).  Does nothing where that selection is not the ctx's last one or the step would not use the cache. */
 int lrqk_victim_fill(lrqk_ctx* ctx, const void* k, const void* v, int64_t l, int64_t cap, int b, int hq, int hkv, int d,
                      int dtype, void* stream);
 /* Rows that lrqk_decode_step fetched over the host link since the last reset (the other missed

@@ -1825,9 +1825,9 @@ extern "C" int lrqk_proxy_scores(const void* a_k, int64_t head_stride, const voi
   return launch_scores<bf16_t>(a_k, head_stride, q_hat, bh, m, r, round_bf16, nullptr, 0, out_scores, st);
 }
 
-extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
-                                 int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
-                                 int64_t out_stride, void* stream) {
+static int score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh, int64_t m, int r,
+                        int topk, int dtype, int round_bf16, int32_t* out_idx, int64_t out_stride, bool list_next,
+                        void* stream) {
   if (ctx) ctx->pool.enter((hipStream_t)stream);
   int rc = check_select_args(ctx, bh, m, topk, out_idx, out_stride);
   if (rc) return rc;
@@ -1843,7 +1843,7 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
   // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it (without memory for
   // the list, or in a capture that would have to take it, there is none)
   NextList next{};
-  if (ctx->vic_req > 0 && ctx->vic_dirty) {
+  if (list_next && topk <= kFusedDiffMaxK && ctx->vic_req > 0 && ctx->vic_dirty) {
     const int cap = std::min(topk, ctx->vic_req);
     const size_t need = (size_t)bh * (cap + 1) * sizeof(int32_t);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -1867,6 +1867,18 @@ extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_st
     rc = dispatch_filter_select<bf16_t>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, round_bf16, topk, out_idx,
                                         out_stride, df, st, true, list);
   return rc ? rc : topk;
+}
+
+extern "C" int lrqk_score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
+                                 int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
+                                 int64_t out_stride, void* stream) {
+  return score_select(ctx, a_k, head_stride, q_hat, bh, m, r, topk, dtype, round_bf16, out_idx, out_stride, false, stream);
+}
+
+extern "C" int lrqk_score_select_next(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,
+                                      int64_t m, int r, int topk, int dtype, int round_bf16, int32_t* out_idx,
+                                      int64_t out_stride, void* stream) {
+  return score_select(ctx, a_k, head_stride, q_hat, bh, m, r, topk, dtype, round_bf16, out_idx, out_stride, true, stream);
 }
 
 extern "C" int lrqk_score_select_diff(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh,

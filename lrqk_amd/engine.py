@@ -303,10 +303,14 @@ class LightAttentionIndicesFactory:
             # score index that this first scan builds then stays valid for the decode steps
             lb = seq_len - L
             if not custom:
-                ops.score_select(self.ws, self._A_K.data, A_Q, lb, k, self.round_scores_to_storage, out=self._active_idx)
+                # (a [K|V] row of more than 1 KB is fetched without the cache)
+                fill = (self.fill_victims and not self.no_hit_miss and self._fetch_mode == "direct" and key_states.is_cuda
+                        and 2 * key_states.shape[3] * key_states.element_size() <= 1024)
+                ops.score_select(self.ws, self._A_K.data, A_Q, lb, k, self.round_scores_to_storage, out=self._active_idx,
+                                 list_next=fill)
                 self._hit_len = k
                 ops.fill_active(key_states, value_states, self._active_idx, self.Kgpu, self.Vgpu, k)
-                if self.fill_victims and not self.no_hit_miss and self._fetch_mode == "direct" and key_states.is_cuda:
+                if fill:
                     ops.victim_fill(self.ws, key_states, value_states, self.Kgpu.shape[1], self.KVcpu.data.shape[2])
             else:
                 hit = self.compute_hit_indices(query_states=A_Q, key_states=self._A_K.data.narrow(2, 0, lb))

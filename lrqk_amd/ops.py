@@ -179,10 +179,10 @@ def proxy_scores(a_k: torch.Tensor, q_hat: torch.Tensor, m: Optional[int] = None
 
 def score_select(ws: Workspace, a_k: torch.Tensor, q_hat: torch.Tensor, m: int, topk: int,
                  round_to_storage: bool = True, out: Optional[torch.Tensor] = None,
-                 head_rows: Optional[int] = None) -> torch.Tensor:
+                 head_rows: Optional[int] = None, list_next: bool = False) -> torch.Tensor:
     """Top-k token ids (ascending) of q_hat . a_k[:m]^T per head: int32 [b,H,min(topk,m)].
     a_k is [b,H,cap,r] contiguous, or (with head_rows) a view whose heads start head_rows rows
-    apart and whose rows are contiguous."""
+    apart and whose rows are contiguous.  list_next: ``victim_fill`` follows."""
     _need_cuda(a_k, q_hat)
     b, H, cap, r = a_k.shape
     if head_rows is None:
@@ -195,9 +195,10 @@ def score_select(ws: Workspace, a_k: torch.Tensor, q_hat: torch.Tensor, m: int, 
     if out is None:
         out = torch.empty((b, H, kk), dtype=torch.int32, device=a_k.device)
     assert out.dtype == torch.int32 and out.is_contiguous() and out.shape[-1] >= kk
-    check(_lib.load().lrqk_score_select(ws.handle, a_k.data_ptr(), cap * r, qh.data_ptr(), b * H, m, r, topk,
-                                        _dt(a_k), 1 if (round_to_storage and a_k.dtype == torch.bfloat16) else 0,
-                                        out.data_ptr(), out.shape[-1], _stream(a_k)))
+    lib = _lib.load()
+    select = lib.lrqk_score_select_next if list_next else lib.lrqk_score_select
+    check(select(ws.handle, a_k.data_ptr(), cap * r, qh.data_ptr(), b * H, m, r, topk, _dt(a_k),
+                 1 if (round_to_storage and a_k.dtype == torch.bfloat16) else 0, out.data_ptr(), out.shape[-1], _stream(a_k)))
     return out
 
 
@@ -319,8 +320,8 @@ def fill_active(k: torch.Tensor, v: torch.Tensor, active_idx: torch.Tensor, k_ac
 
 
 def victim_fill(ws: Workspace, k: torch.Tensor, v: torch.Tensor, hq: int, capacity: int):
-    """The rows of k, v [b,Hkv,l,d] of the tokens that the last ``score_select`` of ``ws`` left out by the least go into its
-    empty victim cache; ``capacity``: rows of the host store of the steps to come."""
+    """The rows of k, v [b,Hkv,l,d] of the tokens that the last ``score_select`` of ``ws``, called with ``list_next``, left
+    out by the least go into its empty victim cache; ``capacity``: rows of the host store of the steps to come."""
     _need_cuda(k, v)
     b, hkv, l, d = k.shape
     assert k.is_contiguous() and v.is_contiguous() and v.shape == k.shape and k.dtype == v.dtype

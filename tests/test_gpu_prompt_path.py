@@ -442,6 +442,32 @@ def test_cache_filled_by_the_prompt_is_invisible(ops, dtype, batch, hq, hkv, d, 
     assert filled < without or d == 256 or rows < 96   # (a few rows are replaced before they are asked for)
 
 
+@pytest.mark.parametrize("engine,d,listed", [("plain", 8, True), ("switched off", 8, False), ("no hit miss", 8, False),
+                                             ("staged fetch", 8, False), ("offload", 8, False), ("plain", 256, False)])
+def test_a_prompt_lists_tokens_only_for_a_cache_that_it_fills(ops, monkeypatch, engine, d, listed):
+    """The list of a prompt's next best tokens (128 heads x 1700: a block of its own) is given memory only where the prompt
+    then fills the cache from it."""
+    from lrqk_amd import engine as E
+    kind = {"offload": E.LightAttentionIndicesOffloadPrefill, "no hit miss": E.LightAttentionIndicesNoHitMiss}
+    eng = kind.get(engine, E.LightAttentionIndicesFactory)(num_lite_tokens=8, attn_topk=1700, num_key_value_groups=8, r=8,
+                                                           max_iter=1, tol=0.0, capacity=2100)
+    if engine == "switched off":
+        eng.fill_victims = False
+    if engine == "staged fetch":
+        eng.fetch_mode = "staged"
+    sizes, alloc = [], torch.cuda.caching_allocator_alloc
+
+    def recorded(size, *a, **kw):
+        sizes.append(size)
+        return alloc(size, *a, **kw)
+    gen = torch.Generator(device=DEV).manual_seed(d)
+    q, k, v = (torch.randn((16, h, 2000, d), generator=gen, device=DEV) for h in (8, 1, 1))
+    monkeypatch.setattr(torch.cuda, "caching_allocator_alloc", recorded)
+    eng.prefill(q, k, v)
+    need = 128 * 1701 * 4
+    assert (need + need // 4 in sizes) == listed
+
+
 @pytest.mark.parametrize("batch,hkv,l", [(1, 1, 300), (2, 3, 517), (1, 16, 1031)])
 def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
     """A prompt whose first heads go ahead of the others (one head: a single copy; 6 and 16: pieces of 1 + 5, 2 + 14) is
