@@ -32,7 +32,9 @@ struct BufPool {
   void* take(size_t bytes) {
     if (alloc) return alloc(bytes, (void*)stream, user);
     void* p = nullptr;
-    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();  // (who asked for the block reports it; the check behind the next launch must not)
+    return nullptr;
   }
   void give(void* p) {
     if (alloc)

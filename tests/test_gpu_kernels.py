@@ -134,6 +134,25 @@ def test_score_select_full_size_with_score_index(ops, oracle, H, m):
     assert full >= H and fast >= H, (fast, full)
 
 
+def test_memory_that_is_not_to_be_had_is_reported_once(ops, ws):
+    """A ctx without the caller's allocator that could not get a block (88 TB here) says so, and the next call, which needs
+    no such block, does not fail for it."""
+    import ctypes
+    from types import SimpleNamespace
+    from lrqk_amd import _lib
+    lib, handle = _lib.load(), ctypes.c_void_p()
+    _lib.check(lib.lrqk_ctx_create(ctypes.byref(handle)))
+    try:
+        with pytest.raises(_lib.LrqkError, match="device memory"):
+            _lib.check(lib.lrqk_ctx_reserve_on(handle, 1, 1 << 44, 16, 32, 16, 64, None))
+        g = torch.Generator().manual_seed(5)
+        A, q = (torch.randn((1, 2, n, 16), generator=g).to(DEV) for n in (500, 1))
+        assert torch.equal(ops.score_select(SimpleNamespace(handle=handle), A, q, 500, 40), ops.score_select(ws, A, q, 500, 40))
+        torch.cuda.synchronize()
+    finally:
+        _lib.check(lib.lrqk_ctx_destroy(handle))
+
+
 def test_score_select_filtered_path(ops, oracle):
     """Repeated calls on one workspace with a slowly drifting query: after the first call the
     heads are served from the candidate list of the streaming filter; every result must
