@@ -1855,7 +1855,6 @@ static int score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, con
       next = NextList{(int32_t*)ctx->next_ids.p, (int32_t*)ctx->next_ids.p + (size_t)bh * cap, cap};
       ctx->next_cap = cap;
       ctx->next_bh = bh;
-      ctx->next_valid = true;
     }
   }
   DiffArgs df{nullptr, 0, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, 0};
@@ -1866,6 +1865,7 @@ static int score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, con
   else
     rc = dispatch_filter_select<bf16_t>(ctx, sb, a_k, head_stride, q_hat, bh, m, r, round_bf16, topk, out_idx,
                                         out_stride, df, st, true, list);
+  ctx->next_valid = list && rc == LRQK_OK;
   return rc ? rc : topk;
 }
 

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void victim_fill_kernel(const uint4* __restric
                                                           const int32_t* __restrict__ ids, const int* __restrict__ cnt,
                                                           int id_cap, VictimView vic, int hq, int hkv, int cpr) {
   const int h = blockIdx.y;
-  const int n = min(cnt[h], min(id_cap, vic.nv));
+  const int n = max(0, min(cnt[h], min(id_cap, vic.nv)));
   const int64_t src0 = ((int64_t)(h / hq) * hkv + (h % hq) / (hq / hkv)) * l;
   const int chunks = 2 * cpr;  // at most 64
   const int c = threadIdx.x % chunks, tpb = 256 / chunks;

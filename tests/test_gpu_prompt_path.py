@@ -468,6 +468,36 @@ def test_a_prompt_lists_tokens_only_for_a_cache_that_it_fills(ops, monkeypatch, 
     assert (need + need // 4 in sizes) == listed
 
 
+def test_a_selection_that_failed_leaves_no_list(ops, monkeypatch):
+    """A selection that raises before its kernels are launched (no memory for the score index) has listed nothing: nothing is
+    put into the cache, which would take its 1.3 MB here."""
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    a_k, q = (torch.randn((1, 4, n, 32), generator=gen, device=DEV) for n in (9000, 1))
+    K, V = (torch.randn((1, 2, 9000, 64), generator=gen, device=DEV) for _ in range(2))
+    ws = ops.Workspace()
+    ws.victim_cache(512)
+    ws.score_index(True)
+    ops.score_select(ws, a_k, q, 9000, 300, list_next=True)
+    want = ops.score_select(ws, a_k, q, 9000, 300)
+    bigger = torch.cat([a_k, a_k], 2)
+    sizes, alloc = [], torch.cuda.caching_allocator_alloc
+
+    def refused(size, *a, **kw):
+        sizes.append(size)
+        if size > 1 << 20 and fails:
+            raise torch.cuda.OutOfMemoryError("planted")
+        return alloc(size, *a, **kw)
+    monkeypatch.setattr(torch.cuda, "caching_allocator_alloc", refused)
+    fails = True
+    with pytest.raises(Exception, match="device memory"):
+        ops.score_select(ws, bigger, q, 9000, 300, list_next=True)
+    fails, sizes[:] = False, []
+    ops.victim_fill(ws, K, V, 4, 9000)
+    torch.cuda.synchronize()
+    assert not sizes
+    assert torch.equal(ops.score_select(ws, a_k, q, 9000, 300), want)
+
+
 @pytest.mark.parametrize("batch,hkv,l", [(1, 1, 300), (2, 3, 517), (1, 16, 1031)])
 def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
     """A prompt whose first heads go ahead of the others (one head: a single copy; 6 and 16: pieces of 1 + 5, 2 + 14) is
