@@ -171,7 +171,8 @@ int lrqk_ctx_victim_cache(lrqk_ctx* ctx, int rows_per_head);
 /* After lrqk_score_select_next over a prompt of l tokens: puts the K and V rows of the tokens that it listed into the
  * empty victim cache, from the prompt's k, v ([b][hkv][l][d] on the device); the first steps then find most of the tokens
  * that enter the active set there.  cap: rows of the store that lrqk_decode_step will be given (another one empties the
- * cache).  Does nothing where that selection is not the ctx's last one or the step would not use the cache. */
+ * cache).  Does nothing where that selection is not the ctx's last one or the step would not use the cache, where the
+ * memory of the cache is not to be had (the first step asks for it again), and in a stream capture. */
 int lrqk_victim_fill(lrqk_ctx* ctx, const void* k, const void* v, int64_t l, int64_t cap, int b, int hq, int hkv, int d,
                      int dtype, void* stream);
 /* Rows that lrqk_decode_step fetched over the host link since the last reset (the other missed

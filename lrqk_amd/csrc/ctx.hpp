@@ -186,6 +186,13 @@ inline int per_device_slot() {
   if (hipGetDevice(&dev) != hipSuccess) dev = 0;
   return dev >= 0 && dev < kMaxDeviceSlots ? dev : 0;
 }
+// Is this stream being captured into a graph?  (Yes, too, where another stream's capture forbids the question.)
+inline bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
 // Proxy-score scan + top-k with the hit/miss diff fused into the select kernel when the
 // sizes allow.  Returns 1 if the diff ran, 0 if the caller still has to, negative on error.
 int score_select_diff(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, const void* q_hat, int bh, int64_t m, int r,

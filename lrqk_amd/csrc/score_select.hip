@@ -1841,17 +1841,12 @@ static int score_select(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, con
   SelectBufs sb;
   if ((rc = prepare_select(ctx, bh, m, topk, st, &sb))) return rc;
   // a prompt of a ctx with a victim cache that holds nothing yet: what lrqk_victim_fill puts into it (without memory for
-  // the list, or in a capture that would have to take it, there is none)
+  // the list, or in a capture, which that function leaves alone, there is none)
   NextList next{};
-  if (list_next && topk <= kFusedDiffMaxK && ctx->vic_req > 0 && ctx->vic_dirty) {
+  if (list_next && topk <= kFusedDiffMaxK && ctx->vic_req > 0 && ctx->vic_dirty && !stream_capturing(st)) {
     const int cap = std::min(topk, ctx->vic_req);
     const size_t need = (size_t)bh * (cap + 1) * sizeof(int32_t);
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (need > ctx->next_ids.bytes && hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-      (void)hipGetLastError();  // (another stream's capture)
-      capturing = hipStreamCaptureStatusActive;
-    }
-    if (capturing == hipStreamCaptureStatusNone && ctx->next_ids.ensure(need) == LRQK_OK) {
+    if (ctx->next_ids.ensure(need) == LRQK_OK) {
       next = NextList{(int32_t*)ctx->next_ids.p, (int32_t*)ctx->next_ids.p + (size_t)bh * cap, cap};
       ctx->next_cap = cap;
       ctx->next_bh = bh;

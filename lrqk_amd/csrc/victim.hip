@@ -16,6 +16,14 @@ __global__ __launch_bounds__(256) void victim_init_kernel(int32_t* tok, int64_t 
   for (int64_t i = i0; i < n_counters; i += stride) counters[i] = 0;
 }
 
+// Memory of a cache of nv rows per head.  meta: tok i32 [bh][nv] | counters i32 [3][bh] (ptr, base, host_rows) |
+// pos i16 [bh][cap]
+static int victim_reserve(lrqk_ctx* ctx, int bh, int nv, int64_t cap, int chunks) {
+  ctx->vic_dirty = true;  // (a block that grows loses its contents, also where the other one is not to be had)
+  const int rc = ctx->vic_rows.ensure((size_t)bh * nv * chunks * sizeof(uint4));
+  return rc ? rc : ctx->vic_meta.ensure(((size_t)bh * nv + (size_t)3 * bh) * 4 + (size_t)bh * cap * 2 + 16);
+}
+
 int victim_prepare(lrqk_ctx* ctx, int bh, int64_t cap, int chunks, hipStream_t st) {
   if (ctx->vic_req <= 0) {
     ctx->vic.nv = 0;
@@ -24,11 +32,9 @@ int victim_prepare(lrqk_ctx* ctx, int bh, int64_t cap, int chunks, hipStream_t s
   const int nv = ctx->vic_req;
   const bool same = ctx->vic.nv == nv && ctx->vic_bh == bh && ctx->vic.cap == cap && ctx->vic_chunks == chunks;
   if (same && !ctx->vic_dirty) return LRQK_OK;
-  int rc;
-  if ((rc = ctx->vic_rows.ensure((size_t)bh * nv * chunks * sizeof(uint4)))) return rc;
-  // meta: tok i32 [bh][nv] | counters i32 [3][bh] (ptr, base, host_rows) | pos i16 [bh][cap]
+  const int rc = victim_reserve(ctx, bh, nv, cap, chunks);
+  if (rc) return rc;
   const size_t n_tok = (size_t)bh * nv, n_cnt = (size_t)3 * bh, n_pos = (size_t)bh * cap;
-  if ((rc = ctx->vic_meta.ensure((n_tok + n_cnt) * 4 + n_pos * 2 + 16))) return rc;
   VictimView v{};
   v.rows = (uint4*)ctx->vic_rows.p;
   v.tok = (int32_t*)ctx->vic_meta.p;
@@ -90,6 +96,9 @@ extern "C" int lrqk_victim_fill(lrqk_ctx* ctx, const void* k, const void* v, int
   const bool listed = ctx->next_valid && ctx->next_bh == bh && ctx->vic_req > 0 && ctx->vic_dirty;
   ctx->next_valid = false;
   if (!listed || 2 * cpr > kWave) return LRQK_OK;  // (rows that the step fetches without the cache)
+  // The cache changes no result, and the first step makes an empty one where there is none: a prompt does not fail for its
+  // memory.  In a capture it is left alone: a replay would fill one that the steps in between have used.
+  if (stream_capturing((hipStream_t)stream) || victim_reserve(ctx, bh, ctx->vic_req, cap, 2 * cpr) != LRQK_OK) return LRQK_OK;
   int rc = victim_prepare(ctx, bh, cap, 2 * cpr, (hipStream_t)stream);
   if (rc) return rc;
   const int32_t* ids = (const int32_t*)ctx->next_ids.p;

@@ -498,6 +498,77 @@ def test_a_selection_that_failed_leaves_no_list(ops, monkeypatch):
     assert torch.equal(ops.score_select(ws, a_k, q, 9000, 300), want)
 
 
+@pytest.mark.parametrize("refused", ["rows", "positions"])
+def test_a_prompt_does_not_fail_for_the_cache(ops, monkeypatch, refused):
+    """Without memory for the victim cache (its rows; its position table) a prompt goes on, and the steps, for which there is
+    memory again, are those after a prompt that does not fill it."""
+    from lrqk_amd.engine import LightAttentionIndicesFactory as Engine
+    gen = torch.Generator(device=DEV).manual_seed(3)
+
+    def draw(heads, n):
+        return torch.randn((1, heads, n, 64), generator=gen, device=DEV).to(torch.bfloat16)
+    l, k, heads, capacity = 1200, 100, 8, 80000
+    engines = [Engine(num_lite_tokens=8, attn_topk=k, num_key_value_groups=2, r=16, max_iter=1, tol=0.0, capacity=capacity)
+               for _ in range(2)]
+    prompt = draw(heads, l), draw(heads // 2, l), draw(heads // 2, l)
+    start = tuple(torch.randn((1, heads, l, 16), generator=gen, device=DEV) for _ in range(2))
+    rows = 1024
+    need = {"rows": heads * rows * 16 * 16, "positions": (heads * rows + 3 * heads) * 4 + heads * capacity * 2 + 16}[refused]
+    asked, alloc = [], torch.cuda.caching_allocator_alloc
+
+    def without(size, *a, **kw):
+        asked.append(size)
+        if size == need + need // 4:
+            raise torch.cuda.OutOfMemoryError("planted")
+        return alloc(size, *a, **kw)
+    for fill, eng in enumerate(engines):
+        eng.fill_victims, eng.victim_rows, eng.attn_in_step, eng.init_factors = bool(fill), rows, True, start
+        with monkeypatch.context() as m:
+            m.setattr(torch.cuda, "caching_allocator_alloc", without)
+            eng.prefill(*prompt)
+    assert asked.count(need + need // 4) == 1
+    for step in range(4):
+        t = draw(heads, 1), draw(heads // 2, 1), draw(heads // 2, 1)
+        for eng in engines:
+            eng.decode(*t)
+        assert torch.equal(engines[0]._active_idx, engines[1]._active_idx), step
+        assert torch.equal(engines[0].last_attn, engines[1].last_attn), step
+
+
+def test_a_captured_prompt_leaves_the_cache_alone(ops, monkeypatch):
+    """Selection and fill in a graph: the cache is neither given memory nor taken for filled (every replay would fill it
+    again, under the steps that use it); the same calls outside of it fill it."""
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    a_k, q = (torch.randn((1, 4, n, 16), generator=gen, device=DEV) for n in (3000, 1))
+    K, V = (torch.randn((1, 2, 3000, 64), generator=gen, device=DEV) for _ in range(2))
+    ws, out = ops.Workspace(), torch.empty((1, 4, 300), dtype=torch.int32, device=DEV)
+    ws.victim_cache(512)
+    ops.score_select(ws, a_k, q, 3000, 300, out=out, list_next=True)   # (its workspace is there)
+    want = out.clone()
+    sizes, alloc = [], torch.cuda.caching_allocator_alloc
+
+    def recorded(size, *a, **kw):
+        sizes.append(size)
+        return alloc(size, *a, **kw)
+    monkeypatch.setattr(torch.cuda, "caching_allocator_alloc", recorded)
+
+    def prompt():
+        ops.score_select(ws, a_k, q, 3000, 300, out=out, list_next=True)
+        ops.victim_fill(ws, K, V, 4, 3100)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        prompt()
+    assert not sizes
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    prompt()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and 4 * 512 * 32 * 16 * 5 // 4 in sizes
+
+
 @pytest.mark.parametrize("batch,hkv,l", [(1, 1, 300), (2, 3, 517), (1, 16, 1031)])
 def test_prompt_rows_in_two_copies(ops, monkeypatch, batch, hkv, l):
     """A prompt whose first heads go ahead of the others (one head: a single copy; 6 and 16: pieces of 1 + 5, 2 + 14) is
