@@ -3,12 +3,27 @@ current stream; every computation below happens in liblrqk_hip.so."""
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import Optional, Tuple
 
 import torch
 
 from . import _lib
-from ._lib import check
+
+_interrupted = threading.local()   # .raised: what ended an allocator callback of the library call under way
+
+
+def check(rc: int) -> int:
+    """The library call's result, or the exception that it stands for.  An interrupt that ended an allocator callback is
+    raised here: the library may have done without the block."""
+    raised = _interrupted.__dict__.pop("raised", None)
+    if raised is None:
+        return _lib.check(rc)
+    try:
+        _lib.check(rc)
+    except (_lib.LrqkError, ValueError) as e:
+        raise e from raised
+    raise raised
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -40,8 +55,10 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 def _torch_alloc(nbytes, stream, user):
     try:
         return torch.cuda.caching_allocator_alloc(nbytes, stream=stream or 0)
-    except BaseException:  # nothing may pass through the C frames, an interrupt included: a callback that is left by an
-        return None        # exception hands C an address that nobody wrote.  The library reports the size it did not get.
+    except BaseException as e:  # nothing may pass through the C frames, an interrupt included: a callback that is left by an
+        if user and not isinstance(e, Exception):   # exception hands C an address that nobody wrote.  The library reports
+            _interrupted.raised = e                 # the size it did not get, or does without it.
+        return None
 
 
 @_lib.RELEASE_FN
@@ -60,7 +77,7 @@ class Workspace:
         lib = _lib.load()
         check(lib.lrqk_ctx_create(ctypes.byref(self._h)))
         self._allocator = (_torch_alloc, _torch_release)  # alive as long as the ctx may call them
-        check(lib.lrqk_ctx_set_allocator(self._h, *self._allocator, None))
+        check(lib.lrqk_ctx_set_allocator(self._h, *self._allocator, self._h))
 
     @property
     def handle(self):

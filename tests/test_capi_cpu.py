@@ -122,6 +122,26 @@ def test_an_allocator_that_raises_hands_out_nothing(monkeypatch, raised):
     assert not left
 
 
+@pytest.mark.parametrize("raised", [KeyboardInterrupt, SystemExit, MemoryError])
+def test_an_interrupt_inside_the_allocator_is_not_lost(monkeypatch, raised):
+    """A call whose allocator callback was interrupted raises the interrupt also where the library went on without the
+    block (a shortage of memory is the library's to report), once; a call that failed raises its error as ever."""
+    def interrupted(*a, **kw):
+        raise raised("planted")
+    ws = ops.Workspace()
+    monkeypatch.setattr(torch.cuda, "caching_allocator_alloc", interrupted)
+    assert ws._allocator[0](64, None, ws.handle.value) is None
+    if raised is MemoryError:
+        assert ops.check(0) == 0
+    else:
+        with pytest.raises(raised, match="planted"):
+            ops.check(0)
+    assert ops.check(7) == 7
+    with pytest.raises(_lib.LrqkError, match="device memory"):
+        ws.reserve(1, 1 << 20, 16, 32, 16, 64)
+    assert ops.check(0) == 0
+
+
 @pytest.mark.parametrize("dtype,d,r,l,kernels,per_iteration", [
     (torch.bfloat16, 128, 32, 100, "pf_sums_kernel", False), (torch.bfloat16, 128, 64, 256, "pf_stream_sums_kernel", False),
     (torch.bfloat16, 64, 16, 4096, "pf_stream_sums_kernel", False), (torch.bfloat16, 64, 16, 127, "pf_pass_bf16_kernel", True),
