@@ -348,6 +348,7 @@ int score_index_prepare(lrqk_ctx* ctx, const void* a_k, int64_t head_stride, int
                      ctx->sidx_dtype == dtype && ctx->sidx_bh == bh;
   if (!bound) {
     int rc;
+    ctx->sidx_a_k = nullptr;  // (a block that grows loses what was indexed, also where the next one is not to be had)
     if ((rc = ctx->sidx_qa.ensure((size_t)bh * head_rows * r))) return rc;
     if ((rc = ctx->sidx_qs.ensure((size_t)bh * head_rows * sizeof(uint16_t)))) return rc;
     if ((rc = ctx->sidx_wm.ensure((size_t)bh * (r * r + r) * sizeof(float)))) return rc;

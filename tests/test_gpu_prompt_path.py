@@ -498,6 +498,29 @@ def test_a_selection_that_failed_leaves_no_list(ops, monkeypatch):
     assert torch.equal(ops.score_select(ws, a_k, q, 9000, 300), want)
 
 
+def test_an_index_whose_memory_was_had_in_part_is_dropped(ops, monkeypatch):
+    """The rows of a larger index are there, its scales are not to be had: the selection raises, and the next one over the
+    smaller factors, whose index went with the block that grew, indexes them again."""
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    a_k, q = (torch.randn((1, 4, n, 16), generator=gen, device=DEV) for n in (9000, 1))
+    bigger = torch.randn((1, 4, 120000, 16), generator=gen, device=DEV)
+    ws = ops.Workspace()
+    ws.score_index(True)
+    want = ops.score_select(ws, a_k, q, 9000, 300)
+    alloc, scales = torch.cuda.caching_allocator_alloc, 4 * 120000 * 2
+
+    def refused(size, *a, **kw):
+        if size == scales + scales // 4:
+            raise torch.cuda.OutOfMemoryError("planted")
+        return alloc(size, *a, **kw)
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "caching_allocator_alloc", refused)
+        with pytest.raises(Exception, match=f"no {scales + scales // 4} bytes of device memory"):
+            ops.score_select(ws, bigger, q, 120000, 300)
+    for step in range(2):
+        assert torch.equal(ops.score_select(ws, a_k, q, 9000, 300), want), step
+
+
 @pytest.mark.parametrize("refused", ["rows", "positions"])
 def test_a_prompt_does_not_fail_for_the_cache(ops, monkeypatch, refused):
     """Without memory for the victim cache (its rows; its position table) a prompt goes on, and the steps, for which there is
