@@ -14,6 +14,7 @@
 // generic VALU version for every other shape.  All write the same partial-sum layout.
 #include <algorithm>
 #include <stdlib.h>
+#include <string.h>
 #include <type_traits>
 
 #include "common.hpp"
@@ -1381,7 +1382,7 @@ __global__ __launch_bounds__(kPfWideThreads, 4) void pf_pass_wide_kernel(const f
 }
 
 // The stages of pf_small_generic_kernel for 32 < r <= 64 and d <= 128, with its operations in its order (same results to
-// the bit): wave w keeps rows 8 w .. 8 w + 7 of [G | RHS] in registers, lane and column lane + 64 k; a pivot row goes
+// the bit; the sums of the stopping test alone are taken in another order, by all threads instead of one): wave w keeps rows 8 w .. 8 w + 7 of [G | RHS] in registers, lane and column lane + 64 k; a pivot row goes
 // round through LDS, one barrier per pivot (two slots).  Workgroup (h, 0): B_Q (stages 0 and 2), then Mt; (h, 1): B_K.
 // A dependent chain of 0.2 us a pivot: 24 heads, rank 64: 947 -> 104 us a stage (median).
 constexpr int kPfWideLdb = 128 + 20;
@@ -1594,8 +1595,11 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
   // fp32 rows stay with the row-by-row formulation.  Its factors are 5e-6 .. 8e-5 off the ones from Gram matrices, and a
   // decode step of an ill-conditioned head makes up to 4e-4 of that (a token at the edge of the active set changes
   // places): more than fp32 results may move, whichever side is the closer one.
+  // LRQK_PREFILL_ROWWISE, for comparisons: every prompt row by row; `general`: ranks above 32 by the general kernels
+  const char* const rowwise = getenv("LRQK_PREFILL_ROWWISE");
+  const bool general = rowwise && !strcmp(rowwise, "general");
   if constexpr (sizeof(T) == 2) {
-    const bool gram_domain = aligned && (d == 64 || d == 128) && !getenv("LRQK_PREFILL_ROWWISE") &&
+    const bool gram_domain = aligned && (d == 64 || d == 128) && !rowwise &&
                              ((d == 128 && r <= 32) || l >= 2 * d);
     if (gram_domain)
       return prefill_gram_domain(ctx, (const T*)q, (const T*)k, a_q, a_k, out, b, hq, hkv, l, r, d, iters, tol, st);
@@ -1654,7 +1658,7 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
     }
   }
   auto small = !small32 ? pf_small_generic_kernel : r <= 16 ? pf_small32_kernel<16> : pf_small32_kernel<32>;
-  const bool wide = sizeof(T) == 4 && r > 32 && r <= 64 && (d == 64 || d == 128) && aligned;
+  const bool wide = sizeof(T) == 4 && r > 32 && r <= 64 && (d == 64 || d == 128) && aligned && !general;
   if constexpr (sizeof(T) == 4) {
     if (wide) {
       pass = d == 64 ? pf_pass_wide_kernel<64> : pf_pass_wide_kernel<128>;
@@ -1662,7 +1666,7 @@ static int prefill_impl(lrqk_ctx* ctx, const void* q, const void* k, float* a_q,
       smem_pass = (size_t)(32 * (d + 20) + 32 * kPfWideLda + 64 * (d + 20)) * sizeof(float);
     }
   }
-  const bool small_wide = r > 32 && r <= 64 && d <= 128;
+  const bool small_wide = r > 32 && r <= 64 && d <= 128 && !general;
   if (small_wide) small = pf_small_wide_kernel;
   const size_t smem_small = small_wide ? 0 : small32 ? ((size_t)3 * ne + 4 + (size_t)r * (d + 4)) * sizeof(float)
                                     : ((size_t)ne + (size_t)r * (r + d + 1) + (size_t)r * (d + 1)) * sizeof(float);
