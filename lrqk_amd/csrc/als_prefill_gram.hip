@@ -1378,12 +1378,13 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
                         : hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
-  // In slices while a launch of an iteration has few workgroups per CU (96 heads of 128 at ranks to 32, 64 above): four
-  // iterations, the whole fit of 8192 rows of 32 heads 313 -> 258 us at rank 32 and 681 -> 492 at rank 64; 64 heads 295 ->
-  // 271 and 632 -> 606; 96 heads 262 -> 250 and 689 -> 708; 128 heads 359 -> 396 and 760 -> 1000 (what the slices repeat
-  // then costs more than idle CUs do); d = 64: 32 heads 170 -> 145, 96 heads 156 -> 151.  Ranks up to 16: an iteration
-  // whole takes 16 .. 24 us, two launches as long.
-  const bool slices = RP > 16 && (int64_t)bh * (d / 32 + 1) <= (RP == 32 ? 480 : 320);
+  // In slices while a launch of an iteration has few workgroups per CU; with more, what the slices repeat costs more than
+  // idle CUs do (a launch is rounded up to 8 heads).  The whole fit of 4096 rows with four iterations, whole -> in
+  // slices, us:  d = 128, ranks to 32: 48 heads 282 -> 231, 64 303 -> 286, 72 321 -> 326, 96 360 -> 371;  above: 48 heads
+  // 622 -> 448, 64 664 -> 657, 72 696 -> 722, 96 758 -> 798;  d = 64, ranks to 32: 64 heads 188 -> 163, 112 222 -> 216, 128 238 ->
+  // 238, 144 261 -> 281;  above: 80 heads 460 -> 370, 88 497 -> 507, 106 518 -> 543.  Ranks up to 16: an iteration whole
+  // takes 16 .. 24 us, two launches as long.
+  const bool slices = RP > 16 && bh <= (d == 128 ? 64 : RP == 32 ? 112 : 80);
   const size_t g_parts = slices ? d / 32 : 1;
   const size_t n_state = slices ? (size_t)bh * 2 * (RP * d + RP * RP)
                                 : (size_t)bh * RP * d + (RP == 64 ? (size_t)bh * 2 * RP * (RP + 1) : 0);
@@ -1451,8 +1452,8 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   if (slices)
     rc = d == 64 ? (RP == 32 ? LRQK_GS_RUN(2, 64) : LRQK_GS_RUN(4, 64)) : (RP == 32 ? LRQK_GS_RUN(2, 128) : LRQK_GS_RUN(4, 128));
   else
-  rc = d == 64 ? (RP == 16 ? LRQK_GD_RUN(1, 64) : RP == 32 ? LRQK_GD_RUN(2, 64) : LRQK_GD_RUN(4, 64))
-               : (RP == 16 ? LRQK_GD_RUN(1, 128) : RP == 32 ? LRQK_GD_RUN(2, 128) : LRQK_GD_RUN(4, 128));
+    rc = d == 64 ? (RP == 16 ? LRQK_GD_RUN(1, 64) : RP == 32 ? LRQK_GD_RUN(2, 64) : LRQK_GD_RUN(4, 64))
+                 : (RP == 16 ? LRQK_GD_RUN(1, 128) : RP == 32 ? LRQK_GD_RUN(2, 128) : LRQK_GD_RUN(4, 128));
 #undef LRQK_GD_RUN
 #undef LRQK_GS_RUN
   if (rc) return rc;

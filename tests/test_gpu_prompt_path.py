@@ -232,11 +232,13 @@ def test_fit_on_gram_matrices(ops, oracle, dtype, d, r, l, hq, hkv, iters):
 
 
 @pytest.mark.parametrize("d,r,heads,tol", [(64, 17, 160, 0.0), (64, 32, 161, 0.0), (128, 32, 96, 0.0), (128, 24, 97, 0.0),
-                                           (128, 33, 64, 0.0), (128, 64, 65, 0.0), (64, 64, 1, 0.0), (128, 32, 9, 1e30)])
+                                           (128, 33, 64, 0.0), (128, 64, 65, 0.0), (64, 64, 1, 0.0), (128, 32, 9, 1e30),
+                                           (64, 17, 112, 0.0), (64, 32, 113, 0.0), (64, 33, 80, 0.0), (64, 40, 81, 0.0),
+                                           (128, 32, 64, 0.0), (128, 24, 65, 0.0)])
 def test_fit_in_slices_and_whole(ops, oracle, d, r, heads, tol):
-    """The iteration in slices of a head's columns (up to 96 heads of 128 and 160 of 64 at ranks to 32, 64 heads of 128
-    above; head counts that are no multiple of the XCDs) and whole (one head more), and a fit that stops at its second iteration: against the oracle in fp64, with
-    the limit of the test above."""
+    """The iteration in slices of a head's columns (up to 64 heads of 128; of 64 up to 112 at ranks to 32, 80 above; head
+    counts that are no multiple of the XCDs) and whole (one head more), and a fit that stops at its second iteration:
+    against the oracle in fp64, with the limit of the test above."""
     gen = torch.Generator().manual_seed(heads + r)
     from lrqk_amd import synth
     l = 2 * d + 5
