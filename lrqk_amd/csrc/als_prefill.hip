@@ -1382,8 +1382,9 @@ __global__ __launch_bounds__(kPfWideThreads, 4) void pf_pass_wide_kernel(const f
 }
 
 // The stages of pf_small_generic_kernel for 32 < r <= 64 and d <= 128, with its operations in its order (same results to
-// the bit; the sums of the stopping test alone are taken in another order, by all threads instead of one): wave w keeps rows 8 w .. 8 w + 7 of [G | RHS] in registers, lane and column lane + 64 k; a pivot row goes
-// round through LDS, one barrier per pivot (two slots).  Workgroup (h, 0): B_Q (stages 0 and 2), then Mt; (h, 1): B_K.
+// the bit; the sums of the stopping test alone are taken in another order, by all threads instead of one): wave w keeps
+// rows 8 w .. 8 w + 7 of [G | RHS] in registers, lane and column lane + 64 k; a pivot row goes round through LDS, one
+// barrier per pivot (two slots).  Workgroup (h, 0): B_Q (stages 0 and 2), then Mt; (h, 1): B_K.
 // A dependent chain of 0.2 us a pivot: 24 heads, rank 64: 947 -> 104 us a stage (median).
 constexpr int kPfWideLdb = 128 + 20;
 __global__ __launch_bounds__(kPfWideThreads, 2) void pf_small_wide_kernel(

@@ -1379,11 +1379,11 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
                         : hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
   // In slices while a launch of an iteration has few workgroups per CU; with more, what the slices repeat costs more than
-  // idle CUs do (a launch is rounded up to 8 heads).  The whole fit of 4096 rows with four iterations, whole -> in
-  // slices, us:  d = 128, ranks to 32: 48 heads 282 -> 231, 64 303 -> 286, 72 321 -> 326, 96 360 -> 371;  above: 48 heads
-  // 622 -> 448, 64 664 -> 657, 72 696 -> 722, 96 758 -> 798;  d = 64, ranks to 32: 64 heads 188 -> 163, 112 222 -> 216, 128 238 ->
-  // 238, 144 261 -> 281;  above: 80 heads 460 -> 370, 88 497 -> 507, 106 518 -> 543.  Ranks up to 16: an iteration whole
-  // takes 16 .. 24 us, two launches as long.
+  // idle CUs do (a launch is rounded up to 8 heads).  The fit of 4096 rows with four iterations, whole -> in slices, us:
+  // d = 128, ranks to 32: 48 heads 282 -> 231, 64 303 -> 286, 72 321 -> 326, 96 360 -> 371;  above: 48 heads 622 -> 448, 64
+  // 664 -> 657, 72 696 -> 722, 96 758 -> 798;  d = 64, ranks to 32: 64 heads 188 -> 163, 112 222 -> 216, 128 238 -> 238, 144
+  // 261 -> 281;  above: 80 heads 460 -> 370, 88 497 -> 507, 106 518 -> 543.  Ranks up to 16: an iteration whole takes
+  // 16 .. 24 us, two launches as long.
   const bool slices = RP > 16 && bh <= (d == 128 ? 64 : RP == 32 ? 112 : 80);
   const size_t g_parts = slices ? d / 32 : 1;
   const size_t n_state = slices ? (size_t)bh * 2 * (RP * d + RP * RP)

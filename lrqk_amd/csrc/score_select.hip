@@ -1521,13 +1521,10 @@ constexpr int kCalmCalls = 32;  // usable lists in a row before a head's slack i
 // ones, and the same instructions took 11.2 .. 11.8 us (32 heads x 32K rows) and 15.1 .. 16.2 (256 x 128K) by their address,
 // which moves with every other kernel of this file.  On multiples of 8 KB 11.3 and 15.4, of 64 KB 11.7 and 15.7.
 template <typename T, int R>
-__global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void select_step_kernel(const uint2* __restrict__ cand_all, int cand_cap,
-                                                                  SelState st, uint32_t* __restrict__ keys_all,
-                                                                  int64_t key_stride, const T* __restrict__ a_k,
-                                                                  int64_t head_stride, const T* __restrict__ q_hat,
-                                                                  int64_t m, int r, int round_bf16, int k,
-                                                                  int32_t* __restrict__ out_all, int64_t out_stride,
-                                                                  DiffArgs df) {
+__global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void select_step_kernel(
+    const uint2* __restrict__ cand_all, int cand_cap, SelState st, uint32_t* __restrict__ keys_all, int64_t key_stride,
+    const T* __restrict__ a_k, int64_t head_stride, const T* __restrict__ q_hat, int64_t m, int r, int round_bf16, int k,
+    int32_t* __restrict__ out_all, int64_t out_stride, DiffArgs df) {
   LRQK_SEL_LDS(L);
   const int h = blockIdx.x;
   const int n = __builtin_amdgcn_readfirstlane(st.cand_count[h * kCountStride]);

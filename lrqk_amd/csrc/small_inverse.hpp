@@ -35,10 +35,11 @@ __device__ __forceinline__ float half_pair(float lo_src, float hi_src, int hp) {
 // algebraically equal update with the inverse of the 2 x 2 pivot block loses digits when that block is nearly
 // singular; this form is the two sweeps themselves.)  An odd r ends with a sweep on one pivot.  B_p = d - 1
 // cancels badly for large d, so the matrix is first scaled to unit diagonal (then every pivot is <= 1); the
-// scaling is undone on the way out.  Rows and columns >= r are an identity block and are skipped.
+// scaling is undone on the way out.  Rows and columns >= r form an identity block.
 // g(i, j) returns element (i, j); sbuf: 32 floats of LDS owned by this wave; inv: [32][kLdi].
 // PIVOTS (16 or 32, at least r): an even r sweeps that many without a test -- pivots of the identity block change nothing.
-// Behind a test per pair the compiler copies the accumulators twice per pair (r 16, eight iterations: 12.8 -> 10.4 us of the solve with the shorter products below; r 32: 0.1 us).
+// Behind a test per pair the compiler copies the accumulators twice per pair (r 16, eight iterations: 12.8 -> 10.4 us of
+// the solve, together with the iterations' vectors of 16 instead of 32 elements; r 32: 0.1 us).
 template <int PIVOTS, bool ODD, typename GetG>
 __device__ __forceinline__ void invert_sweep_mfma(GetG&& g, int r, float* sbuf, float* inv) {
   const int lane = lane_id();
