@@ -10,13 +10,15 @@ import torch
 
 from . import _lib
 
-_interrupted = threading.local()   # .raised: what ended an allocator callback of the library call under way
+_interrupted = {}   # by thread: what ended an allocator callback of the library call under way
 
 
 def check(rc: int) -> int:
     """The library call's result, or the exception that it stands for.  An interrupt that ended an allocator callback is
     raised here: the library may have done without the block."""
-    raised = _interrupted.__dict__.pop("raised", None)
+    if rc >= 0 and not _interrupted:   # (a prompt makes some thirty calls)
+        return rc
+    raised = _interrupted.pop(threading.get_ident(), None)
     if raised is None:
         return _lib.check(rc)
     try:
@@ -57,7 +59,7 @@ def _torch_alloc(nbytes, stream, user):
         return torch.cuda.caching_allocator_alloc(nbytes, stream=stream or 0)
     except BaseException as e:  # nothing may pass through the C frames, an interrupt included: a callback that is left by an
         if user and not isinstance(e, Exception):   # exception hands C an address that nobody wrote.  The library reports
-            _interrupted.raised = e                 # the size it did not get, or does without it.
+            _interrupted[threading.get_ident()] = e  # the size it did not get, or does without it.
         return None
 
 
