@@ -111,8 +111,14 @@ __device__ __forceinline__ void als_index_append_body(const FinishArgs& fa, int 
 // One workgroup (kFinThreads threads) per head h: batch-wide stopping decision, line-search update
 // of B_Q and B_K (held in registers as 16-byte vectors: vector vi = tid + 256 u covers row
 // vi >> vshift, columns (vi & (vpr-1)) * VEC ..), rounded q_hat / k_hat outputs, k_hat -> A_K row.
-template <typename T>
-__device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
+struct FinLds {
+  float hat[2][kFinMaxR];
+  float err[2][256];
+  float red[kFinThreads / kWave][2][256];
+};
+// MV: vectors per thread and matrix.
+template <typename T, int MV>
+__device__ __forceinline__ void als_finish_body_mv(const FinishArgs& fa, int h, FinLds& L) {
   T* __restrict__ b_q = (T*)fa.b_q;
   T* __restrict__ b_k = (T*)fa.b_k;
   const T* __restrict__ q = (const T*)fa.q;
@@ -126,33 +132,43 @@ __device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
   T* __restrict__ a_k = (T*)fa.a_k;
   const int64_t head_stride = fa.head_stride, append_row = fa.append_row;
   constexpr int VEC = Vec16<T>::N;
-  constexpr int kMaxVec = 8;  // vectors per thread per matrix: r * d / VEC <= 2048
-  __shared__ float hat[2][kFinMaxR];
-  __shared__ float err[2][256];
-  __shared__ float red[kFinThreads / kWave][2][256];
-  __shared__ int s_it;
+  auto& hat = L.hat;
+  auto& err = L.err;
+  auto& red = L.red;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int b = h / hq, head = h % hq;
   const int kvh = head / (hq / hkv);
   const int vpr = 1 << vshift;  // vectors per row, a power of two <= 64
   const int nvec = r << vshift;
   // B tiles -> registers (independent loads, issued first)
-  Vec16<T> vq[kMaxVec], vk[kMaxVec];
+  Vec16<T> vq[MV], vk[MV];
 #pragma unroll
-  for (int u = 0; u < kMaxVec; ++u) {
+  for (int u = 0; u < MV; ++u) {
     const int vi = min(tid + u * kFinThreads, nvec - 1);
     vq[u].load(b_q + (int64_t)h * r * d + (int64_t)vi * VEC);
     vk[u].load(b_k + (int64_t)h * r * d + (int64_t)vi * VEC);
   }
   const float qreg = ld_f32<T>(q, (int64_t)h * d + min(tid, d - 1));
   const float kreg = ld_f32<T>(k_new, ((int64_t)b * hkv + kvh) * d + min(tid, d - 1));
-  if (wave == 0) {
+  // Every wave decides for itself, with the iterates on their way: behind wave 0's decision the chosen one was a barrier and
+  // a round trip to memory more.
+  constexpr int kAhead = 8;
+  float hat_mine;
+  if (max_iter <= kAhead) {  // (uniform)
+    float sacc[kAhead], cand[kAhead];
+    als_delta_sums<kAhead>(deltas, bh, max_iter, sacc);
+#pragma unroll
+    for (int it = 0; it < kAhead; ++it)
+      cand[it] = iter_out[((int64_t)h * max_iter + min(it, max_iter - 1)) * 2 * r + min(tid, 2 * r - 1)];
+    const int chosen = als_decide<kAhead>(sacc, bh, max_iter, r, tol);
+    hat_mine = cand[0];
+#pragma unroll
+    for (int it = 1; it < kAhead; ++it) hat_mine = chosen == it ? cand[it] : hat_mine;
+  } else {
     const int chosen = als_choose_iterate(deltas, bh, max_iter, r, tol);
-    if (lane == 0) s_it = chosen;
+    hat_mine = iter_out[((int64_t)h * max_iter + chosen) * 2 * r + min(tid, 2 * r - 1)];
   }
-  __syncthreads();
-  const float* o = iter_out + ((int64_t)h * max_iter + s_it) * 2 * r;
-  if (tid < 2 * r) hat[tid >= r ? 1 : 0][tid >= r ? tid - r : tid] = o[tid];
+  if (tid < 2 * r) hat[tid >= r ? 1 : 0][tid >= r ? tid - r : tid] = hat_mine;
   __syncthreads();
   // column sums  sum_i hat[i] B[i][c]  for this thread's column group, both matrices
   const int cg = tid & (vpr - 1);  // vpr divides 256, so the column group is fixed per thread
@@ -160,7 +176,7 @@ __device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
 #pragma unroll
   for (int e = 0; e < VEC; ++e) pq[e] = pk[e] = 0.0f;
 #pragma unroll
-  for (int u = 0; u < kMaxVec; ++u) {
+  for (int u = 0; u < MV; ++u) {
     const int vi = tid + u * kFinThreads;
     if (vi < nvec) {
       const int row = vi >> vshift;
@@ -206,26 +222,26 @@ __device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
   }
   en0 = wave_sum(en0);
   en1 = wave_sum(en1);
+  static_assert(kFinMaxR <= kWave, "a lane per element of the iterates");
+  const float hx = lane < r ? hat[0][lane] : 0.0f, hy = lane < r ? hat[1][lane] : 0.0f;
+  const float hnq = wave_sum(hx * hx), hnk = wave_sum(hy * hy);
   __syncthreads();  // everyone is done reading red
   if (lane == 0) {
     red[wave][0][0] = en0;
     red[wave][1][0] = en1;
   }
   __syncthreads();
-  float e2q = 0.0f, e2k = 0.0f, hnq = 0.0f, hnk = 0.0f;
+  float e2q = 0.0f, e2k = 0.0f;
+#pragma unroll
   for (int w = 0; w < kFinThreads / kWave; ++w) {
     e2q += red[w][0][0];
     e2k += red[w][1][0];
-  }
-  for (int i = 0; i < r; ++i) {
-    hnq = fmaf(hat[0][i], hat[0][i], hnq);
-    hnk = fmaf(hat[1][i], hat[1][i], hnk);
   }
   // dB = hat^T e : |dB|^2 = |hat|^2 |e|^2 ; hat dB = |hat|^2 e : |hat dB|^2 = |hat|^4 |e|^2
   const float lrq = (hnq * e2q) / (hnq * hnq * e2q + 1e-6f);
   const float lrk = (hnk * e2k) / (hnk * hnk * e2k + 1e-6f);
 #pragma unroll
-  for (int u = 0; u < kMaxVec; ++u) {
+  for (int u = 0; u < MV; ++u) {
     const int vi = tid + u * kFinThreads;
     if (vi < nvec) {
       const int row = vi >> vshift;
@@ -251,6 +267,20 @@ __device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
     st_f32<T>(k_hat_out, (int64_t)h * r + tid, hat[1][tid]);
     if (append_row >= 0) st_f32<T>(a_k, (int64_t)h * head_stride + append_row * r + tid, hat[1][tid]);
   }
+}
+
+// As many vectors as the sizes need (r * d / VEC <= 2048 of them): with eight at every size the registers did not hold them
+// beside the iterates, and the first ones were waited for, to be spilled, before anything else was asked for.
+template <typename T>
+__device__ __forceinline__ void als_finish_body(const FinishArgs& fa, int h) {
+  __shared__ FinLds L;
+  const int nvec = fa.r << fa.vshift;
+  if (nvec <= 2 * kFinThreads)  // (uniform)
+    als_finish_body_mv<T, 2>(fa, h, L);
+  else if (nvec <= 4 * kFinThreads)
+    als_finish_body_mv<T, 4>(fa, h, L);
+  else
+    als_finish_body_mv<T, 8>(fa, h, L);
 }
 
 }  // namespace lrqk

@@ -117,19 +117,29 @@ __device__ __forceinline__ void attn_scan_w(const float* __restrict__ w, float s
     // that condition, where it becomes a branch with a full wait per row group)
 #pragma unroll
     for (int u = 0; u < U; ++u) asm volatile("" : "+v"(wl[u]));
+    // One maximum and one rescaling per batch: the workgroups of the launch that this runs in keep every SIMD's issue busy, and
+    // a maximum, two exponentials and a rescaled accumulator per row were most of what this role issued.
+    float m_new = st.m;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      wl[u] = ok[u] ? wl[u] * scale_log2e : -INFINITY;
+      m_new = fmaxf(m_new, wl[u]);
+    }
+    const float m_use = m_new == -INFINITY ? 0.0f : m_new;  // (nothing valid yet: every exponent is -inf, every weight 0)
+    const float alpha = exp2f(st.m - m_use);
+    st.l *= alpha;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) st.acc[e] *= alpha;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       float vf[VEC];
       vv[u].unpack(vf);
-      const float sc = ok[u] ? wl[u] * scale_log2e : -INFINITY;
-      const float m_new = fmaxf(st.m, sc);
-      const float alpha = (m_new == -INFINITY) ? 0.0f : exp2f(st.m - m_new);
-      const float p = (m_new == -INFINITY) ? 0.0f : exp2f(sc - m_new);
-      st.l = st.l * alpha + p;
+      const float p = exp2f(wl[u] - m_use);
+      st.l += p;
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) st.acc[e] = st.acc[e] * alpha + p * vf[e];
-      st.m = m_new;
+      for (int e = 0; e < VEC; ++e) st.acc[e] = fmaf(p, vf[e], st.acc[e]);
     }
+    st.m = m_new;
   }
 }
 
@@ -255,12 +265,18 @@ __global__ __launch_bounds__(kAttnThreads) void attn_partial_kernel(const T* __r
 // the registers of its 2*cpr lanes (cpr K chunks, then cpr V chunks) the lanes also form the row's
 // attention term, so the refetched slots never have to be read again.  The workgroup's rows are
 // merged into one (max, sum, acc) triple at `pout` (an empty triple if it had no row).
+// Bound by the instructions that it issues as much as by its round trips (four workgroups of the launch share a CU, a wave
+// gets every fourth turn of its SIMD): what is the same for a head is in scalar registers and offsets have 32 bits, a
+// workgroup beyond the head's misses leaves at once, and a second row per lane group is handled only where there is one.
+// With that, the roles beside it made shorter and nothing waited for behind the host link but the rows themselves, the launch
+// went 15.1 -> 12.6 us (32 heads x 128K, r 32, k 2048), 36.7 -> 33.3 (128 heads), 10.5 -> 7.6 (28 fp32 heads x 4K, k 512) and
+// 21.1 -> 19.0 (r 64, k 4096).
 template <typename T>
 __device__ __forceinline__ void fetch_rows_attn_body(const uint4* __restrict__ store, int64_t cap,
                                                      uint4* __restrict__ k_act, uint4* __restrict__ v_act, int n_slots,
                                                      const int32_t* __restrict__ hit, int64_t hit_stride,
                                                      const int32_t* __restrict__ miss_slots,
-                                                     const int32_t* __restrict__ miss_count, int hq, int hkv, int cpr,
+                                                     const int32_t* __restrict__ miss_count, int group, int lpr_log2,
                                                      int k, int h, int blk, int nblk, const T* __restrict__ q, int d,
                                                      float scale_log2e, float* __restrict__ pout,
                                                      const int32_t* __restrict__ miss_old, const VictimView& vic,
@@ -269,151 +285,169 @@ __device__ __forceinline__ void fetch_rows_attn_body(const uint4* __restrict__ s
   constexpr int VEC = Vec16<T>::N;
   __shared__ float accs[8][256 + 2];               // [row group][m, l, acc[d]] (at most 8 groups are merged at a time)
   const int tid = threadIdx.x, lane = lane_id();
-  const int cnt = miss_count[h];
-  const int chunks = 2 * cpr;  // per store row; a power of two <= 64 here
-  const int rpb = kAttnThreads / chunks;
-  const int b = h / hq, head = h % hq;
-  const int kvh = head / (hq / hkv);
-  const int jl = tid / chunks, c = tid % chunks;
+  const int cl2 = lpr_log2 + 1;                    // a store row has 2^cl2 <= 64 chunks of 16 bytes
+  const int chunks = 1 << cl2, cpr = 1 << lpr_log2;
+  const int rpb = kAttnThreads >> cl2;
+  const int jl = tid >> cl2, c = tid & (chunks - 1);
   const bool is_k = c < cpr;
-  float qf[VEC];
-  {
-    Vec16<T> qv;
-    qv.load(q + (int64_t)h * d + (is_k ? c : 0) * VEC);
-    qv.unpack(qf);
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) qf[e] *= scale_log2e;
-  }
-  AttnAcc<VEC> st;  // meaningful in the V lanes
-  st.init();
   const int nv = vic.nv;  // uniform
-  const int vbase = nv > 0 ? vic.base[h] : 0;
+  const int32_t* slots_h = miss_slots + (int64_t)h * k;
+  const int32_t* new_h = miss_new ? miss_new + (int64_t)h * k : nullptr;
+  const int32_t* old_h = nv > 0 ? miss_old + (int64_t)h * k : slots_h;
   // Every load is unconditional (clamped index, valid address) so that the loads of one stage go out
   // together: j -> (slot, token, previous token) -> FIFO positions -> row (+ FIFO tags) -> stores.
-  // A lane group handles kFR rows per trip, stage by stage, so that one trip covers the usual number of misses.
+  // A lane group handles up to kFR rows per trip, stage by stage, so that one trip covers the usual number of misses.
   constexpr int kFR = 2;
-  const int per_trip = kFR * nblk * rpb;
-  for (int it = 0;; ++it) {
-    int j[kFR], slot[kFR];
-    int32_t tok[kFR], old[kFR];
+  const int pass = nblk * rpb;
+  const int j0 = blk * rpb + jl;
+  int slot[kFR];
+  int32_t tok[kFR], old[kFR];
+  auto lists = [&](int first) {
 #pragma unroll
     for (int u = 0; u < kFR; ++u) {
-      j[u] = blk * rpb + jl + (it * kFR + u) * nblk * rpb;
-      const int jc = min(j[u], k - 1);
-      slot[u] = miss_slots[(int64_t)h * k + jc];
-      tok[u] = miss_new ? miss_new[(int64_t)h * k + jc] : 0;
-      old[u] = nv > 0 ? miss_old[(int64_t)h * k + jc] : -1;
+      const uint32_t jc = (uint32_t)min(first + u * pass, k - 1);
+      slot[u] = slots_h[jc];
+      tok[u] = new_h ? new_h[jc] : 0;
+      old[u] = old_h[jc];
     }
-    const int trips = (cnt + per_trip - 1) / per_trip;  // uniform over the workgroup (first use of cnt)
-    if (it >= trips) break;
-    bool ok[kFR];
-    int64_t dst[kFR];
-    const uint4* host_src[kFR];
-    const uint4* own[kFR];
+  };
+  lists(j0);  // (in front of the count's first use)
+  Vec16<T> qv;
+  qv.load(q + (int64_t)h * d + (is_k ? c : 0) * VEC);
+  const int vbase = nv > 0 ? __builtin_amdgcn_readfirstlane(vic.base[h]) : 0;
+  const int cnt = __builtin_amdgcn_readfirstlane(miss_count[h]);
+  if (blk * rpb >= cnt) {  // no row: an empty triple
+    for (int t = tid; t < d + 2; t += kAttnThreads) pout[t] = t == 0 ? -INFINITY : 0.0f;
+    return;
+  }
+  float qf[VEC];
+  qv.unpack(qf);
 #pragma unroll
-    for (int u = 0; u < kFR; ++u) {
-      ok[u] = j[u] < cnt && slot[u] >= 0 && slot[u] < k;
+  for (int e = 0; e < VEC; ++e) qf[e] *= scale_log2e;
+  AttnAcc<VEC> st;  // meaningful in the V lanes
+  st.init();
+  const int vcap = (int)min(vic.cap, (int64_t)INT32_MAX);
+  const uint4* store_h = store + ((int64_t)(h / group) * cap << cl2) + c;
+  uint4* own_h = (is_k ? k_act + c : v_act + (c - cpr)) + ((int64_t)h * n_slots << lpr_log2);
+  uint4* rows_h = vic.rows + ((int64_t)h * nv << cl2);
+  int32_t* tags_h = vic.tok + (int64_t)h * nv;
+  int16_t* pos_h = vic.pos + (int64_t)h * vic.cap;
+  const int n_ins = min(cnt, nv);
+
+  auto trip = [&](auto nr_c, int first) {
+    constexpr int NR = decltype(nr_c)::value;
+    bool ok[NR];
+    const uint4* host_src[NR];
+    uint4* own[NR];
+    uint4 val[NR];
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      ok[u] = first + u * pass < cnt && slot[u] >= 0 && slot[u] < k;
       slot[u] = ok[u] ? slot[u] : 0;
-    }
-    if (!miss_new) {
-#pragma unroll
-      for (int u = 0; u < kFR; ++u) tok[u] = hit[(int64_t)h * hit_stride + slot[u]];
-    }
-#pragma unroll
-    for (int u = 0; u < kFR; ++u) {
+      if (!new_h) tok[u] = hit[(int64_t)h * hit_stride + slot[u]];
       ok[u] = ok[u] && tok[u] >= 0 && tok[u] < cap;
       tok[u] = ok[u] ? tok[u] : 0;
-      dst[u] = ((int64_t)h * n_slots + slot[u]) * cpr;
-      host_src[u] = store + (((int64_t)b * hkv + kvh) * cap + tok[u]) * chunks + c;
+      host_src[u] = store_h + ((int64_t)tok[u] << cl2);
       // a lane without a row reads a device address (its own slot), never the host store
-      own[u] = is_k ? k_act + dst[u] + c : v_act + dst[u] + (c - cpr);
+      own[u] = own_h + ((uint32_t)slot[u] << lpr_log2);
     }
-    uint4 val[kFR];
     if (nv > 0) {
       // Victim cache.  The row that leaves the slot goes to FIFO position base + j (unless the
       // cache still holds it); the row that enters is taken from the FIFO if it is there and
       // not being replaced in this very step.  All reads of the metadata come before the writes,
       // and a row's lanes share one wave, so they decide alike.
-      const int n_ins = min(cnt, nv);
-      int p_ins[kFR], q_old[kFR], p_new[kFR];
-      bool do_ins[kFR], old_cached[kFR], from_fifo[kFR];
+      // Three dependent round trips, each stage's requests together: the lists; FIFO positions, outgoing rows and the tags that
+      // they will replace; tags, then the incoming rows.  What comes back is waited for in order, so the rows, which may come
+      // over the host link, are requested last and everything else is done while they are on their way.
+      int p_ins[NR], q_old[NR], p_new[NR], prev_pos[NR];
+      bool do_ins[NR], old_cached[NR], from_fifo[NR];
+      uint4 old_val[NR];
+      int32_t tag_new[NR], tag_old[NR], prev[NR];
 #pragma unroll
-      for (int u = 0; u < kFR; ++u) {
-        p_ins[u] = (vbase + min(j[u], k - 1)) % nv;
-        do_ins[u] = ok[u] && j[u] < nv && old[u] >= 0 && old[u] < vic.cap;
-        q_old[u] = vic.pos[(int64_t)h * vic.cap + (do_ins[u] ? old[u] : 0)];
-        p_new[u] = vic.pos[(int64_t)h * vic.cap + (tok[u] < vic.cap ? tok[u] : 0)];
-      }
-      uint4 old_val[kFR];
-      int32_t tag_new[kFR], tag_old[kFR], prev[kFR];
-#pragma unroll
-      for (int u = 0; u < kFR; ++u) {
-        old_cached[u] = do_ins[u] && q_old[u] >= 0 && q_old[u] < nv && !victim_slot_in_flight(q_old[u], vbase, n_ins, nv);
-        from_fifo[u] = ok[u] && tok[u] < vic.cap && p_new[u] >= 0 && p_new[u] < nv &&
-                       !victim_slot_in_flight(p_new[u], vbase, n_ins, nv);
-        // the row is requested from where the position table points; the tags confirm it afterwards
-        const uint4* src = from_fifo[u] ? vic.rows + ((int64_t)h * nv + p_new[u]) * chunks + c : (ok[u] ? host_src[u] : own[u]);
-        val[u] = *src;
+      for (int u = 0; u < NR; ++u) {
+        const int j = first + u * pass;
+        p_ins[u] = vbase + min(j, nv - 1);  // (rows from nv on are not kept)
+        p_ins[u] = p_ins[u] >= nv ? p_ins[u] - nv : p_ins[u];
+        do_ins[u] = ok[u] && j < nv && old[u] >= 0 && old[u] < vcap;
+        q_old[u] = pos_h[(uint32_t)(do_ins[u] ? old[u] : 0)];
+        p_new[u] = pos_h[(uint32_t)(tok[u] < vcap ? tok[u] : 0)];
+        prev[u] = tags_h[(uint32_t)p_ins[u]];
         old_val[u] = *own[u];
-        tag_new[u] = vic.tok[(int64_t)h * nv + (from_fifo[u] ? p_new[u] : 0)];
-        tag_old[u] = vic.tok[(int64_t)h * nv + (old_cached[u] ? q_old[u] : 0)];
-        prev[u] = vic.tok[(int64_t)h * nv + p_ins[u]];
       }
-      int prev_pos[kFR];
 #pragma unroll
-      for (int u = 0; u < kFR; ++u) {
+      for (int u = 0; u < NR; ++u) {
+        old_cached[u] = do_ins[u] && q_old[u] >= 0 && q_old[u] < nv && !victim_slot_in_flight(q_old[u], vbase, n_ins, nv);
+        from_fifo[u] = ok[u] && tok[u] < vcap && p_new[u] >= 0 && p_new[u] < nv &&
+                       !victim_slot_in_flight(p_new[u], vbase, n_ins, nv);
+        tag_new[u] = tags_h[(uint32_t)(from_fifo[u] ? p_new[u] : 0)];
+        tag_old[u] = tags_h[(uint32_t)(old_cached[u] ? q_old[u] : 0)];
+        const bool named = do_ins[u] && prev[u] >= 0 && prev[u] < vcap;
+        prev_pos[u] = pos_h[(uint32_t)(named ? prev[u] : 0)];
+        prev_pos[u] = named ? prev_pos[u] : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        // the row is requested from where the position table points; the tags confirm it afterwards
+        const uint4* src = from_fifo[u] ? rows_h + (((uint32_t)p_new[u] << cl2) + c) : (ok[u] ? host_src[u] : own[u]);
+        val[u] = *src;
+      }
+#pragma unroll
+      for (int u = 0; u < NR; ++u) {
+        // (used by some lanes only: the compiler would move the requests behind the tests, and the tests behind the rows)
+        asm volatile("" : "+v"(old_val[u].x), "+v"(old_val[u].y), "+v"(old_val[u].z), "+v"(old_val[u].w), "+v"(prev_pos[u]));
         if (old_cached[u] && tag_old[u] == old[u]) do_ins[u] = false;
         if (from_fifo[u] && tag_new[u] != tok[u]) {  // (the table and the tags disagree: take the row from the store)
           from_fifo[u] = false;
           val[u] = *host_src[u];
         }
-        prev_pos[u] = -1;
-        if (do_ins[u] && prev[u] >= 0 && prev[u] < vic.cap) prev_pos[u] = vic.pos[(int64_t)h * vic.cap + prev[u]];
       }
 #pragma unroll
-      for (int u = 0; u < kFR; ++u) {
+      for (int u = 0; u < NR; ++u) {
         if (do_ins[u]) {
-          vic.rows[((int64_t)h * nv + p_ins[u]) * chunks + c] = old_val[u];
+          rows_h[((uint32_t)p_ins[u] << cl2) + c] = old_val[u];
           if (c == 0) {
-            if (prev_pos[u] == p_ins[u]) vic.pos[(int64_t)h * vic.cap + prev[u]] = -1;
-            vic.tok[(int64_t)h * nv + p_ins[u]] = old[u];
-            vic.pos[(int64_t)h * vic.cap + old[u]] = (int16_t)p_ins[u];
+            if (prev_pos[u] == p_ins[u]) pos_h[(uint32_t)prev[u]] = -1;
+            tags_h[(uint32_t)p_ins[u]] = old[u];
+            pos_h[(uint32_t)old[u]] = (int16_t)p_ins[u];
           }
         }
       }
       {  // statistics: rows taken from the host store (one addition per wave: additions to one line are served in turn)
         int n_host = 0;
 #pragma unroll
-        for (int u = 0; u < kFR; ++u) n_host += __popcll(__ballot(ok[u] && c == 0 && !from_fifo[u]));
-        if (n_host && lane_id() == 0) atomicAdd(&vic.host_rows[h], n_host);
+        for (int u = 0; u < NR; ++u) n_host += __popcll(__ballot(ok[u] && c == 0 && !from_fifo[u]));
+        if (n_host && lane == 0) atomicAdd(&vic.host_rows[h], n_host);
       }
       // the K rows that leave their slots, in the order of the miss list, for the kept sums of the factor update
       if (evk) {
 #pragma unroll
-        for (int u = 0; u < kFR; ++u)
-          if (ok[u] && is_k && j[u] < evk_rows) evk[((int64_t)h * evk_rows + j[u]) * cpr + c] = old_val[u];
+        for (int u = 0; u < NR; ++u) {
+          const int j = first + u * pass;
+          if (ok[u] && is_k && j < evk_rows) evk[(((int64_t)h * evk_rows + j) << lpr_log2) + c] = old_val[u];
+        }
       }
     } else {
-      uint4 old_val[kFR];
+      uint4 old_val[NR];
       if (evk) {  // (uniform)
 #pragma unroll
-        for (int u = 0; u < kFR; ++u) old_val[u] = *own[u];
+        for (int u = 0; u < NR; ++u) old_val[u] = *own[u];
       }
 #pragma unroll
-      for (int u = 0; u < kFR; ++u) val[u] = *(ok[u] ? host_src[u] : own[u]);
+      for (int u = 0; u < NR; ++u) val[u] = *(ok[u] ? host_src[u] : own[u]);
       if (evk) {
 #pragma unroll
-        for (int u = 0; u < kFR; ++u)
-          if (ok[u] && is_k && j[u] < evk_rows) evk[((int64_t)h * evk_rows + j[u]) * cpr + c] = old_val[u];
+        for (int u = 0; u < NR; ++u) {
+          const int j = first + u * pass;
+          if (ok[u] && is_k && j < evk_rows) evk[(((int64_t)h * evk_rows + j) << lpr_log2) + c] = old_val[u];
+        }
       }
     }
 #pragma unroll
-    for (int u = 0; u < kFR; ++u) {
-      if (ok[u]) {
-        if (is_k) k_act[dst[u] + c] = val[u]; else v_act[dst[u] + (c - cpr)] = val[u];
-      } else {
+    for (int u = 0; u < NR; ++u) {
+      if (ok[u])
+        *own[u] = val[u];
+      else
         val[u] = make_uint4(0, 0, 0, 0);
-      }
       Vec16<T> vv;
       vv.raw = *reinterpret_cast<decltype(vv.raw)*>(&val[u]);
       float f[VEC];
@@ -436,6 +470,14 @@ __device__ __forceinline__ void fetch_rows_attn_body(const uint4* __restrict__ s
         st.m = m_new;
       }
     }
+  };
+  if (cnt <= pass) {  // (uniform)
+    trip(std::integral_constant<int, 1>{}, j0);
+  } else {
+    for (int first = j0; first - jl < cnt; first += kFR * pass) {  // (first - jl: uniform)
+      if (first != j0) lists(first);
+      trip(std::integral_constant<int, kFR>{}, first);
+    }
   }
   // merge the row groups: V lane (jl, cv) owns columns cv*VEC .. of group jl
   const int groups = rpb;  // <= 8 for rows of >= 512 bytes; larger counts are merged in rounds of 8
@@ -452,16 +494,30 @@ __device__ __forceinline__ void fetch_rows_attn_body(const uint4* __restrict__ s
       for (int e = 0; e < VEC; ++e) row[2 + (c - cpr) * VEC + e] = st.acc[e];
     }
     __syncthreads();
+    // (all reads of a round together: one after the other, with the group count as the loop's end, they took 1 us)
     const int ng = min(8, groups - g0);
-    float Mg = M;
-    for (int g = 0; g < ng; ++g) Mg = fmaxf(Mg, accs[g][0]);
+    float mg[8], lg[8], xg[8], Mg = M;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const float* row = accs[g];
+      mg[g] = row[0];
+      lg[g] = row[1];
+      xg[g] = row[min(tid, d + 1)];
+    }
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      mg[g] = g < ng ? mg[g] : -INFINITY;
+      Mg = fmaxf(Mg, mg[g]);
+    }
     const float a_old = (Mg == -INFINITY) ? 0.0f : exp2f(M - Mg);
     Lsum *= a_old;
     col *= a_old;
-    for (int g = 0; g < ng; ++g) {
-      const float fg = (Mg == -INFINITY || accs[g][0] == -INFINITY) ? 0.0f : exp2f(accs[g][0] - Mg);
-      Lsum = fmaf(accs[g][1], fg, Lsum);
-      if (tid >= 2 && tid < d + 2) col = fmaf(accs[g][tid], fg, col);
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const bool live = mg[g] != -INFINITY;  // (rows of LDS beyond the groups hold anything)
+      const float fg = live ? exp2f(mg[g] - Mg) : 0.0f;
+      Lsum = fmaf(live ? lg[g] : 0.0f, fg, Lsum);
+      col = fmaf(live ? xg[g] : 0.0f, fg, col);
     }
     M = Mg;
   }
@@ -488,7 +544,7 @@ template <typename T>
 __global__ __launch_bounds__(kAttnThreads, 4) void fetch_attn_partial_kernel(
     const uint4* __restrict__ store, int64_t cap, int32_t* __restrict__ hit, int64_t hit_stride,
     const int32_t* __restrict__ miss_slots, const int32_t* __restrict__ miss_count, const uint8_t* __restrict__ evict,
-    int hq, int hkv, int cpr, int k, int n_fetch, const T* __restrict__ q, T* __restrict__ K, T* __restrict__ V,
+    int group, int k, int n_fetch, const T* __restrict__ q, T* __restrict__ K, T* __restrict__ V,
     int n_slots, int d, int lpr_log2, float scale_log2e, float* __restrict__ part, int S, int with_finish,
     FinishArgs fa, const int32_t* __restrict__ miss_old, VictimView vic, const int32_t* __restrict__ miss_new,
     const float* __restrict__ kq, uint4* __restrict__ evk, int evk_rows, int32_t* __restrict__ count_copy) {
@@ -503,8 +559,8 @@ __global__ __launch_bounds__(kAttnThreads, 4) void fetch_attn_partial_kernel(
     return;
   }
   if ((int)blockIdx.x < n_fetch) {
-    fetch_rows_attn_body<T>(store, cap, (uint4*)K, (uint4*)V, n_slots, hit, hit_stride, miss_slots, miss_count, hq, hkv,
-                            cpr, k, h, blockIdx.x, n_fetch, q, d, scale_log2e,
+    fetch_rows_attn_body<T>(store, cap, (uint4*)K, (uint4*)V, n_slots, hit, hit_stride, miss_slots, miss_count,
+                            group, lpr_log2, k, h, blockIdx.x, n_fetch, q, d, scale_log2e,
                             part + ((int64_t)h * (S + n_fetch) + S + blockIdx.x) * (d + 2), miss_old, vic, miss_new, evk,
                             evk_rows);
     return;
@@ -723,7 +779,7 @@ static int fetch_attention_impl(lrqk_ctx* ctx, const void* dev_store, int64_t ca
   ctx->kq_valid = false;
   hipLaunchKernelGGL((fetch_attn_partial_kernel<T>), dim3((unsigned)(n_fetch + S + with_finish + index_role), (unsigned)bh),
                      dim3(kAttnThreads), 0, st, (const uint4*)dev_store, cap, hit, hit_stride, miss_slots, miss_count,
-                     evict, hq, hkv, cpr, k, n_fetch, (const T*)q, (T*)k_act, (T*)v_act, n_slots, d, lpr_log2,
+                     evict, hq / hkv, k, n_fetch, (const T*)q, (T*)k_act, (T*)v_act, n_slots, d, lpr_log2,
                      scale_log2e, (float*)ctx->attn_part.p, S, with_finish, ctx->fin, miss_old, vic, miss_new, kq,
                      (uint4*)evk, evk_rows, count_copy);
   LRQK_HIP_CHECK(hipGetLastError());

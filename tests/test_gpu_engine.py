@@ -1224,3 +1224,57 @@ def test_cast_functions(lrqk, oracle):
     assert torch.equal(dev["B_Q"].cpu(), x["B_Q"])
     for got, exp in zip((nB_Q, nB_K, qh, kh), ref):
         assert _rel(got, exp) < 2e-4
+
+
+@pytest.mark.parametrize("d,r,dtype", [(128, 16, torch.bfloat16), (64, 32, torch.bfloat16), (128, 64, torch.float32),
+                                       (16, 8, torch.float32), (256, 32, torch.bfloat16)])
+@pytest.mark.parametrize("share", [0.01, 0.1, 0.3, 1.0])
+@torch.inference_mode()
+def test_fetch_of_few_and_many_rows(lrqk, d, r, dtype, share):
+    """One launch fetches the missed rows and attends over everything; how its workgroups share a head's misses (one row per
+    lane group, two, several trips, none) goes by their number, about k / 8 and k / 4.  A share of the resident slots is
+    given tokens that will not be selected: rows, attention and, with and without the cache of evicted rows, every bit."""
+    from lrqk_amd import synth
+    k, L, l, hq, hkv = 264, 8, 2000, 6, 2
+    wl = synth.Workload("f", hq, hkv, d, 1, dtype, l, r, k, L, (2, 2), (1e-2, 1e-2), 4, rho=min(r + 8, d))
+    Q, K, V, bases, gen = synth.prompt_qkv(wl, 3, l, device=torch.device(DEV))
+    A0 = synth.init_factors(wl, l, 4, device=torch.device(DEV))
+    kh, vh = (t.repeat_interleave(hq // hkv, 1) for t in (K, V))
+    engs = []
+    for rows in (0, 4 * k, 40):
+        e = lrqk.LightAttentionIndicesFactory(num_lite_tokens=L, attn_topk=k, num_key_value_groups=hq // hkv, r=r,
+                                              max_iter=(2, 2), tol=(1e-2, 1e-2), capacity=4096)
+        e.victim_rows, e.attn_in_step = rows, True
+        e.init_factors = (A0[0].clone(), A0[1].clone())
+        e.prefill(Q, K, V)
+        engs.append(e)
+    # the slots of every head that get the tokens with the lowest proxy scores
+    scores = (engs[0].last_A_Q_row.float() @ engs[0].A_K[:, :, :l - L].float().transpose(2, 3))[:, :, 0]
+    low = scores.argsort(-1)[:, :, :k].sort(-1).values
+    n = max(1, int(share * k))
+    slots = torch.randperm(k, generator=torch.Generator().manual_seed(n))[:n].sort().values.to(DEV)
+    for e in engs:
+        e._active_idx[:, :, slots] = low[:, :, slots].to(torch.int32)
+        for act, src in ((e.Kgpu, kh), (e.Vgpu, vh)):
+            act[:, :, slots] = src.gather(2, low[:, :, slots, None].expand(-1, -1, -1, d))
+    stream = synth.DecodeStream(wl, Q[:, :, -1:], bases, gen)
+    for step in range(4):
+        q, kn, vn = [t.contiguous() for t in stream.next()]
+        kh, vh = (torch.cat((t, x.repeat_interleave(hq // hkv, 1)), 2) for t, x in ((kh, kn), (vh, vn)))
+        for e in engs:
+            e.decode(q, kn, vn)
+        a = engs[0]
+        ids = a._active_idx.long()[..., None].expand(-1, -1, -1, d)
+        assert torch.equal(a.Kgpu, kh.gather(2, ids)) and torch.equal(a.Vgpu, vh.gather(2, ids)), step
+        p = (q.double() @ a.Kgpu.double().transpose(2, 3) / d ** 0.5).softmax(-1) @ a.Vgpu.double()
+        p = p.to(dtype)
+        limit = _attention_limit(TOL["attention_fp32" if dtype == torch.float32 else "attention_bf16"], p)
+        rel = _rel(a.last_attn, p)
+        _say("misses", a.last_miss_count.flatten().tolist(), "attention", rel, "limit", limit)
+        assert rel <= limit, step
+        for e in engs[1:]:
+            assert torch.equal(a._active_idx, e._active_idx) and torch.equal(a.last_miss_count, e.last_miss_count), step
+            assert torch.equal(a.Kgpu, e.Kgpu) and torch.equal(a.Vgpu, e.Vgpu), step
+            assert torch.equal(a.last_attn, e.last_attn) and torch.equal(a.B_Q, e.B_Q) and torch.equal(a.B_K, e.B_K), step
+        if step == 0:
+            assert int(a.last_miss_count.max()) >= n // 2
