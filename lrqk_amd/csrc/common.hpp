@@ -154,6 +154,16 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
   return x;
 }
 
+// The same inside each row of 16 lanes.
+__device__ __forceinline__ int row_inclusive_sum(int v) {
+  int x = v + dpp_mov0<kDppRowShr1, 0xf, 0xf>(v);
+  x += dpp_mov0<kDppRowShr2, 0xf, 0xf>(v);
+  x += dpp_mov0<kDppRowShr3, 0xf, 0xf>(v);
+  x += dpp_mov0<kDppRowShr4, 0xf, 0xe>(x);
+  x += dpp_mov0<kDppRowShr8, 0xf, 0xc>(x);
+  return x;
+}
+
 // Butterflies inside each row of 16 lanes; afterwards every lane of a row holds the row's result.
 template <typename Op>
 __device__ __forceinline__ float row_reduce(float v, Op op) {

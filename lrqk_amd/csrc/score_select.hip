@@ -746,25 +746,25 @@ struct DiffArgs {
 
 // mode: 0 = use the candidate list if valid, else compute the head's keys from A_K;
 //       1 = keys[] already holds the head's keys (caller-provided scores).
-// Dynamic LDS: gt | eq bitmaps (2 * kChunkWords words), then, with a diff, 10*k bytes.
-// LDS blocks of the selector (declared by the kernels, so that the two bodies below share them)
+// Dynamic LDS: the fixed blocks below, then gt | eq bitmaps (2 * kChunkWords words), then, with a diff, 10*k bytes.
+// (All of it dynamic: a body that is a function of its own then finds the same blocks as the kernel that calls it.)
 struct SelLds {
-  uint32_t* dyn;     // dynamic LDS
   uint32_t* hist;    // [kBins]
   uint32_t* hist_b;  // [kBins], directly behind hist
   int* scratch;      // [2 * kSelWaves]
   uint32_t* wred;    // [2 * kSelWaves]
   int* s_res;        // [8]
   int* s_n;          // [1]
+  uint32_t* dyn;     // the rest
 };
-#define LRQK_SEL_LDS(L)                                           \
-  extern __shared__ __align__(16) uint32_t dyn_lds[];             \
-  __shared__ __align__(16) uint32_t hist2_lds[2 * kBins];         \
-  __shared__ int scratch_lds[2 * kSelWaves];                      \
-  __shared__ uint32_t wred_lds[2 * kSelWaves];                    \
-  __shared__ int s_res_lds[8];                                    \
-  __shared__ int s_n_lds;                                         \
-  SelLds L{dyn_lds, hist2_lds, hist2_lds + kBins, scratch_lds, wred_lds, s_res_lds, &s_n_lds};
+constexpr int kSelFixedWords = 2 * kBins + 4 * kSelWaves + 8 + 4;
+static_assert(kSelFixedWords % 4 == 0, "the bitmaps are cleared 16 bytes at a time");
+__device__ __forceinline__ SelLds select_lds() {
+  extern __shared__ __align__(16) uint32_t sel_lds[];
+  uint32_t* const scratch = sel_lds + 2 * kBins;
+  int* const s_res = (int*)(scratch + 4 * kSelWaves);
+  return SelLds{sel_lds, sel_lds + kBins, (int*)scratch, scratch + 2 * kSelWaves, s_res, s_res + 8, sel_lds + kSelFixedWords};
+}
 
 // n_list: the length of the head's candidate list if the caller has read it already (and every thread of the
 // workgroup with it), else -1.
@@ -786,7 +786,9 @@ __device__ __forceinline__ void select_generic(const SelLds& L, int mode, const 
   int& s_n = *L.s_n;
   uint32_t* gt = dyn;
   uint32_t* eq = dyn + kChunkWords;
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (see select_step_fast)
+  const int lane = tid & (kWave - 1), wave = wave_id();
   const int h = blockIdx.x;
   uint32_t* keys = keys_all + (int64_t)h * key_stride;
   const uint2* cand = cand_all + (int64_t)h * cand_cap;
@@ -1173,7 +1175,7 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(int mode, const uin
                                                              int64_t head_stride, const T* __restrict__ q_hat, int64_t m,
                                                              int r, int round_bf16, int k, int32_t* __restrict__ out_all,
                                                              int64_t out_stride, DiffArgs df, NextList next) {
-  LRQK_SEL_LDS(L);
+  const SelLds L = select_lds();
   select_generic<T, R, LIST>(L, mode, cand_all, cand_cap, st, keys_all, key_stride, a_k, head_stride, q_hat, m, r, round_bf16,
                              k, out_all, out_stride, df, -1, 0, next);
 }
@@ -1189,30 +1191,32 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(int mode, const uin
 // moves, the wave totals rescanned by every wave).  Anything else (no list, overflow, longer contexts) goes
 // through select_generic in the same launch.
 
-// Exclusive scan of two counters in thread order; one barrier.  slot: 2 * kSelWaves ints; consecutive calls must
-// be separated by a barrier.
-__device__ __forceinline__ void step_scan2(int a, int b, int* slot, int& ex_a, int& ex_b, int& tot_a, int& tot_b) {
+// What bounds the step's select is the instructions that its sixteen waves issue (four share a SIMD: 150 a microsecond and
+// wave) beside its barriers: with 512 threads it takes 2 .. 5 us more.  So counters that cannot exceed 16 bits (a list has at
+// most 16 K entries) go through a scan two at a time, the sums of the sixteen waves through one row of lanes, bitmaps 16 bytes
+// at a time; the tied candidates are cut at the id of the last one that is taken, not ranked; what is read is requested first,
+// and what is the same for a launch is read where it is needed.  Launch, us: 32 heads x 32K 11.3 -> 10.2, x 128K 12.4 -> 10.0,
+// 128 heads 14.1 -> 12.1, 28 fp32 heads x 4K 12.3 -> 10.2, k 4096 15.7 -> 13.7, r 16 / k 1024 12.1 -> 9.2.
+
+// Exclusive scan of a counter (or of two, of 16 bits each) in thread order; one barrier.  slot: kSelWaves ints; consecutive
+// calls must be separated by a barrier.
+__device__ __forceinline__ uint32_t step_scan(uint32_t a, int* slot, uint32_t& tot) {
+  static_assert(kSelWaves <= 16, "the waves' sums fit a row of lanes");
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(wave_id());
-  const int ia = wave_inclusive_sum(a), ib = wave_inclusive_sum(b);
-  if (lane == kWave - 1) {
-    slot[wave] = ia;
-    slot[kSelWaves + wave] = ib;
-  }
+  const uint32_t ia = (uint32_t)wave_inclusive_sum((int)a);
+  if (lane == kWave - 1) slot[wave] = (int)ia;
   __syncthreads();
-  const int ta = lane < kSelWaves ? slot[lane] : 0;
-  const int tb = lane < kSelWaves ? slot[kSelWaves + lane] : 0;
-  const int sa = wave_inclusive_sum(ta), sb = wave_inclusive_sum(tb);
-  const int base_a = wave ? __builtin_amdgcn_readlane(sa, wave - 1) : 0;
-  const int base_b = wave ? __builtin_amdgcn_readlane(sb, wave - 1) : 0;
-  tot_a = __builtin_amdgcn_readlane(sa, kSelWaves - 1);
-  tot_b = __builtin_amdgcn_readlane(sb, kSelWaves - 1);
-  ex_a = base_a + ia - a;
-  ex_b = base_b + ib - b;
+  const uint32_t sa = (uint32_t)row_inclusive_sum(lane < kSelWaves ? slot[lane] : 0);
+  const uint32_t base = wave ? (uint32_t)__builtin_amdgcn_readlane((int)sa, wave - 1) : 0u;
+  tot = (uint32_t)__builtin_amdgcn_readlane((int)sa, kSelWaves - 1);
+  return base + ia - a;
 }
 
-// Like find_digits, with the one-barrier scan; cnt_a: number of elements in the digit found for need_a.
-// s_res: 5 ints.  Two barriers.
+// From two histograms of kBins bins (kBinsPT bins per thread; SAME: one histogram asked twice): the digit of the need_a-th
+// largest element of hist_a and of the need_b-th largest of hist_b, with the ranks inside those digits; cnt_a: number of
+// elements in the digit found for need_a.  s_res: 5 ints.  Two barriers.
+template <bool SAME>
 __device__ __forceinline__ void step_find_digits(const uint32_t* hist_a, const uint32_t* hist_b, int need_a, int need_b,
                                                  int* slot, int* s_res, int& dig_a, int& rem_a, int& dig_b, int& rem_b,
                                                  int& cnt_a) {
@@ -1221,13 +1225,15 @@ __device__ __forceinline__ void step_find_digits(const uint32_t* hist_a, const u
 #pragma unroll
   for (int x = 0; x < kBinsPT; ++x) {
     ca[x] = (int)hist_a[tid * kBinsPT + x];
-    cb[x] = (int)hist_b[tid * kBinsPT + x];
     la += ca[x];
+    cb[x] = SAME ? ca[x] : (int)hist_b[tid * kBinsPT + x];
     lb += cb[x];
   }
-  int ea, eb, ta, tb;
-  step_scan2(la, lb, slot, ea, eb, ta, tb);
-  const int above_a = ta - ea - la, above_b = tb - eb - lb;  // elements in bins above this thread's bins
+  uint32_t tot;
+  const uint32_t ex = step_scan(SAME ? (uint32_t)la : ((uint32_t)lb << 16) | (uint32_t)la, slot, tot);
+  // elements in bins above this thread's bins
+  const int above_a = (int)(tot & 0xffffu) - (int)(ex & 0xffffu) - la;
+  const int above_b = SAME ? above_a : (int)(tot >> 16) - (int)(ex >> 16) - lb;
   if (above_a < need_a && need_a <= above_a + la) {
     int c = above_a;
 #pragma unroll
@@ -1263,14 +1269,58 @@ __device__ __forceinline__ void step_find_digits(const uint32_t* hist_a, const u
 // outgoing tokens (i32 [k] each), freed slots (u16 [k]).
 static inline size_t step_select_words4(int64_t m) { return (size_t)(((m + 31) >> 5) + 3) & ~(size_t)3; }
 static inline size_t step_select_smem(int64_t m, int k) {
-  return step_select_words4(m) * (3 * 4 + 2) + (size_t)k * (4 + 4 + 4 + 2) + 16;
+  return (size_t)kSelFixedWords * 4 + step_select_words4(m) * (3 * 4 + 2) + (size_t)k * (4 + 4 + 2) + 16;
+}
+
+constexpr int kStepIpt = kFusedDiffMaxK / kSelThreads;  // resident ids per thread
+// Clears the three bitmaps, the first histogram and the small counters.
+__device__ __forceinline__ void select_step_clear(const SelLds& L, int64_t m, int tid) {
+  const int words4 = ((int)((m + 31) >> 5) + 3) & ~3;
+  uint4* z = reinterpret_cast<uint4*>(L.dyn);
+  for (int i = tid; i < 3 * words4 / 4; i += kSelThreads) z[i] = make_uint4(0, 0, 0, 0);
+  for (int i = tid; i < kBins / 4; i += kSelThreads) reinterpret_cast<uint4*>(L.hist)[i] = make_uint4(0, 0, 0, 0);
+  if (tid < 8) L.s_res[tid] = 0;
+  if (tid < 2) L.wred[tid] = 0;
+}
+__device__ __forceinline__ void select_step_ids(const DiffArgs& df, int h, int k, int tid, int32_t (&hv)[kStepIpt]) {
+  const int32_t* hit = df.hit + (int64_t)h * df.hit_stride;
+  const int ipt = (k + kSelThreads - 1) / kSelThreads;  // contiguous per thread, to keep slot order
+#pragma unroll
+  for (int u = 0; u < kStepIpt; ++u) hv[u] = hit[min(tid * ipt + min(u, ipt - 1), k - 1)];
+}
+
+// What the kernel is launched with, its only parameter.  The bodies read a member where they need it (scalar loads): taken as
+// separate parameters all of them are read at the start, and two thirds were moved to lanes of vector registers and back,
+// 45 + 60 instructions.
+struct StepSelectArgs {
+  const uint2* cand;
+  int cand_cap;
+  SelState st;
+  uint32_t* keys;
+  int64_t key_stride;
+  const void* a_k;
+  int64_t head_stride;
+  const void* q_hat;
+  int64_t m;
+  int r, round_bf16, k;
+  int32_t* out;
+  int64_t out_stride;
+  DiffArgs df;
+};
+__device__ __forceinline__ const StepSelectArgs* step_select_args() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (const StepSelectArgs*)p;
 }
 
 template <int CPT>
-__device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* __restrict__ cand, int N, uint32_t lo,
-                                                 SelState st, int h, int64_t m, int k, int k2, const DiffArgs& df) {
-  const int tid = threadIdx.x;
-  const int words = (int)((m + 31) >> 5);
+__device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2 (&c)[CPT], const int32_t (&hv)[kStepIpt], int N,
+                                                 uint32_t lo, float q_cur, int vic_at, int h, int m, int k, int k2) {
+  // (a value of this body's own: what the bodies of one kernel compute alike from the thread's index would be computed in front
+  // of the branch between them, held for all of them at once and spilled)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int words = (m + 31) >> 5;
   const int words4 = (words + 3) & ~3;
   uint32_t* bmS = L.dyn;              // selected tokens
   uint32_t* bmE = bmS + words4;       // candidates tied at the threshold
@@ -1278,46 +1328,38 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
   uint16_t* wpre = reinterpret_cast<uint16_t*>(bmH + words4);  // [words4] marked tokens in the words before
   int32_t* miss_s = reinterpret_cast<int32_t*>(wpre + words4);  // [k] incoming tokens, ascending
   int32_t* ev_old = miss_s + k;                                 // [k] tokens of the freed slots
-  int32_t* hit_s = ev_old + k;                                  // [k] resident token of every slot (as the step found it)
-  uint16_t* ev_slot = reinterpret_cast<uint16_t*>(hit_s + k);   // [k] freed slots, ascending
+  uint16_t* ev_slot = reinterpret_cast<uint16_t*>(ev_old + k);  // [k] freed slots, ascending
   uint32_t* hist = L.hist;
   uint32_t* hist_b = L.hist_b;
   uint32_t* bmM = L.hist;             // incoming tokens (takes the place of the two histograms, 2 * kBins words)
   int* s_res = L.s_res;
-  int32_t* hit = df.hit + (int64_t)h * df.hit_stride;
 
-  // ---- requests first: the candidates and the resident ids (contiguous per thread, to keep slot order)
-  uint2 c[CPT];
-#pragma unroll
-  for (int u = 0; u < CPT; ++u) c[u] = cand[min(tid + u * kSelThreads, N - 1)];
-  constexpr int kIpt = kFusedDiffMaxK / kSelThreads;
+  constexpr int kIpt = kStepIpt;
   const int ipt = (k + kSelThreads - 1) / kSelThreads;
-  int32_t hv[kIpt];
+  const int n_quads = words4 >> 2;
+  const int qpt = (n_quads + kSelThreads - 1) / kSelThreads;  // 16-byte pieces of a bitmap per thread (m <= kChunkBits: two at most)
+  constexpr int kQpt = kChunkWords / 4 / kSelThreads;
+  // the marked tokens of this thread's pieces of a bitmap, and how many
+  auto count_marks = [&](const uint32_t* bm, uint4 (&w)[kQpt]) {
+    int cnt = 0;
 #pragma unroll
-  for (int u = 0; u < kIpt; ++u) hv[u] = hit[min(tid * ipt + u, k - 1)];
-  // ---- meanwhile: clear the bitmaps and the first histogram
-  {
-    uint4* z = reinterpret_cast<uint4*>(bmS);
-    for (int i = tid; i < 3 * words4 / 4; i += kSelThreads) z[i] = make_uint4(0, 0, 0, 0);
-    for (int i = tid; i < kBins; i += kSelThreads) hist[i] = 0;
-    if (tid < 8) s_res[tid] = 0;
-    if (tid < 2) L.wred[tid] = 0;
-  }
-  __syncthreads();
-  // ---- resident bitmap (the ids also go to LDS: they are needed again after the selection, and registers held
-  // that long were spilled); range of the keys
+    for (int x = 0; x < kQpt; ++x) {
+      w[x] = make_uint4(0, 0, 0, 0);
+      if (x < qpt && tid * qpt + x < n_quads) w[x] = reinterpret_cast<const uint4*>(bm)[tid * qpt + x];
+      cnt += __popc(w[x].x) + __popc(w[x].y) + __popc(w[x].z) + __popc(w[x].w);
+    }
+    return cnt;
+  };
+  // ---- resident bitmap; range of the keys (the blocks are cleared: select_step_clear)
 #pragma unroll
   for (int u = 0; u < kIpt; ++u) {
     const int32_t v = hv[u];
-    if (u < ipt && tid * ipt + u < k) {
-      hit_s[tid * ipt + u] = v;
-      if (v >= 0 && v < m) atomicOr(&bmH[v >> 5], 1u << (v & 31));
-    }
+    if (u < ipt && tid * ipt + u < k && v >= 0 && v < m) atomicOr(&bmH[v >> 5], 1u << (v & 31));
   }
   uint32_t vmax = 0u, vor = 0u;
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
-    if (tid + u * kSelThreads < N) {
+    if (u * kSelThreads < N && tid + u * kSelThreads < N) {
       vmax = max(vmax, c[u].x);
       vor |= c[u].x - lo;
     }
@@ -1337,11 +1379,12 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
   const int s1 = max(nbits - 12, 0), s2 = max(s1 - 12, 0);
   // ---- radix select of the k-th and k2-th largest keys (one pass for bf16-rounded scores)
 #pragma unroll
-  for (int u = 0; u < CPT; ++u)
-    if (tid + u * kSelThreads < N) atomicAdd(&hist[((c[u].x - lo) >> tz) >> s1], 1u);
+  for (int u = 0; u < CPT; ++u) {
+    if (u * kSelThreads < N && tid + u * kSelThreads < N) atomicAdd(&hist[((c[u].x - lo) >> tz) >> s1], 1u);
+  }
   __syncthreads();
   int D1, need1, E1, needE, cntT;
-  step_find_digits(hist, hist, k, k2, L.scratch, s_res, D1, need1, E1, needE, cntT);
+  step_find_digits<true>(hist, hist, k, k2, L.scratch, s_res, D1, need1, E1, needE, cntT);
   uint32_t offT = (uint32_t)D1 << s1, offE = (uint32_t)E1 << s1;
   int need_eq = need1;
   if (s1 > 0) {
@@ -1359,7 +1402,7 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
     }
     __syncthreads();
     int D2, need2, E2, needE2;
-    step_find_digits(hist, hist_b, need1, needE, L.scratch, s_res, D2, need2, E2, needE2, cntT);
+    step_find_digits<false>(hist, hist_b, need1, needE, L.scratch, s_res, D2, need2, E2, needE2, cntT);
     offT |= (uint32_t)D2 << s2;
     offE |= (uint32_t)E2 << s2;
     need_eq = need2;
@@ -1377,23 +1420,24 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
       }
       __syncthreads();
       int D3, need3, dd, dr;
-      step_find_digits(hist, hist, need2, need2, L.scratch, s_res, D3, need3, dd, dr, cntT);
+      step_find_digits<true>(hist, hist, need2, need2, L.scratch, s_res, D3, need3, dd, dr, cntT);
       offT |= (uint32_t)D3;
       need_eq = need3;
     }
   }
   const uint32_t Tk = lo + (offT << tz);
   if (tid == 0) {
+    const SelState& st = step_select_args()->st;
     st.t_low[h] = lo + (offE << tz);
-    st.q_norm[h] = st.q_cur[h];
+    st.q_norm[h] = q_cur;
   }
   const bool all_eq = need_eq >= cntT;  // every candidate tied at the threshold is selected: no order needed
   // ---- classify (the histograms are dead: their block becomes the bitmap of the incoming tokens)
-  for (int i = tid; i < words4; i += kSelThreads) bmM[i] = 0;
+  for (int i = tid; i < n_quads; i += kSelThreads) reinterpret_cast<uint4*>(bmM)[i] = make_uint4(0, 0, 0, 0);
   uint32_t selmask = 0u, eqmask = 0u;
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
-    if (tid + u * kSelThreads < N) {
+    if (u * kSelThreads < N && tid + u * kSelThreads < N) {
       const uint32_t key = c[u].x, idx = c[u].y;
       if (key > Tk || (all_eq && key == Tk)) {
         selmask |= 1u << u;
@@ -1405,50 +1449,50 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
     }
   }
   __syncthreads();
-  const int wpt = (words4 + kSelThreads - 1) / kSelThreads;  // bitmap words per thread (<= kWordsPT)
-  const int w0 = tid * wpt;
+  // the need_eq lowest token ids among the tied candidates are selected: all up to the need_eq-th in the order of the ids
+  int32_t last_eq = -1;
   if (!all_eq) {
-    // the need_eq lowest token ids among the tied candidates: rank = marked tokens before it
-    int cnt = 0;
-    for (int x = 0; x < wpt; ++x) cnt += (w0 + x < words4) ? __popc(bmE[w0 + x]) : 0;
-    int ex, exb, tot, totb;
-    step_scan2(cnt, 0, L.scratch, ex, exb, tot, totb);
-    for (int x = 0; x < wpt; ++x) {
-      if (w0 + x < words4) {
-        wpre[w0 + x] = (uint16_t)ex;
-        ex += __popc(bmE[w0 + x]);
-      }
-    }
-    __syncthreads();
+    uint4 w[kQpt];
+    const int cnt = count_marks(bmE, w);
+    uint32_t tot;
+    int left = need_eq - (int)step_scan((uint32_t)cnt, L.scratch, tot);
+    if (left > 0 && left <= cnt) {  // (one thread)
 #pragma unroll
-    for (int u = 0; u < CPT; ++u) {
-      if ((eqmask >> u) & 1u) {
-        const uint32_t idx = c[u].y;
-        const int rank = (int)wpre[idx >> 5] + __popc(bmE[idx >> 5] & ((1u << (idx & 31)) - 1u));
-        if (rank < need_eq) {
-          selmask |= 1u << u;
-          atomicOr(&bmS[idx >> 5], 1u << (idx & 31));
+      for (int x = 0; x < kQpt; ++x) {
+        const int p0 = __popc(w[x].x), p1 = p0 + __popc(w[x].y), p2 = p1 + __popc(w[x].z), p3 = p2 + __popc(w[x].w);
+        if (left > 0 && left <= p3) {
+          const int at = (left > p0) + (left > p1) + (left > p2);
+          uint32_t v = at == 0 ? w[x].x : at == 1 ? w[x].y : at == 2 ? w[x].z : w[x].w;
+          const int skip = at == 0 ? 0 : at == 1 ? p0 : at == 2 ? p1 : p2;
+          for (int i = skip + 1; i < left; ++i) v &= v - 1u;
+          s_res[5] = ((4 * (tid * qpt + x) + at) << 5) + __ffs((int)v) - 1;
         }
+        left -= p3;
       }
     }
     __syncthreads();
+    last_eq = s_res[5];
+#pragma unroll
+    for (int u = 0; u < CPT; ++u)
+      if (((eqmask >> u) & 1u) && (int32_t)c[u].y <= last_eq) selmask |= 1u << u;
   }
   // ---- diff: slots whose token left the selection; selected tokens that are not resident
-  bool ev[kIpt];
-  int n_ev = 0;
+  uint32_t ev = 0u;
 #pragma unroll
   for (int u = 0; u < kIpt; ++u) {
-    const bool live = u < ipt && tid * ipt + u < k;
-    const int32_t v = hit_s[live ? tid * ipt + u : 0];
-    const bool in_range = v >= 0 && v < m;
-    const bool found = in_range && ((bmS[in_range ? (v >> 5) : 0] >> (v & 31)) & 1u);
-    ev[u] = live && !found;
-    n_ev += ev[u] ? 1 : 0;
+    if (u < ipt) {  // (uniform)
+      const bool live = tid * ipt + u < k;
+      const int32_t v = hv[u];
+      const bool in_range = v >= 0 && v < m;
+      const uint32_t word = in_range ? (uint32_t)v >> 5 : 0u, bit = 1u << (v & 31);
+      const bool found = in_range && ((bmS[word] & bit) || (v <= last_eq && (bmE[word] & bit)));
+      if (live && !found) ev |= 1u << u;
+    }
   }
   uint32_t missmask = 0u;
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
-    if ((selmask >> u) & 1u) {
+    if (u * kSelThreads < N && ((selmask >> u) & 1u)) {
       const uint32_t idx = c[u].y;
       if (!((bmH[idx >> 5] >> (idx & 31)) & 1u)) {
         missmask |= 1u << u;
@@ -1457,34 +1501,42 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
     }
   }
   __syncthreads();
-  int cnt_m = 0;
-  for (int x = 0; x < wpt; ++x) cnt_m += (w0 + x < words4) ? __popc(bmM[w0 + x]) : 0;
-  int ex_ev, ex_m, n_evict, n_missing;
-  step_scan2(n_ev, cnt_m, L.scratch, ex_ev, ex_m, n_evict, n_missing);
+  uint4 mw[kQpt];
+  const int cnt_m = count_marks(bmM, mw);
+  uint32_t tot2;
+  const uint32_t ex2 = step_scan(((uint32_t)cnt_m << 16) | (uint32_t)__popc(ev), L.scratch, tot2);
+  int ex_ev = (int)(ex2 & 0xffffu), ex_m = (int)(ex2 >> 16);
+  const int n_evict = (int)(tot2 & 0xffffu), n_missing = (int)(tot2 >> 16);
 #pragma unroll
   for (int u = 0; u < kIpt; ++u) {
-    if (ev[u]) {
+    if ((ev >> u) & 1u) {
       ev_slot[ex_ev] = (uint16_t)(tid * ipt + u);
-      ev_old[ex_ev] = hit_s[tid * ipt + u];
+      ev_old[ex_ev] = hv[u];
       ++ex_ev;
     }
   }
-  for (int x = 0; x < wpt; ++x) {
-    if (w0 + x < words4) {
-      wpre[w0 + x] = (uint16_t)ex_m;
-      ex_m += __popc(bmM[w0 + x]);
+#pragma unroll
+  for (int x = 0; x < kQpt; ++x) {
+    if (x < qpt && tid * qpt + x < n_quads) {  // four prefixes of 16 bits
+      const int e1 = ex_m + __popc(mw[x].x), e2 = e1 + __popc(mw[x].y), e3 = e2 + __popc(mw[x].z);
+      reinterpret_cast<uint2*>(wpre)[tid * qpt + x] =
+          make_uint2((uint32_t)ex_m | ((uint32_t)e1 << 16), (uint32_t)e2 | ((uint32_t)e3 << 16));
+      ex_m = e3 + __popc(mw[x].w);
     }
   }
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
-    if ((missmask >> u) & 1u) {
+    if (u * kSelThreads < N && ((missmask >> u) & 1u)) {
       const uint32_t idx = c[u].y;
       miss_s[(int)wpre[idx >> 5] + __popc(bmM[idx >> 5] & ((1u << (idx & 31)) - 1u))] = (int32_t)idx;
     }
   }
   __syncthreads();
   const int n_pair = min(n_missing, n_evict);
+  const StepSelectArgs* const args = step_select_args();
+  const DiffArgs& df = args->df;
+  int32_t* hit = df.hit + (int64_t)h * df.hit_stride;
   for (int j = tid; j < n_pair; j += kSelThreads) {
     const int s = ev_slot[j];
     const int32_t t_new = miss_s[j];
@@ -1496,16 +1548,16 @@ __device__ __forceinline__ void select_step_fast(const SelLds& L, const uint2* _
   if (df.evict) {
 #pragma unroll
     for (int u = 0; u < kIpt; ++u)
-      if (u < ipt && tid * ipt + u < k) df.evict[(int64_t)h * k + tid * ipt + u] = ev[u] ? 1 : 0;
+      if (u < ipt && tid * ipt + u < k) df.evict[(int64_t)h * k + tid * ipt + u] = (uint8_t)((ev >> u) & 1u);
   }
   if (tid == 0) {
     if (df.vic_ptr) {
-      const int base = df.vic_ptr[h];
-      df.vic_base[h] = base;
-      df.vic_ptr[h] = (base + min(n_pair, df.vic_nv)) % df.vic_nv;
+      df.vic_base[h] = vic_at;
+      const int next = vic_at + min(n_pair, df.vic_nv);  // (vic_at < vic_nv)
+      df.vic_ptr[h] = next >= df.vic_nv ? next - df.vic_nv : next;
     }
     if (df.miss_count) df.miss_count[h] = n_pair;
-    st.cand_count[h * kCountStride] = 0;  // re-arm for the next call
+    args->st.cand_count[h * kCountStride] = 0;  // re-arm for the next call
   }
 }
 
@@ -1517,18 +1569,59 @@ __device__ __forceinline__ int bound_rank(int k, int level, int64_t n) {
 }
 constexpr int kCalmCalls = 32;  // usable lists in a row before a head's slack is halved again
 
-// Where the 80 KB of code begin is pinned: the caches of a CU's instructions hold 64 KB and every launch starts with cold
-// ones, and the same instructions took 11.2 .. 11.8 us (32 heads x 32K rows) and 15.1 .. 16.2 (256 x 128K) by their address,
-// which moves with every other kernel of this file.  On multiples of 8 KB 11.3 and 15.4, of 64 KB 11.7 and 15.7.
+// The head scanned again, as a function: inlined beside the usual bodies, whose entries are requested before the choice between
+// them, it had those spilled across it.
 template <typename T, int R>
-__global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void select_step_kernel(
-    const uint2* __restrict__ cand_all, int cand_cap, SelState st, uint32_t* __restrict__ keys_all, int64_t key_stride,
-    const T* __restrict__ a_k, int64_t head_stride, const T* __restrict__ q_hat, int64_t m, int r, int round_bf16, int k,
-    int32_t* __restrict__ out_all, int64_t out_stride, DiffArgs df) {
-  LRQK_SEL_LDS(L);
-  const int h = blockIdx.x;
-  const int n = __builtin_amdgcn_readfirstlane(st.cand_count[h * kCountStride]);
-  const int lvl = __builtin_amdgcn_readfirstlane(st.level[h]);
+__device__ __attribute__((noinline)) void select_step_rescan(const StepSelectArgs* a, int n, int bound_rank_k) {
+  select_generic<T, R>(select_lds(), 0, a->cand, a->cand_cap, a->st, a->keys, a->key_stride, (const T*)a->a_k, a->head_stride,
+                       (const T*)a->q_hat, a->m, a->r, a->round_bf16, a->k, a->out, a->out_stride, a->df, n, bound_rank_k);
+}
+
+// Where the code begins is pinned: the caches of a CU's instructions hold 64 KB and every launch starts with cold ones, and the
+// same instructions (an earlier form of them, 80 KB) took 11.2 .. 11.8 us (32 heads x 32K rows) and 15.1 .. 16.2 (256 x 128K) by
+// their address, which moves with every other kernel of this file.  On multiples of 8 KB 11.3 and 15.4, of 64 KB 11.7 and 15.7.
+template <typename T, int R>
+__global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void select_step_kernel(StepSelectArgs) {
+  const SelLds L = select_lds();
+  const StepSelectArgs* const args = step_select_args();
+  const int h = blockIdx.x, tid = threadIdx.x;
+  const int cand_cap = args->cand_cap, k = args->k, m = (int)args->m;
+  // Everything that is read is requested at once, and the blocks that are counted in are cleared meanwhile: the list's length
+  // and the head's state, the entries of the usual list (the buffer has room for four per thread whatever the length, and for
+  // eight where k is large; what lies beyond the length is not looked at) and the resident ids.  The entries were behind the
+  // wait for the length (0.9 us), the clearing behind both (0.9) and single values waited for by one wave in two later phases
+  // (0.7 each).
+  const uint2* cand = args->cand + (int64_t)h * cand_cap;
+  const int n_v = args->st.cand_count[h * kCountStride], lvl_v = args->st.level[h];
+  const uint32_t lo_v = args->st.t_used[h];
+  float q_cur = args->st.q_cur[h];
+  int vic_at = args->df.vic_ptr ? args->df.vic_ptr[h] : 0;
+  constexpr int kAhead = 8;
+  const bool ahead8 = k > 2 * kSelThreads;  // (the usual list has 1.5 k entries; cand_cap >= 8 k)
+  uint2 c4[4], c8[kAhead];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) c4[u] = cand[tid + u * kSelThreads];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) c8[u] = make_uint2(0, 0);
+  if (ahead8) {  // (uniform)
+#pragma unroll
+    for (int u = 4; u < kAhead; ++u) c8[u] = cand[tid + u * kSelThreads];
+  }
+  int32_t hv[kStepIpt];
+  select_step_ids(args->df, h, k, tid, hv);
+  select_step_clear(L, m, tid);
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {  // (not moved behind the branch on the length)
+    if (u < 4) c8[u] = c4[u];
+    asm volatile("" : "+v"(c8[u].x), "+v"(c8[u].y));
+    if (u < 4) c4[u] = c8[u];
+  }
+#pragma unroll
+  for (int u = 0; u < kStepIpt; ++u) asm volatile("" : "+v"(hv[u]));
+  asm volatile("" : "+v"(q_cur), "+v"(vic_at));
+  __syncthreads();
+  const int n = __builtin_amdgcn_readfirstlane(n_v);
+  const int lvl = __builtin_amdgcn_readfirstlane(lvl_v);
   const bool fast = n >= k && n <= cand_cap && n <= 16 * kSelThreads;
   int level = lvl & 0xff, calm = lvl >> 8;
   if (!fast) {
@@ -1538,23 +1631,47 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void se
     --level;
     calm = 0;
   }
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(lo_v);
+  // (a path of its own to the end: with the usual list as one branch of several its entries are held, that is spilled, across
+  // the others)
+  if (fast && n <= 4 * kSelThreads) {
+    select_step_fast<4>(L, c4, hv, n, lo, q_cur, vic_at, h, m, k, bound_rank(k, level, n));
+    if (tid == 0) {
+      atomicAdd(&args->st.stats[0], 1);
+      args->st.level[h] = level | (calm << 8);
+    }
+    return;
+  }
+  if (fast && ahead8 && n <= kAhead * kSelThreads) {
+    select_step_fast<kAhead>(L, c8, hv, n, lo, q_cur, vic_at, h, m, k, bound_rank(k, level, n));
+    if (tid == 0) {
+      atomicAdd(&args->st.stats[0], 1);
+      args->st.level[h] = level | (calm << 8);
+    }
+    return;
+  }
   if (fast) {
-    if (threadIdx.x == 0) atomicAdd(&st.stats[0], 1);
-    const uint2* cand = cand_all + (int64_t)h * cand_cap;
-    const uint32_t lo = st.t_used[h];
-    const int k2 = bound_rank(k, level, n);
-    if (n <= 4 * kSelThreads)
-      select_step_fast<4>(L, cand, n, lo, st, h, m, k, k2, df);
-    else if (n <= 8 * kSelThreads)
-      select_step_fast<8>(L, cand, n, lo, st, h, m, k, k2, df);
+    if (tid == 0) atomicAdd(&args->st.stats[0], 1);
+    auto longer = [&](auto cpt_c) {
+      constexpr int CPT = decltype(cpt_c)::value;
+      int t = tid;
+      asm volatile("" : "+v"(t));  // (see select_step_fast)
+      uint2 c[CPT];
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) c[u] = cand[min(t + u * kSelThreads, n - 1)];
+      int32_t ids[kStepIpt];
+      select_step_ids(args->df, h, k, t, ids);
+      select_step_fast<CPT>(L, c, ids, n, lo, q_cur, vic_at, h, m, k, bound_rank(k, level, n));
+    };
+    if (n <= 8 * kSelThreads)
+      longer(std::integral_constant<int, 8>{});
     else
-      select_step_fast<16>(L, cand, n, lo, st, h, m, k, k2, df);
+      longer(std::integral_constant<int, 16>{});
   } else {
-    select_generic<T, R>(L, 0, cand_all, cand_cap, st, keys_all, key_stride, a_k, head_stride, q_hat, m, r, round_bf16, k,
-                         out_all, out_stride, df, n, bound_rank(k, level, m));
+    select_step_rescan<T, R>(args, n, bound_rank(k, level, m));
   }
   // (both bodies hold barriers, so every thread has read the old value by now)
-  if (threadIdx.x == 0) st.level[h] = level | (calm << 8);
+  if (tid == 0) args->st.level[h] = level | (calm << 8);
 }
 
 // --------------------------------------------------------------------------- host side
@@ -1582,7 +1699,7 @@ static int launch_scores(const void* a_k, int64_t head_stride, const void* q_hat
 }
 
 static size_t select_smem(int k, bool with_diff) {
-  return (size_t)2 * kChunkWords * sizeof(uint32_t) + (with_diff ? (size_t)k * 10 : 0);
+  return (size_t)(kSelFixedWords + 2 * kChunkWords) * sizeof(uint32_t) + (with_diff ? (size_t)k * 10 : 0);
 }
 
 struct SelectBufs {
@@ -1636,9 +1753,8 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
   size_t smem = select_smem(topk, df.hit != nullptr);
   // the decode step's select + diff (no ascending output): as long as its bitmaps fit the LDS beside the
   // generic path's blocks
-  constexpr size_t kLdsStatic = (size_t)2 * kBins * 4 + 1024;
   const bool step_path = !want_out && df.hit != nullptr && !df.replace_all && m <= kChunkBits && topk <= kFusedDiffMaxK &&
-                         std::max(smem, step_select_smem(m, topk)) + kLdsStatic <= (size_t)160 * 1024;
+                         std::max(smem, step_select_smem(m, topk)) <= (size_t)160 * 1024;
   if (step_path) {
     smem = std::max(smem, step_select_smem(m, topk));
     static std::atomic<size_t> step_allowed_dev[kMaxDeviceSlots];
@@ -1731,9 +1847,9 @@ static int launch_filter_select(lrqk_ctx* ctx, const SelectBufs& sb, const void*
     ++ctx->tev_used;
   }
   if (step_path)
-    hipLaunchKernelGGL((select_step_kernel<T, R>), dim3((unsigned)bh), dim3(kSelThreads), smem, st, sb.cand, sb.cand_cap,
-                       sb.st, sb.keys, sb.key_stride, (const T*)a_k, head_stride, (const T*)q_hat, m, r, round_bf16, topk,
-                       out_idx, out_stride, df);
+    hipLaunchKernelGGL((select_step_kernel<T, R>), dim3((unsigned)bh), dim3(kSelThreads), smem, st,
+                       StepSelectArgs{sb.cand, sb.cand_cap, sb.st, sb.keys, sb.key_stride, a_k, head_stride, q_hat, m, r,
+                                      round_bf16, topk, out_idx, out_stride, df});
   else
     hipLaunchKernelGGL(select, dim3((unsigned)bh), dim3(kSelThreads), smem, st, 0, sb.cand, sb.cand_cap, sb.st, sb.keys,
                        sb.key_stride, (const T*)a_k, head_stride, (const T*)q_hat, m, r, round_bf16, topk, out_idx,
@@ -1963,4 +2079,3 @@ extern "C" int lrqk_select_stats(lrqk_ctx* ctx, int* fast_heads, int* full_heads
   if (reset) LRQK_HIP_CHECK(hipMemset(stats, 0, sizeof(v)));
   return LRQK_OK;
 }
-

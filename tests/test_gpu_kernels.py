@@ -398,6 +398,32 @@ def test_score_select_diff_unordered(ops, oracle, m, k, H, dtype, r, index, ties
     assert fast > 0
 
 
+@pytest.mark.parametrize("m,k", [(33, 1), (1000, 63), (4000, 1024), (4096, 2048), (8000, 1025), (8190, 2049), (16000, 2049),
+                                 (130, 128)])
+@pytest.mark.parametrize("values", [1, 2, 3])
+def test_score_select_diff_few_distinct_scores(ops, oracle, m, k, values):
+    """Scores of one, two or three values: the whole list, or nearly, is tied at the threshold, and the last token that is
+    taken lies anywhere in the bitmap.  List lengths on both sides of what a thread holds (4, 8, 16 entries)."""
+    g = torch.Generator().manual_seed(m + 7 * k + values)
+    A = torch.zeros((1, 3, m, 16))
+    A[..., 0] = 1.0 + torch.randint(0, values, (1, 3, m), generator=g).float()
+    q = torch.zeros((1, 3, 1, 16))
+    q[..., 0] = 1.0
+    A, q = A.bfloat16(), q.bfloat16()
+    now = torch.stack([torch.randperm(m, generator=g)[:k] for _ in range(3)]).view(1, 3, k, 1)
+    hit = now[..., 0].to(torch.int32).to(DEV).contiguous()
+    ws, Ad = ops.Workspace(), A.to(DEV)
+    new = oracle.compute_hit_indices(q, A, k, True)
+    for rnd in range(3):   # (the first call has no bound yet)
+        if rnd == 2:       # another resident set
+            now = torch.stack([torch.randperm(m, generator=g)[:k] for _ in range(3)]).view(1, 3, k, 1)
+            hit.copy_(now[..., 0])
+        now, gone = oracle.only_indices_in_cpu(now, new)
+        _, evict, slots, count = ops.score_select_diff(ws, Ad, q.to(DEV), m, k, hit, want_new=False)
+        assert torch.equal(hit.cpu().long(), now[..., 0]) and torch.equal(evict.cpu().bool(), gone), rnd
+        assert torch.equal(count.cpu().long(), gone.sum(-1)), rnd
+
+
 def test_score_select_many_chunks(ops, ws, oracle):
     """More candidates than one bitmap chunk covers (262144): the ordered output runs chunk by chunk."""
     _say("score_select many chunks")
