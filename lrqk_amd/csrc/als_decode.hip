@@ -284,6 +284,8 @@ __global__ __launch_bounds__(kGramThreads) void als_gram_kernel(const T* __restr
 // cost); a wave walks its rows chunk by chunk with the next chunk's K and A rows and the ids of the chunk after
 // it already requested, and no workgroup barrier inside the loop; all LDS is one static block shared by the
 // roles, so the launch is bounded by registers (4 workgroups per CU), not by the extra workgroups' B tile.
+// Launch, us, before and after its loads took one id and 32-bit offsets: 32 heads x 2112 slots 9.3 -> 9.1 (every second step's
+// operands from HBM: 11.0 -> 10.6), 128 heads 25.4 -> 24.4, 32 x 1040 slots at r 16 7.5 -> 6.5.
 typedef __bf16 gram_bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int kGramSmemFloats = 32 * (128 + 1) + 2 * 128;  // the extra workgroups' need at d = 128 (>= 4 * kGramNe)
 static_assert(kGramSmemFloats >= kGramWaves * kGramNe, "the cross-wave reduction fits the shared block");
@@ -292,6 +294,163 @@ __device__ __forceinline__ void gram_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The ring append of the step, by the first lanes of one workgroup per head: the new token's rows into their slot, its id into
+// the table.  (The workgroups that walk the slots take the new token's row from where the caller left it.)
+template <typename T, int LPR>
+__device__ __forceinline__ void gram_append(const GramAppend& ap, T* k_prev, int64_t idx_stride, int kprev_slots, int h) {
+  constexpr int VEC = Vec16<T>::N, d = LPR * VEC;
+  const int lane = threadIdx.x;
+  if (ap.slot < 0 || lane >= LPR) return;
+  const int64_t so = ((int64_t)(h / ap.hq) * ap.hkv + (h % ap.hq) / (ap.hq / ap.hkv)) * d + lane * VEC;
+  const int64_t dof = ((int64_t)h * kprev_slots + ap.slot) * d + lane * VEC;
+  Vec16<T> kx, vx;
+  kx.load((const T*)ap.k_new + so);
+  vx.load((const T*)ap.v_new + so);
+  *reinterpret_cast<decltype(kx.raw)*>(k_prev + dof) = kx.raw;
+  *reinterpret_cast<decltype(vx.raw)*>((T*)ap.v_act + dof) = vx.raw;
+  if (lane == 0) ap.idx_out[(int64_t)h * idx_stride + ap.slot] = ap.token;
+}
+
+// The same pass as als_gram_kernel, sums in the same order, for rows of LPR pieces of 16 bytes (d = 32 .. 128) and A_K rows of
+// whole, aligned pieces.  That kernel asks for 16 token ids per lane, then for half of the K rows, the other half and 16
+// single elements of A, one wait after the other, in 1900 instructions; here a lane has one id and 16-byte pieces of A, which
+// reach the operand layout through a wave-private tile in LDS, and the K rows are on their way with them: two round trips.
+// Launch, us: 28 fp32 heads of 128 x 544 slots 9.9 -> 6.7, 96 bf16 heads of 64 x 1040 slots 17.9 -> 11.3.
+constexpr int kGramLd = 36;  // floats per tile row (16-byte aligned, rows four banks apart)
+constexpr int kGramTile = kGramChunk * kGramLd;
+constexpr int kGramVecSmem = kGramWaves * (kGramTile + kGramChunk);  // also the waves' sums, also the extra workgroups' B
+static_assert(kGramVecSmem >= kGramWaves * kGramNe && kGramVecSmem >= 32 * (128 + 1) + 2 * 128, "one block for all");
+template <typename T, int LPR>
+__global__ __launch_bounds__(kGramThreads) void als_gram_vec_kernel(
+    const T* __restrict__ a_k, int64_t head_stride, int64_t a_rows, const int32_t* __restrict__ active_idx, int64_t idx_stride,
+    T* k_prev, int kprev_slots, int n, const T* __restrict__ q, int r, float* __restrict__ part, int S, GramAppend ap,
+    const T* __restrict__ b_q, const T* __restrict__ b_k, const T* __restrict__ k_new, int hq, int hkv, float* __restrict__ pre,
+    float* __restrict__ kq_out) {
+  constexpr int VEC = Vec16<T>::N, d = LPR * VEC, gpw = kWave / LPR;
+  constexpr int KL = kGramChunk / gpw;                // K loads per lane and chunk
+  constexpr int PR = 32 / VEC;                        // pieces of a tile row
+  constexpr int AL = kGramChunk * PR / kWave;         // A loads per lane and chunk
+  constexpr int kLprLog2 = LPR == 8 ? 3 : LPR == 16 ? 4 : 5;
+  static_assert(LPR == 8 || LPR == 16 || LPR == 32, "");
+  __shared__ __align__(16) float gsm[kGramVecSmem];
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int h = blockIdx.y, s = blockIdx.x;
+  if (s >= S) {  // two workgroups per head beside the S splits
+    als_bgram_body<T>(b_q, b_k, q, k_new, h, hq, hkv, r, d, kLprLog2, pre + (int64_t)h * kPreNe, gsm, s - S);
+    if (s == S + 1) gram_append<T, LPR>(ap, k_prev, idx_stride, kprev_slots, h);
+    return;
+  }
+  float* At = gsm + wave * (kGramTile + kGramChunk);  // this wave's A rows [32][kGramLd]
+  float* w_s = At + kGramTile;                        // and products K q
+  const int sub = lane & (LPR - 1), grp = lane / LPR;
+  const int rows_per_split = (n + S - 1) / S;
+  const int s0 = s * rows_per_split;
+  const int s1 = min(n, s0 + rows_per_split);
+  const int rows_per_wave = (rows_per_split + kGramWaves - 1) / kGramWaves;
+  const int w0 = s0 + wave * rows_per_wave;
+  const int w1 = min(s1, w0 + rows_per_wave);
+  const int n_chunks = (rows_per_wave + kGramChunk - 1) / kGramChunk;
+  const T* A = a_k + (int64_t)h * head_stride;
+  const T* Kp = k_prev + (int64_t)h * kprev_slots * d;
+  // (without a table slot t holds token t; the load then reads something and its value is not used)
+  const int32_t* ids = active_idx ? active_idx + (int64_t)h * idx_stride : reinterpret_cast<const int32_t*>(q);
+  const int col = lane & 31, khalf = lane >> 5;
+  const int pieces = r / VEC;
+  // the new token's K row (its slot holds another token's, or already this one: gram_append)
+  const int64_t so = ap.slot >= 0 ? ((int64_t)(h / hq) * hkv + (h % hq) / (hq / hkv)) * d + sub * VEC : 0;
+  Vec16<T> kn;
+  kn.load((ap.slot >= 0 ? (const T*)ap.k_new : Kp) + so);
+  Vec16<T> qv;
+  qv.load(q + (int64_t)h * d + sub * VEC);
+  v16f acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+  float racc = 0.0f;
+  const uint32_t k_off = (uint32_t)((w0 + grp) * d + sub * VEC) * sizeof(T), k_last = (uint32_t)((n - 1) * d + sub * VEC) * sizeof(T);
+  for (int ch = 0; ch < n_chunks; ++ch) {
+    const int c0 = w0 + ch * kGramChunk;
+    // every load is unconditional: indices are clamped into range and the results masked afterwards
+    const int t_mine = min(c0 + (lane & (kGramChunk - 1)), n - 1);
+    int id = ids[active_idx ? t_mine : 0];
+    Vec16<T> kv[KL];
+#pragma unroll
+    for (int u = 0; u < KL; ++u)
+      kv[u].load(reinterpret_cast<const T*>(reinterpret_cast<const char*>(Kp) +
+                                            min(k_off + (uint32_t)((ch * kGramChunk + u * gpw) * d * (int)sizeof(T)), k_last)));
+    __builtin_amdgcn_sched_barrier(0);  // (the K rows do not wait for the id: left to itself the compiler asks for them behind)
+    id = t_mine == ap.slot ? ap.token : active_idx ? id : t_mine;
+    id = c0 + (lane & (kGramChunk - 1)) < w1 && (int64_t)id < a_rows ? id : -1;  // (-1: the row does not count)
+    Vec16<T> av[AL];
+    int row_id[AL];
+#pragma unroll
+    for (int j = 0; j < AL; ++j) {
+      const int p = lane + j * kWave;
+      row_id[j] = __shfl(id, p / PR, kWave);
+      av[j].load(A + (int64_t)max(row_id[j], 0) * r + min(p % PR, pieces - 1) * VEC);
+    }
+    float qf[VEC];
+    qv.unpack(qf);
+    if (ap.slot >= c0 && ap.slot < c0 + kGramChunk) {  // (uniform)
+#pragma unroll
+      for (int u = 0; u < KL; ++u)
+        if (c0 + u * gpw + grp == ap.slot) kv[u].raw = kn.raw;
+    }
+#pragma unroll
+    for (int u = 0; u < KL; ++u) {
+      const int row = u * gpw + grp;
+      float kf[VEC];
+      kv[u].unpack(kf);
+      float wv = 0.0f;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) wv = fmaf(kf[e], qf[e], wv);
+      wv = group_sum(wv, LPR);
+      if (sub == 0) w_s[row] = (c0 + row < w1) ? wv : 0.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < AL; ++j) {
+      const int p = lane + j * kWave, pc = p % PR;
+      const bool ok = row_id[j] >= 0 && pc < pieces;
+      float f[VEC];
+      av[j].unpack(f);
+#pragma unroll
+      for (int x = 0; x < VEC / 4; ++x)
+        *reinterpret_cast<float4*>(At + (p / PR) * kGramLd + pc * VEC + 4 * x) =
+            ok ? make_float4(f[4 * x], f[4 * x + 1], f[4 * x + 2], f[4 * x + 3]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    gram_wave_sync();
+    // K q of the wave's rows for the attention that ends the step (it then reads only V)
+    if (kq_out && lane < kGramChunk && c0 + lane < w1) kq_out[(int64_t)h * n + c0 + lane] = w_s[lane];
+    // lane (col, khalf) takes element col of tokens 2g + khalf
+    float a0[kGramChunk / 2], wr[kGramChunk / 2];
+#pragma unroll
+    for (int g = 0; g < kGramChunk / 2; ++g) {
+      a0[g] = At[(2 * g + khalf) * kGramLd + col];
+      wr[g] = w_s[2 * g + khalf];
+    }
+#pragma unroll
+    for (int g = 0; g < kGramChunk / 2; ++g) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[g], a0[g], acc, 0, 0, 0);
+      racc = fmaf(wr[g], a0[g], racc);
+    }
+    gram_wave_sync();  // the tile and w_s are rewritten by the next chunk
+  }
+  racc += __shfl_xor(racc, 32, kWave);
+  // ---- cross-wave reduction through the same block of LDS
+  __syncthreads();
+  float* red = gsm;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) red[wave * kGramNe + mfma_row(lane, v) * 32 + col] = acc[v];
+  if (lane < 32) red[wave * kGramNe + 32 * 32 + col] = racc;
+  __syncthreads();
+  float* pout = part + ((int64_t)h * S + s) * kGramNe;
+  for (int e = tid; e < kGramNe; e += kGramThreads) {
+    float v = 0.0f;
+#pragma unroll
+    for (int wv = 0; wv < kGramWaves; ++wv) v += red[wv * kGramNe + e];
+    pout[e] = v;
+  }
 }
 
 __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
@@ -306,6 +465,7 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
   const int h = blockIdx.y, s = blockIdx.x;
   if (s >= S) {
     als_bgram_body<bf16_t>(b_q, b_k, q, k_new, h, hq, hkv, r, d, lpr_log2, pre + (int64_t)h * kPreNe, gsm, s - S);
+    if (s == S + 1) gram_append<bf16_t, lpr>(ap, k_prev, idx_stride, kprev_slots, h);
     return;
   }
   // wave-private: the chunk's A rows as bf16 [32][32] (64-byte rows), and its 32 products K q
@@ -326,11 +486,11 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
   const bf16_t* A = a_k + (int64_t)h * head_stride;
   const bf16_t* Kp = k_prev + (int64_t)h * kprev_slots * d;
   const int col = lane & 31, khalf = lane >> 5;
-  const bf16_t* knew_h = Kp;
-  if (ap.slot >= 0) {
-    const int bb = h / ap.hq, kvh = (h % ap.hq) / (ap.hq / ap.hkv);
-    knew_h = (const bf16_t*)ap.k_new + ((int64_t)bb * ap.hkv + kvh) * d;
-  }
+  // the new token's K row (its slot holds another token's, or already this one: gram_append)
+  const int bb = h / hq, kvh = (h % hq) / (hq / hkv);
+  const int64_t so = ap.slot >= 0 ? ((int64_t)bb * hkv + kvh) * d + sub * VEC : 0;
+  Vec16<bf16_t> kn;
+  kn.load((ap.slot >= 0 ? (const bf16_t*)ap.k_new : Kp) + so);
   uint32_t qw[4];  // this lane's eight elements of q, as stored
   {
     Vec16<bf16_t> qv;
@@ -340,44 +500,52 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
     qw[2] = qv.raw.z;
     qw[3] = qv.raw.w;
   }
-  // every load is unconditional: indices are clamped into range and the results masked afterwards
-  auto load_ids = [&](int c0, int32_t (&tok)[2]) {
+  // Every load is unconditional: indices are clamped into range and the results masked afterwards.  A lane has the id of one
+  // token of a chunk (-1: the row does not count), and offsets have 32 bits: with two ids, 64-bit products and the choice of the
+  // new token's row per load, a wave had issued 280 instructions before its last load went out.
+  const int32_t* ids = active_idx ? active_idx + (int64_t)h * idx_stride : reinterpret_cast<const int32_t*>(q);
+  auto load_ids = [&](int c0) { return ids[active_idx ? min(c0 + (lane & (kGramChunk - 1)), n - 1) : 0]; };
+  auto counted = [&](int c0, int32_t id) {
+    const int t = c0 + (lane & (kGramChunk - 1));
+    id = t == ap.slot ? ap.token : active_idx ? id : t;
+    return t < w1 && (int64_t)id < a_rows ? id : -1;
+  };
+  auto load_a = [&](int32_t id, int32_t (&tok)[2], uint4 (&av)[2]) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int t = min(c0 + arow + 16 * j, n - 1);
-      const int32_t id = active_idx ? active_idx[(int64_t)h * idx_stride + t] : t;
-      tok[j] = t == ap.slot ? ap.token : id;
+      tok[j] = __shfl(id, arow + 16 * j, kWave);
+      av[j] = *reinterpret_cast<const uint4*>(A + (int64_t)max(tok[j], 0) * r + aqc * 8);
     }
   };
-  auto load_a = [&](const int32_t (&tok)[2], uint4 (&av)[2]) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int64_t sr = min(max((int64_t)tok[j], (int64_t)0), a_rows - 1);
-      av[j] = *reinterpret_cast<const uint4*>(A + sr * r + aqc * 8);
-    }
-  };
+  const uint32_t k_last = (uint32_t)((n - 1) * d + sub * VEC) * 2u;
   auto load_k = [&](int c0, Vec16<bf16_t> (&kv)[KL]) {
+    const uint32_t off = (uint32_t)((c0 + grp) * d + sub * VEC) * 2u;
 #pragma unroll
-    for (int u = 0; u < KL; ++u) {
-      const int row = min(c0 + u * gpw + grp, n - 1);
-      kv[u].load((row == ap.slot ? knew_h : Kp + (int64_t)row * d) + sub * VEC);
-    }
+    for (int u = 0; u < KL; ++u)
+      kv[u].load(reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(Kp) + min(off + (uint32_t)(u * gpw * d * 2), k_last)));
   };
 
   v16f acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
   float racc = 0.0f;
-  int32_t tok_cur[2], tok_nxt[2];
+  int32_t tok_cur[2], id_nxt;
   uint4 a_cur[2];
   Vec16<bf16_t> kv[KL];
-  load_ids(w0, tok_cur);
+  const int32_t id_first = load_ids(w0);
   load_k(w0, kv);
-  load_ids(w0 + kGramChunk, tok_nxt);
-  load_a(tok_cur, a_cur);
+  id_nxt = load_ids(w0 + kGramChunk);
+  __builtin_amdgcn_sched_barrier(0);  // (the K rows do not wait for the ids: left to itself the compiler asks for them behind)
+  load_a(counted(w0, id_first), tok_cur, a_cur);
 
-  for (int ch = 0; ch < n_chunks; ++ch) {
+  int ch = 0;
+  do {  // (at least one chunk: the first loads are not moved behind a test)
     const int c0 = w0 + ch * kGramChunk;
+    if (ap.slot >= c0 && ap.slot < c0 + kGramChunk) {  // (uniform)
+#pragma unroll
+      for (int u = 0; u < KL; ++u)
+        if (c0 + u * gpw + grp == ap.slot) kv[u].raw = kn.raw;
+    }
     // K q of the chunk's rows: products of bf16 pairs summed in fp32 (q stays in its storage form)
 #pragma unroll
     for (int u = 0; u < KL; ++u) {
@@ -393,16 +561,16 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
     }
     // the next chunk's rows and the ids of the one after it (wave-uniform conditions)
     uint4 a_nxt[2] = {a_cur[0], a_cur[1]};
-    int32_t tok_nn[2] = {0, 0};
+    int32_t tok_nxt[2] = {-1, -1}, id_nn = 0;
     if (ch + 1 < n_chunks) {
       load_k(c0 + kGramChunk, kv);
-      load_a(tok_nxt, a_nxt);
+      load_a(counted(c0 + kGramChunk, id_nxt), tok_nxt, a_nxt);
     }
-    if (ch + 2 < n_chunks) load_ids(c0 + 2 * kGramChunk, tok_nn);
+    if (ch + 2 < n_chunks) id_nn = load_ids(c0 + 2 * kGramChunk);
     // this chunk's A rows into the tile (rows that do not count, and columns >= r, as zeros)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const bool ok = (c0 + arow + 16 * j < w1) && tok_cur[j] >= 0 && (int64_t)tok_cur[j] < a_rows && aq < lpa;
+      const bool ok = tok_cur[j] >= 0 && aq < lpa;
       const uint4 v = ok ? a_cur[j] : make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4*>(At + (arow + 16 * j) * 32 + aq * 8) = v;
     }
@@ -430,21 +598,10 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
     for (int j = 0; j < 2; ++j) {
       a_cur[j] = a_nxt[j];
       tok_cur[j] = tok_nxt[j];
-      tok_nxt[j] = tok_nn[j];
     }
-  }
+    id_nxt = id_nn;
+  } while (++ch < n_chunks);
   racc += __shfl_xor(racc, 32, kWave);
-  if (ap.slot >= w0 && ap.slot < w1 && lane < lpr) {  // this wave owns the new token's slot
-    const int bb = h / ap.hq, kvh = (h % ap.hq) / (ap.hq / ap.hkv);
-    const int64_t so = ((int64_t)bb * ap.hkv + kvh) * d + lane * VEC;
-    const int64_t dof = ((int64_t)h * kprev_slots + ap.slot) * d + lane * VEC;
-    Vec16<bf16_t> kx, vx;
-    kx.load((const bf16_t*)ap.k_new + so);
-    vx.load((const bf16_t*)ap.v_new + so);
-    *reinterpret_cast<decltype(kx.raw)*>(k_prev + dof) = kx.raw;
-    *reinterpret_cast<decltype(vx.raw)*>((bf16_t*)ap.v_act + dof) = vx.raw;
-    if (lane == 0) ap.idx_out[(int64_t)h * idx_stride + ap.slot] = ap.token;
-  }
   // ---- cross-wave reduction through the same block of LDS
   __syncthreads();
   float* red = gsm;
@@ -1112,7 +1269,7 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
   if (S < 1) S = 1;
   if (S > 32) S = 32;
   // bf16, d = 128, r in {8, 16, 24, 32}, 16-byte aligned rows: the pipelined pass on the bf16 matrix cores
-  const bool fast_bf16 = sizeof(T) == 2 && d == 128 && r % 8 == 0 && ((uintptr_t)a_k % 16 == 0) &&
+  const bool fast_bf16 = sizeof(T) == 2 && d == 128 && r % 8 == 0 && ((uintptr_t)a_k % 16 == 0) && n < (1 << 23) &&
                          (head_stride * sizeof(T)) % 16 == 0 && !getenv("LRQK_GRAM_OLD");
   // (the pipelined pass: two chunks per wave measured best at 1, 4 and 8 sequences of the Llama-3-8B shape)
   if (fast_bf16) S = std::min(32, std::max(1, (n + 2 * kGramWaves * kGramChunk - 1) / (2 * kGramWaves * kGramChunk)));
@@ -1145,11 +1302,20 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
     if ((rc = ctx->als_kq.ensure((size_t)bh * n * sizeof(float)))) return rc;
     kq_out = (float*)ctx->als_kq.p;
   }
+  // whole 16-byte pieces of A_K rows, K rows of 8, 16 or 32 pieces (and few enough slots for 32-bit offsets): see
+  // als_gram_vec_kernel
+  const bool vec_rows = r % VEC == 0 && ((uintptr_t)a_k % 16 == 0) && (head_stride * sizeof(T)) % 16 == 0 && d <= 128 &&
+                        (lpr == 8 || lpr == 16 || lpr == 32) && n < (1 << 22);
   if (fast_bf16) {
     hipLaunchKernelGGL(als_gram_bf16_kernel, dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), 0, st,
                        (const bf16_t*)a_k, head_stride, a_rows, active_idx, idx_stride, (bf16_t*)k_prev, kprev_slots, n,
                        (const bf16_t*)q, r, part, S, ap, (const bf16_t*)b_q, (const bf16_t*)b_k, (const bf16_t*)k_new,
                        hq, hkv, pre, kq_out);
+  } else if (vec_rows) {
+    const auto gram = lpr == 8 ? als_gram_vec_kernel<T, 8> : lpr == 16 ? als_gram_vec_kernel<T, 16> : als_gram_vec_kernel<T, 32>;
+    hipLaunchKernelGGL(gram, dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), 0, st, (const T*)a_k, head_stride, a_rows,
+                       active_idx, idx_stride, (T*)k_prev, kprev_slots, n, (const T*)q, r, part, S, ap, (const T*)b_q,
+                       (const T*)b_k, (const T*)k_new, hq, hkv, pre, kq_out);
   } else {
     hipLaunchKernelGGL((als_gram_kernel<T>), dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), smem_gram, st,
                        (const T*)a_k, head_stride, a_rows, active_idx, idx_stride, (T*)k_prev, kprev_slots, n,

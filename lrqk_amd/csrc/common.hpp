@@ -188,8 +188,15 @@ __device__ __forceinline__ float group_sum(float v, int n) {
   if (n > 2) v += dpp_self<kDppQuadXor2>(v);
   if (n > 4) v += dpp_self<kDppRowHalfMirror>(v);
   if (n > 8) v += dpp_self<kDppRowMirror>(v);
-  if (n > 16) v += __shfl_xor(v, 16, kWave);
-  if (n > 32) v += __shfl_xor(v, 32, kWave);
+  // (the two operands after the exchange are the lane's own value and its partner's, in either order)
+  if (n > 16) {
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
+  if (n > 32) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+  }
   return v;
 }
 // wave-wide reductions of unsigned values, result in every lane
