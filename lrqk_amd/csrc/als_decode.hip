@@ -620,12 +620,6 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
 
 // Everything in the solve kernel works on 32 x 32 tiles padded with an identity block (rows
 // and columns >= r), so every loop has a compile-time trip count and its LDS reads pipeline.
-// Sum of x over lanes 0..31 of the wave (the first two rows of 16 lanes); every lane must call it.
-__device__ __forceinline__ float sum_lanes_0_31(float x) {
-  x = row_reduce(x, [](float a, float b) { return a + b; });
-  return lane_bcast(x, 0) + lane_bcast(x, 16);
-}
-
 // iter_out per head: [max_iter][2r] (q_hat then k_hat of each iteration);
 // deltas: [bh][max_iter] sum over r of (k_hat - k_hat')^2.
 // KS: compile-time bound of the number of Gram splits S (S <= KS): that many 16-byte loads per thread
@@ -633,6 +627,10 @@ __device__ __forceinline__ float sum_lanes_0_31(float x) {
 // (Two workgroups per CU as the launch bound where the partial sums leave room: with at most 256 registers per
 // lane the matrix cores take their accumulators in ordinary registers, and a sweep reads its pivot row without
 // copying the whole tile out of the accumulation registers.)
+// One workgroup per head: latency and the instructions of one wave bound it, not memory.  Launch, us, before and after the
+// matrices went to LDS complete and the products of the iterations took their vector by the row of lanes (every step's
+// average): 32 heads, r = 32, two iterations 8.4 -> 7.1; 4 x 32 heads 8.6 -> 7.5; r = 16, eight iterations 10.6 -> 7.6.  Mean
+// error of q_hat and k_hat against 64 bits: 1.000 and 0.999 of what it was.
 template <int KS>
 __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_kernel(const float* __restrict__ pre,
                                                                   const float* __restrict__ part, int S, int r,
@@ -644,18 +642,13 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
   __shared__ float s_qk;
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int h = blockIdx.x;
-  float* G = sm;                    // [kGramNe] summed A^T [A | w]
+  float* G = sm;                    // [32*32] G_Q = B_Q B_Q^T + A^T A, then [32] A^T w
   float* Mx = G + kGramNe;          // [2][32] row scales of the two inversions (16-byte aligned)
   float* GKi = Mx + 2 * 32;         // [32][kLdi]
   float* GQi = GKi + 32 * kLdi;     // [32][kLdi]
-  float* rhs_q = GQi + 32 * kLdi;   // 6 vectors of 32
+  float* rhs_q = GQi + 32 * kLdi;   // 2 vectors of 32
   float* kB = rhs_q + 32;
-  float* hat_k = kB + 32;
-  float* hat_q = hat_k + 32;
-  float* new_k = hat_q + 32;
-  float* tmp = new_k + 32;
-  float* cred = tmp + 32;           // [2 matrices][2 halves of d][32*32] tiles of B B^T (from the Gram launch)
-  (void)hat_k; (void)hat_q; (void)new_k; (void)tmp;
+  float* GKm = kB + 32;             // [32*32] G_K = B_K B_K^T
 
   // ---- every global load of the kernel is issued here, back to back
   const float* pin = part + (int64_t)h * S * kGramNe;
@@ -671,12 +664,10 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
 #pragma unroll
       for (int t = 0; t < KS; ++t) y[t] = pin4[(int64_t)min(t, S - 1) * kVec + min(kSolveThreads + tid, kVec - 1)];
     }
-    float4 tl4[4];  // the four B B^T tiles: 4096 floats, 16 per thread
+    float4 tl4[4];  // the four B B^T tiles (B_Q, B_K, each over the two halves of d): 4096 floats, 16 per thread
 #pragma unroll
     for (int u = 0; u < 4; ++u) tl4[u] = reinterpret_cast<const float4*>(pr)[tid + u * kSolveThreads];
     const float pv = pr[4 * 1024 + min(tid, 64)];  // q B_Q^T [32] | k B_K^T [32] | q . k
-#pragma unroll
-    for (int u = 0; u < 4; ++u) reinterpret_cast<float4*>(cred)[tid + u * kSolveThreads] = tl4[u];
     auto sum_splits = [&](const float4 (&v)[KS]) {  // fixed order 0..S-1, element-wise
       float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
@@ -688,7 +679,10 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
       }
       return a;
     };
-    reinterpret_cast<float4*>(G)[tid] = sum_splits(x);
+    // (thread tid has the same four elements of every tile and of the partial sums, so both matrices go to LDS complete)
+    auto add4 = [](const float4& a, const float4& b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); };
+    reinterpret_cast<float4*>(GKm)[tid] = add4(tl4[2], tl4[3]);
+    reinterpret_cast<float4*>(G)[tid] = add4(add4(tl4[0], tl4[1]), sum_splits(x));
     if (wave == 0 && kSolveThreads + tid < kVec) reinterpret_cast<float4*>(G)[kSolveThreads + tid] = sum_splits(y);
     // rhs_q = q B_Q^T + (q K^T) A: the second term (G[1024 + i]) is added after the barrier; kB = k B_K^T
     if (tid < 32) rhs_q[tid] = pv;
@@ -699,9 +693,8 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
   if (tid < 32) rhs_q[tid] += G[32 * 32 + tid];  // (read again only after the barriers of the inversion)
   // G_K = B_K B_K^T (first wave) and G_Q = B_Q B_Q^T + A^T A (second wave), each inverted by its wave
   if (wave < 2) {
-    const float* c0 = cred + (wave ? 0 : 2048);
-    const float gsel = wave ? 1.0f : 0.0f;
-    auto elem = [&](int i, int j) { return fmaf(gsel, G[i * 32 + j], c0[i * 32 + j] + c0[1024 + i * 32 + j]); };
+    const float* m = wave ? G : GKm;
+    auto elem = [&](int i, int j) { return m[i * 32 + j]; };
     float* const inv = wave ? GQi : GKi;
     if (r & 1)  // (uniform)
       invert_sweep_mfma<32, true>(elem, r, Mx + 32 * wave, inv);
@@ -711,56 +704,60 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
       invert_sweep_mfma<32, false>(elem, r, Mx + 32 * wave, inv);
   }
   __syncthreads();
-  // ---- k_hat_0 and the alternating rank-1 solves, all inside the first wave: lane c (and c + 32)
-  // holds column c of both inverses and element c of every vector; a vector element is
-  // broadcast with readlane, so the chain of small solves needs no barrier and no LDS round trip.
+  // ---- k_hat_0 and the alternating rank-1 solves, all inside the first wave, which nothing runs beside: the chain is what it
+  // issues.  Element c of a vector lies in lane c of every N lanes, and a product with an inverse multiplies by an element that
+  // the row of 16 lanes hands round in the same instruction (32 elements: each half of the wave takes 16 of the terms), so
+  // it is 16 instructions, and 6 more where N is 32, with no scalar register, barrier or LDS round trip in it.
   // (N: the elements that can differ from zero, 16 or 32)
   auto iterate = [&](auto n_c) {
     constexpr int N = decltype(n_c)::value;
-    const int c = lane & 31;
-    float cK[N], cQ[N];
+    const int c = lane & (N - 1), half = lane >> 5;
+    float cK[16], cQ[16];
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      cK[i] = GKi[i * kLdi + c];
-      cQ[i] = GQi[i * kLdi + c];
+    for (int i = 0; i < 16; ++i) {
+      cK[i] = GKi[(i + (N == 32 ? 16 * half : 0)) * kLdi + c];
+      cQ[i] = GQi[(i + (N == 32 ? 16 * half : 0)) * kLdi + c];
     }
     const float rq = rhs_q[c], kb = kB[c], sqk = s_qk;
-    // y_c = sum_i b_i col[i]  (b lane-distributed)
-    auto vecmat = [&](float bvec, const float (&col)[N]) {
-      float y0 = 0.0f, y1 = 0.0f;
-#pragma unroll
-      for (int i = 0; i < N; i += 2) {
-        y0 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i)), col[i], y0);
-        y1 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i + 1)), col[i + 1], y1);
-      }
-      return y0 + y1;
+    // y_c = sum_i b_i G_ic
+    auto vecmat = [&](float bvec, const float (&col)[16]) {
+      float x = bvec;
+      if constexpr (N == 32) x = row_pair(bvec, half);
+      float y = row_dot16(x, col);
+      if constexpr (N == 32) y = half_sum(y);
+      return y;
     };
-    auto dot32 = [&](float a, float bb) { return sum_lanes_0_31(a * bb); };
-    // x = b (G + v^T v)^-1 from G^-1 (Sherman-Morrison): x = y - (y.v / (1 + z.v)) z, y = b G^-1, z = v G^-1.
-    // Both right-hand sides have the form b = b0 + s v, so y = b0 G^-1 + s z: b0 G^-1 is formed once
-    // (for the k side it is k_hat_0 itself) and every solve costs one vector-matrix product.
-    auto rank1 = [&](float y0, float v, const float (&col)[N]) {
+    auto dotn = [&](float a, float bb) {
+      const float x = row_reduce(a * bb, [](float p, float q2) { return p + q2; });
+      if constexpr (N == 32) return row_sum2(x);
+      return x;
+    };
+    // x = b (G + v^T v)^-1 from G^-1 (Sherman-Morrison).  Both right-hand sides have the form b = b0 + s v, so with
+    // y0 = b0 G^-1 (formed once; for the k side it is k_hat_0 itself) and z = v G^-1
+    //   x = y0 + s z - ((y0.v + s z.v) / (1 + z.v)) z = y0 + ((s - y0.v) / (1 + z.v)) z:
+    // one vector-matrix product per solve, and y0.v does not wait for it.
+    auto rank1 = [&](float y0, float v, const float (&col)[16]) {
+      const float a = dotn(y0, v);
       const float z = vecmat(v, col);
-      const float y = fmaf(sqk, z, y0);
-      const float alpha = dot32(y, v) / (1.0f + dot32(z, v));
-      return fmaf(-alpha, z, y);
+      return fmaf((sqk - a) / (1.0f + dotn(z, v)), z, y0);
     };
     const float hk0 = vecmat(kb, cK);  // k_hat_0 = kB G_K^-1
     const float yq0 = vecmat(rq, cQ);  // rhs_q G_Q^-1
-    float hk = hk0;
-    for (int it = 0; it < max_iter; ++it) {
+    float hk = hk0, delta = 0.0f;
+    // lanes 0 .. r - 1 store q_hat, lanes 32 .. 32 + r - 1 k_hat; lane `it` keeps the change of iteration it to the end
+    const bool writes = (lane & 31) < r;
+    float* o = iter_out + (int64_t)h * max_iter * 2 * r + (half ? r : 0) + (lane & 31);
+    for (int it = 0; it < max_iter; ++it, o += 2 * r) {
       const float hq = rank1(yq0, hk, cQ);  // q_hat (G_Q + k_hat^T k_hat) = rhs_q + s k_hat
       const float nk = rank1(hk0, hq, cK);  // k_hat' (G_K + q_hat^T q_hat) = kB + s q_hat
       const float df = c < r ? hk - nk : 0.0f;
-      const float dsq = dot32(df, df);
-      if (lane == 0) deltas[(int64_t)h * max_iter + it] = dsq;
-      float* o = iter_out + ((int64_t)h * max_iter + it) * 2 * r;
-      if (lane < r) {
-        o[lane] = hq;
-        o[r + lane] = nk;
-      }
+      const float dsq = dotn(df, df);
+      delta = lane == it ? dsq : delta;
+      if (writes) *o = half ? nk : hq;
       hk = nk;
     }
+    static_assert(LRQK_MAX_DECODE_ITERS <= kWave, "a lane per iteration");
+    if (lane < max_iter) deltas[(int64_t)h * max_iter + lane] = delta;
   };
   if (wave != 0) return;
   if (r <= 16)  // (uniform)
@@ -1281,8 +1278,8 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
   float* deltas = iter_out + (size_t)bh * max_iter * 2 * r;
   const int64_t a_rows = head_stride / r;
 
-  const size_t smem_solve = ((size_t)kGramNe + 2 * 32 + 2 * 32 * kLdi + 6 * 32 + 4 * 1024) * sizeof(float);
-  static_assert(((size_t)kGramNe + 2 * 32 + 2 * 32 * kLdi + 6 * 32 + 4 * 1024) * sizeof(float) <= 48 * 1024,
+  const size_t smem_solve = ((size_t)kGramNe + 2 * 32 + 2 * 32 * kLdi + 2 * 32 + 1024) * sizeof(float);
+  static_assert(((size_t)kGramNe + 2 * 32 + 2 * 32 * kLdi + 2 * 32 + 1024) * sizeof(float) <= 48 * 1024,
                 "the solve kernel's LDS fits the default dynamic limit");
   // the Gram launch carries two more workgroups per head, each with B_Q or B_K (fp32, padded rows) in LDS
   const size_t smem_gram = ((size_t)32 * (d + 1) + 2 * d) * sizeof(float);

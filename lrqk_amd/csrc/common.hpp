@@ -164,13 +164,23 @@ __device__ __forceinline__ int row_inclusive_sum(int v) {
   return x;
 }
 
+// A move within the row whose source lane always exists, in a wave that is active as a whole: written so that the compiler can
+// make it part of the instruction that uses it (with the lane's own value for a missing source it was a copy and a move more).
+template <int CTRL>
+__device__ __forceinline__ int dpp_full(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_full(float v) {
+  return __int_as_float(dpp_full<CTRL>(__float_as_int(v)));
+}
 // Butterflies inside each row of 16 lanes; afterwards every lane of a row holds the row's result.
 template <typename Op>
 __device__ __forceinline__ float row_reduce(float v, Op op) {
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kDppQuadXor1, 0xf, 0xf, false)));
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kDppQuadXor2, 0xf, 0xf, false)));
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kDppRowHalfMirror, 0xf, 0xf, false)));
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), kDppRowMirror, 0xf, 0xf, false)));
+  v = op(v, dpp_full<kDppQuadXor1>(v));
+  v = op(v, dpp_full<kDppQuadXor2>(v));
+  v = op(v, dpp_full<kDppRowHalfMirror>(v));
+  v = op(v, dpp_full<kDppRowMirror>(v));
   return v;
 }
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
@@ -179,15 +189,11 @@ __device__ __forceinline__ float lane_bcast(float v, int lane) {
 
 // Sum over aligned groups of `n` adjacent lanes (n a power of two); every lane of a group gets
 // the group's sum.  Steps inside a row of 16 lanes are register moves, wider ones shuffles.
-template <int CTRL>
-__device__ __forceinline__ float dpp_self(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
 __device__ __forceinline__ float group_sum(float v, int n) {
-  if (n > 1) v += dpp_self<kDppQuadXor1>(v);
-  if (n > 2) v += dpp_self<kDppQuadXor2>(v);
-  if (n > 4) v += dpp_self<kDppRowHalfMirror>(v);
-  if (n > 8) v += dpp_self<kDppRowMirror>(v);
+  if (n > 1) v += dpp_full<kDppQuadXor1>(v);
+  if (n > 2) v += dpp_full<kDppQuadXor2>(v);
+  if (n > 4) v += dpp_full<kDppRowHalfMirror>(v);
+  if (n > 8) v += dpp_full<kDppRowMirror>(v);
   // (the two operands after the exchange are the lane's own value and its partner's, in either order)
   if (n > 16) {
     const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -202,10 +208,10 @@ __device__ __forceinline__ float group_sum(float v, int n) {
 // wave-wide reductions of unsigned values, result in every lane
 template <typename Op>
 __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t v, Op op) {
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kDppQuadXor1, 0xf, 0xf, false));
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kDppQuadXor2, 0xf, 0xf, false));
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kDppRowHalfMirror, 0xf, 0xf, false));
-  v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, kDppRowMirror, 0xf, 0xf, false));
+  v = op(v, (uint32_t)dpp_full<kDppQuadXor1>((int)v));
+  v = op(v, (uint32_t)dpp_full<kDppQuadXor2>((int)v));
+  v = op(v, (uint32_t)dpp_full<kDppRowHalfMirror>((int)v));
+  v = op(v, (uint32_t)dpp_full<kDppRowMirror>((int)v));
   const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
   const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
   return op(op(a, b), op(c, d));

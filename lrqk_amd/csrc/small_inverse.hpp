@@ -1,5 +1,5 @@
 // Inverse of a small symmetric positive definite matrix on the matrix cores, shared by the decode
-// and the prefill half of the factorisation.
+// and the prefill half of the factorisation, and products of a vector in a wave's lanes with one.
 #pragma once
 #include <type_traits>
 
@@ -19,6 +19,37 @@ constexpr int kLdi = 33;  // row stride of an inverse in LDS
 __device__ __forceinline__ float half_pair(float lo_src, float hi_src, int hp) {
   const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo_src), __float_as_uint(hi_src), false, false);
   return __uint_as_float(hp ? sw[1] : sw[0]);
+}
+
+// y + sum_i x_i col[i] over the 16 lanes of a row, x_i being lane i of the row: the multiply-add itself hands the lane's value round
+// (row_newbcast).  (In assembly: from the builtins come a move and a multiply-add each.  A moved operand must be two
+// instructions old, and so must the result for whoever moves it on.)
+__device__ __forceinline__ float row_dot16(float x, const float* col, float y = 0.0f) {
+#define LRQK_BCAST_FMA(I, C) "v_fmac_f32_dpp %0, %1, %" #C " row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t" LRQK_BCAST_FMA(0, 2) LRQK_BCAST_FMA(1, 3) LRQK_BCAST_FMA(2, 4) LRQK_BCAST_FMA(3, 5) LRQK_BCAST_FMA(4, 6)
+          LRQK_BCAST_FMA(5, 7) LRQK_BCAST_FMA(6, 8) LRQK_BCAST_FMA(7, 9) LRQK_BCAST_FMA(8, 10) LRQK_BCAST_FMA(9, 11)
+              LRQK_BCAST_FMA(10, 12) LRQK_BCAST_FMA(11, 13) LRQK_BCAST_FMA(12, 14) LRQK_BCAST_FMA(13, 15)
+                  LRQK_BCAST_FMA(14, 16) LRQK_BCAST_FMA(15, 17) "s_nop 1"
+      : "+v"(y)
+      : "v"(x), "v"(col[0]), "v"(col[1]), "v"(col[2]), "v"(col[3]), "v"(col[4]), "v"(col[5]), "v"(col[6]), "v"(col[7]),
+        "v"(col[8]), "v"(col[9]), "v"(col[10]), "v"(col[11]), "v"(col[12]), "v"(col[13]), "v"(col[14]), "v"(col[15]));
+#undef LRQK_BCAST_FMA
+  return y;
+}
+// Of a vector that both halves of the wave hold in their two rows: its first 16 elements in both rows of the lower half, the
+// other 16 in those of the upper.
+__device__ __forceinline__ float row_pair(float x, int half) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(half ? sw[1] : sw[0]);
+}
+// Sums over a pair of rows, over the two halves; every lane gets its own.
+__device__ __forceinline__ float row_sum2(float x) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+__device__ __forceinline__ float half_sum(float x) {
+  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
 }
 
 // Inverse of one SPD 32 x 32 matrix by one wave, as symmetric sweeps on the matrix cores, two pivots at a time.  The
