@@ -1219,7 +1219,7 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
     if ((rc = ctx->als_iter.ensure((size_t)bh * max_iter * (2 * r + 1) * sizeof(float)))) return rc;
     float* iter_out = (float*)ctx->als_iter.p;
     float* deltas = iter_out + (size_t)bh * max_iter * 2 * r;
-    if (als_r64_supported(sizeof(T) == 2 ? LRQK_BF16 : LRQK_F32, r, d, a_k, head_stride)) {
+    if (als_r64_supported(sizeof(T) == 2 ? LRQK_BF16 : LRQK_F32, r, d, n, a_k, head_stride)) {
       // bf16 rows of 128 elements: both launches on the matrix cores
       float* kq_out = nullptr;
       if (defer_finish && ap.slot >= 0 && n == kprev_slots) {

@@ -5,12 +5,18 @@
 //   gram  : grid (S, heads).  A^T A (64 x 64: three 32 x 32 tiles, the fourth is a transpose), A^T w and w = K q over
 //           the active rows, as in the pass for r <= 32: 16-byte loads, a wave-private LDS tile that turns the rows into
 //           the operand layout of the bf16 matrix cores (bf16 x bf16 products are exact in fp32), the next chunk's rows
-//           in flight while a chunk is multiplied.  Per-workgroup partial sums go to HBM.
-//   solve : one workgroup of 512 threads per head.  Adds the partial sums; B_Q B_Q^T, B_K B_K^T, q B_Q^T and k B_K^T on
-//           the bf16 matrix cores straight from the stored rows (a lane's operand is 16 contiguous bytes of a row); each
-//           64 x 64 matrix is then inverted by ONE wave as 32 symmetric sweeps on pairs of pivots, on 2 x 2 accumulator
-//           tiles of the fp32 matrix cores (four rank-2 updates per pair, no barrier), G_Q and G_K side by side on two
-//           waves; one wave runs the alternating rank-1 (Sherman-Morrison) iterations with a vector per lane.
+//           in flight while a chunk is multiplied.  Per-workgroup partial sums go to HBM.  The eight waves that a CU holds
+//           are bound by what they issue, so the addresses are what is worth sparing: one id per lane instead of eight,
+//           offsets of 32 bits, a partial result without the mirrored tile (32 heads, 2048 active rows, r = 64: 19.7 ->
+//           14.7 us).
+//   solve : one workgroup of 512 threads per head.  Adds the partial sums (sixteen results in flight); B_Q B_Q^T, B_K B_K^T,
+//           q B_Q^T and k B_K^T on the bf16 matrix cores straight from the stored rows (a lane's operand is 16 contiguous
+//           bytes of a row); each 64 x 64 matrix is then inverted by ONE wave as 32 symmetric sweeps on pairs of pivots, on
+//           2 x 2 accumulator tiles of the fp32 matrix cores (four rank-2 updates per pair, no barrier), G_Q and G_K side by
+//           side on two waves, while a third puts the new token into the ring; one wave runs the alternating rank-1
+//           (Sherman-Morrison) iterations with a vector per lane.  21.7 us (24.9 before the iterations kept the inverses in
+//           registers and the loads were put in flight together): 4.3 loads, 3.6 tiles, 9.4 inversion -- a serial chain of 32
+//           pairs of pivots --, 3.6 two iterations.
 // Same outputs as the kernels for r <= 32 (iter_out, deltas), so the finish stage and the scan take over unchanged.
 #include <algorithm>
 #include <atomic>
@@ -29,8 +35,8 @@ constexpr int kG64Threads = 256;
 constexpr int kG64Waves = kG64Threads / kWave;
 constexpr int kG64Chunk = 32;           // tokens per wave and chunk
 constexpr int kG64Ld = 72;              // 16-bit elements per staged row of A: 144 bytes, see the operand gather below
-constexpr int kG64Ne = 64 * 64 + 64;    // floats of a partial result: A^T A (row stride 64), then A^T w
-constexpr int kG64Red = 3 * 1024 + 64;  // floats a wave contributes to the cross-wave sum: tiles (0,0), (0,1), (1,1), A^T w
+constexpr int kG64Ne = 3 * 1024 + 64;   // floats of a partial result: tiles (0,0), (0,1), (1,1) of A^T A, then A^T w
+constexpr int kG64Red = kG64Ne;         // what a wave contributes to the cross-wave sum
 static_assert(kG64Waves * (kG64Chunk * kG64Ld / 2 + kG64Chunk) <= kG64Waves * kG64Red, "the tiles fit the shared block");
 
 __device__ __forceinline__ void r64_wave_sync() {
@@ -67,10 +73,11 @@ __global__ __launch_bounds__(kG64Threads, 2) void als_gram64_bf16_kernel(
   const bf16_t* A = a_k + (int64_t)h * head_stride;
   const bf16_t* Kp = k_prev + (int64_t)h * kprev_slots * d;
   const int col = lane & 31, khalf = lane >> 5;
-  const bf16_t* knew_h = Kp;
-  if (ap.slot >= 0) {
-    const int bb = h / ap.hq, kvh = (h % ap.hq) / (ap.hq / ap.hkv);
-    knew_h = (const bf16_t*)ap.k_new + ((int64_t)bb * ap.hkv + kvh) * d;
+  // the new token's K row (its slot still holds another token's: als_solve64_bf16_kernel puts the rows there)
+  uint4 kn;
+  {
+    const int64_t so = ap.slot >= 0 ? ((int64_t)(h / ap.hq) * ap.hkv + (h % ap.hq) / (ap.hq / ap.hkv)) * d + sub * VEC : 0;
+    kn = *reinterpret_cast<const uint4*>((ap.slot >= 0 ? (const bf16_t*)ap.k_new : Kp) + so);
   }
   uint32_t qw[4];  // this lane's eight elements of q, as stored
   {
@@ -80,44 +87,49 @@ __global__ __launch_bounds__(kG64Threads, 2) void als_gram64_bf16_kernel(
     qw[2] = qv.z;
     qw[3] = qv.w;
   }
-  // every load is unconditional: indices are clamped into range and the results masked afterwards
-  auto load_ids = [&](int c0, int32_t (&tok)[AL]) {
-#pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      const int t = min(c0 + arow + 8 * j, n - 1);
-      const int32_t id = active_idx ? active_idx[(int64_t)h * idx_stride + t] : t;
-      tok[j] = t == ap.slot ? ap.token : id;
-    }
+  // Every load is unconditional: indices are clamped into range and the results masked afterwards.  A lane has the id of one
+  // token of a chunk (-1: the row does not count), and offsets have 32 bits (see als_gram_bf16_kernel).
+  const int32_t* ids = active_idx ? active_idx + (int64_t)h * idx_stride : reinterpret_cast<const int32_t*>(q);
+  auto load_ids = [&](int c0) { return ids[active_idx ? min(c0 + (lane & (kG64Chunk - 1)), n - 1) : 0]; };
+  auto counted = [&](int c0, int32_t id) {
+    const int t = c0 + (lane & (kG64Chunk - 1));
+    id = t == ap.slot ? ap.token : active_idx ? id : t;
+    return t < w1 && (int64_t)id < a_rows ? id : -1;
   };
-  auto load_a = [&](const int32_t (&tok)[AL], uint4 (&av)[AL]) {
+  auto load_a = [&](int32_t id, uint4 (&av)[AL]) {
 #pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      const int64_t sr = min(max((int64_t)tok[j], (int64_t)0), a_rows - 1);
-      av[j] = *reinterpret_cast<const uint4*>(A + sr * r + aqc * 8);
-    }
+    for (int j = 0; j < AL; ++j)
+      av[j] = *reinterpret_cast<const uint4*>(A + (int64_t)max(__shfl(id, arow + 8 * j, kWave), 0) * r + aqc * 8);
   };
+  const uint32_t k_last = (uint32_t)((n - 1) * d + sub * VEC) * 2u;
   auto load_k = [&](int c0, uint4 (&kv)[KL]) {
+    const uint32_t off = (uint32_t)((c0 + grp) * d + sub * VEC) * 2u;
 #pragma unroll
-    for (int u = 0; u < KL; ++u) {
-      const int row = min(c0 + u * gpw + grp, n - 1);
-      kv[u] = *reinterpret_cast<const uint4*>((row == ap.slot ? knew_h : Kp + (int64_t)row * d) + sub * VEC);
-    }
+    for (int u = 0; u < KL; ++u)
+      kv[u] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(Kp) + min(off + (uint32_t)(u * gpw * d * 2), k_last));
   };
 
   v16f acc00, acc01, acc11;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc00[v] = acc01[v] = acc11[v] = 0.0f;
   float racc0 = 0.0f, racc1 = 0.0f;
-  int32_t tok_cur[AL], tok_nxt[AL];
   uint4 a_cur[AL];
   uint4 kv[KL];
-  load_ids(w0, tok_cur);
+  int32_t id_cur = load_ids(w0);
   load_k(w0, kv);
-  load_ids(w0 + kG64Chunk, tok_nxt);
-  load_a(tok_cur, a_cur);
+  int32_t id_nxt = load_ids(w0 + kG64Chunk);
+  __builtin_amdgcn_sched_barrier(0);  // (the K rows do not wait for the ids)
+  id_cur = counted(w0, id_cur);
+  load_a(id_cur, a_cur);
 
-  for (int ch = 0; ch < n_chunks; ++ch) {
+  int ch = 0;
+  do {  // (at least one chunk)
     const int c0 = w0 + ch * kG64Chunk;
+    if (ap.slot >= c0 && ap.slot < c0 + kG64Chunk) {  // (uniform)
+#pragma unroll
+      for (int u = 0; u < KL; ++u)
+        if (c0 + u * gpw + grp == ap.slot) kv[u] = kn;
+    }
     // K q of the chunk's rows: products of bf16 pairs summed in fp32 (q stays in its storage form)
 #pragma unroll
     for (int u = 0; u < KL; ++u) {
@@ -131,26 +143,20 @@ __global__ __launch_bounds__(kG64Threads, 2) void als_gram64_bf16_kernel(
       wv = group_sum(wv, lpr);
       if (sub == 0) w_s[row] = (c0 + row < w1) ? wv : 0.0f;
     }
-    // the next chunk's rows and the ids of the one after it (wave-uniform conditions)
-    uint4 a_nxt[AL];
-    int32_t tok_nn[AL];
-#pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      a_nxt[j] = a_cur[j];
-      tok_nn[j] = 0;
-    }
-    if (ch + 1 < n_chunks) {
-      load_k(c0 + kG64Chunk, kv);
-      load_a(tok_nxt, a_nxt);
-    }
-    if (ch + 2 < n_chunks) load_ids(c0 + 2 * kG64Chunk, tok_nn);
     // this chunk's A rows into the tile (rows that do not count, and columns >= r, as zeros)
 #pragma unroll
     for (int j = 0; j < AL; ++j) {
-      const bool ok = (c0 + arow + 8 * j < w1) && tok_cur[j] >= 0 && (int64_t)tok_cur[j] < a_rows && aq < lpa;
+      const bool ok = __shfl(id_cur, arow + 8 * j, kWave) >= 0 && aq < lpa;
       const uint4 v = ok ? a_cur[j] : make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4*>(At + (arow + 8 * j) * kG64Ld + aq * 8) = v;
     }
+    // the next chunk's rows and the ids of the one after it (wave-uniform conditions)
+    if (ch + 1 < n_chunks) {
+      load_k(c0 + kG64Chunk, kv);
+      id_cur = counted(c0 + kG64Chunk, id_nxt);
+      load_a(id_cur, a_cur);
+    }
+    if (ch + 2 < n_chunks) id_nxt = load_ids(c0 + 2 * kG64Chunk);
     r64_wave_sync();
     if (kq_out && lane < kG64Chunk && c0 + lane < w1) kq_out[(int64_t)h * n + c0 + lane] = w_s[lane];
     // Lane (col, khalf) takes eight tokens of a group of 16 as the k elements of one bf16 MFMA: tokens
@@ -181,25 +187,9 @@ __global__ __launch_bounds__(kG64Threads, 2) void als_gram64_bf16_kernel(
       acc11 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(op1, op1, acc11, 0, 0, 0);
     }
     r64_wave_sync();  // the tile and w_s are rewritten by the next chunk
-#pragma unroll
-    for (int j = 0; j < AL; ++j) {
-      a_cur[j] = a_nxt[j];
-      tok_cur[j] = tok_nxt[j];
-      tok_nxt[j] = tok_nn[j];
-    }
-  }
+  } while (++ch < n_chunks);
   racc0 += __shfl_xor(racc0, 32, kWave);
   racc1 += __shfl_xor(racc1, 32, kWave);
-  if (ap.slot >= w0 && ap.slot < w1 && lane < lpr) {  // this wave owns the new token's slot
-    const int bb = h / ap.hq, kvh = (h % ap.hq) / (ap.hq / ap.hkv);
-    const int64_t so = ((int64_t)bb * ap.hkv + kvh) * d + lane * VEC;
-    const int64_t dof = ((int64_t)h * kprev_slots + ap.slot) * d + lane * VEC;
-    const uint4 kx = *reinterpret_cast<const uint4*>((const bf16_t*)ap.k_new + so);
-    const uint4 vx = *reinterpret_cast<const uint4*>((const bf16_t*)ap.v_new + so);
-    *reinterpret_cast<uint4*>(k_prev + dof) = kx;
-    *reinterpret_cast<uint4*>((bf16_t*)ap.v_act + dof) = vx;
-    if (lane == 0) ap.idx_out[(int64_t)h * idx_stride + ap.slot] = ap.token;
-  }
   // ---- cross-wave reduction through the same block of LDS
   __syncthreads();
   float* red = gsm + wave * kG64Red;
@@ -216,21 +206,18 @@ __global__ __launch_bounds__(kG64Threads, 2) void als_gram64_bf16_kernel(
   }
   __syncthreads();
   float* pout = part + ((int64_t)h * S + s) * kG64Ne;
-  for (int e = tid; e < kG64Ne; e += kG64Threads) {
-    int src;
-    if (e < 64 * 64) {
-      const int i = e >> 6, j = e & 63;
-      if (i < 32)
-        src = j < 32 ? i * 32 + j : 1024 + i * 32 + (j - 32);
-      else
-        src = j < 32 ? 1024 + j * 32 + (i - 32) : 2048 + (i - 32) * 32 + (j - 32);
-    } else {
-      src = 3072 + (e - 64 * 64);
-    }
-    float v = 0.0f;
+  static_assert(kG64Ne % 4 == 0, "a partial result is whole vectors");
+  for (int e = tid; e < kG64Ne / 4; e += kG64Threads) {
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-    for (int wv = 0; wv < kG64Waves; ++wv) v += gsm[wv * kG64Red + src];
-    pout[e] = v;
+    for (int wv = 0; wv < kG64Waves; ++wv) {
+      const float4 x = reinterpret_cast<const float4*>(gsm + wv * kG64Red)[e];
+      v.x += x.x;
+      v.y += x.y;
+      v.z += x.z;
+      v.w += x.w;
+    }
+    reinterpret_cast<float4*>(pout)[e] = v;
   }
 }
 
@@ -278,7 +265,6 @@ __device__ __forceinline__ void invert64_sweep_mfma(float* G, int r, float* sbuf
     }
   // (lane-dependent cases by weights of 0 and 1, not by selects between expressions, which compile to divergent
   // branches; the matrix is finite, so a product with a weight of 0 is 0)
-  const float in0 = half == 0 ? 1.0f : 0.0f, in1 = 1.0f - in0;
 #pragma unroll
   for (int p = 0; p < PIVOTS; p += 2) {
     {
@@ -343,7 +329,8 @@ __device__ __forceinline__ void invert64_sweep_mfma(float* G, int r, float* sbuf
 __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
     const float* __restrict__ part, int S, const bf16_t* __restrict__ b_q, const bf16_t* __restrict__ b_k,
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_new, int hq, int hkv, int r, int max_iter,
-    float* __restrict__ iter_out, float* __restrict__ deltas) {
+    float* __restrict__ iter_out, float* __restrict__ deltas, GramAppend ap, bf16_t* k_prev, int kprev_slots,
+    int64_t idx_stride) {
   constexpr int d = 128;
   __shared__ __align__(16) float GQ[64 * kS64Ld];
   __shared__ __align__(16) float GK[64 * kS64Ld];
@@ -380,29 +367,27 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
       for (int kk = 0; kk < 8; ++kk) opj[kk] = make_uint4(0, 0, 0, 0);
     }
   }
-  // ---- the partial sums of A^T A and A^T w: 1040 16-byte vectors per partial result, three per thread
+  // ---- the partial sums of A^T A and A^T w: 784 16-byte vectors per partial result, two per thread, of sixteen results at a time
+  uint4 vop[8], qk_a, qk_b;
   {
-    constexpr int NV = kG64Ne / 4;
+    constexpr int NV = kG64Ne / 4, NP = (NV + kS64Threads - 1) / kS64Threads, kAhead = 16;
     const float4* pin = reinterpret_cast<const float4*>(part + (int64_t)h * S * kG64Ne);
-    float4 ps[3];
-    int f[3];
+    float4 ps[NP];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      ps[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      f[i] = tid + kS64Threads * i;
-    }
+    for (int i = 0; i < NP; ++i) ps[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll 1
-    for (int s0 = 0; s0 < S; s0 += 8) {
-      float4 t[8][3];
+    for (int s0 = 0; s0 < S; s0 += kAhead) {
+      float4 t[kAhead][NP];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
+      for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-        for (int i = 0; i < 3; ++i) t[u][i] = pin[(int64_t)min(s0 + u, S - 1) * NV + min(f[i], NV - 1)];
+        for (int i = 0; i < NP; ++i)
+          t[u][i] = pin[(uint32_t)(min(s0 + u, S - 1) * NV + min(tid + kS64Threads * i, NV - 1))];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kAhead; ++u) {
         const float wgt = s0 + u < S ? 1.0f : 0.0f;  // (finite values: a weight of 0 drops the repeated load)
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
+        for (int i = 0; i < NP; ++i) {
           ps[i].x = fmaf(wgt, t[u][i].x, ps[i].x);
           ps[i].y = fmaf(wgt, t[u][i].y, ps[i].y);
           ps[i].z = fmaf(wgt, t[u][i].z, ps[i].z);
@@ -410,16 +395,28 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
         }
       }
     }
+    // (what the products with the vectors need, while the sums go to LDS)
+    const bf16_t* vec = mat ? qh : kh;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int kk = 0; kk < 8; ++kk) vop[kk] = *reinterpret_cast<const uint4*>(vec + 16 * kk + 8 * khalf);
+    qk_a = *reinterpret_cast<const uint4*>(qh + 8 * min(lane, d / 8 - 1));
+    qk_b = *reinterpret_cast<const uint4*>(kh + 8 * min(lane, d / 8 - 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int f = tid + kS64Threads * i;
       const float v4[4] = {ps[i].x, ps[i].y, ps[i].z, ps[i].w};
-      if (f[i] < 1024) {
-        const int e = 4 * f[i], row = e >> 6, c = e & 63;
+      if (f < 768) {  // tile (0,0), (0,1) -- also (1,0), transposed -- or (1,1)
+        const int tile = f >> 8, row = (f >> 3) & 31, c = 4 * (f & 7);
+        const int gi = row + (tile == 2 ? 32 : 0), gj = c + (tile ? 32 : 0);
 #pragma unroll
-        for (int x = 0; x < 4; ++x) GQ[row * kS64Ld + c + x] = v4[x];
-      } else if (f[i] < NV) {
+        for (int x = 0; x < 4; ++x) {
+          GQ[gi * kS64Ld + gj + x] = v4[x];
+          if (tile == 1) GQ[(gj + x) * kS64Ld + gi] = v4[x];
+        }
+      } else if (f < NV) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) aw_s[4 * (f[i] - 1024) + x] = v4[x];
+        for (int x = 0; x < 4; ++x) aw_s[4 * (f - 768) + x] = v4[x];
       }
     }
   }
@@ -441,13 +438,9 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   // ---- q B_Q^T and k B_K^T: the waves of the first tile row multiply once more, with the vector as row 0 of the
   // left operand (all other rows zero) and the operands of B they already hold; row 0 of the result is the product
   if (TI == 0) {
-    const bf16_t* vec = mat ? qh : kh;
     v16f vacc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) vacc[v] = 0.0f;
-    uint4 vop[8];
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) vop[kk] = *reinterpret_cast<const uint4*>(vec + 16 * kk + 8 * khalf);
     if (col != 0) {
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) vop[kk] = make_uint4(0, 0, 0, 0);
@@ -462,8 +455,7 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   if (wave == kS64Threads / kWave - 1) {
     float v = 0.0f;
     if (lane < d / 8) {
-      const uint4 a = *reinterpret_cast<const uint4*>(qh + 8 * lane), c = *reinterpret_cast<const uint4*>(kh + 8 * lane);
-      const uint32_t a4[4] = {a.x, a.y, a.z, a.w}, b4[4] = {c.x, c.y, c.z, c.w};
+      const uint32_t a4[4] = {qk_a.x, qk_a.y, qk_a.z, qk_a.w}, b4[4] = {qk_b.x, qk_b.y, qk_b.z, qk_b.w};
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         v = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(r64_bf16x2, a4[e]), __builtin_bit_cast(r64_bf16x2, b4[e]), v, false);
@@ -482,6 +474,14 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   }
   if (tid < 64) rhs_s[tid] += tid < r ? aw_s[tid] : 0.0f;
   __syncthreads();
+  // ---- the ring append, by a wave that has nothing else to do
+  if (wave == 2 && ap.slot >= 0 && lane < d / 8) {
+    const int64_t so = ((int64_t)(h / ap.hq) * ap.hkv + (h % ap.hq) / (ap.hq / ap.hkv)) * d + lane * 8;
+    const int64_t dof = ((int64_t)h * kprev_slots + ap.slot) * d + lane * 8;
+    *reinterpret_cast<uint4*>(k_prev + dof) = *reinterpret_cast<const uint4*>((const bf16_t*)ap.k_new + so);
+    *reinterpret_cast<uint4*>((bf16_t*)ap.v_act + dof) = *reinterpret_cast<const uint4*>((const bf16_t*)ap.v_new + so);
+    if (lane == 0) ap.idx_out[(int64_t)h * idx_stride + ap.slot] = ap.token;
+  }
   // ---- both inverses, side by side
   if (wave < 2) {
     if (r <= 48)  // (uniform)
@@ -491,46 +491,57 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   }
   __syncthreads();
   if (wave != 0) return;
-  // ---- the alternating iterations, lane c <-> element c of every vector (zeros beyond r)
-  // out[c] = sum_i in[i] G[i][c]
-  auto vecmat = [&](float in_lane, const float* G) {
-    float v = 0.0f;
+  // ---- the alternating iterations, lane c <-> element c of every vector (zeros beyond r), the inverses' columns in the lanes'
+  // registers (see als_solve_kernel; with every product reading the columns from LDS and handing the vector round by scalar
+  // registers the launch took 24.9 us instead of 22.1)
+  float cQ[64], cK[64];
 #pragma unroll
-    for (int i = 0; i < 64; ++i)
-      v = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(in_lane), i)), G[i * kS64Ld + lane], v);
-    return v;
+  for (int i = 0; i < 64; ++i) {
+    cK[i] = GK[i * kS64Ld + lane];
+    cQ[i] = GQ[i * kS64Ld + lane];
+  }
+  // out_c = sum_i in_i G_ic
+  auto vecmat = [&](float in, const float (&g)[64]) {
+    const uint32_t u = __float_as_uint(in);
+    const auto e = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // rows 0, 0, 2, 2 and 1, 1, 3, 3
+    const auto f = __builtin_amdgcn_permlane32_swap(e[0], e[0], false, false);  // row 0 everywhere, row 2 everywhere
+    const auto k = __builtin_amdgcn_permlane32_swap(e[1], e[1], false, false);
+    float y = row_dot16(__uint_as_float(f[0]), g);
+    y = row_dot16(__uint_as_float(k[0]), g + 16, y);
+    y = row_dot16(__uint_as_float(f[1]), g + 32, y);
+    return row_dot16(__uint_as_float(k[1]), g + 48, y);
+  };
+  auto dot = [&](float a, float c) {
+    return half_sum(row_sum2(row_reduce(a * c, [](float p, float q2) { return p + q2; })));
   };
   const float sqk = sqk_s;
-  const float hk0 = vecmat(kb_s[lane], GK);    // k_hat_0 = k B_K^T G_K^-1
-  const float yq0 = vecmat(rhs_s[lane], GQ);   // rhs_q G_Q^-1
-  float hk = hk0;
-  // x = b (G + v^T v)^-1 with b = b0 + s v, from G^-1 (Sherman-Morrison): z = v G^-1, y = y0 + s z,
-  // x = y - (y . v / (1 + z . v)) z
-  auto rank1 = [&](float y0, float v, const float* G) {
-    const float z = vecmat(v, G);
-    const float y = fmaf(sqk, z, y0);
-    const float yv = wave_sum(y * v);
-    const float zv = wave_sum(z * v);
-    const float alpha = yv / (1.0f + zv);
-    return fmaf(-alpha, z, y);
+  const float hk0 = vecmat(kb_s[lane], cK);    // k_hat_0 = k B_K^T G_K^-1
+  const float yq0 = vecmat(rhs_s[lane], cQ);   // rhs_q G_Q^-1
+  float hk = hk0, delta = 0.0f;
+  auto rank1 = [&](float y0, float v, const float (&g)[64]) {
+    const float a = dot(y0, v);
+    const float z = vecmat(v, g);
+    return fmaf((sqk - a) / (1.0f + dot(z, v)), z, y0);
   };
-  for (int it = 0; it < max_iter; ++it) {
-    const float hqv = rank1(yq0, hk, GQ);   // q_hat (G_Q + k_hat^T k_hat) = rhs_q + s k_hat
-    const float hkn = rank1(hk0, hqv, GK);  // k_hat' (G_K + q_hat^T q_hat) = k B_K^T + s q_hat
-    float df = hk - hkn;
-    df = wave_sum(df * df);
-    if (lane == 0) deltas[(int64_t)h * max_iter + it] = df;
-    float* o = iter_out + ((int64_t)h * max_iter + it) * 2 * r;
+  float* o = iter_out + (int64_t)h * max_iter * 2 * r + lane;
+  for (int it = 0; it < max_iter; ++it, o += 2 * r) {
+    const float hqv = rank1(yq0, hk, cQ);   // q_hat (G_Q + k_hat^T k_hat) = rhs_q + s k_hat
+    const float hkn = rank1(hk0, hqv, cK);  // k_hat' (G_K + q_hat^T q_hat) = k B_K^T + s q_hat
+    const float df = hk - hkn;
+    const float dsq = dot(df, df);
+    delta = lane == it ? dsq : delta;  // (kept to the end by lane `it`)
     if (lane < r) {
-      o[lane] = hqv;
-      o[r + lane] = hkn;
+      o[0] = hqv;
+      o[r] = hkn;
     }
     hk = hkn;
   }
+  if (lane < max_iter) deltas[(int64_t)h * max_iter + lane] = delta;
 }
 
-bool als_r64_supported(int dtype, int r, int d, const void* a_k, int64_t head_stride) {
-  return dtype == LRQK_BF16 && d == 128 && r > 32 && r <= 64 && r % 8 == 0 && ((uintptr_t)a_k % 16 == 0) &&
+bool als_r64_supported(int dtype, int r, int d, int n, const void* a_k, int64_t head_stride) {
+  // (n: a head's active K rows are addressed by 32-bit byte offsets)
+  return dtype == LRQK_BF16 && d == 128 && r > 32 && r <= 64 && r % 8 == 0 && n <= (1 << 23) && ((uintptr_t)a_k % 16 == 0) &&
          (head_stride * 2) % 16 == 0;
 }
 
@@ -560,7 +571,7 @@ int als_r64_update(lrqk_ctx* ctx, const void* b_q, const void* b_k, const void* 
   LRQK_HIP_CHECK(hipGetLastError());
   hipLaunchKernelGGL(als_solve64_bf16_kernel, dim3((unsigned)bh), dim3(kS64Threads), 0, st,
                      (const float*)ctx->als_part.p, S, (const bf16_t*)b_q, (const bf16_t*)b_k, (const bf16_t*)q,
-                     (const bf16_t*)k_new, hq, hkv, r, max_iter, iter_out, deltas);
+                     (const bf16_t*)k_new, hq, hkv, r, max_iter, iter_out, deltas, ap, (bf16_t*)k_prev, kprev_slots, idx_stride);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
