@@ -167,20 +167,20 @@ def prefill_roofline(w, l, iters, ms):
         # problems), and the long axis is read a fixed number of times whatever the iteration count: Q twice (sums over
         # the given factors together with Q^T Q; the final A_Q = Q Mq) or, at rows of 128 and ranks above 32, three times
         # (Q^T Q on its own), K three times, once per kv head (sums over the given factors, K^T K, the final A_K = K Mk;
-        # rows of 64 with a kv head per query head: K^T K with the sums).  HBM bytes: those + the initial factors read +
+        # rows of 128 at ranks up to 32, and rows of 64 with a kv head per query head: K^T K with the sums, two).  HBM bytes: those + the initial factors read +
         # the final factors written (fp32).
         reads_q = 2 if tuned or d == 64 else 3
-        reads_k = 2 if d == 64 and bh == bkv else 3
+        reads_k = 2 if tuned or (d == 64 and bh == bkv) else 3
         bytes_g = (float(reads_q) * bh + float(reads_k) * bkv) * l * d * e + 4.0 * bh * l * r * 4
         gbs = bytes_g / (ms * 1e-3) / 1e9
         # executed bf16 MFMAs of 32x32x16 per 32 rows, with ta x 32 columns of factors and td x 32 of X: the initial Grams
-        # (three-piece operands, 16 per tile of A^T A and 6 per tile of A^T X), X^T X (two per block; the tuned kernels
-        # form both triangles) and the apply (three pieces): 40, 32 and 24 at rows of 128 and ranks up to 32
+        # (three-piece operands, 16 per tile of A^T A and 6 per tile of A^T X), X^T X (two per block on and
+        # above the diagonal) and the apply (three pieces): 40, 20 and 24 at rows of 128 and ranks up to 32
         ta, td = (r + 31) // 32, d // 32
         mf_given, mf_apply = 8 * ta * (ta + 1) + 6 * ta * td, 6 * ta * td
-        mf_xtx = 2 * td * td if tuned else td * (td + 1)
+        mf_xtx = td * (td + 1)
         exec_flops = (l / 32.0) * (bh * 2 * (mf_given + mf_apply) + (bh + bkv) * mf_xtx) * 2.0 * 32 * 32 * 16
-        passes = ("pf_sums_kernel + pf_pass_bf16_kernel + pf_xtx_kernel + pf_apply_shared_kernel" if tuned else
+        passes = ("pf_sums_kernel + pf_apply_shared_kernel" if tuned else
                   "pf_stream_sums_kernel + pf_stream_apply_kernel")
         roof = {"bound": "hbm", "kernel": f"{passes} ({reads_q} readings of Q, {reads_k} of K); pf_gramdom_kernel (fp64 "
                                           "d x d algebra per head, latency-bound) between them",

@@ -29,287 +29,331 @@
 
 namespace lrqk {
 
-// ----------------------------------------------------------------------------- X^T X
-// grid (S, x heads); 8 waves share the rows (128 per step, staged in LDS as they lie in memory); wave w owns
-// the output blocks (w / 2, 2 (w % 2)) and (w / 2, 2 (w % 2) + 1) of 32 x 32.  A lane's operand for column
-// block nb is eight rows of one column, which the transposing LDS read delivers four at a time; every 32-row
-// tile is summed in a fresh accumulator and added to the running total in fp32 (the matrix cores do not round
-// to nearest when they add to a large accumulator).
+// ----------------------------------------------------------------------------- X^T X and the sums over given factors
+// Both sides in one launch, one reading of the rows for all sums: a workgroup stages 128 rows of X and of the given
+// factors A (fp32, [head][l][r]) per step and its waves form X^T X and (A^T A, A^T X).  Workgroups [0, bh * S): head and
+// split of the Q side; behind them the K side, where the query heads of a kv head take their X from it and X^T X of split
+// s is left to head s % nh of the group.  Those heads lie 8 workgroups apart, on one XCD, and walk the same rows at the same
+// time: K comes from that XCD's L2 after the first of them.
+//
+// The rows of A are split into three bf16 pieces (8 + 8 + 8 mantissa bits, exact) on their way to LDS, so every number is
+// split once; all operands then come out of LDS by the transposing read.  Wave (g, ch) = (w / 2, w % 2) takes the 32-row
+// group g of the step, there two of the four column blocks of A^T X, k block ch of A^T A and five of the ten blocks of X^T X
+// on and above the diagonal.  Which: block i of a wave is block i of X for ch = 0 and block (2, 0, 3, 1)[i] for ch = 1, and
+// both take the columns 0, 3 and the products (0,0) (3,3) (0,1) (1,2) (2,3) of their own numbering -- the path 0-1-2-3 through
+// the four blocks and its complement 2-0-3-1, so the code is the same and only LDS addresses differ.
+// Products per 32 rows as in the row-by-row pass: all piece pairs of A^T A except lo x lo, three pieces of A times X; every
+// 32-row group in a fresh accumulator (the matrix cores do not round to nearest when they add to a large one), which is
+// added to the running total in fp32.
+//
+// A step's rows are requested a step ahead, into registers (fp32 sums leave the accumulators 128 of the 256 a wave has), and
+// go to the other half of the LDS tile, one barrier a step.  The sides' workgroups alternate in chunks, so that the Q side's,
+// which the HBM bounds, and the K side's, which read a third as much of it, run side by side.  32 heads of 32K rows (8 kv
+// heads), rank 32, us: 165 (600 MB; 140 with the loads alone, 138 with the arithmetic alone); the same sums in three launches
+// (Q; K and its given factors; K^T K), whose waves formed all 16 blocks of X^T X and split every factor twice: 122 + 73 + 20.
+// On the way: the sides one after the other 182, a branch on X^T X inside the loop 173, all waves in step 172; with 20
+// registers spilled (scratch reloads wait for the requested rows) 215.
 constexpr int kXtxWaves = 8, kXtxThreads = kXtxWaves * kWave, kXtxRows = 128, kXtxD = 128;
-constexpr int kXtxLd = kXtxD + 16;  // bf16 elements per staged row: 288 bytes, so four successive rows start 8 banks apart
+constexpr int kSumXTile = kXtxRows * kXtxD, kSumATile = kXtxRows * 32;  // elements: rows of X, one piece of the rows of A
+constexpr int kSumBuf = kSumXTile + 3 * kSumATile;
+constexpr int kSumLdr = 33;                                             // floats per row of a tile on its way out
+constexpr int kSumSmem = 2 * kSumBuf * (int)sizeof(uint16_t);
+static_assert(kXtxWaves * 3 * 32 * kSumLdr * (int)sizeof(float) <= kSumSmem, "the reduction uses the tiles' LDS");
 
-__global__ __launch_bounds__(kXtxThreads) void pf_xtx_kernel(const bf16_t* __restrict__ X, int64_t l,
-                                                             float* __restrict__ part, int S) {
-  __shared__ __align__(16) uint16_t x_s[kXtxRows * kXtxLd];
-  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-  const int col = lane & 31, half = lane >> 5;
-  const int xh = blockIdx.y, s = blockIdx.x;
-  const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
-  const int nb1 = wave >> 1, nb2 = 2 * (wave & 1);
-  constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);  // 16-byte loads per thread and step
-  // One step ahead is all that pays: with two steps of rows in flight per workgroup the kernel is slower
-  // (65 against 54 us at 32 heads x 32K rows).
-  uint4 pre_a[NL];
-  auto issue = [&](int64_t t0, uint4 (&dst)[NL]) {
+struct SumsArgs {
+  const bf16_t *q, *k;
+  const float *a_q, *a_k;
+  float *part_q, *part_k;    // [head][S][r][r + d]
+  float *xq_part, *xk_part;  // [head of X][S][d][d]
+  int64_t l;
+  int bh, nh, r, S;
+};
+
+// ALIGNED: rows of A of whole 16-byte pieces
+template <bool ALIGNED>
+__global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(SumsArgs g) {
+  extern __shared__ __align__(16) uint16_t sum_s[];
+  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
+  const int col = lane & 31, half = lane >> 5, s16 = lane & 15;
+  const int wg = wave >> 1, ch = wave & 1;
+  const int S = g.S, r = g.r, nh = g.nh;
+  const int64_t l = g.l;
+  // chunks of 8 nh workgroups, the sides in turn
+  const int chunk = (int)blockIdx.x / (8 * nh), at = (int)blockIdx.x % (8 * nh);
+  const bool k_side = chunk & 1;
+  int h, s;
+  if (!k_side) {
+    const int w = (chunk >> 1) * 8 * nh + at;
+    if (w >= g.bh * S) return;
+    h = w / S;
+    s = w % S;
+  } else {
+    // eight (kv head, split) pairs side by side, then the same eight for the group's next head
+    const int pair = (chunk >> 1) * 8 + at % 8;
+    if (pair >= g.bh / nh * S) return;
+    h = pair / S * nh + at / 8;
+    s = pair % S;
+  }
+  const int xh = k_side ? h / nh : h;
+  const bool xtx = !k_side || h % nh == s % nh;
+  const bf16_t* Xh = (k_side ? g.k : g.q) + (int64_t)xh * l * kXtxD;
+  const float* Ah = (k_side ? g.a_k : g.a_q) + (int64_t)h * l * r;
+
+  // ---- rows into registers, registers into LDS
+  constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);  // 16-byte pieces of X per thread and step
+  const int x_row = tid >> 4, x_piece = tid & 15;           // of the first: the others are 32 rows further each
+  const int a_row = tid >> 2, a_col = (tid & 3) * 4;        // this thread's factors: a_col .. + 3 and 16 further
+  gd_u32x4 px[NL];
+  gd_floatx4 pa[2];
+  auto issue = [&](int64_t t0) {
+    const bf16_t* xb = Xh + t0 * kXtxD;
+    const float* ab = Ah + t0 * r;
     const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
+    if (last == kXtxRows - 1) {
+      const uint32_t at = (uint32_t)(x_row * kXtxD + 8 * x_piece) * 2u;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int e = (i * kXtxThreads + tid) * 8;  // element of the 128 x 128 step
-      dst[i] = gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
+      for (int i = 0; i < NL; ++i) px[i] = gd_at<gd_u32x4>(xb + i * 32 * kXtxD, at);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+        px[i] = gd_at<gd_u32x4>(xb, (uint32_t)(min(x_row + 32 * i, last) * kXtxD + 8 * x_piece) * 2u);
+    }
+    const uint32_t a_at = __umul24((uint32_t)min(a_row, last), 4u * (uint32_t)r);
+    if constexpr (ALIGNED) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) pa[j] = gd_at<gd_floatx4>(ab, a_at + 4u * (uint32_t)min(a_col + 16 * j, r - 4));
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) pa[q >> 2][q & 3] = gd_at<float>(ab, a_at + 4u * (uint32_t)min(a_col + 16 * (q >> 2) + (q & 3), r - 1));
     }
   };
-  gd_floatx16 acc0, acc1;
+  // block nb (64 bytes) of row t of X lies at place nb ^ (t & 3): four successive rows of a block then meet all LDS banks
+  auto stage = [&](int64_t t0, char* tile) {
+    const int rows = (int)min((int64_t)kXtxRows, l - t0);
+    char* xp = tile + 2 * (x_row * kXtxD + 8 * (x_piece ^ ((x_row & 3) << 2)));
+    char* ap = tile + 2 * (kSumXTile + a_row * 32 + a_col);
+    const bool whole = rows == kXtxRows && r == 32;
+    if (!whole) {
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.0f;
-  // An operand of the 32x32x16 product, lane (col, half): rows row0 + 8 half .. + 7 of column 32 nb + col.  The
-  // transposing LDS read hands a lane four successive rows of its column: within 16 lanes, lane s points at
-  // row s / 4, columns 4 (s % 4) .. + 3, and lane t receives column t of the four rows.
-  auto operand = [&](int row0, int nb) {
-    const int s16 = lane & 15;
-    const uint16_t* p = &x_s[(row0 + 8 * half + (s16 >> 2)) * kXtxLd + 32 * nb + (col & 16) + 4 * (s16 & 3)];
+      for (int i = 0; i < NL; ++i)
+        if (x_row + 32 * i >= rows) px[i] = gd_u32x4{0, 0, 0, 0};
+      const int valid = a_row < rows ? r - a_col : 0;  // columns from a_col on that are there
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (16 * (q >> 2) + (q & 3) >= valid) pa[q >> 2][q & 3] = 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<gd_u32x4*>(xp + i * 32 * kXtxD * 2) = px[i];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      uint32_t pc[3][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) gd_split3(pa[j][q], pc[0][q], pc[1][q], pc[2][q]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+        *reinterpret_cast<uint2*>(ap + 2 * (p * kSumATile + 16 * j)) =
+            make_uint2(gd_pack2(pc[p][0], pc[p][1]), gd_pack2(pc[p][2], pc[p][3]));
+    }
+  };
+
+  // ---- operands: rows 32 wg + 16 kb + 4 half .. + 3 and the same + 8 (the same order on both sides of a product) of 32
+  // columns.  Within 16 lanes, lane s points at row s / 4, columns 4 (s % 4) .. + 3, and lane t receives column t of the
+  // four rows.
+  const int row0 = 32 * wg + 4 * half + (s16 >> 2);
+  const int c0 = (col & 16) + 4 * (s16 & 3);
+  const uint32_t x_at = 2u * (uint32_t)(row0 * kXtxD + 32 * (s16 >> 2) + c0);  // block nb: x_at ^ 64 nb
+  const uint32_t a_at = 2u * (uint32_t)(kSumXTile + row0 * 32 + c0);
+  auto read8 = [&](const char* p, int rows8) {  // rows8: bytes from a row to the one 8 further
     const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
-    const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 4 * kXtxLd));
+    const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + rows8));
     return __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  // split s takes the steps s, s + S, ...: the workgroups of a head walk the head's rows side by side
-  const int64_t stride = (int64_t)S * kXtxRows;
-  // one step: stage `cur` (the rows from t0 on), ask for the next step into `cur`, multiply
-  auto step = [&](int64_t t0, uint4 (&cur)[NL]) {
-    const int rows = (int)min((int64_t)kXtxRows, l - t0);
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int e = (i * kXtxThreads + tid) * 8;
-      const int row = e / kXtxD;
-      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = row < rows ? cur[i] : make_uint4(0, 0, 0, 0);
-    }
-    __syncthreads();
-    if (t0 + stride < l) issue(t0 + stride, cur);
-    const int tiles = (int)min((int64_t)4, (l - t0 + 31) / 32);
-    for (int tile = 0; tile < tiles; ++tile) {
-      gd_floatx16 t0a, t1a;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) t0a[v] = t1a[v] = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int row0 = 32 * tile + 16 * kb;
-        const gd_bf16x8 a = operand(row0, nb1);
-        const gd_bf16x8 b0 = operand(row0, nb2), b1 = operand(row0, nb2 + 1);
-        t0a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, t0a, 0, 0, 0);
-        t1a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, t1a, 0, 0, 0);
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc0[v] += t0a[v];
-        acc1[v] += t1a[v];
-      }
-    }
-    __syncthreads();
-  };
-  const int64_t first = (int64_t)s * kXtxRows;
-  if (first < l) issue(first, pre_a);
-  for (int64_t t0 = first; t0 < l; t0 += stride) step(t0, pre_a);
-  float* out = part + ((int64_t)xh * S + s) * kXtxD * kXtxD;
+  const int order = ch ? 0x1302 : 0x3210;  // block i of this wave
+
+  gd_floatx16 gAA, gAX[2], gXX[5];
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    const int i = 32 * nb1 + gd_mfma_row(lane, v);
-    out[i * kXtxD + 32 * nb2 + col] = acc0[v];
-    out[i * kXtxD + 32 * (nb2 + 1) + col] = acc1[v];
+    gAA[v] = gAX[0][v] = gAX[1][v] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) gXX[i][v] = 0.0f;
   }
+  auto multiply = [&](char* tile, auto with_xtx) {
+    const char* ar = tile + a_at;
+    gd_bf16x8 x[4][2];
+    auto read_x = [&](int i) {
+      const char* at = tile + (x_at ^ (uint32_t)(64 * ((order >> (4 * i)) & 3)));
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) x[i][kb] = read8(at + kb * 16 * kXtxD * 2, 8 * kXtxD * 2);
+    };
+    read_x(0);
+    read_x(3);
+    if constexpr (decltype(with_xtx)::value) {
+      auto block = [&](int i, const gd_bf16x8 (&a)[2], const gd_bf16x8 (&b)[2]) {
+        gd_floatx16 t;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kb], b[kb], t, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) gXX[i][v] += t[v];
+      };
+      read_x(1);
+      read_x(2);
+      block(0, x[0], x[0]);
+      block(2, x[0], x[1]);
+      block(3, x[1], x[2]);
+      block(4, x[2], x[3]);
+      block(1, x[3], x[3]);
+      __builtin_amdgcn_sched_barrier(0);  // (in this order the operands fit the registers)
+    }
+    {
+      gd_bf16x8 c[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) c[p] = read8(ar + ch * 16 * 32 * 2 + p * kSumATile * 2, 8 * 32 * 2);
+      gd_floatx16 t;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+      // k block ch of A^T A, smallest pieces first
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[1], c[2], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[2], c[1], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[0], c[2], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[2], c[0], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[1], c[1], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[0], c[1], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[1], c[0], t, 0, 0, 0);
+      t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[0], c[0], t, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) gAA[v] += t[v];
+    }
+    gd_bf16x8 cp[3][2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) cp[p][kb] = read8(ar + (p * kSumATile + kb * 16 * 32) * 2, 8 * 32 * 2);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      gd_floatx16 t;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) t[v] = 0.0f;
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cp[p][kb], x[3 * j][kb], t, 0, 0, 0);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) gAX[j][v] += t[v];
+    }
+  };
+
+  // split s takes the steps s, s + S, ...: the workgroups of a head walk the head's rows side by side
+  const int64_t stride = (int64_t)S * kXtxRows;
+  const int64_t first = (int64_t)s * kXtxRows;
+  // Between two barriers a wave multiplies one step and puts the next one into the other half of the tile.  Of the two waves
+  // of a SIMD one does so first and the other last, so that matrix and vector work meet.
+  const bool stage_first = wave >= kXtxWaves / 2;
+  auto walk = [&](auto with_xtx, auto ahead) {
+    constexpr int kTileBytes = kSumBuf * (int)sizeof(uint16_t);
+    char* const tiles = (char*)sum_s;
+    int buf = 0;
+    auto fetch = [&](int64_t t0, int half_at) {  // the step from t0 on, requested before, into LDS; the next one requested
+      stage(t0, tiles + half_at);
+      if (t0 + stride < l) issue(t0 + stride);
+    };
+    if (first < l) {
+      issue(first);
+      if constexpr (decltype(ahead)::value) fetch(first, 0);
+    }
+    for (int64_t t0 = first; t0 < l; t0 += stride) {
+      if constexpr (!decltype(ahead)::value) fetch(t0, buf);
+      __syncthreads();
+      if constexpr (decltype(ahead)::value)
+        if (t0 + stride < l) fetch(t0 + stride, kTileBytes - buf);
+      multiply(tiles + buf, with_xtx);  // (rows beyond the end are zeros)
+      buf = kTileBytes - buf;
+    }
+  };
+  // (a loop each: a branch inside one costs the accumulators copies; all meet the same barriers)
+  if (xtx) {
+    if (stage_first)
+      walk(std::true_type(), std::true_type());
+    else
+      walk(std::true_type(), std::false_type());
+  } else {
+    if (stage_first)
+      walk(std::false_type(), std::true_type());
+    else
+      walk(std::false_type(), std::false_type());
+  }
+
+  // ---- the waves' sums, up to three tiles at a time: add(tile, waves' step, first wave, row, column)
+  float* sm = reinterpret_cast<float*>(sum_s);
+  constexpr int kTile = 32 * kSumLdr;
+  auto put = [&](int slot, const gd_floatx16& acc) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sm[(slot * kXtxWaves + wave) * kTile + gd_mfma_row(lane, v) * kSumLdr + col] = acc[v];
+  };
+  auto add4 = [&](int slot, int c, int m, int n) {  // over the waves with ch = c
+    const float* p = sm + (slot * kXtxWaves + c) * kTile + m * kSumLdr + n;
+    return (p[0] + p[2 * kTile]) + (p[4 * kTile] + p[6 * kTile]);
+  };
+  const int ld = r + kXtxD;
+  float* outp = (k_side ? g.part_k : g.part_q) + ((int64_t)h * S + s) * r * ld;
+  __syncthreads();
+  put(0, gAA);
+  put(1, gAX[0]);
+  put(2, gAX[1]);
+  __syncthreads();
+  for (int e = tid; e < 1024; e += kXtxThreads) {
+    const int m = e >> 5, n = e & 31;
+    if (m < r && n < r) outp[m * ld + n] = add4(0, 0, m, n) + add4(0, 1, m, n);
+  }
+  for (int e = tid; e < 32 * kXtxD; e += kXtxThreads) {
+    const int m = e / kXtxD, n = e % 32, nb = (e / 32) % 4;
+    // column block nb is the first or second one of ch 0: 0, 3, or of ch 1: 2, 1
+    if (m < r) outp[m * ld + r + 32 * nb + n] = add4(nb == 0 || nb == 2 ? 1 : 2, nb == 1 || nb == 2, m, n);
+  }
+  if (!xtx) return;
+  float* outx = (k_side ? g.xk_part : g.xq_part) + ((int64_t)xh * S + s) * kXtxD * kXtxD;
+  // blocks of X of product i, for ch 0 and 1: rows, columns
+  auto write = [&](int slot, int bi, int bj) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int ri = c ? (0x1302 >> (4 * bi)) & 3 : bi, rj = c ? (0x1302 >> (4 * bj)) & 3 : bj;
+      for (int e = tid; e < 1024; e += kXtxThreads) {
+        const int m = e >> 5, n = e & 31;
+        outx[(32 * ri + m) * kXtxD + 32 * rj + n] = add4(slot, c, m, n);
+        if (bi != bj) outx[(32 * rj + m) * kXtxD + 32 * ri + n] = add4(slot, c, n, m);
+      }
+    }
+  };
+  __syncthreads();
+  put(0, gXX[0]);
+  put(1, gXX[1]);
+  put(2, gXX[2]);
+  __syncthreads();
+  write(0, 0, 0);
+  write(1, 3, 3);
+  write(2, 0, 1);
+  __syncthreads();
+  put(0, gXX[3]);
+  put(1, gXX[4]);
+  __syncthreads();
+  write(0, 1, 2);
+  write(1, 2, 3);
 }
 
-// ----------------------------------------------------------------------------- X^T X and the sums over given factors
-// One reading of X for both (the Q side, where every head has rows of its own): the workgroup stages 128 rows of X
-// per step as pf_xtx_kernel does and its waves form, besides their two blocks of X^T X, the sums (A^T A, A^T X)
-// over the given factors A (fp32, [head][l][r]).  Wave (a, ch) = (w / 2, w % 2) takes the 32-row group a of the
-// step and the column blocks 2 ch, 2 ch + 1 of A^T X; of A^T A it takes the products of k block ch (the two
-// waves' halves are added at the end).  The rows of A are read in the accumulator layout (element v of lane l: row
-// gd_mfma_row(l, v), column l % 32) and split into three bf16 pieces (8 + 8 + 8 mantissa bits, exact); taken
-// eight at a time these are an operand's k elements, and X's come out of LDS in the same order by the transposing
-// read.  Products per 32 rows as in the row-by-row pass: all piece pairs of A^T A except lo x lo, three pieces of
-// A times X; every 32-row group in a fresh accumulator.  part: [head][S][r][r + d] like the row-by-row pass
-// writes them; xtx_part: [head][S][d][d].
-// (Several heads that share their X -- the K side -- in one workgroup were tried and are slower: a wave then works
-// through its heads' row groups one after the other, and their rows of A in flight together do not fit the
-// registers.  Requesting the rows of A a step ahead also made this kernel slower: 142 against 126 us at 32 heads
-// x 32K rows.)
-__global__ __launch_bounds__(kXtxThreads) void pf_sums_kernel(const bf16_t* __restrict__ X, int64_t l,
-                                                              const float* __restrict__ A, int r,
-                                                              float* __restrict__ part, float* __restrict__ xtx_part,
-                                                              int S) {
-  // the tile of X; at the end the waves' sums pass through it
-  __shared__ __align__(16) uint16_t x_s[kXtxRows * kXtxLd];
-  static_assert(sizeof(x_s) >= kXtxWaves * 1024 * sizeof(float), "the reduction uses the tile's LDS");
-  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
-  const int col = lane & 31, half = lane >> 5;
-  const int xh = blockIdx.y, s = blockIdx.x;
-  const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
-  const int wa = wave >> 1, ch = wave & 1;
-  const int nb1 = wa, nb2 = 2 * ch;  // blocks of X^T X
-  const float* Ah = A + (int64_t)xh * l * r;
-  constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);
-  uint4 pre_a[NL];
-  auto issue = [&](int64_t t0, uint4 (&dst)[NL]) {
-    const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int e = (i * kXtxThreads + tid) * 8;
-      dst[i] = gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
-    }
-  };
-  gd_floatx16 acc0, acc1, gAA, gAX[2];
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = gAA[v] = gAX[0][v] = gAX[1][v] = 0.0f;
-  auto operand = [&](int row0, int nb) {  // rows row0 + 8 half .. + 7 of column 32 nb + col
-    const int s16 = lane & 15;
-    const uint16_t* p = &x_s[(row0 + 8 * half + (s16 >> 2)) * kXtxLd + 32 * nb + (col & 16) + 4 * (s16 & 3)];
-    const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
-    const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 4 * kXtxLd));
-    return __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  };
-  auto operand_acc = [&](int row0, int nb) {  // rows row0 + 4 half .. + 3 and the same + 8: the accumulator's order
-    const int s16 = lane & 15;
-    const uint16_t* p = &x_s[(row0 + 4 * half + (s16 >> 2)) * kXtxLd + 32 * nb + (col & 16) + 4 * (s16 & 3)];
-    const gd_v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)p);
-    const gd_v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((gd_lds_v4s)(p + 8 * kXtxLd));
-    return __builtin_bit_cast(gd_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-  };
-  const int64_t stride = (int64_t)S * kXtxRows;
-  float arow[16];  // this wave's rows of A of the step being multiplied, requested at the start of the step
-  auto step = [&](int64_t t0, uint4 (&cur)[NL]) {
-    const int rows = (int)min((int64_t)kXtxRows, l - t0);
-    const int group_rows = rows - 32 * wa;  // of this wave's group: below 1 beyond the end
-    {
-      const float* group = Ah + min(t0 + 32 * wa, l - 1) * r;
-      const int last = max(group_rows, 1) - 1;
-#pragma unroll
-      for (int v = 0; v < 16; ++v)  // (requested first, consumed after the blocks of X^T X below)
-        arow[v] = gd_factor(group, gd_mfma_row(lane, v), last, r, min(col, r - 1));
-    }
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      const int e = (i * kXtxThreads + tid) * 8;
-      const int row = e / kXtxD;
-      *reinterpret_cast<uint4*>(&x_s[row * kXtxLd + e % kXtxD]) = row < rows ? cur[i] : make_uint4(0, 0, 0, 0);
-    }
-    __syncthreads();
-    if (t0 + stride < l) issue(t0 + stride, cur);
-    const int tiles = (int)min((int64_t)4, (l - t0 + 31) / 32);
-    for (int tile = 0; tile < tiles; ++tile) {
-      gd_floatx16 t0a, t1a;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) t0a[v] = t1a[v] = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const int row0 = 32 * tile + 16 * kb;
-        const gd_bf16x8 a = operand(row0, nb1);
-        const gd_bf16x8 b0 = operand(row0, nb2), b1 = operand(row0, nb2 + 1);
-        t0a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, t0a, 0, 0, 0);
-        t1a = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, t1a, 0, 0, 0);
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        acc0[v] += t0a[v];
-        acc1[v] += t1a[v];
-      }
-    }
-    if (group_rows > 0) {  // (wave-uniform)
-      const int valid = (col < r ? group_rows : 0) - 4 * half;
-      // the three pieces of the group's rows of A, eight rows (one k block) at a time
-      gd_bf16x8 cp[3][2];
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        uint32_t pc[3][8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int v = 8 * kb + q;
-          gd_split3(gd_mfma_row0(v) < valid ? arow[v] : 0.0f, pc[0][q], pc[1][q], pc[2][q]);
-        }
-#pragma unroll
-        for (int pp = 0; pp < 3; ++pp)
-          cp[pp][kb] = __builtin_bit_cast(gd_bf16x8, make_uint4(gd_pack2(pc[pp][0], pc[pp][1]), gd_pack2(pc[pp][2], pc[pp][3]),
-                                                                gd_pack2(pc[pp][4], pc[pp][5]), gd_pack2(pc[pp][6], pc[pp][7])));
-      }
-      {
-        gd_floatx16 t;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) t[v] = 0.0f;
-        // k block ch of A^T A, smallest pieces first
-        const gd_bf16x8 c0 = ch ? cp[0][1] : cp[0][0], c1 = ch ? cp[1][1] : cp[1][0], c2 = ch ? cp[2][1] : cp[2][0];
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, c2, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c2, c1, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, c2, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c2, c0, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, c1, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, c1, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c1, c0, t, 0, 0, 0);
-        t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(c0, c0, t, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) gAA[v] += t[v];
-      }
-#pragma unroll
-      for (int nbi = 0; nbi < 2; ++nbi) {
-        gd_bf16x8 xb[2];
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) xb[kb] = operand_acc(32 * wa + 16 * kb, 2 * ch + nbi);
-        gd_floatx16 t;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) t[v] = 0.0f;
-#pragma unroll
-        for (int pp = 2; pp >= 0; --pp)
-#pragma unroll
-          for (int kb = 0; kb < 2; ++kb) t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cp[pp][kb], xb[kb], t, 0, 0, 0);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) gAX[nbi][v] += t[v];
-      }
-    }
-    __syncthreads();
-  };
-  const int64_t first = (int64_t)s * kXtxRows;
-  if (first < l) issue(first, pre_a);
-  for (int64_t t0 = first; t0 < l; t0 += stride) step(t0, pre_a);
-  {
-    float* out = xtx_part + ((int64_t)xh * S + s) * kXtxD * kXtxD;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int i = 32 * nb1 + gd_mfma_row(lane, v);
-      out[i * kXtxD + 32 * nb2 + col] = acc0[v];
-      out[i * kXtxD + 32 * (nb2 + 1) + col] = acc1[v];
-    }
-  }
-  // the waves' sums: pass 0 is A^T A (all waves), passes 1, 2 the column blocks 2 ch + 0 / + 1 of A^T X (the waves
-  // with the same ch)
-  float* sm = reinterpret_cast<float*>(x_s);
-  const int ne = r * (r + kXtxD);
-  float* outp = part + ((int64_t)xh * S + s) * ne;
-#pragma unroll 1
-  for (int blk = 0; blk < 3; ++blk) {
-    float* mine = sm + wave * 1024;
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-      mine[gd_mfma_row(lane, v) * 32 + col] = blk == 0 ? gAA[v] : (blk == 1 ? gAX[0][v] : gAX[1][v]);
-    __syncthreads();
-    const int n_out = (blk == 0 ? 1 : 2) * 1024;
-    for (int o = tid; o < n_out; o += kXtxThreads) {
-      const int e = o & 1023, c_half = blk == 0 ? -1 : (o >> 10);
-      float v = 0.0f;
-#pragma unroll
-      for (int w = 0; w < kXtxWaves; ++w)
-        if (c_half < 0 || (w & 1) == c_half) v += sm[w * 1024 + e];
-      const int m = e >> 5, n = e & 31;
-      if (blk == 0) {
-        if (m < r && n < r) outp[m * (r + kXtxD) + n] = v;
-      } else {
-        const int cx = 32 * (2 * c_half + (blk - 1)) + n;
-        if (m < r) outp[m * (r + kXtxD) + r + cx] = v;
-      }
-    }
-    __syncthreads();
-  }
+static int prefill_sums(const SumsArgs& g, hipStream_t st) {
+  const bool aligned = g.r % 4 == 0 && (uintptr_t)g.a_q % 16 == 0 && (uintptr_t)g.a_k % 16 == 0;
+  const auto kern = aligned ? pf_sums_kernel<true> : pf_sums_kernel<false>;
+  LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kSumSmem));
+  const int pairs = g.bh / g.nh * g.S;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((pairs + 7) / 8 * 8 * g.nh * 2)), dim3(kXtxThreads), kSumSmem, st, g);
+  LRQK_HIP_CHECK(hipGetLastError());
+  return LRQK_OK;
 }
 
 // ----------------------------------------------------------------------------- A = X Mt^T for heads that share X
 // The K side's last pass: the NH query heads of a kv head take their rows of A_K from the same rows of K, so one
-// workgroup stages 128 rows of K per step (as pf_xtx_kernel does) and applies the NH heads' Mt to them: K is read
+// workgroup stages 128 rows of K per step (as pf_sums_kernel does) and applies the NH heads' Mt to them: K is read
 // once per kv head instead of once per query head.  Mt (fp32) lies in LDS as three bf16 pieces per head, X as it
 // is; wave w takes head w / (8 / NH) and NH / 2 of the step's four 32-row groups; 24 products of 32x32x16 per
 // group (X times the three pieces), fp32 accuracy as in the row-by-row pass.  grid (S, kv heads); split s takes
@@ -1372,11 +1416,7 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
     return (int)std::max<int64_t>(1, std::min<int64_t>(v, (l + 127) / 128));
   };
   const int S = splits(bh), Sx = S;
-  // (K^T K: with 64 splits of 8 heads the partial sums are 33 MB to write and to add up: 25.6 + 18.5 us against
-  // 19.7 + 11.1 with 32.  No bound on the rows of a split here: its sums are of exact products, and 32 kv heads of 64K
-  // rows add 8192 of them up in fp32)
-  const int Sxk = tuned ? (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + 511) / 512))
-                        : hkv == hq ? S : splits(bkv);
+  const int Sxk = tuned || hkv == hq ? S : splits(bkv);
   const size_t n_flags = ((size_t)iters + 2) & ~(size_t)1;
   // In slices while a launch of an iteration has few workgroups per CU; with more, what the slices repeat costs more than
   // idle CUs do (a launch is rounded up to 8 heads).  The fit of 4096 rows with four iterations, whole -> in slices, us:
@@ -1437,12 +1477,7 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
   a.tol = tol;
 
   if (tuned) {
-    hipLaunchKernelGGL(pf_sums_kernel, dim3((unsigned)S, (unsigned)bh), dim3(kXtxThreads), 0, st, q, l, a_q0, r,
-                       partQ, xq_part, S);
-    if ((rc = prefill_given_sums_bf16(k, hkv, hq, b, l, r, a_k0, partK, S, st))) return rc;
-    hipLaunchKernelGGL(pf_xtx_kernel, dim3((unsigned)Sxk, (unsigned)bkv), dim3(kXtxThreads), 0, st, k, l, xk_part,
-                       Sxk);
-    LRQK_HIP_CHECK(hipGetLastError());
+    if ((rc = prefill_sums({q, k, a_q0, a_k0, partQ, partK, xq_part, xk_part, l, bh, hq / hkv, r, S}, st))) return rc;
   } else {
     if ((rc = prefill_stream_sums(q, k, hq, hkv, b, l, r, d, a_q0, a_k0, partQ, partK, S, xq_part, xk_part, Sxk, st)))
       return rc;

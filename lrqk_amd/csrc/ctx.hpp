@@ -212,7 +212,7 @@ struct PrefillOut {
 // Prefill iterations on Gram matrices (bf16 rows); see als_prefill_gram.hip.
 int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* a_q0, float* a_k0, const PrefillOut& out,
                         int b, int hq, int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st);
-// Its passes over the long axis; see als_prefill_stream.hip (every shape) and als_prefill.hip (rows of 128, r <= 32).
+// Its passes over the long axis; see als_prefill_stream.hip (rows of 128 and r <= 32: the sums have a kernel of their own).
 int prefill_stream_sums(const bf16_t* q, const bf16_t* k, int hq, int hkv, int b, int64_t l, int r, int d, const float* a_q,
                         const float* a_k, float* part_q, float* part_k, int S, float* xq_part, float* xk_part, int Sxk,
                         hipStream_t st);
@@ -220,8 +220,6 @@ template <typename OUT>
 int prefill_stream_apply(const bf16_t* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride,
                          const bf16_t* q, int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r,
                          int d, hipStream_t st);
-int prefill_given_sums_bf16(const bf16_t* x, int xh, int hq, int b, int64_t l, int r, float* a, float* part, int S,
-                            hipStream_t st);
 template <typename OUT>
 int prefill_store(const float* src, int64_t src_stride, OUT* dst, int64_t dst_stride, int64_t n, int heads, hipStream_t st);
 // The factor update with the ring append of (k_new, v_new) at slot `slot` as token `token` folded

@@ -9,6 +9,7 @@ typedef __bf16 gd_bf16x8 __attribute__((ext_vector_type(8)));
 // 16 bytes of rows on their way to LDS (a native vector: arrays of the uint4 struct that are filled under a condition
 // end up in scratch memory, with a wait behind every load)
 typedef uint32_t gd_u32x4 __attribute__((ext_vector_type(4)));
+typedef float gd_floatx4 __attribute__((ext_vector_type(4)));
 typedef short gd_v4s __attribute__((ext_vector_type(4)));
 typedef gd_v4s __attribute__((address_space(3))) * gd_lds_v4s;
 

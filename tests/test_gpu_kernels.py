@@ -762,6 +762,36 @@ def test_als_prefill(ops, ws, oracle, dtype, hq, hkv, l, d, r, iters, tol):
         assert rel < (5e-3 if name in ("A_K", "B_K", "A_Q", "B_Q") else 1e-3), (name, float(rel))
 
 
+@pytest.mark.parametrize("b,hq,hkv,l,r,offset", [
+    (1, 4, 2, 127, 32, 0), (1, 4, 1, 128, 32, 0), (1, 2, 2, 129, 32, 0),     # steps of 128 rows: one short, whole, one and a row
+    (1, 6, 2, 1000, 28, 0), (1, 7, 1, 515, 12, 0), (2, 8, 2, 333, 16, 0),    # groups of 3 and 7 heads; a batch
+    (1, 4, 2, 700, 31, 0), (1, 4, 4, 260, 1, 0), (1, 4, 2, 640, 32, 1),      # factor rows of no whole 16-byte pieces
+    (3, 24, 3, 40, 4, 0), (1, 32, 8, 5000, 32, 0)])                          # a split per head; several steps per split
+def test_als_prefill_given_sums(ops, ws, oracle, b, hq, hkv, l, r, offset):
+    """bf16 rows of 128 elements, ranks up to 32: the sums over the given factors (no iteration: B = G^-1 C) and X^T X (one
+    iteration).  Random rows and factors; the sums are fp32 of exact products (below 1e-6 at these lengths), and the r x r
+    systems of random factors have condition numbers below 10 from 4 r rows on, 30 from 2 r (127 x 32): 3e-5."""
+    _say("als_prefill given sums", b, hq, hkv, l, r, offset)
+    g = torch.Generator().manual_seed(l + r)
+    d = 128
+    Q = torch.randn((b, hq, l, d), generator=g).to(torch.bfloat16)
+    K = torch.randn((b, hkv, l, d), generator=g).to(torch.bfloat16)
+    A0 = [torch.randn((b, hq, l, r), generator=g) for _ in range(2)]
+    for iters in (0, 1):
+        ref = oracle.als_prefill_w1(Q.double(), oracle.repeat_kv(K, hq // hkv).double(), A0[0].double(), A0[1].double(),
+                                    iters, 0.0)
+        dev = []
+        for a in A0:
+            block = torch.empty(a.numel() + 4, device=DEV)
+            dev.append(block[offset:offset + a.numel()].view(a.shape))
+            dev[-1].copy_(a)
+        got = ops.als_prefill(ws, Q.to(DEV), K.to(DEV), *dev, iters, 0.0)
+        for name, x, y in zip(("A_Q", "B_Q", "A_K", "B_K"), got, ref):
+            rel = float((x.cpu().double() - y).norm() / y.norm())
+            print(iters, name, "rel err %.3e" % rel, flush=True)
+            assert rel < 3e-5, (iters, name, rel)
+
+
 def test_als_prefill_large_sums_every_head(ops, ws, oracle):
     """128K rows of rank-r data factorised at rank r from random factors: after the first iteration the K side's
     r x r systems have diagonals around 1e12 and condition numbers around 1e5.  The elimination used to leave
