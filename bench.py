@@ -180,7 +180,7 @@ def prefill_roofline(w, l, iters, ms):
         mf_given, mf_apply = 8 * ta * (ta + 1) + 6 * ta * td, 6 * ta * td
         mf_xtx = td * (td + 1)
         exec_flops = (l / 32.0) * (bh * 2 * (mf_given + mf_apply) + (bh + bkv) * mf_xtx) * 2.0 * 32 * 32 * 16
-        passes = ("pf_sums_kernel + pf_apply_shared_kernel" if tuned else
+        passes = ("pf_sums_kernel + pf_stream_apply_kernel" if tuned else
                   "pf_stream_sums_kernel + pf_stream_apply_kernel")
         roof = {"bound": "hbm", "kernel": f"{passes} ({reads_q} readings of Q, {reads_k} of K); pf_gramdom_kernel (fp64 "
                                           "d x d algebra per head, latency-bound) between them",

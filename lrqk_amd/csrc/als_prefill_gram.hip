@@ -351,102 +351,6 @@ static int prefill_sums(const SumsArgs& g, hipStream_t st) {
   return LRQK_OK;
 }
 
-// ----------------------------------------------------------------------------- A = X Mt^T for heads that share X
-// The K side's last pass: the NH query heads of a kv head take their rows of A_K from the same rows of K, so one
-// workgroup stages 128 rows of K per step (as pf_sums_kernel does) and applies the NH heads' Mt to them: K is read
-// once per kv head instead of once per query head.  Mt (fp32) lies in LDS as three bf16 pieces per head, X as it
-// is; wave w takes head w / (8 / NH) and NH / 2 of the step's four 32-row groups; 24 products of 32x32x16 per
-// group (X times the three pieces), fp32 accuracy as in the row-by-row pass.  grid (S, kv heads); split s takes
-// the steps s, s + S, ...
-constexpr int kApLd = kXtxD + 8;  // bf16 elements per staged row: 16-byte operand reads want rows 4 banks apart
-template <int NH, typename OUT>
-__global__ __launch_bounds__(kXtxThreads) void pf_apply_shared_kernel(const bf16_t* __restrict__ X, int64_t l,
-                                                                      const float* __restrict__ Mt, int r,
-                                                                      OUT* __restrict__ A, int64_t a_stride, int S) {
-  static_assert(NH == 2 || NH == 4, "query heads per kv head");
-  extern __shared__ __align__(16) uint16_t ap_s[];
-  uint16_t* x_s = ap_s;                          // [128][kApLd]
-  uint16_t* mt_s = ap_s + kXtxRows * kApLd;      // [NH][3][32][kApLd]
-  const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
-  const int col = lane & 31, half = lane >> 5;
-  const int xh = blockIdx.y, s = blockIdx.x;
-  const bf16_t* Xh = X + (int64_t)xh * l * kXtxD;
-  constexpr int WPH = kXtxWaves / NH, GPW = 4 / WPH;  // waves per head, row groups per wave and step
-  const int hl = wave / WPH, g0 = (wave % WPH) * GPW;
-  OUT* Ah = A + ((int64_t)xh * NH + hl) * a_stride;
-  for (int e = tid; e < NH * 32 * kXtxD; e += kXtxThreads) {
-    const int hh = e / (32 * kXtxD), n = (e / kXtxD) % 32, k = e % kXtxD;
-    const float v = n < r ? Mt[(((int64_t)xh * NH + hh) * r + n) * kXtxD + k] : 0.0f;
-    uint32_t p0, p1, p2;
-    gd_split3(v, p0, p1, p2);
-    mt_s[((hh * 3 + 0) * 32 + n) * kApLd + k] = (uint16_t)(p0 >> 16);
-    mt_s[((hh * 3 + 1) * 32 + n) * kApLd + k] = (uint16_t)(p1 >> 16);
-    mt_s[((hh * 3 + 2) * 32 + n) * kApLd + k] = (uint16_t)(p2 >> 16);
-  }
-  constexpr int NL = kXtxRows * kXtxD / (kXtxThreads * 8);
-  static_assert(NL == 4, "four 16-byte loads per thread and step");
-  uint4 pre0 = make_uint4(0, 0, 0, 0), pre1 = pre0, pre2 = pre0, pre3 = pre0;
-  auto issue = [&](int64_t t0) {
-    const int last = (int)min((int64_t)kXtxRows, l - t0) - 1;
-    auto ld = [&](int i) {
-      const int e = (i * kXtxThreads + tid) * 8;
-      return gd_at<uint4>(Xh + t0 * kXtxD, (uint32_t)(min(e / kXtxD, last) * kXtxD + e % kXtxD) * 2u);
-    };
-    pre0 = ld(0);
-    pre1 = ld(1);
-    pre2 = ld(2);
-    pre3 = ld(3);
-  };
-  auto stage = [&](int i, const uint4& v) {
-    const int e = (i * kXtxThreads + tid) * 8;
-    *reinterpret_cast<uint4*>(&x_s[(e / kXtxD) * kApLd + e % kXtxD]) = v;  // (rows beyond l are never stored from)
-  };
-  const int64_t stride = (int64_t)S * kXtxRows;
-  const int64_t first = (int64_t)s * kXtxRows;
-  if (first < l) issue(first);
-  for (int64_t t0 = first; t0 < l; t0 += stride) {
-    stage(0, pre0);
-    stage(1, pre1);
-    stage(2, pre2);
-    stage(3, pre3);
-    __syncthreads();  // (the first one also covers the staging of Mt)
-    if (t0 + stride < l) issue(t0 + stride);
-#pragma unroll
-    for (int j = 0; j < GPW; ++j) {
-      const int g = g0 + j;
-      if (t0 + 32 * g >= l) continue;  // (wave-uniform)
-      gd_floatx16 c;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) c[v] = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < kXtxD / 16; ++kb) {
-        const gd_bf16x8 xa = *reinterpret_cast<const gd_bf16x8*>(&x_s[(32 * g + col) * kApLd + kb * 16 + 8 * half]);
-#pragma unroll
-        for (int pp = 0; pp < 3; ++pp) {
-          const gd_bf16x8 m =
-              *reinterpret_cast<const gd_bf16x8*>(&mt_s[((hl * 3 + pp) * 32 + col) * kApLd + kb * 16 + 8 * half]);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, m, c, 0, 0, 0);
-        }
-      }
-      gd_store_tile(Ah + (t0 + 32 * g) * r, c, (int)min((int64_t)32, l - t0 - 32 * g), col, half, r);
-    }
-    __syncthreads();
-  }
-}
-
-template <typename OUT>
-static int apply_shared(const void* k, const float* mt_k, OUT* a_k, int64_t a_stride, int bkv, int nh, int64_t l, int r,
-                        hipStream_t st) {
-  const int S = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 / bkv), (l + kXtxRows - 1) / kXtxRows));
-  const size_t smem = (size_t)(kXtxRows + nh * 3 * 32) * kApLd * sizeof(uint16_t);
-  auto kern = nh == 2 ? pf_apply_shared_kernel<2, OUT> : pf_apply_shared_kernel<4, OUT>;
-  LRQK_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-  hipLaunchKernelGGL(kern, dim3((unsigned)S, (unsigned)bkv), dim3(kXtxThreads), smem, st, (const bf16_t*)k, l, mt_k, r,
-                     a_k, a_stride, S);
-  LRQK_HIP_CHECK(hipGetLastError());
-  return LRQK_OK;
-}
-
 // ----------------------------------------------------------------------------- d x d algebra, fp64
 // Everything below is templated on RT, the number of 16-row tiles that the rank is padded to (ranks up to 16, 32, 64:
 // RT = 1, 2, 4), and on the row width D (64 or 128); RP = 16 RT is the padded rank.  Padding costs the matrix cores'
@@ -1403,8 +1307,7 @@ static int gramslice_run(const GdArgs& a, const float* xq_part, int Sx, const fl
 int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* a_q0, float* a_k0, const PrefillOut& out,
                         int b, int hq, int hkv, int64_t l, int r, int d, int iters, float tol, hipStream_t st) {
   const int bh = b * hq, bkv = b * hkv;
-  // rows of 128 elements and ranks up to 32 have kernels of their own for the passes: the Q side's sums with Q^T Q
-  // from one reading of Q, K^T K alone, A_K for several query heads from one reading of K
+  // rows of 128 elements and ranks up to 32 have a kernel of their own for the sums
   const bool tuned = d == 128 && r <= 32;
   const int RP = r <= 16 ? 16 : r <= 32 ? 32 : 64;
   const size_t ne = (size_t)r * (r + d), dd = (size_t)d * d;
@@ -1499,12 +1402,8 @@ int prefill_gram_domain(lrqk_ctx* ctx, const bf16_t* q, const bf16_t* k, float* 
       return rcs ? rcs : prefill_store<OUT>(a_k0, l * r, a_k, out.a_k_stride, l * r, bh, st);
     }
     const int64_t rows = out.a_q_rows;  // (the last ones)
-    const int nh = hq / hkv;
-    const bool shared = tuned && (nh == 2 || nh == 4);
-    int rcs = prefill_stream_apply<OUT>(shared ? nullptr : k, hkv, l, a.Mt_k, a_k, out.a_k_stride, q + (l - rows) * d, rows,
-                                        l * d, a.Mt_q, a_q, hq, b, r, d, st);
-    if (!rcs && shared) rcs = apply_shared<OUT>(k, a.Mt_k, a_k, out.a_k_stride, bkv, nh, l, r, st);
-    return rcs;
+    return prefill_stream_apply<OUT>(k, hkv, l, a.Mt_k, a_k, out.a_k_stride, q + (l - rows) * d, rows, l * d, a.Mt_q, a_q, hq, b,
+                                     r, d, st);
   };
   if (out.storage) return finish((bf16_t*)out.a_q, (bf16_t*)out.a_k);
   return finish((float*)out.a_q, (float*)out.a_k);

@@ -1,5 +1,5 @@
-// The passes over the long axis for the prefill iterations on Gram matrices, for every input that als_prefill_gram.hip
-// has no kernel tuned for: rows of 64 elements, ranks 33 .. 64.
+// The passes over the long axis for the prefill iterations on Gram matrices (the sums of rows of 128 at ranks up to 32 are in
+// als_prefill_gram.hip).
 //
 //   sums   S = X^T X, and over given factors A the sums G = A^T A, C = A^T X
 //   apply  A = X M
@@ -9,7 +9,7 @@
 // (every input read once), so the shape of the kernels follows the memory: a wave streams 32-row groups of its own
 // through a private LDS tile, the next group already requested, and never meets another wave before the end.
 // 32 heads of 16384 bf16 rows of 128, rank 64: all sums 193 us (435 MB; two waves' worth of matrix-core and vector work
-// on one wave per SIMD, which the accumulators leave room for), A_K 34 us; the row-by-row kernels for this rank took
+// on one wave per SIMD, which the accumulators leave room for), A_K 42 us; the row-by-row kernels for this rank took
 // 1.3 ms per pass, ten passes for four iterations.
 #include <algorithm>
 
@@ -267,23 +267,27 @@ __global__ __launch_bounds__(kStThreads) void pf_stream_sums_kernel(StSums g) {
 }
 
 // A = X M for every query head (its kv head's X): M^T (fp32, [head][r][d]) in LDS as three bf16 pieces, X through the
-// wave's private tile.  One launch for the sides given: workgroups (s, head) with s below side[0].S are the first side's
-// splits, the others the second's (a cache asks for one row of A_Q: alone that is a launch and 8 us).  The workgroups of
-// the query heads that share a kv head lie next to each other, so K comes from the last-level cache after the first of
-// them (not from an L2: they are on different XCDs, and the counters show K once per query head beyond the L2s).
+// wave's private tile.  One launch for both sides (a cache asks for one row of A_Q: alone that is a launch and 8 us), whose
+// workgroups alternate where both have as many; else the second side's come last.  The query heads that share a kv head's
+// rows lie eight workgroups apart, on one XCD, and walk the same rows at the same time.
+// Bound by HBM.  32 heads (8 kv heads), us: 32K rows of 128 at rank 32, both sides 100 (470 MB) -- A_K from rows staged for
+// four heads at a time and A_Q in launches of their own: 48 + 64; A_K and one row of A_Q 45 (42 + 8); 16K rows at rank 64 42
+// (59 with the heads of a kv head wherever they fell).  With M's pieces in registers and more, smaller workgroups: 106 for 100.
 template <typename OUT>
 struct StApply {
   const bf16_t* x;
-  int xh, S;          // heads of x per sequence; splits of the rows (0: no such side)
+  int S;              // splits of the rows
   int64_t l, x_stride;  // rows; elements between the heads of x
   const float* mt;
   OUT* a;             // heads a_stride elements apart, rows of r
   int64_t a_stride;
+  int nh, pairs, chunks;  // heads that share a head of x (one, or as many as the launch's other side has at most); pairs of a
+                          // head of x and a split; chunks of workgroups
 };
 constexpr int kStApplyWaves = 8;
 template <int AT, int DB, typename OUT>
 __global__ __launch_bounds__(kStApplyWaves * kWave) void pf_stream_apply_kernel(StApply<OUT> first_side,
-                                                                               StApply<OUT> second_side, int hq, int r) {
+                                                                               StApply<OUT> second_side, int r) {
   constexpr int D = 32 * DB;
   constexpr int NW = kStApplyWaves, NT = NW * kWave;
   constexpr int VEC = Vec16<bf16_t>::N;
@@ -294,13 +298,20 @@ __global__ __launch_bounds__(kStApplyWaves * kWave) void pf_stream_apply_kernel(
   const int tid = threadIdx.x, lane = lane_id(), wave = gd_wave();
   uint16_t* x_s = mt_s + 3 * 32 * AT * LDM + wave * 32 * LDX;                            // this wave's rows of X
   const int col = lane & 31, half = lane >> 5;
-  const int h = blockIdx.y;
-  const bool second = (int)blockIdx.x >= first_side.S;
+  // (unit workgroups, chunk): a chunk has eight (head of x, split) pairs side by side, then the same eight for the next head
+  // that shares x
+  const bool turns = first_side.chunks == second_side.chunks;
+  const bool second = turns ? blockIdx.y & 1 : (int)blockIdx.y >= first_side.chunks;
   const StApply<OUT>& g = second ? second_side : first_side;
-  const int s = second ? (int)blockIdx.x - first_side.S : (int)blockIdx.x, S = g.S;
+  const int chunk = turns ? blockIdx.y >> 1 : (int)blockIdx.y - (second ? first_side.chunks : 0);
+  const int nh = g.nh, S = g.S;
+  const int pair = nh == 1 ? chunk * (int)gridDim.x + (int)blockIdx.x : chunk * 8 + (int)(blockIdx.x & 7);
+  if (pair >= g.pairs) return;
+  const int xhead = (int)((uint32_t)pair / (uint32_t)S), s = pair - xhead * S;
+  const int h = nh == 1 ? xhead : xhead * nh + (int)(blockIdx.x >> 3);
   const int64_t l = g.l;
   const float* __restrict__ Mt = g.mt;
-  const bf16_t* __restrict__ Xh = g.x + ((int64_t)(h / hq) * g.xh + (h % hq) / (hq / g.xh)) * g.x_stride;
+  const bf16_t* __restrict__ Xh = g.x + (int64_t)xhead * g.x_stride;
   OUT* __restrict__ Ah = g.a + (int64_t)h * g.a_stride;
   for (int e = tid; e < 32 * AT * D; e += NT) {
     const int n = e / D, k = e % D;
@@ -402,7 +413,7 @@ int prefill_stream_sums(const bf16_t* q, const bf16_t* k, int hq, int hkv, int b
 }
 
 template <int AT, int DB, typename OUT>
-static int apply_impl(StApply<OUT> g0, StApply<OUT> g1, int hq, int b, int r, hipStream_t st) {
+static int apply_impl(StApply<OUT> g0, StApply<OUT> g1, int bh, int r, hipStream_t st) {
   constexpr int D = 32 * DB, NW = kStApplyWaves;
   constexpr size_t smem = (size_t)(3 * 32 * AT + NW * 32) * (D + 8) * sizeof(bf16_t);
   static_assert(smem <= 160 * 1024, "LDS");
@@ -414,25 +425,28 @@ static int apply_impl(StApply<OUT> g0, StApply<OUT> g1, int hq, int b, int r, hi
     attr = true;
   }
   // every workgroup stages M (52 KB in, up to 104 KB of fp32 read): enough of them to fill the GPU once, no more
-  const int bh = b * hq;
   const int per_cu = std::max(1, (int)(160 * 1024 / smem));
-  for (StApply<OUT>* g : {&g0, &g1})
-    g->S = !g->x ? 0 : (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (g->l + 32 * NW - 1) / (32 * NW)));
-  hipLaunchKernelGGL(kern, dim3((unsigned)(g0.S + g1.S), (unsigned)bh), dim3(NW * kWave), smem, st, g0, g1, hq, r);
+  const int unit = 8 * std::max(g0.nh, g1.nh);
+  for (StApply<OUT>* g : {&g0, &g1}) {
+    g->S = (int)std::max<int64_t>(1, std::min<int64_t>(std::max(1, 256 * per_cu / bh), (g->l + 32 * NW - 1) / (32 * NW)));
+    g->pairs = bh / g->nh * g->S;
+    g->chunks = g->nh == 1 ? (g->pairs + unit - 1) / unit : (g->pairs + 7) / 8;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)unit, (unsigned)(g0.chunks + g1.chunks)), dim3(NW * kWave), smem, st, g0, g1, r);
   LRQK_HIP_CHECK(hipGetLastError());
   return LRQK_OK;
 }
 
-// A_K = K Mk (l rows) and A_Q = Q Mq (q_rows rows) for all b * hq query heads; without k only the latter.  q: the first of
+// A_K = K Mk (l rows) and A_Q = Q Mq (q_rows rows) for all b * hq query heads.  q: the first of
 // those rows, heads q_stride elements apart.
 template <typename OUT>
 int prefill_stream_apply(const bf16_t* k, int hkv, int64_t l, const float* mt_k, OUT* a_k, int64_t a_k_stride,
                          const bf16_t* q, int64_t q_rows, int64_t q_stride, const float* mt_q, OUT* a_q, int hq, int b, int r,
                          int d, hipStream_t st) {
-  const StApply<OUT> gk{k, hkv, 0, l, l * d, mt_k, a_k, a_k_stride};
-  const StApply<OUT> gq{q, hq, 0, q_rows, q_stride, mt_q, a_q, q_rows * r};
-  if (d == 64) return r <= 32 ? apply_impl<1, 2>(gk, gq, hq, b, r, st) : apply_impl<2, 2>(gk, gq, hq, b, r, st);
-  return r <= 32 ? apply_impl<1, 4>(gk, gq, hq, b, r, st) : apply_impl<2, 4>(gk, gq, hq, b, r, st);
+  const StApply<OUT> gk{k, 0, l, l * d, mt_k, a_k, a_k_stride, hq / hkv, 0, 0};
+  const StApply<OUT> gq{q, 0, q_rows, q_stride, mt_q, a_q, q_rows * r, 1, 0, 0};
+  if (d == 64) return r <= 32 ? apply_impl<1, 2>(gk, gq, b * hq, r, st) : apply_impl<2, 2>(gk, gq, b * hq, r, st);
+  return r <= 32 ? apply_impl<1, 4>(gk, gq, b * hq, r, st) : apply_impl<2, 4>(gk, gq, b * hq, r, st);
 }
 template int prefill_stream_apply<float>(const bf16_t*, int, int64_t, const float*, float*, int64_t, const bf16_t*, int64_t,
                                          int64_t, const float*, float*, int, int, int, int, hipStream_t);
