@@ -621,6 +621,16 @@ def test_als_decode_split_counts(ops, ws, oracle, n):
     _check_als_decode(ops, ws, oracle, torch.float32, 2, 1, n, 64, 16, 2, 0.0)
 
 
+@pytest.mark.parametrize("dtype,d,r", [(torch.float32, 128, 4), (torch.float32, 64, 32), (torch.float32, 32, 12),
+                                       (torch.bfloat16, 64, 24), (torch.bfloat16, 128, 64), (torch.bfloat16, 128, 40),
+                                       (torch.bfloat16, 128, 32)])
+@pytest.mark.parametrize("n", [1, 15, 17, 31, 32, 33, 64, 127, 128, 129, 257])
+def test_als_decode_slot_counts(ops, ws, oracle, dtype, d, r, n):
+    """Passes over the active rows whose waves take 16 or 32 slots at a time, in splits of 128 and 256 (rows of 8, 16 and 32
+    pieces of 16 bytes; ranks 33 to 64): a slot short of a group, a whole one, a slot more."""
+    _check_als_decode(ops, ws, oracle, dtype, 2, 1, n, d, r, 2, 0.0)
+
+
 def _check_als_decode(ops, ws, oracle, dtype, hq, hkv, n, d, r, max_iter, tol):
     _say("als_decode", dtype, hq, n, d, r, max_iter, tol)
     g = torch.Generator().manual_seed(n + r)
