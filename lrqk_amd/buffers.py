@@ -76,12 +76,15 @@ class AutoIncreaseTensor:
         self.data.narrow(self.dim, self.current_len, length).copy_(x)
         self.current_len += length
 
-    @torch.inference_mode()
     def extend(self, like_shape, length: int, overwritten: bool = False) -> int:
         """Make room for ``length`` more entries exactly as ``append`` would, without writing
         them (a kernel fills the rows).  Returns the index of the first new entry.  ``overwritten``: every
         one of these rows is written before it is read, so a first allocation clears the rest only."""
-        self._ensure(like_shape, length, overwritten)
+        if torch.is_inference_mode_enabled():   # (every decode step: entering the mode once more is 2 us of host time)
+            self._ensure(like_shape, length, overwritten)
+        else:
+            with torch.inference_mode():
+                self._ensure(like_shape, length, overwritten)
         first = self.current_len
         self.current_len += length
         return first
