@@ -223,8 +223,19 @@ __device__ __forceinline__ void als_finish_body_mv(const FinishArgs& fa, int h, 
   en0 = wave_sum(en0);
   en1 = wave_sum(en1);
   static_assert(kFinMaxR <= kWave, "a lane per element of the iterates");
-  const float hx = lane < r ? hat[0][lane] : 0.0f, hy = lane < r ? hat[1][lane] : 0.0f;
-  const float hnq = wave_sum(hx * hx), hnk = wave_sum(hy * hy);
+  float hnq = 0.0f, hnk = 0.0f;
+  if (sizeof(T) == 4 && r > 32) {
+    // (the general solve, whose fp32 steps are ill-conditioned enough that the last bit of these sums decides on tokens at the
+    // edge of the active set and moves q_hat by 1e-3 some steps on: one element after the other, the order they always had)
+    for (int i = 0; i < r; ++i) {
+      hnq = fmaf(hat[0][i], hat[0][i], hnq);
+      hnk = fmaf(hat[1][i], hat[1][i], hnk);
+    }
+  } else {
+    const float hx = lane < r ? hat[0][lane] : 0.0f, hy = lane < r ? hat[1][lane] : 0.0f;
+    hnq = wave_sum(hx * hx);
+    hnk = wave_sum(hy * hy);
+  }
   __syncthreads();  // everyone is done reading red
   if (lane == 0) {
     red[wave][0][0] = en0;
