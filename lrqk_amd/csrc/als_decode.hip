@@ -631,7 +631,11 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
 // matrices went to LDS complete and the products of the iterations took their vector by the row of lanes (every step's
 // average): 32 heads, r = 32, two iterations 8.4 -> 7.1; 4 x 32 heads 8.6 -> 7.5; r = 16, eight iterations 10.6 -> 7.6.  Mean
 // error of q_hat and k_hat against 64 bits: 1.000 and 0.999 of what it was.
-template <int KS>
+// IN_ORDER (fp32 rows): the iterations add up element after element and in the formula y - (y.v / (1 + z.v)) z, as they always
+// did.  Neither form is closer to 64 bits, but a last bit of an fp32 iterate decides on tokens at the edge of the active set
+// some steps on (32 heads x 50K tokens, r = 16, eight iterations: outputs 4e-4 apart after five steps), more than fp32 results
+// may move; bf16 rows round it away.
+template <int KS, bool IN_ORDER>
 __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_kernel(const float* __restrict__ pre,
                                                                   const float* __restrict__ part, int S, int r,
                                                                   int max_iter, float* __restrict__ iter_out,
@@ -704,6 +708,61 @@ __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_ker
       invert_sweep_mfma<32, false>(elem, r, Mx + 32 * wave, inv);
   }
   __syncthreads();
+  if constexpr (IN_ORDER) {
+    // inside the first wave: lane c (and c + 32) holds column c of both inverses and element c of every vector
+    auto iterate = [&](auto n_c) {
+      constexpr int N = decltype(n_c)::value;
+      const int c = lane & 31;
+      float cK[N], cQ[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        cK[i] = GKi[i * kLdi + c];
+        cQ[i] = GQi[i * kLdi + c];
+      }
+      const float rq = rhs_q[c], kb = kB[c], sqk = s_qk;
+      auto vecmat = [&](float bvec, const float (&col)[N]) {
+        float y0 = 0.0f, y1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < N; i += 2) {
+          y0 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i)), col[i], y0);
+          y1 = fmaf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bvec), i + 1)), col[i + 1], y1);
+        }
+        return y0 + y1;
+      };
+      auto dot32 = [&](float a, float bb) {
+        const float x = row_reduce(a * bb, [](float p, float q2) { return p + q2; });
+        return lane_bcast(x, 0) + lane_bcast(x, 16);
+      };
+      auto rank1 = [&](float y0, float v, const float (&col)[N]) {
+        const float z = vecmat(v, col);
+        const float y = fmaf(sqk, z, y0);
+        const float alpha = dot32(y, v) / (1.0f + dot32(z, v));
+        return fmaf(-alpha, z, y);
+      };
+      const float hk0 = vecmat(kb, cK);  // k_hat_0 = kB G_K^-1
+      const float yq0 = vecmat(rq, cQ);  // rhs_q G_Q^-1
+      float hk = hk0;
+      for (int it = 0; it < max_iter; ++it) {
+        const float hq = rank1(yq0, hk, cQ);
+        const float nk = rank1(hk0, hq, cK);
+        const float df = c < r ? hk - nk : 0.0f;
+        const float dsq = dot32(df, df);
+        if (lane == 0) deltas[(int64_t)h * max_iter + it] = dsq;
+        float* o = iter_out + ((int64_t)h * max_iter + it) * 2 * r;
+        if (lane < r) {
+          o[lane] = hq;
+          o[r + lane] = nk;
+        }
+        hk = nk;
+      }
+    };
+    if (wave != 0) return;
+    if (r <= 16)  // (uniform)
+      iterate(std::integral_constant<int, 16>{});
+    else
+      iterate(std::integral_constant<int, 32>{});
+    return;
+  }
   // ---- k_hat_0 and the alternating rank-1 solves, all inside the first wave, which nothing runs beside: the chain is what it
   // issues.  Element c of a vector lies in lane c of every N lanes, and a product with an inverse multiplies by an element that
   // the row of 16 lanes hands round in the same instruction (32 elements: each half of the wave takes 16 of the terms), so
@@ -1328,7 +1387,7 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
     ctx->kq_n = n;
   }
 #define LRQK_SOLVE_CASE(KS)                                                                                     \
-  hipLaunchKernelGGL((als_solve_kernel<KS>), dim3((unsigned)bh), dim3(kSolveThreads), smem_solve, st, (const float*)pre, \
+  hipLaunchKernelGGL((als_solve_kernel<KS, sizeof(T) == 4>), dim3((unsigned)bh), dim3(kSolveThreads), smem_solve, st, (const float*)pre, \
                      (const float*)part, S, r, max_iter, iter_out, deltas)
   switch ((S + 3) / 4) {
     case 1: LRQK_SOLVE_CASE(4); break;

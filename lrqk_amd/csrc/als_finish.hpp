@@ -224,9 +224,9 @@ __device__ __forceinline__ void als_finish_body_mv(const FinishArgs& fa, int h, 
   en1 = wave_sum(en1);
   static_assert(kFinMaxR <= kWave, "a lane per element of the iterates");
   float hnq = 0.0f, hnk = 0.0f;
-  if (sizeof(T) == 4 && r > 32) {
-    // (the general solve, whose fp32 steps are ill-conditioned enough that the last bit of these sums decides on tokens at the
-    // edge of the active set and moves q_hat by 1e-3 some steps on: one element after the other, the order they always had)
+  if constexpr (sizeof(T) == 4) {
+    // (fp32 rows: a last bit of these sums decides on tokens at the edge of the active set and moves q_hat by up to 1e-3 some
+    // steps on: one element after the other, the order they always had)
     for (int i = 0; i < r; ++i) {
       hnq = fmaf(hat[0][i], hat[0][i], hnq);
       hnk = fmaf(hat[1][i], hat[1][i], hnk);
