@@ -23,14 +23,15 @@ __device__ __forceinline__ float half_pair(float lo_src, float hi_src, int hp) {
 
 // y + sum_i x_i col[i] over the 16 lanes of a row, x_i being lane i of the row: the multiply-add itself hands the lane's value round
 // (row_newbcast).  (In assembly: from the builtins come a move and a multiply-add each.  A moved operand must be two
-// instructions old, and so must the result for whoever moves it on.)
+// instructions old, and so must the result for whoever moves it on.  The first instruction writes y and the others still read
+// the operands: y takes a register that none of them has, also where one has y's value.)
 __device__ __forceinline__ float row_dot16(float x, const float* col, float y = 0.0f) {
 #define LRQK_BCAST_FMA(I, C) "v_fmac_f32_dpp %0, %1, %" #C " row_newbcast:" #I " row_mask:0xf bank_mask:0xf\n\t"
   asm("s_nop 1\n\t" LRQK_BCAST_FMA(0, 2) LRQK_BCAST_FMA(1, 3) LRQK_BCAST_FMA(2, 4) LRQK_BCAST_FMA(3, 5) LRQK_BCAST_FMA(4, 6)
           LRQK_BCAST_FMA(5, 7) LRQK_BCAST_FMA(6, 8) LRQK_BCAST_FMA(7, 9) LRQK_BCAST_FMA(8, 10) LRQK_BCAST_FMA(9, 11)
               LRQK_BCAST_FMA(10, 12) LRQK_BCAST_FMA(11, 13) LRQK_BCAST_FMA(12, 14) LRQK_BCAST_FMA(13, 15)
                   LRQK_BCAST_FMA(14, 16) LRQK_BCAST_FMA(15, 17) "s_nop 1"
-      : "+v"(y)
+      : "+&v"(y)
       : "v"(x), "v"(col[0]), "v"(col[1]), "v"(col[2]), "v"(col[3]), "v"(col[4]), "v"(col[5]), "v"(col[6]), "v"(col[7]),
         "v"(col[8]), "v"(col[9]), "v"(col[10]), "v"(col[11]), "v"(col[12]), "v"(col[13]), "v"(col[14]), "v"(col[15]));
 #undef LRQK_BCAST_FMA
