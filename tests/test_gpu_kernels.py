@@ -802,6 +802,25 @@ def test_als_prefill_given_sums(ops, ws, oracle, b, hq, hkv, l, r, offset):
             assert rel < 3e-5, (iters, name, rel)
 
 
+@pytest.mark.parametrize("hq,hkv,l,r", [(4, 2, 131072, 32), (6, 2, 100001, 31), (4, 4, 131072, 8)])
+def test_als_prefill_given_sums_have_no_bias(ops, ws, oracle, hq, hkv, l, r):
+    """bf16 rows of 128 elements, ranks up to 32: the sums over random factors (B = G^-1 C) of a long prompt.  An element of
+    A^T X of l random rows is around sqrt(l).  Rounding alone leaves 4e-8 of that (six products per 32 rows, each rounded at
+    2^-21) and 7e-8 (16 additions per wave and split at up to 22), 8e-8 together; the matrix cores round down, and with that
+    on one side in every step the error was 3.5e-7 and more at these lengths.  Twice the rounding."""
+    _say("als_prefill sums without a bias", hq, hkv, l, r)
+    g = torch.Generator().manual_seed(l + r)
+    Q = torch.randn((1, hq, l, 128), generator=g).to(torch.bfloat16)
+    K = torch.randn((1, hkv, l, 128), generator=g).to(torch.bfloat16)
+    A0 = [torch.randn((1, hq, l, r), generator=g) for _ in range(2)]
+    ref = oracle.als_prefill_w1(Q.double(), oracle.repeat_kv(K, hq // hkv).double(), A0[0].double(), A0[1].double(), 0, 0.0)
+    got = ops.als_prefill(ws, Q.to(DEV), K.to(DEV), *(a.to(DEV) for a in A0), 0, 0.0)
+    for name, x, y in (("B_Q", got[1], ref[1]), ("B_K", got[3], ref[3])):
+        rel = float((x.cpu().double() - y).norm() / y.norm())
+        print(name, "rel err %.3e" % rel, flush=True)
+        assert rel < 1.6e-7, (name, rel)
+
+
 def test_als_prefill_large_sums_every_head(ops, ws, oracle):
     """128K rows of rank-r data factorised at rank r from random factors: after the first iteration the K side's
     r x r systems have diagonals around 1e12 and condition numbers around 1e5.  The elimination used to leave
