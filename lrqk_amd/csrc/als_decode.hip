@@ -17,7 +17,6 @@
 // last-arriving workgroup continues was measured slower: the device-scope fence it needs
 // costs ~15 us per workgroup because each XCD has its own L2.)
 #include <algorithm>
-#include <stdlib.h>
 
 #include "common.hpp"
 #include "ctx.hpp"
@@ -321,7 +320,7 @@ __device__ __forceinline__ void gram_append(const GramAppend& ap, T* k_prev, int
 constexpr int kGramLd = 36;  // floats per tile row (16-byte aligned, rows four banks apart)
 constexpr int kGramTile = kGramChunk * kGramLd;
 constexpr int kGramVecSmem = kGramWaves * (kGramTile + kGramChunk);  // also the waves' sums, also the extra workgroups' B
-static_assert(kGramVecSmem >= kGramWaves * kGramNe && kGramVecSmem >= 32 * (128 + 1) + 2 * 128, "one block for all");
+static_assert(kGramVecSmem >= kGramWaves * kGramNe, "the cross-wave reduction fits the shared block");
 template <typename T, int LPR>
 __global__ __launch_bounds__(kGramThreads) void als_gram_vec_kernel(
     const T* __restrict__ a_k, int64_t head_stride, int64_t a_rows, const int32_t* __restrict__ active_idx, int64_t idx_stride,
@@ -334,6 +333,7 @@ __global__ __launch_bounds__(kGramThreads) void als_gram_vec_kernel(
   constexpr int AL = kGramChunk * PR / kWave;         // A loads per lane and chunk
   constexpr int kLprLog2 = LPR == 8 ? 3 : LPR == 16 ? 4 : 5;
   static_assert(LPR == 8 || LPR == 16 || LPR == 32, "");
+  static_assert(kGramVecSmem >= 32 * (d + 1) + 2 * d, "B_Q or B_K fits the shared block");
   __shared__ __align__(16) float gsm[kGramVecSmem];
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id();
   const int h = blockIdx.y, s = blockIdx.x;
@@ -1326,7 +1326,7 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
   if (S > 32) S = 32;
   // bf16, d = 128, r in {8, 16, 24, 32}, 16-byte aligned rows: the pipelined pass on the bf16 matrix cores
   const bool fast_bf16 = sizeof(T) == 2 && d == 128 && r % 8 == 0 && ((uintptr_t)a_k % 16 == 0) && n < (1 << 23) &&
-                         (head_stride * sizeof(T)) % 16 == 0 && !getenv("LRQK_GRAM_OLD");
+                         (head_stride * sizeof(T)) % 16 == 0;
   // (the pipelined pass: two chunks per wave measured best at 1, 4 and 8 sequences of the Llama-3-8B shape)
   if (fast_bf16) S = std::min(32, std::max(1, (n + 2 * kGramWaves * kGramChunk - 1) / (2 * kGramWaves * kGramChunk)));
   int rc = ctx->als_part.ensure((size_t)bh * S * kGramNe * sizeof(float));
@@ -1359,17 +1359,25 @@ static int als_decode_impl(lrqk_ctx* ctx, void* b_q, void* b_k, void* a_k, int64
     kq_out = (float*)ctx->als_kq.p;
   }
   // whole 16-byte pieces of A_K rows, K rows of 8, 16 or 32 pieces (and few enough slots for 32-bit offsets): see
-  // als_gram_vec_kernel
-  const bool vec_rows = r % VEC == 0 && ((uintptr_t)a_k % 16 == 0) && (head_stride * sizeof(T)) % 16 == 0 && d <= 128 &&
-                        (lpr == 8 || lpr == 16 || lpr == 32) && n < (1 << 22);
+  // als_gram_vec_kernel.  bf16 rows of 128 elements go through the pipelined pass, so that leaves 8 pieces (64 elements).
+  const auto vec_gram = [&] {
+    if constexpr (sizeof(T) == 2)
+      return lpr == 8 ? als_gram_vec_kernel<T, 8> : nullptr;
+    else
+      return lpr == 8    ? als_gram_vec_kernel<T, 8>
+             : lpr == 16 ? als_gram_vec_kernel<T, 16>
+             : lpr == 32 ? als_gram_vec_kernel<T, 32>
+                         : nullptr;
+  }();
+  const bool vec_rows = vec_gram && r % VEC == 0 && ((uintptr_t)a_k % 16 == 0) && (head_stride * sizeof(T)) % 16 == 0 &&
+                        n < (1 << 22);
   if (fast_bf16) {
     hipLaunchKernelGGL(als_gram_bf16_kernel, dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), 0, st,
                        (const bf16_t*)a_k, head_stride, a_rows, active_idx, idx_stride, (bf16_t*)k_prev, kprev_slots, n,
                        (const bf16_t*)q, r, part, S, ap, (const bf16_t*)b_q, (const bf16_t*)b_k, (const bf16_t*)k_new,
                        hq, hkv, pre, kq_out);
   } else if (vec_rows) {
-    const auto gram = lpr == 8 ? als_gram_vec_kernel<T, 8> : lpr == 16 ? als_gram_vec_kernel<T, 16> : als_gram_vec_kernel<T, 32>;
-    hipLaunchKernelGGL(gram, dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), 0, st, (const T*)a_k, head_stride, a_rows,
+    hipLaunchKernelGGL(vec_gram, dim3((unsigned)S + 2, (unsigned)bh), dim3(kGramThreads), 0, st, (const T*)a_k, head_stride, a_rows,
                        active_idx, idx_stride, (T*)k_prev, kprev_slots, n, (const T*)q, r, part, S, ap, (const T*)b_q,
                        (const T*)b_k, (const T*)k_new, hq, hkv, pre, kq_out);
   } else {

@@ -45,3 +45,15 @@ def test_row_dot_accumulator_has_a_register_of_its_own(tmp_path, start, zero):
     assert len({acc for acc, _, _ in steps}) == 1
     acc = steps[0][0]
     assert all(acc not in (x, c) for _, x, c in steps), steps
+
+
+LIB = os.path.join(os.path.dirname(CSRC), "liblrqk_hip.so")
+
+
+@pytest.mark.skipif(not os.path.exists(LIB) or not shutil.which("nm"), reason="needs the built library and nm")
+def test_gram_pass_is_compiled_for_the_rows_that_reach_it():
+    """The factor update's pass on 16-byte pieces: fp32 rows of 32, 64 and 128 elements and bf16 rows of 64 (8, 16, 32 and 8
+    pieces).  bf16 rows of 128 have a pass of their own, and those of 256 need more LDS than the pass has."""
+    names = subprocess.run(["nm", "-C", LIB], check=True, capture_output=True, text=True).stdout
+    assert set(re.findall(r"lrqk::als_gram_vec_kernel<([^>]*)>", names)) == {
+        "float, 8", "float, 16", "float, 32", "lrqk::bf16_t, 8"}
