@@ -20,6 +20,7 @@
 //                  occupied range fills the 4096 bins: one or two passes instead of three.
 //                  The selected ids are emitted in order through two bitmaps (key > T,
 //                  key == T) and, when asked, diffed in place against the resident set.
+#include <algorithm>
 #include <vector>
 
 #include "common.hpp"
@@ -1289,6 +1290,19 @@ __device__ __forceinline__ void select_step_ids(const DiffArgs& df, int h, int k
   for (int u = 0; u < kStepIpt; ++u) hv[u] = hit[min(tid * ipt + min(u, ipt - 1), k - 1)];
 }
 
+// Entries of a head's list that the kernel asks for before it knows the list's length, clamped by nothing but the buffer: four per
+// thread, and eight where k is large (the usual list has 1.5 k entries).  The buffer has room for them whatever the length.
+constexpr int kStepAheadUsual = 4, kStepAheadLong = 8;
+__host__ __device__ constexpr bool step_reads_long(int k) { return k > 2 * kSelThreads; }
+constexpr int list_capacity(int k) { return std::max(8 * k, kStepAheadUsual * kSelThreads); }
+constexpr bool step_reads_fit(int k) {
+  return list_capacity(k) >= (step_reads_long(k) ? kStepAheadLong : kStepAheadUsual) * kSelThreads;
+}
+// (the capacity does not shrink with k and the reads change once: the ends of both ranges stand for all of them)
+static_assert(step_reads_fit(1) && step_reads_fit(2 * kSelThreads) && step_reads_fit(2 * kSelThreads + 1) &&
+                  step_reads_long(2 * kSelThreads + 1) && !step_reads_long(2 * kSelThreads),
+              "reads ahead of the list's length stay in the head's buffer");
+
 // What the kernel is launched with, its only parameter.  The bodies read a member where they need it (scalar loads): taken as
 // separate parameters all of them are read at the start, and two thirds were moved to lanes of vector registers and back,
 // 45 + 60 instructions.
@@ -1587,34 +1601,33 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void se
   const int h = blockIdx.x, tid = threadIdx.x;
   const int cand_cap = args->cand_cap, k = args->k, m = (int)args->m;
   // Everything that is read is requested at once, and the blocks that are counted in are cleared meanwhile: the list's length
-  // and the head's state, the entries of the usual list (the buffer has room for four per thread whatever the length, and for
-  // eight where k is large; what lies beyond the length is not looked at) and the resident ids.  The entries were behind the
-  // wait for the length (0.9 us), the clearing behind both (0.9) and single values waited for by one wave in two later phases
-  // (0.7 each).
+  // and the head's state, the entries of the usual list (see list_capacity; what lies beyond the length is not looked at) and the
+  // resident ids.  The entries were behind the wait for the length (0.9 us), the clearing behind both (0.9) and single values
+  // waited for by one wave in two later phases (0.7 each).
   const uint2* cand = args->cand + (int64_t)h * cand_cap;
   const int n_v = args->st.cand_count[h * kCountStride], lvl_v = args->st.level[h];
   const uint32_t lo_v = args->st.t_used[h];
   float q_cur = args->st.q_cur[h];
   int vic_at = args->df.vic_ptr ? args->df.vic_ptr[h] : 0;
-  constexpr int kAhead = 8;
-  const bool ahead8 = k > 2 * kSelThreads;  // (the usual list has 1.5 k entries; cand_cap >= 8 k)
-  uint2 c4[4], c8[kAhead];
+  constexpr int kShort = kStepAheadUsual, kAhead = kStepAheadLong;
+  const bool ahead8 = step_reads_long(k);
+  uint2 c4[kShort], c8[kAhead];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) c4[u] = cand[tid + u * kSelThreads];
+  for (int u = 0; u < kShort; ++u) c4[u] = cand[tid + u * kSelThreads];
 #pragma unroll
   for (int u = 0; u < kAhead; ++u) c8[u] = make_uint2(0, 0);
   if (ahead8) {  // (uniform)
 #pragma unroll
-    for (int u = 4; u < kAhead; ++u) c8[u] = cand[tid + u * kSelThreads];
+    for (int u = kShort; u < kAhead; ++u) c8[u] = cand[tid + u * kSelThreads];
   }
   int32_t hv[kStepIpt];
   select_step_ids(args->df, h, k, tid, hv);
   select_step_clear(L, m, tid);
 #pragma unroll
   for (int u = 0; u < kAhead; ++u) {  // (not moved behind the branch on the length)
-    if (u < 4) c8[u] = c4[u];
+    if (u < kShort) c8[u] = c4[u];
     asm volatile("" : "+v"(c8[u].x), "+v"(c8[u].y));
-    if (u < 4) c4[u] = c8[u];
+    if (u < kShort) c4[u] = c8[u];
   }
 #pragma unroll
   for (int u = 0; u < kStepIpt; ++u) asm volatile("" : "+v"(hv[u]));
@@ -1634,8 +1647,8 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((aligned(8192))) void se
   const uint32_t lo = __builtin_amdgcn_readfirstlane(lo_v);
   // (a path of its own to the end: with the usual list as one branch of several its entries are held, that is spilled, across
   // the others)
-  if (fast && n <= 4 * kSelThreads) {
-    select_step_fast<4>(L, c4, hv, n, lo, q_cur, vic_at, h, m, k, bound_rank(k, level, n));
+  if (fast && n <= kShort * kSelThreads) {
+    select_step_fast<kShort>(L, c4, hv, n, lo, q_cur, vic_at, h, m, k, bound_rank(k, level, n));
     if (tid == 0) {
       atomicAdd(&args->st.stats[0], 1);
       args->st.level[h] = level | (calm << 8);
@@ -1717,7 +1730,7 @@ static int prepare_select(lrqk_ctx* ctx, int bh, int64_t m, int topk, hipStream_
   sb->key_stride = (m + 63) & ~(int64_t)63;
   if ((rc = ctx->keys.ensure((size_t)bh * sb->key_stride * 4))) return rc;
   sb->keys = (uint32_t*)ctx->keys.p;
-  sb->cand_cap = 8 * topk < 4096 ? 4096 : 8 * topk;  // (the register-resident paths take up to 8192 and 16384 entries)
+  sb->cand_cap = list_capacity(topk);  // (the register-resident paths take up to 8192 and 16384 entries)
   if ((rc = ctx->cand.ensure((size_t)bh * sb->cand_cap * sizeof(uint2)))) return rc;
   sb->cand = (uint2*)ctx->cand.p;
   // layout: t_low u32 [bh] | q_norm f32 [bh] | t_used u32 [bh] | q_cur f32 [bh] | (unused) [bh] | level i32 [bh] |
