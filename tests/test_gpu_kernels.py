@@ -422,6 +422,9 @@ def test_score_select_diff_few_distinct_scores(ops, oracle, m, k, values):
         _, evict, slots, count = ops.score_select_diff(ws, Ad, q.to(DEV), m, k, hit, want_new=False)
         assert torch.equal(hit.cpu().long(), now[..., 0]) and torch.equal(evict.cpu().bool(), gone), rnd
         assert torch.equal(count.cpu().long(), gone.sum(-1)), rnd
+        # the first call has to scan its three heads; the lists of the others fit (at most m entries of max(4096, 8 k)), so
+        # both are answered from them and not by another scan
+        assert ws.select_stats() == ((0, 3) if rnd == 0 else (3, 0)), rnd
 
 
 def test_score_select_many_chunks(ops, ws, oracle):
@@ -629,6 +632,60 @@ def test_als_decode_slot_counts(ops, ws, oracle, dtype, d, r, n):
     """Passes over the active rows whose waves take 16 or 32 slots at a time, in splits of 128 and 256 (rows of 8, 16 and 32
     pieces of 16 bytes; ranks 33 to 64): a slot short of a group, a whole one, a slot more."""
     _check_als_decode(ops, ws, oracle, dtype, 2, 1, n, d, r, 2, 0.0)
+
+
+@pytest.mark.parametrize("dtype,d,r", [(torch.float32, 128, 16), (torch.float32, 64, 32), (torch.float32, 32, 12),
+                                       (torch.bfloat16, 64, 24), (torch.bfloat16, 128, 32), (torch.bfloat16, 128, 64),
+                                       (torch.bfloat16, 128, 40)])
+def test_decode_step_ring_slot(ops, ws, oracle, dtype, d, r):
+    """The new token's slot at every place of the ring, one step each from the same state: 288 slots, so groups of 32, splits and
+    waves begin and end at many of them.  The pass over the active rows takes the token's K row and id from the caller while
+    another workgroup (ranks to 32) or the next launch (above) writes them into the slot; q_hat, k_hat and the attention see
+    it (its A_K row and its key are large), K, V and id lie in the slot, and the ring's other slots are what they were."""
+    _say("decode_step ring slots", dtype, d, r)
+    g = torch.Generator().manual_seed(d + r)
+    hq, hkv, lite, m = 2, 1, 287, 64
+    n, token = 1 + lite, 400
+    x = _als_inputs(g, 1, hq, hkv, n, d, r, token + 1, dtype)
+    x["A"][:, :, token] *= 4.0
+    x["k"] = x["k"] * 2.0
+    V, v = torch.randn((1, hq, n, d), generator=g).to(dtype), torch.randn((1, hkv, 1, d), generator=g).to(dtype)
+    idx = torch.cat((torch.zeros((1, hq, 1), dtype=torch.long),
+                     torch.stack([m + torch.randperm(token - m, generator=g)[:lite] for _ in range(hq)]).view(1, hq, lite)), 2)
+    store = torch.randn((1, hkv, token + 1, 2 * d), generator=g).to(dtype).pin_memory()
+    kn, vn = oracle.repeat_kv(x["k"], hq)[0, :, 0], oracle.repeat_kv(v, hq)[0, :, 0]
+    # all places at once, as a batch
+    ids = idx.repeat(lite, 1, 1)
+    Kp = x["Kp"].repeat(lite, 1, 1, 1)
+    for i in range(lite):
+        ids[i, :, 1 + i] = token
+        Kp[i, :, 1 + i] = kn
+    big = {k_: x[k_].double().repeat(lite, 1, 1, 1) for k_ in ("B_Q", "B_K", "q")}
+    A_act = torch.take_along_dim(x["A"].double().expand(lite, -1, -1, -1), ids.unsqueeze(-1), 2)
+    ref = oracle.als_decode_w1(big["B_Q"], A_act, big["B_K"], Kp.double(), big["q"], kn.double()[None, :, None], 2, 0.0)
+    lim = 6e-3 if dtype == torch.bfloat16 else 2e-4        # as in _check_als_decode, and the attention as in test_attention
+    lim_attn = 3e-3 if dtype == torch.bfloat16 else 1e-5
+    dev = {k_: t.to(DEV) for k_, t in x.items()}
+    dev.update(V=V.to(DEV), v=v.to(DEV), idx=idx.to(torch.int32).to(DEV))
+    q_hat, k_hat = (torch.empty((1, hq, 1, r), dtype=dtype, device=DEV) for _ in range(2))
+    attn = torch.empty((1, hq, 1, d), dtype=dtype, device=DEV)
+    for i in range(lite):
+        st = {k_: dev[k_].clone() for k_ in ("B_Q", "B_K", "A", "Kp", "V", "idx")}
+        ops.decode_step(ws, st["B_Q"], st["B_K"], st["A"], st["idx"], st["Kp"], st["V"], store, dev["q"], dev["k"], dev["v"],
+                        topk=1, lite=lite, ring_slot=i, token=token, m=m, flush_row0=-1, max_iter=2, tol=0.0,
+                        round_scores=True, no_hit_miss=False, q_hat=q_hat, k_hat=k_hat, attn_out=attn)
+        K1, V1, ids1 = st["Kp"][0].cpu(), st["V"][0].cpu(), st["idx"][0].cpu()
+        want_V = V[0].clone()
+        want_V[:, 1 + i] = vn
+        assert torch.equal(K1[:, 1:], Kp[i, :, 1:]) and torch.equal(V1[:, 1:], want_V[:, 1:]), i
+        assert torch.equal(ids1[:, 1:].long(), ids[i, :, 1:]), i
+        for name, got, exp in (("q_hat", q_hat, ref[2][i]), ("k_hat", k_hat, ref[3][i])):
+            rel = (got[0].cpu().double() - exp).norm() / exp.norm()
+            assert rel < lim, (i, name, float(rel))
+        assert torch.equal(st["A"][0, :, token].cpu(), k_hat[0, :, 0].cpu()), i
+        exp = oracle.attention(x["q"], K1[None], V1[None])
+        rel = (attn.cpu().double() - exp).norm() / exp.norm()
+        assert rel < lim_attn, (i, "attention", float(rel))
 
 
 def _check_als_decode(ops, ws, oracle, dtype, hq, hkv, n, d, r, max_iter, tol):
