@@ -629,12 +629,14 @@ __global__ __launch_bounds__(kGramThreads, 4) void als_gram_bf16_kernel(
 // copying the whole tile out of the accumulation registers.)
 // One workgroup per head: latency and the instructions of one wave bound it, not memory.  Launch, us, before and after the
 // matrices went to LDS complete and the products of the iterations took their vector by the row of lanes (every step's
-// average): 32 heads, r = 32, two iterations 8.4 -> 7.1; 4 x 32 heads 8.6 -> 7.5; r = 16, eight iterations 10.6 -> 7.6.  Mean
-// error of q_hat and k_hat against 64 bits: 1.000 and 0.999 of what it was.
+// average): 32 heads, r = 32, two iterations 8.4 -> 7.1; 4 x 32 heads 8.6 -> 7.5; r = 16, eight iterations 10.6 -> 7.6.
 // IN_ORDER (fp32 rows): the iterations add up element after element and in the formula y - (y.v / (1 + z.v)) z, as they always
-// did.  Neither form is closer to 64 bits, but a last bit of an fp32 iterate decides on tokens at the edge of the active set
-// some steps on (32 heads x 50K tokens, r = 16, eight iterations: outputs 4e-4 apart after five steps), more than fp32 results
-// may move; bf16 rows round it away.
+// did.  That form adds s z and takes most of it away again: on low-rank prompts its iterates are 3 .. 4 times as far from 64 bits
+// (rms over 32 heads, ranks 8 .. 32, 544 .. 4224 slots, one to eight iterations: 7e-6 against 2e-6; random rows 2e-7 with either, 0.95
+// .. 1.06 of each other).  But a last bit of an iterate decides on tokens at the edge of the active set some steps on (32 heads x 50K
+// tokens, r = 16, eight iterations: outputs 4e-4 apart after five steps), which is more than fp32 results may move.  bf16 results
+// move as well, 2e-3 of the attention from step to step (a value that rounds to its other neighbour, and with it a token at the
+// edge), within what their rounding leaves and towards the 64-bit result.
 template <int KS, bool IN_ORDER>
 __global__ __launch_bounds__(kSolveThreads, KS <= 16 ? 2 : 1) void als_solve_kernel(const float* __restrict__ pre,
                                                                   const float* __restrict__ part, int S, int r,

@@ -492,8 +492,8 @@ __global__ __launch_bounds__(kS64Threads) void als_solve64_bf16_kernel(
   __syncthreads();
   if (wave != 0) return;
   // ---- the alternating iterations, lane c <-> element c of every vector (zeros beyond r), the inverses' columns in the lanes'
-  // registers (see als_solve_kernel; with every product reading the columns from LDS and handing the vector round by scalar
-  // registers the launch took 24.9 us instead of 22.1)
+  // registers (see als_solve_kernel, also for the formula of rank1: against 64 bits the iterates at ranks 40 .. 64 are 2e-6 off on
+  // low-rank prompts, where y - (y.v / (1 + z.v)) z left 9e-6, and 3.5e-7 on random rows with either)
   float cQ[64], cK[64];
 #pragma unroll
   for (int i = 0; i < 64; ++i) {

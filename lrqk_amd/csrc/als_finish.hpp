@@ -226,7 +226,8 @@ __device__ __forceinline__ void als_finish_body_mv(const FinishArgs& fa, int h, 
   float hnq = 0.0f, hnk = 0.0f;
   if constexpr (sizeof(T) == 4) {
     // (fp32 rows: a last bit of these sums decides on tokens at the edge of the active set and moves q_hat by up to 1e-3 some
-    // steps on: one element after the other, the order they always had)
+    // steps on: one element after the other, the order they always had, although the sum by the wave is the closer one: 4e-8
+    // of 64 bits at every rank against 5e-8 at rank 8 and 1.2e-7 at 64)
     for (int i = 0; i < r; ++i) {
       hnq = fmaf(hat[0][i], hat[0][i], hnq);
       hnk = fmaf(hat[1][i], hat[1][i], hnk);

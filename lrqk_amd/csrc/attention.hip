@@ -118,7 +118,8 @@ __device__ __forceinline__ void attn_scan_w(const float* __restrict__ w, float s
 #pragma unroll
     for (int u = 0; u < U; ++u) asm volatile("" : "+v"(wl[u]));
     // One maximum and one rescaling per batch: the workgroups of the launch that this runs in keep every SIMD's issue busy, and
-    // a maximum, two exponentials and a rescaled accumulator per row were most of what this role issued.
+    // a maximum, two exponentials and a rescaled accumulator per row were most of what this role issued.  (The output is as far
+    // from 64 bits as with one per row, within 0.2 %: 6.0e-7 of 28 fp32 heads with 512 tokens, 6.7e-7 with 4096.)
     float m_new = st.m;
 #pragma unroll
     for (int u = 0; u < U; ++u) {

@@ -164,8 +164,9 @@ __device__ __forceinline__ int row_inclusive_sum(int v) {
   return x;
 }
 
-// A move within the row whose source lane always exists, in a wave that is active as a whole: written so that the compiler can
-// make it part of the instruction that uses it (with the lane's own value for a missing source it was a copy and a move more).
+// A move within the row whose source lane always exists, in a wave that is active as a whole (an inactive source lane gives 0, not
+// the lane's own value): written so that the compiler can make it part of the instruction that uses it (with the lane's own value
+// for a missing source it was a copy and a move more).
 template <int CTRL>
 __device__ __forceinline__ int dpp_full(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
@@ -174,7 +175,8 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_full(float v) {
   return __int_as_float(dpp_full<CTRL>(__float_as_int(v)));
 }
-// Butterflies inside each row of 16 lanes; afterwards every lane of a row holds the row's result.
+// Butterflies inside each row of 16 lanes; afterwards every lane of a row holds the row's result.  Every lane of the row must be
+// active.
 template <typename Op>
 __device__ __forceinline__ float row_reduce(float v, Op op) {
   v = op(v, dpp_full<kDppQuadXor1>(v));
@@ -188,7 +190,8 @@ __device__ __forceinline__ float lane_bcast(float v, int lane) {
 }
 
 // Sum over aligned groups of `n` adjacent lanes (n a power of two); every lane of a group gets
-// the group's sum.  Steps inside a row of 16 lanes are register moves, wider ones shuffles.
+// the group's sum.  Every lane of the group must be active.  Steps inside a row of 16 lanes are register moves, wider ones
+// exchanges of rows.
 __device__ __forceinline__ float group_sum(float v, int n) {
   if (n > 1) v += dpp_full<kDppQuadXor1>(v);
   if (n > 2) v += dpp_full<kDppQuadXor2>(v);
@@ -205,7 +208,8 @@ __device__ __forceinline__ float group_sum(float v, int n) {
   }
   return v;
 }
-// wave-wide reductions of unsigned values, result in every lane
+// Wave-wide reductions of unsigned values, result in every lane.  Every lane of the wave must be active: a lane that has
+// nothing to add takes part with the operation's neutral value.
 template <typename Op>
 __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t v, Op op) {
   v = op(v, (uint32_t)dpp_full<kDppQuadXor1>((int)v));
@@ -217,7 +221,7 @@ __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t v, Op op) {
   return op(op(a, b), op(c, d));
 }
 
-// result in every lane
+// Result in every lane; every lane of the wave must be active, as above.
 __device__ __forceinline__ float wave_sum(float v) {
   v = row_reduce(v, [](float a, float b) { return a + b; });
   return (lane_bcast(v, 0) + lane_bcast(v, 16)) + (lane_bcast(v, 32) + lane_bcast(v, 48));
