@@ -182,8 +182,8 @@ def prefill_roofline(w, l, iters, ms):
         exec_flops = (l / 32.0) * (bh * 2 * (mf_given + mf_apply) + (bh + bkv) * mf_xtx) * 2.0 * 32 * 32 * 16
         passes = ("pf_sums_kernel + pf_stream_apply_kernel" if tuned else
                   "pf_stream_sums_kernel + pf_stream_apply_kernel")
-        roof = {"bound": "hbm", "kernel": f"{passes} ({reads_q} readings of Q, {reads_k} of K); pf_gramdom_kernel (fp64 "
-                                          "d x d algebra per head, latency-bound) between them",
+        roof = {"bound": "hbm", "kernel": f"{passes} ({reads_q} readings of Q, {reads_k} of K); pf_gs_kernel (up to rank "
+                                          "16 pf_gramdom_kernel; fp64 d x d algebra per head, latency-bound) between them",
                 "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
                 "traffic": None, "hbm_bytes_per_call": round(bytes_g),
                 "algorithmic_flops_per_call": round(flops), "algorithmic_equiv_tflops": round(tf, 2),
